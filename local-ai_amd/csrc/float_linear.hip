@@ -1,12 +1,14 @@
 // Products of activations with bf16 weights [N, K]:
+//   linear_phased_kernel bf16 activations, K a multiple of 64, enough tiles of 128 x 128 for the chip: eight waves in two phases
 //   linear_mfma_kernel   bf16 activations, K a multiple of 8: LDS-tiled bf16 MFMA 16x16x32, tiles loaded straight into LDS
 //   linear_plain_kernel  everything else: f32 FMA on 64 x 64 tiles (the 32-bit runs, ragged K)
 //   matvec_bf16_kernel   one row, HBM-bound weight streaming, with the norm before the product done while x is staged
-// All three end in the same column segments (bias, activation, layout, residual add), and the first two also run the
-// experts of a mixture on the tiles of a routing plan.
+// All end in the same column segments (bias, activation, layout, residual add), and linear_mfma_kernel and linear_plain_kernel also
+// run the experts of a mixture on the tiles of a routing plan.
 #include "float_linear.hpp"
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 namespace {
 
@@ -97,48 +99,234 @@ __device__ __forceinline__ void store4(const LhLinear& a, uint32_t slot, uint32_
     }
 }
 
-// A finished tile into a value cache: a thread stores a quarter of a block of 32 positions of one column, which is 16 bytes where
-// the tile has all of them.  `tile` as linear_mfma_kernel leaves it.
-template <int BM, int BN>
-__device__ __forceinline__ void store_blocks(const LhLinear& a, uint32_t s, const float* tile, const RowTile& rt, uint32_t n0, uint32_t pos0) {
+// Place of four-column piece c of row m in a wave's tile of N columns in LDS.
+template <int N> __device__ __forceinline__ uint32_t piece(uint32_t m, uint32_t c) { return m * (N / 4) + (c ^ (m & (N / 4 < 8 ? N / 4 - 1 : 7))); }
+
+// A wave's finished tile of N columns into a value cache: four lanes store the quarters of a block of 32 positions of one column,
+// 16 bytes each where the tile has all of a quarter.
+template <int N>
+__device__ __forceinline__ void store_blocks(const LhLinear& a, uint32_t s, const float* tile, const RowTile& rt, uint32_t n0, uint32_t pos0, uint32_t lane) {
     const uint32_t first = pos0 + rt.begin, last = min(pos0 + rt.end, a.seg.rows[s]), b0 = first >> 5;      // positions [first, last)
     if (first >= last) return;
-    const uint32_t blocks = ((last - 1) >> 5) - b0 + 1, cols = min((uint32_t)BN, a.N - n0);
-    uint16_t* out = static_cast<uint16_t*>(a.seg.out[s]);
+    const uint32_t blocks = ((last - 1) >> 5) - b0 + 1, g = lane & 3;
 #pragma unroll 1
-    for (uint32_t e = threadIdx.x; e < blocks * cols * 4; e += 256) {
-        const uint32_t g = e & 3, j = (e >> 2) % cols, b = b0 + (e >> 2) / cols, n = n0 + j;
-        uint32_t c = n - a.seg.n0[s];
+    for (uint32_t j = lane >> 2; j < N && n0 + j < a.N; j += 16) {
+        uint32_t c = n0 + j - a.seg.n0[s];
         if (a.seg.head[s] != a.seg.padded[s]) { const uint32_t h = c / a.seg.head[s]; c = h * a.seg.padded[s] + (c - h * a.seg.head[s]); }
-        uint16_t* d = out + ((size_t)b * a.seg.ld[s] + c) * 32 + g * 8;
-        const float bias = a.bias ? a.bias[n] : 0.0f;
-        uint16_t v[8];
-        bool all = true, in[8];
+        uint16_t* d = static_cast<uint16_t*>(a.seg.out[s]) + ((size_t)b0 * a.seg.ld[s] + c) * 32 + g * 8;
+        const float bias = a.bias ? a.bias[n0 + j] : 0.0f;
+#pragma unroll 1
+        for (uint32_t b = b0; b < b0 + blocks; b++, d += (size_t)a.seg.ld[s] * 32) {
+            uint16_t v[8];
+            bool all = true, in[8];
 #pragma unroll
-        for (uint32_t i = 0; i < 8; i++) {                    // entries 8 g + i: positions 4 g + i and 16 + 4 g + i - 4
-            const uint32_t p = b * 32 + (i >> 2) * 16 + g * 4 + (i & 3);
-            in[i] = p >= first && p < last;
-            all = all && in[i];
-            const uint32_t m = in[i] ? p - first : 0u;
-            v[i] = lh_f2bf(lh_activate(tile[(m * (BN / 4) + ((j >> 2) ^ (m & 7))) * 4 + (j & 3)] + bias, a.seg.act[s]));
-        }
-        if (all) *reinterpret_cast<uint4*>(d) = make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
-        else {
+            for (uint32_t i = 0; i < 8; i++) {                // entries 8 g + i: positions 4 g + i and 16 + 4 g + i - 4
+                const uint32_t p = b * 32 + (i >> 2) * 16 + g * 4 + (i & 3);
+                in[i] = p >= first && p < last;
+                all = all && in[i];
+                const uint32_t m = in[i] ? p - first : 0u;
+                v[i] = lh_f2bf(lh_activate(tile[piece<N>(m, j >> 2) * 4 + (j & 3)] + bias, a.seg.act[s]));
+            }
+            if (all) *reinterpret_cast<uint4*>(d) = make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16, v[6] | (uint32_t)v[7] << 16);
+            else {
 #pragma unroll
-            for (uint32_t i = 0; i < 8; i++) if (in[i]) d[i] = v[i];
+                for (uint32_t i = 0; i < 8; i++) if (in[i]) d[i] = v[i];
+            }
         }
     }
 }
+
+// A wave's finished tile of M x N from LDS to its destination.
+template <int M, int N>
+__device__ __forceinline__ void store_tile(const LhLinear& a, const float4* tile, const RowTile& rt, uint32_t n0, uint32_t pos0, uint32_t lane) {
+    const uint32_t s = lh_segment_of(a.seg, n0);
+    if (a.seg.layout[s] == LH_BLOCKS_AT_POSITION && !a.seg.f32[s] && s == lh_segment_of(a.seg, min(n0 + N, a.N) - 1) && a.ex.tiles == nullptr) {
+        store_blocks<N>(a, s, reinterpret_cast<const float*>(tile), rt, n0, pos0, lane);
+        return;
+    }
+#pragma unroll 1
+    for (uint32_t e = lane; e < M * N / 4; e += 64) {
+        const uint32_t m = e / (N / 4), c = e % (N / 4), n = n0 + c * 4, slot = rt.begin + m;
+        if (slot >= rt.end || n >= a.N) continue;
+        store4(a, slot, n, tile[piece<N>(m, c)], pos0);
+    }
+}
+
+// What is left to do for the tile of TI * 16 rows and TJ * 16 columns that a wave has in registers (column 4 TJ (lane >> 4) + 4 j + t
+// of row lane & 15 in register t of acc[i][j]: the kernels deal the rows of W to the matrix instructions that way).  A lane finishes
+// its 4 TJ neighbouring columns in registers and stores them in 16-byte pieces.  Value blocks, and segments that are not made of
+// multiples of 4 TJ, go through LDS, `box`, which is the wave's own.  (All through LDS, in pieces of four columns with their
+// segments looked up one by one: 93 us instead of 60 for the product of 2048 x 2048 x 8192 with gelu.)
+enum { kThroughLds = -1, kNoActivation = 0, kGelu, kSilu, kSiluPairs, kReluSquared };   // kSilu, kReluSquared: of the segments that have it
+
+// Where a lane's columns go, the same for all its rows.
+struct LaneColumns {
+    uint32_t n, s, c, ld, act, f32, at_position, rows;         // first column, its segment and its place there
+    char* out;                                                // of row 0
+    __device__ __forceinline__ LaneColumns(const LhSegments& seg, uint32_t first) : n(first), s(lh_segment_of(seg, first)) {
+        c = n - seg.n0[s];
+        act = seg.act[s]; f32 = seg.f32[s]; ld = seg.ld[s]; rows = seg.rows[s];
+        if (act == LH_ACT_SILU_PAIRS) c >>= 1;
+        else if (seg.head[s] != seg.padded[s]) { const uint32_t h = c / seg.head[s]; c = h * seg.padded[s] + (c - h * seg.head[s]); }
+        at_position = lh_segment_at_position(seg, s);
+        out = static_cast<char*>(seg.out[s]) + (size_t)c * (f32 ? 4 : 2);
+    }
+};
+// (bf16 results: the hardware's exponential and reciprocal, each good to an ulp of 32 bits)
+__device__ __forceinline__ float quick_sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z)); }
+template <int EPI> __device__ __forceinline__ float quick_activate(float v, uint32_t act) {
+    if constexpr (EPI == kGelu) return v * quick_sigmoid(1.5957691216057308f * (v + 0.044715f * v * v * v));
+    if constexpr (EPI == kSilu) return act == LH_ACT_SILU ? v * quick_sigmoid(v) : v;
+    if constexpr (EPI == kReluSquared) { const float r = fmaxf(v, 0.0f); return act == LH_ACT_RELU_SQUARED ? r * r : v; }
+    return v;
+}
+template <int EPI, int TI, int TJ>
+__device__ __forceinline__ void store_columns(const LhLinear& a, const lh_f32x4 (*acc)[TJ], const LaneColumns& col, uint32_t slot0, uint32_t end, uint32_t pos0) {
+    constexpr int CN = 4 * TJ;
+    if (col.n >= a.N) return;
+    float bias[CN];
+#pragma unroll
+    for (int j = 0; j < CN; j++) bias[j] = a.bias ? a.bias[col.n + j] : 0.0f;
+    // A row's destination; what is there already is requested a row ahead.
+    struct Row { uint32_t p; float weight; bool valid; };
+    auto row = [&](int i) {
+        const uint32_t slot = slot0 + i * 16;
+        Row r{0, 1.0f, slot < end};
+        if (r.valid) {
+            const OutRow o = out_row(a, slot);
+            r.p = col.at_position ? pos0 + o.row : o.row; r.weight = o.weight;
+            r.valid = r.p < col.rows;
+        }
+        return r;
+    };
+    const bool add = EPI == kNoActivation && a.seg.accumulate && col.f32;
+    float4 x[2][TJ];
+    auto fetch = [&](const Row& r, float4 (&d)[TJ]) {
+        if (!add || !r.valid) return;
+#pragma unroll
+        for (int j = 0; j < TJ; j++) d[j] = reinterpret_cast<const float4*>(col.out + (size_t)r.p * col.ld * 4)[j];
+    };
+    Row next = row(0);
+    fetch(next, x[0]);
+#pragma unroll
+    for (int i = 0; i < TI; i++) {
+        const Row r = next;
+        if (i + 1 < TI) { next = row(i + 1); fetch(next, x[(i + 1) & 1]); }
+        if (!r.valid) continue;
+        float v[CN];
+#pragma unroll
+        for (int j = 0; j < CN; j++) v[j] = quick_activate<EPI>(acc[i][j >> 2][j & 3] * r.weight + bias[j], col.act);
+        if (EPI != kSiluPairs && col.f32) {
+            float4* d = reinterpret_cast<float4*>(col.out + (size_t)r.p * col.ld * 4);
+            if (add) {
+#pragma unroll
+                for (int j = 0; j < TJ; j++) { const float4 y = x[i & 1][j]; v[4 * j] += y.x; v[4 * j + 1] += y.y; v[4 * j + 2] += y.z; v[4 * j + 3] += y.w; }
+            }
+#pragma unroll
+            for (int j = 0; j < TJ; j++) d[j] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+            continue;
+        }
+        constexpr int W = EPI == kSiluPairs ? TJ : 2 * TJ;     // words of two bf16
+        uint32_t w[W];
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            if constexpr (EPI == kSiluPairs) w[j] = lh_pack_bf(v[4 * j] * quick_sigmoid(v[4 * j]) * v[4 * j + 1], v[4 * j + 2] * quick_sigmoid(v[4 * j + 2]) * v[4 * j + 3]);
+            else w[j] = lh_pack_bf(v[2 * j], v[2 * j + 1]);
+        }
+        char* d = col.out + (size_t)r.p * col.ld * 2;
+        if constexpr (W == 8) { reinterpret_cast<uint4*>(d)[0] = make_uint4(w[0], w[1], w[2], w[3]); reinterpret_cast<uint4*>(d)[1] = make_uint4(w[4], w[5], w[6], w[7]); }
+        else if constexpr (W == 4) *reinterpret_cast<uint4*>(d) = make_uint4(w[0], w[1], w[2], w[3]);
+        else if constexpr (W == 2) *reinterpret_cast<uint2*>(d) = make_uint2(w[0], w[1]);
+        else *reinterpret_cast<uint32_t*>(d) = w[0];
+    }
+}
+
+// The same into a value cache, for whole blocks of 32 positions.  Four neighbouring lanes have positions 4 q .. 4 q + 3 of four
+// columns; transposed among themselves, over the two 16-row tiles of a block, each has the 16 bytes 4 g .. of one column's block.
+__device__ __forceinline__ void transpose_quads(uint32_t (&u)[4], uint32_t lane) {
+    const bool odd = lane & 1, high = lane & 2;
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {                          // 2 x 2 blocks
+        const uint32_t give = odd ? u[e] : u[e + 1], got = (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR1>((int)give);
+        if (odd) u[e] = got; else u[e + 1] = got;
+    }
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const uint32_t give = high ? u[e] : u[e + 2], got = (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR2>((int)give);
+        if (high) u[e] = got; else u[e + 2] = got;
+    }
+}
+template <int EPI, int TI, int TJ>
+__device__ __forceinline__ void store_whole_blocks(const LhLinear& a, const lh_f32x4 (*acc)[TJ], const LaneColumns& col, uint32_t position, uint32_t lane) {
+    const uint32_t q = (lane >> 2) & 3, k = lane & 3;
+    uint16_t* out = reinterpret_cast<uint16_t*>(a.seg.out[col.s]) + ((size_t)(position >> 5) * col.ld + col.c + k) * 32 + q * 8;
+#pragma unroll
+    for (int j = 0; j < TJ; j++) {
+        float bias[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) bias[t] = a.bias ? a.bias[col.n + 4 * j + t] : 0.0f;
+#pragma unroll
+        for (int b = 0; b < TI / 2; b++) {
+            uint32_t u[4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) u[t] = lh_pack_bf(quick_activate<EPI>(acc[2 * b][j][t] + bias[t], col.act), quick_activate<EPI>(acc[2 * b + 1][j][t] + bias[t], col.act));
+            transpose_quads(u, lane);
+            *reinterpret_cast<uint4*>(out + ((size_t)b * col.ld + 4 * j) * 32) =
+                make_uint4(__builtin_amdgcn_perm(u[1], u[0], 0x05040100u), __builtin_amdgcn_perm(u[3], u[2], 0x05040100u),
+                           __builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u));
+        }
+    }
+}
+
+template <int EPI, int TI, int TJ>
+__device__ __forceinline__ void finish_tile(const LhLinear& a, const lh_f32x4 (*acc)[TJ], const RowTile& rt, uint32_t row0, uint32_t nw, uint32_t lane, float4* box) {
+    if (nw >= a.N) return;
+    const uint32_t pos0 = a.seg.position ? *a.seg.position : 0u, g = lane >> 4;
+    if constexpr (EPI != kThroughLds) {
+        const uint32_t s0 = lh_segment_of(a.seg, nw), s1 = lh_segment_of(a.seg, min(nw + 16 * TJ, a.N) - 1), first = rt.begin + row0, at = pos0 + first;
+        const bool blocks = a.seg.layout[s0] == LH_BLOCKS_AT_POSITION;
+        if (!blocks && a.seg.layout[s1] != LH_BLOCKS_AT_POSITION) {
+            store_columns<EPI, TI, TJ>(a, acc, LaneColumns(a.seg, nw + g * 4 * TJ), first + (lane & 15), rt.end, pos0);
+            return;
+        }
+        if constexpr (EPI != kSiluPairs && TI % 2 == 0) {
+            if (blocks && s0 == s1 && !a.seg.f32[s0] && nw + 16 * TJ <= a.N && at % 32 == 0 && first + TI * 16 <= rt.end && at + TI * 16 <= a.seg.rows[s0] && a.ex.tiles == nullptr) {
+                store_whole_blocks<EPI, TI, TJ>(a, acc, LaneColumns(a.seg, nw + g * 4 * TJ), at, lane);
+                return;
+            }
+        }
+    }
+    constexpr int RP = TI < 4 ? TI : 4;                       // 16-row tiles at a time
+#pragma unroll
+    for (int h = 0; h < TI / RP; h++) {
+#pragma unroll
+        for (int i = 0; i < RP; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) {
+                const lh_f32x4 v = acc[h * RP + i][j];
+                box[piece<16 * TJ>(i * 16 + (lane & 15), g * TJ + j)] = make_float4(v[0], v[1], v[2], v[3]);
+            }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const uint32_t b = rt.begin + row0 + h * RP * 16;
+        if (b < rt.end) store_tile<RP * 16, 16 * TJ>(a, box, RowTile{b, min(b + RP * 16, rt.end), rt.expert}, nw, pos0, lane);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+}
+
+// Rows of W in the order in which the lanes 0 .. 15 of tile j take them, and the chunk permutation under which eight neighbouring
+// lanes read different banks.
+template <int TJ> __device__ __forceinline__ uint32_t dealt_row(uint32_t lane, uint32_t j) { return ((lane & 15) >> 2) * 4 * TJ + j * 4 + (lane & 3); }
+template <int TJ> __device__ __forceinline__ uint32_t dealt_swizzle(uint32_t row) { return (row & 3) | (row / (4 * TJ) & 1) << 2; }
 
 // ---- matrix cores ------------------------------------------------------------------------------------------------------
 // 256 threads, 2 x 2 waves of BM/2 x BN/2 outputs.  A k step is 64 wide: a tile row is eight 16-byte chunks, chunk c of row r
 // kept at place c ^ (r & 7) of its row so that the fragment reads of sixteen rows fall on different banks (the loads
 // write LDS in order, so the permutation is applied to their global addresses).  NS buffers, one barrier per step: step kt is
 // multiplied while the loads of the NS - 1 steps after it are on their way.
-// The weights are the MFMA's row operand: lane = output row (lane & 15), four consecutive output columns per tile.
+// The weights are the MFMA's row operand: lane = output row (lane & 15), four output columns per tile.
 template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
 
-template <int BM, int BN, int NS>
+template <int BM, int BN, int NS, int EPI>
 __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
     constexpr int TI = BM / 32, TJ = BN / 32, CA = BM / 32, CB = BN / 32;
     static_assert(NS * (BM + BN) * 128 >= BM * BN * 4, "the output tile must fit the staging buffers");
@@ -155,14 +343,15 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
 
     const uint16_t* pa[CA];
     const uint16_t* pb[CB];
-    const uint32_t src = (tid & 7) ^ ((tid >> 3) & 7);        // the chunk this thread brings in, of every row it serves
+    // the chunk this thread brings in, of every row it serves
+    const uint32_t src = (tid & 7) ^ ((tid >> 3) & 7), src_b = (tid & 7) ^ dealt_swizzle<TJ>(tid >> 3);
 #pragma unroll
     for (int i = 0; i < CA; i++) {
         const uint32_t r = min(rt.begin + i * 32 + (tid >> 3), rt.end - 1);
         pa[i] = A + (size_t)a_row(a, r) * a.lda + src * 8;
     }
 #pragma unroll
-    for (int i = 0; i < CB; i++) pb[i] = W + (size_t)min(n0 + i * 32 + (tid >> 3), a.N - 1) * K + src * 8;
+    for (int i = 0; i < CB; i++) pb[i] = W + (size_t)min(n0 + i * 32 + (tid >> 3), a.N - 1) * K + src_b * 8;
 
     auto load_step = [&](int buf, uint32_t kt) {
         uint4* base = &sm[buf][wave * 64];
@@ -172,11 +361,11 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
 #pragma unroll
             for (int i = 0; i < CB; i++) load_lds16(pb[i] + kt * 64, base + (CA + i) * 256);
         } else {                                             // the last step of a ragged K: chunks past it read zeros
-            const bool past = kt * 64 + src * 8 >= K;
+            const bool past = kt * 64 + src * 8 >= K, past_b = kt * 64 + src_b * 8 >= K;
 #pragma unroll
             for (int i = 0; i < CA; i++) load_lds16(past ? (const void*)&g_zero16 : (const void*)(pa[i] + kt * 64), base + i * 256);
 #pragma unroll
-            for (int i = 0; i < CB; i++) load_lds16(past ? (const void*)&g_zero16 : (const void*)(pb[i] + kt * 64), base + (CA + i) * 256);
+            for (int i = 0; i < CB; i++) load_lds16(past_b ? (const void*)&g_zero16 : (const void*)(pb[i] + kt * 64), base + (CA + i) * 256);
         }
     };
 
@@ -208,8 +397,8 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
             }
 #pragma unroll
             for (int j = 0; j < TJ; j++) {
-                const uint32_t r = wn * (BN / 2) + j * 16 + (lane & 15);
-                fb[j] = __builtin_bit_cast(lh_bf16x8, bs[r * 8 + (c ^ (r & 7))]);
+                const uint32_t r = wn * (BN / 2) + dealt_row<TJ>(lane, j);
+                fb[j] = __builtin_bit_cast(lh_bf16x8, bs[r * 8 + (c ^ (lane & 7))]);
             }
 #pragma unroll
             for (int i = 0; i < TI; i++)
@@ -218,30 +407,177 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
         }
     }
 
-    // The tile goes through LDS, so that a wave stores whole stretches of a row (and the store code exists once): four columns
-    // of row m are the 16-byte piece n / 4, kept at place (n / 4) ^ (m & 7).
     __syncthreads();
-    float4* tile = reinterpret_cast<float4*>(&sm[0][0]);
+    finish_tile<EPI, TI, TJ>(a, acc, rt, wm * (BM / 2), n0 + wn * (BN / 2), lane, reinterpret_cast<float4*>(&sm[0][0]) + wave * (BM * BN / 16));
+}
+
+// Large products, K a multiple of 64.  Eight waves in two groups of four, one wave of either group on each SIMD, half a period
+// apart: while one group multiplies, the other fetches its next fragments from LDS and requests tiles, so that the matrix cores of
+// a SIMD always have one wave's work (2140 cycles per step of 64 on a 256 x 256 tile, of which 2048 are matrix-core cycles; with all
+// waves in the same phase: 3100).  A phase ends in a barrier that all waves pass; a wave waits for its own requests, counted, before
+// the barrier behind which they are read.  Tiles per step and buffers:
+//   256 x 256  waves of 128 x 64, two buffers of 64 KB, refilled in two parts as soon as both groups have read a part
+//   256 x 128  waves of 64 x 64, three buffers of 48 KB
+//   128 x 128  waves of 64 x 64; the groups take the even and the odd steps, five buffers of 32 KB (with four, requests were half a
+//              period later: 81 us instead of 74 at 2048 x 8192 x 2048 with weights from HBM), and their sums meet at the end
+// Rows and chunks as in linear_mfma_kernel.
+__device__ __forceinline__ void phase_end() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+// The fragments asked for in this phase are here, and all but the last N requested pieces.
+template <int N> __device__ __forceinline__ void read_end() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int BM, int BN, int EPI>
+__global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
+    constexpr bool kWide = BN == 256, kHalves = BM == 128;               // (256 x 128 is neither)
+    constexpr int TI = kWide ? 8 : 4, SLOT = (BM + BN) * 8;              // 16-row tiles of a wave; 16-byte pieces of a buffer
+    constexpr int T = kHalves ? 256 : 512, CA = BM * 8 / T, CB = BN * 8 / T;
+    extern __shared__ uint4 sm[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = wave >> 2;
+    const uint32_t wm = kWide ? group : kHalves ? (wave >> 1) & 1 : wave >> 1, wn = kWide ? wave & 3 : wave & 1;
+    const uint32_t mt_n = a.ex.tiles ? a.ex.n_tiles : (a.M + BM - 1) / BM, nt_n = (a.N + BN - 1) / BN;
+    uint32_t mt, nt;
+    tile_of_block(mt_n, nt_n, mt, nt);
+    const RowTile rt = row_tile(a, mt, BM);
+    if (rt.begin >= rt.end) return;
+    const uint32_t n0 = nt * BN, K = a.K, nk = K / 64;
+    const char* A = static_cast<const char*>(a.A);
+    const char* W = reinterpret_cast<const char*>(a.W + (size_t)rt.expert * a.N * K);
+
+    const uint32_t lt = kHalves ? tid & 255 : tid, src = ((lt & 7) ^ ((lt >> 3) & 7)) * 16, src_b = ((lt & 7) ^ dealt_swizzle<4>(lt >> 3)) * 16;
+    uint32_t pa[CA], pb[CB];                                   // byte offsets: the host has checked that they fit
+#pragma unroll
+    for (int i = 0; i < CA; i++) pa[i] = a_row(a, min(rt.begin + i * (T / 8) + (lt >> 3), rt.end - 1)) * a.lda * 2 + src;
+#pragma unroll
+    for (int i = 0; i < CB; i++) pb[i] = min(n0 + i * (T / 8) + (lt >> 3), a.N - 1) * K * 2 + src_b;
+    uint4* const to = sm + (kHalves ? wave & 3 : wave) * 64;
+    auto load_a = [&](uint32_t buf, uint32_t kt, int i) { load_lds16(A + kt * 128 + pa[i], to + buf * SLOT + i * T); };
+    auto load_b = [&](uint32_t buf, uint32_t kt, int i) { load_lds16(W + kt * 128 + pb[i], to + buf * SLOT + BM * 8 + i * T); };
+    auto load_step = [&](uint32_t buf, uint32_t kt) {
+#pragma unroll
+        for (int i = 0; i < CA; i++) load_a(buf, kt, i);
+#pragma unroll
+        for (int i = 0; i < CB; i++) load_b(buf, kt, i);
+    };
+
+    lh_f32x4 acc[TI][4];
 #pragma unroll
     for (int i = 0; i < TI; i++)
 #pragma unroll
-        for (int j = 0; j < TJ; j++) {
-            const uint32_t m = wm * (BM / 2) + i * 16 + (lane & 15), c = (wn * (BN / 2) + j * 16) / 4 + (lane >> 4);
-            tile[m * (BN / 4) + (c ^ (m & 7))] = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+        for (int j = 0; j < 4; j++) acc[i][j] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
+    const uint32_t g = lane >> 4, at[2] = {g ^ (lane & 7), (g + 4) ^ (lane & 7)};
+    const uint4 *ra = sm + (wm * TI * 16 + (lane & 15)) * 8, *rb = sm + (BM + wn * 64 + dealt_row<4>(lane, 0)) * 8;
+    lh_bf16x8 fa[2][4], fb[2][4];
+    auto read_a = [&](uint32_t buf, int h) {
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) fa[s][i] = __builtin_bit_cast(lh_bf16x8, ra[buf * SLOT + (h * 4 + i) * 128 + at[s]]);
+    };
+    auto read_b = [&](uint32_t buf) {
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) fb[s][j] = __builtin_bit_cast(lh_bf16x8, rb[buf * SLOT + j * 32 + at[s]]);
+    };
+    auto multiply = [&](int h) {                              // 64 x 64 outputs over 64 columns of k, the wave ahead of the one that reads
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[h * 4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[s][j], fa[s][i], acc[h * 4 + i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+    };
+
+    if constexpr (kWide) {
+        // Part one of a buffer: B and the rows that the waves multiply first (0 .. 63 of either half); part two: the other rows.
+        auto part1 = [&](uint32_t kt) { for (int i = 0; i < 4; i++) load_b(kt & 1, kt, i); load_a(kt & 1, kt, 0); load_a(kt & 1, kt, 2); };
+        auto part2 = [&](uint32_t kt) { load_a(kt & 1, kt, 1); load_a(kt & 1, kt, 3); };
+        part1(0); part2(0);
+        if (nk > 1) { part1(1); read_end<8>(); } else read_end<2>();
+        if (group) phase_end();
+        uint32_t kt = 0;
+        for (; kt + 2 < nk; kt++) {
+            read_b(kt & 1); read_a(kt & 1, 0); part2(kt + 1); read_end<8>();
+            multiply(0); phase_end();
+            read_a(kt & 1, 1); part1(kt + 2); read_end<8>();
+            multiply(1); phase_end();
         }
-    __syncthreads();
-    const uint32_t pos0 = a.seg.position ? *a.seg.position : 0u;
-    const uint32_t s = lh_segment_of(a.seg, n0);
-    if (a.seg.layout[s] == LH_BLOCKS_AT_POSITION && !a.seg.f32[s] && s == lh_segment_of(a.seg, min(n0 + BN, a.N) - 1) && a.ex.tiles == nullptr) {
-        store_blocks<BM, BN>(a, s, reinterpret_cast<const float*>(tile), rt, n0, pos0);
-        return;
+        if (kt + 1 < nk) {
+            read_b(kt & 1); read_a(kt & 1, 0); part2(kt + 1); read_end<8>();
+            multiply(0); phase_end();
+            read_a(kt & 1, 1); read_end<2>();
+            multiply(1); phase_end();
+            kt++;
+        }
+        read_b(kt & 1); read_a(kt & 1, 0); read_end<0>();
+        multiply(0); phase_end();
+        read_a(kt & 1, 1); read_end<0>();
+        multiply(1); phase_end();
+    } else if constexpr (kHalves) {
+        // A group's steps are kt = group, group + 2, ...  Step kt is in buffer kt mod 5; while a group reads step kt it requests its step
+        // kt + 4: step kt - 1, which was there, has been read by the other group.
+        const uint32_t mine = (nk + 1 - group) / 2, most = (nk + 1) / 2;
+        if (mine > 0) load_step(group, group);
+        if (mine > 1) { load_step(group + 2, group + 2); wait_loads<8>(); } else wait_loads<0>();
+        phase_end();
+        if (group) phase_end();
+        uint32_t kt = group, buf = group;
+        for (uint32_t i = 0; i < most; i++) {
+            if (i + 2 < mine) load_step(buf == 0 ? 4 : buf - 1, kt + 4);
+            if (i < mine) { read_a(buf, 0); read_b(buf); }
+            read_end<63>();
+            if (i < mine) multiply(0);
+            if (i + 2 < mine) wait_loads<8>(); else wait_loads<0>();
+            phase_end();
+            kt += 2;
+            buf = buf >= 3 ? buf - 3 : buf + 2;
+        }
+    } else {
+        // Step kt is in buffer kt mod 3; a wave requests step kt + 2 while it reads step kt: step kt - 1, which was there, has been
+        // read by both groups.
+        load_step(0, 0);
+        if (nk > 1) { load_step(1, 1); read_end<6>(); } else read_end<0>();
+        if (group) phase_end();
+        uint32_t buf = 0, kt = 0;
+        for (; kt + 2 < nk; kt++) {
+            read_a(buf, 0); read_b(buf); load_step(buf == 0 ? 2 : buf - 1, kt + 2);
+            buf = buf == 2 ? 0 : buf + 1;
+            read_end<6>();
+            multiply(0); phase_end();
+        }
+        for (; kt < nk; kt++) {
+            read_a(buf, 0); read_b(buf);
+            buf = buf == 2 ? 0 : buf + 1;
+            read_end<0>();
+            multiply(0); phase_end();
+        }
     }
-#pragma unroll 1
-    for (uint32_t e = tid; e < BM * BN / 4; e += 256) {
-        const uint32_t m = e / (BN / 4), c = e % (BN / 4), n = n0 + c * 4, slot = rt.begin + m;
-        if (slot >= rt.end || n >= a.N) continue;
-        store4(a, slot, n, tile[m * (BN / 4) + (c ^ (m & 7))], pos0);
+    if (!group) phase_end();
+
+    uint32_t row0 = wm * TI * 16;
+    if constexpr (kHalves) {                                  // group 0 finishes the upper 32 rows of a wave's tile, group 1 the lower
+        lh_f32x4* const box = reinterpret_cast<lh_f32x4*>(sm) + (wave & 3) * 512 + lane;
+#pragma unroll
+        for (int e = 0; e < 8; e++) box[group * 2048 + e * 64] = group ? acc[e >> 2][e & 3] : acc[2 + (e >> 2)][e & 3];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const lh_f32x4 other = box[(group ^ 1) * 2048 + e * 64];
+            acc[e >> 2][e & 3] = group ? other + acc[2 + (e >> 2)][e & 3] : acc[e >> 2][e & 3] + other;
+        }
+        row0 += group * 32;
+        __syncthreads();
     }
+    finish_tile<EPI, kHalves ? 2 : TI, 4>(a, acc, rt, row0, n0 + wn * 64, lane, reinterpret_cast<float4*>(sm) + wave * 1024);
 }
 
 // ---- f32 FMA -----------------------------------------------------------------------------------------------------------
@@ -619,6 +955,57 @@ int vector_entry(lh_batch* batch, const char* op, int stage, const VectorStage& 
 
 uint32_t lh_expert_tile_rows(uint32_t slots, uint32_t experts) { return slots / (experts ? experts : 1) >= 128 ? 128u : 64u; }
 
+// Whether a lane can finish `per_lane` neighbouring columns by itself, and which activations it then meets.
+static int epilogue_of(const LhSegments& seg, uint32_t per_lane) {
+    bool none = true, gelu = true, silu = true, pairs = true, relu = true;
+    for (uint32_t s = 0; s < seg.count; s++) {
+        const uint32_t act = seg.act[s], size = seg.f32[s] ? 4 : 2;
+        if (seg.n0[s] % per_lane || seg.n0[s + 1] % per_lane || (act != LH_ACT_NONE && seg.f32[s])) return kThroughLds;
+        if (seg.head[s] != seg.padded[s] && seg.head[s] % per_lane) return kThroughLds;
+        if (((uintptr_t)seg.out[s] | (uintptr_t)seg.ld[s] * size | (uintptr_t)seg.padded[s] * size) & 15) return kThroughLds;
+        none = none && act == LH_ACT_NONE;
+        gelu = gelu && act == LH_ACT_GELU_TANH;
+        silu = silu && (act == LH_ACT_NONE || act == LH_ACT_SILU);
+        relu = relu && (act == LH_ACT_NONE || act == LH_ACT_RELU_SQUARED);
+        pairs = pairs && act == LH_ACT_SILU_PAIRS;
+    }
+    if (seg.accumulate && !none) return kThroughLds;
+    return none ? kNoActivation : gelu ? kGelu : silu ? kSilu : relu ? kReluSquared : pairs ? kSiluPairs : kThroughLds;
+}
+
+template <class Launch>
+static void with_epilogue(int epilogue, Launch launch) {
+    switch (epilogue) {
+        case kNoActivation: launch(std::integral_constant<int, kNoActivation>()); break;
+        case kGelu: launch(std::integral_constant<int, kGelu>()); break;
+        case kSilu: launch(std::integral_constant<int, kSilu>()); break;
+        case kSiluPairs: launch(std::integral_constant<int, kSiluPairs>()); break;
+        case kReluSquared: launch(std::integral_constant<int, kReluSquared>()); break;
+        default: launch(std::integral_constant<int, kThroughLds>());
+    }
+}
+template <int BM, int BN, int NS>
+static int launch_mfma(lh_context* ctx, const LhLinear& a, uint64_t grid, const char* op) {
+    LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: %u x %u outputs", op, a.M, a.N);
+    if (grid == 0) return LH_OK;
+    with_epilogue(epilogue_of(a.seg, BN / 8), [&](auto epi) {
+        hipLaunchKernelGGL((linear_mfma_kernel<BM, BN, NS, decltype(epi)::value>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a);
+    });
+    return lh_check_launch(op);
+}
+template <int BM, int BN>
+static int launch_phased(lh_context* ctx, const LhLinear& a, uint64_t grid, const char* op) {
+    LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: %u x %u outputs", op, a.M, a.N);
+    if (grid == 0) return LH_OK;
+    constexpr size_t lds = (BN == 256 ? 2 : BM == 256 ? 3 : 5) * (BM + BN) * 128;
+    int r = LH_OK;
+    with_epilogue(epilogue_of(a.seg, 16), [&](auto epi) {
+        r = lh_raise_dynamic_lds(ctx, (const void*)linear_phased_kernel<BM, BN, decltype(epi)::value>, lds, op);
+        if (r == LH_OK) hipLaunchKernelGGL((linear_phased_kernel<BM, BN, decltype(epi)::value>), dim3((uint32_t)grid), dim3(512), lds, ctx->stream, a);
+    });
+    return r == LH_OK ? lh_check_launch(op) : r;
+}
+
 int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     LhLinear a = given;
     if (a.lda == 0) a.lda = a.K;
@@ -631,23 +1018,33 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
         else hipLaunchKernelGGL((linear_plain_kernel<uint16_t>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a);
         return lh_check_launch(op);
     }
+    const uint64_t want = (uint64_t)ctx->cu_count, steps = a.K / 64;
     auto tiles = [&](uint32_t bm, uint32_t bn) { return (uint64_t)(a.ex.tiles ? a.ex.n_tiles : (a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
-#define LH_GEMM(BM_, BN_, NS_)                                                                                             \
-    do {                                                                                                                \
-        const uint64_t grid = tiles(BM_, BN_);                                                                          \
-        LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: %u x %u outputs", op, a.M, a.N);                                          \
-        if (grid) hipLaunchKernelGGL((linear_mfma_kernel<BM_, BN_, NS_>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a); \
-    } while (0)
-    const uint64_t want = (uint64_t)ctx->cu_count;
+    // Byte offsets of the phased kernels are 32 bits wide.
+    const uint64_t a_bytes = (uint64_t)(a.ex.tiles ? (a.ex.gather ? a.ex.rows : a.ex.slots) : a.M) * a.lda * 2, w_bytes = (uint64_t)a.N * a.K * 2;
+    const bool phased = a.K % 64 == 0 && a_bytes < (1ull << 32) && w_bytes < (1ull << 32);
     if (a.ex.tiles) {
-        if (a.ex.tile_rows == 128) { if (tiles(128, 128) >= want) LH_GEMM(128, 128, 2); else LH_GEMM(128, 64, 3); }
-        else LH_GEMM(64, 64, 4);
-    } else if (tiles(128, 128) >= 2 * want) LH_GEMM(128, 128, 2);
-    else if (tiles(128, 64) >= want) LH_GEMM(128, 64, 3);
-    else if (tiles(64, 64) >= want || a.M > 32) LH_GEMM(64, 64, 4);
-    else LH_GEMM(32, 32, 4);
-#undef LH_GEMM
-    return lh_check_launch(op);
+        if (a.ex.tile_rows != 128) return launch_mfma<64, 64, 4>(ctx, a, tiles(64, 64), op);
+        if (tiles(128, 128) >= want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
+        return launch_mfma<128, 64, 3>(ctx, a, tiles(128, 64), op);
+    }
+    if (phased && 4 * tiles(128, 128) >= 3 * want) {
+        // One workgroup fits a CU, so a launch takes whole rounds of them, and the form is the one whose rounds are the shortest.  A
+        // round's time in nanoseconds, measured with 64 columns of k per step: 256 x 256 9000 + 1650 per step, 256 x 128 8000 + 800,
+        // 128 x 128 7000 + 520.  Before / now, bf16 results: 2048 x 2048 x 8192 85 / 60 us (256 x 256; the matrix cores alone would take
+        // 28 at 2.4 GHz, but with all CUs at it the clock falls to 1.3 GHz), 2048 x 2048 x 4096 39 / 34 and 2048 x 2048 x 3072 35 / 28
+        // (256 x 128), 2048 x 8192 x 2048 90 / 74 (128 x 128).  With fewer than three tiles of 128 x 128 to four CUs the small tiles
+        // win: 128 of them (953 x 2048 x 2048) 22 us against 17.
+        auto rounds = [&](uint32_t bm, uint32_t bn) { return (tiles(bm, bn) + want - 1) / want; };
+        const uint64_t t256 = rounds(256, 256) * (9000 + 1650 * steps), t384 = rounds(256, 128) * (8000 + 800 * steps), t128 = rounds(128, 128) * (7000 + 520 * steps);
+        if (t256 <= t384 && t256 <= t128) return launch_phased<256, 256>(ctx, a, tiles(256, 256), op);
+        if (t384 <= t128) return launch_phased<256, 128>(ctx, a, tiles(256, 128), op);
+        return launch_phased<128, 128>(ctx, a, tiles(128, 128), op);
+    }
+    if (tiles(128, 128) >= 2 * want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
+    if (tiles(128, 64) >= want) return launch_mfma<128, 64, 3>(ctx, a, tiles(128, 64), op);
+    if (tiles(64, 64) >= want || a.M > 32) return launch_mfma<64, 64, 4>(ctx, a, tiles(64, 64), op);
+    return launch_mfma<32, 32, 4>(ctx, a, tiles(32, 32), op);
 }
 
 extern "C" {

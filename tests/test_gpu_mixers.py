@@ -81,6 +81,63 @@ def test_linear_rows(ai, gpu, dtype, m, k, n):
         close(download(ai, v, n, ai.F32), ACTS[act](want)[0], F32_TOL, "vector")
 
 
+@pytest.mark.parametrize("m,k,n", [(2048, 64, 8192), (1990, 192, 8176), (1793, 128, 8150), (2048, 320, 3072), (1830, 64, 2064), (1500, 256, 3000), (2048, 192, 2048),
+                                   (1930, 64, 2000), (1921, 448, 1936), (2048, 576, 1920)])
+@pytest.mark.parametrize("act", [0, 1, 2, 3])
+def test_large_products(ai, gpu, m, k, n, act):
+    """The 256 x 256, 256 x 128 and 128 x 128 tiles of large products: whole and ragged, one step of k to nine, every way a lane
+    finishes its columns; bf16 and f32 outputs, with and without the residual."""
+    ctx, K = gpu
+    g = np.random.default_rng(m + k + n)
+    x, w, b = M.rounded(g.standard_normal((m, k))), M.rounded(g.standard_normal((n, k)) / np.sqrt(k)), g.standard_normal(n).astype(np.float32)
+    want = ACTS[act](x @ w.T + b)
+    L = ai.linear_weight
+    lin = L.StackedLinear(ctx, [M.bf16_bits(w)], [L.Segment(n, act)], [b])
+    xb, out, wide, res = upload(ai, ctx, x, ai.BF16), empty(ai, ctx, m * n, ai.BF16), empty(ai, ctx, m * n, ai.F32), upload(ai, ctx, np.ones((m, n)), ai.F32)
+    print(f"large product {m} {k} {n} {act}", flush=True)
+    batch = ai.CommandBatch(ctx)
+    lin.rows_into(batch, K, xb, ai.BF16, m, [out], ai.BF16)
+    lin.rows_into(batch, K, xb, ai.BF16, m, [wide], ai.F32)
+    lin.rows_add_into(batch, K, xb, ai.BF16, m, res)
+    batch.commit_and_wait()
+    got = download(ai, out, m * n, ai.BF16).reshape(m, n)
+    assert (np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + F32_TOL * np.abs(want).max()).all()      # one rounding to bf16
+    close(download(ai, wide, m * n, ai.F32).reshape(m, n), want, F32_TOL, "f32 output")
+    close(download(ai, res, m * n, ai.F32).reshape(m, n), want + 1, F32_TOL, "residual")
+
+
+@pytest.mark.parametrize("m,pos,k,heads,dim,pad,vdim", [(2048, 0, 64, 8, 128, 128, 128), (1500, 32, 128, 8, 96, 128, 160), (1500, 5, 64, 8, 96, 128, 160),
+                                                        (1100, 64, 64, 12, 80, 96, 144), (130, 32, 64, 2, 32, 32, 64), (300, 0, 128, 3, 40, 64, 96), (64, 96, 72, 2, 32, 32, 64)])
+def test_caches_of_many_rows(ai, gpu, m, pos, k, heads, dim, pad, vdim):
+    """Whole and partial blocks of 32 positions of the value cache, padded keys at a position and a gated pair layout from products of many rows."""
+    ctx, K = gpu
+    g, L, cap = np.random.default_rng(pos + m), ai.linear_weight, (pos + m + 40) // 32 * 32
+    ws = [M.rounded(g.standard_normal((heads * d, k)) / np.sqrt(k)) for d in (dim, dim, vdim)]
+    x = M.rounded(g.standard_normal((m, k)))
+    b = [g.standard_normal(w.shape[0]).astype(np.float32) for w in ws]
+    lin = L.StackedLinear(ctx, [M.bf16_bits(w) for w in ws], [L.Segment(heads * dim, ai.ACT_SILU, dim, pad), L.Segment(heads * dim, 0, dim, pad, ai.ROWS_AT_POSITION),
+                                                              L.Segment(heads * vdim, 0, vdim, vdim, ai.BLOCKS_AT_POSITION)], b)
+    q, kc, v = (empty(ai, ctx, c, ai.BF16) for c in (m * heads * pad, cap * heads * pad, cap * heads * vdim))
+    print(f"caches {m} {pos} {k}", flush=True)
+    batch = ai.CommandBatch(ctx)
+    lin.rows_into(batch, K, upload(ai, ctx, x, ai.BF16), ai.BF16, m, [q, kc, v], ai.BF16, ai.Buffer.from_slice(ctx, np.array([pos], np.uint32)))
+    pairs = L.StackedLinear(ctx, [M.bf16_bits(ws[0])], [L.Segment(heads * dim, ai.ACT_SILU_PAIRS)])
+    h = empty(ai, ctx, m * heads * dim // 2, ai.BF16)
+    pairs.rows_into(batch, K, upload(ai, ctx, x, ai.BF16), ai.BF16, m, [h], ai.BF16)
+    batch.commit_and_wait()
+    got = download(ai, q, m * heads * pad, ai.BF16).reshape(m, heads, pad)
+    close(got[:, :, :dim], O.silu(x @ ws[0].T + b[0]).reshape(m, heads, dim), BF16_TOL, "q")
+    assert not got[:, :, dim:].any()
+    got = download(ai, kc, cap * heads * pad, ai.BF16).reshape(cap, heads, pad)
+    close(got[pos:pos + m, :, :dim], (x @ ws[1].T + b[1]).reshape(m, heads, dim), BF16_TOL, "k")
+    assert not got[:pos].any() and not got[pos + m:].any() and not got[:, :, dim:].any()
+    got = values_from_cache(download(ai, v, cap * heads * vdim, ai.BF16), heads * vdim)
+    close(got[pos:pos + m], x @ ws[2].T + b[2], BF16_TOL, "v")
+    assert not got[:pos].any() and not got[pos + m:].any()
+    z = (x @ ws[0].T).reshape(m, -1, 2)
+    close(download(ai, h, m * heads * dim // 2, ai.BF16).reshape(m, -1), O.silu(z[:, :, 0]) * z[:, :, 1], BF16_TOL, "pairs")
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("m,pos,width,heads,dim,pad,vdim,vpad", [(5, 30, 64, 3, 20, 32, 12, 32), (1, 31, 64, 3, 20, 32, 12, 32), (70, 1, 40, 2, 32, 32, 64, 64),
                                                                  (1, 32, 520, 1, 5, 32, 33, 64), (33, 63, 36, 2, 24, 32, 40, 64), (40, 100, 64, 2, 16, 32, 32, 32)])
