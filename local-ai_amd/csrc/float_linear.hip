@@ -1,7 +1,8 @@
 // Products of activations with bf16 weights [N, K]:
 //   linear_phased_kernel bf16 activations, K a multiple of 64, enough tiles of 128 x 128 for the chip: eight waves in two phases
 //   linear_mfma_kernel   bf16 activations, K a multiple of 8: LDS-tiled bf16 MFMA 16x16x32, tiles loaded straight into LDS
-//   linear_plain_kernel  everything else: f32 FMA on 64 x 64 tiles (the 32-bit runs, ragged K)
+//   split_rows_kernel    f32 activations as three bf16 terms, for the two kernels above (the 32-bit runs)
+//   linear_plain_kernel  everything else: f32 FMA on 64 x 64 tiles (ragged K, pieces that are not aligned)
 //   matvec_bf16_kernel   one row, HBM-bound weight streaming, with the norm before the product done while x is staged
 // All end in the same column segments (bias, activation, layout, residual add), and linear_mfma_kernel and linear_plain_kernel also
 // run the experts of a mixture on the tiles of a routing plan.
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
     tile_of_block(mt_n, nt_n, mt, nt);
     const RowTile rt = row_tile(a, mt, BM);
     if (rt.begin >= rt.end) return;
-    const uint32_t n0 = nt * BN, K = a.K, nk = (K + 63) / 64;
+    const uint32_t n0 = nt * BN, K = a.K, steps = (K + 63) / 64, nk = steps * a.parts;
     const uint16_t* A = static_cast<const uint16_t*>(a.A);
     const uint16_t* W = a.W + (size_t)rt.expert * a.N * K;
 
@@ -353,17 +354,19 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
 #pragma unroll
     for (int i = 0; i < CB; i++) pb[i] = W + (size_t)min(n0 + i * 32 + (tid >> 3), a.N - 1) * K + src_b * 8;
 
-    auto load_step = [&](int buf, uint32_t kt) {
+    auto load_step = [&](int buf, uint32_t step) {
         uint4* base = &sm[buf][wave * 64];
+        const uint32_t part = (step >= steps) + (step >= 2 * steps), kt = step - part * steps;
+        const size_t ka = (size_t)part * a.part_stride + kt * 64;
         if (kt * 64 + 64 <= K) {
 #pragma unroll
-            for (int i = 0; i < CA; i++) load_lds16(pa[i] + kt * 64, base + i * 256);
+            for (int i = 0; i < CA; i++) load_lds16(pa[i] + ka, base + i * 256);
 #pragma unroll
             for (int i = 0; i < CB; i++) load_lds16(pb[i] + kt * 64, base + (CA + i) * 256);
         } else {                                             // the last step of a ragged K: chunks past it read zeros
             const bool past = kt * 64 + src * 8 >= K, past_b = kt * 64 + src_b * 8 >= K;
 #pragma unroll
-            for (int i = 0; i < CA; i++) load_lds16(past ? (const void*)&g_zero16 : (const void*)(pa[i] + kt * 64), base + i * 256);
+            for (int i = 0; i < CA; i++) load_lds16(past ? (const void*)&g_zero16 : (const void*)(pa[i] + ka), base + i * 256);
 #pragma unroll
             for (int i = 0; i < CB; i++) load_lds16(past_b ? (const void*)&g_zero16 : (const void*)(pb[i] + kt * 64), base + (CA + i) * 256);
         }
@@ -446,7 +449,7 @@ __global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
     tile_of_block(mt_n, nt_n, mt, nt);
     const RowTile rt = row_tile(a, mt, BM);
     if (rt.begin >= rt.end) return;
-    const uint32_t n0 = nt * BN, K = a.K, nk = K / 64;
+    const uint32_t n0 = nt * BN, K = a.K, steps = K / 64, nk = steps * a.parts;
     const char* A = static_cast<const char*>(a.A);
     const char* W = reinterpret_cast<const char*>(a.W + (size_t)rt.expert * a.N * K);
 
@@ -457,8 +460,12 @@ __global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
 #pragma unroll
     for (int i = 0; i < CB; i++) pb[i] = min(n0 + i * (T / 8) + (lt >> 3), a.N - 1) * K * 2 + src_b;
     uint4* const to = sm + (kHalves ? wave & 3 : wave) * 64;
-    auto load_a = [&](uint32_t buf, uint32_t kt, int i) { load_lds16(A + kt * 128 + pa[i], to + buf * SLOT + i * T); };
-    auto load_b = [&](uint32_t buf, uint32_t kt, int i) { load_lds16(W + kt * 128 + pb[i], to + buf * SLOT + BM * 8 + i * T); };
+    auto part_of = [&](uint32_t kt) { return (uint32_t)(kt >= steps) + (kt >= 2 * steps); };
+    auto load_a = [&](uint32_t buf, uint32_t kt, int i) {
+        const uint32_t part = part_of(kt);
+        load_lds16(A + (size_t)part * a.part_stride * 2 + (kt - part * steps) * 128 + pa[i], to + buf * SLOT + i * T);
+    };
+    auto load_b = [&](uint32_t buf, uint32_t kt, int i) { load_lds16(W + (kt - part_of(kt) * steps) * 128 + pb[i], to + buf * SLOT + BM * 8 + i * T); };
     auto load_step = [&](uint32_t buf, uint32_t kt) {
 #pragma unroll
         for (int i = 0; i < CA; i++) load_a(buf, kt, i);
@@ -578,6 +585,41 @@ __global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
         __syncthreads();
     }
     finish_tile<EPI, kHalves ? 2 : TI, 4>(a, acc, rt, row0, n0 + wn * 64, lane, reinterpret_cast<float4*>(sm) + wave * 1024);
+}
+
+// ---- f32 rows as bf16 terms ----------------------------------------------------------------------------------------------
+// An f32 value is the sum of three bf16 values that are cut off, not rounded, so that all have its sign: 8 bits each, 24 in all.  The
+// products with bf16 weights are then exact and summed in f32, as FMA has them, on the matrix cores; a row becomes its lowest terms,
+// its middle terms and its leading terms, one after the other.  A term that is zero of a value that is not becomes a tiny one of
+// its sign, far below what f32 sums see: an infinite weight then gives the infinity that it gives times the value itself.
+// (333 x 1024 x 4096: 185 us on the FMA units, 17 us for both launches.)
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, uint16_t* __restrict__ out, uint32_t rows, uint32_t K, uint32_t lda, uint32_t stride) {
+    const uint32_t per = stride / 4, row = blockIdx.y * 4 + threadIdx.x / 64;
+    if (row >= rows) return;
+    for (uint32_t c = blockIdx.x * 64 + (threadIdx.x & 63); c < per; c += gridDim.x * 64) {
+        const uint32_t k = c * 4;
+        const float4 v = k < K ? *reinterpret_cast<const float4*>(x + (size_t)row * lda + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float f[4] = {v.x, v.y, v.z, v.w};
+        uint32_t t[3][4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t u = __builtin_bit_cast(uint32_t, f[j]);
+            if ((u & 0x7F800000u) == 0x7F800000u) {           // infinite, or no number (which stays none when it is cut off)
+                t[0][j] = t[1][j] = t[2][j] = (u >> 16) | ((u & 0x007FFFFFu) ? 0x40u : 0u);
+                continue;
+            }
+            const float hi = __builtin_bit_cast(float, u & 0xFFFF0000u), r = f[j] - hi;
+            const uint32_t ru = __builtin_bit_cast(uint32_t, r), tiny = __builtin_bit_cast(uint32_t, f[j] * 0x1p-100f) >> 16;
+            const float mid = __builtin_bit_cast(float, ru & 0xFFFF0000u);
+            const uint32_t lo = __builtin_bit_cast(uint32_t, r - mid) >> 16;
+            t[0][j] = (lo & 0x7FFFu) ? lo : tiny;
+            t[1][j] = (ru & 0x7FFF0000u) ? ru >> 16 : tiny;
+            t[2][j] = u >> 16;
+        }
+        uint16_t* o = out + (size_t)row * 3 * stride + k;
+#pragma unroll
+        for (int z = 0; z < 3; z++) *reinterpret_cast<uint2*>(o + (size_t)z * stride) = make_uint2(t[z][0] | t[z][1] << 16, t[z][2] | t[z][3] << 16);
+    }
 }
 
 // ---- f32 FMA -----------------------------------------------------------------------------------------------------------
@@ -1009,6 +1051,17 @@ static int launch_phased(lh_context* ctx, const LhLinear& a, uint64_t grid, cons
 int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     LhLinear a = given;
     if (a.lda == 0) a.lda = a.K;
+    a.parts = 1; a.part_stride = 0;
+    const uint32_t a_rows = a.ex.tiles ? (a.ex.gather ? a.ex.rows : a.ex.slots) : a.M, stride = (a.K + 63) / 64 * 64;
+    if (a.a_f32 && a.K % 8 == 0 && a.lda % 4 == 0 && (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0 && (uint64_t)a_rows * stride * 6 <= ctx->workspace_bytes &&
+        a_rows <= 4 * 65535u) {
+        if (a_rows == 0) return LH_OK;
+        hipLaunchKernelGGL(split_rows_kernel, dim3((stride + 1023) / 1024, (a_rows + 3) / 4), dim3(256), 0, ctx->stream, static_cast<const float*>(a.A),
+                           static_cast<uint16_t*>(ctx->workspace), a_rows, a.K, a.lda, stride);
+        const int r = lh_check_launch(op);
+        if (r != LH_OK) return r;
+        a.A = ctx->workspace; a.a_f32 = 0; a.lda = 3 * stride; a.parts = 3; a.part_stride = stride;
+    }
     const bool mfma = !a.a_f32 && a.K % 8 == 0 && a.lda % 8 == 0 && (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0;
     if (!mfma) {
         const uint64_t mt = a.ex.tiles ? a.ex.n_tiles : ((uint64_t)a.M + 63) / 64, grid = mt * ((a.N + 63) / 64);
@@ -1018,10 +1071,10 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
         else hipLaunchKernelGGL((linear_plain_kernel<uint16_t>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a);
         return lh_check_launch(op);
     }
-    const uint64_t want = (uint64_t)ctx->cu_count, steps = a.K / 64;
+    const uint64_t want = (uint64_t)ctx->cu_count, steps = (uint64_t)a.K / 64 * a.parts;
     auto tiles = [&](uint32_t bm, uint32_t bn) { return (uint64_t)(a.ex.tiles ? a.ex.n_tiles : (a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
     // Byte offsets of the phased kernels are 32 bits wide.
-    const uint64_t a_bytes = (uint64_t)(a.ex.tiles ? (a.ex.gather ? a.ex.rows : a.ex.slots) : a.M) * a.lda * 2, w_bytes = (uint64_t)a.N * a.K * 2;
+    const uint64_t a_bytes = (uint64_t)a_rows * a.lda * 2, w_bytes = (uint64_t)a.N * a.K * 2;
     const bool phased = a.K % 64 == 0 && a_bytes < (1ull << 32) && w_bytes < (1ull << 32);
     if (a.ex.tiles) {
         if (a.ex.tile_rows != 128) return launch_mfma<64, 64, 4>(ctx, a, tiles(64, 64), op);

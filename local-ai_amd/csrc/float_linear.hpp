@@ -19,6 +19,7 @@ struct LhLinear {
     const uint16_t* W;              // [N, K] (of every expert, one after the other)
     const float* bias;
     uint32_t M, N, K, lda;
+    uint32_t parts, part_stride;    // bf16 rows that hold K columns `parts` times (0: once), part_stride elements apart: terms of f32 values
     LhSegments seg;
     LhExpertRows ex;
 };

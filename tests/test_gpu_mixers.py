@@ -106,6 +106,34 @@ def test_large_products(ai, gpu, m, k, n, act):
     close(download(ai, res, m * n, ai.F32).reshape(m, n), want + 1, F32_TOL, "residual")
 
 
+@pytest.mark.parametrize("m,k,n", [(40, 72, 50), (333, 1024, 256), (2048, 64, 2048), (3, 4096, 16)])
+def test_f32_rows_as_terms(ai, gpu, m, k, n):
+    """32-bit activations on the matrix cores: all 24 bits of every value, whatever its size, and what is infinite or no number comes
+    out as f32 products and sums have it."""
+    ctx, K = gpu
+    g, L = np.random.default_rng(m + k), ai.linear_weight
+    x, w = (g.standard_normal((m, k)) * 10.0 ** g.integers(-6, 7, (m, k))).astype(np.float32), M.rounded(g.standard_normal((n, k)) / np.sqrt(k))
+    x[0, 5], x[1, 0], x[2, 1:3] = np.inf, np.nan, (np.inf, -np.inf)
+    w[1, 5], w[2, 7], w[3, 5] = np.inf, -np.inf, 0.0
+    w[4, 3:5] = np.inf, np.nan
+    x[:, 7] = np.where(np.arange(m) % 3 == 0, 0.0, np.where(np.arange(m) % 3 == 1, 1.5, -2.0 ** -20))
+    xd = x.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(xd * r).sum(1) for r in w], 1)
+        size = np.abs(np.where(np.isfinite(xd), xd, 0.0)) @ np.abs(np.where(np.isfinite(w), w, 0.0)).T
+    out = empty(ai, ctx, m * n, ai.F32)
+    lin = L.StackedLinear(ctx, [M.bf16_bits(w)], [L.Segment(n)])
+    print(f"terms {m} {k} {n}", flush=True)
+    batch = ai.CommandBatch(ctx)
+    lin.rows_into(batch, K, upload(ai, ctx, x, ai.F32), ai.F32, m, [out], ai.F32)
+    batch.commit_and_wait()
+    got = download(ai, out, m * n, ai.F32).reshape(m, n)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fine = np.isfinite(want)
+    # a rounding for each 32 exact products of each of the three terms, and the product's own 32
+    assert (np.abs(got[fine] - want[fine]) <= ((3 * k / 32 + 32) * 2.0 ** -24 * size)[fine]).all()
+
+
 @pytest.mark.parametrize("m,pos,k,heads,dim,pad,vdim", [(2048, 0, 64, 8, 128, 128, 128), (1500, 32, 128, 8, 96, 128, 160), (1500, 5, 64, 8, 96, 128, 160),
                                                         (1100, 64, 64, 12, 80, 96, 144), (130, 32, 64, 2, 32, 32, 64), (300, 0, 128, 3, 40, 64, 96), (64, 96, 72, 2, 32, 32, 64)])
 def test_caches_of_many_rows(ai, gpu, m, pos, k, heads, dim, pad, vdim):
