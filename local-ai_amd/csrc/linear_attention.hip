@@ -4,7 +4,7 @@
 // kept as [head][value column][DQ key columns] (the key columns that exist, then zeros).
 //
 // Recurrent form: one workgroup per head and 16 value columns; a row of 16 lanes holds one value column's state in
-// registers (DQ / 16 values each) and walks the rows.
+// registers (DQ / 16 values each) and walks the rows.  From eight rows on the inputs come in several rows ahead.
 //
 // Chunked form (64 rows a chunk, bf16 inputs on the matrix cores, everything else f32):
 //   1. every chunk's own contribution to the state, U = sum over rows s of a^(L-1-s) k_s (x) v_s (all chunks at once)
@@ -78,6 +78,83 @@ __global__ __launch_bounds__(256) void recurrent_kernel(const RecurrentArgs a) {
     if (on) {
 #pragma unroll
         for (int i = 0; i < NR; i++) if (k0 + i < dq) st[i] = s[i];
+    }
+}
+
+// N neighbouring values, as they are stored.
+template <typename T, int N> struct Packed;
+template <int N> struct Packed<float, N> {
+    float v[N];
+    __device__ __forceinline__ void load(const float* p) {
+        if constexpr (N == 2) { const float2 x = *reinterpret_cast<const float2*>(p); v[0] = x.x; v[1] = x.y; }
+        else
+#pragma unroll
+            for (int i = 0; i < N; i += 4) { const float4 x = *reinterpret_cast<const float4*>(p + i); v[i] = x.x; v[i + 1] = x.y; v[i + 2] = x.z; v[i + 3] = x.w; }
+    }
+    __device__ __forceinline__ float get(int i) const { return v[i]; }
+};
+template <int N> struct Packed<uint16_t, N> {
+    uint32_t v[N / 2];
+    __device__ __forceinline__ void load(const uint16_t* p) {
+        if constexpr (N == 2) v[0] = *reinterpret_cast<const uint32_t*>(p);
+        else if constexpr (N == 4) { const uint2 x = *reinterpret_cast<const uint2*>(p); v[0] = x.x; v[1] = x.y; }
+        else
+#pragma unroll
+            for (int i = 0; i < N / 2; i += 4) { const uint4 x = *reinterpret_cast<const uint4*>(p + 2 * i); v[i] = x.x; v[i + 1] = x.y; v[i + 2] = x.z; v[i + 3] = x.w; }
+    }
+    __device__ __forceinline__ float get(int i) const { return __builtin_bit_cast(float, i & 1 ? v[i >> 1] & 0xFFFF0000u : v[i >> 1] << 16); }
+};
+
+// The same recurrence over many rows.  A step is a few dozen instructions behind its inputs, so the inputs of AHEAD rows are on their
+// way at any time, in whole pieces, and no load is conditional (one row ahead and a value at a time: 2 us a row; now 0.2).
+template <typename T, int NR, int AHEAD, bool SELECTIVE>
+__global__ __launch_bounds__(256) void recurrent_rows_kernel(const RecurrentArgs a) {
+    const uint32_t dim = a.dim, dq = a.dq, vdim = a.vdim, heads = a.heads, rows = a.rows;
+    const uint32_t vt = (vdim + 15) / 16, h = blockIdx.x / vt, col = (blockIdx.x % vt) * 16 + (threadIdx.x >> 4), part = threadIdx.x & 15;
+    const bool on = col < vdim, has = part * NR < dq;             // (dq is a multiple of NR: a lane has all of its values, or none)
+    const uint32_t c = on ? col : vdim - 1, k0 = has ? part * NR : 0u, in = !has ? 0u : k0 < dim ? min(dim - k0, (uint32_t)NR) : 0u;
+    const size_t step = (size_t)a.key_heads * dq, first = (size_t)(h / (heads / a.key_heads)) * dq + k0;
+    const T *q = static_cast<const T*>(a.q) + first, *k = static_cast<const T*>(a.k) + first, *v = static_cast<const T*>(a.v) + (size_t)h * vdim + c;
+    float* st = a.state + ((size_t)h * vdim + c) * dq + k0;
+    float s[NR];
+#pragma unroll
+    for (int i = 0; i < NR; i++) s[i] = has ? st[i] : 0.0f;
+    const float fixed = SELECTIVE ? 0.0f : a.decay[h], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
+                skip = SELECTIVE ? a.skip[h] : 0.0f;
+    struct Row { Packed<T, NR> k, q; T v; float z; } next[AHEAD];
+    auto fetch = [&](Row& r, uint32_t t) {
+        const size_t u = min(t, rows - 1);
+        r.k.load(k + u * step);
+        r.q.load(q + u * step);
+        r.v = v[u * heads * vdim];
+        if (SELECTIVE) r.z = a.dt_raw[u * heads + h];
+    };
+    auto walk = [&](const Row& r, uint32_t t) {
+        const float x = lh_ld(&r.v, 0), dt = SELECTIVE ? softplus(r.z + bias) : 1.0f, d = SELECTIVE ? expf(rate * dt) : fixed, vc = SELECTIVE ? dt * x : x;
+        float o = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            s[i] = __builtin_fmaf((uint32_t)i < in ? r.k.get(i) : 0.0f, vc, d * s[i]);
+            o = __builtin_fmaf(s[i], (uint32_t)i < in ? r.q.get(i) : 0.0f, o);
+        }
+        o = lh_group_sum(o, 16);
+        if (part == 0 && on) a.out[((size_t)t * heads + h) * vdim + col] = SELECTIVE ? __builtin_fmaf(skip, x, o) : o * a.scale;
+    };
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) fetch(next[j], j);
+    uint32_t t = 0;
+    for (; t + AHEAD <= rows; t += AHEAD) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) {
+            walk(next[j], t + j);
+            fetch(next[j], t + AHEAD + j);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) if (t + j < rows) walk(next[j], t + j);
+    if (on && has) {
+#pragma unroll
+        for (int i = 0; i < NR; i++) st[i] = s[i];
     }
 }
 
@@ -370,6 +447,17 @@ template <typename T, bool SELECTIVE>
 int launch_recurrent(lh_context* ctx, const RecurrentArgs& a, const char* op) {
     const uint64_t grid = (uint64_t)a.heads * ((a.vdim + 15) / 16);
     LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: heads %u, vdim %u", op, a.heads, a.vdim);
+    if (a.rows >= 8 && (((uintptr_t)a.q | (uintptr_t)a.k) & 15) == 0) {        // (a row's keys and queries start at multiples of 32 values)
+#define LH_REC(NR_, AHEAD_) hipLaunchKernelGGL((recurrent_rows_kernel<T, NR_, AHEAD_, SELECTIVE>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a)
+        if (a.dq <= 32) LH_REC(2, 8);
+        else if (a.dq <= 64) LH_REC(4, 8);
+        else if (a.dq <= 128) LH_REC(8, 8);
+        else if (a.dq <= 256) LH_REC(16, 4);
+        else if (a.dq <= 512) LH_REC(32, 2);
+        else LH_REC(64, 1);
+#undef LH_REC
+        return lh_check_launch(op);
+    }
 #define LH_REC(NR_) hipLaunchKernelGGL((recurrent_kernel<T, NR_, SELECTIVE>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a)
     if (a.dq <= 32) LH_REC(2);
     else if (a.dq <= 64) LH_REC(4);

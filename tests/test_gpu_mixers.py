@@ -355,6 +355,35 @@ def test_attention_rejects(ai, gpu):
 
 
 # ---- linear attention --------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("dim", [5, 32, 40, 64, 100, 128, 200, 300, 512, 700, 1024])
+@pytest.mark.parametrize("rows", [7, 8, 9, 17, 40])
+def test_recurrence_over_rows(ai, gpu, dtype, dim, rows):
+    """Around the number of rows whose inputs are on their way together, for every number of state values a lane holds."""
+    ctx, K = gpu
+    dt = ai.BF16 if dtype == "bf16" else ai.F32
+    g, H, vdim = np.random.default_rng(dim + rows), 2, 19
+    dq = K.linear_attention_padded_dim(dim)
+    q, k, v = (stored(g.standard_normal(s) / np.sqrt(dim), ai, dt) for s in ((rows, H, dim), (rows, H, dim), (rows, H, vdim)))
+    decay, S = np.array([0.5, 0.97], np.float32), g.standard_normal((H, dim, vdim)).astype(np.float32)
+    pad = np.full((rows, H, dq), 7.0)                  # what pads a row is not read
+    qp, kp = pad.copy(), pad.copy()
+    qp[..., :dim], kp[..., :dim] = q, k
+    state = np.zeros((H, vdim, dq), np.float32)
+    state[:, :, :dim] = S.transpose(0, 2, 1)
+    st, out = ai.Buffer.from_slice(ctx, state), empty(ai, ctx, rows * H * vdim, ai.F32)
+    print(f"recurrence {dtype} {dim} {rows}", flush=True)
+    batch = ai.CommandBatch(ctx)
+    K.linear_attention_recurrent_into(batch, upload(ai, ctx, qp, dt), upload(ai, ctx, kp, dt), upload(ai, ctx, v, dt), dt, st, ai.Buffer.from_slice(ctx, decay), out,
+                                      rows, H, dim, vdim, 0.5)
+    batch.commit_and_wait()
+    want, end = O.lightning_recurrence(q, k, v, decay.astype(np.float64), S.astype(np.float64))
+    close(download(ai, out, rows * H * vdim, ai.F32).reshape(rows, H, vdim), 0.5 * want, F32_TOL, "output")
+    got = st.as_array(np.float32, H * vdim * dq).reshape(H, vdim, dq)
+    close(got[:, :, :dim], end.transpose(0, 2, 1), F32_TOL, "state")
+    assert not got[:, :, dim:].any()
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(4, 32, 48), (3, 20, 33), (2, 64, 128), (1, 128, 80), (2, 200, 48), (2, 8, 100)])
 @pytest.mark.parametrize("cuts", [[1, 1, 1], [16, 2], [64], [17, 65, 130], [63, 1, 64], [300]])
 def test_linear_attention_forms(ai, gpu, heads, dim, vdim, cuts):
