@@ -14,6 +14,7 @@
 //   attention_tile_kernel   many rows: four waves share key and value blocks through LDS
 //   attention_split_kernel  few rows: every wave walks its own share of the blocks straight from global memory; the
 //                           workgroup's four partial results are merged in LDS, the workgroups' by attention_merge_kernel
+//   attention_wide_kernel   f32 caches: f32 matrix instructions, 16 packed rows a workgroup
 // Plain form (any dtype, any dim): attention_plain_kernel, one workgroup per query row and head.
 #include "softmax_attention.hpp"
 
@@ -359,6 +360,171 @@ int launch_dv(lh_context* ctx, AttentionArgs& a, uint32_t mp, const char* op, ui
     }
 }
 
+// f32 queries, keys and values on the f32 matrix instructions (16 x 16 x 4): products and sums are those of FMA.  A workgroup takes 16
+// packed rows of a kv head, its four waves the blocks of 32 keys in turn, straight from global memory; their results meet in LDS.
+// A matrix instruction takes one value of k per lane, and which one is free as long as both operands agree: over the dimensions of a
+// head lane group g has its g-th quarter of 16, over the keys of a tile its keys 4 g .. 4 g + 3, which is where S^T leaves the weights
+// and what a value block keeps side by side.  (attention_plain_kernel reads keys a value at a time, every thread its own row: 333 rows
+// of 8 heads with two maps over 64 dimensions, values of 128: 380 us; this form 35 us.)
+constexpr uint32_t kWideMaxDim = 256;      // of a key, per map
+template <int DV, int MAPS>
+__global__ __launch_bounds__(256) void attention_wide_kernel(const AttentionArgs a) {
+    constexpr int TD = DV / 16, kRow = DV + 4;
+    extern __shared__ __align__(16) float dyn[];              // queries [MAPS][16][dq + 4], later results [4 waves][MAPS][16][DV + 4]
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, gr = lane >> 4, lr = lane & 15;
+    const uint32_t g = blockIdx.x % a.kv_heads, R = a.heads / a.kv_heads, packed = a.rows * R, tiles = (packed + 15) / 16;
+    const uint32_t row0 = (tiles - 1 - blockIdx.x / a.kv_heads) * 16, start = *a.position;          // the long tiles first
+    const uint32_t row_last = min(row0 + 16, packed) - 1, last_key = min(start + row_last / R, a.capacity - 1);
+    const uint32_t row = row0 + lr, limit = min(start + row / R, last_key), first_limit = start + row0 / R, ldq = a.dq + 4, nc = (a.dim + 15) / 16;
+    for (uint32_t i = tid; i < MAPS * 16 * a.dq; i += 256) {
+        const uint32_t k = i % a.dq, r = i / a.dq % 16, mp = i / a.dq / 16, pr = row0 + r, t = pr / R, h = g * R + pr - t * R;
+        dyn[(mp * 16 + r) * ldq + k] = t < a.rows && k < a.dim ? static_cast<const float*>(a.q)[(((size_t)t * a.heads + h) * MAPS + mp) * a.dq + k] : 0.0f;
+    }
+    __syncthreads();
+    lh_f32x4 o[MAPS][TD];
+    float m[MAPS], l[MAPS];
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++) {
+        m[mp] = -INFINITY; l[mp] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < TD; d++) o[mp][d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    const float* K = static_cast<const float*>(a.keys) + (size_t)g * MAPS * a.dq;
+    const float* V = static_cast<const float*>(a.values) + (size_t)g * DV * 32;
+    const size_t krow = (size_t)a.kv_heads * MAPS * a.dq, vblock = (size_t)a.kv_heads * DV * 32;
+    for (uint32_t b = wave; b * 32 <= last_key; b += 4) {
+        float p[MAPS][8];
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            lh_f32x4 s[2] = {(lh_f32x4){0.f, 0.f, 0.f, 0.f}, (lh_f32x4){0.f, 0.f, 0.f, 0.f}};
+            const float* qr = dyn + (mp * 16 + lr) * ldq + gr * 4;
+            const float *ka = K + min(b * 32 + lr, last_key) * krow + mp * a.dq + gr * 4, *kb = K + min(b * 32 + 16 + lr, last_key) * krow + mp * a.dq + gr * 4;
+            for (uint32_t c0 = 0; c0 < nc; c0 += 4) {         // 64 dimensions at a time, all their loads ahead of the products
+                lh_f32x4 x[4], y[4], q4[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const uint32_t c = min(c0 + u, nc - 1) * 16;
+                    x[u] = *reinterpret_cast<const lh_f32x4*>(ka + c);
+                    y[u] = *reinterpret_cast<const lh_f32x4*>(kb + c);
+                    q4[u] = *reinterpret_cast<const lh_f32x4*>(qr + c);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const bool in = (c0 + u) * 16 + gr * 4 + j < a.dim;   // (what pads a key row may be anything)
+                        s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? x[u][j] : 0.0f, in ? q4[u][j] : 0.0f, s[0], 0, 0, 0);
+                        s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? y[u][j] : 0.0f, in ? q4[u][j] : 0.0f, s[1], 0, 0, 0);
+                    }
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                p[mp][i] = s[i >> 2][i & 3] * a.scale;
+                if (b * 32 + 31 > first_limit && b * 32 + (i >> 2) * 16 + gr * 4 + (i & 3) > limit) p[mp][i] = -INFINITY;
+                mx = fmaxf(mx, p[mp][i]);
+            }
+            const float nm = fmaxf(m[mp], lh_column_max(mx)), base = nm == -INFINITY ? 0.0f : nm, alpha = expf(m[mp] - base);
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) { p[mp][i] = expf(p[mp][i] - base); sum += p[mp][i]; }
+            l[mp] = l[mp] * alpha + sum;                      // this lane's keys; the four lanes of a row are added at the end
+            m[mp] = nm;
+#pragma unroll
+            for (int d = 0; d < TD; d++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[mp][d][r] *= alpha;
+        }
+        const bool end = b * 32 + 31 > last_key;              // entries of a block past the last key may be anything
+#pragma unroll
+        for (int d = 0; d < TD; d++) {
+            const float* vr = V + b * vblock + (d * 16 + lr) * 32 + gr * 8;
+            lh_f32x4 x = *reinterpret_cast<const lh_f32x4*>(vr), y = *reinterpret_cast<const lh_f32x4*>(vr + 4);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (end && b * 32 + gr * 4 + j > last_key) x[j] = 0.0f;
+                if (end && b * 32 + 16 + gr * 4 + j > last_key) y[j] = 0.0f;
+#pragma unroll
+                for (int mp = 0; mp < MAPS; mp++) {
+                    o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], p[mp][j], o[mp][d], 0, 0, 0);
+                    o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j], p[mp][4 + j], o[mp][d], 0, 0, 0);
+                }
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++) {
+        float* d0 = dyn + ((wave * MAPS + mp) * 16 + lr) * kRow;
+        const float sum = lh_column_sum(l[mp]);
+        if (gr == 0) { d0[DV] = m[mp]; d0[DV + 1] = sum; }
+#pragma unroll
+        for (int d = 0; d < TD; d++) *reinterpret_cast<lh_f32x4*>(d0 + d * 16 + gr * 4) = o[mp][d];
+    }
+    __syncthreads();
+    // a wave finishes four of the rows, 16 lanes a row
+    const uint32_t r = wave * 4 + gr, pr = row0 + r, t = pr / R, h = g * R + pr - t * R;
+    float f[MAPS][4];
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++) {
+        float top = -INFINITY, sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) top = fmaxf(top, dyn[((w * MAPS + mp) * 16 + r) * kRow + DV]);
+        const float sink = MAPS == 1 && a.sink && t < a.rows ? a.sink[h] : -INFINITY;
+        top = fmaxf(top, sink);
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const float* d0 = dyn + ((w * MAPS + mp) * 16 + r) * kRow;
+            f[mp][w] = expf(d0[DV] - top);
+            sum += f[mp][w] * d0[DV + 1];
+        }
+        sum += expf(sink - top);
+#pragma unroll
+        for (int w = 0; w < 4; w++) f[mp][w] /= sum;
+    }
+    float v[TD], ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TD; i++) {
+        float x[MAPS];
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            x[mp] = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 4; w++) x[mp] += f[mp][w] * dyn[((w * MAPS + mp) * 16 + r) * kRow + i * 16 + lr];
+        }
+        v[i] = x[0];
+        if constexpr (MAPS == 2) v[i] -= a.lambda * x[MAPS - 1];
+        if (i * 16 + lr < a.vdim) ss += v[i] * v[i];
+    }
+    float z = 1.0f;
+    if constexpr (MAPS == 2) z = rsqrtf(lh_group_sum(ss, 16) / (float)a.vdim + a.eps) * a.out_scale;
+    if (t >= a.rows) return;
+    if (MAPS == 1 && a.gate) z = lh_sigmoid(a.gate[(size_t)t * a.heads + h]);
+    float* out = static_cast<float*>(a.out) + ((size_t)t * a.heads + h) * a.vdim;
+#pragma unroll
+    for (int i = 0; i < TD; i++) if (i * 16 + lr < a.vdim) out[i * 16 + lr] = v[i] * z;
+}
+
+template <int DV, int MAPS>
+int launch_wide(lh_context* ctx, const AttentionArgs& a, const char* op) {
+    const uint64_t grid = ((uint64_t)a.rows * (a.heads / a.kv_heads) + 15) / 16 * a.kv_heads;
+    LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: %u rows", op, a.rows);
+    const size_t lds = std::max<size_t>((size_t)MAPS * 16 * (a.dq + 4), (size_t)4 * MAPS * 16 * (DV + 4)) * 4;
+    const int r = lh_raise_dynamic_lds(ctx, (const void*)attention_wide_kernel<DV, MAPS>, lds, op);
+    if (r != LH_OK) return r;
+    hipLaunchKernelGGL((attention_wide_kernel<DV, MAPS>), dim3((uint32_t)grid), dim3(256), lds, ctx->stream, a);
+    return lh_check_launch(op);
+}
+template <int MAPS>
+int launch_wide_dv(lh_context* ctx, const AttentionArgs& a, const char* op) {
+    switch (a.dv) {
+        case 32: return launch_wide<32, MAPS>(ctx, a, op);
+        case 64: return launch_wide<64, MAPS>(ctx, a, op);
+        case 128: return launch_wide<128, MAPS>(ctx, a, op);
+        default: return launch_wide<256, MAPS>(ctx, a, op);
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -403,6 +569,9 @@ int lh_attention_rows_into(lh_batch* batch, const lh_buffer* q, const lh_buffer*
         else if (a.dq == 128) r = launch_dv<128>(batch->ctx, a, max_position, op, launches);
         else if (a.dq == 192) r = launch_dv<192>(batch->ctx, a, max_position, op, launches);
         else r = launch_dv<256>(batch->ctx, a, max_position, op, launches);
+    } else if (dtype == LH_F32 && aligned && a.dq <= kWideMaxDim && (a.dv == 32 || a.dv == 64 || a.dv == 128 || a.dv == 256)) {
+        r = maps == 2 ? launch_wide_dv<2>(batch->ctx, a, op) : launch_wide_dv<1>(batch->ctx, a, op);
+        launches = 1;
     } else {
         LH_REQUIRE((uint64_t)rows * heads < 0x7FFFFFFFull, "%s: %u rows", op, rows);
         const size_t lds = (size_t)maps * dim * 4;

@@ -340,6 +340,14 @@ def test_attention_ignores_what_lies_behind_the_last_position(ai, gpu, rows):
     assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("dim,vdim", [(32, 32), (20, 33), (64, 64), (33, 128), (128, 128), (100, 256), (136, 64), (192, 128), (200, 250), (256, 256)])
+@pytest.mark.parametrize("start,rows", [(0, 1), (70, 1), (31, 18), (5, 150)])
+@pytest.mark.parametrize("maps", [1, 2])
+def test_wide_attention_every_head_size(ai, gpu, maps, dim, vdim, start, rows):
+    a = attention_case(ai, gpu, "f32", maps, 4, 2, dim, vdim, start, rows, 256)
+    assert np.array_equal(a, attention_case(ai, gpu, "f32", maps, 4, 2, dim, vdim, start, rows, 256, stale=True))
+
+
 def test_attention_long_context_splits(ai, gpu):
     for rows in (1, 5):
         attention_case(ai, gpu, "bf16", 2, 2, 1, 32, 32, 9000, rows, 9056, spike=(0, 37))
