@@ -749,6 +749,10 @@ __device__ void stage_vector(const VectorStage& st, float* xs, float* scratch, u
 struct RowWalk {
     const uint32_t first, count, pairs;
     __device__ __forceinline__ uint32_t row(uint32_t i) const { return pairs ? 2 * (first + (i >> 1) * count) + (i & 1) : first + i * count; }
+    __device__ __forceinline__ uint32_t rows(uint32_t N) const {  // how many of N
+        const uint32_t n = pairs ? N / 2 : N, r = first < n ? (n - first - 1) / count + 1 : 0u;
+        return pairs ? 2 * r : r;
+    }
 };
 
 // Stores the finished sums of rows i0 .. i0 + n - 1 of a walk, one per lane.
@@ -769,13 +773,23 @@ struct RowSums {
     const RowWalk& walk;
     const uint32_t lane;
     uint32_t i0 = 0, n = 0;
-    float mine = 0.0f;
+    float mine = 0.0f, before = 0.0f;
+    bool known = false;
+    // What the first 64 sums are added to is requested ahead of the products, where it is one plain row of values.
+    __device__ __forceinline__ void request(uint32_t rows) {
+        known = seg.accumulate && seg.count == 1 && !seg.pairs && !lh_segment_at_position(seg, 0) && seg.head[0] == seg.padded[0];
+        if (known && lane < rows) before = static_cast<const float*>(seg.out[0])[walk.row(lane)];
+    }
+    __device__ __forceinline__ void keep(float total) { mine = n++ == lane ? total : mine; }      // up to 64 of them, then a flush
     __device__ __forceinline__ void add(float total) {
-        mine = n == lane ? total : mine;
-        if (++n == 64) flush();
+        keep(total);
+        if (n == 64) flush();
     }
     __device__ __forceinline__ void flush() {
-        store_sums(seg, bias, walk, i0, n, lane, mine);
+        if (known && i0 == 0) {
+            const uint32_t row = walk.row(lane);
+            if (lane < n) static_cast<float*>(seg.out[0])[row] = before + lh_activate(bias ? mine + bias[row] : mine, seg.act[0]);
+        } else store_sums(seg, bias, walk, i0, n, lane, mine);
         i0 += n;
         n = 0;
     }
@@ -843,81 +857,86 @@ __global__ __launch_bounds__(256) void matvec_bf16_kernel(const VectorStage st, 
     sums.flush();
 }
 
-// The same with the vector in registers (K up to 512 * NL): the first row's weights are requested before the vector.
+// The same with the vector in registers (K up to 512 * NL), eight waves that bring it in together; the weights of two rows are
+// requested right behind it and every wait leaves the younger loads on their way.  What bounds it is the length of one such chain, not
+// the bytes.  (Four waves, each with the vector for itself and one row ahead: 10.0 us a launch on average over the products of a step
+// behind a norm, 2048 columns and 2048 to 32000 rows, 10.6 behind a gate, 5.9 with neither; now 8.9, 5.8 and 4.0.)
 template <int STAGE, int NL>
-__global__ __launch_bounds__(256) void matvec_bf16_reg_kernel(const VectorStage st, const uint16_t* __restrict__ W, const float* __restrict__ bias, const LhSegments seg,
+__global__ __launch_bounds__(512) void matvec_bf16_reg_kernel(const VectorStage st, const uint16_t* __restrict__ W, const float* __restrict__ bias, const LhSegments seg,
                                                              uint32_t N, uint32_t K) {
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, last = (K >> 3) - 1;
-    const RowWalk walk{blockIdx.x * 4 + wave, gridDim.x * 4, seg.pairs};
-    auto issue = [&](uint4 (&v)[NL], uint32_t r) {
-        const uint16_t* wr = W + (size_t)r * K;
+    __shared__ LhVectorSpace space;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), last = (K >> 3) - 1;
+    const RowWalk walk{blockIdx.x * kVectorWaves + wave, gridDim.x * kVectorWaves, seg.pairs};
+    const uint32_t rows = walk.rows(N);
+    struct Row { uint4 w[NL]; } v[2];
+    auto issue = [&](Row& x, uint32_t i) {
+        const uint16_t* wr = W + (size_t)min(walk.row(i), N - 1) * K;
 #pragma unroll
-        for (int c = 0; c < NL; c++) v[c] = lh_ld16_stream(wr + 8 * min(64u * c + lane, last));
+        for (int c = 0; c < NL; c++) x.w[c] = lh_ld16_stream(wr + 8 * min(64u * c + lane, last));
     };
-    uint32_t at = 0;
-    if (walk.row(0) >= N) return;
-    uint4 p[NL], q[NL];
-    issue(p, walk.row(0));
+    LhSharedVector<STAGE, NL> x;
+    x.fetch(st, K, lane, wave);
+    lh_first_rows(v, max(rows, 1u), [&](Row& r, uint32_t i) { issue(r, rows ? i : 0u); });
     RowSums sums{seg, bias, walk, lane};
     float xr[NL][8];
-    lh_vector_registers<STAGE, NL>(st, K, lane, blockIdx.x == 0 && wave == 0 && st.store != nullptr, xr);
-    auto step = [&](const uint4 (&cur)[NL], uint4 (&nxt)[NL]) {   // false: that was the wave's last row
-        const uint32_t next = walk.row(++at);
-        const bool more = next < N;
-        if (more) issue(nxt, next);
+    x.finish(st, K, lane, wave, blockIdx.x == 0 && st.store != nullptr, space, xr);
+    if (rows == 0) return;
+    sums.request(rows);
+    lh_walk_rows(v, rows, issue, [&](const Row& r, uint32_t) {
         float acc = 0.0f;
 #pragma unroll
-        for (int c = 0; c < NL; c++) acc = lh_dot8(cur[c], xr[c], acc);
-        sums.add(lh_group_sum(acc, 64));
-        return more;
-    };
-    while (step(p, q) && step(q, p)) {}
+        for (int c = 0; c < NL; c++) acc = lh_dot8(r.w[c], xr[c], acc);
+        sums.keep(lh_group_sum(acc, 64));
+    });
     sums.flush();
 }
 
-// Rows longer than a wave's registers: the four waves of a workgroup take a quarter of the columns each, and the quarters of up to 64 rows meet in LDS.  Plain vectors only: a norm would need all quarters.
-template <int NL>
-__global__ __launch_bounds__(256) void matvec_bf16_quarter_kernel(const VectorStage st, const uint16_t* __restrict__ W, const float* __restrict__ bias, const LhSegments seg,
-                                                                 uint32_t N, uint32_t K, uint32_t quarter) {
-    __shared__ float sums[4][64];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, k0 = wave * quarter, len = k0 < K ? min(quarter, K - k0) : 0u;   // quarter: a multiple of 8
+// Rows longer than a wave's registers: the eight waves of a workgroup take an eighth of the columns each, and the parts of up to 64
+// rows, all that a workgroup takes, meet in LDS, where wave 0 adds them.  Plain vectors only: a norm would need all parts.  (Four waves with a
+// quarter each and one row ahead: 9.6 us for 2048 x 8192; now 7.8.)
+template <int NL, int R>
+__global__ __launch_bounds__(512) void matvec_bf16_part_kernel(const VectorStage st, const uint16_t* __restrict__ W, const float* __restrict__ bias, const LhSegments seg,
+                                                              uint32_t N, uint32_t K, uint32_t part) {
+    __shared__ float sums[kVectorWaves][64];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), k0 = wave * part, len = k0 < K ? min(part, K - k0) : 0u;   // part: a multiple of 8
     const uint32_t last = len ? (len >> 3) - 1 : 0u, kb = len ? k0 : 0u;
-    auto issue = [&](uint4 (&v)[NL], uint32_t r) {
-        const uint16_t* wr = W + (size_t)r * K + kb;
-#pragma unroll
-        for (int c = 0; c < NL; c++) v[c] = lh_ld16_stream(wr + 8 * min(64u * c + lane, last));
-    };
     const RowWalk walk{blockIdx.x, gridDim.x, seg.pairs};
-    uint32_t at = 0, i0 = 0, n = 0;
-    if (walk.row(0) >= N) return;
-    uint4 p[NL], q[NL];
-    issue(p, walk.row(0));
-    VectorStage part = st;
-    part.x = st.x_f32 ? (const void*)(static_cast<const float*>(st.x) + kb) : (const void*)(static_cast<const uint16_t*>(st.x) + kb);
-    float xr[NL][8], mine = 0.0f;
-    lh_vector_registers<kPlain, NL>(part, len, lane, false, xr);
-    auto flush = [&]() {
-        sums[wave][lane] = mine;
-        __syncthreads();
-        if (wave == 0) store_sums(seg, bias, walk, i0, n, lane, (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]));
-        __syncthreads();
-        i0 += n;
-        n = 0;
+    const uint32_t rows = walk.rows(N);
+    if (rows == 0) return;
+    struct Row { uint4 w[NL]; } v[R];
+    auto issue = [&](Row& x, uint32_t i) {
+        const uint16_t* wr = W + (size_t)walk.row(i) * K + kb;
+#pragma unroll
+        for (int c = 0; c < NL; c++) x.w[c] = lh_ld16_stream(wr + 8 * min(64u * c + lane, last));
     };
-    auto step = [&](const uint4 (&cur)[NL], uint4 (&nxt)[NL]) {
-        const uint32_t next = walk.row(++at);
-        const bool more = next < N;
-        if (more) issue(nxt, next);
+    LhEither8 raw[NL];                                        // the vector first (see LhSharedVector)
+#pragma unroll
+    for (int c = 0; c < NL; c++) raw[c].load(st.x, st.x_f32, kb + 8 * min(64u * c + lane, last));
+    lh_first_rows(v, rows, issue);
+    RowSums total{seg, bias, walk, lane};
+    float xr[NL][8], mine = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NL; c++) {
+        raw[c].get(st.x_f32, xr[c]);
+#pragma unroll
+        for (int j = 0; j < 8; j++) xr[c][j] = (64u * c + lane) * 8 < len ? xr[c][j] : 0.0f;
+    }
+    if (wave == 0) total.request(rows);
+    lh_walk_rows(v, rows, issue, [&](const Row& x, uint32_t i) {
         float acc = 0.0f;
 #pragma unroll
-        for (int c = 0; c < NL; c++) acc = lh_dot8(cur[c], xr[c], acc);
+        for (int c = 0; c < NL; c++) acc = lh_dot8(x.w[c], xr[c], acc);
         acc = lh_group_sum(acc, 64);
-        mine = n == lane ? acc : mine;
-        if (++n == 64) flush();
-        return more;
-    };
-    while (step(p, q) && step(q, p)) {}
-    if (n) flush();
+        mine = i == lane ? acc : mine;
+    });
+    sums[wave][lane] = mine;
+    lh_vector_barrier();
+    if (wave != 0) return;
+    float t = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kVectorWaves; w++) t += sums[w][lane];
+    total.mine = t; total.n = rows;
+    total.flush();
 }
 
 constexpr uint32_t kMaxVectorK = 36864;   // 144 KB of staged f32 activations
@@ -929,8 +948,13 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
     const uint32_t takes = seg.pairs ? N / 2 : N;             // rows, or pairs of rows
     const bool vec = K % 8 == 0 && ((uintptr_t)W & 15) == 0;
     if (vec && K <= 4096 && lh_stage_aligned(st)) {
-        const uint32_t grid = (uint32_t)std::min<uint64_t>(((uint64_t)takes + 3) / 4, (uint64_t)ctx->cu_count * (K <= 2048 ? 4 : 2));
-#define LH_MVR(NLOADS) hipLaunchKernelGGL((matvec_bf16_reg_kernel<STAGE, NLOADS>), dim3(grid), dim3(256), 0, ctx->stream, st, W, bias, seg, N, K)
+        // A workgroup for every CU first; a second one where rows are short and each of its waves still has two (32000 x 1024: 11.9 us
+        // against 12.5; 8192 x 2048: 7.8 against 7.65).
+        const uint64_t cus = (uint64_t)ctx->cu_count, most = std::max(cus, K <= 1024 ? std::min<uint64_t>(2 * cus, ((uint64_t)takes + 15) / 16) : 0);
+        const uint32_t each = seg.pairs ? 32 : 64;           // a wave's sums fit its lanes
+        const uint32_t grid = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(((uint64_t)takes + kVectorWaves - 1) / kVectorWaves, most),
+                                                           ((uint64_t)takes + kVectorWaves * each - 1) / (kVectorWaves * each));
+#define LH_MVR(NLOADS) hipLaunchKernelGGL((matvec_bf16_reg_kernel<STAGE, NLOADS>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K)
         if (K <= 512) LH_MVR(1);
         else if (K <= 1024) LH_MVR(2);
         else if (K <= 2048) LH_MVR(4);
@@ -939,10 +963,10 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
         return lh_check_launch(op);
     }
     if constexpr (STAGE == kPlain) if (vec && K <= 16384 && lh_stage_aligned(st)) {
-        const uint32_t quarter = ((K + 3) / 4 + 7) / 8 * 8, grid = (uint32_t)std::min<uint64_t>(takes, (uint64_t)ctx->cu_count * 4);
-        if (quarter <= 1024) hipLaunchKernelGGL((matvec_bf16_quarter_kernel<2>), dim3(grid), dim3(256), 0, ctx->stream, st, W, bias, seg, N, K, quarter);
-        else if (quarter <= 2048) hipLaunchKernelGGL((matvec_bf16_quarter_kernel<4>), dim3(grid), dim3(256), 0, ctx->stream, st, W, bias, seg, N, K, quarter);
-        else hipLaunchKernelGGL((matvec_bf16_quarter_kernel<8>), dim3(grid), dim3(256), 0, ctx->stream, st, W, bias, seg, N, K, quarter);
+        const uint32_t part = ((K + 7) / 8 + 7) / 8 * 8, each = seg.pairs ? 32 : 64;
+        const uint32_t grid = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(takes, (uint64_t)ctx->cu_count), ((uint64_t)takes + each - 1) / each);
+        if (part <= 1024) hipLaunchKernelGGL((matvec_bf16_part_kernel<2, 4>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
+        else hipLaunchKernelGGL((matvec_bf16_part_kernel<4, 2>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
         return lh_check_launch(op);
     }
     const uint32_t grid = (uint32_t)std::min<uint64_t>(((uint64_t)takes + 3) / 4, (uint64_t)ctx->cu_count * 4);

@@ -28,7 +28,7 @@ uint32_t lh_expert_tile_rows(uint32_t slots, uint32_t experts);
 
 // ---- one row: the activation vector in registers -------------------------------------------------------------------------
 // Up to 4096 columns a wave keeps the vector itself: lane l holds the NL chunks of eight elements 8 (64 c + l), which is what
-// it multiplies in every row.  The norm before the product is then a sum over the wave, with no barrier and no LDS.
+// it multiplies in every row.
 enum { kPlain = 0, kNorm = 1, kGated = 2, kResidual = 3 };
 struct VectorStage {
     const void* x;             // plain: x_f32 ? f32 : bf16; the others: f32
@@ -52,88 +52,134 @@ __device__ __forceinline__ void lh_ld8(const uint16_t* p, float (&v)[8]) {
     for (int j = 0; j < 4; j++) { v[2 * j] = __builtin_bit_cast(float, w[j] << 16); v[2 * j + 1] = __builtin_bit_cast(float, w[j] & 0xFFFF0000u); }
 }
 
-// K a multiple of 8, all pointers 16-byte aligned; chunks past K are zero.  `store` whether this wave stores x + add.
+// A vector for the registers of eight waves, K a multiple of 8 up to 512 NL, all pointers 16-byte aligned, zero past K: wave c brings in
+// the chunks 64 c + lane and what they need, the sums of the norm meet in LDS, and every wave takes the finished vector from there.
+// (Every wave for itself: 16 KB from the caches per wave for 2048 columns with a norm, as much as the weights of two rows.)
+//
+// Loads return in order, so what is requested first can be waited for alone: the vector first (`fetch`), then the weights of the first
+// rows, then `finish`.  And behind a load that not every path makes the compiler waits for all there are, so every load here is
+// made: lanes and waves without a chunk load one that exists, and an operand that is not there is read from x.
+constexpr int kVectorWaves = 8;
+struct LhVectorSpace { float4 x[16][64]; float part[kVectorWaves]; };
+__device__ __forceinline__ void lh_vector_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Eight values at element k, stored as f32 or bf16.
+struct LhEither8 {
+    uint4 a, b;
+    __device__ __forceinline__ void load(const void* p, bool f32, uint32_t k) {
+        const char* q = static_cast<const char*>(p) + (size_t)k * (f32 ? 4 : 2);
+        a = *reinterpret_cast<const uint4*>(q);
+        b = *reinterpret_cast<const uint4*>(q + (f32 ? 16 : 0));
+    }
+    __device__ __forceinline__ void get(bool f32, float (&v)[8]) const {
+        const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = __builtin_bit_cast(float, f32 ? w[j] : j & 1 ? w[j >> 1] & 0xFFFF0000u : w[j >> 1] << 16);
+    }
+};
+
 template <int STAGE, int NL>
-__device__ __forceinline__ void lh_vector_registers(const VectorStage& st, uint32_t K, uint32_t lane, bool store, float (&xr)[NL][8]) {
-    constexpr bool kNormed = STAGE == kNorm || STAGE == kGated || STAGE == kResidual;
-    float w[kNormed ? NL : 1][8], s[kNormed ? NL : 1], total = 0.0f;
+struct LhSharedVector {
+    static_assert(NL <= kVectorWaves, "a chunk per wave");
+    static constexpr bool kNormed = STAGE == kNorm || STAGE == kGated || STAGE == kResidual;
+    static constexpr bool kAdds = STAGE == kNorm || STAGE == kResidual;
+    LhEither8 x, gate;
+    float w[8], more[8];
+
+    __device__ __forceinline__ void fetch(const VectorStage& st, uint32_t K, uint32_t lane, uint32_t wave) {
+        const uint32_t k = wave < NL ? min((64 * wave + lane) * 8, K - 8) : 0u;
+        x.load(st.x, STAGE != kPlain || st.x_f32, k);
+        if constexpr (kNormed) lh_ld8((st.norm_weight ? st.norm_weight : static_cast<const float*>(st.x)) + k, w);
+        if constexpr (kAdds) lh_ld8((st.add ? st.add : static_cast<const float*>(st.x)) + k, more);
+        if constexpr (STAGE == kGated) gate.load(st.gate, st.gate_f32, k);
+    }
+    __device__ __forceinline__ void finish(const VectorStage& st, uint32_t K, uint32_t lane, uint32_t wave, bool store, LhVectorSpace& sp, float (&xr)[NL][8]) {
+        const uint32_t k = (64 * wave + lane) * 8;
+        const bool owner = wave < NL, in = owner && k < K;
+        float v[8], sum = 0.0f;
+        x.get(STAGE != kPlain || st.x_f32, v);
+        if constexpr (STAGE == kNorm)
 #pragma unroll
-    for (int c = 0; c < NL; c++) {
-        const uint32_t k = (64 * c + lane) * 8;
+            for (int j = 0; j < 8; j++) v[j] = st.add ? v[j] + more[j] : v[j];
+        if constexpr (STAGE == kGated) {
+            float g[8];
+            gate.get(st.gate_f32, g);
 #pragma unroll
-        for (int j = 0; j < 8; j++) xr[c][j] = 0.0f;
-        if constexpr (kNormed) s[c] = 0.0f;
-        if (k >= K) continue;
-        if (STAGE == kPlain && !st.x_f32) lh_ld8(static_cast<const uint16_t*>(st.x) + k, xr[c]);
-        else lh_ld8(static_cast<const float*>(st.x) + k, xr[c]);
-        if constexpr (STAGE == kNorm) if (st.add) {
-            float b[8];
-            lh_ld8(st.add + k, b);
-#pragma unroll
-            for (int j = 0; j < 8; j++) xr[c][j] += b[j];
+            for (int j = 0; j < 8; j++) {
+                const float f = lh_gate(g[j], st.gate_act);
+                w[j] = st.norm_weight ? w[j] : 1.0f;
+                if (st.gate_first) v[j] *= f; else w[j] *= f;
+            }
         }
         if constexpr (kNormed) {
-            if (STAGE != kGated || st.norm_weight) lh_ld8(st.norm_weight + k, w[c]);
-            else
 #pragma unroll
-                for (int j = 0; j < 8; j++) w[c][j] = 1.0f;
-            if constexpr (STAGE == kGated) {
-                float g[8];
-                if (st.gate_f32) lh_ld8(static_cast<const float*>(st.gate) + k, g);
-                else lh_ld8(static_cast<const uint16_t*>(st.gate) + k, g);
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float f = lh_gate(g[j], st.gate_act);
-                    if (st.gate_first) xr[c][j] *= f; else w[c][j] *= f;
-                }
+            for (int j = 0; j < 8; j++) {
+                if constexpr (STAGE == kResidual) { sum += more[j] * more[j]; w[j] *= more[j]; }      // the weighted branch
+                else sum += v[j] * v[j];
             }
-            if constexpr (STAGE == kResidual) {               // w becomes the weighted branch
-                float y[8];
-                lh_ld8(st.add + k, y);
+            sum = in ? sum : 0.0f;
+            const bool parts = STAGE == kGated && st.group != K;   // group / 8 chunks: a power of two of lanes, or whole sets of 64
+            const uint32_t cg = parts ? st.group >> 3 : 64u, width = min(cg, 64u);
+            sum = lh_group_sum(sum, (int)width);
+            if (width == 64) {
+                if (lane == 0) sp.part[wave] = sum;
+                lh_vector_barrier();
+                const uint32_t per = parts ? cg >> 6 : (uint32_t)kVectorWaves, w0 = wave / per;
+                sum = 0.0f;
 #pragma unroll
-                for (int j = 0; j < 8; j++) { s[c] += y[j] * y[j]; w[c][j] *= y[j]; }
-            } else
-#pragma unroll
-                for (int j = 0; j < 8; j++) s[c] += xr[c][j] * xr[c][j];
-            total += s[c];
-        }
-    }
-    if constexpr (kNormed) {
-        float r[NL];
-        if (STAGE == kGated && st.group != K) {               // group / 8 chunks: a power of two of lanes, or whole sets of 64
-            const uint32_t cg = st.group >> 3;
-#pragma unroll
-            for (int c = 0; c < NL; c++) s[c] = lh_group_sum(s[c], (int)min(cg, 64u));
-            const uint32_t per = cg > 64 ? cg >> 6 : 1u;
-#pragma unroll
-            for (int c = 0; c < NL; c++) {
-                float t = 0.0f;
-#pragma unroll
-                for (int e = 0; e < NL; e++) t += (uint32_t)e / per == (uint32_t)c / per ? s[e] : 0.0f;
-                r[c] = rsqrtf(t / (float)st.group + st.eps);
+                for (int e = 0; e < kVectorWaves; e++) sum += (uint32_t)e / per == w0 ? sp.part[e] : 0.0f;
             }
-        } else {
-            const float all = rsqrtf(lh_group_sum(total, 64) / (float)K + st.eps);
-#pragma unroll
-            for (int c = 0; c < NL; c++) r[c] = all;
-        }
-#pragma unroll
-        for (int c = 0; c < NL; c++) {
-            const uint32_t k = (64 * c + lane) * 8;
-            if (k >= K) continue;
+            const float r = rsqrtf(sum / (float)(parts ? st.group : K) + st.eps);
             if constexpr (STAGE == kResidual)
 #pragma unroll
-                for (int j = 0; j < 8; j++) xr[c][j] = __builtin_fmaf(w[c][j], r[c], xr[c][j]);
-            if (STAGE != kGated && store) {
-                *reinterpret_cast<float4*>(st.store + k) = make_float4(xr[c][0], xr[c][1], xr[c][2], xr[c][3]);
-                *reinterpret_cast<float4*>(st.store + k + 4) = make_float4(xr[c][4], xr[c][5], xr[c][6], xr[c][7]);
+                for (int j = 0; j < 8; j++) v[j] = __builtin_fmaf(w[j], r, v[j]);
+            if (STAGE != kGated && store && in) {
+                *reinterpret_cast<float4*>(st.store + k) = make_float4(v[0], v[1], v[2], v[3]);
+                *reinterpret_cast<float4*>(st.store + k + 4) = make_float4(v[4], v[5], v[6], v[7]);
             }
             if constexpr (STAGE != kResidual)
 #pragma unroll
-                for (int j = 0; j < 8; j++) xr[c][j] = xr[c][j] * r[c] * w[c][j];
+                for (int j = 0; j < 8; j++) v[j] = v[j] * r * w[j];
+        }
+        if (owner) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[j] = in ? v[j] : 0.0f;
+            sp.x[2 * wave][lane] = make_float4(v[0], v[1], v[2], v[3]);
+            sp.x[2 * wave + 1][lane] = make_float4(v[4], v[5], v[6], v[7]);
+        }
+        lh_vector_barrier();
+#pragma unroll
+        for (int c = 0; c < NL; c++) {
+            const float4 a = sp.x[2 * c][lane], b = sp.x[2 * c + 1][lane];
+            xr[c][0] = a.x; xr[c][1] = a.y; xr[c][2] = a.z; xr[c][3] = a.w; xr[c][4] = b.x; xr[c][5] = b.y; xr[c][6] = b.z; xr[c][7] = b.w;
         }
     }
+};
+
+// Rows 0 .. count - 1 (at least one) of a walk with R of them on their way: issue(v, i) requests row i, use(v, i) multiplies it.
+template <int R, class V, class Issue>
+__device__ __forceinline__ void lh_first_rows(V (&v)[R], uint32_t count, Issue issue) {
+#pragma unroll
+    for (int r = 0; r < R; r++) issue(v[r], min((uint32_t)r, count - 1));
 }
+template <int R, class V, class Issue, class Use>
+__device__ __forceinline__ void lh_walk_rows(V (&v)[R], uint32_t count, Issue issue, Use use) {
+    uint32_t i = 0;
+    for (; i + 2 * R <= count; i += R) {
+#pragma unroll
+        for (int r = 0; r < R; r++) { use(v[r], i + r); issue(v[r], i + R + r); }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (i + r < count) {
+            use(v[r], i + r);
+            if (i + R + r < count) issue(v[r], i + R + r);
+        }
+    i += R;
+#pragma unroll
+    for (int r = 0; r < R; r++) if (i + r < count) use(v[r], i + r);
+}
+
 static inline bool lh_stage_aligned(const VectorStage& st) {
     return (((uintptr_t)st.x | (uintptr_t)st.add | (uintptr_t)st.store | (uintptr_t)st.norm_weight | (uintptr_t)st.gate) & 15) == 0;
 }

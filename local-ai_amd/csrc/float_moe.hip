@@ -150,35 +150,38 @@ __global__ __launch_bounds__(256) void vector_up_kernel(const float* __restrict_
     }
 }
 
-// The same with the normed vector in registers (width a multiple of 8, up to 512 * NL): a workgroup keeps to one expert's rows
-// (blockIdx.y: the choice), and the first row's weights are requested as soon as the selection is known.
+// The same with the normed vector in registers (width a multiple of 8, up to 512 * NL), brought in by eight waves together: a
+// workgroup keeps to one expert's rows (blockIdx.y: the choice), and the weights of two rows are requested as soon as the selection is known.
 template <int NL>
-__global__ __launch_bounds__(256) void vector_up_reg_kernel(const VectorStage st, const float* __restrict__ logits, const uint16_t* __restrict__ up,
+__global__ __launch_bounds__(512) void vector_up_reg_kernel(const VectorStage st, const float* __restrict__ logits, const uint16_t* __restrict__ up,
                                                            float* __restrict__ hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act) {
-    __shared__ uint32_t ids[4][kMaxTop];
-    __shared__ float weights[4][kMaxTop];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = blockIdx.y, last = (width >> 3) - 1;
+    __shared__ uint32_t ids[kVectorWaves][kMaxTop];
+    __shared__ float weights[kVectorWaves][kMaxTop];
+    __shared__ LhVectorSpace space;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = blockIdx.y, last = (width >> 3) - 1;
+    LhSharedVector<kNorm, NL> x;
+    x.fetch(st, width, lane, wave);
     select_experts(logits, experts, c + 1, lane, ids[wave], weights[wave]);    // every wave for itself: no barrier
-    const uint32_t e = ids[wave][c];
+    const uint32_t e = __builtin_amdgcn_readfirstlane(ids[wave][c]);
     const float weight = weights[wave][c];
     const uint16_t* base = up + (size_t)e * ff * width;
-    uint32_t row = blockIdx.x * 4 + wave;
-    uint4 w[NL];
-    auto issue = [&](uint32_t r) {
+    const uint32_t first = blockIdx.x * kVectorWaves + wave, step = gridDim.x * kVectorWaves, rows = first < ff ? (ff - first - 1) / step + 1 : 0u;
+    struct Row { uint4 w[NL]; } v[2];
+    auto issue = [&](Row& x, uint32_t i) {
 #pragma unroll
-        for (int i = 0; i < NL; i++) w[i] = lh_ld16_stream(base + (size_t)min(r, ff - 1) * width + 8 * min(64u * i + lane, last));
+        for (int j = 0; j < NL; j++) x.w[j] = lh_ld16_stream(base + (size_t)(first + i * step) * width + 8 * min(64u * j + lane, last));
     };
-    issue(row);
+    if (rows) lh_first_rows(v, rows, issue);
     float xr[NL][8];
-    lh_vector_registers<kNorm, NL>(st, width, lane, false, xr);
-    for (; row < ff; row += gridDim.x * 4) {
+    x.finish(st, width, lane, wave, false, space, xr);
+    if (rows == 0) return;
+    lh_walk_rows(v, rows, issue, [&](const Row& r, uint32_t i) {
         float acc = 0.0f;
 #pragma unroll
-        for (int i = 0; i < NL; i++) acc = lh_dot8(w[i], xr[i], acc);
-        if (row + gridDim.x * 4 < ff) issue(row + gridDim.x * 4);
+        for (int j = 0; j < NL; j++) acc = lh_dot8(r.w[j], xr[j], acc);
         acc = lh_group_sum(acc, 64);
-        if (lane == 0) hidden[c * ff + row] = lh_activate(weight * acc, act);
-    }
+        if (lane == 0) hidden[c * ff + first + i * step] = lh_activate(weight * acc, act);
+    });
 }
 
 // residual[r] += sum_c down[e_c][r] . hidden[c]
@@ -201,15 +204,16 @@ __global__ __launch_bounds__(256) void vector_down_kernel(const float* __restric
 // The same with the hidden values of all choices in registers as one vector of top * ff (ff a multiple of 8): a lane's chunk
 // belongs to one choice, so it has its own place in the weights.
 template <int NL>
-__global__ __launch_bounds__(256) void vector_down_reg_kernel(const float* __restrict__ hidden, const float* __restrict__ logits, const uint16_t* __restrict__ down,
+__global__ __launch_bounds__(512) void vector_down_reg_kernel(const float* __restrict__ hidden, const float* __restrict__ logits, const uint16_t* __restrict__ down,
                                                              float* __restrict__ residual, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff) {
-    __shared__ uint32_t ids[4][kMaxTop];
-    __shared__ float weights[4][kMaxTop];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, chunks = top * (ff >> 3), row_step = gridDim.x * 4;
+    __shared__ uint32_t ids[kVectorWaves][kMaxTop];
+    __shared__ float weights[kVectorWaves][kMaxTop];
+    __shared__ LhVectorSpace space;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), chunks = top * (ff >> 3);
     VectorStage st{};
     st.x = hidden; st.x_f32 = 1;
-    float xr[NL][8];
-    lh_vector_registers<kPlain, NL>(st, top * ff, lane, false, xr);
+    LhSharedVector<kPlain, NL> x;
+    x.fetch(st, top * ff, lane, wave);
     select_experts(logits, experts, top, lane, ids[wave], weights[wave]);
     const uint16_t* base[NL];
 #pragma unroll
@@ -217,23 +221,25 @@ __global__ __launch_bounds__(256) void vector_down_reg_kernel(const float* __res
         const uint32_t q = min(64u * i + lane, chunks - 1), c = q / (ff >> 3);
         base[i] = down + (size_t)ids[wave][c] * width * ff + 8 * (q - c * (ff >> 3));
     }
-    uint32_t n = blockIdx.x * 4 + wave;
-    if (n >= width) return;
-    uint4 w[NL];
-    auto issue = [&](uint32_t r) {
+    const uint32_t first = blockIdx.x * kVectorWaves + wave, step = gridDim.x * kVectorWaves, rows = first < width ? (width - first - 1) / step + 1 : 0u;
+    struct Row { uint4 w[NL]; float before; } v[2];
+    auto issue = [&](Row& x, uint32_t i) {
+        const uint32_t n = first + i * step;
+        x.before = residual[n];
 #pragma unroll
-        for (int i = 0; i < NL; i++) w[i] = lh_ld16_stream(base[i] + (size_t)r * ff);
+        for (int j = 0; j < NL; j++) x.w[j] = lh_ld16_stream(base[j] + (size_t)n * ff);
     };
-    issue(n);
-    for (; n < width; n += row_step) {
-        const float before = lane == 0 ? residual[n] : 0.0f;
+    if (rows) lh_first_rows(v, rows, issue);
+    float xr[NL][8];
+    x.finish(st, top * ff, lane, wave, false, space, xr);
+    if (rows == 0) return;
+    lh_walk_rows(v, rows, issue, [&](const Row& r, uint32_t i) {
         float acc = 0.0f;
 #pragma unroll
-        for (int i = 0; i < NL; i++) acc = lh_dot8(w[i], xr[i], acc);
-        if (n + row_step < width) issue(n + row_step);
+        for (int j = 0; j < NL; j++) acc = lh_dot8(r.w[j], xr[j], acc);
         acc = lh_group_sum(acc, 64);
-        if (lane == 0) residual[n] = before + acc;
-    }
+        if (lane == 0) residual[first + i * step] = r.before + acc;
+    });
 }
 
 int check_shape(const char* op, uint32_t rows, uint32_t experts, uint32_t top) {
@@ -366,8 +372,8 @@ int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const lh_buff
     VectorStage st{};
     st.x = input->ptr; st.x_f32 = 1; st.norm_weight = (const float*)norm_weight->ptr; st.eps = eps;
     if (width % 8 == 0 && width <= 4096 && ((uintptr_t)up->ptr & 15) == 0 && lh_stage_aligned(st)) {
-        const dim3 grid(std::min<uint32_t>((ff + 3) / 4, std::max<uint32_t>(1, (uint32_t)batch->ctx->cu_count * 4 / top)), top);
-#define LH_UP(NL) hipLaunchKernelGGL((vector_up_reg_kernel<NL>), grid, dim3(256), 0, batch->ctx->stream, st, (const float*)logits->ptr, (const uint16_t*)up->ptr, \
+        const dim3 grid(std::min<uint32_t>((ff + kVectorWaves - 1) / kVectorWaves, std::max<uint32_t>(1, (uint32_t)batch->ctx->cu_count / top)), top);
+#define LH_UP(NL) hipLaunchKernelGGL((vector_up_reg_kernel<NL>), grid, dim3(64 * kVectorWaves), 0, batch->ctx->stream, st, (const float*)logits->ptr, (const uint16_t*)up->ptr, \
                                      (float*)hidden->ptr, experts, top, width, ff, act)
         if (width <= 512) LH_UP(1);
         else if (width <= 1024) LH_UP(2);
@@ -400,8 +406,8 @@ int lh_moe_vector_down_into(lh_batch* batch, const lh_buffer* hidden, const lh_b
     LH_NEED(down, (size_t)experts * ff * width * 2, op, "down");
     LH_NEED(residual, (size_t)width * 4, op, "residual");
     if (ff % 8 == 0 && (uint64_t)top * ff <= 4096 && (((uintptr_t)down->ptr | (uintptr_t)hidden->ptr) & 15) == 0) {
-        const uint32_t blocks = (uint32_t)std::min<uint64_t>(((uint64_t)width + 3) / 4, (uint64_t)batch->ctx->cu_count * 4);
-#define LH_DOWN(NL) hipLaunchKernelGGL((vector_down_reg_kernel<NL>), dim3(blocks), dim3(256), 0, batch->ctx->stream, (const float*)hidden->ptr, (const float*)logits->ptr, \
+        const uint32_t blocks = (uint32_t)std::min<uint64_t>(((uint64_t)width + kVectorWaves - 1) / kVectorWaves, (uint64_t)batch->ctx->cu_count);
+#define LH_DOWN(NL) hipLaunchKernelGGL((vector_down_reg_kernel<NL>), dim3(blocks), dim3(64 * kVectorWaves), 0, batch->ctx->stream, (const float*)hidden->ptr, (const float*)logits->ptr, \
                                        (const uint16_t*)down->ptr, (float*)residual->ptr, experts, top, width, ff)
         if (top * ff <= 512) LH_DOWN(1);
         else if (top * ff <= 1024) LH_DOWN(2);

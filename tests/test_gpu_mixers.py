@@ -236,6 +236,33 @@ def test_linear_vector_stages(ai, gpu, k, n):
         lin.normed_vector_into(batch, K, xb, nb, eps, [outs[0]], ai.F32, None, ab, xb)
 
 
+@pytest.mark.parametrize("k,n", [(8, 2047), (8, 2049), (520, 4098), (1024, 8200), (1032, 6145), (2048, 10250), (2056, 4097), (4096, 2060), (16, 140000),
+                                 (4104, 258), (4160, 770), (8192, 1290), (8200, 515), (16384, 1030), (4104, 16390)])
+@pytest.mark.parametrize("pairs", [False, True])
+def test_one_row_walks(ai, gpu, k, n, pairs):
+    """One row times more weight rows than there are waves: each takes none to six of them or more than a wave has lanes, with an
+    addition to what the output held, and in pairs."""
+    ctx, K = gpu
+    g, L = np.random.default_rng(k + n), ai.linear_weight
+    n += n % 2 if pairs else 0
+    some = M.rounded(g.standard_normal((min(n, 1009), k)) / np.sqrt(k))
+    x, pick, b = stored(g.standard_normal(k), ai, ai.F32), np.arange(n) % len(some), g.standard_normal(n).astype(np.float32)
+    want = (some @ x)[pick] + b
+    lin = L.StackedLinear(ctx, [M.bf16_bits(some)[pick]], [L.Segment(n, ai.ACT_SILU_PAIRS if pairs else ai.ACT_NONE)], [b])
+    print(f"one row {k} {n} {pairs}", flush=True)
+    if pairs:
+        want = want[0::2] * O.sigmoid(want[0::2]) * want[1::2]
+    out, res, batch = empty(ai, ctx, len(want), ai.F32), upload(ai, ctx, np.ones(n), ai.F32), ai.CommandBatch(ctx)
+    xb = upload(ai, ctx, x, ai.F32)
+    lin.vector_into(batch, K, xb, ai.F32, [out], ai.F32)
+    if not pairs:
+        K.linear_vector_into(batch, xb, ai.F32, lin.weight, lin.bias, k, lin.segments, [res], ai.F32, True)
+    batch.commit_and_wait()
+    close(download(ai, out, len(want), ai.F32), want, F32_TOL, "stored")
+    if not pairs:
+        close(download(ai, res, n, ai.F32), want + 1, F32_TOL, "added")
+
+
 @pytest.mark.parametrize("rows,dim", [(1, 64), (5, 100), (3, 1024), (2, 4096), (4, 5000), (70, 33)])
 def test_row_norms_and_gather(ai, gpu, rows, dim):
     ctx, K = gpu
