@@ -117,6 +117,9 @@ struct XPrologue {
 int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const* matrices, const void* const* vectors,
                               void* const* outputs, lh_dtype xt, lh_dtype yt, uint32_t rows, uint32_t K, uint32_t xstride,
                               uint32_t ystride, const XPrologue& pro = XPrologue{kXProNone, nullptr, 0.0f}, uint64_t mstride = 0);
+// The same for up to eight matrices and one vector, f16 in and out (matvec_tq2_direct.hip); -1: not for this form.
+int lh_launch_matvec_tq2_direct(lh_context* ctx, uint32_t count, const void* const* matrices, const void* vector, void* const* outputs, uint32_t rows,
+                                uint32_t K, const XPrologue& pro);
 // The m rows of a small activation batch against one quantized matrix, as m matvecs in one launch (matvec_quant.hip).
 // Returns LH_OK, an error, or -1 when the fast kernels do not take the shape (the caller then uses its own kernel).
 int lh_matvec_rows(lh_batch* batch, lh_quant fmt, uint32_t m, const lh_buffer* weight, const lh_buffer* input, lh_dtype at,
@@ -269,6 +272,33 @@ __device__ __forceinline__ void lh_rotate_pair(float x0, float x1, uint32_t i, u
 // compiler from folding a preceding multiply into v_fma_mixlo_f16, which rounds the exact
 // product once (a different result in double-rounding cases) and turns -0 into +0.
 __device__ __forceinline__ uint16_t lh_f2h_exact(float f) { asm volatile("" : "+v"(f)); return lh_f2h(f); }
+// A workgroup barrier for data in LDS: loads from memory stay on their way.
+__device__ __forceinline__ void lh_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Rows 0 .. count - 1 (at least one) of a walk with R of them on their way: issue(v, i) requests row i, use(v, i) multiplies it.
+template <int R, class V, class Issue>
+__device__ __forceinline__ void lh_first_rows(V (&v)[R], uint32_t count, Issue issue) {
+#pragma unroll
+    for (int r = 0; r < R; r++) issue(v[r], min((uint32_t)r, count - 1));
+}
+template <int R, class V, class Issue, class Use>
+__device__ __forceinline__ void lh_walk_rows(V (&v)[R], uint32_t count, Issue issue, Use use) {
+    uint32_t i = 0;
+    for (; i + 2 * R <= count; i += R) {
+#pragma unroll
+        for (int r = 0; r < R; r++) { use(v[r], i + r); issue(v[r], i + R + r); }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (i + r < count) {
+            use(v[r], i + r);
+            if (i + R + r < count) issue(v[r], i + R + r);
+        }
+    i += R;
+#pragma unroll
+    for (int r = 0; r < R; r++) if (i + r < count) use(v[r], i + r);
+}
+
 // x * rms * w of a norm as a rounded f32 value in a register.  Every kernel that evaluates a norm -- stand-alone, as the
 // prologue of a product or as its epilogue -- goes through this, so that none of them has the product contracted into a
 // following addition or narrowed to f16 in one mixed-precision instruction while another has not (the results then

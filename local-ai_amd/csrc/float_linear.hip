@@ -930,7 +930,7 @@ __global__ __launch_bounds__(512) void matvec_bf16_part_kernel(const VectorStage
         mine = i == lane ? acc : mine;
     });
     sums[wave][lane] = mine;
-    lh_vector_barrier();
+    lh_lds_barrier();
     if (wave != 0) return;
     float t = 0.0f;
 #pragma unroll

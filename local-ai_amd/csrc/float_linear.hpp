@@ -61,7 +61,6 @@ __device__ __forceinline__ void lh_ld8(const uint16_t* p, float (&v)[8]) {
 // made: lanes and waves without a chunk load one that exists, and an operand that is not there is read from x.
 constexpr int kVectorWaves = 8;
 struct LhVectorSpace { float4 x[16][64]; float part[kVectorWaves]; };
-__device__ __forceinline__ void lh_vector_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Eight values at element k, stored as f32 or bf16.
 struct LhEither8 {
@@ -123,7 +122,7 @@ struct LhSharedVector {
             sum = lh_group_sum(sum, (int)width);
             if (width == 64) {
                 if (lane == 0) sp.part[wave] = sum;
-                lh_vector_barrier();
+                lh_lds_barrier();
                 const uint32_t per = parts ? cg >> 6 : (uint32_t)kVectorWaves, w0 = wave / per;
                 sum = 0.0f;
 #pragma unroll
@@ -147,7 +146,7 @@ struct LhSharedVector {
             sp.x[2 * wave][lane] = make_float4(v[0], v[1], v[2], v[3]);
             sp.x[2 * wave + 1][lane] = make_float4(v[4], v[5], v[6], v[7]);
         }
-        lh_vector_barrier();
+        lh_lds_barrier();
 #pragma unroll
         for (int c = 0; c < NL; c++) {
             const float4 a = sp.x[2 * c][lane], b = sp.x[2 * c + 1][lane];
@@ -155,30 +154,6 @@ struct LhSharedVector {
         }
     }
 };
-
-// Rows 0 .. count - 1 (at least one) of a walk with R of them on their way: issue(v, i) requests row i, use(v, i) multiplies it.
-template <int R, class V, class Issue>
-__device__ __forceinline__ void lh_first_rows(V (&v)[R], uint32_t count, Issue issue) {
-#pragma unroll
-    for (int r = 0; r < R; r++) issue(v[r], min((uint32_t)r, count - 1));
-}
-template <int R, class V, class Issue, class Use>
-__device__ __forceinline__ void lh_walk_rows(V (&v)[R], uint32_t count, Issue issue, Use use) {
-    uint32_t i = 0;
-    for (; i + 2 * R <= count; i += R) {
-#pragma unroll
-        for (int r = 0; r < R; r++) { use(v[r], i + r); issue(v[r], i + R + r); }
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++)
-        if (i + r < count) {
-            use(v[r], i + r);
-            if (i + R + r < count) issue(v[r], i + R + r);
-        }
-    i += R;
-#pragma unroll
-    for (int r = 0; r < R; r++) if (i + r < count) use(v[r], i + r);
-}
 
 static inline bool lh_stage_aligned(const VectorStage& st) {
     return (((uintptr_t)st.x | (uintptr_t)st.add | (uintptr_t)st.store | (uintptr_t)st.norm_weight | (uintptr_t)st.gate) & 15) == 0;

@@ -112,9 +112,6 @@ __device__ __forceinline__ float lh_block_sum(float v, float* scratch) {
     return t;
 }
 
-// Barrier over LDS accesses only: global loads that are on their way stay on their way.
-__device__ __forceinline__ void lh_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Maximum and sum over the four lanes that differ in their 16s and 32s (the column of a 16 x 16 matrix-product tile).
 // v_permlane16_swap / v_permlane32_swap on two copies leave the even and the odd rows (the lower and the upper half) of a
 // value in all rows (both halves).

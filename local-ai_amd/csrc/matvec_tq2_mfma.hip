@@ -464,6 +464,14 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
                               void* const* outputs, lh_dtype xt, lh_dtype yt, uint32_t rows, uint32_t K, uint32_t xstride,
                               uint32_t ystride, const XPrologue& pro, uint64_t mstride) {
     const bool strided = xstride != 0 || ystride != 0 || mstride != 0;   // problem i = problem 0 advanced by i strides: no descriptor table
+    // One vector of f16 values and not too many rows: the form without quantised activations.  (More than two grouped matrices inside a
+    // captured graph are refused below, evenly spaced or not.)
+    bool one_vector = xt == (pro.kind == kXProRotate ? LH_F32 : LH_F16) && yt == LH_F16 && count <= 8 && (!strided || count == 1) && (count <= 2 || !ctx->capturing);
+    for (uint32_t i = 1; one_vector && i < count; i++) one_vector = vectors[i] == vectors[0];
+    if (one_vector) {
+        const int r = lh_launch_matvec_tq2_direct(ctx, count, matrices, vectors[0], outputs, rows, K, pro);
+        if (r != -1) return r;
+    }
     const uint32_t nb = K >> 8;
     const uint64_t tiles = (uint64_t)((rows + 15) >> 4) * count;
     // small jobs: one wave per workgroup so the tiles spread over all CUs; large jobs: four waves share one
@@ -472,10 +480,6 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
     uint32_t split_waves = 1;
     if (tiles < (uint64_t)ctx->cu_count * 2) {
         for (uint32_t w = 4; w >= 2; w--) if (ngroups % w == 0) { split_waves = w; break; }
-        // six groups of blocks (12288 columns, the down projection of the wide feed-forward layers): a wave per group,
-        // and twice the threads for the activation staging (f16 in and out only: the decode path's types)
-        const size_t lds6 = lds_head_bytes(K) + 128 + 6 * (size_t)kImageBytes + 3 * kStageLoads * 64 * 2 + kSplitAreaBytes;
-        if (ngroups % 6 == 0 && xt == LH_F16 && yt == LH_F16 && lds6 <= kMaxLdsBytes) split_waves = 6;
     }
     const uint32_t splitk = split_waves > 1 ? 1u : 0u;
     constexpr int wg256_tiles_per_cu = 2, wg_cu = 3;
@@ -493,15 +497,6 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
         // the block groups of a tile on neighbouring waves: the segments of one row are then fetched close together in time
         if (ngroups > 1 && 12 % ngroups == 0) wide_split = ngroups;   // (one wave walking all groups of its tile: 0.65 against 0.71)
     }
-    // Few tiles, split over four waves each, f16 in and out, an even number of tiles (the decode path's down projection over
-    // 8192 columns): two tiles per workgroup of eight waves, so that twice the threads stage the activation vector and half
-    // as many workgroups stage it at all (a single-token decode layer: 64.4 -> 63.5 us).
-    bool pair_tiles = false;
-    if (splitk && split_waves == 4 && xt == LH_F16 && yt == LH_F16 && count == 1 && (((rows + 15) >> 4) & 1) == 0 && lds_for(8) <= kMaxLdsBytes) {
-        pair_tiles = true;
-        threads = 512;
-        wide_split = 4;
-    }
     const uint32_t waves = threads / 64;
     const uint32_t tiles_per_slot = wide_split ? waves / wide_split : (splitk ? 1u : waves);
     const uint64_t slots = (uint64_t)(((rows + 15) >> 4) + tiles_per_slot - 1) / tiles_per_slot * count;
@@ -514,14 +509,12 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
     if ((slots / grid + 1) * ngroups > 0xFFFFFFFFull)   // the kernel counts a workgroup's (tile, block group) items in 32 bits
         return lh_fail(LH_ERR_INVALID_ARGUMENT, "matvec_tq2_0: %u problems of %u rows are more than one launch takes", count, rows);
     const void* fn;
-    if (pair_tiles) fn = (const void*)matvec_tq2_mfma_kernel<uint16_t, uint16_t, true, 512>;
-    else if (split_waves == 6) fn = (const void*)matvec_tq2_mfma_kernel<uint16_t, uint16_t, true, 384>;
 #define LH_FN(XT, YT) (wide_split ? (const void*)matvec_tq2_mfma_kernel<XT, YT, true, 768, true>                                       \
                             : wide ? (const void*)matvec_tq2_mfma_kernel<XT, YT, false, 768>                                      \
                             : splitk ? (const void*)matvec_tq2_mfma_kernel<XT, YT, true>                                          \
                             : ngroups == 1 ? (const void*)matvec_tq2_mfma_kernel<XT, YT, false, 256, true>                        \
                                            : (const void*)matvec_tq2_mfma_kernel<XT, YT, false>)
-    else if (xt == LH_F32 && yt == LH_F32) fn = LH_FN(float, float);
+    if (xt == LH_F32 && yt == LH_F32) fn = LH_FN(float, float);
     else if (xt == LH_F16 && yt == LH_F16) fn = LH_FN(uint16_t, uint16_t);
     else if (xt == LH_F16 && yt == LH_F32) fn = LH_FN(uint16_t, float);
     else fn = LH_FN(float, uint16_t);

@@ -61,8 +61,8 @@ __device__ __forceinline__ void xpro_norm_add8(const void* xv, const XPrologue& 
 // 1/sqrt(head_dim) and the sign vector, rounded to f16 once: what hadamard_rotate_kernel<float, f16> stores, bit for bit
 // (the same butterflies in the same order of stages; a sum does not depend on which operand is named first).  Stages
 // 1, 2, 4 pair elements of one lane, the others pair the lanes of a head, head_dim / 8 <= 64 consecutive lanes of a wave.
-// Every lane of the wave calls it; lanes past the vector carry zeros.
-__device__ __forceinline__ void xpro_rotate8(float (&v)[8], const XPrologue& pro, uint32_t e0) {
+// Every lane of the wave calls it; lanes past the vector carry zeros.  s0, s1: the eight elements' signs.
+__device__ __forceinline__ void xpro_rotate8_regs(float (&v)[8], const XPrologue& pro, const float4 s0, const float4 s1) {
 #pragma unroll
     for (int len = 1; len < 8; len <<= 1) {
 #pragma unroll
@@ -82,11 +82,13 @@ __device__ __forceinline__ void xpro_rotate8(float (&v)[8], const XPrologue& pro
             v[i] = upper ? __fsub_rn(other, v[i]) : __fadd_rn(v[i], other);
         }
     }
-    const uint32_t d0 = e0 & (pro.head_dim - 1);
-    const float4 s0 = *reinterpret_cast<const float4*>(pro.signs + d0), s1 = *reinterpret_cast<const float4*>(pro.signs + d0 + 4);
     const float sg[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = lh_h2f(lh_f2h_exact(__fmul_rn(__fmul_rn(v[i], pro.scale), sg[i])));
+}
+__device__ __forceinline__ void xpro_rotate8(float (&v)[8], const XPrologue& pro, uint32_t e0) {
+    const float* s = pro.signs + (e0 & (pro.head_dim - 1));
+    xpro_rotate8_regs(v, pro, *reinterpret_cast<const float4*>(s), *reinterpret_cast<const float4*>(s + 4));
 }
 
 // Second level of the fixed point, for blocks whose first-level step would be too coarse.  A block with max|x| = m has
