@@ -723,6 +723,20 @@ int matvec_dispatch(lh_batch* batch, lh_quant fmt, uint32_t count, const lh_buff
                           (const char*)outputs[i]->ptr == y0 + (size_t)i * ystride;
         }
     }
+    // One vector of f16 values and not too many rows: the form without quantised activations.  (More than two grouped matrices inside a
+    // captured graph are refused below, unless they are evenly spaced.)
+    bool one_vector = xt == (pro.kind == kXProRotate ? LH_F32 : LH_F16) && yt == LH_F16 && count <= 8 && !regular && (count <= 2 || !ctx->capturing) &&
+                      !(fmt == LH_TQ2_0 && !tq2_on_matrix_cores());
+    for (uint32_t i = 1; one_vector && i < count; i++) one_vector = vectors[i]->ptr == vectors[0]->ptr;
+    if (one_vector) {
+        const void* pm[8]; void* py[8];
+        for (uint32_t i = 0; i < count; i++) { pm[i] = matrices[i]->ptr; py[i] = outputs[i]->ptr; }
+        const int r = lh_launch_matvec_direct(ctx, fmt, count, pm, vectors[0]->ptr, py, rows, cols, pro);
+        if (r != -1) {
+            if (r == LH_OK) batch->dispatch_count++;
+            return r;
+        }
+    }
     if (fmt == LH_TQ2_0 && tq2_on_matrix_cores() && cols <= 12288 && ((cols / 256) % 8 == 0 || min_slack >= 16)) {
         if (regular) {
             const void* pm1[1] = {matrices[0]->ptr}; const void* px1[1] = {vectors[0]->ptr}; void* py1[1] = {outputs[0]->ptr};

@@ -464,14 +464,6 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
                               void* const* outputs, lh_dtype xt, lh_dtype yt, uint32_t rows, uint32_t K, uint32_t xstride,
                               uint32_t ystride, const XPrologue& pro, uint64_t mstride) {
     const bool strided = xstride != 0 || ystride != 0 || mstride != 0;   // problem i = problem 0 advanced by i strides: no descriptor table
-    // One vector of f16 values and not too many rows: the form without quantised activations.  (More than two grouped matrices inside a
-    // captured graph are refused below, evenly spaced or not.)
-    bool one_vector = xt == (pro.kind == kXProRotate ? LH_F32 : LH_F16) && yt == LH_F16 && count <= 8 && (!strided || count == 1) && (count <= 2 || !ctx->capturing);
-    for (uint32_t i = 1; one_vector && i < count; i++) one_vector = vectors[i] == vectors[0];
-    if (one_vector) {
-        const int r = lh_launch_matvec_tq2_direct(ctx, count, matrices, vectors[0], outputs, rows, K, pro);
-        if (r != -1) return r;
-    }
     const uint32_t nb = K >> 8;
     const uint64_t tiles = (uint64_t)((rows + 15) >> 4) * count;
     // small jobs: one wave per workgroup so the tiles spread over all CUs; large jobs: four waves share one

@@ -204,40 +204,44 @@ def test_matvec_fused_prologues(pkg, gpu, oracle, fmt, rows, cols, count):
 
 @pytest.mark.parametrize("rows,cols,count", [(1, 256, 1), (3, 768, 2), (4095, 1536, 2), (4097, 2048, 1), (32768, 256, 1), (32770, 256, 1), (2049, 2304, 1), (700, 4096, 3),
                                              (515, 4352, 1), (1537, 6144, 1), (77, 8192, 2), (33, 10240, 1), (1030, 12288, 1), (9, 512, 8)])
+@pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
 @pytest.mark.parametrize("kind", ["none", "norm", "gelu", "rotate"])
-def test_tq2_products_of_one_vector(pkg, gpu, oracle, rows, cols, count, kind):
+def test_products_of_one_vector(pkg, gpu, oracle, fmt, rows, cols, count, kind):
     """Every split of a row over waves and of the vector over threads, odd row counts, more rows than waves, the largest job of the form
     without quantised activations and the smallest behind it; every prologue.  An f16 result is the nearest one up to the f32 sums:
     half an f16 step, and 2^-24 per addition (one per four products, five levels of lanes, six waves) of the terms' magnitude."""
     from oracle import layer_glue as G
     ctx, K = gpu
     g = pkg.synth.rng(77, rows + cols + count)
-    raws = [refgen.tq2_0_payload(min(rows, 2050), cols, 0x5A + i) for i in range(count)]
-    pick = np.arange(rows) % min(rows, 2050)
-    ws = [pkg.QuantWeight.from_bytes(ctx, np.ascontiguousarray(r.reshape(min(rows, 2050), -1)[pick]).reshape(-1), pkg.TQ2_0, rows, cols) for r in raws]
+    some, ty = min(rows, 2050), pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0
+    cols -= 64 if fmt == "q4_0" and kind != "rotate" and cols > 512 else 0          # a ragged last lane
+    payload, expand = (refgen.q4_0_payload, oracle.expand_q4_0_f32) if fmt == "q4_0" else (refgen.tq2_0_payload, oracle.expand_tq2_0_f32)
+    raws = [payload(some, cols, 0x5A + i) for i in range(count)]
+    pick = np.arange(rows) % some
+    ws = [pkg.QuantWeight.from_bytes(ctx, np.ascontiguousarray(r.reshape(some, -1)[pick]).reshape(-1), ty, rows, cols) for r in raws]
     x = g.standard_normal(cols, dtype=np.float32).astype(np.float16)
     aux = (1.0 + 0.2 * g.standard_normal(cols, dtype=np.float32)).astype(np.float16)
     outs, batch = [pkg.Buffer.empty(ctx, rows * 2) for _ in range(count)], pkg.CommandBatch(ctx)
     xb, ab = pkg.Buffer.from_slice(ctx, x), pkg.Buffer.from_slice(ctx, aux)
-    print(f"one vector {rows}x{cols} x{count} {kind}", flush=True)
+    print(f"one vector {fmt} {rows}x{cols} x{count} {kind}", flush=True)
     if kind == "rotate":
         if count > 1:
             return                                                    # a rotation takes one matrix
         signs = np.where(g.random(256) < 0.5, -1.0, 1.0).astype(np.float32)
         x32 = g.standard_normal(cols, dtype=np.float32)
         staged = oracle.hadamard_rotate(x32, signs, 256, cols // 256, False, True).astype(np.float16)
-        K.matvec_quant_rotated_into(batch, pkg.TQ2_0, ws[0].buf, pkg.Buffer.from_slice(ctx, x32), pkg.Buffer.from_slice(ctx, signs), 256, outs[0], rows, cols)
+        K.matvec_quant_rotated_into(batch, ty, ws[0].buf, pkg.Buffer.from_slice(ctx, x32), pkg.Buffer.from_slice(ctx, signs), 256, outs[0], rows, cols)
     elif kind == "none":
         staged = x
         for w, o in zip(ws, outs):
             w.matvec_into(batch, K, xb, o)
     else:
         staged = G.rms_norm(x, aux, cols, 1, 1e-6) if kind == "norm" else G.gelu_mul(x, aux)
-        K.matvec_quant_fused_into(batch, pkg.TQ2_0, [w.buf for w in ws], xb, K.PROLOGUE_RMS_NORM if kind == "norm" else K.PROLOGUE_GELU_MUL, ab, 1e-6, outs, rows, cols)
+        K.matvec_quant_fused_into(batch, ty, [w.buf for w in ws], xb, K.PROLOGUE_RMS_NORM if kind == "norm" else K.PROLOGUE_GELU_MUL, ab, 1e-6, outs, rows, cols)
     batch.commit_and_wait()
     v = staged.astype(np.float64)
     for r, o in zip(raws, outs):
-        dq = oracle.expand_tq2_0_f32(r, min(rows, 2050), cols).astype(np.float64)
+        dq = expand(r, some, cols).astype(np.float64)
         want, size = (dq @ v)[pick], (np.abs(dq) @ np.abs(v))[pick]
         tol = np.abs(want) * 2.0 ** -11 + size * (16 + 5 + 6) * 2.0 ** -24 + 2.0 ** -24
         if rows > 32768:                                              # the matrix-core form: 16-bit block fixed point of the vector
