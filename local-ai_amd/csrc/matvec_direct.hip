@@ -32,6 +32,7 @@ struct DirectArgs {
     uint16_t* y[8];
     const void* x;             // f16; before a rotation f32
     uint32_t count, rows, K;
+    uint32_t xstride, ystride; // bytes between the vectors of a batch and their outputs: vector blockIdx.y (one matrix, no prologue)
     XPrologue pro;
 };
 
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(MAXT) void matvec_direct_kernel(const DirectArgs a)
     uint4 va[NR], vb[NR];
     [[maybe_unused]] uint4 vr[NR], vg[NR];
     [[maybe_unused]] float4 sa[NR], sb[NR];
-    const uint16_t* const xh = static_cast<const uint16_t*>(a.x);
+    const uint16_t* const xh = reinterpret_cast<const uint16_t*>(static_cast<const char*>(a.x) + (size_t)blockIdx.y * a.xstride);
 #pragma unroll
     for (int i = 0; i < NR; i++) {
         const uint32_t e = min((i * nthreads + tid) * 8, a.K - 8);
@@ -228,14 +229,14 @@ __global__ __launch_bounds__(MAXT) void matvec_direct_kernel(const DirectArgs a)
     }
     if (l < count) {
         const uint32_t q = first + l * step, pr = problem(q), row = 2 * (q - pr * pairs) + half;
-        if (row < a.rows) a.y[pr][row] = lh_f2h(mine);
+        if (row < a.rows) reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(a.y[pr]) + (size_t)blockIdx.y * a.ystride)[row] = lh_f2h(mine);
     }
 }
 
 }  // namespace
 
 int lh_launch_matvec_direct(lh_context* ctx, lh_quant fmt, uint32_t count, const void* const* matrices, const void* vector, void* const* outputs, uint32_t rows,
-                                uint32_t K, const XPrologue& pro) {
+                                uint32_t K, const XPrologue& pro, uint32_t batch, uint32_t xstride, uint32_t ystride) {
     const uint32_t ng = (K + 2047) / 2048;
     if (count > 8 || ng > 6) return -1;
     const uint32_t waves = ng == 1 || ng == 2 || ng == 4 ? 8 : 2 * ng, teams = waves / ng, rounds = (ng * 2048 + waves * 512 - 1) / (waves * 512);   // rounds: 1 or 2
@@ -243,15 +244,19 @@ int lh_launch_matvec_direct(lh_context* ctx, lh_quant fmt, uint32_t count, const
     // matrix cores do the rest of the work for nothing: 65536 x 1536 (16 per wave) 13.1 us against 11.2 there, 32768 x 2048 (8) 8.3
     // against 8.7; 16384 x 12288 (16) 19.1 against 22.2.
     const uint64_t total = (uint64_t)((rows + 1) / 2) * count;
-    if (total > (uint64_t)ctx->cu_count * teams * (ng == 1 ? 8 : 16)) return -1;
-    const uint32_t grid = (uint32_t)std::min<uint64_t>((total + teams - 1) / teams, (uint64_t)ctx->cu_count);
-    DirectArgs a{{}, {}, vector, count, rows, K, pro};
+    // A batch of vectors, in microseconds against the form with v_dot4: up to 12 per wave 8 x 1536 x 12288 18.0 and 29.4, 4 x 12288 x 1536 11.3 and
+    // 12.8, 8 x 256 x 1536 3.7 and 4.7; 16 (8 x 8192 x 2048) 14.0 and 13.4, 24 (4 x 24576 x 1536) 19.6 and 18.6.
+    const uint32_t most = batch > 1 ? 12 : ng == 1 ? 8 : 16;
+    if (batch * total > (uint64_t)ctx->cu_count * teams * most) return -1;
+    const uint64_t fill = std::max<uint64_t>(batch == 1 ? ctx->cu_count : 2 * ctx->cu_count / batch, (total + (uint64_t)teams * most - 1) / ((uint64_t)teams * most));
+    const dim3 grid((uint32_t)std::min<uint64_t>((total + teams - 1) / teams, fill), batch);
+    DirectArgs a{{}, {}, vector, count, rows, K, xstride, ystride, pro};
     for (uint32_t i = 0; i < count; i++) { a.m[i] = (const uint8_t*)matrices[i]; a.y[i] = (uint16_t*)outputs[i]; }
     const size_t lds = (size_t)ng * 4096 + ((size_t)waves * 64 + 32) * 4;
 #define LH_DIRECT(FMT, KIND, NR)                                                                                                              \
     do {                                                                                                                                      \
-        if (waves <= 8) hipLaunchKernelGGL((matvec_direct_kernel<FMT, KIND, NR, 512>), dim3(grid), dim3(64 * waves), lds, ctx->stream, a);     \
-        else hipLaunchKernelGGL((matvec_direct_kernel<FMT, KIND, NR, 768>), dim3(grid), dim3(64 * waves), lds, ctx->stream, a);                \
+        if (waves <= 8) hipLaunchKernelGGL((matvec_direct_kernel<FMT, KIND, NR, 512>), grid, dim3(64 * waves), lds, ctx->stream, a);     \
+        else hipLaunchKernelGGL((matvec_direct_kernel<FMT, KIND, NR, 768>), grid, dim3(64 * waves), lds, ctx->stream, a);                \
     } while (0)
 #define LH_DIRECT_KIND(FMT, KIND) do { if (rounds == 1) LH_DIRECT(FMT, KIND, 1); else LH_DIRECT(FMT, KIND, 2); } while (0)
 #define LH_DIRECT_FMT(FMT)                                                    \

@@ -821,6 +821,11 @@ int matvec_rows_impl(lh_batch* batch, lh_quant fmt, uint32_t m, const lh_buffer*
     const size_t wbytes = (size_t)n * (k / blk) * (fmt == LH_Q4_0 ? 18 : 66);
     const size_t slack = weight->len - wbytes + weight->slack;
     int r;
+    if (at == LH_F16 && ct == LH_F16 && !(fmt == LH_TQ2_0 && !tq2_on_matrix_cores())) {
+        const void* pm[1] = {weight->ptr}; void* py[1] = {output->ptr};
+        r = lh_launch_matvec_direct(ctx, fmt, 1, pm, input->ptr, py, n, k, XPrologue{kXProNone, nullptr, 0.0f}, m, (uint32_t)xstride, (uint32_t)ystride);
+        if (r != -1) return r;
+    }
     if (fmt == LH_TQ2_0 && tq2_on_matrix_cores() && k <= 12288 && ((k / 256) % 8 == 0 || slack >= 16)) {
         const void* pm[1] = {weight->ptr}; const void* px[1] = {input->ptr}; void* py[1] = {output->ptr};
         r = lh_launch_matvec_tq2_mfma(ctx, m, pm, px, py, at, ct, n, k, (uint32_t)xstride, (uint32_t)ystride);

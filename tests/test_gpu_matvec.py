@@ -255,6 +255,31 @@ def test_products_of_one_vector(pkg, gpu, oracle, fmt, rows, cols, count, kind):
         assert np.all(np.abs(got - want) <= tol), (worst, got[worst], want[worst], tol[worst])
 
 
+@pytest.mark.parametrize("rows,cols,m", [(1, 64, 2), (257, 1536, 3), (4096, 2048, 4), (1536, 6144, 8), (700, 8256, 5), (6144, 2048, 8), (6150, 2048, 8)])
+def test_vectors_of_a_batch_as_single_ones(pkg, gpu, oracle, rows, cols, m):
+    """A few f16 vectors against one 4-bit matrix give what each gives alone, bit for bit, where both take the form without quantised
+    activations (6150 rows of eight vectors do not).  All are held to the f64 dot: half an f16 step, and 2^-15 of the terms' magnitude for
+    the other form's 16-bit fixed point."""
+    ctx, K = gpu
+    g = pkg.synth.rng(78, rows + cols + m)
+    raw = refgen.q4_0_payload(rows, cols, 0x33)
+    w = pkg.QuantWeight.from_bytes(ctx, raw, pkg.Q4_0, rows, cols)
+    x = g.standard_normal((m, cols), dtype=np.float32).astype(np.float16)
+    y, batch = pkg.Buffer.empty(ctx, m * rows * 2), pkg.CommandBatch(ctx)
+    print(f"batch of vectors {rows}x{cols} m{m}", flush=True)
+    w.matmul_nt_into(batch, K, pkg.Buffer.from_slice(ctx, x), y, m)
+    single = [pkg.Buffer.empty(ctx, rows * 2) for _ in range(m)]
+    for i, o in enumerate(single):
+        w.matvec_into(batch, K, pkg.Buffer.from_slice(ctx, x[i]), o)
+    batch.commit_and_wait()
+    got, dq = y.as_array(np.float16, m * rows).reshape(m, rows), oracle.expand_q4_0_f32(raw, rows, cols).astype(np.float64)
+    want, size = x.astype(np.float64) @ dq.T, np.abs(x.astype(np.float64)) @ np.abs(dq).T
+    assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -11 + size * 2.0 ** -15 + 2.0 ** -24)
+    for i, o in enumerate(single):
+        if rows != 6150:
+            assert np.array_equal(got[i].view(np.uint16), o.as_array(np.uint16, rows))
+
+
 @pytest.mark.parametrize("fmt,rows,cols,count", [("q4_0", 256, 2048, 1), ("tq2_0", 8192, 2048, 2), ("tq2_0", 300, 512, 2),
                                                  ("q4_0", 64, 8192, 1)])
 @pytest.mark.parametrize("second_norm", [True, False])
