@@ -229,6 +229,12 @@ class Buffer:
         _check(lib().lh_buffer_read(self._h, C.c_size_t(offset), C.c_void_p(out.ctypes.data), C.c_size_t(out.nbytes)))
         return out
 
+    def read_into(self, out: np.ndarray, offset: int = 0) -> None:
+        """The first bytes from `offset` into a contiguous array of the caller's."""
+        if not out.flags.c_contiguous or not out.flags.writeable:
+            raise InvalidArgument("read_into needs a contiguous array that can be written")
+        _check(lib().lh_buffer_read(self._h, C.c_size_t(offset), C.c_void_p(out.ctypes.data), C.c_size_t(out.nbytes)))
+
     def fill_zero(self) -> None:
         _check(lib().lh_buffer_fill_zero(self._h))
 
@@ -258,6 +264,11 @@ class CommandBatch:
     def blit_copy(self, src: Buffer, src_offset: int, dst: Buffer, dst_offset: int, length: int) -> None:
         _check(lib().lh_batch_blit_copy(self._h, src._h, C.c_size_t(src_offset), dst._h, C.c_size_t(dst_offset),
                                         C.c_size_t(length)))
+
+    def write(self, dst: Buffer, src, offset: int = 0) -> None:
+        """Host data for `dst` in the order of the batch's dispatches; no wait up to 2 KB."""
+        a = np.ascontiguousarray(src)
+        _check(lib().lh_batch_write(self._h, dst._h, C.c_size_t(offset), C.c_void_p(a.ctypes.data), C.c_size_t(a.nbytes)))
 
     def commit_and_wait(self) -> None:
         _check(lib().lh_batch_commit_and_wait(self._h))

@@ -108,6 +108,20 @@ int lh_check_fault_word(lh_context* ctx) {
     return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: a kernel reported fault code %u", code);
 }
 
+// ---- small writes: host words that travel as kernel arguments (lh_batch_write) ----
+template <int N> struct SentWords { uint32_t w[N]; };
+template <class W>
+__global__ __launch_bounds__(256) static void write_words_kernel(const W, uint8_t* to, uint32_t len) {
+    // the words are read where the arguments lie: they are the first of them
+    const auto* from = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+    for (uint32_t i = threadIdx.x; 4 * i < len; i += 256) {
+        const uint32_t v = from[i], at = 4 * i;
+        if (at + 4 <= len && ((uintptr_t)to & 3) == 0) *reinterpret_cast<uint32_t*>(to + at) = v;
+        else
+            for (uint32_t b = 0; b < 4 && at + b < len; b++) to[at + b] = (uint8_t)(v >> (8 * b));
+    }
+}
+
 extern "C" {
 
 const char* lh_last_error(void) { return g_last_error; }
@@ -410,6 +424,28 @@ int lh_batch_blit_copy(lh_batch* batch, const lh_buffer* src, size_t src_offset,
     int r = lh_check_launch("blit_copy");
     if (r == LH_OK) batch->dispatch_count++;
     return r;
+}
+
+// A few words (a token, the rows of a portion) as the arguments of a one-workgroup launch: the copy engine with a wait behind it holds a
+// step up for 14 us, this for 4.
+int lh_batch_write(lh_batch* batch, lh_buffer* dst, size_t offset, const void* src, size_t len) {
+    if (!batch || !dst || (!src && len)) return lh_fail(LH_ERR_INVALID_ARGUMENT, "batch_write: null argument");
+    if (batch->ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "batch_write: not while a graph is being captured");
+    if (offset > dst->len || len > dst->len - offset)
+        return lh_fail(LH_ERR_INVALID_ARGUMENT, "batch_write: range %zu+%zu exceeds %zu", offset, len, dst->len);
+    if (!len) return LH_OK;
+    char* to = (char*)dst->ptr + offset;
+    const auto send = [&](auto words) {
+        memcpy(words.w, src, len);
+        hipLaunchKernelGGL(write_words_kernel<decltype(words)>, dim3(1), dim3(256), 0, batch->ctx->stream, words, (uint8_t*)to, (uint32_t)len);
+        return lh_check_launch("batch_write");
+    };
+    if (dst->ctx == batch->ctx && len <= sizeof(SentWords<16>)) return send(SentWords<16>{});
+    if (dst->ctx == batch->ctx && len <= sizeof(SentWords<512>)) return send(SentWords<512>{});
+    hipError_t e = hipMemcpyAsync(to, src, len, hipMemcpyHostToDevice, batch->ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(batch->ctx->stream);
+    if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: batch_write: %s", hipGetErrorString(e));
+    return LH_OK;
 }
 
 int lh_batch_commit_and_wait(lh_batch* batch) {

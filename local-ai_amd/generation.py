@@ -152,7 +152,7 @@ class PipelineSequences:
                 seq.decode_step(int(tokens[lo]))
                 for i, p in enumerate(want):
                     if p == lo:
-                        out[i] = seq.logits()
+                        seq.logits_buf.read_into(out[i])
                 lo += 1
                 continue
             hi = min([p for p in want if p > lo] + [last, lo + seq.max_batch])

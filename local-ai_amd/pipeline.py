@@ -309,13 +309,13 @@ class DecodePipeline:
         and the per-layer inputs of every row into ple_all.  Returns whether per-layer inputs exist."""
         cfg, K, bs = self.config, self.kernels, self.batch_scratch
         n, h = len(tokens), cfg.hidden_size
-        self._tokens_buf.copy_from_bytes(np.asarray(tokens, np.uint32))
+        batch.write(self._tokens_buf, np.asarray(tokens, np.uint32))
         self.token_embd.dequant_rows_into(batch, K, self._tokens_buf, n, bs.hidden_a, math.sqrt(h))
         if self.per_layer_input is None:
             return False
         pld, nl = cfg.hidden_size_per_layer_input, cfg.num_hidden_layers
         total = n * pld * nl
-        self._ple_tokens_buf.copy_from_bytes(np.asarray(ple_tokens, np.uint32))
+        batch.write(self._ple_tokens_buf, np.asarray(ple_tokens, np.uint32))
         self.ple_table.dequant_rows_into(batch, K, self._ple_tokens_buf, n, bs.ple_tok, math.sqrt(pld))
         self.per_layer_model_proj.matmul_nt_into(batch, K, bs.hidden_a, bs.ple_proj, n)
         K.scale_in_place_gpu_into(batch, bs.ple_proj, 1.0 / math.sqrt(h), total)
@@ -432,8 +432,8 @@ class DecodePipeline:
         for lane, pos in enumerate(positions):
             if pos >= state.lane_capacity:
                 raise InvalidArgument(f"lane {lane} position {pos} exceeds capacity {state.lane_capacity}")
-        state.pos_buf.copy_from_bytes(np.asarray(positions, np.uint32))
         batch = CommandBatch(self.ctx)
+        batch.write(state.pos_buf, np.asarray(positions, np.uint32))
         self._embed_rows(batch, tokens, ple_tokens)
         self.encode_batch_step(batch, state, n)
         batch.commit_and_wait()

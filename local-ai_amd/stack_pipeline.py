@@ -117,8 +117,9 @@ class StackPipeline:
         for lo in range(0, n, self.max_rows):
             hi = min(lo + self.max_rows, n)
             at = [i for i, p in enumerate(want) if lo <= p < hi]
-            got = self._forward(seq, tokens[lo:hi], [want[i] - lo for i in at])
-            if at:
+            got = out if len(at) == len(want) else np.empty((len(at), self.vocab_size), np.float32)
+            self._forward(seq, tokens[lo:hi], [want[i] - lo for i in at], got)
+            if at and got is not out:
                 out[at] = got
         return out
 
@@ -126,8 +127,10 @@ class StackPipeline:
         """One decoded token whose successor is picked on the device."""
         if seq.position + 1 > self.max_tokens:
             raise InvalidArgument(f"position {seq.position + 1} beyond the {self.max_tokens} tokens of a sequence")
-        self._decode(seq, token)
-        return int(self.next_buf.as_array(np.uint32, 1)[0])
+        batch = self._decode(seq, token)
+        picked = int(self.next_buf.as_array(np.uint32, 1)[0])
+        self._finish(batch, seq, 1)
+        return picked
 
     # ---- encoding -------------------------------------------------------------------------------------------------------
     def _encode_stack(self, batch, seq: SequenceSlot, n: int, max_position: int) -> Buffer:
@@ -150,14 +153,18 @@ class StackPipeline:
         Norm.flush(r)
         return r.x
 
-    def _forward(self, seq: SequenceSlot, tokens, want) -> Optional[np.ndarray]:
+    def _forward(self, seq: SequenceSlot, tokens, want, out: np.ndarray) -> None:
+        """Results are read behind the work, in stream order: one wait for both."""
         n = len(tokens)
         if n == 1 and self.observe is None:
-            self._decode(seq, int(tokens[0]))
-            return np.repeat(self.logits_buf.as_array(np.float32, self.vocab_size)[None], len(want), 0) if want else None
+            batch = self._decode(seq, int(tokens[0]))
+            if want:
+                self.logits_buf.read_into(out[0])
+                out[1:] = out[0]
+            return self._finish(batch, seq, 1)
         K, width = self.kernels, self.config.width
-        self.tokens_buf.copy_from_bytes(np.asarray(tokens, np.uint32))
         batch = CommandBatch(self.ctx)
+        batch.write(self.tokens_buf, np.asarray(tokens, np.uint32))
         x = self._encode_stack(batch, seq, n, seq.position)
         K.advance_position_into(batch, seq.position_buf, n)
         logits = None
@@ -167,16 +174,20 @@ class StackPipeline:
         elif want:
             m = len(want)
             index = self.ws.get("want", 4 * self.max_rows)
-            index.copy_from_bytes(np.asarray(want, np.uint32))
+            batch.write(index, np.asarray(want, np.uint32))
             logits = self.ws.get("logits", m * self.vocab_size * 4)
             size = 4 if self.dtype == F32 else 2
             h = self.ws.get("wanted", m * width * size)
             K.norm_rows_f32_into(batch, x, None, self.final_norm.weight, None, index, h, self.dtype, width, m, self.config.eps)
             self.head.rows_into(batch, K, h, self.dtype, m, [logits], F32)
             self._encode_cap(batch, logits, m)
+        if want:
+            logits.read_into(out)
+        self._finish(batch, seq, n)
+
+    def _finish(self, batch, seq: SequenceSlot, n: int) -> None:
         batch.commit_and_wait()
         seq.position += n
-        return logits.as_array(np.float32, len(want) * self.vocab_size).reshape(len(want), -1) if want else None
 
     def _encode_head(self, batch, row: Buffer) -> None:
         self.head.normed_vector_into(batch, self.kernels, row, self.final_norm.weight, self.config.eps, [self.logits_buf], F32)
@@ -191,12 +202,12 @@ class StackPipeline:
         self.kernels.argmax_rows_f32_into(batch, self.logits_buf, self.next_buf, 1, self.vocab_size)
         self.kernels.advance_position_into(batch, seq.position_buf, 1)
 
-    def _decode(self, seq: SequenceSlot, token: int) -> None:
-        """One token: logits in logits_buf, the largest one's index in next_buf.  The first decoded token of a slot runs
+    def _decode(self, seq: SequenceSlot, token: int) -> CommandBatch:
+        """One token, encoded: logits in logits_buf, the largest one's index in next_buf.  The first decoded token of a slot runs
         dispatch by dispatch, the next one records the step into a graph that later ones replay as long as the scratch buffers
         stay where they are (everything that changes from step to step is in device memory)."""
-        self.tokens_buf.copy_from_bytes(np.asarray([token], np.uint32))
         batch = CommandBatch(self.ctx)
+        batch.write(self.tokens_buf, np.asarray([token], np.uint32))
         if seq.graph is not None and seq.graph_version == self.ws.version:
             seq.graph.launch()
         elif self.graphs and seq.graph_ready:
@@ -212,5 +223,4 @@ class StackPipeline:
         else:
             self._encode_decode(batch, seq, seq.position)
             seq.graph_ready = True
-        batch.commit_and_wait()
-        seq.position += 1
+        return batch

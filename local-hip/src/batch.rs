@@ -1,6 +1,7 @@
 //! `CommandBatch`: the dispatches of one step on the context's in-order stream, behind the method names of
 //! `local_metal::CommandBatch` (local-metal/src/batch.rs:147-291).  Metal encodes into a command buffer and runs it at
 //! commit; here a dispatch starts as soon as it is encoded and `commit_and_wait` is the wait.
+use core::ffi::c_void;
 use core::ptr;
 
 use crate::buffer::Buffer;
@@ -49,6 +50,11 @@ impl CommandBatch {
 
     /// `commit_and_wait()` (batch.rs:240-250).  The reference consumes the batch; this one stays usable, which is what
     /// `commit_and_renew` gives there.
+    /// Host bytes for `dst` in the order of the batch's dispatches; no wait up to 2 KB.
+    pub fn write(&mut self, dst: &Buffer, offset: usize, src: &[u8]) -> Result<()> {
+        check(unsafe { ffi::lh_batch_write(self.raw, dst.as_ptr(), offset, src.as_ptr() as *const c_void, src.len()) })
+    }
+
     pub fn commit_and_wait(&mut self) -> Result<()> {
         // SAFETY: live handle.
         check(unsafe { ffi::lh_batch_commit_and_wait(self.raw) })

@@ -69,6 +69,7 @@ extern "C" {
     pub fn lh_batch_free(batch: *mut lh_batch);
     pub fn lh_batch_dispatch_count(batch: *const lh_batch) -> u32;
     pub fn lh_batch_blit_copy(batch: *mut lh_batch, src: *const lh_buffer, src_offset: usize, dst: *mut lh_buffer, dst_offset: usize, len: usize) -> c_int;
+    pub fn lh_batch_write(batch: *mut lh_batch, dst: *mut lh_buffer, offset: usize, src: *const c_void, len: usize) -> c_int;
     pub fn lh_batch_commit_and_wait(batch: *mut lh_batch) -> c_int;
     pub fn lh_debug_set_tq2_split_spin_limit(polls: u32);
     pub fn lh_debug_set_attention_pair_spin_limit(polls: u32);

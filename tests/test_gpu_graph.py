@@ -150,3 +150,32 @@ def test_graph_released_during_capture_does_not_disturb_it(pkg, gpu):
         ctx.synchronize()
         assert (out.as_array(np.float16, n) == 3.0 + 3 * step).all()
     graph.free()
+
+
+@pytest.mark.parametrize("size", [1, 3, 4, 63, 64, 65, 1028, 2047, 2048, 2049, 5001])
+@pytest.mark.parametrize("offset", [0, 1, 4, 6])
+def test_host_bytes_in_the_order_of_the_batch(pkg, gpu, size, offset):
+    """CommandBatch.write: as kernel arguments up to 2 KB and copied beyond, in order with the dispatches around it, from a source that
+    is overwritten at once; what lies around the range stays, and it is refused past the end and while a graph is recorded."""
+    ctx, K = gpu
+    g = pkg.synth.rng(5, size + offset)
+    first, second = (g.integers(0, 256, size, dtype=np.uint8) for _ in range(2))
+    a, b, batch = pkg.Buffer.from_slice(ctx, np.full(6000, 7, np.uint8)), pkg.Buffer.empty(ctx, 6000), pkg.CommandBatch(ctx)
+    src = first.copy()
+    batch.write(a, src, offset)
+    src[:] = second
+    batch.blit_copy(a, 0, b, 0, 6000)
+    batch.write(a, src, offset)
+    batch.commit_and_wait()
+    for buf, want in ((a, second), (b, first)):
+        got, around = buf.as_array(np.uint8), np.full(6000, 7, np.uint8)
+        around[offset:offset + size] = want
+        assert np.array_equal(got, around)
+    with pytest.raises(pkg.InvalidArgument):
+        batch.write(a, src, 6001 - size)
+    batch.begin_capture()
+    with pytest.raises(pkg.InvalidArgument):
+        batch.write(a, src, 0)
+    batch.end_capture()
+    batch.write(a, src, 0)
+    batch.commit_and_wait()
