@@ -921,6 +921,172 @@ __global__ __launch_bounds__(256, 2) void matmul_skinny_kernel(const uint16_t* _
     }
 }
 
+// ---- the same rows against many weight rows: activations shared by a workgroup ----------------------------------------------------
+// With enough 64-row blocks for every CU no product needs its k range split over waves: here the four waves of a workgroup take 64
+// weight rows each (PAIR: 32 of gate and the same 32 of up) over all of k and share the activations, which come in 128 columns at a
+// time into one of two LDS buffers in the fragment order of matmul_skinny_kernel.  A workgroup per 64 rows reads all
+// activations from L2 for itself and adds four partial tiles through LDS: 64 x 1536 x 262144 (Q4_0, f32 out) 176 us, here 95; 256 rows,
+// gate and up of 12288 x 1536 (TQ2_0) 39 and 34.
+// The codes are two steps ahead in registers, the activations one in registers and one in LDS; one barrier per step.
+template <int FMT, int CDT, bool PAIR>
+__global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W_one, void* __restrict__ C_one, uint32_t M,
+                                                            uint32_t K, uint32_t N_one, uint32_t blocks, GroupArgs grp) {
+    constexpr int UK = Skinny<FMT>::unit_k, NF = Skinny<FMT>::frags, UNITS = 128 / UK;       // units of codes per step
+    __shared__ f32x4 stage[2][16 * 64];                       // [buffer][fragment f of the step, activation group j][cell]
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const uint32_t block = blockIdx.x * 4 + wave;             // a workgroup's last waves may have none: they only bring in activations
+    const bool on = block < blocks;
+    const uint8_t* W = W_one;
+    void* C = C_one;
+    uint32_t N = N_one, tile = (on ? block : blocks - 1) >> 1;
+    if (!PAIR && grp.count) {
+        const uint32_t gi = group_of_tile(grp, tile);
+        W = grp.W[gi]; C = grp.C[gi]; N = grp.N[gi];
+        tile -= grp.tile0[gi];
+    }
+    const uint32_t n0 = PAIR ? (on ? block : blocks - 1) * 32 : tile * BN + ((on ? block : blocks - 1) & 1) * 64;
+    const size_t row_bytes = FMT == kQ4 ? (size_t)(K >> 5) * 18 : (size_t)(K >> 8) * 66, tile_bytes = 16 * row_bytes;
+    const uint32_t m0 = blockIdx.y * 64;
+
+    // Codes: the 64 rows' bytes of a step (Q4_0: 72 a row; TQ2_0: 32 of codes, and the scale of the block by itself) come in with coalesced
+    // loads, consecutive lanes along a row, and are parked in the wave's own LDS area, from which every lane takes what it multiplies.
+    // (A lane loading its eight bytes itself costs a cache access per lane, one per clock and CU: 135 us where this takes 95.)
+    constexpr uint32_t PIECES = FMT == kQ4 ? 9 : 4, PITCH = FMT == kQ4 ? 76 : 36, NL = PIECES;     // 8-byte pieces per row; bytes per row in LDS (an odd number of words); loads of 64 lanes
+    __shared__ __align__(16) uint8_t codes[4][64 * PITCH];
+    uint8_t* const mine = codes[wave];
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    typedef u32x2_t __attribute__((aligned(2))) u32x2_a2;
+    // row of a workgroup's 64: rows 0..31 gate, 32..63 up of a pair
+    const uint8_t *wrow = W + (size_t)n0 * row_bytes, *wrow_up = PAIR ? grp.W[1] + (size_t)n0 * row_bytes : nullptr;
+    uint32_t c_at[NL], c_to[NL];
+#pragma unroll
+    for (uint32_t i = 0; i < NL; i++) {
+        const uint32_t at = 64 * i + lane, row = at / PIECES, piece = at - row * PIECES;
+        c_at[i] = (PAIR ? row & 31 : row) * (uint32_t)row_bytes + 8 * piece;
+        c_to[i] = row * PITCH + 8 * piece;
+    }
+    struct Codes { u32x2_t w[NL]; uint32_t d; } ra[2];
+    auto load_a = [&](Codes& raw, uint32_t k0) {
+        const size_t at = FMT == kQ4 ? (size_t)(k0 >> 6) * 36 : (size_t)(k0 >> 8) * 66, half = FMT == kQ4 ? 0 : 32 * ((k0 >> 7) & 1);
+#pragma unroll
+        for (uint32_t i = 0; i < NL; i++) {
+            // (pair: with 64 rows of PIECES pieces, load i is of gate rows in its first half and of up rows in its second)
+            const uint8_t* p = PAIR ? (c_to[i] >= 32 * PITCH ? wrow_up : wrow) : wrow;
+            raw.w[i] = *reinterpret_cast<const u32x2_a2*>(p + at + half + c_at[i]);
+        }
+        if constexpr (FMT == kTQ2) raw.d = *reinterpret_cast<const uint16_t*>((PAIR ? (lane >= 32 ? wrow_up : wrow) : wrow) + at + 64 + (PAIR ? lane & 31 : lane) * (uint32_t)row_bytes);
+    };
+    auto park_a = [&](const Codes& raw) {
+#pragma unroll
+        for (uint32_t i = 0; i < NL; i++) { *reinterpret_cast<uint32_t*>(mine + c_to[i]) = raw.w[i].x; *reinterpret_cast<uint32_t*>(mine + c_to[i] + 4) = raw.w[i].y; }
+        if constexpr (FMT == kTQ2) *reinterpret_cast<uint16_t*>(mine + lane * PITCH + 32) = (uint16_t)raw.d;
+    };
+    // the lane's codes and scale of unit v of the parked step, row r of tile t
+    auto take = [&](int v, int t) {
+        const uint8_t* p = mine + (16 * t + r) * PITCH;
+        SkinnyRaw c;
+        if constexpr (FMT == kQ4) {
+            const uint32_t* q = reinterpret_cast<const uint32_t*>(p + 36 * v + (g < 2 ? 8 * g : 8 * g + 4));      // blocks at bytes 0 and 18 of the 36: codes from byte 2, 10, 20, 28
+            const uint32_t a = q[0], b = q[1], e = q[g < 2 ? 2 : 1], sh = g < 2 ? 16 : 0;
+            c.w0 = __builtin_amdgcn_alignbit(b, a, sh);
+            c.w1 = __builtin_amdgcn_alignbit(e, b, sh);
+            c.d = *reinterpret_cast<const uint16_t*>(p + 36 * v + 18 * (g >> 1)) * 0x10001u;
+        } else {
+            const uint32_t* q = reinterpret_cast<const uint32_t*>(p + 8 * g);
+            c.w0 = q[0]; c.w1 = q[1];
+            c.d = *reinterpret_cast<const uint16_t*>(p + 32) * 0x10001u;
+        }
+        return c;
+    };
+    const uint32_t ld_row = tid >> 4, ld_q = tid & 15;
+    const uint32_t ld_f = FMT == kQ4 ? 2 * (ld_q >> 3) + ((ld_q & 3) >> 1) : ld_q >> 2, ld_g = FMT == kQ4 ? 2 * ((ld_q >> 2) & 1) + (ld_q & 1) : ld_q & 3;
+    const uint32_t cell = ld_f * 256 + ld_g * 16 + (ld_row ^ (ld_g | ((ld_f & 1) << 2)));
+    uint32_t x_at[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) x_at[j] = (std::min(m0 + 16 * j + ld_row, M - 1) * K + 8 * ld_q) * 2;      // rows past M repeat the last one
+    f32x4 rb[4];
+    auto load_b = [&](uint32_t k0) {
+        const char* base = reinterpret_cast<const char*>(X) + (size_t)k0 * 2;
+#pragma unroll
+        for (int j = 0; j < 4; j++) rb[j] = *reinterpret_cast<const f32x4*>(base + x_at[j]);
+    };
+    auto park_b = [&](f32x4* to) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) to[cell + 64 * j] = rb[j];
+    };
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const f32x4* from) {
+        SkinnyRaw c[4];
+#pragma unroll
+        for (int f = 0; f < 4; f++) {
+            if (f % NF == 0)
+#pragma unroll
+                for (int t = 0; t < 4; t++) c[t] = take(f / NF, t);
+            f16x8 bf[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) bf[j] = __builtin_bit_cast(f16x8, from[(f * 4 + j) * 64 + g * 16 + (r ^ (g | ((f & 1) << 2)))]);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const f16x8 a = skinny_fragment<FMT>(c[t], f % NF);
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bf[j], acc[t][j], 0, 0, 0);
+            }
+        }
+    };
+
+    const uint32_t steps = K >> 7, last = K - 128;            // loads past the end re-read the last step
+    load_b(0);
+    load_a(ra[0], 0);
+    load_a(ra[1], std::min(128u, last));
+    park_b(stage[0]);
+    load_b(std::min(128u, last));
+    lh_lds_barrier();
+    auto step = [&](auto set_tag, uint32_t s) {
+        constexpr int set = decltype(set_tag)::value;
+        park_b(stage[set ^ 1]);                               // read last in the step before, behind its barrier
+        load_b(std::min((s + 2) * 128, last));
+        park_a(ra[set]);                                      // the wave's own area: its last reads are behind it
+        load_a(ra[set], std::min((s + 2) * 128, last));
+        multiply(stage[set]);
+        lh_lds_barrier();
+    };
+    for (uint32_t s = 0; s < steps; s += 2) { step(std::integral_constant<int, 0>{}, s); step(std::integral_constant<int, 1>{}, s + 1); }      // K: a multiple of 256
+    if (!on) return;
+
+    // D[row 4g + i of tile t][activation row r of group j]
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t m = m0 + 16 * j + r;
+        if (m >= M) continue;
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                uint16_t h[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) h[i] = lh_gelu_mul_h(lh_f2h(acc[t][j][i]), lh_f2h(acc[t + 2][j][i]));
+                *reinterpret_cast<uint2*>(static_cast<uint16_t*>(grp.C[0]) + (size_t)m * grp.N[0] + n0 + 16 * t + 4 * g) =
+                    make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const f32x4 v = acc[t][j];
+                const size_t at = (size_t)m * N + n0 + 16 * t + 4 * g;
+                if constexpr (CDT == LH_F32) *reinterpret_cast<f32x4*>(static_cast<float*>(C) + at) = v;
+                else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(C) + at) = make_uint2(pack_h2(v[0], v[1]), pack_h2(v[2], v[3]));
+            }
+        }
+    }
+}
+
+// Whether `blocks` 64-row blocks (pairs: of 32) times the groups of 64 activation rows give every CU a workgroup of the above; with
+// fewer, k split over the waves is the shorter way (256 rows, gate and up of 6144 x 1536: 192 workgroups, 21.7 us split).
+bool wide_pays(const lh_context* ctx, uint32_t blocks, uint32_t mgroups) { return (uint64_t)((blocks + 3) / 4) * mgroups >= (uint64_t)ctx->cu_count; }
+
 // Most activation rows the skinny kernel takes (256: a prefill chunk).  Beyond 64 rows
 // every group of 64 gets workgroups of its own, which re-read the codes from L2 while the activation traffic grows with
 // rows x weight rows; measured on a 256-row chunk of the layer bench: 197 -> 163 us per layer, no gain at 512 rows.
@@ -1112,7 +1278,11 @@ bool try_skinny(lh_context* ctx, const void* A, const uint8_t* W, void* C, lh_dt
             float* partial = (splits > 1 || keep) ? static_cast<float*>(ctx->workspace) : nullptr;
             const dim3 grid(blocks, mgroups, splits);
             const uint16_t* X = static_cast<const uint16_t*>(A);
-            if (FMT == kQ4 && m <= (uint32_t)kMaxMultivecM) {   // unrounded weights for the small batches (2 blocks per unit)
+            if (!keep && splits == 1 && !(FMT == kQ4 && m <= (uint32_t)kMaxMultivecM) && wide_pays(ctx, blocks, mgroups)) {
+                const dim3 wide((blocks + 3) / 4, mgroups);
+                if (ct == LH_F32) hipLaunchKernelGGL((matmul_wide_kernel<FMT, LH_F32, false>), wide, dim3(256), 0, s, X, W, C, m, k, n, blocks, grp);
+                else hipLaunchKernelGGL((matmul_wide_kernel<FMT, LH_F16, false>), wide, dim3(256), 0, s, X, W, C, m, k, n, blocks, grp);
+            } else if (FMT == kQ4 && m <= (uint32_t)kMaxMultivecM) {   // unrounded weights for the small batches (2 blocks per unit)
                 if (ct == LH_F32) hipLaunchKernelGGL((matmul_small_q4_kernel<LH_F32>), grid, dim3(256), 0, s, X, W, C, m, k, n, partial, 2 * (per_wg / splits), grp);
                 else hipLaunchKernelGGL((matmul_small_q4_kernel<LH_F16>), grid, dim3(256), 0, s, X, W, C, m, k, n, partial, 2 * (per_wg / splits), grp);
             } else if (ct == LH_F32) hipLaunchKernelGGL((matmul_skinny_kernel<FMT, LH_F32>), grid, dim3(256), 0, s, X, W, C, m, k, n, partial, per_wg / splits, grp);
@@ -1544,7 +1714,11 @@ int lh_matmul_nt_quant_gelu_mul_into(lh_batch* b, lh_quant fmt, const lh_buffer*
         grp.C[0] = out->ptr; grp.N[0] = n;
         const uint16_t* X = static_cast<const uint16_t*>(in->ptr);
         const uint32_t per_wave = k / unit_k / 4;
-        if (fmt == LH_Q4_0) hipLaunchKernelGGL((matmul_skinny_kernel<kQ4, LH_F16, true>), dim3(blocks, mgroups), dim3(256), 0, ctx->stream, X, grp.W[0], out->ptr, m, k, n, (float*)nullptr, per_wave, grp);
+        const dim3 wide((blocks + 3) / 4, mgroups);
+        if (k % 256 == 0 && wide_pays(ctx, blocks, mgroups)) {
+            if (fmt == LH_Q4_0) hipLaunchKernelGGL((matmul_wide_kernel<kQ4, LH_F16, true>), wide, dim3(256), 0, ctx->stream, X, grp.W[0], out->ptr, m, k, n, blocks, grp);
+            else hipLaunchKernelGGL((matmul_wide_kernel<kTQ2, LH_F16, true>), wide, dim3(256), 0, ctx->stream, X, grp.W[0], out->ptr, m, k, n, blocks, grp);
+        } else if (fmt == LH_Q4_0) hipLaunchKernelGGL((matmul_skinny_kernel<kQ4, LH_F16, true>), dim3(blocks, mgroups), dim3(256), 0, ctx->stream, X, grp.W[0], out->ptr, m, k, n, (float*)nullptr, per_wave, grp);
         else hipLaunchKernelGGL((matmul_skinny_kernel<kTQ2, LH_F16, true>), dim3(blocks, mgroups), dim3(256), 0, ctx->stream, X, grp.W[0], out->ptr, m, k, n, (float*)nullptr, per_wave, grp);
     } else {
         // any other shape: the two products as matmul_nt_quant_grouped_into computes them, staged in the third quarter of the

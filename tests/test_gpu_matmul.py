@@ -391,6 +391,58 @@ def test_matmul_gelu_mul_fused_equals_separate_kernels(pkg, gpu, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
+@pytest.mark.parametrize("m,k,ns", [(17, 512, [65536]), (64, 1536, [65664]), (33, 1024, [40064, 25600]), (130, 512, [21888]), (256, 1024, [16384]),
+                                    (193, 512, [128, 16256, 128])])
+def test_rows_against_many_weight_rows(pkg, gpu, oracle, fmt, m, k, ns):
+    """The form in which four waves share the activations, from the fewest weight rows that reach it: whole and ragged groups of 64
+    activation rows, a last workgroup with idle waves, several matrices, both output types and the pair of the feed-forward.  Against the
+    f64 product of the f16 weights: half a step of the output, and 2^-24 of the terms' magnitude per 32 columns of a step."""
+    ctx, K = gpu
+    g = pkg.synth.rng(55, m + k + len(ns))
+    ty, x = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, g.standard_normal((m, k), dtype=np.float32).astype(np.float16)
+    some = [min(n, 1021) for n in ns]
+    raws = [payload(fmt, c, k, 0x61 + i) for i, c in enumerate(some)]
+    picks = [np.arange(n) % c for n, c in zip(ns, some)]
+    ws = [pkg.QuantWeight.from_bytes(ctx, np.ascontiguousarray(r.reshape(c, -1)[p]).reshape(-1), ty, n, k) for r, c, p, n in zip(raws, some, picks, ns)]
+    print(f"many weight rows {fmt} {m} {k} {ns}", flush=True)
+    xb, batch = pkg.Buffer.from_slice(ctx, x), pkg.CommandBatch(ctx)
+    outs = [pkg.Buffer.empty(ctx, m * n * 2) for n in ns]
+    K.matmul_nt_quant_grouped_into(batch, ty, xb, [w.buf for w in ws], outs, m, k, ns)
+    wide = [pkg.Buffer.empty(ctx, m * n * 4) for n in ns]
+    for w, o in zip(ws, wide):
+        w.matmul_nt_typed_into(batch, K, xb, pkg.F16, o, pkg.F32, m)
+    batch.commit_and_wait()
+    for i, n in enumerate(ns):
+        dq = expand(oracle, fmt, raws[i], some[i], k).astype(np.float16).astype(np.float64)
+        want, size = (x.astype(np.float64) @ dq.T)[:, picks[i]], (np.abs(x.astype(np.float64)) @ np.abs(dq).T)[:, picks[i]]
+        tol = size * 2.0 ** -24 * (k // 32 + 32)
+        assert np.all(np.abs(wide[i].as_array(np.float32, m * n).reshape(m, n) - want) <= tol), i
+        assert np.all(np.abs(outs[i].as_array(np.float16, m * n).reshape(m, n) - want) <= tol + np.abs(want) * 2.0 ** -11 + 2.0 ** -24), i
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
+@pytest.mark.parametrize("m,k,n", [(64, 512, 32768), (130, 512, 11008), (256, 1536, 8320)])
+def test_gate_and_up_against_many_weight_rows(pkg, gpu, fmt, m, k, n):
+    """The pair in that form against the grouped product and gelu_mul: bit for bit where that takes the form too; beyond 64 rows it takes
+    another, whose sums run in another order: a step of f16 in gate and in up (gelu' stays below 1.13) and one in the result."""
+    ctx, K = gpu
+    ty, g = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, pkg.synth.rng(79, m + k + n)
+    print(f"gate and up {fmt} {m} {k} {n}", flush=True)
+    wg, wu = (pkg.QuantWeight.from_bytes(ctx, pkg.synth.weights(fmt, n, k, g), ty, n, k) for _ in range(2))
+    x = pkg.Buffer.from_slice(ctx, (g.standard_normal((m, k), dtype=np.float32) * 0.5).astype(np.float16))
+    gate, up, want, got = (pkg.Buffer.empty(ctx, m * n * 2) for _ in range(4))
+    batch = pkg.CommandBatch(ctx)
+    K.matmul_nt_quant_grouped_into(batch, ty, x, [wg.buf, wu.buf], [gate, up], m, k, [n, n])
+    K.gelu_mul_into(batch, gate, up, want, m * n)
+    K.matmul_nt_quant_gelu_mul_into(batch, ty, x, wg.buf, wu.buf, got, m, k, n)
+    batch.commit_and_wait()
+    if m <= 64:
+        assert np.array_equal(got.as_array(np.uint16), want.as_array(np.uint16))
+    a, b, v, u = (t.as_array(np.float16).astype(np.float64) for t in (gate, up, want, got))
+    assert np.all(np.abs(u - v) <= 2.13 * 2.0 ** -10 * np.abs(a * b) + 2.0 ** -10 * np.abs(v) + 2.0 ** -24)
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
 def test_matmul_gelu_mul_strided_fused_equals_separate_kernels(pkg, gpu, fmt):
     """matmul_nt_quant_gelu_mul_strided_into against matmul_nt + gelu_mul_strided (itself gather_strided + gelu_mul), bit for
     bit: decode batches (the gelu kernel sums the split tiles), rows served as matvecs, a prefill chunk."""
