@@ -664,7 +664,7 @@ __global__ __launch_bounds__(256 + 64 * PW) void matmul_mfma128_kernel(const uin
 // k range; its four waves split that range in quarters, every wave multiplying all four tiles against all activation
 // rows for its quarter (one B fragment feeds four MFMAs), and the four partial tiles are added through LDS at the end.
 //
-// A lane fetches the codes it turns into its own A fragments, 8 bytes at a time, one "unit" ahead:
+// A lane turns 8 bytes of codes of a "unit" at a time into its own A fragments; the units come in one ahead:
 //   Q4_0  unit = 2 blocks (64 k).  Lane (row r, g) reads qs bytes 8(g&1) .. +8 of block (g>>1): the low nibbles are
 //         elements 8(g&1) .. +8 of that block (fragment 0), the high nibbles elements 16 + 8(g&1) .. +8 (fragment 1).
 //   TQ2_0 unit = half a block (128 k).  Lane (r, g) reads bytes 8g .. +8 of the half: field f of those bytes is
@@ -685,6 +685,24 @@ __device__ __forceinline__ uint2 ld8_align2(const uint8_t* p) {
     typedef u32x2_t __attribute__((aligned(2))) u32x2_a2;
     const u32x2_t v = *reinterpret_cast<const u32x2_a2*>(p);
     return make_uint2(v.x, v.y);
+}
+
+// (words written, words and halves read: types that may alias)
+typedef uint32_t __attribute__((may_alias)) lds_word_t;
+typedef uint16_t __attribute__((may_alias)) lds_half_t;
+
+// The codes and the scale that k group g takes from a unit as it lies in LDS: Q4_0 its 36 bytes (two blocks of a scale and 16 bytes of
+// codes, those of the group from byte 2, 10, 20 or 28), TQ2_0 32 bytes of codes and the block's scale.
+template <int FMT>
+__device__ __forceinline__ SkinnyRaw skinny_take(const uint8_t* p, uint32_t g) {
+    if constexpr (FMT == kQ4) {
+        const lds_word_t* q = reinterpret_cast<const lds_word_t*>(p + (g < 2 ? 8 * g : 8 * g + 4));
+        const uint32_t a = q[0], b = q[1], e = q[g < 2 ? 2 : 1], shift = g < 2 ? 16 : 0;
+        return {__builtin_amdgcn_alignbit(b, a, shift), __builtin_amdgcn_alignbit(e, b, shift), *reinterpret_cast<const lds_half_t*>(p + 18 * (g >> 1)) * 0x10001u};
+    } else {
+        const lds_word_t* q = reinterpret_cast<const lds_word_t*>(p + 8 * g);
+        return {q[0], q[1], *reinterpret_cast<const lds_half_t*>(p + 32) * 0x10001u};
+    }
 }
 
 template <int FMT>
@@ -734,26 +752,37 @@ __global__ __launch_bounds__(256, 2) void matmul_skinny_kernel(const uint16_t* _
         tile -= grp.tile0[gi];
     }
     const uint32_t n0 = PAIR ? blockIdx.x * 32 : tile * BN + (blockIdx.x & 1) * 64;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t r = lane & 15, g = lane >> 4;
     const size_t row_bytes = FMT == kQ4 ? (size_t)(K >> 5) * 18 : (size_t)(K >> 8) * 66;
     const uint32_t k_begin = (blockIdx.z * 4 + wave) * units_per_wave * UK;
     const uint32_t m0 = blockIdx.y * 64;                      // more than 64 activation rows: one workgroup per 64 of them
 
-    const uint8_t* wrow = W + (size_t)(n0 + r) * row_bytes;   // tile t starts 16 rows further on
-    const size_t tile_bytes = 16 * row_bytes;
-    const uint8_t* wrow_up = PAIR ? grp.W[1] + (size_t)(n0 + r) * row_bytes : nullptr;
-    auto load_a = [&](SkinnyRaw (&raw)[4], uint32_t k0) {
-        size_t off, doff;
-        if constexpr (FMT == kQ4) { const size_t b = (k0 >> 5) + (g >> 1); doff = b * 18; off = doff + 2 + 8 * (g & 1); }
-        else { const size_t b = k0 >> 8; doff = b * 66 + 64; off = b * 66 + 32 * ((k0 >> 7) & 1) + 8 * g; }
+    // A unit's codes of the 64 rows (Q4_0: 36 bytes a row; TQ2_0: 32, and the block's scale by itself) come in along the rows and are
+    // parked in the wave's own area, from which a lane takes its eight bytes: fetched by the lane itself they cost a cache access
+    // each (per launch of a 256-row chunk: 1536 columns 9.2 us, now 8.3; 6144 and 12288 columns 25.2, now 22.8).
+    constexpr uint32_t PIECES = FMT == kQ4 ? 5 : 4, PITCH = 36, UB = FMT == kQ4 ? 36 : 32;   // 8-byte pieces of a row (the last may overlap), bytes per row in LDS (an odd number of words)
+    __shared__ __align__(16) uint8_t codes[4][64 * PITCH];
+    uint8_t* const mine = codes[wave];
+    const uint8_t *wrow = W + (size_t)n0 * row_bytes, *wrow_up = PAIR ? grp.W[1] + (size_t)n0 * row_bytes : nullptr;   // rows 32 .. 63 of a pair: up
+    uint32_t c_at[PIECES], c_to[PIECES];
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const uint8_t* p = PAIR ? (t < 2 ? wrow : wrow_up) + (t & 1) * tile_bytes : wrow + t * tile_bytes;
-            const uint2 w = ld8_align2(p + off);
-            const uint32_t d = *reinterpret_cast<const uint16_t*>(p + doff);
-            raw[t].w0 = w.x; raw[t].w1 = w.y; raw[t].d = d | (d << 16);
-        }
+    for (uint32_t i = 0; i < PIECES; i++) {
+        const uint32_t at = 64 * i + lane, row = at / PIECES, piece = std::min(8 * (at - row * PIECES), UB - 8);
+        c_at[i] = (PAIR ? row & 31 : row) * (uint32_t)row_bytes + piece;
+        c_to[i] = row * PITCH + piece;
+    }
+    struct Codes { uint2 w[PIECES]; uint32_t d; };
+    auto load_a = [&](Codes& raw, uint32_t k0) {
+        const size_t at = FMT == kQ4 ? (size_t)(k0 >> 6) * 36 : (size_t)(k0 >> 8) * 66, half = FMT == kQ4 ? 0 : 32 * ((k0 >> 7) & 1);
+#pragma unroll
+        for (uint32_t i = 0; i < PIECES; i++) raw.w[i] = ld8_align2((PAIR && c_to[i] >= 32 * PITCH ? wrow_up : wrow) + at + half + c_at[i]);
+        if constexpr (FMT == kTQ2) raw.d = *reinterpret_cast<const uint16_t*>((PAIR && lane >= 32 ? wrow_up : wrow) + at + 64 + (PAIR ? lane & 31 : lane) * (uint32_t)row_bytes);
+    };
+    auto park_a = [&](const Codes& raw) {
+#pragma unroll
+        for (uint32_t i = 0; i < PIECES; i++) { *reinterpret_cast<lds_word_t*>(mine + c_to[i]) = raw.w[i].x; *reinterpret_cast<lds_word_t*>(mine + c_to[i] + 4) = raw.w[i].y; }
+        if constexpr (FMT == kTQ2) *reinterpret_cast<lds_half_t*>(mine + lane * PITCH + 32) = (uint16_t)raw.d;
     };
     // The activations of a unit (64 rows x UK columns) come in with coalesced loads -- a lane takes 16 bytes of one row,
     // CPR consecutive lanes one row's UK columns -- one unit ahead, and are parked in the wave's LDS area in fragment
@@ -823,7 +852,11 @@ __global__ __launch_bounds__(256, 2) void matmul_skinny_kernel(const uint16_t* _
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](const SkinnyRaw (&raw)[4]) {
+    auto multiply = [&](const Codes& parked) {
+        park_a(parked);
+        SkinnyRaw raw[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) raw[t] = skinny_take<FMT>(mine + (16 * t + r) * PITCH, g);
 #pragma unroll
         for (int f = 0; f < NF; f++) {
             f16x8 bf[4];
@@ -840,7 +873,7 @@ __global__ __launch_bounds__(256, 2) void matmul_skinny_kernel(const uint16_t* _
 
     // two register sets for the codes, one for the activations, the unit after the one being multiplied always in flight;
     // the load past the end re-reads the last unit
-    SkinnyRaw ra0[4], ra1[4];
+    Codes ra0, ra1;
     f32x4 rb[NLD];
     const uint32_t last = k_begin + (units_per_wave - 1) * UK;
     load_a(ra0, k_begin);
@@ -978,25 +1011,8 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
     };
     auto park_a = [&](const Codes& raw) {
 #pragma unroll
-        for (uint32_t i = 0; i < NL; i++) { *reinterpret_cast<uint32_t*>(mine + c_to[i]) = raw.w[i].x; *reinterpret_cast<uint32_t*>(mine + c_to[i] + 4) = raw.w[i].y; }
-        if constexpr (FMT == kTQ2) *reinterpret_cast<uint16_t*>(mine + lane * PITCH + 32) = (uint16_t)raw.d;
-    };
-    // the lane's codes and scale of unit v of the parked step, row r of tile t
-    auto take = [&](int v, int t) {
-        const uint8_t* p = mine + (16 * t + r) * PITCH;
-        SkinnyRaw c;
-        if constexpr (FMT == kQ4) {
-            const uint32_t* q = reinterpret_cast<const uint32_t*>(p + 36 * v + (g < 2 ? 8 * g : 8 * g + 4));      // blocks at bytes 0 and 18 of the 36: codes from byte 2, 10, 20, 28
-            const uint32_t a = q[0], b = q[1], e = q[g < 2 ? 2 : 1], sh = g < 2 ? 16 : 0;
-            c.w0 = __builtin_amdgcn_alignbit(b, a, sh);
-            c.w1 = __builtin_amdgcn_alignbit(e, b, sh);
-            c.d = *reinterpret_cast<const uint16_t*>(p + 36 * v + 18 * (g >> 1)) * 0x10001u;
-        } else {
-            const uint32_t* q = reinterpret_cast<const uint32_t*>(p + 8 * g);
-            c.w0 = q[0]; c.w1 = q[1];
-            c.d = *reinterpret_cast<const uint16_t*>(p + 32) * 0x10001u;
-        }
-        return c;
+        for (uint32_t i = 0; i < NL; i++) { *reinterpret_cast<lds_word_t*>(mine + c_to[i]) = raw.w[i].x; *reinterpret_cast<lds_word_t*>(mine + c_to[i] + 4) = raw.w[i].y; }
+        if constexpr (FMT == kTQ2) *reinterpret_cast<lds_half_t*>(mine + lane * PITCH + 32) = (uint16_t)raw.d;
     };
     const uint32_t ld_row = tid >> 4, ld_q = tid & 15;
     const uint32_t ld_f = FMT == kQ4 ? 2 * (ld_q >> 3) + ((ld_q & 3) >> 1) : ld_q >> 2, ld_g = FMT == kQ4 ? 2 * ((ld_q >> 2) & 1) + (ld_q & 1) : ld_q & 3;
@@ -1025,7 +1041,7 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
         for (int f = 0; f < 4; f++) {
             if (f % NF == 0)
 #pragma unroll
-                for (int t = 0; t < 4; t++) c[t] = take(f / NF, t);
+                for (int t = 0; t < 4; t++) c[t] = skinny_take<FMT>(mine + (16 * t + r) * PITCH + 36 * (f / NF), g);
             f16x8 bf[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) bf[j] = __builtin_bit_cast(f16x8, from[(f * 4 + j) * 64 + g * 16 + (r ^ (g | ((f & 1) << 2)))]);
