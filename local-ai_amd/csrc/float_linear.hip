@@ -592,7 +592,7 @@ __global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
 // products with bf16 weights are then exact and summed in f32, as FMA has them, on the matrix cores; a row becomes its lowest terms,
 // its middle terms and its leading terms, one after the other.  A term that is zero of a value that is not becomes a tiny one of
 // its sign, far below what f32 sums see: an infinite weight then gives the infinity that it gives times the value itself.
-// (333 x 1024 x 4096: 185 us on the FMA units, 17 us for both launches.)
+// (The products of a pass over 333 rows at width 1024: 184 us on average on the FMA units, 30 and 6 for the terms.)
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, uint16_t* __restrict__ out, uint32_t rows, uint32_t K, uint32_t lda, uint32_t stride) {
     const uint32_t per = stride / 4, row = blockIdx.y * 4 + threadIdx.x / 64;
     if (row >= rows) return;
