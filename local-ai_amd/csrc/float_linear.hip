@@ -285,8 +285,10 @@ __device__ __forceinline__ void finish_tile(const LhLinear& a, const lh_f32x4 (*
     const uint32_t pos0 = a.seg.position ? *a.seg.position : 0u, g = lane >> 4;
     if constexpr (EPI != kThroughLds) {
         const uint32_t s0 = lh_segment_of(a.seg, nw), s1 = lh_segment_of(a.seg, min(nw + 16 * TJ, a.N) - 1), first = rt.begin + row0, at = pos0 + first;
-        const bool blocks = a.seg.layout[s0] == LH_BLOCKS_AT_POSITION;
-        if (!blocks && a.seg.layout[s1] != LH_BLOCKS_AT_POSITION) {
+        bool blocks = false;                                  // in any of the segments: the wave's columns may hold a whole one between two others
+#pragma unroll
+        for (uint32_t s = 0; s < 4; s++) blocks = blocks || (s >= s0 && s <= s1 && a.seg.layout[s] == LH_BLOCKS_AT_POSITION);
+        if (!blocks) {
             store_columns<EPI, TI, TJ>(a, acc, LaneColumns(a.seg, nw + g * 4 * TJ), first + (lane & 15), rt.end, pos0);
             return;
         }

@@ -208,6 +208,33 @@ def test_segments_write_caches_at_the_position(ai, gpu, dtype, m, pos, width, he
         check()
 
 
+@pytest.mark.parametrize("sizes,blocks", [((16, 32, 16), 1), ((8, 8, 16), 1), ((32, 16, 16), 0), ((16, 16, 32), 2), ((96, 32, 64, 64), 1), ((48, 16, 32, 160), 2)])
+@pytest.mark.parametrize("m,k", [(20, 64), (40, 64), (32800, 72), (65600, 72), (24640, 64), (32800, 64), (65600, 64)])
+def test_value_blocks_among_other_segments(ai, gpu, sizes, blocks, m, k):
+    """A value cache's segment before, between and behind others, narrower than the columns that a wave finishes at once, on every tile
+    size (32 to 256 rows; 200 columns and more take the wide ones)."""
+    ctx, K = gpu
+    g, L, pos, cap, few = np.random.default_rng(m + k + sum(sizes)), ai.linear_weight, 32, m // 32 * 32 + 64, min(m, 1000)
+    w, x = M.rounded(g.standard_normal((sum(sizes), k)) / np.sqrt(k)), M.rounded(g.standard_normal((few, k)))
+    rows = np.arange(m) % few
+    lin = L.StackedLinear(ctx, [M.bf16_bits(w)], [L.Segment(sum(sizes))])
+    segments = L.Segments([L.Segment(n, 0, 0, 0, ai.BLOCKS_AT_POSITION if i == blocks else ai.ROWS) for i, n in enumerate(sizes)])
+    outs = [empty(ai, ctx, (cap if i == blocks else m) * n, ai.BF16) for i, n in enumerate(sizes)]
+    print(f"blocks among segments {sizes} {blocks} {m} {k}", flush=True)
+    batch = ai.CommandBatch(ctx)
+    lin.rows_into(batch, K, ai.Buffer.from_slice(ctx, M.bf16_bits(x)[rows]), ai.BF16, m, outs, ai.BF16, ai.Buffer.from_slice(ctx, np.array([pos], np.uint32)), segments)
+    batch.commit_and_wait()
+    want, at = x @ w.T, 0
+    for i, n in enumerate(sizes):
+        got = download(ai, outs[i], (cap if i == blocks else m) * n, ai.BF16)
+        if i == blocks:
+            got = values_from_cache(got, n)
+            assert not got[:pos].any() and not got[pos + m:].any()
+            got = got[pos:pos + m]
+        close(got.reshape(m, n), want[rows, at:at + n], BF16_TOL, f"segment {i}")
+        at += n
+
+
 @pytest.mark.parametrize("k,n", [(64, 40), (60, 33), (512, 130), (1000, 64), (1536, 20), (4096, 70), (9000, 12), (2501, 9)])
 def test_linear_vector_stages(ai, gpu, k, n):
     """The norm (with an addition and a stored sum) and the gated norm in front of a one-row product."""
