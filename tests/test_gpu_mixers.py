@@ -106,6 +106,52 @@ def test_large_products(ai, gpu, m, k, n, act):
     close(download(ai, res, m * n, ai.F32).reshape(m, n), want + 1, F32_TOL, "residual")
 
 
+@pytest.mark.parametrize("act", ["silu", "gelu", "pairs"])
+@pytest.mark.parametrize("m", [1024, 64])
+def test_activations_of_bf16_results(ai, gpu, act, m):
+    """Activations of many rows round to bf16 from 32-bit values, infinities and NaN as f32 arithmetic has them.  A result lies half a
+    bf16 step from the f64 activation of the same f32 sum, and 7 x 2^-24 of its size: the exponential (one ulp, two of these units), the
+    constant ln 2 (one, up to |z| = 20), two sums and the quotient (one each), a second factor (one); gelu's argument carries three roundings,
+    which the exponential multiplies by its size."""
+    ctx, K = gpu
+    g, L, n, k = np.random.default_rng(m), ai.linear_weight, 4096, 64
+    x, w, b = M.rounded(g.uniform(-4, 4, m)), M.rounded(g.uniform(-4, 4, n)), g.uniform(-4, 4, n).astype(np.float32)
+    b[:16] = (np.inf, -np.inf, np.nan, 3e38, -3e38, 88.5, -88.5, -86.0, -95.0, 130.0, -130.0, 0.0, -0.0, 1e-30, -1e-30, -1e20)
+    w[:16] = 0.0
+    xs, ws = np.zeros((m, k)), np.zeros((n, k))
+    xs[:, 0], ws[:, 0] = x, w                               # one exact product and one addition: the sum is known to the bit
+    lin = L.StackedLinear(ctx, [M.bf16_bits(ws)], [L.Segment(n, {"silu": ai.ACT_SILU, "gelu": ai.ACT_GELU_TANH, "pairs": ai.ACT_SILU_PAIRS}[act])], [b])
+    width = n // 2 if act == "pairs" else n
+    out, batch = empty(ai, ctx, m * width, ai.BF16), ai.CommandBatch(ctx)
+    print(f"activations {act} {m}", flush=True)
+    lin.rows_into(batch, K, upload(ai, ctx, xs, ai.BF16), ai.BF16, m, [out], ai.BF16)
+    batch.commit_and_wait()
+    got = download(ai, out, m * width, ai.BF16).reshape(m, width)
+    v = ((x[:, None] * w).astype(np.float32) + b).astype(np.float64)
+    with np.errstate(all="ignore"):
+        first, second = (v[:, 0::2], v[:, 1::2]) if act == "pairs" else (v, 1.0)
+        z = 1.5957691216057308 * (first + 0.044715 * first ** 3) if act == "gelu" else first
+        e = np.exp(-z)
+        want = first / (1.0 + e) * second
+        slack = (7 + 3 * np.minimum(np.abs(z), 100) * e / (1 + e) * (act == "gelu")) * 2.0 ** -24
+        half = np.exp2(np.floor(np.log2(np.abs(want)))) * 2.0 ** -8
+        usual = np.isfinite(v[:, 0::2] + v[:, 1::2] if act == "pairs" else v) & (np.abs(z) < 20) & (np.abs(want) > 1e-30) & (np.abs(want) < 3e38)
+        assert usual.mean() > 0.6
+        over = (np.abs(got - want) - half) / np.abs(want) / 2.0 ** -24
+        assert (over <= slack * 2.0 ** 24)[usual].all(), over[usual].max()
+        plain = empty(ai, ctx, m * width, ai.F32)              # f32 results go through expf and a division
+        lin.rows_into(batch, K, upload(ai, ctx, xs, ai.BF16), ai.BF16, m, [plain], ai.F32)
+        batch.commit_and_wait()
+        missed, expected = (int((np.abs(r - want) > half)[usual].sum()) for r in (got, M.rounded(download(ai, plain, m * width, ai.F32).reshape(m, width))))
+        print(f"not nearest: {missed}, rounded from f32 {expected}, of {usual.sum()}", flush=True)
+        assert missed <= 1.2 * expected + 8
+        alone = ai.Buffer.empty(ctx, 4 * width)               # a single row keeps expf and the division
+        lin.vector_into(batch, K, upload(ai, ctx, xs[0], ai.F32), ai.F32, [alone], ai.F32)
+        batch.commit_and_wait()
+        special, same = got[0, :16 if width == n else 8], M.rounded(alone.as_array(np.float32, width)[:16 if width == n else 8])
+        assert np.array_equal(np.isnan(special), np.isnan(same)) and np.allclose(special, same, 2.0 ** -7, 1e-36, equal_nan=True), (special, same)
+
+
 @pytest.mark.parametrize("m,k,n", [(40, 72, 50), (333, 1024, 256), (2048, 64, 2048), (3, 4096, 16)])
 def test_f32_rows_as_terms(ai, gpu, m, k, n):
     """32-bit activations on the matrix cores: all 24 bits of every value, whatever its size, and what is infinite or no number comes
