@@ -961,10 +961,21 @@ __global__ __launch_bounds__(256, 2) void matmul_skinny_kernel(const uint16_t* _
 // activations from L2 for itself and adds four partial tiles through LDS: 64 x 1536 x 262144 (Q4_0, f32 out) 176 us, here 95; 256 rows,
 // gate and up of 12288 x 1536 (TQ2_0) 39 and 34.
 // The codes are two steps ahead in registers, the activations one in registers and one in LDS; one barrier per step.
+// An address in global memory that is the same in all lanes, kept in scalar registers: a load at it plus 32 bits of offset of the lane's own
+// needs no vector registers for addresses.  (The builtin gives a signed word: it must not be widened as one.)
+typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;
+__device__ __forceinline__ uint64_t uniform_address(const void* p) {
+    const uint64_t a = (uint64_t)p;
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32;
+}
+// (the compiler must not see through either, or it keeps steps of a loop in a pair of vector registers for every load)
+__device__ __forceinline__ GlobalBytes load_base(uint64_t address) { asm volatile("" : "+s"(address)); return (GlobalBytes)address; }
+__device__ __forceinline__ uint32_t lane_offset(uint32_t offset) { asm volatile("" : "+v"(offset)); return offset; }
+
 template <int FMT, int CDT, bool PAIR>
 __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W_one, void* __restrict__ C_one, uint32_t M,
                                                             uint32_t K, uint32_t N_one, uint32_t blocks, GroupArgs grp) {
-    constexpr int UK = Skinny<FMT>::unit_k, NF = Skinny<FMT>::frags, UNITS = 128 / UK;       // units of codes per step
+    constexpr int UK = Skinny<FMT>::unit_k, NF = Skinny<FMT>::frags;
     __shared__ f32x4 stage[2][16 * 64];                       // [buffer][fragment f of the step, activation group j][cell]
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const uint32_t block = blockIdx.x * 4 + wave;             // a workgroup's last waves may have none: they only bring in activations
@@ -978,40 +989,50 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
         tile -= grp.tile0[gi];
     }
     const uint32_t n0 = PAIR ? (on ? block : blocks - 1) * 32 : tile * BN + ((on ? block : blocks - 1) & 1) * 64;
-    const size_t row_bytes = FMT == kQ4 ? (size_t)(K >> 5) * 18 : (size_t)(K >> 8) * 66, tile_bytes = 16 * row_bytes;
+    const size_t row_bytes = FMT == kQ4 ? (size_t)(K >> 5) * 18 : (size_t)(K >> 8) * 66;
     const uint32_t m0 = blockIdx.y * 64;
 
     // Codes: the 64 rows' bytes of a step (Q4_0: 72 a row; TQ2_0: 32 of codes, and the scale of the block by itself) come in with coalesced
     // loads, consecutive lanes along a row, and are parked in the wave's own LDS area, from which every lane takes what it multiplies.
     // (A lane loading its eight bytes itself costs a cache access per lane, one per clock and CU: 135 us where this takes 95.)
-    constexpr uint32_t PIECES = FMT == kQ4 ? 9 : 4, PITCH = FMT == kQ4 ? 76 : 36, NL = PIECES;     // 8-byte pieces per row; bytes per row in LDS (an odd number of words); loads of 64 lanes
+    // A load of the wave takes whole rows (Q4_0: seven of nine pieces of 8 bytes, the last lane repeating one; TQ2_0: sixteen of four), so that
+    // loads are a constant apart; the last Q4_0 load repeats row 63.
+    constexpr uint32_t PIECES = FMT == kQ4 ? 9 : 4, RPL = 64 / PIECES, NL = (64 + RPL - 1) / RPL, PITCH = FMT == kQ4 ? 76 : 36;   // PITCH: bytes per row in LDS, an odd number of words
     __shared__ __align__(16) uint8_t codes[4][64 * PITCH];
     uint8_t* const mine = codes[wave];
     typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
     typedef u32x2_t __attribute__((aligned(2))) u32x2_a2;
-    // row of a workgroup's 64: rows 0..31 gate, 32..63 up of a pair
-    const uint8_t *wrow = W + (size_t)n0 * row_bytes, *wrow_up = PAIR ? grp.W[1] + (size_t)n0 * row_bytes : nullptr;
-    uint32_t c_at[NL], c_to[NL];
-#pragma unroll
-    for (uint32_t i = 0; i < NL; i++) {
-        const uint32_t at = 64 * i + lane, row = at / PIECES, piece = at - row * PIECES;
-        c_at[i] = (PAIR ? row & 31 : row) * (uint32_t)row_bytes + 8 * piece;
-        c_to[i] = row * PITCH + 8 * piece;
-    }
+    // rows 0 .. 31 of a pair: gate; 32 .. 63: up, from `up` on counted as those
+    const uint64_t wrow = uniform_address(W + (size_t)n0 * row_bytes), up = PAIR ? uniform_address(grp.W[1] + (size_t)n0 * row_bytes - 32 * row_bytes) : wrow;
+    const uint32_t cl = std::min(lane, RPL * PIECES - 1), c_row = cl / PIECES, c_piece = cl - c_row * PIECES, last_row = FMT == kQ4 ? std::min((NL - 1) * RPL + c_row, 63u) : 0u;
+    const uint32_t c_at = c_row * (uint32_t)row_bytes + 8 * c_piece, c_to = c_row * PITCH + 8 * c_piece;
+    const uint32_t last_at = (last_row - (NL - 1) * RPL) * (uint32_t)row_bytes + 8 * c_piece, last_to = last_row * PITCH + 8 * c_piece;
     struct Codes { u32x2_t w[NL]; uint32_t d; } ra[2];
     auto load_a = [&](Codes& raw, uint32_t k0) {
-        const size_t at = FMT == kQ4 ? (size_t)(k0 >> 6) * 36 : (size_t)(k0 >> 8) * 66, half = FMT == kQ4 ? 0 : 32 * ((k0 >> 7) & 1);
+        const uint32_t at = FMT == kQ4 ? (k0 >> 6) * 36 : (k0 >> 8) * 66 + 32 * ((k0 >> 7) & 1);
+        const uint32_t some_at = lane_offset(c_at), tail_at = lane_offset(last_at);
 #pragma unroll
         for (uint32_t i = 0; i < NL; i++) {
-            // (pair: with 64 rows of PIECES pieces, load i is of gate rows in its first half and of up rows in its second)
-            const uint8_t* p = PAIR ? (c_to[i] >= 32 * PITCH ? wrow_up : wrow) : wrow;
-            raw.w[i] = *reinterpret_cast<const u32x2_a2*>(p + at + half + c_at[i]);
+            const uint32_t first = i * RPL, lane_at = FMT == kQ4 && i == NL - 1 ? tail_at : some_at;
+            const bool both = PAIR && first < 32 && first + RPL > 32;         // row 32 of a Q4_0 pair lies within load 4
+            GlobalBytes p = load_base((PAIR && first >= 32 ? up : wrow) + at + first * row_bytes);
+            if (both && first + c_row >= 32) p = (GlobalBytes)(up + at + first * row_bytes);
+            raw.w[i] = *(const __attribute__((address_space(1))) u32x2_a2*)(p + lane_at);
         }
-        if constexpr (FMT == kTQ2) raw.d = *reinterpret_cast<const uint16_t*>((PAIR ? (lane >= 32 ? wrow_up : wrow) : wrow) + at + 64 + (PAIR ? lane & 31 : lane) * (uint32_t)row_bytes);
+        if constexpr (FMT == kTQ2) {
+            const uint32_t d_at = (k0 >> 8) * 66 + 64;
+            GlobalBytes p = load_base(wrow + d_at);
+            if (PAIR && lane >= 32) p = (GlobalBytes)(up + d_at);
+            raw.d = *(const __attribute__((address_space(1))) uint16_t*)(p + lane_offset(lane * (uint32_t)row_bytes));
+        }
     };
     auto park_a = [&](const Codes& raw) {
 #pragma unroll
-        for (uint32_t i = 0; i < NL; i++) { *reinterpret_cast<lds_word_t*>(mine + c_to[i]) = raw.w[i].x; *reinterpret_cast<lds_word_t*>(mine + c_to[i] + 4) = raw.w[i].y; }
+        for (uint32_t i = 0; i < NL; i++) {
+            uint8_t* const to = mine + (FMT == kQ4 && i == NL - 1 ? last_to : c_to + i * RPL * PITCH);
+            *reinterpret_cast<lds_word_t*>(to) = raw.w[i].x;
+            *reinterpret_cast<lds_word_t*>(to + 4) = raw.w[i].y;
+        }
         if constexpr (FMT == kTQ2) *reinterpret_cast<lds_half_t*>(mine + lane * PITCH + 32) = (uint16_t)raw.d;
     };
     const uint32_t ld_row = tid >> 4, ld_q = tid & 15;
@@ -1021,10 +1042,11 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
 #pragma unroll
     for (int j = 0; j < 4; j++) x_at[j] = (std::min(m0 + 16 * j + ld_row, M - 1) * K + 8 * ld_q) * 2;      // rows past M repeat the last one
     f32x4 rb[4];
+    const uint64_t activations = uniform_address(X);
     auto load_b = [&](uint32_t k0) {
-        const char* base = reinterpret_cast<const char*>(X) + (size_t)k0 * 2;
+        const GlobalBytes base = load_base(activations + 2 * k0);
 #pragma unroll
-        for (int j = 0; j < 4; j++) rb[j] = *reinterpret_cast<const f32x4*>(base + x_at[j]);
+        for (int j = 0; j < 4; j++) rb[j] = *(const __attribute__((address_space(1))) f32x4*)(base + lane_offset(x_at[j]));
     };
     auto park_b = [&](f32x4* to) {
 #pragma unroll
@@ -1035,7 +1057,25 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](const f32x4* from) {
+    // The sums run in four quarters of k that are added at the end, as matmul_skinny_kernel's waves have them: a product gives the same
+    // bits in both forms (alone, grouped, in a pair, behind a fused step), and no chain of f32 additions is longer than there.  (In one
+    // chain: 64 x 1536 x 262144 91 us where this takes 94, gate and up of 12288 x 1536 (TQ2_0) for 256 rows 28.8 and 30.4.)
+    f32x4 total[4][4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) total[t][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const uint32_t quarter = (K >> 2) / UK;
+    uint32_t left = quarter;                                  // units of the quarter that are still to come
+    auto end_unit = [&]() __attribute__((always_inline)) {
+        if (--left) return;
+        left = quarter;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) { total[t][j] += acc[t][j]; acc[t][j] = (f32x4){0.f, 0.f, 0.f, 0.f}; }
+    };
+    auto multiply = [&](const f32x4* from) __attribute__((always_inline)) {
         SkinnyRaw c[4];
 #pragma unroll
         for (int f = 0; f < 4; f++) {
@@ -1051,6 +1091,7 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
 #pragma unroll
                 for (int j = 0; j < 4; j++) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bf[j], acc[t][j], 0, 0, 0);
             }
+            if (f % NF == NF - 1) end_unit();
         }
     };
 
@@ -1083,14 +1124,14 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
             for (int t = 0; t < 2; t++) {
                 uint16_t h[4];
 #pragma unroll
-                for (int i = 0; i < 4; i++) h[i] = lh_gelu_mul_h(lh_f2h(acc[t][j][i]), lh_f2h(acc[t + 2][j][i]));
+                for (int i = 0; i < 4; i++) h[i] = lh_gelu_mul_h(lh_f2h(total[t][j][i]), lh_f2h(total[t + 2][j][i]));
                 *reinterpret_cast<uint2*>(static_cast<uint16_t*>(grp.C[0]) + (size_t)m * grp.N[0] + n0 + 16 * t + 4 * g) =
                     make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
             }
         } else {
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const f32x4 v = acc[t][j];
+                const f32x4 v = total[t][j];
                 const size_t at = (size_t)m * N + n0 + 16 * t + 4 * g;
                 if constexpr (CDT == LH_F32) *reinterpret_cast<f32x4*>(static_cast<float*>(C) + at) = v;
                 else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(C) + at) = make_uint2(pack_h2(v[0], v[1]), pack_h2(v[2], v[3]));
@@ -1718,7 +1759,7 @@ int lh_matmul_nt_quant_gelu_mul_into(lh_batch* b, lh_quant fmt, const lh_buffer*
     const uint32_t unit_k = fmt == LH_Q4_0 ? Skinny<kQ4>::unit_k : Skinny<kTQ2>::unit_k;
     const uint32_t blocks = n / 32;
     // one launch where the grouped product of the pair takes the skinny kernel without a k split (split products need
-    // their sums before the gelu); the same workgroup count and k ranges, hence the same sums
+    // their sums before the gelu); the same quarters of k in either kernel, hence the same sums
     const uint32_t mgroups = (m + 63) / 64;
     if (m >= skinny_min_m(fmt == LH_Q4_0 ? kQ4 : kTQ2) && (fmt != LH_Q4_0 || m > (uint32_t)kMaxMultivecM) && m <= skinny_max_m() &&
         n % BN == 0 && k % (4 * unit_k) == 0 &&
