@@ -17,6 +17,7 @@
 //   attention_wide_kernel   f32 caches: f32 matrix instructions, 16 packed rows a workgroup
 // Plain form (any dtype, any dim): attention_plain_kernel, one workgroup per query row and head.
 #include "softmax_attention.hpp"
+#include <type_traits>
 
 namespace {
 
@@ -392,7 +393,9 @@ __global__ __launch_bounds__(256) void attention_wide_kernel(const AttentionArgs
     const float* K = static_cast<const float*>(a.keys) + (size_t)g * MAPS * a.dq;
     const float* V = static_cast<const float*>(a.values) + (size_t)g * DV * 32;
     const size_t krow = (size_t)a.kv_heads * MAPS * a.dq, vblock = (size_t)a.kv_heads * DV * 32;
-    for (uint32_t b = wave; b * 32 <= last_key; b += 4) {
+    // DIAGONAL: not all of the 16 rows see all of the block's keys, or the cache's last ones lie behind the last row.
+    auto block = [&](uint32_t b, auto diagonal) __attribute__((always_inline)) {
+        constexpr bool DIAGONAL = decltype(diagonal)::value;
         float p[MAPS][8];
 #pragma unroll
         for (int mp = 0; mp < MAPS; mp++) {
@@ -421,7 +424,7 @@ __global__ __launch_bounds__(256) void attention_wide_kernel(const AttentionArgs
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 p[mp][i] = s[i >> 2][i & 3] * a.scale;
-                if (b * 32 + 31 > first_limit && b * 32 + (i >> 2) * 16 + gr * 4 + (i & 3) > limit) p[mp][i] = -INFINITY;
+                if (DIAGONAL && b * 32 + (i >> 2) * 16 + gr * 4 + (i & 3) > limit) p[mp][i] = -INFINITY;
                 mx = fmaxf(mx, p[mp][i]);
             }
             const float nm = fmaxf(m[mp], lh_column_max(mx)), base = nm == -INFINITY ? 0.0f : nm, alpha = expf(m[mp] - base);
@@ -435,23 +438,54 @@ __global__ __launch_bounds__(256) void attention_wide_kernel(const AttentionArgs
 #pragma unroll
                 for (int r = 0; r < 4; r++) o[mp][d][r] *= alpha;
         }
-        const bool end = b * 32 + 31 > last_key;              // entries of a block past the last key may be anything
 #pragma unroll
         for (int d = 0; d < TD; d++) {
             const float* vr = V + b * vblock + (d * 16 + lr) * 32 + gr * 8;
-            lh_f32x4 x = *reinterpret_cast<const lh_f32x4*>(vr), y = *reinterpret_cast<const lh_f32x4*>(vr + 4);
+            lh_f32x4 v[2] = {*reinterpret_cast<const lh_f32x4*>(vr), *reinterpret_cast<const lh_f32x4*>(vr + 4)};
+            if constexpr (DIAGONAL) {
+                bool odd = false;
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    if (b * 32 + (i >> 2) * 16 + gr * 4 + (i & 3) > last_key) v[i >> 2][i & 3] = 0.0f;    // may be anything
+                    odd = odd || !(fabsf(v[i >> 2][i & 3]) < INFINITY);
+                }
+                if (__any(odd)) {                             // infinities and NaN must not meet the weight 0 of a row that does not see them
+#pragma unroll
+                    for (int mp = 0; mp < MAPS; mp++) {
+                        // how many of each kind a row sees: 1 for inf, 64 for -inf, 4096 for NaN or an infinity whose weight is 0
+                        lh_f32x4 seen = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int i = 0; i < 8; i++) {
+                            const float x = v[i >> 2][i & 3], w = p[mp][i], infinite = x == INFINITY ? 1.0f : x == -INFINITY ? 64.0f : 0.0f, none = x != x ? 4096.0f : 0.0f;
+                            const bool sees = b * 32 + (i >> 2) * 16 + gr * 4 + (i & 3) <= limit;
+                            seen = __builtin_amdgcn_mfma_f32_16x16x4f32(infinite + none, sees && w != 0.0f ? 1.0f : 0.0f, seen, 0, 0, 0);
+                            seen = __builtin_amdgcn_mfma_f32_16x16x4f32(infinite + none != 0.0f ? 4096.0f : 0.0f, sees && w == 0.0f ? 1.0f : 0.0f, seen, 0, 0, 0);
+                        }
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const uint32_t n = (uint32_t)seen[r];
+                            if (n & 63u) o[mp][d][r] += INFINITY;
+                            if (n >> 6 & 63u) o[mp][d][r] -= INFINITY;
+                            if (n >> 12) o[mp][d][r] = __builtin_nanf("");
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < 8; i++) v[i >> 2][i & 3] = fabsf(v[i >> 2][i & 3]) < INFINITY ? v[i >> 2][i & 3] : 0.0f;
+                }
+            }
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                if (end && b * 32 + gr * 4 + j > last_key) x[j] = 0.0f;
-                if (end && b * 32 + 16 + gr * 4 + j > last_key) y[j] = 0.0f;
 #pragma unroll
                 for (int mp = 0; mp < MAPS; mp++) {
-                    o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], p[mp][j], o[mp][d], 0, 0, 0);
-                    o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[j], p[mp][4 + j], o[mp][d], 0, 0, 0);
+                    o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[0][j], p[mp][j], o[mp][d], 0, 0, 0);
+                    o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[1][j], p[mp][4 + j], o[mp][d], 0, 0, 0);
                 }
             }
         }
-    }
+    };
+    uint32_t b = wave;
+    for (; b * 32 + 31 <= min(first_limit, last_key); b += 4) block(b, std::false_type());
+    for (; b * 32 <= last_key; b += 4) block(b, std::true_type());
     __syncthreads();
 #pragma unroll
     for (int mp = 0; mp < MAPS; mp++) {

@@ -372,7 +372,7 @@ def test_row_norms_and_gather(ai, gpu, rows, dim):
 
 
 # ---- softmax attention -------------------------------------------------------------------------------------------------
-def attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows, cap, seed=0, spike=None, stale=False, lam=0.4, out_scale=0.7):
+def attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows, cap, seed=0, spike=None, stale=False, lam=0.4, out_scale=0.7, poison=()):
     """Caches filled as the projections fill them.  `spike` = (row, key): one key that takes nearly all of a row's weight."""
     ctx, K = gpu
     dt = ai.BF16 if dtype == "bf16" else ai.F32
@@ -388,6 +388,8 @@ def attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows
     kc, vc, qp = np.full((cap, kv_heads, maps, dq), fill), np.full((cap, kv_heads, dv), fill), np.zeros((rows, heads, maps, dq))
     kc[:, :, :, dim:] = vc[:, :, vdim:] = 0.0
     kc[:L, :, :, :dim], vc[:L, :, :vdim], qp[..., :dim] = k, v, q
+    for key, column, value in poison:
+        vc[key, :, column] = value
     blocks = np.zeros((cap // 32, kv_heads * dv, 32))
     blocks[:, :, block_order()] = vc.reshape(cap // 32, 32, kv_heads * dv).transpose(0, 2, 1)
     out, pos = empty(ai, ctx, rows * heads * vdim, dt), ai.Buffer.from_slice(ctx, np.array([start], np.uint32))
@@ -397,6 +399,8 @@ def attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows
                           kv_heads, maps, dim, vdim, cap, scale, lam, out_scale, eps)
     batch.commit_and_wait()
     got = download(ai, out, rows * heads * vdim, dt).reshape(rows, heads, vdim)
+    if poison:
+        return got
     want = np.zeros((rows, heads, vdim))
     for h in range(heads):
         j = h // (heads // kv_heads)
@@ -446,6 +450,30 @@ def test_attention_ignores_what_lies_behind_the_last_position(ai, gpu, rows):
 def test_wide_attention_every_head_size(ai, gpu, maps, dim, vdim, start, rows):
     a = attention_case(ai, gpu, "f32", maps, 4, 2, dim, vdim, start, rows, 256)
     assert np.array_equal(a, attention_case(ai, gpu, "f32", maps, 4, 2, dim, vdim, start, rows, 256, stale=True))
+
+
+@pytest.mark.parametrize("dim,vdim", [(32, 32), (64, 64), (33, 128), (128, 256)])
+@pytest.mark.parametrize("start,rows", [(0, 40), (31, 18), (70, 50)])
+@pytest.mark.parametrize("maps", [1, 2])
+def test_wide_attention_rows_do_not_see_what_follows(ai, gpu, maps, dim, vdim, start, rows):
+    """An infinity or NaN among the values reaches its column of the rows from its position on, and nothing else: that stays as it is up to
+    the order of the f32 sums (F32_TOL with one map; the norm behind two enlarges it)."""
+    keys = (start + 5, start + 14, start + rows - 1)
+    clean = attention_case(ai, gpu, "f32", maps, 4, 2, dim, vdim, start, rows, 256)
+    got = attention_case(ai, gpu, "f32", maps, 4, 2, dim, vdim, start, rows, 256, poison=[(keys[0], 3, np.inf), (keys[1], vdim - 1, np.nan), (keys[2], 7, -np.inf)])
+    close(got[:5], clean[:5], F32_TOL if maps == 1 else 1e-4, "rows before")
+    if maps == 1:
+        for t in range(rows):
+            special = {3: np.inf} if t >= 5 else {}
+            if t >= rows - 1:
+                special[7] = -np.inf
+            for c in range(vdim):
+                if c == vdim - 1 and t >= 14:
+                    assert np.isnan(got[t, :, c]).all()
+                elif c in special:
+                    assert (got[t, :, c] == special[c]).all()
+                else:
+                    assert np.abs(got[t, :, c] - clean[t, :, c]).max() <= F32_TOL * np.abs(clean).max(), (t, c)
 
 
 def test_attention_long_context_splits(ai, gpu):
