@@ -602,8 +602,9 @@ __global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
 // ---- f32 rows as bf16 terms ----------------------------------------------------------------------------------------------
 // An f32 value is the sum of three bf16 values that are cut off, not rounded, so that all have its sign: 8 bits each, 24 in all.  The
 // products with bf16 weights are then exact and summed in f32, as FMA has them, on the matrix cores; a row becomes its lowest terms,
-// its middle terms and its leading terms, one after the other.  A term that is zero of a value that is not becomes a tiny one of
-// its sign, far below what f32 sums see: an infinite weight then gives the infinity that it gives times the value itself.
+// its middle terms and its leading terms, one after the other.  No term is zero, or an infinite weight would give NaN where it gives an
+// infinity times the value itself: a value of fewer bits passes its last one on to the terms below (values from 2^-110 up; smaller ones
+// lose bits below bf16's range).
 // (The products of a pass over 333 rows at width 1024: 184 us on average on the FMA units, 30 and 6 for the terms.)
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, uint16_t* __restrict__ out, uint32_t rows, uint32_t K, uint32_t lda, uint32_t stride) {
     const uint32_t per = stride / 4, row = blockIdx.y * 4 + threadIdx.x / 64;
@@ -621,12 +622,17 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
                 continue;
             }
             const float hi = __builtin_bit_cast(float, u & 0xFFFF0000u), r = f[j] - hi;
-            const uint32_t ru = __builtin_bit_cast(uint32_t, r), tiny = __builtin_bit_cast(uint32_t, f[j] * 0x1p-100f) >> 16;
-            const float mid = __builtin_bit_cast(float, ru & 0xFFFF0000u);
-            const uint32_t lo = __builtin_bit_cast(uint32_t, r - mid) >> 16;
-            t[0][j] = (lo & 0x7FFFu) ? lo : tiny;
-            t[1][j] = (ru & 0x7FFF0000u) ? ru >> 16 : tiny;
-            t[2][j] = u >> 16;
+            // (the last bit of a bf16 value: seven places below its exponent, none where that is below the normal ones)
+            auto bit_of = [](float v, uint32_t places) {
+                const uint32_t e = __builtin_bit_cast(uint32_t, v) & 0x7F800000u, s = __builtin_bit_cast(uint32_t, v) & 0x80000000u;
+                return e > (places << 23) ? __builtin_bit_cast(float, (e - (places << 23)) | s) : 0.0f;
+            };
+            float top = hi, mid = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xFFFF0000u), low = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r - mid) & 0xFFFF0000u);
+            if (r == 0.0f) { mid = low = bit_of(hi, 8); top = hi - (mid + low); }
+            else if (r == mid) { low = bit_of(mid, 7); mid -= low; }
+            t[0][j] = __builtin_bit_cast(uint32_t, low) >> 16;
+            t[1][j] = __builtin_bit_cast(uint32_t, mid) >> 16;
+            t[2][j] = __builtin_bit_cast(uint32_t, top) >> 16;
         }
         uint16_t* o = out + (size_t)row * 3 * stride + k;
 #pragma unroll

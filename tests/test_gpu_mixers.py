@@ -180,6 +180,28 @@ def test_f32_rows_as_terms(ai, gpu, m, k, n):
     assert (np.abs(got[fine] - want[fine]) <= ((3 * k / 32 + 32) * 2.0 ** -24 * size)[fine]).all()
 
 
+@pytest.mark.parametrize("bits", [1, 2, 7, 8, 9, 15, 16, 17, 24])
+def test_terms_of_small_f32_values(ai, gpu, bits):
+    """Values of every number of bits from 2^-100 to 2^100 against infinite weights, and one by one against finite ones: their three terms are
+    exact, so a product of 8 bits more is off by its roundings only, one per term."""
+    ctx, K = gpu
+    g, L, m, k = np.random.default_rng(bits), ai.linear_weight, 201, 64
+    top = g.integers(2 ** (bits - 1), 2 ** bits, (m, k)).astype(np.float64)
+    top[:, :4] = 2.0 ** (bits - 1), 2.0 ** bits - 1, 2.0 ** (bits - 1), 2.0 ** bits - 1
+    x = top * np.where(g.random((m, k)) < 0.5, -1.0, 1.0) * 2.0 ** (np.arange(-100, 101) - bits + 1.0)[:, None]
+    assert np.array_equal(x, x.astype(np.float32))
+    w = np.zeros((2 * k, k))
+    w[np.arange(k), np.arange(k)], w[k + np.arange(k), np.arange(k)] = np.inf, M.rounded(g.standard_normal(k))
+    out, batch = empty(ai, ctx, m * 2 * k, ai.F32), ai.CommandBatch(ctx)
+    lin = L.StackedLinear(ctx, [M.bf16_bits(w)], [L.Segment(2 * k)])
+    print(f"small terms {bits}", flush=True)
+    lin.rows_into(batch, K, upload(ai, ctx, x, ai.F32), ai.F32, m, [out], ai.F32)
+    batch.commit_and_wait()
+    got, want = download(ai, out, m * 2 * k, ai.F32).reshape(m, 2 * k), x * w[k:].sum(1)
+    assert np.array_equal(got[:, :k], np.sign(x) * np.inf)
+    assert (np.abs(got[:, k:] - want) <= 3 * 2.0 ** -24 * np.abs(want)).all()
+
+
 @pytest.mark.parametrize("m,pos,k,heads,dim,pad,vdim", [(2048, 0, 64, 8, 128, 128, 128), (1500, 32, 128, 8, 96, 128, 160), (1500, 5, 64, 8, 96, 128, 160),
                                                         (1100, 64, 64, 12, 80, 96, 144), (130, 32, 64, 2, 32, 32, 64), (300, 0, 128, 3, 40, 64, 96), (64, 96, 72, 2, 32, 32, 64)])
 def test_caches_of_many_rows(ai, gpu, m, pos, k, heads, dim, pad, vdim):
