@@ -32,26 +32,28 @@ struct DirectArgs {
     uint16_t* y[8];
     const void* x;             // f16; before a rotation f32
     uint32_t count, rows, K;
-    uint32_t xstride, ystride; // bytes between the vectors of a batch and their outputs: vector blockIdx.y (one matrix, no prologue)
+    uint32_t batch, xstride, ystride;   // vectors, and bytes between them and between their outputs (several: one matrix, no prologue)
     XPrologue pro;
 };
 
 // A workgroup of ng x teams waves, ng = ceil(K / 2048): wave w takes the block group w % ng of the row pairs of team w / ng.
-// NR: rounds of eight elements per thread that cover the vector.
-template <int FMT, int KIND, int NR, int MAXT>
+// NR: rounds of eight elements per thread that cover the vector.  V: vectors V blockIdx.y .. of a batch that the workgroup multiplies each
+// code with once it is apart (the last ones may repeat the last vector); what a vector gives does not depend on V.
+template <int FMT, int KIND, int NR, int MAXT, int V>
 __global__ __launch_bounds__(MAXT) void matvec_direct_kernel(const DirectArgs a) {
     extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nthreads = blockDim.x;
     const uint32_t ng = (a.K + 2047) >> 11, teams = (nthreads >> 6) / ng, team = wave / ng, grp = wave - team * ng;
-    uint4* const xs = reinterpret_cast<uint4*>(lds);                                   // [ng][8 chunks of 8 elements][32 lanes]
-    float* const parts = reinterpret_cast<float*>(lds + (size_t)ng * 4096);             // [waves][64]
-    float* const sums = parts + (nthreads >> 6) * 64;                                   // [2][16]
+    uint4* const xs = reinterpret_cast<uint4*>(lds);                                   // [V][ng][8 chunks of 8 elements][32 lanes]
+    float* const parts = reinterpret_cast<float*>(lds + (size_t)V * ng * 4096);         // [V][waves][64]
+    float* const sums = parts + V * (nthreads >> 6) * 64;                               // [2][16]
 
     // ---- the vector, requested ahead of the weights: loads return in order
-    uint4 va[NR], vb[NR];
+    static_assert(V == 1 || KIND == kXProNone, "a batch of vectors has no prologue");
+    uint4 va[V * NR], vb[NR];
     [[maybe_unused]] uint4 vr[NR], vg[NR];
     [[maybe_unused]] float4 sa[NR], sb[NR];
-    const uint16_t* const xh = reinterpret_cast<const uint16_t*>(static_cast<const char*>(a.x) + (size_t)blockIdx.y * a.xstride);
+    const uint32_t v0 = blockIdx.y * V;
 #pragma unroll
     for (int i = 0; i < NR; i++) {
         const uint32_t e = min((i * nthreads + tid) * 8, a.K - 8);
@@ -61,9 +63,13 @@ __global__ __launch_bounds__(MAXT) void matvec_direct_kernel(const DirectArgs a)
             vb[i] = *reinterpret_cast<const uint4*>(x + 4);
             sa[i] = *reinterpret_cast<const float4*>(s);
             sb[i] = *reinterpret_cast<const float4*>(s + 4);
-        } else va[i] = *reinterpret_cast<const uint4*>(xh + e);
+        } else
+#pragma unroll
+            for (int j = 0; j < V; j++)
+                va[j * NR + i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(static_cast<const char*>(a.x) + (size_t)min(v0 + j, a.batch - 1) * a.xstride) + e);
         if constexpr (KIND == kXProRmsNorm || KIND == kXProGeluMul) vb[i] = *reinterpret_cast<const uint4*>(a.pro.aux + e);
         if constexpr (KIND == kXProRmsNorm) {
+            const uint16_t* const xh = static_cast<const uint16_t*>(a.x);
             vr[i] = *reinterpret_cast<const uint4*>((a.pro.res ? a.pro.res : xh) + e);
             vg[i] = *reinterpret_cast<const uint4*>((a.pro.aux2 ? a.pro.aux2 : xh) + e);
         }
@@ -130,10 +136,11 @@ __global__ __launch_bounds__(MAXT) void matvec_direct_kernel(const DirectArgs a)
         if (a.pro.aux2) rms2 = rsqrtf(total_of(s, sums + 16) / (float)a.K + a.pro.eps);
     }
 #pragma unroll
-    for (int i = 0; i < NR; i++) {
+    for (int p = 0; p < V * NR; p++) {
+        const int i = p % NR;
         const uint32_t e = (i * nthreads + tid) * 8;
         const bool in = e < a.K;
-        uint32_t w[4] = {va[i].x, va[i].y, va[i].z, va[i].w};
+        uint32_t w[4] = {va[p].x, va[p].y, va[p].z, va[p].w};
         if constexpr (KIND == kXProRmsNorm) {
             if (a.pro.aux2) {
                 const uint32_t g[4] = {vg[i].x, vg[i].y, vg[i].z, vg[i].w};
@@ -169,38 +176,58 @@ __global__ __launch_bounds__(MAXT) void matvec_direct_kernel(const DirectArgs a)
                     w[j] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
                     w[j + 1] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
                 }
-            xs[((e >> 11) * 8 + chunk) * 32 + to] = in ? make_uint4(w[0], w[1], w[2], w[3]) : make_uint4(0u, 0u, 0u, 0u);
+            xs[((p / NR * ng + (e >> 11)) * 8 + chunk) * 32 + to] = in ? make_uint4(w[0], w[1], w[2], w[3]) : make_uint4(0u, 0u, 0u, 0u);
         }
     }
     lh_lds_barrier();
-    uint32_t x[8][4];                                         // the lane's eight chunks
+    uint32_t x[V][8][4];                                      // the lane's eight chunks
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const uint4 t = xs[(grp * 8 + c) * 32 + l];
-        x[c][0] = t.x; x[c][1] = t.y; x[c][2] = t.z; x[c][3] = t.w;
-    }
+    for (int j = 0; j < V; j++)
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const uint4 t = xs[((j * ng + grp) * 8 + c) * 32 + l];
+            x[j][c][0] = t.x; x[j][c][1] = t.y; x[j][c][2] = t.z; x[j][c][3] = t.w;
+        }
 
-    float mine = 0.0f;                                        // lane 32 h + i: row h of the wave's pair i (32 of them at most)
+    float mine[V];                                            // lane 32 h + i: row h of the wave's pair i (32 of them at most)
+#pragma unroll
+    for (int j = 0; j < V; j++) mine[j] = 0.0f;
     lh_walk_rows(v, count, issue, [&](const Pair& p, uint32_t i) {
-        float part = 0.0f;
+        float part[V];
         if constexpr (FMT == LH_TQ2_0) {
-            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            float acc[V][4];
+#pragma unroll
+            for (int j = 0; j < V; j++)
+#pragma unroll
+                for (int f = 0; f < 4; f++) acc[j][f] = 0.0f;
 #pragma unroll
             for (int m = 0; m < 4; m++)
 #pragma unroll
                 for (int f = 0; f < 4; f++) {
                     // the high bytes of f16(code - 1), the low ones are zero: four at a time from a table, then apart
                     const uint32_t hi = __builtin_amdgcn_perm(0u, 0x403C00BCu, (p.w[m] >> (2 * f)) & 0x03030303u);
-                    const uint32_t* xc = &x[2 * f + (m >> 1)][2 * (m & 1)];
-                    acc[f] += lh_dot2h(__builtin_amdgcn_perm(0u, hi, 0x010C000Cu), xc[0], lh_dot2h(__builtin_amdgcn_perm(0u, hi, 0x030C020Cu), xc[1], 0.0f));
+                    const uint32_t c0 = __builtin_amdgcn_perm(0u, hi, 0x010C000Cu), c1 = __builtin_amdgcn_perm(0u, hi, 0x030C020Cu);
+#pragma unroll
+                    for (int j = 0; j < V; j++) {
+                        const uint32_t* xc = &x[j][2 * f + (m >> 1)][2 * (m & 1)];
+                        acc[j][f] += lh_dot2h(c0, xc[0], lh_dot2h(c1, xc[1], 0.0f));
+                    }
                 }
-            part = ((acc[0] + acc[1]) + (acc[2] + acc[3])) * lh_h2f((uint16_t)p.d);
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                part[j] = ((acc[j][0] + acc[j][1]) + (acc[j][2] + acc[j][3])) * lh_h2f((uint16_t)p.d);
+                asm volatile("" : "+v"(part[j]));             // rounded here, not in an addition of the sum over the lanes: in every variant the same
+            }
         } else {
             // scale, 4 words of codes; twice: the first block's codes lie two bytes into a word
             const uint32_t w[9] = {p.w[0], p.w[1], p.w[2], p.w[3], p.w1[0], p.w1[1], p.w1[2], p.w1[3], p.d};
 #pragma unroll
+            for (int j = 0; j < V; j++) part[j] = 0.0f;
+#pragma unroll
             for (int b = 0; b < 2; b++) {
-                float acc[2] = {0.0f, 0.0f};
+                float acc[V][2];
+#pragma unroll
+                for (int j = 0; j < V; j++) acc[j][0] = acc[j][1] = 0.0f;
 #pragma unroll
                 for (int m = 0; m < 4; m++) {
                     const uint32_t c = b ? w[5 + m] : __builtin_amdgcn_alignbit(w[m + 1], w[m], 16), c8 = c >> 8;
@@ -211,25 +238,39 @@ __global__ __launch_bounds__(MAXT) void matvec_direct_kernel(const DirectArgs a)
                     const f16x2 lo1 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, (c8 & 0x000F000Fu) | 0x64006400u), one, z);
                     const f16x2 hi0 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, (c & 0x00F000F0u) | 0x64006400u), sixteenth, z16);
                     const f16x2 hi1 = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, (c8 & 0x00F000F0u) | 0x64006400u), sixteenth, z16);
-                    const uint32_t *xl = &x[4 * b + (m >> 1)][2 * (m & 1)], *xh = &x[4 * b + 2 + (m >> 1)][2 * (m & 1)];
-                    acc[0] += lh_dot2h(lo0, xl[0], lh_dot2h(lo1, xl[1], 0.0f));
-                    acc[1] += lh_dot2h(hi0, xh[0], lh_dot2h(hi1, xh[1], 0.0f));
+#pragma unroll
+                    for (int j = 0; j < V; j++) {
+                        const uint32_t *xl = &x[j][4 * b + (m >> 1)][2 * (m & 1)], *xh = &x[j][4 * b + 2 + (m >> 1)][2 * (m & 1)];
+                        acc[j][0] += lh_dot2h(lo0, xl[0], lh_dot2h(lo1, xl[1], 0.0f));
+                        acc[j][1] += lh_dot2h(hi0, xh[0], lh_dot2h(hi1, xh[1], 0.0f));
+                    }
                 }
-                part = __builtin_fmaf(acc[0] + acc[1], lh_h2f((uint16_t)(b ? w[4] >> 16 : w[0] & 0xFFFFu)), part);
+#pragma unroll
+                for (int j = 0; j < V; j++) part[j] = __builtin_fmaf(acc[j][0] + acc[j][1], lh_h2f((uint16_t)(b ? w[4] >> 16 : w[0] & 0xFFFFu)), part[j]);
             }
         }
-        const float sum = lh_group_sum(part, 32);
-        mine = i == l ? sum : mine;
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+            const float sum = lh_group_sum(part[j], 32);
+            mine[j] = i == l ? sum : mine[j];
+        }
     });
+    const uint32_t waves = nthreads >> 6;
     if (ng > 1) {
-        parts[wave * 64 + lane] = mine;
+#pragma unroll
+        for (int j = 0; j < V; j++) parts[(j * waves + wave) * 64 + lane] = mine[j];
         lh_lds_barrier();
         if (grp != 0) return;
-        for (uint32_t g = 1; g < ng; g++) mine += parts[(wave + g) * 64 + lane];
+#pragma unroll
+        for (int j = 0; j < V; j++)
+            for (uint32_t g = 1; g < ng; g++) mine[j] += parts[(j * waves + wave + g) * 64 + lane];
     }
     if (l < count) {
         const uint32_t q = first + l * step, pr = problem(q), row = 2 * (q - pr * pairs) + half;
-        if (row < a.rows) reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(a.y[pr]) + (size_t)blockIdx.y * a.ystride)[row] = lh_f2h(mine);
+        if (row < a.rows)
+#pragma unroll
+            for (int j = 0; j < V; j++)
+                if (v0 + j < a.batch) reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(a.y[pr]) + (size_t)(v0 + j) * a.ystride)[row] = lh_f2h(mine[j]);
     }
 }
 
@@ -238,25 +279,39 @@ __global__ __launch_bounds__(MAXT) void matvec_direct_kernel(const DirectArgs a)
 int lh_launch_matvec_direct(lh_context* ctx, lh_quant fmt, uint32_t count, const void* const* matrices, const void* vector, void* const* outputs, uint32_t rows,
                                 uint32_t K, const XPrologue& pro, uint32_t batch, uint32_t xstride, uint32_t ystride) {
     const uint32_t ng = (K + 2047) / 2048;
-    if (count > 8 || ng > 6) return -1;
+    if (count > 8 || ng > 6 || (batch > 1 && (count > 1 || pro.kind != kXProNone))) return -1;
     const uint32_t waves = ng == 1 || ng == 2 || ng == 4 ? 8 : 2 * ng, teams = waves / ng, rounds = (ng * 2048 + waves * 512 - 1) / (waves * 512);   // rounds: 1 or 2
-    // A workgroup per CU.  Beyond 8 pairs of rows per wave (16 where a row takes several waves) the unpacking is what takes the time, and the
-    // matrix cores do the rest of the work for nothing: 65536 x 1536 (16 per wave) 13.1 us against 11.2 there, 32768 x 2048 (8) 8.3
-    // against 8.7; 16384 x 12288 (16) 19.1 against 22.2.
-    const uint64_t total = (uint64_t)((rows + 1) / 2) * count;
-    // A batch of vectors, in microseconds against the form with v_dot4: up to 12 per wave 8 x 1536 x 12288 18.0 and 29.4, 4 x 12288 x 1536 11.3 and
-    // 12.8, 8 x 256 x 1536 3.7 and 4.7; 16 (8 x 8192 x 2048) 14.0 and 13.4, 24 (4 x 24576 x 1536) 19.6 and 18.6.
-    const uint32_t most = batch > 1 ? 12 : ng == 1 ? 8 : 16;
-    if (batch * total > (uint64_t)ctx->cu_count * teams * most) return -1;
-    const uint64_t fill = std::max<uint64_t>(batch == 1 ? ctx->cu_count : 2 * ctx->cu_count / batch, (total + (uint64_t)teams * most - 1) / ((uint64_t)teams * most));
-    const dim3 grid((uint32_t)std::min<uint64_t>((total + teams - 1) / teams, fill), batch);
-    DirectArgs a{{}, {}, vector, count, rows, K, xstride, ystride, pro};
+    // Beyond 8 pairs of rows per wave of a workgroup per CU (16 where a row takes several waves) the unpacking is what takes the time, and
+    // the matrix cores do the rest of the work for nothing: 65536 x 1536 (16 per wave) 13.1 us against 11.2 there, 32768 x 2048 (8) 8.3
+    // against 8.7; 16384 x 12288 (16) 19.1 against 22.2.  The line does not depend on the batch: what a vector gives alone it gives in one.
+    const uint64_t total = (uint64_t)((rows + 1) / 2) * count, slots = (uint64_t)ctx->cu_count * teams;
+    if (total > slots * (ng == 1 ? 8 : 16)) return -1;
+    // Vectors of a batch that share the unpacked codes.  Up to a pair of rows per wave (three where a row takes several) each vector has
+    // workgroups of its own, then two share one, from nine on four, where there are 256 registers for them.  Q4_0, in microseconds with 1, 2 and 4, and in
+    // the form with v_dot4: 8 x 256 x 1536 3.6, 4.0, 5.2, 4.6; 3 x 1536 x 2048 5.0, 4.3, 5.3, 5.9; 4 x 8960 x 1536 9.7, 8.1, 8.8, 10.5;
+    // 8 x 24576 x 1536 46, 27, 23, 27.
+    const uint64_t load = batch * total;
+    const uint32_t v = batch == 1 || load <= slots * (ng == 1 ? 1 : 3) ? 1 : batch > 2 && waves <= 8 && load >= slots * 9 ? 4 : 2;
+    const uint32_t groups = (batch + v - 1) / v;
+    // A workgroup per CU, and a wave's results fit its half of the lanes.
+    const uint64_t fill = std::max<uint64_t>({(uint64_t)ctx->cu_count / groups, 1, (total + (uint64_t)teams * 32 - 1) / ((uint64_t)teams * 32)});
+    const dim3 grid((uint32_t)std::min<uint64_t>((total + teams - 1) / teams, fill), groups);
+    DirectArgs a{{}, {}, vector, count, rows, K, batch, xstride, ystride, pro};
     for (uint32_t i = 0; i < count; i++) { a.m[i] = (const uint8_t*)matrices[i]; a.y[i] = (uint16_t*)outputs[i]; }
-    const size_t lds = (size_t)ng * 4096 + ((size_t)waves * 64 + 32) * 4;
-#define LH_DIRECT(FMT, KIND, NR)                                                                                                              \
-    do {                                                                                                                                      \
-        if (waves <= 8) hipLaunchKernelGGL((matvec_direct_kernel<FMT, KIND, NR, 512>), grid, dim3(64 * waves), lds, ctx->stream, a);     \
-        else hipLaunchKernelGGL((matvec_direct_kernel<FMT, KIND, NR, 768>), grid, dim3(64 * waves), lds, ctx->stream, a);                \
+    const size_t lds = (size_t)v * ng * 4096 + ((size_t)v * waves * 64 + 32) * 4;
+    int r = LH_OK;
+#define LH_DIRECT_V(FMT, KIND, NR, MAXT, V)                                                                                                              \
+    do {                                                                                                                                                 \
+        if (lds > 65536) r = lh_raise_dynamic_lds(ctx, (const void*)matvec_direct_kernel<FMT, KIND, NR, MAXT, V>, lds, "matvec_quant");                   \
+        if (r == LH_OK) hipLaunchKernelGGL((matvec_direct_kernel<FMT, KIND, NR, MAXT, V>), grid, dim3(64 * waves), lds, ctx->stream, a);                 \
+    } while (0)
+#define LH_DIRECT(FMT, KIND, NR)                                         \
+    do {                                                                 \
+        if (v == 4) LH_DIRECT_V(FMT, kXProNone, NR, 512, 4);             \
+        else if (v == 2 && waves <= 8) LH_DIRECT_V(FMT, kXProNone, NR, 512, 2); \
+        else if (v == 2) LH_DIRECT_V(FMT, kXProNone, NR, 768, 2);        \
+        else if (waves <= 8) LH_DIRECT_V(FMT, KIND, NR, 512, 1);         \
+        else LH_DIRECT_V(FMT, KIND, NR, 768, 1);                         \
     } while (0)
 #define LH_DIRECT_KIND(FMT, KIND) do { if (rounds == 1) LH_DIRECT(FMT, KIND, 1); else LH_DIRECT(FMT, KIND, 2); } while (0)
 #define LH_DIRECT_FMT(FMT)                                                    \
@@ -271,5 +326,5 @@ int lh_launch_matvec_direct(lh_context* ctx, lh_quant fmt, uint32_t count, const
 #undef LH_DIRECT_FMT
 #undef LH_DIRECT_KIND
 #undef LH_DIRECT
-    return lh_check_launch(fmt == LH_TQ2_0 ? "matvec_tq2_0" : "matvec_q4_0");
+    return r != LH_OK ? r : lh_check_launch(fmt == LH_TQ2_0 ? "matvec_tq2_0" : "matvec_q4_0");
 }

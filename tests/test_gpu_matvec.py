@@ -255,29 +255,35 @@ def test_products_of_one_vector(pkg, gpu, oracle, fmt, rows, cols, count, kind):
         assert np.all(np.abs(got - want) <= tol), (worst, got[worst], want[worst], tol[worst])
 
 
-@pytest.mark.parametrize("rows,cols,m", [(1, 64, 2), (257, 1536, 3), (4096, 2048, 4), (1536, 6144, 8), (700, 8256, 5), (6144, 2048, 8), (6150, 2048, 8)])
-def test_vectors_of_a_batch_as_single_ones(pkg, gpu, oracle, rows, cols, m):
-    """A few f16 vectors against one 4-bit matrix give what each gives alone, bit for bit, where both take the form without quantised
-    activations (6150 rows of eight vectors do not).  All are held to the f64 dot: half an f16 step, and 2^-15 of the terms' magnitude for
-    the other form's 16-bit fixed point."""
+@pytest.mark.parametrize("fmt,rows,cols,m", [("q4_0", 1, 64, 2), ("q4_0", 257, 1536, 3), ("q4_0", 4096, 2048, 4), ("q4_0", 1536, 6144, 8), ("q4_0", 700, 8256, 5),
+                                             ("q4_0", 6144, 2048, 8), ("q4_0", 6150, 2048, 8), ("q4_0", 8960, 1536, 6), ("q4_0", 24577, 1536, 7), ("q4_0", 32768, 512, 2),
+                                             ("q4_0", 32770, 512, 4), ("q4_0", 16384, 4096, 3), ("q4_0", 1500, 12288, 8), ("q4_0", 8191, 10304, 6), ("q4_0", 1, 256, 8),
+                                             ("tq2_0", 1, 256, 2), ("tq2_0", 259, 1536, 3), ("tq2_0", 4100, 2048, 8), ("tq2_0", 1030, 8192, 5), ("tq2_0", 700, 12288, 4),
+                                             ("tq2_0", 9001, 1024, 6), ("tq2_0", 24577, 256, 7)])
+def test_vectors_of_a_batch_as_single_ones(pkg, gpu, oracle, fmt, rows, cols, m):
+    """A few f16 vectors against one matrix give what each gives alone, bit for bit, whichever form the matrix takes (32770 rows: not the one
+    without quantised activations) and however many vectors share its codes there; TQ2_0 at row counts that no tile divides (whole tiles
+    go to the matrix kernels from two rows on).  All are held to the f64 dot: half an f16 step, and 2^-15 of the terms' magnitude for the
+    other form's 16-bit fixed point."""
     ctx, K = gpu
     g = pkg.synth.rng(78, rows + cols + m)
-    raw = refgen.q4_0_payload(rows, cols, 0x33)
-    w = pkg.QuantWeight.from_bytes(ctx, raw, pkg.Q4_0, rows, cols)
+    ty, some = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, min(rows, 2050)
+    raw = (refgen.q4_0_payload if fmt == "q4_0" else refgen.tq2_0_payload)(some, cols, 0x33)
+    pick = np.arange(rows) % some
+    w = pkg.QuantWeight.from_bytes(ctx, np.ascontiguousarray(raw.reshape(some, -1)[pick]).reshape(-1), ty, rows, cols)
     x = g.standard_normal((m, cols), dtype=np.float32).astype(np.float16)
     y, batch = pkg.Buffer.empty(ctx, m * rows * 2), pkg.CommandBatch(ctx)
-    print(f"batch of vectors {rows}x{cols} m{m}", flush=True)
+    print(f"batch of vectors {fmt} {rows}x{cols} m{m}", flush=True)
     w.matmul_nt_into(batch, K, pkg.Buffer.from_slice(ctx, x), y, m)
     single = [pkg.Buffer.empty(ctx, rows * 2) for _ in range(m)]
     for i, o in enumerate(single):
         w.matvec_into(batch, K, pkg.Buffer.from_slice(ctx, x[i]), o)
     batch.commit_and_wait()
-    got, dq = y.as_array(np.float16, m * rows).reshape(m, rows), oracle.expand_q4_0_f32(raw, rows, cols).astype(np.float64)
-    want, size = x.astype(np.float64) @ dq.T, np.abs(x.astype(np.float64)) @ np.abs(dq).T
+    got, dq = y.as_array(np.float16, m * rows).reshape(m, rows), (oracle.expand_q4_0_f32 if fmt == "q4_0" else oracle.expand_tq2_0_f32)(raw, some, cols).astype(np.float64)
+    want, size = (x.astype(np.float64) @ dq.T)[:, pick], (np.abs(x.astype(np.float64)) @ np.abs(dq).T)[:, pick]
     assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -11 + size * 2.0 ** -15 + 2.0 ** -24)
     for i, o in enumerate(single):
-        if rows != 6150:
-            assert np.array_equal(got[i].view(np.uint16), o.as_array(np.uint16, rows))
+        assert np.array_equal(got[i].view(np.uint16), o.as_array(np.uint16, rows)), i
 
 
 @pytest.mark.parametrize("fmt,rows,cols,count", [("q4_0", 256, 2048, 1), ("tq2_0", 8192, 2048, 2), ("tq2_0", 300, 512, 2),
