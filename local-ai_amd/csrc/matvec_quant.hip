@@ -723,9 +723,10 @@ int matvec_dispatch(lh_batch* batch, lh_quant fmt, uint32_t count, const lh_buff
                           (const char*)outputs[i]->ptr == y0 + (size_t)i * ystride;
         }
     }
-    // One vector of f16 values and not too many rows: the form without quantised activations.  (More than two grouped matrices inside a
-    // captured graph are refused below, unless they are evenly spaced.)
-    bool one_vector = xt == (pro.kind == kXProRotate ? LH_F32 : LH_F16) && yt == LH_F16 && count <= 8 && !regular && (count <= 2 || !ctx->capturing) &&
+    // One vector of f16 values and not too many rows: the form without quantised activations, wherever the matrices lie.  (It needs no
+    // descriptors, but more than two matrices inside a captured graph stay refused unless they are evenly spaced: what may be recorded
+    // does not depend on the types.)
+    bool one_vector = xt == (pro.kind == kXProRotate ? LH_F32 : LH_F16) && yt == LH_F16 && count <= 8 && (count <= 2 || regular || !ctx->capturing) &&
                       !(fmt == LH_TQ2_0 && !tq2_on_matrix_cores());
     for (uint32_t i = 1; one_vector && i < count; i++) one_vector = vectors[i]->ptr == vectors[0]->ptr;
     if (one_vector) {

@@ -495,6 +495,53 @@ def test_grouped_evenly_spaced_problems(pkg, gpu, oracle, fmt, rows, cols, count
             refgen.assert_close(a, want, 1e-3, f"{fmt} grouped #{i}")
 
 
+@pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
+@pytest.mark.parametrize("rows,cols,count", [(513, 512, 3), (40, 2048, 8), (1030, 12288, 4), (77, 2304, 5), (6144, 1536, 6)])
+def test_grouped_f16_problems_wherever_they_lie(pkg, gpu, fmt, rows, cols, count):
+    """Up to eight f16 products of one vector in a launch: the same bits whether matrices and outputs are evenly spaced or not, recorded or
+    not, and those of the launches issued one by one where the group as a whole is small enough for their form (6 x 6144 is not)."""
+    ctx, K = gpu
+    g = pkg.synth.rng(46, rows + cols + count)
+    ty, wb = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, pkg.synth.weight_bytes(fmt, rows, cols)
+    raws = [pkg.synth.weights(fmt, rows, cols, g) for _ in range(count)]
+    step = wb + (-wb) % 64
+    big, out = pkg.Buffer.empty(ctx, step * (count + 1)), pkg.Buffer.empty(ctx, (rows + 32) * 2 * (count + 1))
+    x = pkg.Buffer.from_slice(ctx, g.standard_normal(cols, dtype=np.float32).astype(np.float16))
+    one = pkg.Buffer.empty(ctx, rows * 2)
+    print(f"grouped f16 {fmt} {rows}x{cols} x{count}", flush=True)
+    results = []
+    for even in (True, False):
+        place = [i + (not even and i == count - 1) for i in range(count)]
+        for i, r in zip(place, raws):
+            big.copy_from_bytes(r, i * step)
+        ws, ys = [big.view(i * step, wb) for i in place], [out.view(i * (rows + 32) * 2, rows * 2) for i in place]
+        batch = pkg.CommandBatch(ctx)
+        K.matvec_quant_grouped_into(batch, ty, ws, [x] * count, pkg.F16, ys, pkg.F16, rows, cols)
+        assert batch.dispatch_count() == 1
+        batch.commit_and_wait()
+        results.append(np.stack([y.as_array(np.uint16, rows) for y in ys]))
+        for y in ys:
+            y.fill_zero()
+        batch.begin_capture()
+        if even:
+            K.matvec_quant_grouped_into(batch, ty, ws, [x] * count, pkg.F16, ys, pkg.F16, rows, cols)
+        else:
+            with pytest.raises(pkg.InvalidArgument):
+                K.matvec_quant_grouped_into(batch, ty, ws, [x] * count, pkg.F16, ys, pkg.F16, rows, cols)
+        graph = batch.end_capture()
+        if even:
+            for _ in range(3):
+                graph.launch()
+                ctx.synchronize()
+                assert np.array_equal(np.stack([y.as_array(np.uint16, rows) for y in ys]), results[0])
+    assert np.array_equal(results[0], results[1])
+    for i, w in enumerate(ws):
+        K.matvec_quant_typed_into(batch, ty, w, x, pkg.F16, one, pkg.F16, rows, cols)
+        batch.commit_and_wait()
+        if rows != 6144:
+            assert np.array_equal(results[0][i], one.as_array(np.uint16, rows)), i
+
+
 @pytest.mark.parametrize("rows,cols,count,shared_x,half", [(2048, 8192, 52, True, False), (1024, 4096, 100, False, False),
                                                            (2032, 8192, 52, True, False), (2048, 8192, 52, False, True)])
 def test_grouped_long_rows_many_tiles(pkg, gpu, oracle, rows, cols, count, shared_x, half):
