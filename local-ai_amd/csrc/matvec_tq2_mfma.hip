@@ -472,6 +472,10 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
     uint32_t split_waves = 1;
     if (tiles < (uint64_t)ctx->cu_count * 2) {
         for (uint32_t w = 4; w >= 2; w--) if (ngroups % w == 0) { split_waves = w; break; }
+        // six groups of blocks (12288 columns; groups of f16 products with a vector each): a wave per group where every tile has a CU, and twice
+        // the threads for the activation staging (2 x 1536 rows: 10.4 us against 13.9; 3 x 1536: 18.7 against 16.7)
+        const size_t lds6 = lds_head_bytes(K) + 128 + 6 * (size_t)kImageBytes + 3 * kStageLoads * 64 * 2 + kSplitAreaBytes;
+        if (ngroups % 6 == 0 && tiles <= (uint64_t)ctx->cu_count && xt == LH_F16 && yt == LH_F16 && lds6 <= kMaxLdsBytes) split_waves = 6;
     }
     const uint32_t splitk = split_waves > 1 ? 1u : 0u;
     constexpr int wg256_tiles_per_cu = 2, wg_cu = 3;
@@ -506,7 +510,8 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
                             : splitk ? (const void*)matvec_tq2_mfma_kernel<XT, YT, true>                                          \
                             : ngroups == 1 ? (const void*)matvec_tq2_mfma_kernel<XT, YT, false, 256, true>                        \
                                            : (const void*)matvec_tq2_mfma_kernel<XT, YT, false>)
-    if (xt == LH_F32 && yt == LH_F32) fn = LH_FN(float, float);
+    if (split_waves == 6) fn = (const void*)matvec_tq2_mfma_kernel<uint16_t, uint16_t, true, 384>;
+    else if (xt == LH_F32 && yt == LH_F32) fn = LH_FN(float, float);
     else if (xt == LH_F16 && yt == LH_F16) fn = LH_FN(uint16_t, uint16_t);
     else if (xt == LH_F16 && yt == LH_F32) fn = LH_FN(uint16_t, float);
     else fn = LH_FN(float, uint16_t);

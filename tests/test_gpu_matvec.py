@@ -542,6 +542,22 @@ def test_grouped_f16_problems_wherever_they_lie(pkg, gpu, fmt, rows, cols, count
             assert np.array_equal(results[0][i], one.as_array(np.uint16, rows)), i
 
 
+@pytest.mark.parametrize("rows,count", [(17, 2), (1536, 2), (512, 8), (513, 8), (256, 9), (700, 5), (1, 3)])
+def test_grouped_long_f16_problems_with_their_own_vectors(pkg, gpu, oracle, rows, count):
+    """Groups of f16 products over 12288 columns, a vector each: up to a 16-row tile per CU six waves share a tile's columns."""
+    ctx, K = gpu
+    cols, g = 12288, pkg.synth.rng(47, rows + count)
+    raws = [pkg.synth.weights("tq2_0", rows, cols, g) for _ in range(count)]
+    ws = [pkg.QuantWeight.from_bytes(ctx, r, pkg.TQ2_0, rows, cols) for r in raws]
+    xs = [g.standard_normal(cols, dtype=np.float32).astype(np.float16) for _ in range(count)]
+    ys, batch = [pkg.Buffer.empty(ctx, rows * 2) for _ in range(count)], pkg.CommandBatch(ctx)
+    print(f"grouped long f16 {rows} x{count}", flush=True)
+    K.matvec_quant_grouped_into(batch, pkg.TQ2_0, [w.buf for w in ws], [pkg.Buffer.from_slice(ctx, x) for x in xs], pkg.F16, ys, pkg.F16, rows, cols)
+    batch.commit_and_wait()
+    for r, x, y in zip(raws, xs, ys):
+        refgen.assert_close(y.as_array(np.float16, rows).astype(np.float32), oracle.matvec_quant_ref("tq2_0", r, x.astype(np.float32), rows, cols, threads=8), 2e-3, f"{rows} x{count}")
+
+
 @pytest.mark.parametrize("rows,cols,count,shared_x,half", [(2048, 8192, 52, True, False), (1024, 4096, 100, False, False),
                                                            (2032, 8192, 52, True, False), (2048, 8192, 52, False, True)])
 def test_grouped_long_rows_many_tiles(pkg, gpu, oracle, rows, cols, count, shared_x, half):
