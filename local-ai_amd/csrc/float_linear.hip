@@ -875,16 +875,16 @@ __global__ __launch_bounds__(256) void matvec_bf16_kernel(const VectorStage st, 
     sums.flush();
 }
 
-// The same with the vector in registers (K up to 512 * NL), eight waves that bring it in together; the weights of two rows are
+// The same with the vector in registers (K up to 512 * NL), which the waves of a workgroup bring in together; the weights of two rows are
 // requested right behind it and every wait leaves the younger loads on their way.  What bounds it is the length of one such chain, not
 // the bytes.  (Four waves, each with the vector for itself and one row ahead: 10.0 us a launch on average over the products of a step
-// behind a norm, 2048 columns and 2048 to 32000 rows, 10.6 behind a gate, 5.9 with neither; now 8.9, 5.8 and 4.0.)
-template <int STAGE, int NL>
-__global__ __launch_bounds__(512) void matvec_bf16_reg_kernel(const VectorStage st, const uint16_t* __restrict__ W, const float* __restrict__ bias, const LhSegments seg,
+// behind a norm, 2048 columns and 2048 to 32000 rows, 10.6 behind a gate, 5.9 with neither; with eight waves 8.9, 5.8 and 4.0.)
+template <int STAGE, int NL, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void matvec_bf16_reg_kernel(const VectorStage st, const uint16_t* __restrict__ W, const float* __restrict__ bias, const LhSegments seg,
                                                              uint32_t N, uint32_t K) {
-    __shared__ LhVectorSpace space;
+    __shared__ LhVectorSpace<WAVES> space;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), last = (K >> 3) - 1;
-    const RowWalk walk{blockIdx.x * kVectorWaves + wave, gridDim.x * kVectorWaves, seg.pairs};
+    const RowWalk walk{blockIdx.x * WAVES + wave, gridDim.x * WAVES, seg.pairs};
     const uint32_t rows = walk.rows(N);
     struct Row { uint4 w[NL]; } v[2];
     auto issue = [&](Row& x, uint32_t i) {
@@ -892,7 +892,7 @@ __global__ __launch_bounds__(512) void matvec_bf16_reg_kernel(const VectorStage 
 #pragma unroll
         for (int c = 0; c < NL; c++) x.w[c] = lh_ld16_stream(wr + 8 * min(64u * c + lane, last));
     };
-    LhSharedVector<STAGE, NL> x;
+    LhSharedVector<STAGE, NL, WAVES> x;
     x.fetch(st, K, lane, wave);
     lh_first_rows(v, max(rows, 1u), [&](Row& r, uint32_t i) { issue(r, rows ? i : 0u); });
     RowSums sums{seg, bias, walk, lane};
@@ -965,25 +965,36 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
     const size_t lds = (size_t)(K + 511) / 512 * 512 * 4;
     const uint32_t takes = seg.pairs ? N / 2 : N;             // rows, or pairs of rows
     const bool vec = K % 8 == 0 && ((uintptr_t)W & 15) == 0;
-    if (vec && K <= 4096 && lh_stage_aligned(st)) {
+    const uint64_t cus = (uint64_t)ctx->cu_count;
+    // Up to eight rows per CU: workgroups of four waves, so that twice as many CUs have one (2048 x 2048 behind a norm 4.7 us with eight,
+    // 4.1 with four, 1024 x 2048 4.3 and 3.7, 512 x 512 3.1 and 2.8), and beyond 2048 columns, for plain vectors, a row over eight waves
+    // (below: 1024 x 4096 5.2 us and 4.4, 2048 x 4096 6.4 and 5.6; 4096 x 4096 7.5 and 7.8).
+    const bool few = takes <= 8 * cus;
+    if (vec && K <= 4096 && lh_stage_aligned(st) && !(STAGE == kPlain && K > 2048 && few)) {
+        const uint32_t w = K <= 2048 && few ? 4 : kVectorWaves;
         // A workgroup for every CU first; a second one where rows are short and each of its waves still has two (32000 x 1024: 11.9 us
         // against 12.5; 8192 x 2048: 7.8 against 7.65).
-        const uint64_t cus = (uint64_t)ctx->cu_count, most = std::max(cus, K <= 1024 ? std::min<uint64_t>(2 * cus, ((uint64_t)takes + 15) / 16) : 0);
+        const uint64_t most = std::max(cus, K <= 1024 ? std::min<uint64_t>(2 * cus, ((uint64_t)takes + 15) / 16) : 0);
         const uint32_t each = seg.pairs ? 32 : 64;           // a wave's sums fit its lanes
-        const uint32_t grid = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(((uint64_t)takes + kVectorWaves - 1) / kVectorWaves, most),
-                                                           ((uint64_t)takes + kVectorWaves * each - 1) / (kVectorWaves * each));
-#define LH_MVR(NLOADS) hipLaunchKernelGGL((matvec_bf16_reg_kernel<STAGE, NLOADS>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K)
-        if (K <= 512) LH_MVR(1);
-        else if (K <= 1024) LH_MVR(2);
-        else if (K <= 2048) LH_MVR(4);
-        else LH_MVR(8);
+        const uint32_t grid = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(((uint64_t)takes + w - 1) / w, most),
+                                                           ((uint64_t)takes + w * each - 1) / (w * each));
+#define LH_MVR(NLOADS, WAVES) hipLaunchKernelGGL((matvec_bf16_reg_kernel<STAGE, NLOADS, WAVES>), dim3(grid), dim3(64 * WAVES), 0, ctx->stream, st, W, bias, seg, N, K)
+        if (w == 4) {
+            if (K <= 512) LH_MVR(1, 4);
+            else if (K <= 1024) LH_MVR(2, 4);
+            else LH_MVR(4, 4);
+        } else if (K <= 512) LH_MVR(1, 8);
+        else if (K <= 1024) LH_MVR(2, 8);
+        else if (K <= 2048) LH_MVR(4, 8);
+        else LH_MVR(8, 8);
 #undef LH_MVR
         return lh_check_launch(op);
     }
     if constexpr (STAGE == kPlain) if (vec && K <= 16384 && lh_stage_aligned(st)) {
         const uint32_t part = ((K + 7) / 8 + 7) / 8 * 8, each = seg.pairs ? 32 : 64;
-        const uint32_t grid = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(takes, (uint64_t)ctx->cu_count), ((uint64_t)takes + each - 1) / each);
-        if (part <= 1024) hipLaunchKernelGGL((matvec_bf16_part_kernel<2, 4>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
+        const uint32_t grid = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(takes, cus), ((uint64_t)takes + each - 1) / each);
+        if (part <= 512) hipLaunchKernelGGL((matvec_bf16_part_kernel<1, 4>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
+        else if (part <= 1024) hipLaunchKernelGGL((matvec_bf16_part_kernel<2, 4>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
         else hipLaunchKernelGGL((matvec_bf16_part_kernel<4, 2>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
         return lh_check_launch(op);
     }

@@ -52,15 +52,17 @@ __device__ __forceinline__ void lh_ld8(const uint16_t* p, float (&v)[8]) {
     for (int j = 0; j < 4; j++) { v[2 * j] = __builtin_bit_cast(float, w[j] << 16); v[2 * j + 1] = __builtin_bit_cast(float, w[j] & 0xFFFF0000u); }
 }
 
-// A vector for the registers of eight waves, K a multiple of 8 up to 512 NL, all pointers 16-byte aligned, zero past K: wave c brings in
+// A vector for the registers of W waves, K a multiple of 8 up to 512 NL, all pointers 16-byte aligned, zero past K: wave c brings in
 // the chunks 64 c + lane and what they need, the sums of the norm meet in LDS, and every wave takes the finished vector from there.
-// (Every wave for itself: 16 KB from the caches per wave for 2048 columns with a norm, as much as the weights of two rows.)
+// (Every wave for itself: 16 KB from the caches per wave for 2048 columns with a norm, as much as the weights of two rows.)  Up to 512
+// columns, a chunk a lane, every wave does bring it in for itself: there the barriers are what takes the time (512 x 512 behind a
+// norm with eight waves: 3.3 us with them, 3.1 without).
 //
 // Loads return in order, so what is requested first can be waited for alone: the vector first (`fetch`), then the weights of the first
 // rows, then `finish`.  And behind a load that not every path makes the compiler waits for all there are, so every load here is
 // made: lanes and waves without a chunk load one that exists, and an operand that is not there is read from x.
 constexpr int kVectorWaves = 8;
-struct LhVectorSpace { float4 x[16][64]; float part[kVectorWaves]; };
+template <int W = kVectorWaves> struct LhVectorSpace { float4 x[2 * W][64]; float part[W]; };
 
 // Eight values at element k, stored as f32 or bf16.
 struct LhEither8 {
@@ -77,24 +79,25 @@ struct LhEither8 {
     }
 };
 
-template <int STAGE, int NL>
+template <int STAGE, int NL, int W = kVectorWaves>
 struct LhSharedVector {
-    static_assert(NL <= kVectorWaves, "a chunk per wave");
+    static_assert(NL <= W, "a chunk per wave");
+    static constexpr bool kAlone = NL == 1;
     static constexpr bool kNormed = STAGE == kNorm || STAGE == kGated || STAGE == kResidual;
     static constexpr bool kAdds = STAGE == kNorm || STAGE == kResidual;
     LhEither8 x, gate;
     float w[8], more[8];
 
     __device__ __forceinline__ void fetch(const VectorStage& st, uint32_t K, uint32_t lane, uint32_t wave) {
-        const uint32_t k = wave < NL ? min((64 * wave + lane) * 8, K - 8) : 0u;
+        const uint32_t k = kAlone ? min(lane * 8, K - 8) : wave < NL ? min((64 * wave + lane) * 8, K - 8) : 0u;
         x.load(st.x, STAGE != kPlain || st.x_f32, k);
         if constexpr (kNormed) lh_ld8((st.norm_weight ? st.norm_weight : static_cast<const float*>(st.x)) + k, w);
         if constexpr (kAdds) lh_ld8((st.add ? st.add : static_cast<const float*>(st.x)) + k, more);
         if constexpr (STAGE == kGated) gate.load(st.gate, st.gate_f32, k);
     }
-    __device__ __forceinline__ void finish(const VectorStage& st, uint32_t K, uint32_t lane, uint32_t wave, bool store, LhVectorSpace& sp, float (&xr)[NL][8]) {
-        const uint32_t k = (64 * wave + lane) * 8;
-        const bool owner = wave < NL, in = owner && k < K;
+    __device__ __forceinline__ void finish(const VectorStage& st, uint32_t K, uint32_t lane, uint32_t wave, bool store, LhVectorSpace<W>& sp, float (&xr)[NL][8]) {
+        const uint32_t k = (64 * (kAlone ? 0u : wave) + lane) * 8;
+        const bool owner = kAlone || wave < NL, in = owner && k < K;
         float v[8], sum = 0.0f;
         x.get(STAGE != kPlain || st.x_f32, v);
         if constexpr (STAGE == kNorm)
@@ -120,25 +123,30 @@ struct LhSharedVector {
             const bool parts = STAGE == kGated && st.group != K;   // group / 8 chunks: a power of two of lanes, or whole sets of 64
             const uint32_t cg = parts ? st.group >> 3 : 64u, width = min(cg, 64u);
             sum = lh_group_sum(sum, (int)width);
-            if (width == 64) {
+            if (!kAlone && width == 64) {
                 if (lane == 0) sp.part[wave] = sum;
                 lh_lds_barrier();
-                const uint32_t per = parts ? cg >> 6 : (uint32_t)kVectorWaves, w0 = wave / per;
+                const uint32_t per = parts ? cg >> 6 : (uint32_t)W, w0 = wave / per;
                 sum = 0.0f;
 #pragma unroll
-                for (int e = 0; e < kVectorWaves; e++) sum += (uint32_t)e / per == w0 ? sp.part[e] : 0.0f;
+                for (int e = 0; e < W; e++) sum += (uint32_t)e / per == w0 ? sp.part[e] : 0.0f;
             }
             const float r = rsqrtf(sum / (float)(parts ? st.group : K) + st.eps);
             if constexpr (STAGE == kResidual)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = __builtin_fmaf(w[j], r, v[j]);
-            if (STAGE != kGated && store && in) {
+            if (STAGE != kGated && store && in && (!kAlone || wave == 0)) {
                 *reinterpret_cast<float4*>(st.store + k) = make_float4(v[0], v[1], v[2], v[3]);
                 *reinterpret_cast<float4*>(st.store + k + 4) = make_float4(v[4], v[5], v[6], v[7]);
             }
             if constexpr (STAGE != kResidual)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = v[j] * r * w[j];
+        }
+        if constexpr (kAlone) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) xr[0][j] = in ? v[j] : 0.0f;
+            return;
         }
         if (owner) {
 #pragma unroll

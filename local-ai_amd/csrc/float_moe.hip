@@ -150,22 +150,22 @@ __global__ __launch_bounds__(256) void vector_up_kernel(const float* __restrict_
     }
 }
 
-// The same with the normed vector in registers (width a multiple of 8, up to 512 * NL), brought in by eight waves together: a
+// The same with the normed vector in registers (width a multiple of 8, up to 512 * NL), brought in by the waves together: a
 // workgroup keeps to one expert's rows (blockIdx.y: the choice), and the weights of two rows are requested as soon as the selection is known.
-template <int NL>
-__global__ __launch_bounds__(512) void vector_up_reg_kernel(const VectorStage st, const float* __restrict__ logits, const uint16_t* __restrict__ up,
+template <int NL, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void vector_up_reg_kernel(const VectorStage st, const float* __restrict__ logits, const uint16_t* __restrict__ up,
                                                            float* __restrict__ hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act) {
-    __shared__ uint32_t ids[kVectorWaves][kMaxTop];
-    __shared__ float weights[kVectorWaves][kMaxTop];
-    __shared__ LhVectorSpace space;
+    __shared__ uint32_t ids[WAVES][kMaxTop];
+    __shared__ float weights[WAVES][kMaxTop];
+    __shared__ LhVectorSpace<WAVES> space;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = blockIdx.y, last = (width >> 3) - 1;
-    LhSharedVector<kNorm, NL> x;
+    LhSharedVector<kNorm, NL, WAVES> x;
     x.fetch(st, width, lane, wave);
     select_experts(logits, experts, c + 1, lane, ids[wave], weights[wave]);    // every wave for itself: no barrier
     const uint32_t e = __builtin_amdgcn_readfirstlane(ids[wave][c]);
     const float weight = weights[wave][c];
     const uint16_t* base = up + (size_t)e * ff * width;
-    const uint32_t first = blockIdx.x * kVectorWaves + wave, step = gridDim.x * kVectorWaves, rows = first < ff ? (ff - first - 1) / step + 1 : 0u;
+    const uint32_t first = blockIdx.x * WAVES + wave, step = gridDim.x * WAVES, rows = first < ff ? (ff - first - 1) / step + 1 : 0u;
     struct Row { uint4 w[NL]; } v[2];
     auto issue = [&](Row& x, uint32_t i) {
 #pragma unroll
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(512) void vector_down_reg_kernel(const float* __res
                                                              float* __restrict__ residual, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff) {
     __shared__ uint32_t ids[kVectorWaves][kMaxTop];
     __shared__ float weights[kVectorWaves][kMaxTop];
-    __shared__ LhVectorSpace space;
+    __shared__ LhVectorSpace<> space;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), chunks = top * (ff >> 3);
     VectorStage st{};
     st.x = hidden; st.x_f32 = 1;
@@ -372,13 +372,19 @@ int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const lh_buff
     VectorStage st{};
     st.x = input->ptr; st.x_f32 = 1; st.norm_weight = (const float*)norm_weight->ptr; st.eps = eps;
     if (width % 8 == 0 && width <= 4096 && ((uintptr_t)up->ptr & 15) == 0 && lh_stage_aligned(st)) {
-        const dim3 grid(std::min<uint32_t>((ff + kVectorWaves - 1) / kVectorWaves, std::max<uint32_t>(1, (uint32_t)batch->ctx->cu_count / top)), top);
-#define LH_UP(NL) hipLaunchKernelGGL((vector_up_reg_kernel<NL>), grid, dim3(64 * kVectorWaves), 0, batch->ctx->stream, st, (const float*)logits->ptr, (const uint16_t*)up->ptr, \
-                                     (float*)hidden->ptr, experts, top, width, ff, act)
-        if (width <= 512) LH_UP(1);
-        else if (width <= 1024) LH_UP(2);
-        else if (width <= 2048) LH_UP(4);
-        else LH_UP(8);
+        // (four waves where all rows are at most eight per CU, as the one-row products)
+        const uint32_t cus = (uint32_t)batch->ctx->cu_count, w = width <= 2048 && (uint64_t)ff * top <= 8ull * cus ? 4 : kVectorWaves;
+        const dim3 grid(std::min<uint32_t>((ff + w - 1) / w, std::max<uint32_t>(1, (w == 4 ? 2 : 1) * cus / top)), top);
+#define LH_UP(NL, WAVES) hipLaunchKernelGGL((vector_up_reg_kernel<NL, WAVES>), grid, dim3(64 * WAVES), 0, batch->ctx->stream, st, (const float*)logits->ptr, \
+                                            (const uint16_t*)up->ptr, (float*)hidden->ptr, experts, top, width, ff, act)
+        if (w == 4) {
+            if (width <= 512) LH_UP(1, 4);
+            else if (width <= 1024) LH_UP(2, 4);
+            else LH_UP(4, 4);
+        } else if (width <= 512) LH_UP(1, 8);
+        else if (width <= 1024) LH_UP(2, 8);
+        else if (width <= 2048) LH_UP(4, 8);
+        else LH_UP(8, 8);
 #undef LH_UP
         LH_TRY(lh_check_launch(op));
         batch->dispatch_count++;

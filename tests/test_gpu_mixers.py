@@ -358,6 +358,13 @@ def test_one_row_walks(ai, gpu, k, n, pairs):
         close(download(ai, res, n, ai.F32), want + 1, F32_TOL, "added")
 
 
+@pytest.mark.parametrize("k,n", [(8, 1), (512, 2048), (520, 2046), (2048, 2048), (2048, 33), (2056, 1), (2064, 2047), (3000, 300), (4088, 1030), (4096, 2048)])
+@pytest.mark.parametrize("pairs", [False, True])
+def test_one_row_against_few_rows(ai, gpu, k, n, pairs):
+    """The same up to eight weight rows per CU: workgroups of four waves, and a row over eight waves beyond 2048 columns."""
+    test_one_row_walks(ai, gpu, k, n, pairs)
+
+
 @pytest.mark.parametrize("rows,dim", [(1, 64), (5, 100), (3, 1024), (2, 4096), (4, 5000), (70, 33)])
 def test_row_norms_and_gather(ai, gpu, rows, dim):
     ctx, K = gpu
