@@ -1761,10 +1761,13 @@ int lh_matmul_nt_quant_gelu_mul_into(lh_batch* b, lh_quant fmt, const lh_buffer*
     // one launch where the grouped product of the pair takes the skinny kernel without a k split (split products need
     // their sums before the gelu); the same quarters of k in either kernel, hence the same sums
     const uint32_t mgroups = (m + 63) / 64;
+    // (beyond 64 rows and from half as many 128-row tiles as CUs on the group is issued as two products, which may split k where the pair does not:
+    // 129 to 192 rows, n from 4096 to 5376)
+    const bool apart = m > 64 && (uint64_t)(n / BN) * 2 * ((m + 127) / 128) * 2 >= (uint64_t)ctx->cu_count;
     if (m >= skinny_min_m(fmt == LH_Q4_0 ? kQ4 : kTQ2) && (fmt != LH_Q4_0 || m > (uint32_t)kMaxMultivecM) && m <= skinny_max_m() &&
         n % BN == 0 && k % (4 * unit_k) == 0 &&
         blocks <= skinny_max_blocks(ctx) && (m <= 64 || blocks * mgroups <= 8 * (uint32_t)ctx->cu_count) &&
-        skinny_splits(ctx, m, blocks * mgroups, k / unit_k / 4) == 1) {
+        skinny_splits(ctx, m, blocks * mgroups, k / unit_k / 4) == 1 && (!apart || skinny_splits(ctx, m, n / 64 * mgroups, k / unit_k / 4) == 1)) {
         GroupArgs grp{};
         grp.count = 2;
         grp.W[0] = (const uint8_t*)w_gate->ptr; grp.W[1] = (const uint8_t*)w_up->ptr;

@@ -422,7 +422,7 @@ def test_rows_against_many_weight_rows(pkg, gpu, oracle, fmt, m, k, ns):
 
 @pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
 @pytest.mark.parametrize("m,k,n", [(64, 512, 32768), (130, 512, 11008), (256, 1536, 8320), (17, 1536, 32768), (33, 512, 40064), (256, 1536, 12288), (64, 512, 66048),
-                                   (200, 3584, 16384), (256, 2560, 6144)])
+                                   (200, 3584, 16384), (256, 2560, 6144), (160, 2048, 4096), (129, 2048, 5376), (192, 2048, 5504)])
 def test_gate_and_up_against_many_weight_rows(pkg, gpu, fmt, m, k, n):
     """The pair in that form against the grouped product, the products one by one and gelu_mul, bit for bit, on both sides of where each of
     them takes the form."""
