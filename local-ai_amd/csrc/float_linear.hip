@@ -456,19 +456,17 @@ __global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
     extern __shared__ uint4 sm[];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = wave >> 2;
     const uint32_t wm = kWide ? group : kHalves ? (wave >> 1) & 1 : wave >> 1, wn = kWide ? wave & 3 : wave & 1;
-    const uint32_t mt_n = a.ex.tiles ? a.ex.n_tiles : (a.M + BM - 1) / BM, nt_n = (a.N + BN - 1) / BN;
     uint32_t mt, nt;
-    tile_of_block(mt_n, nt_n, mt, nt);
-    const RowTile rt = row_tile(a, mt, BM);
-    if (rt.begin >= rt.end) return;
+    tile_of_block((a.M + BM - 1) / BM, (a.N + BN - 1) / BN, mt, nt);
+    const RowTile rt{mt * BM, min(mt * BM + BM, a.M), 0u};
     const uint32_t n0 = nt * BN, K = a.K, steps = K / 64, nk = steps * a.parts;
     const char* A = static_cast<const char*>(a.A);
-    const char* W = reinterpret_cast<const char*>(a.W + (size_t)rt.expert * a.N * K);
+    const char* W = reinterpret_cast<const char*>(a.W);
 
     const uint32_t lt = kHalves ? tid & 255 : tid, src = ((lt & 7) ^ ((lt >> 3) & 7)) * 16, src_b = ((lt & 7) ^ dealt_swizzle<4>(lt >> 3)) * 16;
     uint32_t pa[CA], pb[CB];                                   // byte offsets: the host has checked that they fit
 #pragma unroll
-    for (int i = 0; i < CA; i++) pa[i] = a_row(a, min(rt.begin + i * (T / 8) + (lt >> 3), rt.end - 1)) * a.lda * 2 + src;
+    for (int i = 0; i < CA; i++) pa[i] = min(rt.begin + i * (T / 8) + (lt >> 3), rt.end - 1) * a.lda * 2 + src;
 #pragma unroll
     for (int i = 0; i < CB; i++) pb[i] = min(n0 + i * (T / 8) + (lt >> 3), a.N - 1) * K * 2 + src_b;
     uint4* const to = sm + (kHalves ? wave & 3 : wave) * 64;
