@@ -224,17 +224,18 @@ def test_products_of_one_vector(pkg, gpu, oracle, fmt, rows, cols, count, kind):
     outs, batch = [pkg.Buffer.empty(ctx, rows * 2) for _ in range(count)], pkg.CommandBatch(ctx)
     xb, ab = pkg.Buffer.from_slice(ctx, x), pkg.Buffer.from_slice(ctx, aux)
     print(f"one vector {fmt} {rows}x{cols} x{count} {kind}", flush=True)
-    if kind == "rotate":
-        if count > 1:
-            return                                                    # a rotation takes one matrix
+    if kind == "rotate":                                              # a rotation takes one matrix
         signs = np.where(g.random(256) < 0.5, -1.0, 1.0).astype(np.float32)
         x32 = g.standard_normal(cols, dtype=np.float32)
         staged = oracle.hadamard_rotate(x32, signs, 256, cols // 256, False, True).astype(np.float16)
-        K.matvec_quant_rotated_into(batch, ty, ws[0].buf, pkg.Buffer.from_slice(ctx, x32), pkg.Buffer.from_slice(ctx, signs), 256, outs[0], rows, cols)
+        for w, o in zip(ws, outs):
+            K.matvec_quant_rotated_into(batch, ty, w.buf, pkg.Buffer.from_slice(ctx, x32), pkg.Buffer.from_slice(ctx, signs), 256, o, rows, cols)
     elif kind == "none":
         staged = x
-        for w, o in zip(ws, outs):
-            w.matvec_into(batch, K, xb, o)
+        if count == 1:
+            ws[0].matvec_into(batch, K, xb, outs[0])
+        else:
+            K.matvec_quant_grouped_into(batch, ty, [w.buf for w in ws], [xb] * count, pkg.F16, outs, pkg.F16, rows, cols)
     else:
         staged = G.rms_norm(x, aux, cols, 1, 1e-6) if kind == "norm" else G.gelu_mul(x, aux)
         K.matvec_quant_fused_into(batch, ty, [w.buf for w in ws], xb, K.PROLOGUE_RMS_NORM if kind == "norm" else K.PROLOGUE_GELU_MUL, ab, 1e-6, outs, rows, cols)
