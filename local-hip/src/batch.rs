@@ -48,13 +48,14 @@ impl CommandBatch {
         Ok(())
     }
 
-    /// `commit_and_wait()` (batch.rs:240-250).  The reference consumes the batch; this one stays usable, which is what
-    /// `commit_and_renew` gives there.
     /// Host bytes for `dst` in the order of the batch's dispatches; no wait up to 2 KB.
     pub fn write(&mut self, dst: &Buffer, offset: usize, src: &[u8]) -> Result<()> {
+        // SAFETY: live handles, `src` outlives the call; the library checks the range.
         check(unsafe { ffi::lh_batch_write(self.raw, dst.as_ptr(), offset, src.as_ptr() as *const c_void, src.len()) })
     }
 
+    /// `commit_and_wait()` (batch.rs:240-250).  The reference consumes the batch; this one stays usable, which is what
+    /// `commit_and_renew` gives there.
     pub fn commit_and_wait(&mut self) -> Result<()> {
         // SAFETY: live handle.
         check(unsafe { ffi::lh_batch_commit_and_wait(self.raw) })
