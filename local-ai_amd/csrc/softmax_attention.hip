@@ -366,7 +366,8 @@ int launch_dv(lh_context* ctx, AttentionArgs& a, uint32_t mp, const char* op, ui
 // A matrix instruction takes one value of k per lane, and which one is free as long as both operands agree: over the dimensions of a
 // head lane group g has its g-th quarter of 16, over the keys of a tile its keys 4 g .. 4 g + 3, which is where S^T leaves the weights
 // and what a value block keeps side by side.  (attention_plain_kernel reads keys a value at a time, every thread its own row: 333 rows
-// of 8 heads with two maps over 64 dimensions, values of 128: 380 us; this form 27 us.)
+// of 8 heads with two maps over 64 dimensions, values of 128: 380 us; this form 27 us.  One row as well, though its workgroups are one per
+// kv head: 8 heads of 128 over 1 or 8, 64, 4096 and 16384 keys 9, 165 to 178 and 735 us, in the plain form 21, 665 and 2690.)
 constexpr uint32_t kWideMaxDim = 256;      // of a key, per map
 template <int DV, int MAPS>
 __global__ __launch_bounds__(256) void attention_wide_kernel(const AttentionArgs a) {
