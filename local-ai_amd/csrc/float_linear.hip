@@ -1136,7 +1136,7 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
         // One workgroup fits a CU, so a launch takes whole rounds of them, and the form is the one whose rounds are the shortest.  A
         // round's time in nanoseconds, measured with 64 columns of k per step: 256 x 256 9000 + 1650 per step, 256 x 128 8000 + 800,
         // 128 x 128 7000 + 520.  Before / now, bf16 results: 2048 x 2048 x 8192 85 / 60 us (256 x 256; the matrix cores alone would take
-        // 28 at 2.4 GHz, but with all CUs at it the clock falls to 1.3 GHz), 2048 x 2048 x 4096 39 / 34 and 2048 x 2048 x 3072 35 / 28
+        // 28 at 2.4 GHz; on random data the clock is 1.5 to 1.8 GHz and they are busy for 70 % of the cycles of such launches), 2048 x 2048 x 4096 39 / 34 and 2048 x 2048 x 3072 35 / 28
         // (256 x 128), 2048 x 8192 x 2048 90 / 74 (128 x 128).  With fewer than three tiles of 128 x 128 to four CUs the small tiles
         // win: 128 of them (953 x 2048 x 2048) 22 us against 17.
         auto rounds = [&](uint32_t bm, uint32_t bn) { return (tiles(bm, bn) + want - 1) / want; };

@@ -954,13 +954,6 @@ __global__ __launch_bounds__(256, 2) void matmul_skinny_kernel(const uint16_t* _
     }
 }
 
-// ---- the same rows against many weight rows: activations shared by a workgroup ----------------------------------------------------
-// With enough 64-row blocks for every CU no product needs its k range split over waves: here the four waves of a workgroup take 64
-// weight rows each (PAIR: 32 of gate and the same 32 of up) over all of k and share the activations, which come in 128 columns at a
-// time into one of two LDS buffers in the fragment order of matmul_skinny_kernel.  A workgroup per 64 rows reads all
-// activations from L2 for itself and adds four partial tiles through LDS: 64 x 1536 x 262144 (Q4_0, f32 out) 176 us, here 95; 256 rows,
-// gate and up of 12288 x 1536 (TQ2_0) 39 and 34.
-// The codes are two steps ahead in registers, the activations one in registers and one in LDS; one barrier per step.
 // An address in global memory that is the same in all lanes, kept in scalar registers: a load at it plus 32 bits of offset of the lane's own
 // needs no vector registers for addresses.  (The builtin gives a signed word: it must not be widened as one.)
 typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;
@@ -972,6 +965,13 @@ __device__ __forceinline__ uint64_t uniform_address(const void* p) {
 __device__ __forceinline__ GlobalBytes load_base(uint64_t address) { asm volatile("" : "+s"(address)); return (GlobalBytes)address; }
 __device__ __forceinline__ uint32_t lane_offset(uint32_t offset) { asm volatile("" : "+v"(offset)); return offset; }
 
+// ---- the same rows against many weight rows: activations shared by a workgroup ----------------------------------------------------
+// With enough 64-row blocks for every CU no product needs its k range split over waves: here the four waves of a workgroup take 64
+// weight rows each (PAIR: 32 of gate and the same 32 of up) over all of k and share the activations, which come in 128 columns at a
+// time into one of two LDS buffers in the fragment order of matmul_skinny_kernel.  A workgroup per 64 rows reads all
+// activations from L2 for itself and adds four partial tiles through LDS: 64 x 1536 x 262144 (Q4_0, f32 out) 176 us, here 94; 256 rows,
+// gate and up of 12288 x 1536 (TQ2_0) 39 and 30.
+// The codes are two steps ahead in registers, the activations one in registers and one in LDS; one barrier per step.
 template <int FMT, int CDT, bool PAIR>
 __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W_one, void* __restrict__ C_one, uint32_t M,
                                                             uint32_t K, uint32_t N_one, uint32_t blocks, GroupArgs grp) {
@@ -994,7 +994,7 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
 
     // Codes: the 64 rows' bytes of a step (Q4_0: 72 a row; TQ2_0: 32 of codes, and the scale of the block by itself) come in with coalesced
     // loads, consecutive lanes along a row, and are parked in the wave's own LDS area, from which every lane takes what it multiplies.
-    // (A lane loading its eight bytes itself costs a cache access per lane, one per clock and CU: 135 us where this takes 95.)
+    // (A lane loading its eight bytes itself costs a cache access per lane, one per clock and CU: 135 us where this took 95.)
     // A load of the wave takes whole rows (Q4_0: seven of nine pieces of 8 bytes, the last lane repeating one; TQ2_0: sixteen of four), so that
     // loads are a constant apart; the last Q4_0 load repeats row 63.
     constexpr uint32_t PIECES = FMT == kQ4 ? 9 : 4, RPL = 64 / PIECES, NL = (64 + RPL - 1) / RPL, PITCH = FMT == kQ4 ? 76 : 36;   // PITCH: bytes per row in LDS, an odd number of words
