@@ -258,8 +258,9 @@ LH_API int lh_matmul_nt_quant_typed_into(lh_batch* batch, lh_quant fmt, const lh
 /* The feed-forward gate and up projections and their gelu_mul as one encoded step:
  * out[m, n] = half(gelu(half(in . w_gate^T)) * half(in . w_up^T)) -- matmul_nt_into twice and gelu_mul_into of the
  * multi-row layer paths (local-engine/src/layer.rs:652-662), with their roundings: bit for bit the result of
- * lh_matmul_nt_quant_grouped_into on the pair and gelu_mul_into.  For a decode batch or prefill chunk (17 .. 256 rows) whose pair needs no k split this is a single kernel that
- * pairs gate and up rows in one workgroup; other shapes run the grouped product into the workspace and gelu_mul. */
+ * lh_matmul_nt_quant_grouped_into on the pair and gelu_mul_into.  For a decode batch or prefill chunk (17 .. 256 rows)
+ * whose pair needs no k split this is a single kernel that pairs gate and up rows in one workgroup; other shapes run the
+ * grouped product into the workspace and gelu_mul. */
 LH_API int lh_matmul_nt_quant_gelu_mul_into(lh_batch* batch, lh_quant fmt, const lh_buffer* input, const lh_buffer* w_gate,
                                             const lh_buffer* w_up, lh_buffer* output, uint32_t m, uint32_t k, uint32_t n);
 /* The per-layer-input gate of the multi-row layer paths as one encoded step (local-engine/src/layer.rs:686-700:
