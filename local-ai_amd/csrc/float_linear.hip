@@ -1,11 +1,12 @@
 // Products of activations with bf16 weights [N, K]:
 //   linear_phased_kernel bf16 activations, K a multiple of 64, enough tiles of 128 x 128 for the chip: eight waves in two phases
 //   linear_mfma_kernel   bf16 activations, K a multiple of 8: LDS-tiled bf16 MFMA 16x16x32, tiles loaded straight into LDS
-//   split_rows_kernel    f32 activations as three bf16 terms, for the two kernels above (the 32-bit runs)
+//   linear_sliced_kernel the same where the tiles are few for the chip: small tiles, k shared out among a workgroup's waves
+//   split_rows_kernel    f32 activations as three bf16 terms, for the three kernels above (the 32-bit runs)
 //   linear_plain_kernel  everything else: f32 FMA on 64 x 64 tiles (ragged K, pieces that are not aligned)
 //   matvec_bf16_kernel   one row, HBM-bound weight streaming, with the norm before the product done while x is staged
-// All end in the same column segments (bias, activation, layout, residual add), and linear_mfma_kernel and linear_plain_kernel also
-// run the experts of a mixture on the tiles of a routing plan.
+// All end in the same column segments (bias, activation, layout, residual add), and linear_mfma_kernel,
+// linear_sliced_kernel and linear_plain_kernel also run the experts of a mixture on the tiles of a routing plan.
 #include "float_linear.hpp"
 #include <algorithm>
 #include <cstring>
@@ -23,13 +24,20 @@ __device__ __forceinline__ void load_lds16(const void* g, void* lds) {
 
 __device__ uint4 g_zero16 = {0u, 0u, 0u, 0u};   // what activation chunks past K read
 
-// The rows this workgroup multiplies: tile `mt` of an ordinary product or of an expert plan.
+// The rows this workgroup multiplies: tile `mt` of an ordinary product, or part `mt` of the tiles of an expert plan, whose rows are
+// a multiple of bm.
 struct RowTile { uint32_t begin, end, expert; };
+__device__ __forceinline__ uint32_t row_tiles(const LhLinear& a, uint32_t bm) {
+    return a.ex.tiles ? a.ex.n_tiles * (a.ex.tile_rows / bm) : (a.M + bm - 1) / bm;
+}
 __device__ __forceinline__ RowTile row_tile(const LhLinear& a, uint32_t mt, uint32_t bm) {
     if (a.ex.tiles == nullptr) return RowTile{mt * bm, min(mt * bm + bm, a.M), 0u};
-    const uint32_t* t = a.ex.tiles + 3 * mt;
+    const uint32_t per = a.ex.tile_rows / bm;
+    const uint32_t* t = a.ex.tiles + 3 * (mt / per);
     RowTile r{t[1], min(t[2], a.ex.slots), t[0]};
-    if (r.expert >= a.ex.experts || r.begin >= r.end) r.begin = r.end = r.expert = 0;
+    if (r.expert >= a.ex.experts || r.begin >= r.end) return RowTile{0u, 0u, 0u};
+    r.begin += mt % per * bm;
+    r.end = min(r.end, r.begin + bm);
     return r;
 }
 __device__ __forceinline__ uint32_t a_row(const LhLinear& a, uint32_t slot) {
@@ -345,9 +353,8 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
     static_assert(NS * (BM + BN) * 128 >= BM * BN * 4, "the output tile must fit the staging buffers");
     __shared__ uint4 sm[NS][(BM + BN) * 8];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-    const uint32_t mt_n = a.ex.tiles ? a.ex.n_tiles : (a.M + BM - 1) / BM, nt_n = (a.N + BN - 1) / BN;
     uint32_t mt, nt;
-    tile_of_block(mt_n, nt_n, mt, nt);
+    tile_of_block(row_tiles(a, BM), (a.N + BN - 1) / BN, mt, nt);
     const RowTile rt = row_tile(a, mt, BM);
     if (rt.begin >= rt.end) return;
     const uint32_t n0 = nt * BN, K = a.K, steps = (K + 63) / 64, nk = steps * a.parts;
@@ -424,6 +431,109 @@ __global__ __launch_bounds__(256) void linear_mfma_kernel(const LhLinear a) {
 
     __syncthreads();
     finish_tile<EPI, TI, TJ>(a, acc, rt, wm * (BM / 2), n0 + wn * (BN / 2), lane, reinterpret_cast<float4*>(&sm[0][0]) + wave * (BM * BN / 16));
+}
+
+// Few tiles for the chip: what bounds a product then is how much of it is on its way to a CU (16 KB a step and three steps ahead in the
+// kernel above: a step takes as long as a third of a trip to memory).  Here every wave multiplies the whole tile over a slice of k,
+// the steps wave, wave + W, ..., out of buffers of its own in LDS, all NS of them requested ahead, with no barrier until the W sums meet
+// at the end, in one order.  A buffer is requested again as soon as its fragments are in registers.
+template <int BM, int BN, int W, int NS, int EPI>
+__global__ __launch_bounds__(64 * W) void linear_sliced_kernel(const LhLinear a) {
+    constexpr int TI = BM / 16, TJ = BN / 16, CA = BM / 8, CB = BN / 8, STEP = (BM + BN) * 8, PER = CA + CB;
+    static_assert((NS - 1) * PER < 64, "requests are counted in six bits");
+    static_assert(NS * STEP * 16 >= BM * BN * 4 + 2048, "a wave's sums and its part of the output tile must fit its buffers");
+    extern __shared__ uint4 sm[];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t mt, nt;
+    tile_of_block(row_tiles(a, BM), (a.N + BN - 1) / BN, mt, nt);
+    const RowTile rt = row_tile(a, mt, BM);
+    if (rt.begin >= rt.end) return;
+    const uint32_t n0 = nt * BN, K = a.K, steps = (K + 63) / 64, nk = steps * a.parts;
+    const uint16_t* A = static_cast<const uint16_t*>(a.A);
+    const uint16_t* Wt = a.W + (size_t)rt.expert * a.N * K;
+
+    const uint16_t *pa[CA], *pb[CB];
+    const uint32_t src = (lane & 7) ^ (lane >> 3);
+#pragma unroll
+    for (int i = 0; i < CA; i++) pa[i] = A + (size_t)a_row(a, min(rt.begin + i * 8 + (lane >> 3), rt.end - 1)) * a.lda + src * 8;
+#pragma unroll
+    for (int i = 0; i < CB; i++) pb[i] = Wt + (size_t)min(n0 + i * 8 + (lane >> 3), a.N - 1) * K + src * 8;
+
+    uint4* const ring = sm + wave * NS * STEP;
+    auto load_step = [&](uint32_t buf, uint32_t step) {
+        uint4* base = ring + buf * STEP;
+        const uint32_t part = (step >= steps) + (step >= 2 * steps), kt = step - part * steps;
+        const size_t ka = (size_t)part * a.part_stride + kt * 64;
+        if (kt * 64 + 64 <= K) {
+#pragma unroll
+            for (int i = 0; i < CA; i++) load_lds16(pa[i] + ka, base + i * 64);
+#pragma unroll
+            for (int i = 0; i < CB; i++) load_lds16(pb[i] + kt * 64, base + (CA + i) * 64);
+        } else {                                             // the last step of a ragged K: chunks past it read zeros
+            const bool past = kt * 64 + src * 8 >= K;
+#pragma unroll
+            for (int i = 0; i < CA; i++) load_lds16(past ? (const void*)&g_zero16 : (const void*)(pa[i] + ka), base + i * 64);
+#pragma unroll
+            for (int i = 0; i < CB; i++) load_lds16(past ? (const void*)&g_zero16 : (const void*)(pb[i] + kt * 64), base + (CA + i) * 64);
+        }
+    };
+
+    lh_f32x4 acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++) acc[i][j] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
+
+    const uint32_t mine = nk > wave ? (nk - wave + W - 1) / W : 0;
+#pragma unroll
+    for (int i = 0; i < NS; i++) if (i < (int)mine) load_step(i, wave + i * W);
+    uint32_t buf = 0;
+    const uint32_t g = lane >> 4, at[2] = {g ^ (lane & 7), (g + 4) ^ (lane & 7)};
+    for (uint32_t i = 0; i < mine; i++) {
+        if (i + NS <= mine) wait_loads<(NS - 1) * PER>();     // step i has arrived; the later steps may still be coming
+        else wait_loads<0>();
+        const uint4 *as = ring + buf * STEP + (lane & 15) * 8, *bs = as + BM * 8;
+        lh_bf16x8 fa[2][TI], fb[2][TJ];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+#pragma unroll
+            for (int t = 0; t < TI; t++) fa[s][t] = __builtin_bit_cast(lh_bf16x8, as[t * 128 + at[s]]);
+#pragma unroll
+            for (int t = 0; t < TJ; t++) fb[s][t] = __builtin_bit_cast(lh_bf16x8, bs[t * 128 + at[s]]);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (i + NS < mine) load_step(buf, wave + (i + NS) * W);
+        buf = buf + 1 == NS ? 0 : buf + 1;
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int t = 0; t < TI; t++)
+#pragma unroll
+                for (int u = 0; u < TJ; u++) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[s][u], fa[s][t], acc[t][u], 0, 0, 0);
+    }
+
+    // Every wave's sums to LDS; a wave then finishes tiles of 32 x 16.
+    lh_f32x4* const sums = reinterpret_cast<lh_f32x4*>(sm);
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < TI; t++)
+#pragma unroll
+        for (int u = 0; u < TJ; u++) sums[(wave * TI * TJ + t * TJ + u) * 64 + lane] = acc[t][u];
+    __syncthreads();
+    float4* const box = reinterpret_cast<float4*>(sums + W * TI * TJ * 64) + wave * 128;
+#pragma unroll 1
+    for (uint32_t e = wave; e < TI / 2 * TJ; e += W) {
+        const uint32_t t = e / TJ * 2, u = e % TJ;
+        lh_f32x4 sum[2][1];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const lh_f32x4* from = sums + ((t + h) * TJ + u) * 64 + lane;
+            sum[h][0] = from[0];
+#pragma unroll
+            for (int w = 1; w < W; w++) sum[h][0] += from[w * TI * TJ * 64];
+        }
+        finish_tile<EPI, 2, 1>(a, sum, rt, t * 16, n0 + u * 16, lane, box);
+    }
 }
 
 // Large products, K a multiple of 64.  Eight waves in two groups of four, one wave of either group on each SIMD, half a period
@@ -1086,6 +1196,19 @@ static int launch_mfma(lh_context* ctx, const LhLinear& a, uint64_t grid, const 
     });
     return lh_check_launch(op);
 }
+template <int BM, int BN, int NS>
+static int launch_sliced(lh_context* ctx, const LhLinear& a, uint64_t grid, const char* op) {
+    LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: %u x %u outputs", op, a.M, a.N);
+    if (grid == 0) return LH_OK;
+    constexpr size_t lds = (size_t)4 * NS * (BM + BN) * 128;
+    int r = LH_OK;
+    with_epilogue(epilogue_of(a.seg, 4), [&](auto epi) {
+        const auto kernel = linear_sliced_kernel<BM, BN, 4, NS, decltype(epi)::value>;
+        r = lh_raise_dynamic_lds(ctx, (const void*)kernel, lds, op);
+        if (r == LH_OK) hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(256), lds, ctx->stream, a);
+    });
+    return r == LH_OK ? lh_check_launch(op) : r;
+}
 template <int BM, int BN>
 static int launch_phased(lh_context* ctx, const LhLinear& a, uint64_t grid, const char* op) {
     LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: %u x %u outputs", op, a.M, a.N);
@@ -1123,32 +1246,43 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
         return lh_check_launch(op);
     }
     const uint64_t want = (uint64_t)ctx->cu_count, steps = (uint64_t)a.K / 64 * a.parts;
-    auto tiles = [&](uint32_t bm, uint32_t bn) { return (uint64_t)(a.ex.tiles ? a.ex.n_tiles : (a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
+    auto tiles = [&](uint32_t bm, uint32_t bn) {
+        return (a.ex.tiles ? (uint64_t)a.ex.n_tiles * (a.ex.tile_rows / bm) : ((uint64_t)a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
+    };
     // Byte offsets of the phased kernels are 32 bits wide.
     const uint64_t a_bytes = (uint64_t)a_rows * a.lda * 2, w_bytes = (uint64_t)a.N * a.K * 2;
     const bool phased = a.K % 64 == 0 && a_bytes < (1ull << 32) && w_bytes < (1ull << 32);
-    if (a.ex.tiles) {
-        if (a.ex.tile_rows != 128) return launch_mfma<64, 64, 4>(ctx, a, tiles(64, 64), op);
-        if (tiles(128, 128) >= want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
-        return launch_mfma<128, 64, 3>(ctx, a, tiles(128, 64), op);
-    }
-    if (phased && 4 * tiles(128, 128) >= 3 * want) {
+    if (a.ex.tiles && a.ex.tile_rows == 128 && tiles(128, 128) >= want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
+    if (phased && !a.ex.tiles && 4 * tiles(128, 128) >= 3 * want) {
         // One workgroup fits a CU, so a launch takes whole rounds of them, and the form is the one whose rounds are the shortest.  A
         // round's time in nanoseconds, measured with 64 columns of k per step: 256 x 256 9000 + 1650 per step, 256 x 128 8000 + 800,
         // 128 x 128 7000 + 520.  Before / now, bf16 results: 2048 x 2048 x 8192 85 / 60 us (256 x 256; the matrix cores alone would take
         // 28 at 2.4 GHz; on random data the clock is 1.5 to 1.8 GHz and they are busy for 70 % of the cycles of such launches), 2048 x 2048 x 4096 39 / 34 and 2048 x 2048 x 3072 35 / 28
         // (256 x 128), 2048 x 8192 x 2048 90 / 74 (128 x 128).  With fewer than three tiles of 128 x 128 to four CUs the small tiles
-        // win: 128 of them (953 x 2048 x 2048) 22 us against 17.
+        // win: 128 of them (953 x 2048 x 2048) 22 us against 18.
         auto rounds = [&](uint32_t bm, uint32_t bn) { return (tiles(bm, bn) + want - 1) / want; };
         const uint64_t t256 = rounds(256, 256) * (9000 + 1650 * steps), t384 = rounds(256, 128) * (8000 + 800 * steps), t128 = rounds(128, 128) * (7000 + 520 * steps);
         if (t256 <= t384 && t256 <= t128) return launch_phased<256, 256>(ctx, a, tiles(256, 256), op);
         if (t384 <= t128) return launch_phased<256, 128>(ctx, a, tiles(256, 128), op);
         return launch_phased<128, 128>(ctx, a, tiles(128, 128), op);
     }
-    if (tiles(128, 128) >= 2 * want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
-    if (tiles(128, 64) >= want) return launch_mfma<128, 64, 3>(ctx, a, tiles(128, 64), op);
-    if (tiles(64, 64) >= want || a.M > 32) return launch_mfma<64, 64, 4>(ctx, a, tiles(64, 64), op);
-    return launch_mfma<32, 32, 4>(ctx, a, tiles(32, 32), op);
+    if (!a.ex.tiles && tiles(128, 128) >= 2 * want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
+    // The rest by its expected time in nanoseconds, measured: 64 x 64 tiles of shared waves, up to three workgroups a CU; or waves that
+    // share out k, on 64 x 32 tiles (one workgroup a CU) or 32 x 32 (two).  Of an expert plan about half the experts' last tiles count:
+    // the plan has one more for each than can be full.  Before / now, weights in the memory-side cache: 512 x 1024 x 4096 25.5 / 12.5 us
+    // and 200 x 2048 x 8192 46.7 / 19.2 (64 x 32), 512 x 1024 x 1024 9.6 / 6.5, 2048 x 16 x 2048 14.0 / 6.0 and 256 x 1024 x 4096 25.2 / 9.4
+    // (32 x 32), 953 x 2048 x 2048 21 / 17.9 and 300 x 6144 x 1536 19.5 / 15.3 (64 x 64, from 128 x 64), 333 x 1024 x 1024 with f32
+    // activations 20.3 / 9.6.
+    auto filled = [&](uint32_t bm, uint32_t bn) {
+        return a.ex.tiles ? ((uint64_t)a.ex.slots / bm + a.ex.experts / 2 + 1) * ((a.N + bn - 1) / bn) : tiles(bm, bn);
+    };
+    const uint64_t n64 = filled(64, 64), n32 = filled(32, 32);
+    const uint64_t t64 = n64 <= want ? 4000 + 345 * steps : n64 <= 2 * want ? 4600 + 430 * steps : (n64 + 3 * want - 1) / (3 * want) * (5000 + 600 * steps);
+    const uint64_t t64_32 = 1000 + (filled(64, 32) + want - 1) / want * (3500 + 100 * steps);
+    const uint64_t t32 = n32 <= want ? 4000 + 75 * steps : 1000 + (n32 + 2 * want - 1) / (2 * want) * (3500 + 150 * steps);
+    if (t64 <= t64_32 && t64 <= t32) return launch_mfma<64, 64, 3>(ctx, a, tiles(64, 64), op);
+    if (t64_32 <= t32) return launch_sliced<64, 32, 3>(ctx, a, tiles(64, 32), op);
+    return launch_sliced<32, 32, 2>(ctx, a, tiles(32, 32), op);
 }
 
 extern "C" {

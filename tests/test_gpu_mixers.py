@@ -106,6 +106,13 @@ def test_large_products(ai, gpu, m, k, n, act):
     close(download(ai, res, m * n, ai.F32).reshape(m, n), want + 1, F32_TOL, "residual")
 
 
+@pytest.mark.parametrize("m,k,n", [(33, 8, 36), (64, 576, 512), (100, 4096, 260), (129, 200, 1000), (511, 1288, 1028), (512, 2048, 1024), (480, 712, 1536)])
+@pytest.mark.parametrize("act", [0, 1, 2, 3])
+def test_products_of_few_tiles(ai, gpu, m, k, n, act):
+    """Waves that share out k: 32 x 32 tiles (the first four) and 64 x 32, fewer steps of k than waves, buffers used again, ragged steps."""
+    test_large_products(ai, gpu, m, k, n, act)
+
+
 @pytest.mark.parametrize("act", ["silu", "gelu", "pairs"])
 @pytest.mark.parametrize("m", [1024, 64])
 def test_activations_of_bf16_results(ai, gpu, act, m):
