@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <stddef.h>
 #include <atomic>
+#include <mutex>
 #include <vector>
 #include "../../include/local_hip.h"
 
@@ -40,6 +41,11 @@ struct lh_context {
     // here, and the next wait on the stream (lh_batch_commit_and_wait, lh_context_synchronize) reports it.
     uint32_t* fault_host;
     uint32_t* fault_dev;   // the same word as the device addresses it
+    // Pinned memory through which lh_buffer_read brings what fits it to the host; one read at a time.
+    static constexpr size_t kReadBytes = (size_t)256 << 10;
+    void* read_host;
+    void* read_dev;        // the same memory as the device addresses it
+    std::mutex read_mutex;
 };
 // Kernel-reported fault codes (lh_context::fault_host).
 enum : uint32_t { LH_FAULT_TQ2_SPLIT_WAIT = 1, LH_FAULT_ATTN_PAIR_WAIT = 2 };

@@ -23,6 +23,13 @@ __global__ __launch_bounds__(256) void blit_copy1_kernel(const uint8_t* __restri
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
 }
 
+// What lh_buffer_read brings to the host: `len` bytes from a 16-byte aligned place.
+__global__ __launch_bounds__(256) void read_out_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, size_t len) {
+    const size_t n16 = len / 16, stride = (size_t)gridDim.x * 256;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += stride) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    if (blockIdx.x == 0 && threadIdx.x < len % 16) dst[n16 * 16 + threadIdx.x] = src[n16 * 16 + threadIdx.x];
+}
+
 static const char* status_prefix(int code) {
     switch (code) {  // Display strings of local_metal::Error (error.rs:1-32)
         case LH_ERR_NO_DEVICE: return "No Metal device found";
@@ -137,6 +144,7 @@ static void ctx_release(lh_context* ctx) {
     for (int i = 0; i < lh_context::kDescSlots; i++) (void)hipEventDestroy(ctx->desc_event[i]);
     (void)hipHostFree(ctx->desc_pinned);
     (void)hipHostFree(ctx->fault_host);
+    (void)hipHostFree(ctx->read_host);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -195,10 +203,22 @@ int lh_context_create(int device_index, lh_context** out) {
         return lh_fail(LH_ERR_BUFFER_ALLOCATION, "size=%zu: pinned fault word", (size_t)64);
     }
     *ctx->fault_host = 0;
+    ctx->read_host = ctx->read_dev = nullptr;
+    if (hipHostMalloc(&ctx->read_host, lh_context::kReadBytes, hipHostMallocDefault) != hipSuccess ||
+        hipHostGetDevicePointer(&ctx->read_dev, ctx->read_host, 0) != hipSuccess) {
+        if (ctx->read_host) (void)hipHostFree(ctx->read_host);
+        (void)hipHostFree(ctx->fault_host);
+        (void)hipHostFree(ctx->desc_pinned);
+        (void)hipFree(ctx->workspace);
+        (void)hipStreamDestroy(ctx->stream);
+        delete ctx;
+        return lh_fail(LH_ERR_BUFFER_ALLOCATION, "size=%zu: pinned memory for reads", lh_context::kReadBytes);
+    }
     for (int i = 0; i < lh_context::kDescSlots; i++) {
         ctx->desc_used[i] = false;
         if (hipEventCreateWithFlags(&ctx->desc_event[i], hipEventDisableTiming) != hipSuccess) {
             for (int j = 0; j < i; j++) (void)hipEventDestroy(ctx->desc_event[j]);
+            (void)hipHostFree(ctx->read_host);
             (void)hipHostFree(ctx->fault_host);
             (void)hipHostFree(ctx->desc_pinned);
             (void)hipFree(ctx->workspace);
@@ -363,12 +383,27 @@ int lh_buffer_write(lh_buffer* buf, size_t offset, const void* src, size_t len) 
     return LH_OK;
 }
 
+// Up to 256 KB a kernel writes the bytes into pinned memory and the host copies them from there: 128 KB behind a kernel 21 us until they
+// are there, through hipMemcpyAsync into memory that it has to pin first 30.  Of 1 MB the second copy takes longer than the pinning.
 int lh_buffer_read(const lh_buffer* buf, size_t offset, void* dst, size_t len) {
     if (!buf || (!dst && len)) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_read: null argument");
     if (buf->ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_read: not while a graph is being captured");
     if (offset > buf->len || len > buf->len - offset)
         return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_read: range %zu+%zu exceeds %zu", offset, len, buf->len);
     if (!len) return LH_OK;
+    lh_context* ctx = buf->ctx;
+    const uint8_t* from = (const uint8_t*)buf->ptr + offset;
+    if (len <= lh_context::kReadBytes && ((uintptr_t)from & 15) == 0) {
+        std::lock_guard<std::mutex> lock(ctx->read_mutex);
+        const size_t grid = (len + 4095) / 4096;
+        hipLaunchKernelGGL(read_out_kernel, dim3((uint32_t)(grid < 256 ? grid : 256)), dim3(256), 0, ctx->stream, from, (uint8_t*)ctx->read_dev, len);
+        const int r = lh_check_launch("buffer_read");
+        if (r != LH_OK) return r;
+        const hipError_t e = hipStreamSynchronize(ctx->stream);
+        if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_read: %s", hipGetErrorString(e));
+        memcpy(dst, ctx->read_host, len);
+        return LH_OK;
+    }
     hipError_t e = hipMemcpyAsync(dst, (const char*)buf->ptr + offset, len, hipMemcpyDeviceToHost, buf->ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(buf->ctx->stream);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_read: %s", hipGetErrorString(e));
