@@ -6,7 +6,8 @@
 // Recurrent form: one workgroup per head and 16 value columns; a row of 16 lanes holds one value column's state in
 // registers (DQ / 16 values each) and walks the rows.  From eight rows on the inputs come in several rows ahead.
 //
-// Chunked form (64 rows a chunk, bf16 inputs on the matrix cores, everything else f32):
+// Chunked form (128 rows a chunk, bf16 inputs on the matrix cores, everything else f32; with 64 the states, which every step
+// writes or reads, are twice as many):
 //   1. every chunk's own contribution to the state, U = sum over rows s of a^(L-1-s) k_s (x) v_s (all chunks at once)
 //   2. a scan over the chunks, M <- a^L M + U, that leaves each chunk's incoming state in place of its U
 //   3. all outputs: y_t = a^(t+1) q_t M_in + sum over s <= t of a^(t-s) (q_t . k_s) v_s
@@ -18,7 +19,7 @@
 
 namespace {
 
-constexpr uint32_t kChunk = 64;
+constexpr uint32_t kChunk = 128, kHalf = 64;   // the callers' powers, and the running sums of a selective state space, reach over half a chunk
 
 // What the step of a token is: fixed per head, or computed from the token (selective state space).
 __device__ __forceinline__ float softplus(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
@@ -158,11 +159,11 @@ __global__ __launch_bounds__(256) void recurrent_rows_kernel(const RecurrentArgs
     }
 }
 
-// The steps of a selective state space, one wave per head and chunk: step sizes, and the running sum of the logarithms of the
-// decays within the chunk.  Rows past the last have step 0 and decay 1.
+// The steps of a selective state space, one wave per head and 64 rows: step sizes, and the running sum of the logarithms of the
+// decays within those rows.  Rows past the last have step 0 and decay 1.
 __global__ __launch_bounds__(64) void chunk_steps_kernel(const float* __restrict__ dt_raw, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
-                                                        float* __restrict__ sums, float* __restrict__ sizes, uint32_t rows, uint32_t heads, uint32_t chunks) {
-    const uint32_t h = blockIdx.x % heads, c = blockIdx.x / heads, lane = threadIdx.x, t = c * kChunk + lane;
+                                                        float* __restrict__ sums, float* __restrict__ sizes, uint32_t rows, uint32_t heads, uint32_t halves) {
+    const uint32_t h = blockIdx.x % heads, c = blockIdx.x / heads, lane = threadIdx.x, t = c * kHalf + lane;
     const float dt = t < rows ? softplus(dt_raw[(size_t)t * heads + h] + dt_bias[h]) : 0.0f;
     float sum = -expf(a_log[h]) * dt;
 #pragma unroll
@@ -170,7 +171,7 @@ __global__ __launch_bounds__(64) void chunk_steps_kernel(const float* __restrict
         const float o = __shfl_up(sum, d, 64);
         if (lane >= d) sum += o;
     }
-    const size_t i = ((size_t)h * chunks + c) * kChunk + lane;
+    const size_t i = ((size_t)h * halves + c) * kHalf + lane;
     sums[i] = sum;
     sizes[i] = dt;
 }
@@ -179,268 +180,387 @@ struct ChunkArgs {
     const uint16_t *q, *k, *v;
     float* state;
     const float* powers;       // fixed decays: [heads][65]
-    const float *sums, *sizes; // selective: [heads][chunks][64]
+    const float *sums, *sizes; // selective: [heads][halves][64]
     const float* skip;         // selective: [heads]
     float* chunk_state;        // [chunk][heads][vdim][dq]
     float* out;
-    uint32_t rows, heads, key_heads, dim, vdim, chunks;
+    uint32_t rows, heads, key_heads, dim, vdim, chunks, halves;
     float scale;
 };
+
+// decay^e, e <= 128, from the powers up to 64 (the power 0 is 1)
+__device__ __forceinline__ float power_of(const float* pw, uint32_t e) { const uint32_t f = min(e, kHalf); return pw[f] * pw[e - f]; }
+// Logarithm of the decay from row s to row t >= s of a chunk, from the running sums of its halves: the sums of the two sides of a
+// half's end are small where the rows are near each other, so that their difference keeps its bits.
+__device__ __forceinline__ float log_between(float at_t, float at_s, bool across, float half_end) { return (across ? half_end - at_s : -at_s) + at_t; }
 
 __device__ __forceinline__ lh_bf16x8 bf8(const uint32_t (&w)[4]) {
     struct { uint32_t v[4]; } t = {{w[0], w[1], w[2], w[3]}};
     return __builtin_bit_cast(lh_bf16x8, t);
 }
-
-constexpr uint32_t kLdT = kChunk + 8;     // row length of a transposed tile: 16-byte aligned, rows on different banks
-
-// 64 rows of 64 value columns, transposed into LDS: thread t brings in rows t / 8 and t / 8 + 32, eight columns each.
-struct ValueTile { uint4 x[2]; };
-__device__ __forceinline__ void load_values(ValueTile& f, const ChunkArgs& a, uint32_t t0, uint32_t L, uint32_t h, uint32_t v0, uint32_t tid) {
-    const uint32_t d = v0 + (tid & 7) * 8;
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const uint32_t s = (tid >> 3) + 32 * i;
-        f.x[i] = make_uint4(0u, 0u, 0u, 0u);
-        if (s >= L || d >= a.vdim) continue;
-        const uint16_t* p = a.v + ((size_t)(t0 + s) * a.heads + h) * a.vdim + d;
-        if ((a.vdim & 7) == 0) f.x[i] = *reinterpret_cast<const uint4*>(p);
-        else {
-            uint32_t w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (uint32_t j = 0; j < 8; j++) if (d + j < a.vdim) w[j >> 1] |= (uint32_t)p[j] << (16 * (j & 1));
-            f.x[i] = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-    }
+// Two values as three bf16 terms each, the first value's in the lower halves.
+__device__ __forceinline__ void split3_pair(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    hi = lh_pack_bf(a, b);
+    const float ra = a - __builtin_bit_cast(float, hi << 16), rb = b - __builtin_bit_cast(float, hi & 0xFFFF0000u);
+    mid = lh_pack_bf(ra, rb);
+    lo = lh_pack_bf(ra - __builtin_bit_cast(float, mid << 16), rb - __builtin_bit_cast(float, mid & 0xFFFF0000u));
 }
-template <bool SLOTS>
-__device__ __forceinline__ void park_values(const ValueTile& f, uint16_t (&vt)[64][kLdT], uint32_t tid) {
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const uint32_t s = (tid >> 3) + 32 * i, place = SLOTS ? (s & 32) + lh_block_slot(s & 31) : s;
-        const uint32_t w[4] = {f.x[i].x, f.x[i].y, f.x[i].z, f.x[i].w};
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) vt[(tid & 7) * 8 + j][place] = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
-    }
+// Element j of the rows in a (lower half) and b (upper half).
+__device__ __forceinline__ uint32_t pick(const uint2& a, const uint2& b, int j) {
+    return __builtin_amdgcn_perm(j & 2 ? b.y : b.x, j & 2 ? a.y : a.x, j & 1 ? 0x07060302u : 0x05040100u);
 }
 
-// Step 1.  A workgroup takes one chunk of one head, 32 key columns and 64 value columns; wave w the value columns 16 w ..
-// 16 w + 15.  Row operand = decayed keys (16 key columns x rows), column operand = values (16 value columns x rows).
-template <int DQ, bool SELECTIVE>
+// What lies `offset` bytes behind a base that is the same for the whole wave.
+template <typename T> __device__ __forceinline__ T at(const void* base, uint32_t offset) { return *reinterpret_cast<const T*>(static_cast<const char*>(base) + offset); }
+// Four neighbouring columns of a row of values from `col`, no further than the last column: where there is none, what comes is not
+// used.  (No load below is conditional: a branch around it would wait for it.)
+template <bool VEC> __device__ __forceinline__ uint2 load_values(const uint16_t* base, uint32_t row_offset, uint32_t col, uint32_t vdim) {
+    if constexpr (VEC) return at<uint2>(base, row_offset + 2 * min(col, vdim - 4));
+    const uint32_t last = vdim - 1;
+    auto one = [&](uint32_t j) { return (uint32_t)at<uint16_t>(base, row_offset + 2 * min(col + j, last)); };
+    return make_uint2(one(0) | one(1) << 16, one(2) | one(3) << 16);
+}
+
+// The matrix products below contract over rows, so an operand's eight values lie in eight rows.  A lane therefore loads a few
+// neighbouring columns of eight rows and sorts them in registers: of columns 4 n .. 4 n + 3 of lane n each goes to a tile of its own.
+// Nothing goes through LDS for that (as two-byte stores of a transposed tile it took most of the time).
+
+// Step 1.  A wave takes 32 key columns and 64 value columns of one chunk of one head.  Row operand = decayed keys, column operand
+// = values.  What binds is the split of the decayed keys (7 vector instructions a value) and the latency of the loads.
+// 2048 rows, 16 heads of 128 x 128: 24.5 -> 13 us (64 key columns a wave: 16, half as many waves to hide the loads).
+template <int DQ, bool SELECTIVE, bool VEC>
 __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
-    __shared__ __align__(16) uint16_t kt[3][32][kLdT], vt[64][kLdT];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t vtiles = (a.vdim + 63) / 64, k0 = blockIdx.x % (DQ / 32) * 32, r = blockIdx.x / (DQ / 32);
-    const uint32_t vb = r % vtiles, h = (r / vtiles) % a.heads, c = r / (vtiles * a.heads);
-    const uint32_t t0 = c * kChunk, L = min(kChunk, a.rows - t0), v0 = vb * 64;
-    ValueTile f;
-    load_values(f, a, t0, L, h, v0, tid);
-    {   // eight key columns of one row per thread
-        const uint32_t s = tid >> 2, d = (tid & 3) * 8;
-        uint4 x = make_uint4(0u, 0u, 0u, 0u);
-        float p = 0.0f;
-        if (s < L) {
-            x = *reinterpret_cast<const uint4*>(a.k + ((size_t)(t0 + s) * a.key_heads + h / (a.heads / a.key_heads)) * DQ + k0 + d);
-            if constexpr (SELECTIVE) {
-                const size_t i = ((size_t)h * a.chunks + c) * kChunk;
-                p = expf(a.sums[i + L - 1] - a.sums[i + s]) * a.sizes[i + s];
-            } else p = a.powers[h * (kChunk + 1) + L - 1 - s];
-        }
-        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+    __shared__ float decays[4][kChunk];                        // [wave][row]: from the row to the chunk's end
+    const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n = lane & 15, g = lane >> 4;
+    constexpr uint32_t kblocks = DQ / 32;
+    const uint32_t vtiles = (a.vdim + 63) / 64, unit = blockIdx.x * 4 + wave;
+    const bool on = unit < kblocks * vtiles * a.heads * a.chunks;
+    const uint32_t kb = unit % kblocks, r0 = unit / kblocks, vb = r0 % vtiles, h = (r0 / vtiles) % a.heads, c = on ? r0 / (vtiles * a.heads) : 0;
+    const uint32_t t0 = c * kChunk, L = min(kChunk, a.rows - t0);
+    const uint32_t kstride = a.key_heads * DQ * 2, vstride = a.heads * a.vdim * 2, kcol = kb * 32 + n * 2, vcol = vb * 64 + n * 4;   // strides in bytes
+    const uint16_t *kp = a.k + ((size_t)t0 * a.key_heads + h / (a.heads / a.key_heads)) * DQ, *vp = a.v + ((size_t)t0 * a.heads + h) * a.vdim;
+    struct Rows { uint32_t k[8]; uint2 v[8]; } rows[4];
+    const uint32_t k0 = 8 * g * kstride, v0 = 8 * g * vstride;
+    auto fetch = [&](Rows& to, uint32_t s0) {                  // (rows past the last: the last again, whose decay is 0 then)
 #pragma unroll
-        for (uint32_t j = 0; j < 8; j++) {
-            const LhSplit3 e = lh_split3(s < L && k0 + d + j < a.dim ? lh_bf2f((uint16_t)(w[j >> 1] >> (16 * (j & 1)))) * p : 0.0f);
-            kt[0][d + j][s] = e.hi; kt[1][d + j][s] = e.mid; kt[2][d + j][s] = e.lo;
+        for (uint32_t i = 0; i < 8; i++) {
+            to.k[i] = at<uint32_t>(kp, min(k0 + (s0 + i) * kstride, (L - 1) * kstride) + 2 * kcol);
+            to.v[i] = load_values<VEC>(vp, min(v0 + (s0 + i) * vstride, (L - 1) * vstride), vcol, a.vdim);
         }
+    };
+    fetch(rows[0], 0);
+    fetch(rows[1], 32);
+#pragma unroll
+    for (uint32_t half = 0; half < 2; half++) {
+        const uint32_t s = half * kHalf + lane, r = min(s, L - 1);
+        float p;
+        if constexpr (SELECTIVE) {
+            const float* sums = a.sums + ((size_t)h * a.halves + 2 * c) * kHalf;
+            const bool across = half == 0 && L > kHalf;
+            p = expf(log_between(sums[L - 1], sums[r], across, sums[min(kHalf, L) - 1])) * a.sizes[((size_t)h * a.halves + 2 * c) * kHalf + r];
+        } else p = power_of(a.powers + h * (kHalf + 1), L - 1 - r);
+        decays[wave][s] = s < L ? p : 0.0f;
     }
-    park_values<false>(f, vt, tid);
     __syncthreads();
-    lh_f32x4 acc[2] = {(lh_f32x4){0.f, 0.f, 0.f, 0.f}, (lh_f32x4){0.f, 0.f, 0.f, 0.f}};
+    if (!on) return;
+    const uint32_t keep = (kcol < a.dim ? 0xFFFFu : 0u) | (kcol + 1 < a.dim ? 0xFFFF0000u : 0u);   // key columns that exist
+    lh_f32x4 acc[2][4];
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-        const uint32_t s = ks * 32 + (lane >> 4) * 8;
-        const lh_bf16x8 vf = *reinterpret_cast<const lh_bf16x8*>(&vt[wave * 16 + (lane & 15)][s]);
+    for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int d = 0; d < 4; d++) acc[j][d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int p = 0; p < 3; p++)
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const lh_bf16x8*>(&kt[p][i * 16 + (lane & 15)][s]), vf, acc[i], 0, 0, 0);
+    for (uint32_t step = 0; step < 4; step++) {
+        const uint32_t s0 = step * 32;
+        if (s0 >= L) break;
+        const Rows& now = rows[step];
+        if (step < 2) fetch(rows[step + 2], s0 + 64);
+        lh_bf16x8 vf[4];
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[i] = pick(now.v[2 * i], now.v[2 * i + 1], d);
+            vf[d] = bf8(w);
+        }
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) p[i] = decays[wave][s0 + 8 * g + i];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            uint32_t w[3][4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float f[2];
+#pragma unroll
+                for (int b = 0; b < 2; b++) {
+                    const uint32_t x = now.k[2 * i + b] & keep;
+                    f[b] = __builtin_bit_cast(float, j ? x & 0xFFFF0000u : x << 16) * p[2 * i + b];
+                }
+                split3_pair(f[0], f[1], w[0][i], w[1][i], w[2][i]);
+            }
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+#pragma unroll
+                for (int z = 0; z < 3; z++) acc[j][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf8(w[z]), vf[d], acc[j][d], 0, 0, 0);
+        }
     }
-    const uint32_t col = v0 + wave * 16 + (lane & 15);
-    if (col >= a.vdim) return;
-    float* U = a.chunk_state + ((size_t)c * a.heads + h) * a.vdim * DQ + (size_t)col * DQ + k0 + (lane >> 4) * 4;
+    // a lane holds eight neighbouring key columns of four value columns
+    float* U = a.chunk_state + ((size_t)c * a.heads + h) * a.vdim * DQ + kb * 32 + g * 8;
 #pragma unroll
-    for (int i = 0; i < 2; i++) *reinterpret_cast<float4*>(U + i * 16) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+    for (int d = 0; d < 4; d++) {
+        if (vcol + d >= a.vdim) continue;
+        float4* to = reinterpret_cast<float4*>(U + (size_t)(vcol + d) * DQ);
+#pragma unroll
+        for (int i = 0; i < 2; i++) to[i] = make_float4(acc[0][d][2 * i], acc[1][d][2 * i], acc[0][d][2 * i + 1], acc[1][d][2 * i + 1]);
+    }
 }
 
-// Step 2.  A thread owns four neighbouring state values and walks the chunks, eight loads ahead.
+// Step 2.  A thread owns four neighbouring state values and walks the chunks, eight loads ahead.  Memory binds: 15 -> 8 us for 2048
+// rows, 16 heads of 128 x 128, with half as many states.
 template <bool SELECTIVE>
 __global__ __launch_bounds__(256) void chunk_scan_kernel(const ChunkArgs a, uint32_t dq) {
     const size_t per_head4 = (size_t)a.vdim * dq / 4, total4 = per_head4 * a.heads, i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= total4) return;
     const uint32_t h = (uint32_t)(i / per_head4);
-    const float* pw = SELECTIVE ? nullptr : a.powers + h * (kChunk + 1);
-    const float full = SELECTIVE ? 0.0f : pw[kChunk];
+    const float* pw = SELECTIVE ? nullptr : a.powers + h * (kHalf + 1);
     float4* st = reinterpret_cast<float4*>(a.state) + i;
     float4* u = reinterpret_cast<float4*>(a.chunk_state) + i;
     float4 s = *st;
     constexpr uint32_t P = 8;
     for (uint32_t c0 = 0; c0 < a.chunks; c0 += P) {
         float4 x[P];
+        float d[P];
 #pragma unroll
-        for (uint32_t j = 0; j < P; j++) x[j] = u[(size_t)min(c0 + j, a.chunks - 1) * total4];
+        for (uint32_t j = 0; j < P; j++) {
+            const uint32_t c = min(c0 + j, a.chunks - 1), L = min(kChunk, a.rows - c * kChunk);
+            x[j] = u[(size_t)c * total4];
+            if constexpr (SELECTIVE) {
+                const float* sums = a.sums + ((size_t)h * a.halves + 2 * c) * kHalf;
+                d[j] = sums[min(L, kHalf) - 1] + (L > kHalf ? sums[L - 1] : 0.0f);
+            } else d[j] = power_of(pw, L);
+        }
 #pragma unroll
         for (uint32_t j = 0; j < P; j++) {
             if (c0 + j >= a.chunks) break;
             u[(size_t)(c0 + j) * total4] = s;
-            const float d = SELECTIVE ? expf(a.sums[((size_t)h * a.chunks + c0 + j) * kChunk + kChunk - 1]) : c0 + j + 1 < a.chunks ? full : pw[a.rows - (a.chunks - 1) * kChunk];
-            s.x = __builtin_fmaf(d, s.x, x[j].x); s.y = __builtin_fmaf(d, s.y, x[j].y);
-            s.z = __builtin_fmaf(d, s.z, x[j].z); s.w = __builtin_fmaf(d, s.w, x[j].w);
+            const float f = SELECTIVE ? expf(d[j]) : d[j];
+            s.x = __builtin_fmaf(f, s.x, x[j].x); s.y = __builtin_fmaf(f, s.y, x[j].y);
+            s.z = __builtin_fmaf(f, s.z, x[j].z); s.w = __builtin_fmaf(f, s.w, x[j].w);
         }
     }
     *st = s;
 }
 
-// Step 3.  A workgroup takes one chunk of one head and 64 value columns; wave w the rows 16 w .. 16 w + 15.
+// Step 3.  A workgroup takes one chunk of one head and 64 value columns; a wave 32 of its rows.
 // Scores transposed (row operand keys, column operand queries), so that the decayed scores are in operand order for
 // O^T = V^T P^T, whose k index 8g + j is row 4g + j of the first 16-row tile (j < 4) or 4g + j - 4 of the second.
-template <int DQ, bool SELECTIVE>
-__global__ __launch_bounds__(256) void chunk_output_kernel(const ChunkArgs a) {
-    __shared__ __align__(16) uint16_t vt[64][kLdT];            // [value column][32-row half][slot]
-    __shared__ float pws[kChunk + 1], sizes[SELECTIVE ? kChunk : 1];   // powers of the decay, or running sums of its logarithm
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4;
+// The state is split into its bf16 terms once, by all waves, into LDS in operand order.  (Every wave of a chunk of 64 rows splitting
+// it for itself was what bound this step: twice the states, four times the splits.)  What binds now is the vector work on the
+// scores, so the operands of keys and values serve 32 rows.  2048 rows, 16 heads of 128 x 128:
+// 32 -> 20.5 us.
+template <int DQ, bool SELECTIVE, bool VEC>
+__global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(const ChunkArgs a) {
+    constexpr int KB = DQ < 128 ? DQ : 128;                    // key columns of the state in LDS at a time
+    __shared__ uint4 terms[3][4][KB / 32][64];                 // [term][value tile][32 key columns][lane]
+    __shared__ float pws[kChunk + 4], sizes[SELECTIVE ? kChunk : 1];   // powers of the decay, or running sums of its logarithm
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), g = lane >> 4, n = lane & 15;
     const uint32_t vtiles = (a.vdim + 63) / 64, vb = blockIdx.x % vtiles, h = (blockIdx.x / vtiles) % a.heads, c = blockIdx.x / (vtiles * a.heads);
     const uint32_t t0 = c * kChunk, L = min(kChunk, a.rows - t0), v0 = vb * 64;
-    ValueTile f;
-    load_values(f, a, t0, L, h, v0, tid);
-    const uint32_t kh = h / (a.heads / a.key_heads);
-    if constexpr (SELECTIVE) {
-        if (tid < kChunk) { pws[tid] = a.sums[((size_t)h * a.chunks + c) * kChunk + tid]; sizes[tid] = a.sizes[((size_t)h * a.chunks + c) * kChunk + tid]; }
-    } else if (tid <= kChunk) pws[tid] = a.powers[h * (kChunk + 1) + tid];
-    const uint32_t t = wave * 16 + (lane & 15), tr = min(t, L - 1);
-    lh_bf16x8 qf[DQ / 32];
+    // late rows see more of the chunk: of two workgroups on a CU one has them on the SIMDs where the other has the early ones
+    const uint32_t w0 = ((blockIdx.x >> 8) & 1 ? 3 - wave : wave) * 32;
+    const bool on = w0 < L;
+    const uint32_t kh = h / (a.heads / a.key_heads), kstride = a.key_heads * DQ * 2, vstride = a.heads * a.vdim * 2;   // strides in bytes
+    const uint16_t *qp = a.q + ((size_t)t0 * a.key_heads + kh) * DQ, *kp = a.k + ((size_t)t0 * a.key_heads + kh) * DQ, *vp = a.v + ((size_t)t0 * a.heads + h) * a.vdim;
+    const float* S = a.chunk_state + (((size_t)c * a.heads + h) * a.vdim) * DQ;
+    constexpr uint32_t each = 4 * (KB / 32) * 64 / 256;        // operands of eight values a thread brings in
+    float4 x[each][2];
+    auto fetch_state = [&](uint32_t k0) {
 #pragma unroll
-    for (int i = 0; i < DQ / 32; i++) {
-        const uint32_t k = i * 32 + g * 8;
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-        if (k < a.dim) {
-            const uint4 x = *reinterpret_cast<const uint4*>(a.q + ((size_t)(t0 + tr) * a.key_heads + kh) * DQ + k);
-            w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (k + 2 * j >= a.dim) w[j] = 0u;
-                else if (k + 2 * j + 1 >= a.dim) w[j] &= 0xFFFFu;
-            }
+        for (uint32_t e = 0; e < each; e++) {
+            const uint32_t u = tid + 256 * e, l = u & 63, i = (u >> 6) % (KB / 32), d = (u >> 6) / (KB / 32);
+            const uint32_t o = (min(v0 + (l & 15) * 4 + d, a.vdim - 1) * DQ + k0 + i * 32 + (l >> 4) * 8) * 4;
+            x[e][0] = at<float4>(S, o);
+            x[e][1] = at<float4>(S, o + 16);
         }
-        qf[i] = bf8(w);
+    };
+    fetch_state(0);
+    lh_bf16x8 qf[2][DQ / 32];
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int i = 0; i < DQ / 32; i++) qf[b][i] = at<lh_bf16x8>(qp, min(w0 + 16 * b + n, L - 1) * kstride + i * 64 + g * 16);
+    struct Rows { lh_bf16x8 k[2][DQ / 32]; uint2 v[8]; } next;
+    auto fetch = [&](uint32_t s0) {                            // 32 rows of keys and values, in operand order
+#pragma unroll
+        for (uint32_t u = 0; u < 2; u++) {
+            const uint32_t o = min(n * kstride + (s0 + u * 16) * kstride, (L - 1) * kstride) + g * 16;
+#pragma unroll
+            for (int i = 0; i < DQ / 32; i++) next.k[u][i] = at<lh_bf16x8>(kp, o + i * 64);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 8; i++)
+            next.v[i] = load_values<VEC>(vp, min(4 * g * vstride + (s0 + (i >> 2) * 16 + (i & 3)) * vstride, (L - 1) * vstride), v0 + n * 4, a.vdim);
+    };
+    fetch(0);
+    if constexpr (SELECTIVE) {
+        if (tid < kChunk) {
+            const size_t i = ((size_t)h * a.halves + 2 * c) * kHalf + min(tid, L - 1);
+            pws[tid] = a.sums[i];
+            sizes[tid] = a.sizes[i];
+        }
+    } else if (tid <= kChunk) pws[tid] = power_of(a.powers + h * (kHalf + 1), tid);
+    if (a.dim != DQ) {                                         // columns that do not exist
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int i = 0; i < DQ / 32; i++)
+#pragma unroll
+                for (uint32_t j = 0; j < 8; j++) if (i * 32 + g * 8 + j >= a.dim) qf[b][i][j] = (__bf16)0.0f;
     }
-    park_values<true>(f, vt, tid);
-    __syncthreads();
-    if (wave * 16 >= L) return;
-    lh_f32x4 o[4];
+    lh_f32x4 o[2][4];
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) o[b][d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
     // the state's part, scaled by decay^(t + 1) afterwards
-    const float* S = a.chunk_state + ((size_t)c * a.heads + h) * a.vdim * DQ;
 #pragma unroll
-    for (int d = 0; d < 4; d++) {
-        o[d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
-        if (v0 + d * 16 >= a.vdim) continue;
-        const float* srow = S + (size_t)min(v0 + d * 16 + (lane & 15), a.vdim - 1) * DQ + g * 8;
+    for (int k0 = 0; k0 < DQ; k0 += KB) {
+        if (k0) { __syncthreads(); fetch_state(k0); }
 #pragma unroll
-        for (int i = 0; i < DQ / 32; i++) {
-            const float4 x = *reinterpret_cast<const float4*>(srow + i * 32), y = *reinterpret_cast<const float4*>(srow + i * 32 + 4);
-            const float f[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+        for (uint32_t e = 0; e < each; e++) {
+            const float f[8] = {x[e][0].x, x[e][0].y, x[e][0].z, x[e][0].w, x[e][1].x, x[e][1].y, x[e][1].z, x[e][1].w};
+            uint32_t p[3][4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) split3_pair(f[2 * j], f[2 * j + 1], p[0][j], p[1][j], p[2][j]);
+#pragma unroll
+            for (int z = 0; z < 3; z++) (&terms[z][0][0][0])[tid + 256 * e] = make_uint4(p[z][0], p[z][1], p[z][2], p[z][3]);
+        }
+        __syncthreads();
+        if (!on) continue;
+#pragma unroll
+        for (int i = 0; i < KB / 32; i++)
+#pragma unroll
+            for (int z = 2; z >= 0; z--) {
+                lh_bf16x8 sf[4];
+#pragma unroll
+                for (int d = 0; d < 4; d++) sf[d] = __builtin_bit_cast(lh_bf16x8, terms[z][d][i][lane]);
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+#pragma unroll
+                    for (int d = 0; d < 4; d++) o[b][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sf[d], qf[b][k0 / 32 + i], o[b][d], 0, 0, 0);
+            }
+    }
+    if (!on) return;
+    const bool late = w0 >= kHalf;                             // rows of the chunk's second half
+    const float half_end = SELECTIVE ? pws[kHalf - 1] : 0.0f;
+    float own[2];                                              // selective: the running sum at the lane's row
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const uint32_t tr = min(w0 + 16 * b + n, L - 1);
+        own[b] = SELECTIVE ? pws[tr] : 0.0f;
+        const float carry = SELECTIVE ? expf(late ? half_end + own[b] : own[b]) : pws[tr + 1];
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[b][d][r] *= carry;
+    }
+    // the chunk's own rows, 32 at a time
+#pragma unroll 1
+    for (uint32_t s0 = 0; s0 <= w0; s0 += 32) {
+        lh_f32x4 sc[2][2];
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                sc[b][u] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < DQ / 32; i++) sc[b][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(next.k[u][i], qf[b][i], sc[b][u], 0, 0, 0);
+            }
+        lh_bf16x8 vf[4];
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[i] = pick(next.v[2 * i], next.v[2 * i + 1], d);
+            vf[d] = bf8(w);
+        }
+        if (s0 < w0) fetch(s0 + 32);
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const uint32_t t = w0 + 16 * b + n;
             uint32_t p[3][4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const LhSplit3 e = lh_split3(f[2 * j]), m = lh_split3(f[2 * j + 1]);
-                p[0][j] = (uint32_t)e.hi | ((uint32_t)m.hi << 16);
-                p[1][j] = (uint32_t)e.mid | ((uint32_t)m.mid << 16);
-                p[2][j] = (uint32_t)e.lo | ((uint32_t)m.lo << 16);
+                float e[2];
+#pragma unroll
+                for (int y = 0; y < 2; y++) {
+                    const int m = 2 * j + y;
+                    const uint32_t s = s0 + (m >> 2) * 16 + g * 4 + (m & 3);
+                    const float f = SELECTIVE ? expf(fminf(log_between(own[b], pws[s], late && s0 < kHalf, half_end), 0.0f)) * sizes[s] : pws[min(t - s, kChunk)];
+                    // the factor is evaluated for rows after t as well: skipping it would take a branch for each
+                    e[y] = (s <= t ? sc[b][m >> 2][m & 3] : 0.0f) * f;
+                }
+                split3_pair(e[0], e[1], p[0][j], p[1][j], p[2][j]);
             }
 #pragma unroll
-            for (int z = 2; z >= 0; z--) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf8(p[z]), qf[i], o[d], 0, 0, 0);
+            for (int z = 2; z >= 0; z--)
+#pragma unroll
+                for (int d = 0; d < 4; d++) o[b][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], bf8(p[z]), o[b][d], 0, 0, 0);
         }
     }
-    const float carry = SELECTIVE ? expf(pws[tr]) : pws[tr + 1];
-#pragma unroll
-    for (int d = 0; d < 4; d++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) o[d][r] *= carry;
-    // the chunk's own rows, 32 at a time
-    for (uint32_t s0 = 0; s0 <= wave * 16 + 15 && s0 < L; s0 += 32) {
-        lh_f32x4 sc[2];
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            sc[u] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
-            const uint32_t s = min(s0 + u * 16 + (lane & 15), L - 1);
-            const uint16_t* kr = a.k + ((size_t)(t0 + s) * a.key_heads + kh) * DQ + g * 8;
-#pragma unroll
-            for (int i = 0; i < DQ / 32; i++) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const lh_bf16x8*>(kr + i * 32), qf[i], sc[u], 0, 0, 0);
-        }
-        uint32_t p[3][4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            LhSplit3 e[2];
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                const int n = 2 * j + b;
-                const uint32_t s = s0 + (n >> 2) * 16 + g * 4 + (n & 3);
-                const float f = SELECTIVE ? expf(fminf(pws[tr] - pws[min(s, kChunk - 1)], 0.0f)) * sizes[min(s, kChunk - 1)] : pws[min(t - s, kChunk)];
-                e[b] = lh_split3(s <= t && s < L ? sc[n >> 2][n & 3] * f : 0.0f);
-            }
-            p[0][j] = (uint32_t)e[0].hi | ((uint32_t)e[1].hi << 16);
-            p[1][j] = (uint32_t)e[0].mid | ((uint32_t)e[1].mid << 16);
-            p[2][j] = (uint32_t)e[0].lo | ((uint32_t)e[1].lo << 16);
-        }
-#pragma unroll
-        for (int d = 0; d < 4; d++) {
-            const lh_bf16x8 vf = *reinterpret_cast<const lh_bf16x8*>(&vt[d * 16 + (lane & 15)][s0 + g * 8]);
-#pragma unroll
-            for (int z = 2; z >= 0; z--) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, bf8(p[z]), o[d], 0, 0, 0);
-        }
-    }
-    if (t >= L) return;
-    float* out = a.out + ((size_t)(t0 + t) * a.heads + h) * a.vdim + v0;
-    const uint16_t* x = a.v + ((size_t)(t0 + t) * a.heads + h) * a.vdim + v0;
+    // a lane holds 16 neighbouring value columns of its rows
     const float skip = SELECTIVE ? a.skip[h] : 0.0f;
 #pragma unroll
-    for (int d = 0; d < 4; d++) {
-        const uint32_t col = d * 16 + g * 4;
-        if (v0 + col >= a.vdim) continue;
+    for (int b = 0; b < 2; b++) {
+        const uint32_t t = w0 + 16 * b + n;
+        if (t >= L) continue;
+        float* out = a.out + ((size_t)(t0 + t) * a.heads + h) * a.vdim;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            if constexpr (SELECTIVE) o[d][r] = __builtin_fmaf(skip, lh_bf2f(x[min(col + r, a.vdim - 1 - v0)]), o[d][r]);
-            else o[d][r] *= a.scale;
-        }
-        if ((a.vdim & 3) == 0) { if (v0 + col < a.vdim) *reinterpret_cast<float4*>(out + col) = make_float4(o[d][0], o[d][1], o[d][2], o[d][3]); }
-        else {
+            const uint32_t col = v0 + g * 16 + r * 4;
+            if (col >= a.vdim) continue;
+            float y[4];
+            if constexpr (SELECTIVE) {
+                const uint2 z = load_values<VEC>(vp, t * vstride, col, a.vdim);
+                y[0] = __builtin_bit_cast(float, z.x << 16); y[1] = __builtin_bit_cast(float, z.x & 0xFFFF0000u);
+                y[2] = __builtin_bit_cast(float, z.y << 16); y[3] = __builtin_bit_cast(float, z.y & 0xFFFF0000u);
+            }
 #pragma unroll
-            for (int r = 0; r < 4; r++) if (v0 + col + r < a.vdim) out[col + r] = o[d][r];
+            for (int d = 0; d < 4; d++) y[d] = SELECTIVE ? __builtin_fmaf(skip, y[d], o[b][d][r]) : o[b][d][r] * a.scale;
+            if constexpr (VEC) *reinterpret_cast<float4*>(out + col) = make_float4(y[0], y[1], y[2], y[3]);
+            else
+#pragma unroll
+                for (uint32_t d = 0; d < 4; d++) if (col + d < a.vdim) out[col + d] = y[d];
         }
     }
 }
 
-template <int DQ, bool SELECTIVE>
+template <int DQ, bool SELECTIVE, bool VEC>
 int launch_chunked(lh_context* ctx, const ChunkArgs& a, const char* op) {
-    const uint32_t grid = a.chunks * a.heads * ((a.vdim + 63) / 64);
-    hipLaunchKernelGGL((chunk_state_kernel<DQ, SELECTIVE>), dim3(grid * (DQ / 32)), dim3(256), 0, ctx->stream, a);
+    const uint32_t grid = a.chunks * a.heads * ((a.vdim + 63) / 64), waves = grid * (DQ / 32);
+    hipLaunchKernelGGL((chunk_state_kernel<DQ, SELECTIVE, VEC>), dim3((waves + 3) / 4), dim3(256), 0, ctx->stream, a);
     int r = lh_check_launch(op);
     if (r != LH_OK) return r;
     const size_t total4 = (size_t)a.heads * a.vdim * DQ / 4;
     hipLaunchKernelGGL((chunk_scan_kernel<SELECTIVE>), dim3((uint32_t)((total4 + 255) / 256)), dim3(256), 0, ctx->stream, a, (uint32_t)DQ);
     r = lh_check_launch(op);
     if (r != LH_OK) return r;
-    hipLaunchKernelGGL((chunk_output_kernel<DQ, SELECTIVE>), dim3(grid), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL((chunk_output_kernel<DQ, SELECTIVE, VEC>), dim3(grid), dim3(256), 0, ctx->stream, a);
     return lh_check_launch(op);
+}
+template <bool SELECTIVE, bool VEC>
+int launch_chunked_vec(lh_context* ctx, const ChunkArgs& a, const char* op) {
+    switch (lh_linear_attention_padded_dim(a.dim)) {
+        case 32: return launch_chunked<32, SELECTIVE, VEC>(ctx, a, op);
+        case 64: return launch_chunked<64, SELECTIVE, VEC>(ctx, a, op);
+        case 128: return launch_chunked<128, SELECTIVE, VEC>(ctx, a, op);
+        default: return launch_chunked<256, SELECTIVE, VEC>(ctx, a, op);
+    }
 }
 template <bool SELECTIVE>
 int launch_chunked_dim(lh_context* ctx, const ChunkArgs& a, const char* op) {
-    switch (lh_linear_attention_padded_dim(a.dim)) {
-        case 32: return launch_chunked<32, SELECTIVE>(ctx, a, op);
-        case 64: return launch_chunked<64, SELECTIVE>(ctx, a, op);
-        case 128: return launch_chunked<128, SELECTIVE>(ctx, a, op);
-        default: return launch_chunked<256, SELECTIVE>(ctx, a, op);
-    }
+    return a.vdim % 4 == 0 ? launch_chunked_vec<SELECTIVE, true>(ctx, a, op) : launch_chunked_vec<SELECTIVE, false>(ctx, a, op);
 }
 
 template <typename T, bool SELECTIVE>
@@ -514,23 +634,24 @@ int lh_linear_attention_chunked_into(lh_batch* batch, const lh_buffer* q, const 
     LH_NEED(k, (size_t)rows * heads * dq * 2, op, "k");
     LH_NEED(v, (size_t)rows * heads * vdim * 2, op, "v");
     LH_NEED(state, (size_t)heads * vdim * dq * 4, op, "state");
-    LH_NEED(decay_powers, (size_t)heads * (kChunk + 1) * 4, op, "decay_powers");
+    LH_NEED(decay_powers, (size_t)heads * (kHalf + 1) * 4, op, "decay_powers");
     LH_NEED(workspace, lh_linear_attention_workspace_bytes(rows, heads, dim, vdim), op, "workspace");
     LH_NEED(output, (size_t)rows * heads * vdim * 4, op, "output");
     LH_REQUIRE((((uintptr_t)q->ptr | (uintptr_t)k->ptr | (uintptr_t)v->ptr | (uintptr_t)state->ptr | (uintptr_t)workspace->ptr | (uintptr_t)output->ptr) & 15) == 0,
                "%s: buffers must be 16-byte aligned", op);
+    LH_REQUIRE((uint64_t)heads * std::max(dq, vdim) < (1u << 24), "%s: %u heads of %u and %u columns", op, heads, dim, vdim);   // offsets within a chunk are 32-bit
     ChunkArgs a{};
     a.q = (const uint16_t*)q->ptr; a.k = (const uint16_t*)k->ptr; a.v = (const uint16_t*)v->ptr; a.state = (float*)state->ptr;
     a.powers = (const float*)decay_powers->ptr; a.chunk_state = (float*)workspace->ptr; a.out = (float*)output->ptr;
-    a.rows = rows; a.heads = a.key_heads = heads; a.dim = dim; a.vdim = vdim; a.chunks = (rows + kChunk - 1) / kChunk; a.scale = scale;
+    a.rows = rows; a.heads = a.key_heads = heads; a.dim = dim; a.vdim = vdim; a.chunks = (rows + kChunk - 1) / kChunk; a.halves = (rows + kHalf - 1) / kHalf; a.scale = scale;
     LH_REQUIRE((uint64_t)a.chunks * heads * ((vdim + 63) / 64) * 8 < 0x7FFFFFFFull, "%s: %u rows", op, rows);
     const int r = launch_chunked_dim<false>(batch->ctx, a, op);
     if (r == LH_OK) batch->dispatch_count += 3;
     return r;
 }
 
-// [heads][chunks][64] running sums, then as many step sizes
-size_t lh_selective_steps_bytes(uint32_t rows, uint32_t heads) { return (size_t)((rows + kChunk - 1) / kChunk) * kChunk * heads * 2 * 4; }
+// [heads][halves][64] running sums, then as many step sizes
+size_t lh_selective_steps_bytes(uint32_t rows, uint32_t heads) { return (size_t)((rows + kHalf - 1) / kHalf) * kHalf * heads * 2 * 4; }
 
 int lh_selective_recurrent_into(lh_batch* batch, const lh_buffer* x, const lh_buffer* b, const lh_buffer* c, int dtype, const lh_buffer* dt_raw,
                                 const lh_buffer* dt_bias, const lh_buffer* a_log, const lh_buffer* skip, lh_buffer* memory, lh_buffer* output, uint32_t rows,
@@ -583,16 +704,17 @@ int lh_selective_chunked_into(lh_batch* batch, const lh_buffer* x, const lh_buff
     LH_NEED(output, (size_t)rows * heads * vdim * 4, op, "output");
     LH_REQUIRE((((uintptr_t)x->ptr | (uintptr_t)b->ptr | (uintptr_t)c->ptr | (uintptr_t)memory->ptr | (uintptr_t)workspace->ptr | (uintptr_t)output->ptr) & 15) == 0,
                "%s: buffers must be 16-byte aligned", op);
+    LH_REQUIRE((uint64_t)heads * std::max(dq, vdim) < (1u << 24), "%s: %u heads of %u and %u columns", op, heads, state, vdim);   // offsets within a chunk are 32-bit
     ChunkArgs a{};
     a.q = (const uint16_t*)c->ptr; a.k = (const uint16_t*)b->ptr; a.v = (const uint16_t*)x->ptr; a.state = (float*)memory->ptr;
     a.chunk_state = (float*)workspace->ptr; a.out = (float*)output->ptr; a.skip = (const float*)skip->ptr;
-    a.rows = rows; a.heads = heads; a.key_heads = groups; a.dim = state; a.vdim = vdim; a.chunks = (rows + kChunk - 1) / kChunk; a.scale = 1.0f;
+    a.rows = rows; a.heads = heads; a.key_heads = groups; a.dim = state; a.vdim = vdim; a.chunks = (rows + kChunk - 1) / kChunk; a.halves = (rows + kHalf - 1) / kHalf; a.scale = 1.0f;
     LH_REQUIRE((uint64_t)a.chunks * heads * ((vdim + 63) / 64) * 8 < 0x7FFFFFFFull, "%s: %u rows", op, rows);
     float* sums = (float*)steps->ptr;
-    float* sizes = sums + (size_t)a.chunks * kChunk * heads;
+    float* sizes = sums + (size_t)a.halves * kHalf * heads;
     a.sums = sums; a.sizes = sizes;
-    hipLaunchKernelGGL(chunk_steps_kernel, dim3(a.chunks * heads), dim3(64), 0, batch->ctx->stream, (const float*)dt_raw->ptr, (const float*)dt_bias->ptr,
-                       (const float*)a_log->ptr, sums, sizes, rows, heads, a.chunks);
+    hipLaunchKernelGGL(chunk_steps_kernel, dim3(a.halves * heads), dim3(64), 0, batch->ctx->stream, (const float*)dt_raw->ptr, (const float*)dt_bias->ptr,
+                       (const float*)a_log->ptr, sums, sizes, rows, heads, a.halves);
     int r = lh_check_launch(op);
     if (r == LH_OK) r = launch_chunked_dim<true>(batch->ctx, a, op);
     if (r == LH_OK) batch->dispatch_count += 4;

@@ -21,7 +21,7 @@ from . import (ACT_GELU_TANH, ACT_NONE, ACT_RELU_SQUARED, ACT_SIGMOID, ACT_SILU,
 from .kv_cache import BlockKvCache, LatentCache, RecurrentState, SelectiveState
 from .linear_weight import Segment, Segments, StackedLinear
 
-CHUNK = 64                 # rows per chunk of lh_linear_attention_chunked_into and lh_selective_chunked_into
+CHUNK = 64                 # the powers that lh_linear_attention_chunked_into takes: decay^0 .. decay^64
 CHUNKED_MIN_ROWS = 17      # below this a portion walks the recurrence
 MAX_CHUNKED_DIM = 256
 GATED_IN_PRODUCT = 2048    # longer gated norms are a step of their own: every wave of the product would repeat them

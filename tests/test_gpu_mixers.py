@@ -592,6 +592,27 @@ def test_linear_attention_forms(ai, gpu, heads, dim, vdim, cuts):
             at += n
 
 
+@pytest.mark.parametrize("heads,dim,vdim,rows", [(64, 64, 64, 1100), (8, 256, 100, 1153), (3, 128, 64, 127), (3, 128, 64, 128), (2, 40, 6, 129), (2, 128, 130, 193)])
+def test_linear_attention_chunks(ai, gpu, heads, dim, vdim, rows):
+    """Chunks of 128 rows: whole, one row short and over, ending in either half; one and several tiles of key and value columns."""
+    ctx, K = gpu
+    g = np.random.default_rng(heads + dim + rows)
+    decay, dq = np.linspace(0.6, 1.0, heads), K.linear_attention_padded_dim(dim)
+    q, k, v = (M.rounded(g.standard_normal(s)) for s in ((rows, heads, dim), (rows, heads, dim), (rows, heads, vdim)))
+    pad = [(0, 0), (0, 0), (0, dq - dim)]
+    state, out = ai.Buffer.empty(ctx, heads * vdim * dq * 4), empty(ai, ctx, rows * heads * vdim, ai.F32)
+    pw = ai.Buffer.from_slice(ctx, (decay[:, None] ** np.arange(65)).astype(np.float32))
+    work = ai.Buffer.empty(ctx, K.linear_attention_workspace_bytes(rows, heads, dim, vdim))
+    print(f"chunks {heads} {dim} {vdim} {rows}", flush=True)
+    batch = ai.CommandBatch(ctx)
+    K.linear_attention_chunked_into(batch, upload(ai, ctx, np.pad(q, pad), ai.BF16), upload(ai, ctx, np.pad(k, pad), ai.BF16), upload(ai, ctx, v, ai.BF16), state, pw,
+                                    work, out, rows, heads, dim, vdim)
+    batch.commit_and_wait()
+    want, end = O.lightning_recurrence(q, k, v, decay, None)
+    close(download(ai, out, rows * heads * vdim, ai.F32).reshape(rows, heads, vdim), want, F32_TOL, "output")
+    close(state.as_array(np.float32).reshape(heads, vdim, dq)[:, :, :dim], end.transpose(0, 2, 1), F32_TOL, "state")
+
+
 # ---- mixture of experts ------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("rows,experts,top,width,ff", [(2, 5, 2, 64, 48), (7, 3, 3, 40, 33), (65, 11, 1, 64, 88), (300, 4, 2, 64, 72), (600, 2, 1, 32, 40),
