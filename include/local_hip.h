@@ -684,6 +684,10 @@ LH_API int lh_linear_norm_vector_into(lh_batch* batch, const lh_buffer* input, c
                                       const uint32_t* acts, const uint32_t* heads, const uint32_t* padded,
                                       const uint32_t* layouts, lh_buffer* const* outputs, int output_dtype,
                                       int accumulate, const lh_buffer* position);
+/* the same for f32 logits: cap * tanh(v / cap) of each of n sums (cap > 0) */
+LH_API int lh_linear_norm_vector_capped_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps,
+                                             const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t n,
+                                             lh_buffer* output, float cap);
 LH_API int lh_linear_residual_vector_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* branch,
                                           lh_buffer* store, const lh_buffer* norm_weight, float eps,
                                           const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t count,
@@ -822,9 +826,11 @@ LH_API int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const 
 LH_API int lh_moe_vector_down_into(lh_batch* batch, const lh_buffer* hidden, const lh_buffer* logits, const lh_buffer* down,
                                    lh_buffer* residual, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff);
 
-/* *position += by (u32), and the index of the largest of each row of f32 logits (ties: the lower index) */
+/* *position += by (u32); the index of the largest of each row of f32 logits (ties: the lower index); both, for one row */
 LH_API int lh_advance_position_into(lh_batch* batch, lh_buffer* position, uint32_t by);
 LH_API int lh_argmax_rows_f32_into(lh_batch* batch, const lh_buffer* logits, lh_buffer* index, uint32_t rows, uint32_t n);
+LH_API int lh_argmax_advance_f32_into(lh_batch* batch, const lh_buffer* logits, lh_buffer* index, uint32_t n, lh_buffer* position,
+                                      uint32_t by);
 
 #ifdef __cplusplus
 }

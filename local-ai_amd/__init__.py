@@ -819,6 +819,10 @@ class Kernels:
                                                   weight._h, _opt(bias), _u32(k), *segments.args, _handles(outputs),
                                                   C.c_int(output_dtype), C.c_int(bool(accumulate)), _opt(position)))
 
+    def linear_norm_vector_capped_into(self, batch, input, norm_weight, eps, weight, bias, k, n, output, cap):
+        _check(self._l.lh_linear_norm_vector_capped_into(batch._h, input._h, norm_weight._h, C.c_float(eps), weight._h, _opt(bias),
+                                                         _u32(k), _u32(n), output._h, C.c_float(cap)))
+
     def linear_residual_vector_into(self, batch, input, branch, store, norm_weight, eps, weight, bias, k, segments, outputs,
                                     output_dtype, accumulate=False, position=None):
         _check(self._l.lh_linear_residual_vector_into(batch._h, input._h, branch._h, _opt(store), norm_weight._h, C.c_float(eps),
@@ -954,6 +958,9 @@ class Kernels:
 
     def argmax_rows_f32_into(self, batch, logits, index, rows, n):
         _check(self._l.lh_argmax_rows_f32_into(batch._h, logits._h, index._h, _u32(rows), _u32(n)))
+
+    def argmax_advance_f32_into(self, batch, logits, index, n, position, by):
+        _check(self._l.lh_argmax_advance_f32_into(batch._h, logits._h, index._h, _u32(n), position._h, _u32(by)))
 
 
 from . import synth  # noqa: E402  (synthetic inputs of the measured configurations)

@@ -885,6 +885,7 @@ struct RowWalk {
 __device__ __forceinline__ void store_sums(const LhSegments& seg, const float* bias, const RowWalk& walk, uint32_t i0, uint32_t n, uint32_t lane, float v) {
     const uint32_t row = walk.row(i0 + lane);
     if (bias && lane < n) v += bias[row];
+    if (seg.cap != 0.0f) v = seg.cap * tanhf(v / seg.cap);
     if (walk.pairs) {                                         // n is even, and a pair's factors are in neighbouring lanes
         const float up = lh_dpp_f<LH_DPP_QUAD_XOR1>(v);
         if (lane < n && !(lane & 1)) lh_segment_put(seg, 0, row >> 1, v * lh_sigmoid(v) * up);
@@ -1137,9 +1138,10 @@ int check_common(lh_batch* batch, const lh_buffer* weight, const lh_buffer* bias
 
 int vector_entry(lh_batch* batch, const char* op, int stage, const VectorStage& st, const lh_buffer* weight, const lh_buffer* bias, uint32_t k,
                  uint32_t count, const uint32_t* ns, const uint32_t* acts, const uint32_t* heads, const uint32_t* padded, const uint32_t* layouts,
-                 lh_buffer* const* outputs, int output_dtype, int accumulate, const lh_buffer* position) {
+                 lh_buffer* const* outputs, int output_dtype, int accumulate, const lh_buffer* position, float cap = 0.0f) {
     LhSegments seg;
     LH_TRY(lh_make_segments(seg, op, 1, 0, count, ns, acts, heads, padded, layouts, outputs, output_dtype, accumulate, position));
+    seg.cap = cap;
     LH_REQUIRE(!seg.pairs || seg.count == 1, "%s: pairs beside other segments", op);
     const uint32_t n = seg.n0[seg.count];
     LH_TRY(check_common(batch, weight, bias, k, n, op));
@@ -1320,11 +1322,10 @@ int lh_linear_vector_into(lh_batch* batch, const lh_buffer* input, int input_dty
     return vector_entry(batch, op, kPlain, st, weight, bias, k, count, ns, acts, heads, padded, layouts, outputs, output_dtype, accumulate, position);
 }
 
-int lh_linear_norm_vector_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* add, lh_buffer* store, const lh_buffer* norm_weight, float eps,
-                               const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t count, const uint32_t* ns, const uint32_t* acts,
-                               const uint32_t* heads, const uint32_t* padded, const uint32_t* layouts, lh_buffer* const* outputs, int output_dtype,
-                               int accumulate, const lh_buffer* position) {
-    const char* op = "linear_norm_vector";
+static int norm_vector(lh_batch* batch, const char* op, const lh_buffer* input, const lh_buffer* add, lh_buffer* store, const lh_buffer* norm_weight, float eps,
+                       const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t count, const uint32_t* ns, const uint32_t* acts,
+                       const uint32_t* heads, const uint32_t* padded, const uint32_t* layouts, lh_buffer* const* outputs, int output_dtype,
+                       int accumulate, const lh_buffer* position, float cap) {
     LH_REQUIRE(batch, "%s: batch is null", op);
     LH_NEED(input, (size_t)k * 4, op, "input");
     LH_NEED(norm_weight, (size_t)k * 4, op, "norm_weight");
@@ -1336,7 +1337,23 @@ int lh_linear_norm_vector_into(lh_batch* batch, const lh_buffer* input, const lh
     VectorStage st{};
     st.x = input->ptr; st.x_f32 = 1; st.add = add ? (const float*)add->ptr : nullptr; st.store = store ? (float*)store->ptr : nullptr;
     st.norm_weight = (const float*)norm_weight->ptr; st.eps = eps;
-    return vector_entry(batch, op, kNorm, st, weight, bias, k, count, ns, acts, heads, padded, layouts, outputs, output_dtype, accumulate, position);
+    return vector_entry(batch, op, kNorm, st, weight, bias, k, count, ns, acts, heads, padded, layouts, outputs, output_dtype, accumulate, position, cap);
+}
+
+int lh_linear_norm_vector_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* add, lh_buffer* store, const lh_buffer* norm_weight, float eps,
+                               const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t count, const uint32_t* ns, const uint32_t* acts,
+                               const uint32_t* heads, const uint32_t* padded, const uint32_t* layouts, lh_buffer* const* outputs, int output_dtype,
+                               int accumulate, const lh_buffer* position) {
+    return norm_vector(batch, "linear_norm_vector", input, add, store, norm_weight, eps, weight, bias, k, count, ns, acts, heads, padded, layouts, outputs, output_dtype,
+                       accumulate, position, 0.0f);
+}
+
+int lh_linear_norm_vector_capped_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps, const lh_buffer* weight,
+                                      const lh_buffer* bias, uint32_t k, uint32_t n, lh_buffer* output, float cap) {
+    const char* op = "linear_norm_vector_capped";
+    LH_REQUIRE(cap > 0.0f, "%s: cap %g", op, (double)cap);
+    const uint32_t act = LH_ACT_NONE, layout = LH_ROWS;
+    return norm_vector(batch, op, input, nullptr, nullptr, norm_weight, eps, weight, bias, k, 1, &n, &act, &n, &n, &layout, &output, LH_F32, 0, nullptr, cap);
 }
 
 int lh_linear_residual_vector_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* branch, lh_buffer* store, const lh_buffer* norm_weight,

@@ -61,6 +61,7 @@ struct LhSegments {
     uint32_t aligned4;              // every boundary is a multiple of 4: four neighbouring columns are of one segment
     uint32_t vec4[4];               // and stay together in the destination
     uint32_t pairs;                 // some segment has LH_ACT_SILU_PAIRS
+    float cap;                      // products of one vector, one segment without activation: v becomes cap * tanh(v / cap); 0: not
     const uint32_t* position;       // device word: position of row 0 (layouts AT_POSITION)
 };
 __device__ __forceinline__ bool lh_segment_at_position(const LhSegments& s, uint32_t i) {

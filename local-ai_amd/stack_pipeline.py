@@ -190,8 +190,12 @@ class StackPipeline:
         seq.position += n
 
     def _encode_head(self, batch, row: Buffer) -> None:
-        self.head.normed_vector_into(batch, self.kernels, row, self.final_norm.weight, self.config.eps, [self.logits_buf], F32)
-        self._encode_cap(batch, self.logits_buf, 1)
+        norm, eps, cap = self.final_norm.weight, self.config.eps, self.config.softcap
+        if cap is None:
+            self.head.normed_vector_into(batch, self.kernels, row, norm, eps, [self.logits_buf], F32)
+        else:
+            self.kernels.linear_norm_vector_capped_into(batch, row, norm, eps, self.head.weight, self.head.bias, self.head.k, self.vocab_size,
+                                                        self.logits_buf, cap)
 
     def _encode_cap(self, batch, logits: Buffer, rows: int) -> None:
         if self.config.softcap is not None:
@@ -199,8 +203,7 @@ class StackPipeline:
 
     def _encode_decode(self, batch, seq: SequenceSlot, max_position: int) -> None:
         self._encode_head(batch, self._encode_stack(batch, seq, 1, max_position))
-        self.kernels.argmax_rows_f32_into(batch, self.logits_buf, self.next_buf, 1, self.vocab_size)
-        self.kernels.advance_position_into(batch, seq.position_buf, 1)
+        self.kernels.argmax_advance_f32_into(batch, self.logits_buf, self.next_buf, self.vocab_size, seq.position_buf, 1)
 
     def _decode(self, seq: SequenceSlot, token: int) -> CommandBatch:
         """One token, encoded: logits in logits_buf, the largest one's index in next_buf.  The first decoded token of a slot runs

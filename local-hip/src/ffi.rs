@@ -173,6 +173,7 @@ extern "C" {
     pub fn lh_linear_rows_into(batch: *mut lh_batch, input: *const lh_buffer, input_dtype: c_int, weight: *const lh_buffer, bias: *const lh_buffer, m: u32, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
     pub fn lh_linear_vector_into(batch: *mut lh_batch, input: *const lh_buffer, input_dtype: c_int, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
     pub fn lh_linear_norm_vector_into(batch: *mut lh_batch, input: *const lh_buffer, add: *const lh_buffer, store: *mut lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
+    pub fn lh_linear_norm_vector_capped_into(batch: *mut lh_batch, input: *const lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, n: u32, output: *mut lh_buffer, cap: f32) -> c_int;
     pub fn lh_linear_residual_vector_into(batch: *mut lh_batch, input: *const lh_buffer, branch: *const lh_buffer, store: *mut lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
     pub fn lh_gated_vector_fits(k: u32, group: u32) -> u32;
     pub fn lh_linear_gated_vector_into(batch: *mut lh_batch, input: *const lh_buffer, gate: *const lh_buffer, gate_dtype: c_int, gate_act: u32, gate_first: c_int, norm_weight: *const lh_buffer, group: u32, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
@@ -203,4 +204,5 @@ extern "C" {
     pub fn lh_moe_vector_down_into(batch: *mut lh_batch, hidden: *const lh_buffer, logits: *const lh_buffer, down: *const lh_buffer, residual: *mut lh_buffer, experts: u32, top: u32, width: u32, ff: u32) -> c_int;
     pub fn lh_advance_position_into(batch: *mut lh_batch, position: *mut lh_buffer, by: u32) -> c_int;
     pub fn lh_argmax_rows_f32_into(batch: *mut lh_batch, logits: *const lh_buffer, index: *mut lh_buffer, rows: u32, n: u32) -> c_int;
+    pub fn lh_argmax_advance_f32_into(batch: *mut lh_batch, logits: *const lh_buffer, index: *mut lh_buffer, n: u32, position: *mut lh_buffer, by: u32) -> c_int;
 }

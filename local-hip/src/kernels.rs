@@ -555,6 +555,13 @@ impl Kernels {
         check(unsafe { ffi::lh_linear_norm_vector_into(batch.as_ptr(), input.as_ptr(), add.as_ptr(), store.as_ptr(), norm_weight.as_ptr(), eps, weight.as_ptr(), bias.as_ptr(), k, count, ns.as_ptr(), acts.as_ptr(), heads.as_ptr(), padded.as_ptr(), layouts.as_ptr(), outputs_raw.as_ptr(), output_dtype, accumulate, position.as_ptr()) })
     }
 
+    /// `lh_linear_norm_vector_capped_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn linear_norm_vector_capped_into(&self, batch: &mut CommandBatch, input: &Buffer, norm_weight: &Buffer, eps: f32, weight: &Buffer, bias: &Buffer, k: u32, n: u32, output: &Buffer, cap: f32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_linear_norm_vector_capped_into(batch.as_ptr(), input.as_ptr(), norm_weight.as_ptr(), eps, weight.as_ptr(), bias.as_ptr(), k, n, output.as_ptr(), cap) })
+    }
+
     /// `lh_linear_residual_vector_into` (include/local_hip.h).
     #[allow(clippy::too_many_arguments)]
     pub fn linear_residual_vector_into(&self, batch: &mut CommandBatch, input: &Buffer, branch: &Buffer, store: &Buffer, norm_weight: &Buffer, eps: f32, weight: &Buffer, bias: &Buffer, k: u32, count: u32, ns: &[u32], acts: &[u32], heads: &[u32], padded: &[u32], layouts: &[u32], outputs: &[&Buffer], output_dtype: c_int, accumulate: c_int, position: &Buffer) -> Result<()> {
@@ -699,5 +706,11 @@ impl Kernels {
     pub fn argmax_rows_f32_into(&self, batch: &mut CommandBatch, logits: &Buffer, index: &Buffer, rows: u32, n: u32) -> Result<()> {
         // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
         check(unsafe { ffi::lh_argmax_rows_f32_into(batch.as_ptr(), logits.as_ptr(), index.as_ptr(), rows, n) })
+    }
+
+    /// `lh_argmax_advance_f32_into` (include/local_hip.h).
+    pub fn argmax_advance_f32_into(&self, batch: &mut CommandBatch, logits: &Buffer, index: &Buffer, n: u32, position: &Buffer, by: u32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_argmax_advance_f32_into(batch.as_ptr(), logits.as_ptr(), index.as_ptr(), n, position.as_ptr(), by) })
     }
 }

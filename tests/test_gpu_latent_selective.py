@@ -409,6 +409,36 @@ def test_destinations_of_mixed_types(ai, gpu):
         close(download(ai, b, m * 20, ai.F32).reshape(m, 20), want[:, heads * 12:], F32_TOL)
 
 
+def test_capped_products(ai, gpu):
+    """Sums capped where they are stored are those of the product with a cap behind it: one and several per wave, every form of the product."""
+    ctx, K = gpu
+    for k, n in ((64, 300), (1024, 33000), (2048, 5000), (6000, 70), (20, 9)):
+        g, batch = np.random.default_rng(k), ai.CommandBatch(ctx)
+        x, w, bias = upload(ai, ctx, g.standard_normal(k) * 3, ai.F32), upload(ai, ctx, g.standard_normal((n, k)), ai.BF16), upload(ai, ctx, g.standard_normal(n), ai.F32)
+        norm, a, b = upload(ai, ctx, np.full(k, 0.5), ai.F32), ai.Buffer.empty(ctx, n * 4), ai.Buffer.empty(ctx, n * 4)
+        K.linear_norm_vector_into(batch, x, None, None, norm, 1e-6, w, bias, k, ai.linear_weight.Segments([ai.linear_weight.Segment(n)]), [a], ai.F32)
+        K.softcap_f32_into(batch, a, n, 15.5)
+        K.linear_norm_vector_capped_into(batch, x, norm, 1e-6, w, bias, k, n, b, 15.5)
+        batch.commit_and_wait()
+        print(f"capped product {k} {n}", flush=True)
+        assert (a.as_array(np.float32) == b.as_array(np.float32)).all()
+    with pytest.raises(ai.InvalidArgument):
+        K.linear_norm_vector_capped_into(batch, x, norm, 1e-6, w, bias, k, n, b, 0.0)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 1000, 16384, 16385, 40000])
+def test_argmax_and_position(ai, gpu, n):
+    """The first of several largest values, wherever they lie, and the position moved on behind it."""
+    ctx, K = gpu
+    g, batch = np.random.default_rng(n), ai.CommandBatch(ctx)
+    pos, best = ai.Buffer.from_slice(ctx, np.array([5], np.uint32)), ai.Buffer.empty(ctx, 4)
+    for i in range(6):
+        z = np.round(g.standard_normal(n) * 2).astype(np.float32) if i else np.full(n, -np.inf, np.float32)
+        K.argmax_advance_f32_into(batch, upload(ai, ctx, z, ai.F32), best, n, pos, 3)
+        batch.commit_and_wait()
+        assert best.as_array(np.uint32, 1)[0] == z.argmax() and pos.as_array(np.uint32, 1)[0] == 8 + 3 * i
+
+
 def test_softcap(ai, gpu):
     ctx, K = gpu
     x = np.linspace(-200, 200, 1037).astype(np.float32)
