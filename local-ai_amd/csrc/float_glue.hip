@@ -5,7 +5,7 @@
 
 namespace {
 
-// VEC: rows of whole 16-byte pieces.  (A value at a time: 5.8 us for one row of 2048, 10.8 for 2048 rows; now @E1@ and @E2@.)
+// VEC: rows of whole 16-byte pieces.  (A value at a time: 5.8 us for one row of 2048, 10.8 for 2048 rows; now 2.6 and 7.7.)
 template <bool VEC>
 __global__ __launch_bounds__(256) void embed_rows_kernel(const uint16_t* __restrict__ table, uint32_t table_rows, uint32_t cols,
                                                         const uint32_t* __restrict__ rows, float* __restrict__ out) {
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void softcap_kernel(float* x, size_t n, float 
 __global__ void advance_position_kernel(uint32_t* position, uint32_t by) { *position += by; }
 
 // Index of the largest value of each row; `position`, if there is one, moves on behind it (a launch of its own for that: 2.5 us of a
-// token's chain).  What the threads find meets in one wave, behind one barrier: 5.1 -> @A1@ us for 32000 values with the position's move.
+// token's chain).  What the threads find meets in one wave, behind one barrier: 5.1 us for 32000 values, with the position or without.
 __global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restrict__ x, uint32_t* __restrict__ index, uint32_t n, uint32_t* position, uint32_t by) {
     __shared__ float sv[1024];
     __shared__ uint32_t si[1024];

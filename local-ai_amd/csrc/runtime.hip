@@ -78,19 +78,32 @@ int lh_raise_dynamic_lds(lh_context* ctx, const void* kernel, size_t bytes, cons
     return LH_OK;
 }
 
+#define LH_TRY_STAGE(expr)              \
+    do {                                \
+        const int rs__ = (expr);        \
+        if (rs__ != LH_OK) return rs__; \
+    } while (0)
+
+// Puts up to kDescSlotBytes into the next slot of the pinned staging memory.  Whoever reads the slot on the stream records its event
+// behind that and marks it used.
+static int stage_slot(lh_context* ctx, const void* host, size_t bytes, const char* op, unsigned& slot) {
+    slot = ctx->desc_next++ % lh_context::kDescSlots;
+    if (ctx->desc_used[slot]) {   // what last read this slot must have run (it has, but for a very deep queue)
+        const hipError_t e = hipEventSynchronize(ctx->desc_event[slot]);
+        if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: %s: staging memory: %s", op, hipGetErrorString(e));
+    }
+    memcpy(static_cast<char*>(ctx->desc_pinned) + (size_t)slot * lh_context::kDescSlotBytes, host, bytes);
+    return LH_OK;
+}
+
 int lh_upload_descriptors(lh_context* ctx, const void* host, size_t bytes, void* device_dst, const char* op) {
     if (ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: a descriptor upload cannot be recorded into a graph", op);
     if (bytes == 0) return LH_OK;
     hipError_t e;
     if (bytes <= lh_context::kDescSlotBytes) {
-        const unsigned slot = ctx->desc_next++ % lh_context::kDescSlots;
-        if (ctx->desc_used[slot]) {   // the copy that last read this slot must have run (it has, but for a very deep queue)
-            e = hipEventSynchronize(ctx->desc_event[slot]);
-            if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: %s: descriptor staging: %s", op, hipGetErrorString(e));
-        }
-        void* stage = static_cast<char*>(ctx->desc_pinned) + (size_t)slot * lh_context::kDescSlotBytes;
-        memcpy(stage, host, bytes);
-        e = hipMemcpyAsync(device_dst, stage, bytes, hipMemcpyHostToDevice, ctx->stream);
+        unsigned slot;
+        LH_TRY_STAGE(stage_slot(ctx, host, bytes, op, slot));
+        e = hipMemcpyAsync(device_dst, static_cast<char*>(ctx->desc_pinned) + (size_t)slot * lh_context::kDescSlotBytes, bytes, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipEventRecord(ctx->desc_event[slot], ctx->stream);
         ctx->desc_used[slot] = true;
     } else {   // larger than a slot: wait for the kernels that still read the previous table, then a blocking copy
@@ -462,7 +475,9 @@ int lh_batch_blit_copy(lh_batch* batch, const lh_buffer* src, size_t src_offset,
 }
 
 // A few words (a token, the rows of a portion) as the arguments of a one-workgroup launch: the copy engine with a wait behind it holds a
-// step up for 14 us, this for 4.
+// step up for 14 us, this for 4.  More, such as the tokens of a long portion, through a slot of the pinned staging memory, which a kernel
+// reads: nobody waits for what is on the stream already (8 KB behind the first half of a prompt of 4096: its second half began 60 us after
+// the first had ended).
 int lh_batch_write(lh_batch* batch, lh_buffer* dst, size_t offset, const void* src, size_t len) {
     if (!batch || !dst || (!src && len)) return lh_fail(LH_ERR_INVALID_ARGUMENT, "batch_write: null argument");
     if (batch->ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "batch_write: not while a graph is being captured");
@@ -477,6 +492,22 @@ int lh_batch_write(lh_batch* batch, lh_buffer* dst, size_t offset, const void* s
     };
     if (dst->ctx == batch->ctx && len <= sizeof(SentWords<16>)) return send(SentWords<16>{});
     if (dst->ctx == batch->ctx && len <= sizeof(SentWords<512>)) return send(SentWords<512>{});
+    if (dst->ctx == batch->ctx && len <= lh_context::kDescSlotBytes) {
+        unsigned slot;
+        LH_TRY_STAGE(stage_slot(batch->ctx, src, len, "batch_write", slot));
+        void* from = nullptr;
+        hipError_t e = hipHostGetDevicePointer(&from, static_cast<char*>(batch->ctx->desc_pinned) + (size_t)slot * lh_context::kDescSlotBytes, 0);
+        if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: batch_write: %s", hipGetErrorString(e));
+        if (((uintptr_t)to & 15) == 0)
+            hipLaunchKernelGGL(read_out_kernel, dim3((uint32_t)((len + 4095) / 4096)), dim3(256), 0, batch->ctx->stream, (const uint8_t*)from, (uint8_t*)to, len);
+        else
+            hipLaunchKernelGGL(blit_copy1_kernel, dim3((uint32_t)((len + 1023) / 1024)), dim3(256), 0, batch->ctx->stream, (const uint8_t*)from, (uint8_t*)to, len);
+        LH_TRY_STAGE(lh_check_launch("batch_write"));
+        e = hipEventRecord(batch->ctx->desc_event[slot], batch->ctx->stream);
+        if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: batch_write: %s", hipGetErrorString(e));
+        batch->ctx->desc_used[slot] = true;
+        return LH_OK;
+    }
     hipError_t e = hipMemcpyAsync(to, src, len, hipMemcpyHostToDevice, batch->ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(batch->ctx->stream);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: batch_write: %s", hipGetErrorString(e));

@@ -11,7 +11,7 @@ from typing import Deque, List, Optional, Sequence
 
 import numpy as np
 
-from . import InvalidArgument
+from . import CommandBatch, InvalidArgument
 from .kv_cache import SlotPool
 
 
@@ -145,6 +145,7 @@ class PipelineSequences:
         self.slots.release(seq)
 
     def step(self, seq, tokens, want=()) -> np.ndarray:
+        """Chunks of rows are only encoded: the token behind them, whose results are waited for, is on the same stream."""
         out = np.empty((len(want), self.vocab_size), np.float32)
         last, lo = len(tokens) - 1, 0
         while lo <= last:
@@ -156,7 +157,7 @@ class PipelineSequences:
                 lo += 1
                 continue
             hi = min([p for p in want if p > lo] + [last, lo + seq.max_batch])
-            seq.forward_tokens_batch(list(tokens[lo:hi]), seq.position)
+            seq.forward_tokens_batch(list(tokens[lo:hi]), seq.position, batch=CommandBatch(seq.ctx))
             seq.position += hi - lo
             lo = hi
         return out

@@ -118,7 +118,7 @@ class StackPipeline:
             hi = min(lo + self.max_rows, n)
             at = [i for i, p in enumerate(want) if lo <= p < hi]
             got = out if len(at) == len(want) else np.empty((len(at), self.vocab_size), np.float32)
-            self._forward(seq, tokens[lo:hi], [want[i] - lo for i in at], got)
+            self._forward(seq, tokens[lo:hi], [want[i] - lo for i in at], got, wait=hi == n)
             if at and got is not out:
                 out[at] = got
         return out
@@ -153,15 +153,15 @@ class StackPipeline:
         Norm.flush(r)
         return r.x
 
-    def _forward(self, seq: SequenceSlot, tokens, want, out: np.ndarray) -> None:
-        """Results are read behind the work, in stream order: one wait for both."""
+    def _forward(self, seq: SequenceSlot, tokens, want, out: np.ndarray, wait: bool) -> None:
+        """Results are read behind the work, in stream order: one wait for both, and for all pieces of a step."""
         n = len(tokens)
         if n == 1 and self.observe is None:
             batch = self._decode(seq, int(tokens[0]))
             if want:
                 self.logits_buf.read_into(out[0])
                 out[1:] = out[0]
-            return self._finish(batch, seq, 1)
+            return self._finish(batch, seq, 1, wait)
         K, width = self.kernels, self.config.width
         batch = CommandBatch(self.ctx)
         batch.write(self.tokens_buf, np.asarray(tokens, np.uint32))
@@ -183,10 +183,11 @@ class StackPipeline:
             self._encode_cap(batch, logits, m)
         if want:
             logits.read_into(out)
-        self._finish(batch, seq, n)
+        self._finish(batch, seq, n, wait)
 
-    def _finish(self, batch, seq: SequenceSlot, n: int) -> None:
-        batch.commit_and_wait()
+    def _finish(self, batch, seq: SequenceSlot, n: int, wait: bool = True) -> None:
+        if wait:
+            batch.commit_and_wait()
         seq.position += n
 
     def _encode_head(self, batch, row: Buffer) -> None:

@@ -179,3 +179,28 @@ def test_host_bytes_in_the_order_of_the_batch(pkg, gpu, size, offset):
     batch.end_capture()
     batch.write(a, src, 0)
     batch.commit_and_wait()
+
+
+@pytest.mark.parametrize("size", [4, 64, 68, 2048, 2052, 2050, 8192, 9001, 65536, 65540])
+@pytest.mark.parametrize("offset", [0, 4])
+def test_writes_in_stream_order(pkg, gpu, size, offset):
+    """Host data of every route -- launch arguments, staging memory, a copy -- lands in the order of the dispatches around it, more
+    writes in a row than there are staging slots, and the source may change as soon as the call is back."""
+    ctx, K = gpu
+    g, batch = np.random.default_rng(size + offset), pkg.CommandBatch(ctx)
+    dst, copies = pkg.Buffer.empty(ctx, offset + size + 16), [pkg.Buffer.empty(ctx, size) for _ in range(7)]
+    dst.copy_from_bytes(np.full(offset + size + 16, 7, np.uint8))
+    want = []
+    for c in copies:
+        src = g.integers(0, 256, size, dtype=np.uint8)
+        want.append(src.copy())
+        batch.write(dst, src, offset)
+        src[:] = 0
+        if offset % 16 == 0 or size % 4 == 0:
+            batch.blit_copy(dst, offset, c, 0, size)
+    batch.commit_and_wait()
+    got = dst.as_array(np.uint8)
+    assert (got[:offset] == 7).all() and (got[offset + size:] == 7).all() and np.array_equal(got[offset:offset + size], want[-1])
+    for c, w in zip(copies, want):
+        if offset % 16 == 0 or size % 4 == 0:
+            assert np.array_equal(c.as_array(np.uint8, size), w)
