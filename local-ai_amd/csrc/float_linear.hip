@@ -5,8 +5,8 @@
 //   split_rows_kernel    f32 activations as three bf16 terms, for the three kernels above (the 32-bit runs)
 //   linear_plain_kernel  everything else: f32 FMA on 64 x 64 tiles (ragged K, pieces that are not aligned)
 //   matvec_bf16_kernel   one row, HBM-bound weight streaming, with the norm before the product done while x is staged
-// All end in the same column segments (bias, activation, layout, residual add), and linear_mfma_kernel,
-// linear_sliced_kernel and linear_plain_kernel also run the experts of a mixture on the tiles of a routing plan.
+// All end in the same column segments (bias, activation, layout, residual add), and all but those for one row also run the experts of
+// a mixture on the tiles of a routing plan.
 #include "float_linear.hpp"
 #include <algorithm>
 #include <cstring>
@@ -567,16 +567,17 @@ __global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = wave >> 2;
     const uint32_t wm = kWide ? group : kHalves ? (wave >> 1) & 1 : wave >> 1, wn = kWide ? wave & 3 : wave & 1;
     uint32_t mt, nt;
-    tile_of_block((a.M + BM - 1) / BM, (a.N + BN - 1) / BN, mt, nt);
-    const RowTile rt{mt * BM, min(mt * BM + BM, a.M), 0u};
+    tile_of_block(row_tiles(a, BM), (a.N + BN - 1) / BN, mt, nt);
+    const RowTile rt = row_tile(a, mt, BM);
+    if (rt.begin >= rt.end) return;
     const uint32_t n0 = nt * BN, K = a.K, steps = K / 64, nk = steps * a.parts;
     const char* A = static_cast<const char*>(a.A);
-    const char* W = reinterpret_cast<const char*>(a.W);
+    const char* W = reinterpret_cast<const char*>(a.W + (size_t)rt.expert * a.N * K);
 
     const uint32_t lt = kHalves ? tid & 255 : tid, src = ((lt & 7) ^ ((lt >> 3) & 7)) * 16, src_b = ((lt & 7) ^ dealt_swizzle<4>(lt >> 3)) * 16;
     uint32_t pa[CA], pb[CB];                                   // byte offsets: the host has checked that they fit
 #pragma unroll
-    for (int i = 0; i < CA; i++) pa[i] = min(rt.begin + i * (T / 8) + (lt >> 3), rt.end - 1) * a.lda * 2 + src;
+    for (int i = 0; i < CA; i++) pa[i] = a_row(a, min(rt.begin + i * (T / 8) + (lt >> 3), rt.end - 1)) * a.lda * 2 + src;
 #pragma unroll
     for (int i = 0; i < CB; i++) pb[i] = min(n0 + i * (T / 8) + (lt >> 3), a.N - 1) * K * 2 + src_b;
     uint4* const to = sm + (kHalves ? wave & 3 : wave) * 64;
@@ -1158,7 +1159,11 @@ int vector_entry(lh_batch* batch, const char* op, int stage, const VectorStage& 
 
 }  // namespace
 
-uint32_t lh_expert_tile_rows(uint32_t slots, uint32_t experts) { return slots / (experts ? experts : 1) >= 128 ? 128u : 64u; }
+// Rows of an expert plan's tiles: a kernel takes them in parts, so they are the largest part that can be of use.
+uint32_t lh_expert_tile_rows(uint32_t slots, uint32_t experts) {
+    const uint32_t each = slots / (experts ? experts : 1);
+    return each >= 192 ? 256u : each >= 128 ? 128u : 64u;
+}
 
 // Whether a lane can finish `per_lane` neighbouring columns by itself, and which activations it then meets.
 static int epilogue_of(const LhSegments& seg, uint32_t per_lane) {
@@ -1254,30 +1259,31 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     // Byte offsets of the phased kernels are 32 bits wide.
     const uint64_t a_bytes = (uint64_t)a_rows * a.lda * 2, w_bytes = (uint64_t)a.N * a.K * 2;
     const bool phased = a.K % 64 == 0 && a_bytes < (1ull << 32) && w_bytes < (1ull << 32);
-    if (a.ex.tiles && a.ex.tile_rows == 128 && tiles(128, 128) >= want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
-    if (phased && !a.ex.tiles && 4 * tiles(128, 128) >= 3 * want) {
+    // Of an expert plan about half the experts' last tiles count: the plan has one more for each than can be full.
+    auto filled = [&](uint32_t bm, uint32_t bn) {
+        return a.ex.tiles ? ((uint64_t)a.ex.slots / bm + a.ex.experts / 2 + 1) * ((a.N + bn - 1) / bn) : tiles(bm, bn);
+    };
+    if (phased && a.ex.tile_rows % 128 == 0 && 4 * filled(128, 128) >= 3 * want) {
         // One workgroup fits a CU, so a launch takes whole rounds of them, and the form is the one whose rounds are the shortest.  A
         // round's time in nanoseconds, measured with 64 columns of k per step: 256 x 256 9000 + 1650 per step, 256 x 128 8000 + 800,
         // 128 x 128 7000 + 520.  Before / now, bf16 results: 2048 x 2048 x 8192 85 / 60 us (256 x 256; the matrix cores alone would take
         // 28 at 2.4 GHz; on random data the clock is 1.5 to 1.8 GHz and they are busy for 70 % of the cycles of such launches), 2048 x 2048 x 4096 39 / 34 and 2048 x 2048 x 3072 35 / 28
         // (256 x 128), 2048 x 8192 x 2048 90 / 74 (128 x 128).  With fewer than three tiles of 128 x 128 to four CUs the small tiles
         // win: 128 of them (953 x 2048 x 2048) 22 us against 18.
-        auto rounds = [&](uint32_t bm, uint32_t bn) { return (tiles(bm, bn) + want - 1) / want; };
+        // The experts of a mixture, 4096 slots of 16: from 2048 to 1024 columns 42 -> 39.5 us (256 x 128), back 54 -> 48 (256 x 256; 60 with 256 x 128; both were on 128 x 128 tiles of four
+        // waves, whose last round is short of tiles).
+        auto rounds = [&](uint32_t bm, uint32_t bn) { return a.ex.tiles && a.ex.tile_rows < bm ? 1u << 20 : (filled(bm, bn) + want - 1) / want; };
         const uint64_t t256 = rounds(256, 256) * (9000 + 1650 * steps), t384 = rounds(256, 128) * (8000 + 800 * steps), t128 = rounds(128, 128) * (7000 + 520 * steps);
         if (t256 <= t384 && t256 <= t128) return launch_phased<256, 256>(ctx, a, tiles(256, 256), op);
         if (t384 <= t128) return launch_phased<256, 128>(ctx, a, tiles(256, 128), op);
         return launch_phased<128, 128>(ctx, a, tiles(128, 128), op);
     }
-    if (!a.ex.tiles && tiles(128, 128) >= 2 * want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
+    if (a.ex.tile_rows % 128 == 0 && filled(128, 128) >= 2 * want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
     // The rest by its expected time in nanoseconds, measured: 64 x 64 tiles of shared waves, up to three workgroups a CU; or waves that
-    // share out k, on 64 x 32 tiles (one workgroup a CU) or 32 x 32 (two).  Of an expert plan about half the experts' last tiles count:
-    // the plan has one more for each than can be full.  Before / now, weights in the memory-side cache: 512 x 1024 x 4096 25.5 / 12.5 us
+    // share out k, on 64 x 32 tiles (one workgroup a CU) or 32 x 32 (two).  Before / now, weights in the memory-side cache: 512 x 1024 x 4096 25.5 / 12.5 us
     // and 200 x 2048 x 8192 46.7 / 19.2 (64 x 32), 512 x 1024 x 1024 9.6 / 6.5, 2048 x 16 x 2048 14.0 / 6.0 and 256 x 1024 x 4096 25.2 / 9.4
     // (32 x 32), 953 x 2048 x 2048 21 / 17.9 and 300 x 6144 x 1536 19.5 / 15.3 (64 x 64, from 128 x 64), 333 x 1024 x 1024 with f32
     // activations 20.3 / 9.6.
-    auto filled = [&](uint32_t bm, uint32_t bn) {
-        return a.ex.tiles ? ((uint64_t)a.ex.slots / bm + a.ex.experts / 2 + 1) * ((a.N + bn - 1) / bn) : tiles(bm, bn);
-    };
     const uint64_t n64 = filled(64, 64), n32 = filled(32, 32);
     const uint64_t t64 = n64 <= want ? 4000 + 345 * steps : n64 <= 2 * want ? 4600 + 430 * steps : (n64 + 3 * want - 1) / (3 * want) * (5000 + 600 * steps);
     const uint64_t t64_32 = 1000 + (filled(64, 32) + want - 1) / want * (3500 + 100 * steps);

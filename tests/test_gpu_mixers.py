@@ -614,6 +614,45 @@ def test_linear_attention_chunks(ai, gpu, heads, dim, vdim, rows):
 
 
 # ---- mixture of experts ------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("rows,experts,top,width,ff", [(1000, 5, 1, 2048, 1024), (770, 6, 2, 1024, 2048), (1600, 3, 1, 192, 4096), (400, 2, 1, 2048, 2048)])
+def test_mixture_of_large_experts(ai, gpu, rows, experts, top, width, ff):
+    """Expert plans with tiles of 256 rows through the kernels of large products: ragged last tiles, an expert with a few rows and one
+    with none.  The reference is f32 arithmetic on the CPU."""
+    ctx, K = gpu
+    g = np.random.default_rng(rows + experts)
+    x = M.rounded(g.standard_normal((rows, width))).astype(np.float32)
+    ups, downs = (M.rounded(g.standard_normal(s) / np.sqrt(s[2])).astype(np.float32) for s in ((experts, ff, width), (experts, width, ff)))
+    logits = g.standard_normal((rows, experts)).astype(np.float32)
+    logits[:, 0] = -50.0                              # nobody's first choice but a few rows'
+    logits[:7, 0] = 9.0
+    if top == 1 and experts > 2:
+        logits[:, 1] = -60.0
+    order = np.argsort(-logits, axis=1, kind="stable")[:, :top]
+    hidden_want, want = np.zeros((rows, top, ff), np.float32), np.zeros((rows, width), np.float32)
+    for e in range(experts):
+        t, c = np.nonzero(order == e)
+        h = M.rounded(O.relu_squared(O.sigmoid(logits[t, e].astype(np.float64))[:, None] * (x[t] @ ups[e].T))).astype(np.float32)
+        hidden_want[t, c] = h
+        np.add.at(want, t, h @ downs[e].T)
+    print(f"large experts {rows} {experts} {top} {width} {ff}", flush=True)
+    plan = ai.Buffer.empty(ctx, 4 * K.moe_plan_words(rows, experts, top))
+    up, down = (ai.Buffer.from_slice(ctx, M.bf16_bits(w)) for w in (ups, downs))
+    hidden, slots, rb = empty(ai, ctx, rows * top * ff, ai.BF16), empty(ai, ctx, rows * top * width, ai.F32), upload(ai, ctx, np.zeros((rows, width)), ai.F32)
+    batch = ai.CommandBatch(ctx)
+    K.moe_route_into(batch, ai.Buffer.from_slice(ctx, logits), plan, rows, experts, top)
+    K.moe_up_into(batch, upload(ai, ctx, x, ai.BF16), ai.BF16, plan, up, hidden, rows, experts, top, width, ff, 3)
+    K.moe_down_into(batch, hidden, ai.BF16, plan, down, slots, rb, rows, experts, top, width, ff)
+    batch.commit_and_wait()
+    words = plan.as_array(np.uint32)
+    S = rows * top
+    place = words[2 * S:3 * S].reshape(rows, top)
+    assert np.array_equal(words[:S].reshape(rows, top), order) and sorted(place.ravel()) == list(range(S))
+    by_expert = np.argsort(order.ravel(), kind="stable")
+    assert np.array_equal(place.ravel()[by_expert], np.arange(S))       # experts in order, each one's slots in theirs
+    close(download(ai, hidden, S * ff, ai.BF16).reshape(S, ff)[place.ravel()].reshape(rows, top, ff), hidden_want, BF16_TOL, "hidden")
+    close(download(ai, rb, rows * width, ai.F32).reshape(rows, width), want, BF16_TOL, "sum")
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("rows,experts,top,width,ff", [(2, 5, 2, 64, 48), (7, 3, 3, 40, 33), (65, 11, 1, 64, 88), (300, 4, 2, 64, 72), (600, 2, 1, 32, 40),
                                                        (33, 70, 8, 32, 16), (130, 130, 3, 24, 24), (5, 1, 1, 60, 20), (90, 6, 2, 136, 257),
