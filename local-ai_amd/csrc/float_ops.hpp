@@ -13,7 +13,12 @@ __device__ __forceinline__ float lh_ld(const float* p, size_t i) { return p[i]; 
 __device__ __forceinline__ void lh_st(uint16_t* p, size_t i, float v) { p[i] = lh_f2bf(v); }
 __device__ __forceinline__ void lh_st(float* p, size_t i, float v) { p[i] = v; }
 
-__device__ __forceinline__ uint32_t lh_pack_bf(float a, float b) { return (uint32_t)lh_f2bf(a) | ((uint32_t)lh_f2bf(b) << 16); }
+// One v_cvt_pk_bf16_f32 (from two roundings put together the compiler makes two, a shift and an or).
+__device__ __forceinline__ uint32_t lh_pack_bf(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
 
 // x as the sum of bf16 terms, each the rounding of what the terms before it leave: two carry 16 bits of x, three all 24.
 struct LhSplit3 { uint16_t hi, mid, lo; };

@@ -184,8 +184,11 @@ __global__ __launch_bounds__(256) void latent_split_kernel(const AttentionArgs a
     for (int i = 0; i < NC; i++) {
         const uint32_t c = i * 4 + wave;
         float f[8];
-        if (row < packed && c < DQ / 32) lh_ld8(static_cast<const float*>(a.q) + (size_t)row * DQ + c * 32 + g * 8, f);
-        else
+        if (row < packed && c < DQ / 32) {
+            lh_ld8(static_cast<const float*>(a.q) + (size_t)row * DQ + c * 32 + g * 8, f);
+#pragma unroll
+            for (int j = 0; j < 8; j++) f[j] *= query_sign(a.scale);
+        } else
 #pragma unroll
             for (int j = 0; j < 8; j++) f[j] = 0.0f;
         uint32_t h[4], l[4];
@@ -202,7 +205,7 @@ __global__ __launch_bounds__(256) void latent_split_kernel(const AttentionArgs a
 #pragma unroll
     for (int d = 0; d < ND; d++) o[d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
     RowState st{-INFINITY, 0.0f};
-    const float scale2 = a.scale * kLog2e;
+    const float scale2 = score_scale2(a.scale);
     // score operand: key lc (+ 16), chunk 4 c + g; value operand: key 4 g + lc / 4 (+ 16), columns 16 d + 4 (lane & 3) ..
     const uint4* kp = sm + (lc >> 3) * (KT * 64) + (lc & 7) * 8;
     const uint32_t vk = g * 4 + (lc >> 2);

@@ -34,6 +34,10 @@ __device__ __forceinline__ void load_queries(lh_bf16x8 (&qf)[MAPS][DQ / 32], con
             u32x4 v = {0u, 0u, 0u, 0u};
             if (on && k < a.dim) {
                 v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.q) + (((size_t)t * a.heads + h) * MAPS + mp) * DQ + k);
+                if (!(a.scale > 0.0f)) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] = a.scale < 0.0f ? v[j] ^ 0x80008000u : 0u;      // (no number: scale2 is none either)
+                }
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     if (k + 2 * j >= a.dim) v[j] = 0u;
@@ -86,22 +90,31 @@ typedef __attribute__((address_space(1))) const void gvoid;
 typedef __attribute__((address_space(3))) void lvoid;
 
 // 64 packed rows, 16 per wave; steps of 32 * NB keys through two LDS buffers.  A key row of the buffer is MAPS * DQ / 8 chunks
-// of 16 bytes, chunk c at place c ^ (key & 7) (see linear_mfma_kernel for why and how).  With more than one split a
-// workgroup takes its share of the key steps and leaves partial records.
-template <int DQ, int DV, int MAPS, int NB>
-__global__ __launch_bounds__(256, MAPS * DV <= 256 ? 2 : 1) void attention_tile_kernel(const AttentionArgs a) {
-    constexpr int KC = MAPS * DQ / 8, KCH = 32 * NB * KC, VB = DV * 4, VCH = NB * VB;    // chunks per key row; per step: keys, values
+// of 16 bytes, chunk c at place c ^ (key & 7) (see linear_mfma_kernel for why and how); a column of a value block is four chunks, placed
+// so that any eight or sixteen neighbouring columns read different banks.  With more than one split a workgroup takes its share of the key
+// steps and leaves partial records.
+// What binds is vector and matrix instructions at the clock that they leave (a step of 64 keys of two maps: 3600 cycles of matrix
+// instructions per SIMD and about 3000 of vector instructions, before two values were rounded and reduced by one instruction each 5000:
+// 2048 rows of 16 heads, two maps, at position 0 104 -> 95 us, at 2048 252 -> 216).  With one map the two blocks of a step belong to two groups of four
+// waves, whose sums meet at the end: 2048 rows of 16 heads of 192 and 128 columns 75 -> 66 us.  With two maps the registers do not suffice for that.
+__device__ __forceinline__ uint32_t value_place(uint32_t col) { return ((col >> 2) & 1) * 2 + (((col >> 1) ^ (col >> 3)) & 1); }
+template <int DQ, int DV, int MAPS, int NB, int G>
+__global__ __launch_bounds__(256 * G, G == 2 ? 4 : MAPS * DV <= 256 ? 2 : 1) void attention_tile_kernel(const AttentionArgs a) {
+    constexpr int KC = MAPS * DQ / 8, KCH = 32 * NB * KC, VB = DV * 4, VCH = NB * VB, T = 256 * G, NW = NB / G;   // chunks per key row; per step: keys, values
     constexpr uint32_t kSwizzle = KC >= 8 ? 7 : KC - 1;
     __shared__ uint4 sm[2][KCH + VCH];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = wave >> 2;
     const uint32_t R = a.heads / a.kv_heads, packed = a.rows * R, tiles = (packed + 63) / 64;
-    const uint32_t split = blockIdx.x % a.splits, gt = blockIdx.x / a.splits;
-    const uint32_t g = gt % a.kv_heads, tile = tiles - 1 - gt / a.kv_heads;              // the long tiles first
+    // The long tiles first; where all workgroups are on the chip at once, two a CU, the second of a CU has as much less to do as the first
+    // has more.
+    const uint32_t order = blockIdx.x < a.resident || gridDim.x > 2 * a.resident ? blockIdx.x : gridDim.x - 1 - (blockIdx.x - a.resident);
+    const uint32_t split = order % a.splits, gt = order / a.splits;
+    const uint32_t g = gt % a.kv_heads, tile = tiles - 1 - gt / a.kv_heads;
     const uint32_t start = *a.position;
     const uint32_t row0 = tile * 64, row_last = min(row0 + 64, packed) - 1;
     const uint32_t last_key = min(start + row_last / R, a.capacity - 1), last_block = last_key / 32, nstep = last_block / NB + 1;
     const uint32_t per = (nstep + a.splits - 1) / a.splits, s0 = min(split * per, nstep), s1 = min(s0 + per, nstep);
-    const uint32_t wrow = row0 + wave * 16, row = wrow + (lane & 15);
+    const uint32_t wrow = row0 + (wave & 3) * 16, row = wrow + (lane & 15);
 
     lh_bf16x8 qf[MAPS][DQ / 32];
     load_queries<DQ, MAPS>(qf, a, g, row, lane);
@@ -120,36 +133,37 @@ __global__ __launch_bounds__(256, MAPS * DV <= 256 ? 2 : 1) void attention_tile_
     const size_t krow = (size_t)a.kv_heads * MAPS * DQ, vblock = (size_t)a.kv_heads * DV * 32;
     auto load_step = [&](int buf, uint32_t s) {
 #pragma unroll
-        for (int i = 0; i < (KCH + 255) / 256; i++) {
-            if (KCH % 256 != 0 && i * 256 + wave * 64 >= KCH) break;                     // whole waves (KCH is a multiple of 64)
-            const uint32_t c = i * 256 + tid, key = c / KC, ch = (c % KC) ^ (key & kSwizzle);
+        for (int i = 0; i < (KCH + T - 1) / T; i++) {
+            if (KCH % T != 0 && i * T + wave * 64 >= KCH) break;                          // whole waves (KCH is a multiple of 64)
+            const uint32_t c = i * T + tid, key = c / KC, ch = (c % KC) ^ (key & kSwizzle);
             const uint32_t p = min(s * (32 * NB) + key, last_key);                        // keys past the last are masked
-            __builtin_amdgcn_global_load_lds((gvoid*)(K + p * krow + ch * 8), (lvoid*)&sm[buf][i * 256 + wave * 64], 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gvoid*)(K + p * krow + ch * 8), (lvoid*)&sm[buf][i * T + wave * 64], 16, 0, 0);
         }
 #pragma unroll
-        for (int i = 0; i < (VCH + 255) / 256; i++) {
-            if (VCH % 256 != 0 && i * 256 + wave * 64 >= VCH) break;
-            const uint32_t c = i * 256 + tid;
-            __builtin_amdgcn_global_load_lds((gvoid*)(V + min(s * NB + c / VB, last_block) * vblock + (c % VB) * 8), (lvoid*)&sm[buf][KCH + i * 256 + wave * 64], 16, 0, 0);
+        for (int i = 0; i < (VCH + T - 1) / T; i++) {
+            if (VCH % T != 0 && i * T + wave * 64 >= VCH) break;
+            const uint32_t c = i * T + tid, e = c % VB, ch = (e & ~3u) | ((e & 3) ^ value_place(e >> 2));
+            __builtin_amdgcn_global_load_lds((gvoid*)(V + min(s * NB + c / VB, last_block) * vblock + ch * 8), (lvoid*)&sm[buf][KCH + i * T + wave * 64], 16, 0, 0);
         }
     };
-    const float scale2 = a.scale * kLog2e;
+    const float scale2 = score_scale2(a.scale);
+    const uint32_t vplace = (lane & 15) * 4 + ((lane >> 4) ^ value_place(lane & 15));
     if (s0 < s1) load_step(s0 & 1, s0);
     for (uint32_t s = s0; s < s1; s++) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (s + 1 < s1) load_step((s + 1) & 1, s + 1);
-        const uint32_t first = s * (32 * NB);
+        const uint32_t first = (s * NB + group * NW) * 32;
         if (first > wave_last) continue;                                                  // nothing here is visible to this wave
-        const uint4* ks = sm[s & 1];
-        const uint4* vs = ks + KCH;
-        const bool bound = first + 32 * NB - 1 > first_limit;
+        const uint4* ks = sm[s & 1] + group * (NW * 32 * KC);
+        const uint4* vs = sm[s & 1] + KCH + group * (NW * VB) + vplace;
+        const bool bound = first + 32 * NW - 1 > first_limit;
 #pragma unroll
         for (int mp = 0; mp < MAPS; mp++) {                                               // (a map at a time: the registers of two halve the waves)
-            lh_bf16x8 w[NB][3];
-            lh_f32x4 sc[2 * NB];
+            lh_bf16x8 w[NW][3];
+            lh_f32x4 sc[2 * NW];
 #pragma unroll
-            for (int t = 0; t < 2 * NB; t++) {
+            for (int t = 0; t < 2 * NW; t++) {
                 sc[t] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
                 const uint32_t key = t * 16 + (lane & 15);
 #pragma unroll
@@ -158,7 +172,7 @@ __global__ __launch_bounds__(256, MAPS * DV <= 256 ? 2 : 1) void attention_tile_
                     sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lh_bf16x8, ks[key * KC + (ch ^ (key & kSwizzle))]), qf[mp][c], sc[t], 0, 0, 0);
                 }
             }
-            const float alpha = softmax_step<NB>(sc, st[mp], scale2, first, limit, bound, lane, w);
+            const float alpha = softmax_step<NW>(sc, st[mp], scale2, first, limit, bound, lane, w);
             if (__ballot(alpha != 1.0f)) {
 #pragma unroll
                 for (int d = 0; d < DV / 16; d++)
@@ -166,10 +180,10 @@ __global__ __launch_bounds__(256, MAPS * DV <= 256 ? 2 : 1) void attention_tile_
                     for (int r = 0; r < 4; r++) o[mp][d][r] *= alpha;
             }
 #pragma unroll
-            for (int b = 0; b < NB; b++)
+            for (int b = 0; b < NW; b++)
 #pragma unroll
                 for (int d = 0; d < DV / 16; d++) {
-                    const lh_bf16x8 vf = __builtin_bit_cast(lh_bf16x8, vs[b * VB + (d * 16 + (lane & 15)) * 4 + (lane >> 4)]);
+                    const lh_bf16x8 vf = __builtin_bit_cast(lh_bf16x8, vs[b * VB + d * 64]);
 #pragma unroll
                     for (int z = 2; z >= 0; z--) o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, w[b][z], o[mp][d], 0, 0, 0);
                 }
@@ -178,6 +192,34 @@ __global__ __launch_bounds__(256, MAPS * DV <= 256 ? 2 : 1) void attention_tile_
     float l[MAPS];
 #pragma unroll
     for (int mp = 0; mp < MAPS; mp++) l[mp] = lh_column_sum(st[mp].l);
+    if constexpr (G == 2) {                                   // a map at a time through LDS
+        static_assert(sizeof(sm) >= 4 * 64 * (DV / 16 * 16 + 8), "the sums of a group must fit the buffers");
+        lh_f32x4* const sums = reinterpret_cast<lh_f32x4*>(&sm[0][0]) + (wave & 3) * (DV / 16) * 64 + lane;
+        float2* const state = reinterpret_cast<float2*>(reinterpret_cast<lh_f32x4*>(&sm[0][0]) + 4 * (DV / 16) * 64) + (wave & 3) * 64 + lane;
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            __syncthreads();
+            if (group) {
+#pragma unroll
+                for (int d = 0; d < DV / 16; d++) sums[d * 64] = o[mp][d];
+                *state = make_float2(st[mp].m, l[mp]);
+            }
+            __syncthreads();
+            if (group) continue;
+            const float2 other = *state;
+            const float m = fmaxf(st[mp].m, other.x), base = m == -INFINITY ? 0.0f : m;
+            const float f0 = __builtin_amdgcn_exp2f(st[mp].m - base), f1 = __builtin_amdgcn_exp2f(other.x - base);
+#pragma unroll
+            for (int d = 0; d < DV / 16; d++) {
+                const lh_f32x4 y = sums[d * 64];
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[mp][d][r] = __builtin_fmaf(f1, y[r], f0 * o[mp][d][r]);
+            }
+            l[mp] = __builtin_fmaf(f1, other.y, f0 * l[mp]);
+            st[mp].m = m;
+        }
+        if (group) return;
+    }
     if (a.splits == 1) { finish_row<DV, MAPS>(a, o, l, st[0].m, g, row, lane); return; }
     if (row >= packed) return;
     constexpr uint32_t kRow = DV + 4;
@@ -230,7 +272,7 @@ __global__ __launch_bounds__(256) void attention_split_kernel(const AttentionArg
 #pragma unroll
         for (int d = 0; d < DV / 16; d++) f.v[d] = *reinterpret_cast<const u32x4*>(V + b * vblock + ((d * 16 + (lane & 15)) * 4 + (lane >> 4)) * 8);
     };
-    const float scale2 = a.scale * kLog2e;
+    const float scale2 = score_scale2(a.scale);
     auto consume = [&](const Block& f, uint32_t b) {
         const bool bound = b * 32 + 31 > first_limit;
         lh_bf16x8 w[MAPS][1][3];
@@ -323,12 +365,15 @@ int launch_mfma(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const 
     a.partial = (float*)ctx->workspace;
     launches = 1;
     if (packed > 64) {
-        constexpr int NB = MAPS * DQ + DV <= (MAPS == 1 ? 320 : 256) ? 2 : 1;
+        constexpr int NB = MAPS * DQ + DV <= (MAPS == 1 ? 320 : 256) ? 2 : 1, G = MAPS == 1 ? NB : 1;
         const uint64_t groups = (packed + 63) / 64 * a.kv_heads;
-        // a share of eight key steps at least, and no more workgroups than two per CU
-        a.splits = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({2 * cus / groups, max_blocks / (8 * NB), room}));
+        // Shares of four key steps at least up to a workgroup per CU, of eight up to two.  512 rows of 8 heads, two maps, with the merge: at
+        // position 0 25 us in whole rows and 20 in two shares, at 1024 31 in three, 32 in six (a workgroup and a half per CU) and 30 in four.
+        a.splits = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(std::max(std::min<uint64_t>(cus / groups, max_blocks / (4 * NB)),
+                                                                               std::min<uint64_t>(2 * cus / groups, max_blocks / (8 * NB))), room));
         LH_REQUIRE(groups * a.splits < 0x7FFFFFFFull, "%s: %u rows", op, a.rows);
-        hipLaunchKernelGGL((attention_tile_kernel<DQ, DV, MAPS, NB>), dim3((uint32_t)(groups * a.splits)), dim3(256), 0, ctx->stream, a);
+        a.resident = (uint32_t)cus;
+        hipLaunchKernelGGL((attention_tile_kernel<DQ, DV, MAPS, NB, G>), dim3((uint32_t)(groups * a.splits)), dim3(256 * G), 0, ctx->stream, a);
         const int r = lh_check_launch(op);
         return r != LH_OK || a.splits == 1 ? r : merge();
     }

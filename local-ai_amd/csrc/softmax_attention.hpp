@@ -21,6 +21,7 @@ struct AttentionArgs {
     float* partial;            // records [16-row tile][kv head][split][map][16] of dv unnormalised sums, maximum, sum of weights
     uint32_t splits;
     uint32_t parts;            // workgroups that share a row's columns in the merge (one map)
+    uint32_t resident;         // tiles: workgroups of a launch before any CU has two
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -30,8 +31,27 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // A row tile's running softmax state for one map; every lane holds the values of packed row (lane & 15).
 struct RowState { float m, l; };
 
+// What is left of a value when its bf16 rounding, one half of `pair`, is taken off (exact).  One instruction instead of two.  The factors
+// (-1, 0) are kept in a register: as a constant in the instruction the compiler writes -1.0, which the hardware reads as (0, -1).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float minus_low(float x, uint32_t pair) {
+    uint32_t factors;
+    asm("s_mov_b32 %0, 0xbf80" : "=s"(factors));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, factors), x, false);
+}
+__device__ __forceinline__ float minus_high(float x, uint32_t pair) {
+    uint32_t factors;
+    asm("s_mov_b32 %0, 0xbf800000" : "=s"(factors));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, factors), x, false);
+}
+
+// The running maximum is taken of the products and scaled then, which wants a scale above zero: the sign of another, or that it is zero,
+// goes into the queries.
+__device__ __forceinline__ float score_scale2(float scale) { return scale == 0.0f ? 1.0f : fabsf(scale) * kLog2e; }
+__device__ __forceinline__ float query_sign(float scale) { return scale > 0.0f ? 1.0f : scale < 0.0f ? -1.0f : scale == 0.0f ? 0.0f : scale; }
+
 // Scores of NB steps of 32 keys -> weights in P V operand order, as three bf16 terms; returns the factor for what was summed
-// before.  `first` is the first key, `limit` the row's last visible key, `bound` whether any lane may have to mask.
+// before.  `first` is the first key, `limit` the row's last visible key, `bound` whether any lane may have to mask; scale2 > 0.
 template <int NB>
 __device__ __forceinline__ float softmax_step(lh_f32x4 (&s)[2 * NB], RowState& st, float scale2, uint32_t first, uint32_t limit, bool bound, uint32_t lane,
                                               lh_bf16x8 (&w)[NB][3]) {
@@ -39,11 +59,11 @@ __device__ __forceinline__ float softmax_step(lh_f32x4 (&s)[2 * NB], RowState& s
     const uint32_t g = lane >> 4;
 #pragma unroll
     for (int i = 0; i < 8 * NB; i++) {
-        v[i] = s[i >> 2][i & 3] * scale2;
+        v[i] = s[i >> 2][i & 3];
         if (bound && first + (i >> 2) * 16 + g * 4 + (i & 3) > limit) v[i] = -INFINITY;
         mx = fmaxf(mx, v[i]);
     }
-    const float nm = fmaxf(st.m, lh_column_max(mx)), base = nm == -INFINITY ? 0.0f : nm;
+    const float nm = fmaxf(st.m, lh_column_max(mx) * scale2), base = nm == -INFINITY ? 0.0f : nm;
     const float alpha = __builtin_amdgcn_exp2f(st.m - base);
     float sum = 0.0f;
 #pragma unroll
@@ -51,12 +71,12 @@ __device__ __forceinline__ float softmax_step(lh_f32x4 (&s)[2 * NB], RowState& s
         uint32_t h[4], m[4], l[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            float p0 = __builtin_amdgcn_exp2f(v[8 * b + 2 * i] - base), p1 = __builtin_amdgcn_exp2f(v[8 * b + 2 * i + 1] - base);
+            float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(v[8 * b + 2 * i], scale2, -base)), p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(v[8 * b + 2 * i + 1], scale2, -base));
             sum += p0 + p1;
             h[i] = lh_pack_bf(p0, p1);
-            p0 -= __builtin_bit_cast(float, h[i] << 16); p1 -= __builtin_bit_cast(float, h[i] & 0xFFFF0000u);
+            p0 = minus_low(p0, h[i]); p1 = minus_high(p1, h[i]);
             m[i] = lh_pack_bf(p0, p1);
-            l[i] = lh_pack_bf(p0 - __builtin_bit_cast(float, m[i] << 16), p1 - __builtin_bit_cast(float, m[i] & 0xFFFF0000u));
+            l[i] = lh_pack_bf(minus_low(p0, m[i]), minus_high(p1, m[i]));
         }
         w[b][0] = __builtin_bit_cast(lh_bf16x8, (u32x4){h[0], h[1], h[2], h[3]});
         w[b][1] = __builtin_bit_cast(lh_bf16x8, (u32x4){m[0], m[1], m[2], m[3]});
@@ -146,8 +166,75 @@ __global__ __launch_bounds__(kMergeThreads) void attention_merge_kernel(const At
     if (threadIdx.x < cols && d < a.vdim) static_cast<uint16_t*>(a.out)[((size_t)t * a.heads + h) * a.vdim + d] = lh_f2bf(v * f);
 }
 
+// A few splits of many (query row, head) pairs: dv / 4 lanes take a pair, four columns each, and request all their records at once; no
+// workgroup waits for itself.  (A workgroup per pair: 46 us for 953 rows of 16 heads and two splits, now 6; 12 for 512 rows of 8 heads, two
+// maps and three splits, now 4.5.)
+constexpr uint32_t kFewSplits = 8;
+template <int MAPS>
+__global__ __launch_bounds__(256) void attention_merge_few_kernel(const AttentionArgs a) {
+    const uint32_t lanes = a.dv / 4, item = blockIdx.x * (256 / lanes) + threadIdx.x / lanes, col = threadIdx.x % lanes * 4;
+    const bool on = item < a.rows * a.heads;
+    const uint32_t th = on ? item : 0u, t = th / a.heads, h = th % a.heads;
+    const uint32_t R = a.heads / a.kv_heads, g = h / R, row = t * R + h % R, kRow = a.dv + 4;
+    const size_t stride = (size_t)MAPS * 16 * kRow;
+    const float* rec = a.partial + (size_t)(((row >> 4) * a.kv_heads + g) * a.splits) * stride + (row & 15) * kRow;
+    float2 st[MAPS][kFewSplits];
+    float4 x[MAPS][kFewSplits];
+#pragma unroll
+    for (uint32_t s = 0; s < kFewSplits; s++) {
+        if (s >= a.splits) break;
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            st[mp][s] = *reinterpret_cast<const float2*>(rec + s * stride + mp * 16 * kRow + a.dv);
+            x[mp][s] = *reinterpret_cast<const float4*>(rec + s * stride + mp * 16 * kRow + col);
+        }
+    }
+    const float sink = a.sink ? a.sink[h] * kLog2e : -INFINITY;
+    float v[MAPS][4];
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++) {
+        float m = sink;
+#pragma unroll
+        for (uint32_t s = 0; s < kFewSplits; s++) if (s < a.splits) m = fmaxf(m, st[mp][s].x);
+        float l = 0.0f;
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (uint32_t s = 0; s < kFewSplits; s++) {
+            if (s >= a.splits) break;
+            const float f = __builtin_amdgcn_exp2f(st[mp][s].x - m);
+            l += f * st[mp][s].y;
+            acc.x += f * x[mp][s].x; acc.y += f * x[mp][s].y; acc.z += f * x[mp][s].z; acc.w += f * x[mp][s].w;
+        }
+        const float inv = 1.0f / (l + __builtin_amdgcn_exp2f(sink - m));
+        v[mp][0] = acc.x * inv; v[mp][1] = acc.y * inv; v[mp][2] = acc.z * inv; v[mp][3] = acc.w * inv;
+    }
+    float ss = 0.0f, f = 1.0f;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+        if constexpr (MAPS == 2) v[0][j] -= a.lambda * v[MAPS - 1][j];
+        if (col + j < a.vdim) ss += v[0][j] * v[0][j];
+    }
+    if constexpr (MAPS == 2) f = rsqrtf(lh_group_sum(ss, (int)lanes) / (float)a.vdim + a.eps) * a.out_scale;
+    if (MAPS == 1 && a.gate) f = lh_sigmoid(a.gate[th]);
+    if (!on) return;
+    uint16_t* out = static_cast<uint16_t*>(a.out) + (size_t)th * a.vdim + col;
+    if ((a.vdim & 3) == 0) {
+        if (col < a.vdim) *reinterpret_cast<uint2*>(out) = make_uint2(lh_pack_bf(v[0][0] * f, v[0][1] * f), lh_pack_bf(v[0][2] * f, v[0][3] * f));
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) if (col + j < a.vdim) out[j] = lh_f2bf(v[0][j] * f);
+    }
+}
+
 template <int MAPS>
 int launch_merge(lh_context* ctx, AttentionArgs& a, const char* op) {
+    const uint64_t pairs = (uint64_t)a.rows * a.heads;
+    // a lane group per pair where the pairs fill the chip and the lanes of one are a power of two
+    if (a.splits <= kFewSplits && a.dv <= 256 && (a.dv & (a.dv - 1)) == 0 && pairs >= 4 * (uint64_t)ctx->cu_count && ((uintptr_t)a.out & 7) == 0) {
+        const uint32_t per = 256 / (a.dv / 4);
+        hipLaunchKernelGGL((attention_merge_few_kernel<MAPS>), dim3((uint32_t)((pairs + per - 1) / per)), dim3(256), 0, ctx->stream, a);
+        return lh_check_launch(op);
+    }
     a.parts = 1;                                              // two maps: the norm needs all columns
     if (MAPS == 1) while (a.dv / a.parts > 64 && (uint64_t)a.rows * a.heads * a.parts * 2 <= (uint64_t)ctx->cu_count) a.parts *= 2;
     hipLaunchKernelGGL((attention_merge_kernel<MAPS>), dim3(a.rows * a.heads * a.parts), dim3(kMergeThreads), 0, ctx->stream, a);

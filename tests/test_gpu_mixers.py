@@ -517,6 +517,14 @@ def test_attention_long_context_splits(ai, gpu):
         attention_case(ai, gpu, "bf16", 2, 2, 1, 32, 32, 9000, rows, 9056, spike=(0, 37))
 
 
+@pytest.mark.parametrize("maps", [1, 2])
+@pytest.mark.parametrize("dim,vdim,heads,start,rows", [(32, 32, 4, 1023, 300), (64, 33, 4, 1500, 260), (20, 128, 8, 700, 129), (128, 250, 4, 1023, 257),
+                                                       (32, 64, 16, 0, 1300), (64, 128, 16, 40, 700)])
+def test_attention_of_many_rows(ai, gpu, maps, dim, vdim, heads, start, rows):
+    """A few splits of many rows, and launches whose workgroups are all on the chip at once, two a CU."""
+    attention_case(ai, gpu, "bf16", maps, heads, 2 if heads < 16 else 4, dim, vdim, start, rows, (start + rows + 31) // 32 * 32)
+
+
 def test_attention_rejects(ai, gpu):
     ctx, K = gpu
     b, batch = ai.Buffer.empty(ctx, 1 << 16), ai.CommandBatch(ctx)
