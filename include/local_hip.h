@@ -272,6 +272,10 @@ LH_API int lh_matmul_nt_quant_gelu_mul_strided_into(lh_batch* batch, lh_quant fm
                                                     const lh_buffer* weight, uint32_t m, uint32_t k, uint32_t n,
                                                     const lh_buffer* gate_rows, uint32_t row_stride,
                                                     uint32_t row_offset, lh_buffer* output);
+/* matmul_nt_quant_typed_into with f32 results and logit_softcap_gpu_into of all of them (pipeline/batched.rs:411-455) */
+LH_API int lh_matmul_nt_quant_capped_into(lh_batch* batch, lh_quant fmt, const lh_buffer* input, lh_dtype input_dtype,
+                                          const lh_buffer* weight, lh_buffer* output, uint32_t m, uint32_t k, uint32_t n,
+                                          float cap);
 /* A product followed by the row-wise norm that consumes it, as one encoded step: out = rms_norm(in[m, k] . w^T,
  * norm_weight) (+ residual) (* scale), and with norm2_weight also out2 = rms_norm(out, norm2_weight).  This is the
  * sequence matmul_nt_into -> rms_norm_add_into (-> scale_in_place_gpu_into) (-> rms_norm_into) of the multi-row layer
@@ -333,6 +337,11 @@ LH_API int lh_rms_norm_add_into(lh_batch* batch, const lh_buffer* input, const l
 LH_API int lh_rms_norm_residual_scale_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* weight,
                                            const lh_buffer* residual, lh_buffer* output, uint32_t dim, uint32_t rows,
                                            float eps, int apply_scale, float scale);
+/* the same with scale_in_place of the input by `before` ahead of it, each step with the rounding of its own kernel: the tail
+ * of the per-layer inputs (pipeline.rs:745-776) */
+LH_API int lh_scale_rms_norm_residual_scale_into(lh_batch* batch, float before, const lh_buffer* input,
+                                                 const lh_buffer* weight, const lh_buffer* residual, lh_buffer* output,
+                                                 uint32_t dim, uint32_t rows, float eps, float scale);
 /* kernels.rs:2215-2280 qk_norm_gpu_into / qk_norm_offset_into (shaders/qk_norm.metal:6-56): per-head RMSNorm in place;
  * weight_offset in bytes into the weight buffer */
 LH_API int lh_qk_norm_gpu_into(lh_batch* batch, lh_buffer* qk_data, const lh_buffer* weight, uint32_t head_dim,
@@ -389,6 +398,9 @@ LH_API int lh_dequant_q4_0_into(lh_batch* batch, const lh_buffer* data, size_t b
                                 size_t num_elements);
 LH_API int lh_dequant_tq2_0_into(lh_batch* batch, const lh_buffer* data, size_t byte_offset, lh_buffer* output,
                                  size_t num_elements);
+/* dequant_{q4_0,tq2_0}_into and scale_in_place of the result by `scale` */
+LH_API int lh_dequant_scaled_into(lh_batch* batch, lh_quant fmt, const lh_buffer* data, size_t byte_offset, lh_buffer* output,
+                                  size_t num_elements, float scale);
 /* Rows `rows[0 .. n_rows)` (a device u32 list; an index past the end reads the last row, init_gemma4_qat.rs:152)
  * of a packed [table_rows, cols] table decoded to a dense f16 [n_rows, cols] matrix in one dispatch: the embedding
  * gather of local-engine/src/pipeline.rs:781-832 (gather_embeddings, which decodes on the CPU one row at a time)

@@ -453,6 +453,11 @@ class Kernels:
                                                      weight._h, output._h, C.c_int(output_dtype), _u32(m), _u32(k),
                                                      _u32(n)))
 
+    def matmul_nt_quant_capped_into(self, batch, fmt, input, input_dtype, weight, output, m, k, n, cap):
+        """matmul_nt_quant_typed_into with f32 output and logit_softcap_gpu_into of it."""
+        _check(self._l.lh_matmul_nt_quant_capped_into(batch._h, C.c_int(fmt), input._h, C.c_int(input_dtype), weight._h, output._h,
+                                                      _u32(m), _u32(k), _u32(n), C.c_float(cap)))
+
     def matmul_nt_quant_grouped_into(self, batch, fmt, input, weights, outputs, m, k, ns):
         """Up to four matrices of one format against the same activations in one launch; output i is [m, ns[i]] f16."""
         n = len(weights)
@@ -526,6 +531,11 @@ class Kernels:
         _check(self._l.lh_rms_norm_add_into(batch._h, input._h, weight._h, residual._h, output._h, _u32(dim), _u32(rows),
                                             C.c_float(eps)))
 
+    def scale_rms_norm_residual_scale_into(self, batch, before, input, weight, residual, output, dim, rows, eps, scale):
+        """scale_in_place_gpu_into of the input, rms_norm_into, residual_add_into and scale_in_place_gpu_into in one dispatch."""
+        _check(self._l.lh_scale_rms_norm_residual_scale_into(batch._h, C.c_float(before), input._h, weight._h, residual._h, output._h,
+                                                             _u32(dim), _u32(rows), C.c_float(eps), C.c_float(scale)))
+
     def rms_norm_residual_scale_into(self, batch, input, weight, residual, output, dim, rows, eps, scale=None):
         """rms_norm_into + residual_add_into (+ scale_in_place_gpu_into when `scale` is given) in one dispatch, with the
         f16 rounding after each step that the separate kernels apply."""
@@ -590,6 +600,11 @@ class Kernels:
     def dequant_tq2_0_into(self, batch, data, byte_offset, output, num_elements):
         _check(self._l.lh_dequant_tq2_0_into(batch._h, data._h, C.c_size_t(byte_offset), output._h,
                                              C.c_size_t(num_elements)))
+
+    def dequant_scaled_into(self, batch, fmt, data, byte_offset, output, num_elements, scale):
+        """dequant_{q4_0,tq2_0}_into and scale_in_place_gpu_into of the result in one dispatch."""
+        _check(self._l.lh_dequant_scaled_into(batch._h, C.c_int(fmt), data._h, C.c_size_t(byte_offset), output._h,
+                                              C.c_size_t(num_elements), C.c_float(scale)))
 
     def dequant_rows_into(self, batch, fmt, table, table_rows, cols, rows, n_rows, output, scale=1.0):
         """Rows `rows[0 .. n_rows)` (device u32 indices, clamped to the last row) of a packed table as a dense f16

@@ -9,7 +9,10 @@
 
 namespace {
 
-__global__ __launch_bounds__(256) void dequant_q4_0_kernel(const uint8_t* __restrict__ data, uint16_t* __restrict__ out, size_t n) {
+// With scale != 1 a decoded value is multiplied and rounded once more, which is what scale_in_place.metal:5-14 would do to it.
+__device__ __forceinline__ uint16_t scaled(uint16_t h, float scale) { return scale != 1.0f ? lh_f2h(lh_h2f(h) * scale) : h; }
+
+__global__ __launch_bounds__(256) void dequant_q4_0_kernel(const uint8_t* __restrict__ data, uint16_t* __restrict__ out, size_t n, float scale) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const uint8_t* bp = data + (i >> 5) * 18;
@@ -17,17 +20,17 @@ __global__ __launch_bounds__(256) void dequant_q4_0_kernel(const uint8_t* __rest
     const uint32_t j = (uint32_t)i & 31u;
     const uint32_t q = bp[2 + (j & 15u)];
     const uint32_t nib = j < 16u ? (q & 0x0Fu) : (q >> 4);
-    out[i] = lh_f2h_exact(__fmul_rn(__fsub_rn((float)nib, 8.0f), d));     // qat_recover.rs:84-93
+    out[i] = scaled(lh_f2h_exact(__fmul_rn(__fsub_rn((float)nib, 8.0f), d)), scale);     // qat_recover.rs:84-93
 }
 
-__global__ __launch_bounds__(256) void dequant_tq2_0_kernel(const uint8_t* __restrict__ data, uint16_t* __restrict__ out, size_t n) {
+__global__ __launch_bounds__(256) void dequant_tq2_0_kernel(const uint8_t* __restrict__ data, uint16_t* __restrict__ out, size_t n, float scale) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const uint8_t* bp = data + (i >> 8) * 66;
     const float d = lh_h2f((uint16_t)(bp[64] | (bp[65] << 8)));
     const uint32_t r = (uint32_t)i & 255u;
     const uint32_t q = (bp[(r >> 7) * 32 + (r & 31u)] >> (2 * ((r >> 5) & 3u))) & 3u;   // qat_recover.rs:39-47
-    out[i] = lh_f2h_exact(__fmul_rn(d, __fsub_rn((float)q, 1.0f)));
+    out[i] = scaled(lh_f2h_exact(__fmul_rn(d, __fsub_rn((float)q, 1.0f))), scale);
 }
 
 __global__ __launch_bounds__(256) void tq2_dequant_legacy_kernel(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales,
@@ -42,8 +45,7 @@ __global__ __launch_bounds__(256) void tq2_dequant_legacy_kernel(const uint8_t* 
 // Rows picked by a device-resident index list out of a packed [table_rows, cols] table, decoded to f16 into a dense
 // [n_rows, cols] matrix: the embedding gather of a prefill chunk or of a step over many lanes
 // (local-engine/src/pipeline.rs:781-832 decodes the rows on the CPU, one call per token).  An index past the end reads the
-// last row (init_gemma4_qat.rs:152).  With scale != 1 each value is multiplied and rounded once more, which is what
-// scale_in_place.metal:5-14 would do to the decoded row.
+// last row (init_gemma4_qat.rs:152).
 template <int FMT>
 __global__ __launch_bounds__(256) void dequant_rows_kernel(const uint8_t* __restrict__ table, const uint32_t* __restrict__ rows, uint16_t* __restrict__ out,
                                                           uint32_t table_rows, uint32_t cols, size_t row_bytes, float scale) {
@@ -68,11 +70,10 @@ __global__ __launch_bounds__(256) void dequant_rows_kernel(const uint8_t* __rest
     } else {
         h = reinterpret_cast<const uint16_t*>(rp)[c];
     }
-    if (scale != 1.0f) h = lh_f2h(lh_h2f(h) * scale);
-    out[(size_t)blockIdx.y * cols + c] = h;
+    out[(size_t)blockIdx.y * cols + c] = scaled(h, scale);
 }
 
-int dequant_dispatch(lh_batch* batch, lh_quant fmt, const lh_buffer* data, size_t byte_offset, lh_buffer* output, size_t num_elements) {
+int dequant_dispatch(lh_batch* batch, lh_quant fmt, const lh_buffer* data, size_t byte_offset, lh_buffer* output, size_t num_elements, float scale = 1.0f) {
     const char* op = fmt == LH_Q4_0 ? "dequant_q4_0" : "dequant_tq2_0";
     if (!batch) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: batch is null", op);
     if (!data || !output) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: null buffer", op);
@@ -84,8 +85,8 @@ int dequant_dispatch(lh_batch* batch, lh_quant fmt, const lh_buffer* data, size_
     LH_NEED(output, n * 2, op, "output");
     const uint8_t* src = (const uint8_t*)data->ptr + byte_offset;
     const dim3 grid((unsigned)((n + 255) / 256));
-    if (fmt == LH_Q4_0) hipLaunchKernelGGL(dequant_q4_0_kernel, grid, dim3(256), 0, batch->ctx->stream, src, (uint16_t*)output->ptr, n);
-    else hipLaunchKernelGGL(dequant_tq2_0_kernel, grid, dim3(256), 0, batch->ctx->stream, src, (uint16_t*)output->ptr, n);
+    if (fmt == LH_Q4_0) hipLaunchKernelGGL(dequant_q4_0_kernel, grid, dim3(256), 0, batch->ctx->stream, src, (uint16_t*)output->ptr, n, scale);
+    else hipLaunchKernelGGL(dequant_tq2_0_kernel, grid, dim3(256), 0, batch->ctx->stream, src, (uint16_t*)output->ptr, n, scale);
     int r = lh_check_launch(op);
     if (r == LH_OK) batch->dispatch_count++;
     return r;
@@ -100,6 +101,11 @@ int lh_dequant_q4_0_into(lh_batch* batch, const lh_buffer* data, size_t byte_off
 }
 int lh_dequant_tq2_0_into(lh_batch* batch, const lh_buffer* data, size_t byte_offset, lh_buffer* output, size_t num_elements) {
     return dequant_dispatch(batch, LH_TQ2_0, data, byte_offset, output, num_elements);
+}
+
+int lh_dequant_scaled_into(lh_batch* batch, lh_quant fmt, const lh_buffer* data, size_t byte_offset, lh_buffer* output, size_t num_elements, float scale) {
+    if (fmt != LH_Q4_0 && fmt != LH_TQ2_0) return lh_fail(LH_ERR_INVALID_ARGUMENT, "dequant_scaled: unknown weight format %d", (int)fmt);
+    return dequant_dispatch(batch, fmt, data, byte_offset, output, num_elements, scale);
 }
 
 int lh_dequant_rows_into(lh_batch* batch, int fmt, const lh_buffer* table, uint32_t table_rows, uint32_t cols, const lh_buffer* rows,

@@ -55,31 +55,43 @@ __device__ __forceinline__ uint4 rms_apply8(const uint4& v, const uint4& g, cons
     return make_uint4(wo[0], wo[1], wo[2], wo[3]);
 }
 
+// Eight values as scale_in_place_gpu_into leaves them.
+__device__ __forceinline__ uint4 scale8(uint4 v, float by) {
+    uint32_t* w = &v.x;
+#pragma unroll
+    for (int j = 0; j < 4; j++) w[j] = (uint32_t)lh_f2h(lh_h2f((uint16_t)(w[j] & 0xFFFF)) * by) | ((uint32_t)lh_f2h(lh_h2f((uint16_t)(w[j] >> 16)) * by) << 16);
+    return v;
+}
+
+// With before != 1 the input is what scale_in_place_gpu_into would have made of it.
 template <bool ADD, int VEC>
 __global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* in, const uint16_t* __restrict__ w, const uint16_t* res, uint16_t* out,   // out may be in or res
-                                                      uint32_t dim, float eps, uint32_t tail = 0, float scale = 1.0f) {
+                                                      uint32_t dim, float eps, uint32_t tail = 0, float scale = 1.0f, float before = 1.0f) {
     __shared__ float scratch[4];
     const size_t row = (size_t)blockIdx.x * dim;
     float s = 0.0f;
+    auto value = [&](uint32_t i) { const float v = h_at(in, row + i); return before != 1.0f ? lh_h2f(lh_f2h(v * before)) : v; };
     if constexpr (VEC == 8) {
         for (uint32_t i = threadIdx.x * 8; i < dim; i += blockDim.x * 8) {
-            const uint4 v = *reinterpret_cast<const uint4*>(in + row + i);
+            uint4 v = *reinterpret_cast<const uint4*>(in + row + i);
+            if (before != 1.0f) v = scale8(v, before);
             rms_sumsq8(v, s);
         }
     } else {
-        for (uint32_t i = threadIdx.x; i < dim; i += blockDim.x) { const float v = h_at(in, row + i); s += v * v; }
+        for (uint32_t i = threadIdx.x; i < dim; i += blockDim.x) { const float v = value(i); s += v * v; }
     }
     const float rms = rsqrtf(block_sum(s, scratch) / (float)dim + eps);
     if constexpr (VEC == 8) {
         for (uint32_t i = threadIdx.x * 8; i < dim; i += blockDim.x * 8) {
-            const uint4 v = *reinterpret_cast<const uint4*>(in + row + i), g = *reinterpret_cast<const uint4*>(w + i);
-            uint4 r = v;
+            const uint4 g = *reinterpret_cast<const uint4*>(w + i);
+            uint4 v = *reinterpret_cast<const uint4*>(in + row + i), r = v;
+            if (before != 1.0f) v = scale8(v, before);
             if (ADD) r = *reinterpret_cast<const uint4*>(res + row + i);
             *reinterpret_cast<uint4*>(out + row + i) = rms_apply8<ADD>(v, g, r, rms, tail, scale);
         }
     } else {
         for (uint32_t i = threadIdx.x; i < dim; i += blockDim.x) {
-            float v = lh_norm_product(h_at(in, row + i), rms, h_at(w, i));
+            float v = lh_norm_product(value(i), rms, h_at(w, i));
             if (ADD) v = tail ? norm_tail(v, h_at(res, row + i), tail, scale) : v + h_at(res, row + i);
             out[row + i] = lh_f2h_exact(v);
         }
@@ -88,11 +100,11 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* in, const
 
 template <bool ADD>
 void launch_rms_norm(hipStream_t stream, const void* in, const void* w, const void* res, void* out, uint32_t dim, uint32_t rows, float eps,
-                     uint32_t tail = 0, float scale = 1.0f) {
+                     uint32_t tail = 0, float scale = 1.0f, float before = 1.0f) {
     const bool vec = (dim & 7) == 0 && (((uintptr_t)in | (uintptr_t)w | (uintptr_t)(res ? res : in) | (uintptr_t)out) & 15) == 0;
     const uint32_t threads = vec ? (dim >= 2048 ? 256u : (dim >= 1024 ? 128u : 64u)) : (dim >= 256 ? 256u : (dim > 64 ? 128u : 64u));
-    if (vec) hipLaunchKernelGGL((rms_norm_kernel<ADD, 8>), dim3(rows), dim3(threads), 0, stream, (const uint16_t*)in, (const uint16_t*)w, (const uint16_t*)res, (uint16_t*)out, dim, eps, tail, scale);
-    else hipLaunchKernelGGL((rms_norm_kernel<ADD, 1>), dim3(rows), dim3(threads), 0, stream, (const uint16_t*)in, (const uint16_t*)w, (const uint16_t*)res, (uint16_t*)out, dim, eps, tail, scale);
+    if (vec) hipLaunchKernelGGL((rms_norm_kernel<ADD, 8>), dim3(rows), dim3(threads), 0, stream, (const uint16_t*)in, (const uint16_t*)w, (const uint16_t*)res, (uint16_t*)out, dim, eps, tail, scale, before);
+    else hipLaunchKernelGGL((rms_norm_kernel<ADD, 1>), dim3(rows), dim3(threads), 0, stream, (const uint16_t*)in, (const uint16_t*)w, (const uint16_t*)res, (uint16_t*)out, dim, eps, tail, scale, before);
 }
 
 // rms_norm_kernel<ADD, 8> with its input taken either from f16 rows or from the f32 partial tiles of a k-split product
@@ -384,6 +396,10 @@ int finish(lh_batch* batch, const char* op) {
 
 }  // namespace
 
+void lh_launch_logit_softcap(hipStream_t stream, float* data, float cap, uint32_t count) {
+    hipLaunchKernelGGL(logit_softcap_kernel, dim3(blocks_for(count)), dim3(256), 0, stream, data, cap, count);
+}
+
 bool lh_norm_fused_supported(uint32_t dim) { return (dim & 7) == 0 && dim <= 8192; }
 
 void lh_launch_gelu_mul(hipStream_t stream, const void* a, const void* b, void* out, uint32_t count) {
@@ -436,17 +452,27 @@ int lh_rms_norm_add_into(lh_batch* batch, const lh_buffer* input, const lh_buffe
     return finish(batch, op);
 }
 
-int lh_rms_norm_residual_scale_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* weight, const lh_buffer* residual,
-                                    lh_buffer* output, uint32_t dim, uint32_t rows, float eps, int apply_scale, float scale) {
-    const char* op = "rms_norm_residual_scale";
+static int norm_residual_scale(lh_batch* batch, const char* op, float before, const lh_buffer* input, const lh_buffer* weight, const lh_buffer* residual,
+                               lh_buffer* output, uint32_t dim, uint32_t rows, float eps, int apply_scale, float scale) {
     if (!batch) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: batch is null", op);
     if (dim == 0 || rows == 0) return LH_OK;
     LH_NEED(input, (size_t)rows * dim * 2, op, "input");
     LH_NEED(weight, (size_t)dim * 2, op, "weight");
     LH_NEED(residual, (size_t)rows * dim * 2, op, "residual");
     LH_NEED(output, (size_t)rows * dim * 2, op, "output");
-    launch_rms_norm<true>(batch->ctx->stream, input->ptr, weight->ptr, residual->ptr, output->ptr, dim, rows, eps, apply_scale ? 2u : 1u, scale);
+    launch_rms_norm<true>(batch->ctx->stream, input->ptr, weight->ptr, residual->ptr, output->ptr, dim, rows, eps, apply_scale ? 2u : 1u, scale, before);
     return finish(batch, op);
+}
+
+int lh_rms_norm_residual_scale_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* weight, const lh_buffer* residual,
+                                    lh_buffer* output, uint32_t dim, uint32_t rows, float eps, int apply_scale, float scale) {
+    return norm_residual_scale(batch, "rms_norm_residual_scale", 1.0f, input, weight, residual, output, dim, rows, eps, apply_scale, scale);
+}
+
+// The tail of the per-layer inputs of a token: four launches of 2 to 3.5 us as one of 3.5.
+int lh_scale_rms_norm_residual_scale_into(lh_batch* batch, float before, const lh_buffer* input, const lh_buffer* weight, const lh_buffer* residual,
+                                          lh_buffer* output, uint32_t dim, uint32_t rows, float eps, float scale) {
+    return norm_residual_scale(batch, "scale_rms_norm_residual_scale", before, input, weight, residual, output, dim, rows, eps, 1, scale);
 }
 
 int lh_qk_norm_offset_into(lh_batch* batch, lh_buffer* qk_data, const lh_buffer* weight, size_t weight_offset, uint32_t head_dim,

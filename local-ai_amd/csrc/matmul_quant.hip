@@ -254,6 +254,7 @@ struct GroupArgs {
     uint32_t N[4];
     uint32_t tile0[5];
     uint32_t count;          // 0: the single matrix of the kernel arguments
+    float cap;               // f32 results of matmul_wide_kernel become cap * tanh(v / cap); 0: they do not
 };
 __device__ __forceinline__ uint32_t group_of_tile(const GroupArgs& g, uint32_t tile) {
     uint32_t i = 0;
@@ -1131,8 +1132,12 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
         } else {
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const f32x4 v = total[t][j];
+                f32x4 v = total[t][j];
                 const size_t at = (size_t)m * N + n0 + 16 * t + 4 * g;
+                if (CDT == LH_F32 && grp.cap != 0.0f) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) v[i] = grp.cap * tanhf(v[i] / grp.cap);
+                }
                 if constexpr (CDT == LH_F32) *reinterpret_cast<f32x4*>(static_cast<float*>(C) + at) = v;
                 else *reinterpret_cast<uint2*>(static_cast<uint16_t*>(C) + at) = make_uint2(pack_h2(v[0], v[1]), pack_h2(v[2], v[3]));
             }
@@ -1295,7 +1300,7 @@ uint32_t skinny_splits(const lh_context* ctx, uint32_t m, uint32_t workgroups, u
 struct SkinnyPartials { const float* partial; uint32_t splits, cols; };
 template <int FMT, int ADT>
 bool try_skinny(lh_context* ctx, const void* A, const uint8_t* W, void* C, lh_dtype ct, uint32_t m, uint32_t k, uint32_t n, const ClipArgs& clip,
-                const GroupArgs& grp, SkinnyPartials* keep = nullptr) {
+                const GroupArgs& grp, SkinnyPartials* keep = nullptr, bool* capped = nullptr) {
     hipStream_t s = ctx->stream;
     const uint32_t tiles_n = grp.count ? grp.tile0[grp.count] : (n + BN - 1) / BN;
     if constexpr (FMT != kF16W && ADT == LH_F32) {
@@ -1337,6 +1342,7 @@ bool try_skinny(lh_context* ctx, const void* A, const uint8_t* W, void* C, lh_dt
             const uint16_t* X = static_cast<const uint16_t*>(A);
             if (!keep && splits == 1 && !(FMT == kQ4 && m <= (uint32_t)kMaxMultivecM) && wide_pays(ctx, blocks, mgroups)) {
                 const dim3 wide((blocks + 3) / 4, mgroups);
+                if (capped) *capped = ct == LH_F32 && grp.cap != 0.0f;
                 if (ct == LH_F32) hipLaunchKernelGGL((matmul_wide_kernel<FMT, LH_F32, false>), wide, dim3(256), 0, s, X, W, C, m, k, n, blocks, grp);
                 else hipLaunchKernelGGL((matmul_wide_kernel<FMT, LH_F16, false>), wide, dim3(256), 0, s, X, W, C, m, k, n, blocks, grp);
             } else if (FMT == kQ4 && m <= (uint32_t)kMaxMultivecM) {   // unrounded weights for the small batches (2 blocks per unit)
@@ -1450,7 +1456,7 @@ int launch_by_in(bool mfma, lh_context* ctx, const void* A, lh_dtype at, const u
 // kind: kQ4 / kTQ2 / kF16W. `force_multivec` is the multivec_nt_* entry (m <= 16 enforced by the caller).
 int matmul_dispatch(lh_batch* batch, const char* op, int kind, const lh_buffer* input, lh_dtype at, const lh_buffer* weight,
                     lh_buffer* output, lh_dtype ct, uint32_t m, uint32_t k, uint32_t n, bool force_multivec,
-                    const ClipArgs& clip = ClipArgs{nullptr, 0.f, 0.f, 0.f, 0.f, 0u}) {
+                    const ClipArgs& clip = ClipArgs{nullptr, 0.f, 0.f, 0.f, 0.f, 0u}, float cap = 0.0f, bool* capped = nullptr) {
     if (!batch) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: batch is null", op);
     if (ct == LH_BF16) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: bf16 output is not supported", op);
     const uint32_t blk = kind == kQ4 ? 32 : (kind == kTQ2 ? 256 : 32);
@@ -1492,6 +1498,17 @@ int matmul_dispatch(lh_batch* batch, const char* op, int kind, const lh_buffer* 
         }
     }
     const uint8_t* W = (const uint8_t*)weight->ptr;
+    if (cap != 0.0f && mfma && at == LH_F16 && kind != kF16W) {   // the first form that the launch below tries, with the cap in its last step
+        GroupArgs grp{};
+        grp.cap = cap;
+        const bool took = kind == kQ4 ? try_skinny<kQ4, LH_F16>(batch->ctx, input->ptr, W, output->ptr, ct, m, k, n, clip, grp, nullptr, capped)
+                                      : try_skinny<kTQ2, LH_F16>(batch->ctx, input->ptr, W, output->ptr, ct, m, k, n, clip, grp, nullptr, capped);
+        if (took) {
+            int r = lh_check_launch(op);
+            if (r == LH_OK) batch->dispatch_count++;
+            return r;
+        }
+    }
     if (kind == kQ4) launch_by_in<kQ4>(mfma, batch->ctx, input->ptr, at, W, output->ptr, ct, m, k, n, clip);
     else if (kind == kTQ2) launch_by_in<kTQ2>(mfma, batch->ctx, input->ptr, at, W, output->ptr, ct, m, k, n, clip);
     else launch_by_in<kF16W>(true, batch->ctx, input->ptr, at, W, output->ptr, ct, m, k, n, clip);
@@ -1528,6 +1545,23 @@ int lh_matmul_nt_quant_typed_into(lh_batch* b, lh_quant fmt, const lh_buffer* in
     return matmul_dispatch(b, fmt == LH_Q4_0 ? "matmul_nt_q4_0" : "matmul_nt_tq2_0", fmt == LH_Q4_0 ? kQ4 : kTQ2, in, at, w, out, ct, m,
                            k, n, false);
 }
+// Logits of many rows: the cap in the product's last step where that is the wide kernel (64 rows over 262144: 99 + 30 us -> 109), a launch
+// behind the others.
+int lh_matmul_nt_quant_capped_into(lh_batch* b, lh_quant fmt, const lh_buffer* in, lh_dtype at, const lh_buffer* w, lh_buffer* out, uint32_t m, uint32_t k,
+                                   uint32_t n, float cap) {
+    const char* op = fmt == LH_Q4_0 ? "matmul_nt_q4_0 + softcap" : "matmul_nt_tq2_0 + softcap";
+    if (fmt != LH_Q4_0 && fmt != LH_TQ2_0) return lh_fail(LH_ERR_INVALID_ARGUMENT, "matmul_nt_quant + softcap: unknown weight format %d", (int)fmt);
+    LH_REQUIRE(cap > 0.0f, "%s: cap %g", op, (double)cap);
+    LH_REQUIRE((uint64_t)m * n < 0x100000000ull, "%s: %u x %u results", op, m, n);
+    bool capped = false;
+    const int r = matmul_dispatch(b, op, fmt == LH_Q4_0 ? kQ4 : kTQ2, in, at, w, out, LH_F32, m, k, n, false, ClipArgs{nullptr, 0.f, 0.f, 0.f, 0.f, 0u}, cap, &capped);
+    if (r != LH_OK || capped || m == 0 || n == 0 || k == 0) return r;
+    lh_launch_logit_softcap(b->ctx->stream, (float*)out->ptr, cap, m * n);
+    const int c = lh_check_launch(op);
+    if (c == LH_OK) b->dispatch_count++;
+    return c;
+}
+
 int lh_matmul_nt_quant_norm_into(lh_batch* b, lh_quant fmt, const lh_buffer* in, const lh_buffer* w, uint32_t m, uint32_t k, uint32_t n,
                                  const lh_buffer* norm_weight, const lh_buffer* residual, lh_buffer* out, float eps, int apply_scale,
                                  float scale, const lh_buffer* norm2_weight, lh_buffer* out2) {

@@ -232,18 +232,14 @@ class DecodePipeline:
             return
         K, cfg = self.kernels, self.config
         pld, n_layer = cfg.hidden_size_per_layer_input, cfg.num_hidden_layers
-        total = pld * n_layer
-        self.ple_table.dequant_row_into(batch, K, token, self.ple_tok)
-        K.scale_in_place_gpu_into(batch, self.ple_tok, math.sqrt(pld), total)
+        self.ple_table.dequant_row_into(batch, K, token, self.ple_tok, math.sqrt(pld))
         self.per_layer_model_proj.matvec_into(batch, K, self.hidden_a, self.ple_proj)
-        K.scale_in_place_gpu_into(batch, self.ple_proj, 1.0 / math.sqrt(cfg.hidden_size), total)
-        K.rms_norm_into(batch, self.ple_proj, self.per_layer_proj_norm, self.ple_proj, pld, n_layer, cfg.rms_norm_eps)
-        K.residual_add_into(batch, self.ple_proj, self.ple_tok, self.per_layer_input, total)
-        K.scale_in_place_gpu_into(batch, self.per_layer_input, math.sqrt(0.5), total)
+        K.scale_rms_norm_residual_scale_into(batch, 1.0 / math.sqrt(cfg.hidden_size), self.ple_proj, self.per_layer_proj_norm, self.ple_tok,
+                                             self.per_layer_input, pld, n_layer, cfg.rms_norm_eps, math.sqrt(0.5))
 
-    def gather_embedding(self, batch, token: int, dst: Buffer) -> None:
+    def gather_embedding(self, batch, token: int, dst: Buffer, scale: float = 1.0) -> None:
         """pipeline.rs:781-790 for one token: row `token` of the tied embedding table as hidden_size f16 values."""
-        self.token_embd.dequant_row_into(batch, self.kernels, token, dst)
+        self.token_embd.dequant_row_into(batch, self.kernels, token, dst, scale)
 
     def forward_token(self, token: int, position: int, ple_token: Optional[int] = None, batch=None) -> bool:
         """pipeline.rs:834-911: embed, scale by sqrt(hidden), per-layer inputs, all layers.  Returns True when the final
@@ -253,8 +249,7 @@ class DecodePipeline:
         own = batch is None
         batch = batch or CommandBatch(self.ctx)
         cfg, K = self.config, self.kernels
-        self.gather_embedding(batch, token, self.hidden_a)
-        K.scale_in_place_gpu_into(batch, self.hidden_a, math.sqrt(cfg.hidden_size), cfg.hidden_size)
+        self.gather_embedding(batch, token, self.hidden_a, math.sqrt(cfg.hidden_size))
         self.compute_per_layer_inputs(batch, token if ple_token is None else ple_token)
         # A layer may leave its last step (post-norm, residual, output scale) to the next layer's first dispatch: its input
         # buffer is dead by then and receives the finished hidden state, so the two buffers keep their roles in that case.
@@ -314,14 +309,11 @@ class DecodePipeline:
         if self.per_layer_input is None:
             return False
         pld, nl = cfg.hidden_size_per_layer_input, cfg.num_hidden_layers
-        total = n * pld * nl
         batch.write(self._ple_tokens_buf, np.asarray(ple_tokens, np.uint32))
         self.ple_table.dequant_rows_into(batch, K, self._ple_tokens_buf, n, bs.ple_tok, math.sqrt(pld))
         self.per_layer_model_proj.matmul_nt_into(batch, K, bs.hidden_a, bs.ple_proj, n)
-        K.scale_in_place_gpu_into(batch, bs.ple_proj, 1.0 / math.sqrt(h), total)
-        K.rms_norm_into(batch, bs.ple_proj, self.per_layer_proj_norm, bs.ple_proj, pld, n * nl, cfg.rms_norm_eps)
-        K.residual_add_into(batch, bs.ple_proj, bs.ple_tok, bs.ple_all, total)
-        K.scale_in_place_gpu_into(batch, bs.ple_all, math.sqrt(0.5), total)
+        K.scale_rms_norm_residual_scale_into(batch, 1.0 / math.sqrt(h), bs.ple_proj, self.per_layer_proj_norm, bs.ple_tok, bs.ple_all, pld,
+                                             n * nl, cfg.rms_norm_eps, math.sqrt(0.5))
         return True
 
     def forward_tokens_batch(self, tokens, start_pos: int, ple_tokens=None, batch=None) -> bool:
@@ -417,9 +409,10 @@ class DecodePipeline:
             cur_in_a, prenormed = not cur_in_a, next_norm is not None
         final_hidden = bs.hidden_a if cur_in_a else bs.hidden_b
         K.rms_norm_into(batch, final_hidden, self.output_norm, bs.normed, h, n, cfg.rms_norm_eps)
-        self.token_embd.matmul_nt_typed_into(batch, K, bs.normed, F16, state.logits_buf, F32, n)
         if self.logit_softcap > 0.0:
-            K.logit_softcap_gpu_into(batch, state.logits_buf, self.logit_softcap, n * cfg.vocab_size)
+            self.token_embd.matmul_nt_capped_into(batch, K, bs.normed, F16, state.logits_buf, n, self.logit_softcap)
+        else:
+            self.token_embd.matmul_nt_typed_into(batch, K, bs.normed, F16, state.logits_buf, F32, n)
 
     def decode_batch_step(self, state: BatchedDecodeState, tokens, ple_tokens, positions, read_logits: bool = True):
         """batched.rs:271-478: one token for each of len(tokens) active lanes (lane l is row l), lane l at

@@ -81,16 +81,20 @@ class QuantWeight:
         kernels.matmul_nt_quant_typed_into(batch, self.ty, x, x_dtype, self.buf, out, out_dtype, m, self.cols,
                                            self.rows)
 
+    def matmul_nt_capped_into(self, batch, kernels: Kernels, x: Buffer, x_dtype: int, out: Buffer, m: int, cap: float) -> None:
+        """f32 logits under a soft cap."""
+        kernels.matmul_nt_quant_capped_into(batch, self.ty, x, x_dtype, self.buf, out, m, self.cols, self.rows, cap)
+
     # layer.rs:269-281: one row dequantised to f16 (embedding gather); row clamps to the last row
-    def dequant_row_into(self, batch, kernels: Kernels, row: int, out: Buffer) -> None:
+    def dequant_row_into(self, batch, kernels: Kernels, row: int, out: Buffer, scale: float = 1.0) -> None:
         row = min(row, self.rows - 1)
         off = row * self.row_bytes()
-        if self.ty == Q4_0:
-            kernels.dequant_q4_0_into(batch, self.buf, off, out, self.cols)
-        elif self.ty == TQ2_0:
-            kernels.dequant_tq2_0_into(batch, self.buf, off, out, self.cols)
-        else:
-            batch.blit_copy(self.buf, off, out, 0, self.cols * 2)   # an f16 row is its own dequantisation
+        if self.ty != W_F16:
+            kernels.dequant_scaled_into(batch, self.ty, self.buf, off, out, self.cols, scale)
+            return
+        batch.blit_copy(self.buf, off, out, 0, self.cols * 2)   # an f16 row is its own dequantisation
+        if scale != 1.0:
+            kernels.scale_in_place_gpu_into(batch, out, scale, self.cols)
 
     def dequant_rows_into(self, batch, kernels: Kernels, rows: Buffer, n_rows: int, out: Buffer, scale: float = 1.0) -> None:
         """The rows listed in the device u32 buffer `rows` as a dense f16 [n_rows, cols] matrix, optionally scaled: the

@@ -120,9 +120,9 @@ class QuantRowTable:
     def bytes(self) -> int:
         return self._bytes
 
-    def dequant_row_into(self, batch, kernels: Kernels, row: int, out: Buffer) -> None:
+    def dequant_row_into(self, batch, kernels: Kernels, row: int, out: Buffer, scale: float = 1.0) -> None:
         """Row `row` (clamped to the last row, init_gemma4_qat.rs:152) as cols f16 values into `out`."""
-        self._w.dequant_row_into(batch, kernels, row, out)
+        self._w.dequant_row_into(batch, kernels, row, out, scale)
 
     def dequant_rows_into(self, batch, kernels: Kernels, rows: Buffer, n_rows: int, out: Buffer, scale: float = 1.0) -> None:
         """Rows listed in a device u32 buffer, decoded side by side (pipeline.rs:1011-1019 loops over the tokens)."""

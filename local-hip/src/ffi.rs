@@ -102,6 +102,7 @@ extern "C" {
     pub fn lh_matmul_nt_quant_typed_into(batch: *mut lh_batch, fmt: lh_quant, input: *const lh_buffer, input_dtype: lh_dtype, weight: *const lh_buffer, output: *mut lh_buffer, output_dtype: lh_dtype, m: u32, k: u32, n: u32) -> c_int;
     pub fn lh_matmul_nt_quant_gelu_mul_into(batch: *mut lh_batch, fmt: lh_quant, input: *const lh_buffer, w_gate: *const lh_buffer, w_up: *const lh_buffer, output: *mut lh_buffer, m: u32, k: u32, n: u32) -> c_int;
     pub fn lh_matmul_nt_quant_gelu_mul_strided_into(batch: *mut lh_batch, fmt: lh_quant, input: *const lh_buffer, weight: *const lh_buffer, m: u32, k: u32, n: u32, gate_rows: *const lh_buffer, row_stride: u32, row_offset: u32, output: *mut lh_buffer) -> c_int;
+    pub fn lh_matmul_nt_quant_capped_into(batch: *mut lh_batch, fmt: lh_quant, input: *const lh_buffer, input_dtype: lh_dtype, weight: *const lh_buffer, output: *mut lh_buffer, m: u32, k: u32, n: u32, cap: f32) -> c_int;
     pub fn lh_matmul_nt_quant_norm_into(batch: *mut lh_batch, fmt: lh_quant, input: *const lh_buffer, weight: *const lh_buffer, m: u32, k: u32, n: u32, norm_weight: *const lh_buffer, residual: *const lh_buffer, output: *mut lh_buffer, eps: f32, apply_scale: c_int, scale: f32, norm2_weight: *const lh_buffer, output2: *mut lh_buffer) -> c_int;
     pub fn lh_matmul_nt_quant_grouped_into(batch: *mut lh_batch, fmt: lh_quant, count: u32, input: *const lh_buffer, weights: *const *const lh_buffer, outputs: *const *mut lh_buffer, ns: *const u32, m: u32, k: u32) -> c_int;
     pub fn lh_matmul_nt_into(batch: *mut lh_batch, input: *const lh_buffer, weight: *const lh_buffer, output: *mut lh_buffer, m: u32, k: u32, n: u32) -> c_int;
@@ -115,6 +116,7 @@ extern "C" {
     pub fn lh_rms_norm_into(batch: *mut lh_batch, input: *const lh_buffer, weight: *const lh_buffer, output: *mut lh_buffer, dim: u32, rows: u32, eps: f32) -> c_int;
     pub fn lh_rms_norm_add_into(batch: *mut lh_batch, input: *const lh_buffer, weight: *const lh_buffer, residual: *const lh_buffer, output: *mut lh_buffer, dim: u32, rows: u32, eps: f32) -> c_int;
     pub fn lh_rms_norm_residual_scale_into(batch: *mut lh_batch, input: *const lh_buffer, weight: *const lh_buffer, residual: *const lh_buffer, output: *mut lh_buffer, dim: u32, rows: u32, eps: f32, apply_scale: c_int, scale: f32) -> c_int;
+    pub fn lh_scale_rms_norm_residual_scale_into(batch: *mut lh_batch, before: f32, input: *const lh_buffer, weight: *const lh_buffer, residual: *const lh_buffer, output: *mut lh_buffer, dim: u32, rows: u32, eps: f32, scale: f32) -> c_int;
     pub fn lh_qk_norm_gpu_into(batch: *mut lh_batch, qk_data: *mut lh_buffer, weight: *const lh_buffer, head_dim: u32, num_heads: u32, eps: f32) -> c_int;
     pub fn lh_qk_norm_offset_into(batch: *mut lh_batch, qk_data: *mut lh_buffer, weight: *const lh_buffer, weight_offset: usize, head_dim: u32, num_heads: u32, eps: f32) -> c_int;
     pub fn lh_qk_norm_rope_available(head_dim: u32) -> c_int;
@@ -136,6 +138,7 @@ extern "C" {
     pub fn lh_smallm_enabled() -> c_int;
     pub fn lh_dequant_q4_0_into(batch: *mut lh_batch, data: *const lh_buffer, byte_offset: usize, output: *mut lh_buffer, num_elements: usize) -> c_int;
     pub fn lh_dequant_tq2_0_into(batch: *mut lh_batch, data: *const lh_buffer, byte_offset: usize, output: *mut lh_buffer, num_elements: usize) -> c_int;
+    pub fn lh_dequant_scaled_into(batch: *mut lh_batch, fmt: lh_quant, data: *const lh_buffer, byte_offset: usize, output: *mut lh_buffer, num_elements: usize, scale: f32) -> c_int;
     pub fn lh_dequant_rows_into(batch: *mut lh_batch, fmt: c_int, table: *const lh_buffer, table_rows: u32, cols: u32, rows: *const lh_buffer, n_rows: u32, scale: f32, output: *mut lh_buffer) -> c_int;
     pub fn lh_tq2_dequant(ctx: *mut lh_context, packed: *const lh_buffer, scales: *const lh_buffer, output: *mut lh_buffer, num_elements: u32) -> c_int;
     pub fn lh_turboquant_levels(dim: u32, bits: u32, levels: *mut f32) -> c_int;

@@ -171,6 +171,13 @@ impl Kernels {
         check(unsafe { ffi::lh_matmul_nt_quant_gelu_mul_strided_into(batch.as_ptr(), fmt, input.as_ptr(), weight.as_ptr(), m, k, n, gate_rows.as_ptr(), row_stride, row_offset, output.as_ptr()) })
     }
 
+    /// `lh_matmul_nt_quant_capped_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn matmul_nt_quant_capped_into(&self, batch: &mut CommandBatch, fmt: ffi::lh_quant, input: &Buffer, input_dtype: ffi::lh_dtype, weight: &Buffer, output: &Buffer, m: u32, k: u32, n: u32, cap: f32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_matmul_nt_quant_capped_into(batch.as_ptr(), fmt, input.as_ptr(), input_dtype, weight.as_ptr(), output.as_ptr(), m, k, n, cap) })
+    }
+
     /// `lh_matmul_nt_quant_norm_into` (include/local_hip.h).
     #[allow(clippy::too_many_arguments)]
     pub fn matmul_nt_quant_norm_into(&self, batch: &mut CommandBatch, fmt: ffi::lh_quant, input: &Buffer, weight: &Buffer, m: u32, k: u32, n: u32, norm_weight: &Buffer, residual: &Buffer, output: &Buffer, eps: f32, apply_scale: c_int, scale: f32, norm2_weight: &Buffer, output2: &Buffer) -> Result<()> {
@@ -254,6 +261,13 @@ impl Kernels {
     pub fn rms_norm_residual_scale_into(&self, batch: &mut CommandBatch, input: &Buffer, weight: &Buffer, residual: &Buffer, output: &Buffer, dim: u32, rows: u32, eps: f32, apply_scale: c_int, scale: f32) -> Result<()> {
         // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
         check(unsafe { ffi::lh_rms_norm_residual_scale_into(batch.as_ptr(), input.as_ptr(), weight.as_ptr(), residual.as_ptr(), output.as_ptr(), dim, rows, eps, apply_scale, scale) })
+    }
+
+    /// `lh_scale_rms_norm_residual_scale_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn scale_rms_norm_residual_scale_into(&self, batch: &mut CommandBatch, before: f32, input: &Buffer, weight: &Buffer, residual: &Buffer, output: &Buffer, dim: u32, rows: u32, eps: f32, scale: f32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_scale_rms_norm_residual_scale_into(batch.as_ptr(), before, input.as_ptr(), weight.as_ptr(), residual.as_ptr(), output.as_ptr(), dim, rows, eps, scale) })
     }
 
     /// `lh_qk_norm_gpu_into` (include/local_hip.h).
@@ -343,6 +357,12 @@ impl Kernels {
     pub fn dequant_tq2_0_into(&self, batch: &mut CommandBatch, data: &Buffer, byte_offset: usize, output: &Buffer, num_elements: usize) -> Result<()> {
         // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
         check(unsafe { ffi::lh_dequant_tq2_0_into(batch.as_ptr(), data.as_ptr(), byte_offset, output.as_ptr(), num_elements) })
+    }
+
+    /// `lh_dequant_scaled_into` (include/local_hip.h).
+    pub fn dequant_scaled_into(&self, batch: &mut CommandBatch, fmt: ffi::lh_quant, data: &Buffer, byte_offset: usize, output: &Buffer, num_elements: usize, scale: f32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_dequant_scaled_into(batch.as_ptr(), fmt, data.as_ptr(), byte_offset, output.as_ptr(), num_elements, scale) })
     }
 
     /// `lh_dequant_rows_into` (include/local_hip.h).

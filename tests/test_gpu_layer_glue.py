@@ -193,3 +193,55 @@ def test_gelu_mul_strided_equals_gather_then_gelu_mul(pkg, gpu):
         assert np.array_equal(a.as_array(np.uint16), want.as_array(np.uint16))
     with pytest.raises(pkg.InvalidArgument):
         K.gelu_mul_strided_into(pkg.CommandBatch(ctx), a, b, stride, off + 64, got, dim, rows)     # last row past the end of b
+
+
+@pytest.mark.parametrize("dim,rows", [(256, 1), (256, 640), (8, 3), (2048, 5), (100, 7), (1000, 2)])
+def test_scaled_norm_tail_is_the_four_steps(pkg, gpu, dim, rows):
+    """Bit for bit scale_in_place, rms_norm, residual_add and scale_in_place, in the 16-byte and the one-element form."""
+    ctx, K = gpu
+    g, n = pkg.synth.rng(23, dim), dim * rows
+    a, r, w = ((g.standard_normal(s, dtype=np.float32) * 2).astype(np.float16) for s in (n, n, dim))
+    ab, rb, wb, one, out = (pkg.Buffer.from_slice(ctx, x) for x in (a, r, w, np.zeros(n, np.float16), np.zeros(n, np.float16)))
+    batch = pkg.CommandBatch(ctx)
+    K.scale_rms_norm_residual_scale_into(batch, 0.0255155, ab, wb, rb, one, dim, rows, 1e-6, 0.70710678)
+    K.scale_in_place_gpu_into(batch, ab, 0.0255155, n)
+    K.rms_norm_into(batch, ab, wb, ab, dim, rows, 1e-6)
+    K.residual_add_into(batch, ab, rb, out, n)
+    K.scale_in_place_gpu_into(batch, out, 0.70710678, n)
+    batch.commit_and_wait()
+    assert np.array_equal(one.as_array(np.uint16), out.as_array(np.uint16)) and out.as_array(np.uint16).any()
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
+def test_scaled_dequant_is_the_two_steps(pkg, gpu, fmt):
+    ctx, K = gpu
+    raw = pkg.synth.weights(fmt, 3, 768, pkg.synth.rng(24))
+    w = pkg.QuantWeight.from_bytes(ctx, raw, pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, 3, 768)
+    one, two, batch = pkg.Buffer.empty(ctx, 768 * 2), pkg.Buffer.empty(ctx, 768 * 2), pkg.CommandBatch(ctx)
+    w.dequant_row_into(batch, K, 2, one, 39.19)
+    w.dequant_row_into(batch, K, 2, two)
+    K.scale_in_place_gpu_into(batch, two, 39.19, 768)
+    batch.commit_and_wait()
+    assert np.array_equal(one.as_array(np.uint16), two.as_array(np.uint16)) and two.as_array(np.uint16).any()
+
+
+@pytest.mark.parametrize("fmt,dtype", [("q4_0", "F16"), ("tq2_0", "F16"), ("q4_0", "F32")])
+@pytest.mark.parametrize("m,k,n", [(1, 512, 300), (16, 512, 256), (17, 1024, 65536), (64, 1024, 65536), (64, 1024, 66000), (100, 1536, 32768), (300, 512, 2048)])
+def test_capped_product_is_the_two_steps(pkg, gpu, fmt, dtype, m, k, n):
+    """Bit for bit the f32 product and logit_softcap, whichever kernel takes the product."""
+    ctx, K = gpu
+    g = pkg.synth.rng(25, m)
+    raw = pkg.synth.weights(fmt, n, k, g)
+    w = pkg.QuantWeight.from_bytes(ctx, raw, pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, n, k)
+    ty = getattr(pkg, dtype)
+    x = pkg.Buffer.from_slice(ctx, (g.standard_normal((m, k), dtype=np.float32) * 4).astype(np.float16 if ty == pkg.F16 else np.float32))
+    one, two, batch = pkg.Buffer.empty(ctx, m * n * 4), pkg.Buffer.empty(ctx, m * n * 4), pkg.CommandBatch(ctx)
+    print(f"capped {fmt} {dtype} {m} {k} {n}", flush=True)
+    w.matmul_nt_capped_into(batch, K, x, ty, one, m, 30.0)
+    w.matmul_nt_typed_into(batch, K, x, ty, two, pkg.F32, m)
+    K.logit_softcap_gpu_into(batch, two, 30.0, m * n)
+    batch.commit_and_wait()
+    got = one.as_array(np.float32)
+    assert np.array_equal(got, two.as_array(np.float32)) and np.abs(got).max() > 0.1 and np.abs(got).max() <= 30.0
+    with pytest.raises(pkg.InvalidArgument):
+        w.matmul_nt_capped_into(batch, K, x, ty, one, m, 0.0)
