@@ -409,6 +409,28 @@ def test_destinations_of_mixed_types(ai, gpu):
         close(download(ai, b, m * 20, ai.F32).reshape(m, 20), want[:, heads * 12:], F32_TOL)
 
 
+@pytest.mark.parametrize("first", [0, 1])
+@pytest.mark.parametrize("rows,dim,group", [(1, 4, 4), (37, 72, 36), (5, 256, 128), (9, 800, 200), (3, 512, 256), (2, 520, 260), (4, 1024, 1024), (3, 2056, 1028), (2, 4096, 4096),
+                                            (2, 3000, 3000), (2, 4100, 4100), (3, 12288, 4096), (70, 33, 11)])
+def test_gated_norm_parts(ai, gpu, rows, dim, group, first):
+    """Parts on a few lanes of a wave, on a workgroup, and those that are not made of whole pieces; with a weight and without."""
+    ctx, K = gpu
+    g = np.random.default_rng(dim + group)
+    x, w = g.standard_normal((rows, dim)).astype(np.float32), g.standard_normal(dim).astype(np.float32)
+    for dt, tol in ((ai.F32, F32_TOL), (ai.BF16, BF16_TOL)):
+        gate = stored(g.standard_normal((rows, dim)), ai, dt)
+        for weight in (w, None):
+            out, batch = empty(ai, ctx, rows * dim, dt), ai.CommandBatch(ctx)
+            K.gated_norm_rows_into(batch, upload(ai, ctx, x, ai.F32), upload(ai, ctx, gate, dt), None if weight is None else upload(ai, ctx, weight, ai.F32), out, dt, dim, rows,
+                                   1e-5, group, ai.ACT_SILU, bool(first))
+            batch.commit_and_wait()
+            print(f"gated norm {rows} {dim} {group} {first} {dt}", flush=True)
+            f = O.silu(gate)
+            y = x * f if first else x
+            want = O.unit_rms(y.reshape(rows, -1, group), 1e-5).reshape(rows, dim) * (1 if weight is None else w) * (1 if first else f)
+            close(download(ai, out, rows * dim, dt).reshape(rows, dim), want, tol)
+
+
 def test_capped_products(ai, gpu):
     """Sums capped where they are stored are those of the product with a cap behind it: one and several per wave, every form of the product."""
     ctx, K = gpu
