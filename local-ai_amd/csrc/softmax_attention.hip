@@ -95,7 +95,7 @@ typedef __attribute__((address_space(3))) void lvoid;
 // steps and leaves partial records.
 // What binds is vector and matrix instructions at the clock that they leave (a step of 64 keys of two maps: 3600 cycles of matrix
 // instructions per SIMD and about 3000 of vector instructions, before two values were rounded and reduced by one instruction each 5000:
-// 2048 rows of 16 heads, two maps, at position 0 104 -> 95 us, at 2048 252 -> 216).  With one map the two blocks of a step belong to two groups of four
+// 2048 rows of 16 heads, two maps, at position 0 104 -> 95 us, at 2048 252 -> 216).  No product waits for the one before it: 95 -> 89.  With one map the two blocks of a step belong to two groups of four
 // waves, whose sums meet at the end: 2048 rows of 16 heads of 192 and 128 columns 75 -> 66 us.  With two maps the registers do not suffice for that.
 __device__ __forceinline__ uint32_t value_place(uint32_t col) { return ((col >> 2) & 1) * 2 + (((col >> 1) ^ (col >> 3)) & 1); }
 template <int DQ, int DV, int MAPS, int NB, int G>
@@ -163,15 +163,14 @@ __global__ __launch_bounds__(256 * G, G == 2 ? 4 : MAPS * DV <= 256 ? 2 : 1) voi
             lh_bf16x8 w[NW][3];
             lh_f32x4 sc[2 * NW];
 #pragma unroll
-            for (int t = 0; t < 2 * NW; t++) {
-                sc[t] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
-                const uint32_t key = t * 16 + (lane & 15);
+            for (int t = 0; t < 2 * NW; t++) sc[t] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int c = 0; c < DQ / 32; c++) {
-                    const uint32_t ch = mp * (DQ / 8) + c * 4 + (lane >> 4);
+            for (int c = 0; c < DQ / 32; c++)
+#pragma unroll
+                for (int t = 0; t < 2 * NW; t++) {
+                    const uint32_t key = t * 16 + (lane & 15), ch = mp * (DQ / 8) + c * 4 + (lane >> 4);
                     sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lh_bf16x8, ks[key * KC + (ch ^ (key & kSwizzle))]), qf[mp][c], sc[t], 0, 0, 0);
                 }
-            }
             const float alpha = softmax_step<NW>(sc, st[mp], scale2, first, limit, bound, lane, w);
             if (__ballot(alpha != 1.0f)) {
 #pragma unroll
@@ -180,13 +179,19 @@ __global__ __launch_bounds__(256 * G, G == 2 ? 4 : MAPS * DV <= 256 ? 2 : 1) voi
                     for (int r = 0; r < 4; r++) o[mp][d][r] *= alpha;
             }
 #pragma unroll
-            for (int b = 0; b < NW; b++)
+            for (int b = 0; b < NW; b++) {
+                constexpr int most = G == 2 ? 4 : 8, DB = DV / 16 < most ? DV / 16 : most;
 #pragma unroll
-                for (int d = 0; d < DV / 16; d++) {
-                    const lh_bf16x8 vf = __builtin_bit_cast(lh_bf16x8, vs[b * VB + d * 64]);
+                for (int d0 = 0; d0 < DV / 16; d0 += DB) {
+                    lh_bf16x8 vf[DB];
 #pragma unroll
-                    for (int z = 2; z >= 0; z--) o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, w[b][z], o[mp][d], 0, 0, 0);
+                    for (int d = 0; d < DB; d++) vf[d] = __builtin_bit_cast(lh_bf16x8, vs[b * VB + (d0 + d) * 64]);
+#pragma unroll
+                    for (int z = 2; z >= 0; z--)
+#pragma unroll
+                        for (int d = 0; d < DB; d++) o[mp][d0 + d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], w[b][z], o[mp][d0 + d], 0, 0, 0);
                 }
+            }
         }
     }
     float l[MAPS];
