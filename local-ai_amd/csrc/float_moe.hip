@@ -101,14 +101,31 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(uint32_t* __restri
     }
 }
 
-// residual[row] += the row's slots in choice order
+// residual[row] += the row's slots in choice order.  VEC: rows of whole 16-byte pieces (a value at a time: 13.5 us for 2048 rows of 2048
+// columns and two choices, 5.5 for 512 of 1024; now 12.4 and 3.4).
+template <bool VEC>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ slots, const uint32_t* __restrict__ plan, float* __restrict__ residual, uint32_t rows,
                                                      uint32_t top, uint32_t width) {
     const uint32_t row = blockIdx.x, S = rows * top;
-    for (uint32_t i = threadIdx.x; i < width; i += 256) {
-        float s = 0.0f;
-        for (uint32_t c = 0; c < top; c++) s += slots[(size_t)plan[2 * S + row * top + c] * width + i];
-        residual[(size_t)row * width + i] += s;
+    const uint32_t* place = plan + 2 * (size_t)S + (size_t)row * top;
+    float* to = residual + (size_t)row * width;
+    if constexpr (VEC) {
+        for (uint32_t i = threadIdx.x * 4; i < width; i += 1024) {
+            const float4 r = *reinterpret_cast<const float4*>(to + i);
+            float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+            for (uint32_t c = 0; c < top; c++) {
+                const float4 x = *reinterpret_cast<const float4*>(slots + (size_t)place[c] * width + i);
+                s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+            }
+            *reinterpret_cast<float4*>(to + i) = make_float4(r.x + s.x, r.y + s.y, r.z + s.z, r.w + s.w);
+        }
+    } else {
+        for (uint32_t i = threadIdx.x; i < width; i += 256) {
+            float s = 0.0f;
+            for (uint32_t c = 0; c < top; c++) s += slots[(size_t)place[c] * width + i];
+            to[i] += s;
+        }
     }
 }
 
@@ -358,7 +375,8 @@ int lh_moe_down_into(lh_batch* batch, const lh_buffer* hidden, int dtype, const 
     LH_TRY(lh_launch_linear(batch->ctx, a, op));
     batch->dispatch_count++;
     if (direct) return LH_OK;
-    hipLaunchKernelGGL(combine_kernel, dim3(rows), dim3(256), 0, batch->ctx->stream, (const float*)slots->ptr, (const uint32_t*)plan->ptr, (float*)residual->ptr, rows,
+    const bool vec = width % 4 == 0 && (((uintptr_t)slots->ptr | (uintptr_t)residual->ptr) & 15) == 0;
+    hipLaunchKernelGGL((vec ? combine_kernel<true> : combine_kernel<false>), dim3(rows), dim3(256), 0, batch->ctx->stream, (const float*)slots->ptr, (const uint32_t*)plan->ptr, (float*)residual->ptr, rows,
                        top, width);
     LH_TRY(lh_check_launch(op));
     batch->dispatch_count++;

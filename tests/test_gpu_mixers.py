@@ -622,6 +622,13 @@ def test_linear_attention_chunks(ai, gpu, heads, dim, vdim, rows):
 
 
 # ---- mixture of experts ------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("rows,experts,top,width,ff", [(9, 3, 2, 33, 20), (300, 2, 2, 1030, 24)])
+def test_mixture_of_odd_widths(ai, gpu, dtype, rows, experts, top, width, ff):
+    """Rows that are not made of 16-byte pieces."""
+    test_mixture_of_experts(ai, gpu, dtype, rows, experts, top, width, ff)
+
+
 @pytest.mark.parametrize("rows,experts,top,width,ff", [(1000, 5, 1, 2048, 1024), (770, 6, 2, 1024, 2048), (1600, 3, 1, 192, 4096), (400, 2, 1, 2048, 2048)])
 def test_mixture_of_large_experts(ai, gpu, rows, experts, top, width, ff):
     """Expert plans with tiles of 256 rows through the kernels of large products: ragged last tiles, an expert with a few rows and one
