@@ -188,11 +188,9 @@ struct ChunkArgs {
     float scale;
 };
 
-// decay^e, e <= 128, from the powers up to 64 (the power 0 is 1)
-__device__ __forceinline__ float power_of(const float* pw, uint32_t e) { const uint32_t f = min(e, kHalf); return pw[f] * pw[e - f]; }
-// Logarithm of the decay from row s to row t >= s of a chunk, from the running sums of its halves: the sums of the two sides of a
-// half's end are small where the rows are near each other, so that their difference keeps its bits.
-__device__ __forceinline__ float log_between(float at_t, float at_s, bool across, float half_end) { return (across ? half_end - at_s : -at_s) + at_t; }
+// A decay from one half of a chunk into the other is taken in two steps, to the end of the first half and on from there: neither power
+// is above the callers' 64, so that what is finite in steps of 64 rows stays so with decays above one, and differences of running sums
+// keep their bits.
 
 __device__ __forceinline__ lh_bf16x8 bf8(const uint32_t (&w)[4]) {
     struct { uint32_t v[4]; } t = {{w[0], w[1], w[2], w[3]}};
@@ -230,7 +228,7 @@ template <bool VEC> __device__ __forceinline__ uint2 load_values(const uint16_t*
 // 2048 rows, 16 heads of 128 x 128: 24.5 -> 13 us (64 key columns a wave: 16, half as many waves to hide the loads).
 template <int DQ, bool SELECTIVE, bool VEC>
 __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
-    __shared__ float decays[4][kChunk];                        // [wave][row]: from the row to the chunk's end
+    __shared__ float decays[4][kChunk];                        // [wave][row]: from the row to its half's end
     const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n = lane & 15, g = lane >> 4;
     constexpr uint32_t kblocks = DQ / 32;
     const uint32_t vtiles = (a.vdim + 63) / 64, unit = blockIdx.x * 4 + wave;
@@ -250,17 +248,16 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
     };
     fetch(rows[0], 0);
     fetch(rows[1], 32);
+    const float *pw = SELECTIVE ? nullptr : a.powers + h * (kHalf + 1), *sums = SELECTIVE ? a.sums + ((size_t)h * a.halves + 2 * c) * kHalf : nullptr;
 #pragma unroll
     for (uint32_t half = 0; half < 2; half++) {
-        const uint32_t s = half * kHalf + lane, r = min(s, L - 1);
+        const uint32_t s = half * kHalf + lane, r = min(s, L - 1), end = min((half + 1) * kHalf, L) - 1;   // (a half without rows: its end is before them)
         float p;
-        if constexpr (SELECTIVE) {
-            const float* sums = a.sums + ((size_t)h * a.halves + 2 * c) * kHalf;
-            const bool across = half == 0 && L > kHalf;
-            p = expf(log_between(sums[L - 1], sums[r], across, sums[min(kHalf, L) - 1])) * a.sizes[((size_t)h * a.halves + 2 * c) * kHalf + r];
-        } else p = power_of(a.powers + h * (kHalf + 1), L - 1 - r);
+        if constexpr (SELECTIVE) p = expf(sums[end] - sums[r]) * a.sizes[((size_t)h * a.halves + 2 * c) * kHalf + r];
+        else p = pw[end - r];
         decays[wave][s] = s < L ? p : 0.0f;
     }
+    const float to_end = L <= kHalf ? 1.0f : SELECTIVE ? expf(sums[L - 1]) : pw[L - kHalf];   // from the first half's end to the chunk's
     __syncthreads();
     if (!on) return;
     const uint32_t keep = (kcol < a.dim ? 0xFFFFu : 0u) | (kcol + 1 < a.dim ? 0xFFFF0000u : 0u);   // key columns that exist
@@ -275,6 +272,11 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
         if (s0 >= L) break;
         const Rows& now = rows[step];
         if (step < 2) fetch(rows[step + 2], s0 + 64);
+        if (s0 == kHalf)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) acc[j][d] *= to_end;
         lh_bf16x8 vf[4];
 #pragma unroll
         for (int d = 0; d < 4; d++) {
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(const ChunkArgs a, uint
     constexpr uint32_t P = 8;
     for (uint32_t c0 = 0; c0 < a.chunks; c0 += P) {
         float4 x[P];
-        float d[P];
+        float d[P], d2[P];                                     // selective: the logarithm; else the decays of the two halves
 #pragma unroll
         for (uint32_t j = 0; j < P; j++) {
             const uint32_t c = min(c0 + j, a.chunks - 1), L = min(kChunk, a.rows - c * kChunk);
@@ -338,13 +340,14 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(const ChunkArgs a, uint
             if constexpr (SELECTIVE) {
                 const float* sums = a.sums + ((size_t)h * a.halves + 2 * c) * kHalf;
                 d[j] = sums[min(L, kHalf) - 1] + (L > kHalf ? sums[L - 1] : 0.0f);
-            } else d[j] = power_of(pw, L);
+            } else { d[j] = pw[min(L, kHalf)]; d2[j] = pw[L - min(L, kHalf)]; }
         }
 #pragma unroll
         for (uint32_t j = 0; j < P; j++) {
             if (c0 + j >= a.chunks) break;
             u[(size_t)(c0 + j) * total4] = s;
             const float f = SELECTIVE ? expf(d[j]) : d[j];
+            if constexpr (!SELECTIVE) { s.x *= d2[j]; s.y *= d2[j]; s.z *= d2[j]; s.w *= d2[j]; }
             s.x = __builtin_fmaf(f, s.x, x[j].x); s.y = __builtin_fmaf(f, s.y, x[j].y);
             s.z = __builtin_fmaf(f, s.z, x[j].z); s.w = __builtin_fmaf(f, s.w, x[j].w);
         }
@@ -363,7 +366,7 @@ template <int DQ, bool SELECTIVE, bool VEC>
 __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(const ChunkArgs a) {
     constexpr int KB = DQ < 128 ? DQ : 128;                    // key columns of the state in LDS at a time
     __shared__ uint4 terms[3][4][KB / 32][64];                 // [term][value tile][32 key columns][lane]
-    __shared__ float pws[kChunk + 4], sizes[SELECTIVE ? kChunk : 1];   // powers of the decay, or running sums of its logarithm
+    __shared__ float pws[SELECTIVE ? kChunk : kHalf + 4], sizes[SELECTIVE ? kChunk : 1];   // powers of the decay, or running sums of its logarithm
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), g = lane >> 4, n = lane & 15;
     const uint32_t vtiles = (a.vdim + 63) / 64, vb = blockIdx.x % vtiles, h = (blockIdx.x / vtiles) % a.heads, c = blockIdx.x / (vtiles * a.heads);
     const uint32_t t0 = c * kChunk, L = min(kChunk, a.rows - t0), v0 = vb * 64;
@@ -409,7 +412,7 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
             pws[tid] = a.sums[i];
             sizes[tid] = a.sizes[i];
         }
-    } else if (tid <= kChunk) pws[tid] = power_of(a.powers + h * (kHalf + 1), tid);
+    } else if (tid <= kHalf) pws[tid] = a.powers[h * (kHalf + 1) + tid];
     if (a.dim != DQ) {                                         // columns that do not exist
 #pragma unroll
         for (int b = 0; b < 2; b++)
@@ -423,7 +426,7 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
     for (int b = 0; b < 2; b++)
 #pragma unroll
         for (int d = 0; d < 4; d++) o[b][d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
-    // the state's part, scaled by decay^(t + 1) afterwards
+    // the state's part, decayed afterwards
 #pragma unroll
     for (int k0 = 0; k0 < DQ; k0 += KB) {
         if (k0) { __syncthreads(); fetch_state(k0); }
@@ -452,19 +455,20 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
             }
     }
     if (!on) return;
-    const bool late = w0 >= kHalf;                             // rows of the chunk's second half
+    // Rows of the second half: what they take from before it is decayed to the first half's end as it comes, and from there when their
+    // own half begins.
+    const uint32_t half0 = w0 >= kHalf ? kHalf : 0;
     const float half_end = SELECTIVE ? pws[kHalf - 1] : 0.0f;
+    if (half0) {
+        const float f = SELECTIVE ? expf(half_end) : pws[kHalf];
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int d = 0; d < 4; d++) o[b][d] *= f;
+    }
     float own[2];                                              // selective: the running sum at the lane's row
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
-        const uint32_t tr = min(w0 + 16 * b + n, L - 1);
-        own[b] = SELECTIVE ? pws[tr] : 0.0f;
-        const float carry = SELECTIVE ? expf(late ? half_end + own[b] : own[b]) : pws[tr + 1];
-#pragma unroll
-        for (int d = 0; d < 4; d++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) o[b][d][r] *= carry;
-    }
+    for (int b = 0; b < 2; b++) own[b] = SELECTIVE ? pws[min(w0 + 16 * b + n, L - 1)] : 0.0f;
     // the chunk's own rows, 32 at a time
 #pragma unroll 1
     for (uint32_t s0 = 0; s0 <= w0; s0 += 32) {
@@ -486,9 +490,18 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
             vf[d] = bf8(w);
         }
         if (s0 < w0) fetch(s0 + 32);
+        const bool across = s0 < half0;
+        if (s0 == half0)
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                const float f = SELECTIVE ? expf(own[b]) : pws[min(w0 + 16 * b + n, L - 1) - half0 + 1];
+#pragma unroll
+                for (int d = 0; d < 4; d++) o[b][d] *= f;
+            }
 #pragma unroll
         for (int b = 0; b < 2; b++) {
-            const uint32_t t = w0 + 16 * b + n;
+            const uint32_t t = w0 + 16 * b + n, to = across ? kHalf - 1 : t;
+            const float sum_to = across ? half_end : own[b];
             uint32_t p[3][4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -497,9 +510,11 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
                 for (int y = 0; y < 2; y++) {
                     const int m = 2 * j + y;
                     const uint32_t s = s0 + (m >> 2) * 16 + g * 4 + (m & 3);
-                    const float f = SELECTIVE ? expf(fminf(log_between(own[b], pws[s], late && s0 < kHalf, half_end), 0.0f)) * sizes[s] : pws[min(t - s, kChunk)];
-                    // the factor is evaluated for rows after t as well: skipping it would take a branch for each
-                    e[y] = (s <= t ? sc[b][m >> 2][m & 3] : 0.0f) * f;
+                    const float f = SELECTIVE ? expf(fminf(sum_to - pws[s], 0.0f)) * sizes[s] : pws[min(to - s, kHalf)];
+                    // the product is made for rows after t as well (skipping it would take a branch for each) and left out whatever it is:
+                    // a step size or a power there may be no finite number
+                    const float x = sc[b][m >> 2][m & 3] * f;
+                    e[y] = s <= t ? x : 0.0f;
                 }
                 split3_pair(e[0], e[1], p[0][j], p[1][j], p[2][j]);
             }

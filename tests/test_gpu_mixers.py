@@ -621,6 +621,28 @@ def test_linear_attention_chunks(ai, gpu, heads, dim, vdim, rows):
     close(state.as_array(np.float32).reshape(heads, vdim, dq)[:, :, :dim], end.transpose(0, 2, 1), F32_TOL, "state")
 
 
+@pytest.mark.parametrize("decay,rows", [(2.0, 17), (2.0, 100), (2.0, 127), (2.0, 130), (1.25, 200), (3.0, 70)])
+def test_linear_attention_decays_above_one(ai, gpu, decay, rows):
+    """Chunked: what is finite in steps of 64 rows is so; a row is judged against its own size, which grows with the decay's powers."""
+    ctx, K = gpu
+    g, heads, dim, vdim = np.random.default_rng(rows), 2, 32, 48
+    q, k, v = (M.rounded(g.standard_normal(s)) for s in ((rows, heads, dim), (rows, heads, dim), (rows, heads, vdim)))
+    k *= 2.0 ** -14
+    decays = np.array([decay, 0.5])
+    state, out = ai.Buffer.empty(ctx, heads * vdim * dim * 4), empty(ai, ctx, rows * heads * vdim, ai.F32)
+    pw = ai.Buffer.from_slice(ctx, (decays[:, None] ** np.arange(65)).astype(np.float32))
+    work = ai.Buffer.empty(ctx, K.linear_attention_workspace_bytes(rows, heads, dim, vdim))
+    print(f"decays above one {decay} {rows}", flush=True)
+    batch = ai.CommandBatch(ctx)
+    K.linear_attention_chunked_into(batch, *(upload(ai, ctx, x, ai.BF16) for x in (q, k, v)), state, pw, work, out, rows, heads, dim, vdim)
+    batch.commit_and_wait()
+    want, end = O.lightning_recurrence(q, k, v, decays, None)
+    size = np.abs(want).max(2, keepdims=True)
+    close(download(ai, out, rows * heads * vdim, ai.F32).reshape(rows, heads, vdim).astype(np.float64) / size, want / size, F32_TOL, "output")
+    got, size = state.as_array(np.float32).reshape(heads, vdim, dim).astype(np.float64), np.abs(end).max((1, 2))[:, None, None]
+    close(got / size, end.transpose(0, 2, 1) / size, F32_TOL, "state")
+
+
 # ---- mixture of experts ------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("rows,experts,top,width,ff", [(9, 3, 2, 33, 20), (300, 2, 2, 1030, 24)])
