@@ -27,10 +27,10 @@ __device__ __forceinline__ float softplus(float z) { return fmaxf(z, 0.0f) + log
 struct RecurrentArgs {
     const void *q, *k, *v;
     float* state;
-    const float* decay;                                     // [heads]
+    const float* decay;                                     // [heads], `decay_step` apart
     const float *dt_raw, *dt_bias, *a_log, *skip;           // selective: [rows, heads], then [heads] each
     float* out;
-    uint32_t rows, heads, key_heads, dim, dq, vdim;
+    uint32_t rows, heads, key_heads, dim, dq, vdim, decay_step;
     float scale;
 };
 
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(256) void recurrent_kernel(const RecurrentArgs a) {
     float s[NR];
 #pragma unroll
     for (int i = 0; i < NR; i++) s[i] = k0 + i < dq ? st[i] : 0.0f;
-    const float fixed = SELECTIVE ? 0.0f : a.decay[h], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
+    const float fixed = SELECTIVE ? 0.0f : a.decay[(size_t)h * a.decay_step], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
                 skip = SELECTIVE ? a.skip[h] : 0.0f;
     float kn[NR], qn[NR], vn, zn = 0.0f;
     auto fetch = [&](uint32_t t) {
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void recurrent_rows_kernel(const RecurrentArgs
     float s[NR];
 #pragma unroll
     for (int i = 0; i < NR; i++) s[i] = has ? st[i] : 0.0f;
-    const float fixed = SELECTIVE ? 0.0f : a.decay[h], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
+    const float fixed = SELECTIVE ? 0.0f : a.decay[(size_t)h * a.decay_step], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
                 skip = SELECTIVE ? a.skip[h] : 0.0f;
     struct Row { Packed<T, NR> k, q; T v; float z; } next[AHEAD];
     auto fetch = [&](Row& r, uint32_t t) {
@@ -375,14 +375,14 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
     const bool on = w0 < L;
     const uint32_t kh = h / (a.heads / a.key_heads), kstride = a.key_heads * DQ * 2, vstride = a.heads * a.vdim * 2;   // strides in bytes
     const uint16_t *qp = a.q + ((size_t)t0 * a.key_heads + kh) * DQ, *kp = a.k + ((size_t)t0 * a.key_heads + kh) * DQ, *vp = a.v + ((size_t)t0 * a.heads + h) * a.vdim;
-    const float* S = a.chunk_state + (((size_t)c * a.heads + h) * a.vdim) * DQ;
+    const float* S = a.chunk_state + (((size_t)c * a.heads + h) * a.vdim + v0) * DQ;
     constexpr uint32_t each = 4 * (KB / 32) * 64 / 256;        // operands of eight values a thread brings in
     float4 x[each][2];
     auto fetch_state = [&](uint32_t k0) {
 #pragma unroll
         for (uint32_t e = 0; e < each; e++) {
             const uint32_t u = tid + 256 * e, l = u & 63, i = (u >> 6) % (KB / 32), d = (u >> 6) / (KB / 32);
-            const uint32_t o = (min(v0 + (l & 15) * 4 + d, a.vdim - 1) * DQ + k0 + i * 32 + (l >> 4) * 8) * 4;
+            const uint32_t o = (min((l & 15) * 4 + d, a.vdim - 1 - v0) * DQ + k0 + i * 32 + (l >> 4) * 8) * 4;
             x[e][0] = at<float4>(S, o);
             x[e][1] = at<float4>(S, o + 16);
         }
@@ -604,6 +604,10 @@ int launch_recurrent(lh_context* ctx, const RecurrentArgs& a, const char* op) {
     return lh_check_launch(op);
 }
 
+// The chunk kernels address the rows of a chunk with 32-bit byte offsets.  Rows of 2^24 values and more (32 MB each) walk the recurrence:
+// their columns alone fill the chip.
+bool chunk_offsets_fit(uint32_t heads, uint32_t dq, uint32_t vdim) { return (uint64_t)heads * std::max(dq, vdim) < (1u << 24); }
+
 }  // namespace
 
 extern "C" {
@@ -631,7 +635,7 @@ int lh_linear_attention_recurrent_into(lh_batch* batch, const lh_buffer* q, cons
     LH_NEED(output, (size_t)rows * heads * vdim * 4, op, "output");
     RecurrentArgs a{};
     a.q = q->ptr; a.k = k->ptr; a.v = v->ptr; a.state = (float*)state->ptr; a.decay = (const float*)decay->ptr; a.out = (float*)output->ptr;
-    a.rows = rows; a.heads = a.key_heads = heads; a.dim = dim; a.dq = dq; a.vdim = vdim; a.scale = scale;
+    a.rows = rows; a.heads = a.key_heads = heads; a.dim = dim; a.dq = dq; a.vdim = vdim; a.decay_step = 1; a.scale = scale;
     const int r = dtype == LH_F32 ? launch_recurrent<float, false>(batch->ctx, a, op) : launch_recurrent<uint16_t, false>(batch->ctx, a, op);
     if (r == LH_OK) batch->dispatch_count++;
     return r;
@@ -654,7 +658,15 @@ int lh_linear_attention_chunked_into(lh_batch* batch, const lh_buffer* q, const 
     LH_NEED(output, (size_t)rows * heads * vdim * 4, op, "output");
     LH_REQUIRE((((uintptr_t)q->ptr | (uintptr_t)k->ptr | (uintptr_t)v->ptr | (uintptr_t)state->ptr | (uintptr_t)workspace->ptr | (uintptr_t)output->ptr) & 15) == 0,
                "%s: buffers must be 16-byte aligned", op);
-    LH_REQUIRE((uint64_t)heads * std::max(dq, vdim) < (1u << 24), "%s: %u heads of %u and %u columns", op, heads, dim, vdim);   // offsets within a chunk are 32-bit
+    if (!chunk_offsets_fit(heads, dq, vdim)) {
+        RecurrentArgs r{};
+        r.q = q->ptr; r.k = k->ptr; r.v = v->ptr; r.state = (float*)state->ptr; r.out = (float*)output->ptr;
+        r.decay = (const float*)decay_powers->ptr + 1; r.decay_step = kHalf + 1;
+        r.rows = rows; r.heads = r.key_heads = heads; r.dim = dim; r.dq = dq; r.vdim = vdim; r.scale = scale;
+        const int rc = launch_recurrent<uint16_t, false>(batch->ctx, r, op);
+        if (rc == LH_OK) batch->dispatch_count++;
+        return rc;
+    }
     ChunkArgs a{};
     a.q = (const uint16_t*)q->ptr; a.k = (const uint16_t*)k->ptr; a.v = (const uint16_t*)v->ptr; a.state = (float*)state->ptr;
     a.powers = (const float*)decay_powers->ptr; a.chunk_state = (float*)workspace->ptr; a.out = (float*)output->ptr;
@@ -719,7 +731,7 @@ int lh_selective_chunked_into(lh_batch* batch, const lh_buffer* x, const lh_buff
     LH_NEED(output, (size_t)rows * heads * vdim * 4, op, "output");
     LH_REQUIRE((((uintptr_t)x->ptr | (uintptr_t)b->ptr | (uintptr_t)c->ptr | (uintptr_t)memory->ptr | (uintptr_t)workspace->ptr | (uintptr_t)output->ptr) & 15) == 0,
                "%s: buffers must be 16-byte aligned", op);
-    LH_REQUIRE((uint64_t)heads * std::max(dq, vdim) < (1u << 24), "%s: %u heads of %u and %u columns", op, heads, state, vdim);   // offsets within a chunk are 32-bit
+    if (!chunk_offsets_fit(heads, dq, vdim)) return lh_selective_recurrent_into(batch, x, b, c, LH_BF16, dt_raw, dt_bias, a_log, skip, memory, output, rows, heads, vdim, groups, state);
     ChunkArgs a{};
     a.q = (const uint16_t*)c->ptr; a.k = (const uint16_t*)b->ptr; a.v = (const uint16_t*)x->ptr; a.state = (float*)memory->ptr;
     a.chunk_state = (float*)workspace->ptr; a.out = (float*)output->ptr; a.skip = (const float*)skip->ptr;

@@ -643,6 +643,43 @@ def test_linear_attention_decays_above_one(ai, gpu, decay, rows):
     close(got / size, end.transpose(0, 2, 1) / size, F32_TOL, "state")
 
 
+def test_linear_attention_of_very_wide_rows(ai, gpu):
+    """Rows of 2^24 values, which a chunk's 32-bit offsets do not reach, and a state of more than 2^32 bytes a head, which they do."""
+    ctx, K = gpu
+    g, rows = np.random.default_rng(1), 2
+    heads, dim, vdim = 1 << 19, 32, 2
+    q, k, v = (g.standard_normal((rows, heads, n)).astype(np.float32) for n in (dim, dim, vdim))
+    q, k, v = ((x.view(np.uint32) & 0xFFFF0000).view(np.float32) for x in (q, k, v))      # bf16 values
+    bits = lambda x: ai.Buffer.from_slice(ctx, (x.view(np.uint32) >> 16).astype(np.uint16))
+    decay = g.uniform(0.5, 1.0, heads).astype(np.float32)
+    state, out = ai.Buffer.empty(ctx, heads * vdim * dim * 4), empty(ai, ctx, rows * heads * vdim, ai.F32)
+    pw, work = ai.Buffer.from_slice(ctx, decay[:, None] ** np.arange(65, dtype=np.float32)), ai.Buffer.empty(ctx, K.linear_attention_workspace_bytes(rows, heads, dim, vdim))
+    print("very wide rows", flush=True)
+    batch = ai.CommandBatch(ctx)
+    K.linear_attention_chunked_into(batch, bits(q), bits(k), bits(v), state, pw, work, out, rows, heads, dim, vdim)
+    batch.commit_and_wait()
+    dot = lambda t, s: (q[t].astype(np.float64) * k[s]).sum(1)[:, None] * v[s]
+    want = np.stack([dot(0, 0), decay[:, None] * dot(1, 0) + dot(1, 1)])
+    close(download(ai, out, rows * heads * vdim, ai.F32).reshape(rows, heads, vdim), want, F32_TOL, "many heads")
+
+    heads, dim, vdim, rows = 1, 256, (1 << 22) + 70, 3          # columns behind the offset at which 32 bits would begin again
+    q, k = (M.rounded(g.standard_normal((rows, dim))) for _ in range(2))
+    v, end = np.zeros((rows, vdim), np.float32), slice(vdim - 70, None)
+    v[:, :70], v[:, end] = M.rounded(g.standard_normal((rows, 70))), M.rounded(g.standard_normal((rows, 70)))
+    state, out = ai.Buffer.empty(ctx, vdim * dim * 4), empty(ai, ctx, rows * vdim, ai.F32)
+    first = g.standard_normal((70, dim)).astype(np.float32)
+    state.fill_zero()
+    state.copy_from_bytes(first, offset=(vdim - 70) * dim * 4)
+    pw, work = ai.Buffer.from_slice(ctx, (0.75 ** np.arange(65)).astype(np.float32)), ai.Buffer.empty(ctx, K.linear_attention_workspace_bytes(rows, heads, dim, vdim))
+    print("a state of four gigabytes", flush=True)
+    K.linear_attention_chunked_into(batch, upload(ai, ctx, q, ai.BF16), upload(ai, ctx, k, ai.BF16), upload(ai, ctx, v, ai.BF16), state, pw, work, out, rows, heads, dim, vdim)
+    batch.commit_and_wait()
+    got = download(ai, out, rows * vdim, ai.F32).reshape(rows, vdim)
+    for part, begin in ((slice(0, 70), np.zeros((1, dim, 70))), (end, first.T[None].astype(np.float64))):
+        want, _ = O.lightning_recurrence(q[:, None], k[:, None], v[:, None, part].astype(np.float64), np.array([0.75]), begin)
+        close(got[:, part], want[:, 0], F32_TOL, f"columns {part}")
+
+
 # ---- mixture of experts ------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("rows,experts,top,width,ff", [(9, 3, 2, 33, 20), (300, 2, 2, 1030, 24)])
