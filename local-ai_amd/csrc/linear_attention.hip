@@ -211,9 +211,19 @@ __device__ __forceinline__ uint32_t pick(const uint2& a, const uint2& b, int j) 
 // What lies `offset` bytes behind a base that is the same for the whole wave.
 template <typename T> __device__ __forceinline__ T at(const void* base, uint32_t offset) { return *reinterpret_cast<const T*>(static_cast<const char*>(base) + offset); }
 // Four neighbouring columns of a row of values from `col`, no further than the last column: where there is none, what comes is not
-// used.  (No load below is conditional: a branch around it would wait for it.)
-template <bool VEC> __device__ __forceinline__ uint2 load_values(const uint16_t* base, uint32_t row_offset, uint32_t col, uint32_t vdim) {
-    if constexpr (VEC) return at<uint2>(base, row_offset + 2 * min(col, vdim - 4));
+// used.  (No load below is conditional: a branch around it would wait for it.)  VALUES: kPieces, the columns a multiple of four;
+// kWords, any four columns or more, the last four of the row shifted into place (a column at a time: 24.9 us for 2048 rows of 3 heads of
+// 20 x 33, all three kernels; now 17.9); kSingles, fewer than four.
+enum Values { kPieces, kWords, kSingles };
+template <Values VALUES> __device__ __forceinline__ uint2 load_values(const uint16_t* base, uint32_t row_offset, uint32_t col, uint32_t vdim) {
+    if constexpr (VALUES == kPieces) return at<uint2>(base, row_offset + 2 * min(col, vdim - 4));
+    if constexpr (VALUES == kWords) {
+        const uint32_t c = min(col, vdim - 4);
+        uint64_t x;                                            // (two-byte aligned)
+        __builtin_memcpy(&x, reinterpret_cast<const char*>(base) + (row_offset + 2 * c), 8);
+        x >>= 16 * ((col - c) & 3);
+        return make_uint2((uint32_t)x, (uint32_t)(x >> 32));
+    }
     const uint32_t last = vdim - 1;
     auto one = [&](uint32_t j) { return (uint32_t)at<uint16_t>(base, row_offset + 2 * min(col + j, last)); };
     return make_uint2(one(0) | one(1) << 16, one(2) | one(3) << 16);
@@ -226,7 +236,7 @@ template <bool VEC> __device__ __forceinline__ uint2 load_values(const uint16_t*
 // Step 1.  A wave takes 32 key columns and 64 value columns of one chunk of one head.  Row operand = decayed keys, column operand
 // = values.  What binds is the split of the decayed keys (7 vector instructions a value) and the latency of the loads.
 // 2048 rows, 16 heads of 128 x 128: 24.5 -> 13 us (64 key columns a wave: 16, half as many waves to hide the loads).
-template <int DQ, bool SELECTIVE, bool VEC>
+template <int DQ, bool SELECTIVE, Values VALUES>
 __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
     __shared__ float decays[4][kChunk];                        // [wave][row]: from the row to its half's end
     const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n = lane & 15, g = lane >> 4;
@@ -243,7 +253,7 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
 #pragma unroll
         for (uint32_t i = 0; i < 8; i++) {
             to.k[i] = at<uint32_t>(kp, min(k0 + (s0 + i) * kstride, (L - 1) * kstride) + 2 * kcol);
-            to.v[i] = load_values<VEC>(vp, min(v0 + (s0 + i) * vstride, (L - 1) * vstride), vcol, a.vdim);
+            to.v[i] = load_values<VALUES>(vp, min(v0 + (s0 + i) * vstride, (L - 1) * vstride), vcol, a.vdim);
         }
     };
     fetch(rows[0], 0);
@@ -362,7 +372,7 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(const ChunkArgs a, uint
 // it for itself was what bound this step: twice the states, four times the splits.)  What binds now is the vector work on the
 // scores, so the operands of keys and values serve 32 rows.  2048 rows, 16 heads of 128 x 128:
 // 32 -> 20.5 us.
-template <int DQ, bool SELECTIVE, bool VEC>
+template <int DQ, bool SELECTIVE, Values VALUES>
 __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(const ChunkArgs a) {
     constexpr int KB = DQ < 128 ? DQ : 128;                    // key columns of the state in LDS at a time
     __shared__ uint4 terms[3][4][KB / 32][64];                 // [term][value tile][32 key columns][lane]
@@ -403,7 +413,7 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
         }
 #pragma unroll
         for (uint32_t i = 0; i < 8; i++)
-            next.v[i] = load_values<VEC>(vp, min(4 * g * vstride + (s0 + (i >> 2) * 16 + (i & 3)) * vstride, (L - 1) * vstride), v0 + n * 4, a.vdim);
+            next.v[i] = load_values<VALUES>(vp, min(4 * g * vstride + (s0 + (i >> 2) * 16 + (i & 3)) * vstride, (L - 1) * vstride), v0 + n * 4, a.vdim);
     };
     fetch(0);
     if constexpr (SELECTIVE) {
@@ -537,13 +547,13 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
             if (col >= a.vdim) continue;
             float y[4];
             if constexpr (SELECTIVE) {
-                const uint2 z = load_values<VEC>(vp, t * vstride, col, a.vdim);
+                const uint2 z = load_values<VALUES>(vp, t * vstride, col, a.vdim);
                 y[0] = __builtin_bit_cast(float, z.x << 16); y[1] = __builtin_bit_cast(float, z.x & 0xFFFF0000u);
                 y[2] = __builtin_bit_cast(float, z.y << 16); y[3] = __builtin_bit_cast(float, z.y & 0xFFFF0000u);
             }
 #pragma unroll
             for (int d = 0; d < 4; d++) y[d] = SELECTIVE ? __builtin_fmaf(skip, y[d], o[b][d][r]) : o[b][d][r] * a.scale;
-            if constexpr (VEC) *reinterpret_cast<float4*>(out + col) = make_float4(y[0], y[1], y[2], y[3]);
+            if constexpr (VALUES == kPieces) *reinterpret_cast<float4*>(out + col) = make_float4(y[0], y[1], y[2], y[3]);
             else
 #pragma unroll
                 for (uint32_t d = 0; d < 4; d++) if (col + d < a.vdim) out[col + d] = y[d];
@@ -551,31 +561,32 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
     }
 }
 
-template <int DQ, bool SELECTIVE, bool VEC>
+template <int DQ, bool SELECTIVE, Values VALUES>
 int launch_chunked(lh_context* ctx, const ChunkArgs& a, const char* op) {
     const uint32_t grid = a.chunks * a.heads * ((a.vdim + 63) / 64), waves = grid * (DQ / 32);
-    hipLaunchKernelGGL((chunk_state_kernel<DQ, SELECTIVE, VEC>), dim3((waves + 3) / 4), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL((chunk_state_kernel<DQ, SELECTIVE, VALUES>), dim3((waves + 3) / 4), dim3(256), 0, ctx->stream, a);
     int r = lh_check_launch(op);
     if (r != LH_OK) return r;
     const size_t total4 = (size_t)a.heads * a.vdim * DQ / 4;
     hipLaunchKernelGGL((chunk_scan_kernel<SELECTIVE>), dim3((uint32_t)((total4 + 255) / 256)), dim3(256), 0, ctx->stream, a, (uint32_t)DQ);
     r = lh_check_launch(op);
     if (r != LH_OK) return r;
-    hipLaunchKernelGGL((chunk_output_kernel<DQ, SELECTIVE, VEC>), dim3(grid), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL((chunk_output_kernel<DQ, SELECTIVE, VALUES>), dim3(grid), dim3(256), 0, ctx->stream, a);
     return lh_check_launch(op);
 }
-template <bool SELECTIVE, bool VEC>
-int launch_chunked_vec(lh_context* ctx, const ChunkArgs& a, const char* op) {
+template <bool SELECTIVE, Values VALUES>
+int launch_chunked_values(lh_context* ctx, const ChunkArgs& a, const char* op) {
     switch (lh_linear_attention_padded_dim(a.dim)) {
-        case 32: return launch_chunked<32, SELECTIVE, VEC>(ctx, a, op);
-        case 64: return launch_chunked<64, SELECTIVE, VEC>(ctx, a, op);
-        case 128: return launch_chunked<128, SELECTIVE, VEC>(ctx, a, op);
-        default: return launch_chunked<256, SELECTIVE, VEC>(ctx, a, op);
+        case 32: return launch_chunked<32, SELECTIVE, VALUES>(ctx, a, op);
+        case 64: return launch_chunked<64, SELECTIVE, VALUES>(ctx, a, op);
+        case 128: return launch_chunked<128, SELECTIVE, VALUES>(ctx, a, op);
+        default: return launch_chunked<256, SELECTIVE, VALUES>(ctx, a, op);
     }
 }
 template <bool SELECTIVE>
 int launch_chunked_dim(lh_context* ctx, const ChunkArgs& a, const char* op) {
-    return a.vdim % 4 == 0 ? launch_chunked_vec<SELECTIVE, true>(ctx, a, op) : launch_chunked_vec<SELECTIVE, false>(ctx, a, op);
+    if (a.vdim % 4 == 0) return launch_chunked_values<SELECTIVE, kPieces>(ctx, a, op);
+    return a.vdim > 4 ? launch_chunked_values<SELECTIVE, kWords>(ctx, a, op) : launch_chunked_values<SELECTIVE, kSingles>(ctx, a, op);
 }
 
 template <typename T, bool SELECTIVE>

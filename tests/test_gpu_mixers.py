@@ -600,7 +600,7 @@ def test_linear_attention_forms(ai, gpu, heads, dim, vdim, cuts):
             at += n
 
 
-@pytest.mark.parametrize("heads,dim,vdim,rows", [(64, 64, 64, 1100), (8, 256, 100, 1153), (3, 128, 64, 127), (3, 128, 64, 128), (2, 40, 6, 129), (2, 128, 130, 193)])
+@pytest.mark.parametrize("heads,dim,vdim,rows", [(64, 64, 64, 1100), (8, 256, 100, 1153), (3, 128, 64, 127), (3, 128, 64, 128), (2, 40, 6, 129), (2, 128, 130, 193), (3, 20, 33, 129), (3, 20, 3, 70), (2, 200, 5, 64)])
 def test_linear_attention_chunks(ai, gpu, heads, dim, vdim, rows):
     """Chunks of 128 rows: whole, one row short and over, ending in either half; one and several tiles of key and value columns."""
     ctx, K = gpu
