@@ -773,7 +773,7 @@ LH_API int lh_latent_queries_into(lh_batch* batch, const lh_buffer* q, const lh_
  * (read and written); output f32 [rows, heads, vdim].  dim_padded is lh_linear_attention_padded_dim(dim).
  * Outputs are multiplied by `scale`.
  *   recurrent  one launch that walks the rows; any dtype
- *   chunked    blocks of 128 rows on the matrix cores: every chunk's contribution to the state, a scan over the chunks,
+ *   chunked    blocks of 64 or 128 rows on the matrix cores: every chunk's contribution to the state, a scan over the chunks,
  *              then all outputs.  bf16, dim <= 256.  `decay_powers` f32 [heads, 65] holds decay^0 .. decay^64;
  *              `workspace` takes lh_linear_attention_workspace_bytes. */
 LH_API uint32_t lh_linear_attention_padded_dim(uint32_t dim);

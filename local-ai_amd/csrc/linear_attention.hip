@@ -6,8 +6,8 @@
 // Recurrent form: one workgroup per head and 16 value columns; a row of 16 lanes holds one value column's state in
 // registers (DQ / 16 values each) and walks the rows.  From eight rows on the inputs come in several rows ahead.
 //
-// Chunked form (128 rows a chunk, bf16 inputs on the matrix cores, everything else f32; with 64 the states, which every step
-// writes or reads, are twice as many):
+// Chunked form (64 or 128 rows a chunk, bf16 inputs on the matrix cores, everything else f32; with 128 the states, which every step
+// writes or reads, are half as many):
 //   1. every chunk's own contribution to the state, U = sum over rows s of a^(L-1-s) k_s (x) v_s (all chunks at once)
 //   2. a scan over the chunks, M <- a^L M + U, that leaves each chunk's incoming state in place of its U
 //   3. all outputs: y_t = a^(t+1) q_t M_in + sum over s <= t of a^(t-s) (q_t . k_s) v_s
@@ -19,7 +19,7 @@
 
 namespace {
 
-constexpr uint32_t kChunk = 128, kHalf = 64;   // the callers' powers, and the running sums of a selective state space, reach over half a chunk
+constexpr uint32_t kHalf = 64;   // rows that the callers' powers, and the running sums of a selective state space, reach over: a chunk or half of one
 
 // What the step of a token is: fixed per head, or computed from the token (selective state space).
 __device__ __forceinline__ float softplus(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
@@ -184,7 +184,7 @@ struct ChunkArgs {
     const float* skip;         // selective: [heads]
     float* chunk_state;        // [chunk][heads][vdim][dq]
     float* out;
-    uint32_t rows, heads, key_heads, dim, vdim, chunks, halves;
+    uint32_t rows, heads, key_heads, dim, vdim, chunk, chunks, halves;    // `chunk`: rows of one, 64 or 128
     float scale;
 };
 
@@ -213,7 +213,7 @@ template <typename T> __device__ __forceinline__ T at(const void* base, uint32_t
 // Four neighbouring columns of a row of values from `col`, no further than the last column: where there is none, what comes is not
 // used.  (No load below is conditional: a branch around it would wait for it.)  VALUES: kPieces, the columns a multiple of four;
 // kWords, any four columns or more, the last four of the row shifted into place (a column at a time: 24.9 us for 2048 rows of 3 heads of
-// 20 x 33, all three kernels; now 17.9); kSingles, fewer than four.
+// 20 x 33, all three kernels; now 15.0); kSingles, fewer than four.
 enum Values { kPieces, kWords, kSingles };
 template <Values VALUES> __device__ __forceinline__ uint2 load_values(const uint16_t* base, uint32_t row_offset, uint32_t col, uint32_t vdim) {
     if constexpr (VALUES == kPieces) return at<uint2>(base, row_offset + 2 * min(col, vdim - 4));
@@ -233,21 +233,33 @@ template <Values VALUES> __device__ __forceinline__ uint2 load_values(const uint
 // neighbouring columns of eight rows and sorts them in registers: of columns 4 n .. 4 n + 3 of lane n each goes to a tile of its own.
 // Nothing goes through LDS for that (as two-byte stores of a transposed tile it took most of the time).
 
+// Rows of a chunk: 64 while those make no more than a workgroup per CU (256) in step 3, which then waits for one chain of a workgroup,
+// half as long; else 128.  All three steps, chunks of 64 / 128 rows: 16 heads of 128 x 128, 64 rows 14.5 / 15.4 us, 128 rows 15.5 / 19.3, 512 rows
+// 22.8 / 22.8, 2048 rows 45.6 / 36.3; 4 heads of 64 x 64, 512 rows 12.5 / 16.4, 2048 rows 16.8 / 18.2; selective, 32 heads, 512 rows
+// 26.6 / 28.9, 2048 rows 49.7 / 42.0.
+uint32_t short_chunks(uint32_t heads, uint32_t vdim) { return (uint32_t)(256 / std::max<uint64_t>(1, (uint64_t)heads * ((vdim + 63) / 64))); }   // that many at most
+uint32_t chunk_rows(uint32_t rows, uint32_t heads, uint32_t vdim) { return (rows + 63) / 64 <= short_chunks(heads, vdim) ? 64 : 128; }
+size_t state_bytes(uint32_t chunks, uint32_t heads, uint32_t dim, uint32_t vdim) { return (size_t)chunks * heads * vdim * lh_linear_attention_padded_dim(dim) * 4; }
+// The chunk for a workspace of `bytes`, which a caller may have sized for 128 rows.
+uint32_t chunk_in(size_t bytes, uint32_t rows, uint32_t heads, uint32_t dim, uint32_t vdim) {
+    return bytes < state_bytes((rows + 63) / 64, heads, dim, vdim) ? 128 : chunk_rows(rows, heads, vdim);
+}
+
 // Step 1.  A wave takes 32 key columns and 64 value columns of one chunk of one head.  Row operand = decayed keys, column operand
 // = values.  What binds is the split of the decayed keys (7 vector instructions a value) and the latency of the loads.
 // 2048 rows, 16 heads of 128 x 128: 24.5 -> 13 us (64 key columns a wave: 16, half as many waves to hide the loads).
-template <int DQ, bool SELECTIVE, Values VALUES>
+template <int DQ, uint32_t CHUNK, bool SELECTIVE, Values VALUES>
 __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
-    __shared__ float decays[4][kChunk];                        // [wave][row]: from the row to its half's end
+    __shared__ float decays[4][CHUNK];                         // [wave][row]: from the row to its half's end
     const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), n = lane & 15, g = lane >> 4;
     constexpr uint32_t kblocks = DQ / 32;
     const uint32_t vtiles = (a.vdim + 63) / 64, unit = blockIdx.x * 4 + wave;
     const bool on = unit < kblocks * vtiles * a.heads * a.chunks;
     const uint32_t kb = unit % kblocks, r0 = unit / kblocks, vb = r0 % vtiles, h = (r0 / vtiles) % a.heads, c = on ? r0 / (vtiles * a.heads) : 0;
-    const uint32_t t0 = c * kChunk, L = min(kChunk, a.rows - t0);
+    const uint32_t t0 = c * CHUNK, L = min(CHUNK, a.rows - t0);
     const uint32_t kstride = a.key_heads * DQ * 2, vstride = a.heads * a.vdim * 2, kcol = kb * 32 + n * 2, vcol = vb * 64 + n * 4;   // strides in bytes
     const uint16_t *kp = a.k + ((size_t)t0 * a.key_heads + h / (a.heads / a.key_heads)) * DQ, *vp = a.v + ((size_t)t0 * a.heads + h) * a.vdim;
-    struct Rows { uint32_t k[8]; uint2 v[8]; } rows[4];
+    struct Rows { uint32_t k[8]; uint2 v[8]; } rows[CHUNK / 32];
     const uint32_t k0 = 8 * g * kstride, v0 = 8 * g * vstride;
     auto fetch = [&](Rows& to, uint32_t s0) {                  // (rows past the last: the last again, whose decay is 0 then)
 #pragma unroll
@@ -258,12 +270,12 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
     };
     fetch(rows[0], 0);
     fetch(rows[1], 32);
-    const float *pw = SELECTIVE ? nullptr : a.powers + h * (kHalf + 1), *sums = SELECTIVE ? a.sums + ((size_t)h * a.halves + 2 * c) * kHalf : nullptr;
+    const float *pw = SELECTIVE ? nullptr : a.powers + h * (kHalf + 1), *sums = SELECTIVE ? a.sums + ((size_t)h * a.halves + CHUNK / kHalf * c) * kHalf : nullptr;
 #pragma unroll
-    for (uint32_t half = 0; half < 2; half++) {
+    for (uint32_t half = 0; half < CHUNK / kHalf; half++) {
         const uint32_t s = half * kHalf + lane, r = min(s, L - 1), end = min((half + 1) * kHalf, L) - 1;   // (a half without rows: its end is before them)
         float p;
-        if constexpr (SELECTIVE) p = expf(sums[end] - sums[r]) * a.sizes[((size_t)h * a.halves + 2 * c) * kHalf + r];
+        if constexpr (SELECTIVE) p = expf(sums[end] - sums[r]) * a.sizes[((size_t)h * a.halves + CHUNK / kHalf * c) * kHalf + r];
         else p = pw[end - r];
         decays[wave][s] = s < L ? p : 0.0f;
     }
@@ -277,11 +289,11 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkArgs a) {
 #pragma unroll
         for (int d = 0; d < 4; d++) acc[j][d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (uint32_t step = 0; step < 4; step++) {
+    for (uint32_t step = 0; step < CHUNK / 32; step++) {
         const uint32_t s0 = step * 32;
         if (s0 >= L) break;
         const Rows& now = rows[step];
-        if (step < 2) fetch(rows[step + 2], s0 + 64);
+        if (step + 2 < CHUNK / 32) fetch(rows[step + 2], s0 + 64);
         if (s0 == kHalf)
 #pragma unroll
             for (int j = 0; j < 2; j++)
@@ -345,10 +357,10 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(const ChunkArgs a, uint
         float d[P], d2[P];                                     // selective: the logarithm; else the decays of the two halves
 #pragma unroll
         for (uint32_t j = 0; j < P; j++) {
-            const uint32_t c = min(c0 + j, a.chunks - 1), L = min(kChunk, a.rows - c * kChunk);
+            const uint32_t c = min(c0 + j, a.chunks - 1), L = min(a.chunk, a.rows - c * a.chunk);
             x[j] = u[(size_t)c * total4];
             if constexpr (SELECTIVE) {
-                const float* sums = a.sums + ((size_t)h * a.halves + 2 * c) * kHalf;
+                const float* sums = a.sums + ((size_t)h * a.halves + a.chunk / kHalf * c) * kHalf;
                 d[j] = sums[min(L, kHalf) - 1] + (L > kHalf ? sums[L - 1] : 0.0f);
             } else { d[j] = pw[min(L, kHalf)]; d2[j] = pw[L - min(L, kHalf)]; }
         }
@@ -372,16 +384,17 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(const ChunkArgs a, uint
 // it for itself was what bound this step: twice the states, four times the splits.)  What binds now is the vector work on the
 // scores, so the operands of keys and values serve 32 rows.  2048 rows, 16 heads of 128 x 128:
 // 32 -> 20.5 us.
-template <int DQ, bool SELECTIVE, Values VALUES>
-__global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(const ChunkArgs a) {
+template <int DQ, uint32_t CHUNK, bool SELECTIVE, Values VALUES>
+__global__ __launch_bounds__(256, DQ <= 64 ? 3 : DQ <= 128 ? 2 : 1) void chunk_output_kernel(const ChunkArgs a) {
     constexpr int KB = DQ < 128 ? DQ : 128;                    // key columns of the state in LDS at a time
+    constexpr int NB = CHUNK / 64;                             // blocks of 16 rows a wave takes
     __shared__ uint4 terms[3][4][KB / 32][64];                 // [term][value tile][32 key columns][lane]
-    __shared__ float pws[SELECTIVE ? kChunk : kHalf + 4], sizes[SELECTIVE ? kChunk : 1];   // powers of the decay, or running sums of its logarithm
+    __shared__ float pws[SELECTIVE ? CHUNK : kHalf + 4], sizes[SELECTIVE ? CHUNK : 1];   // powers of the decay, or running sums of its logarithm
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), g = lane >> 4, n = lane & 15;
     const uint32_t vtiles = (a.vdim + 63) / 64, vb = blockIdx.x % vtiles, h = (blockIdx.x / vtiles) % a.heads, c = blockIdx.x / (vtiles * a.heads);
-    const uint32_t t0 = c * kChunk, L = min(kChunk, a.rows - t0), v0 = vb * 64;
+    const uint32_t t0 = c * CHUNK, L = min(CHUNK, a.rows - t0), v0 = vb * 64;
     // late rows see more of the chunk: of two workgroups on a CU one has them on the SIMDs where the other has the early ones
-    const uint32_t w0 = ((blockIdx.x >> 8) & 1 ? 3 - wave : wave) * 32;
+    const uint32_t w0 = ((blockIdx.x >> 8) & 1 ? 3 - wave : wave) * (16 * NB);
     const bool on = w0 < L;
     const uint32_t kh = h / (a.heads / a.key_heads), kstride = a.key_heads * DQ * 2, vstride = a.heads * a.vdim * 2;   // strides in bytes
     const uint16_t *qp = a.q + ((size_t)t0 * a.key_heads + kh) * DQ, *kp = a.k + ((size_t)t0 * a.key_heads + kh) * DQ, *vp = a.v + ((size_t)t0 * a.heads + h) * a.vdim;
@@ -398,9 +411,9 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
         }
     };
     fetch_state(0);
-    lh_bf16x8 qf[2][DQ / 32];
+    lh_bf16x8 qf[NB][DQ / 32];
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+    for (int b = 0; b < NB; b++)
 #pragma unroll
         for (int i = 0; i < DQ / 32; i++) qf[b][i] = at<lh_bf16x8>(qp, min(w0 + 16 * b + n, L - 1) * kstride + i * 64 + g * 16);
     struct Rows { lh_bf16x8 k[2][DQ / 32]; uint2 v[8]; } next;
@@ -417,23 +430,23 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
     };
     fetch(0);
     if constexpr (SELECTIVE) {
-        if (tid < kChunk) {
-            const size_t i = ((size_t)h * a.halves + 2 * c) * kHalf + min(tid, L - 1);
+        if (tid < CHUNK) {
+            const size_t i = ((size_t)h * a.halves + CHUNK / kHalf * c) * kHalf + min(tid, L - 1);
             pws[tid] = a.sums[i];
             sizes[tid] = a.sizes[i];
         }
     } else if (tid <= kHalf) pws[tid] = a.powers[h * (kHalf + 1) + tid];
     if (a.dim != DQ) {                                         // columns that do not exist
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int i = 0; i < DQ / 32; i++)
 #pragma unroll
                 for (uint32_t j = 0; j < 8; j++) if (i * 32 + g * 8 + j >= a.dim) qf[b][i][j] = (__bf16)0.0f;
     }
-    lh_f32x4 o[2][4];
+    lh_f32x4 o[NB][4];
 #pragma unroll
-    for (int b = 0; b < 2; b++)
+    for (int b = 0; b < NB; b++)
 #pragma unroll
         for (int d = 0; d < 4; d++) o[b][d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
     // the state's part, decayed afterwards
@@ -459,7 +472,7 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
 #pragma unroll
                 for (int d = 0; d < 4; d++) sf[d] = __builtin_bit_cast(lh_bf16x8, terms[z][d][i][lane]);
 #pragma unroll
-                for (int b = 0; b < 2; b++)
+                for (int b = 0; b < NB; b++)
 #pragma unroll
                     for (int d = 0; d < 4; d++) o[b][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sf[d], qf[b][k0 / 32 + i], o[b][d], 0, 0, 0);
             }
@@ -467,24 +480,24 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
     if (!on) return;
     // Rows of the second half: what they take from before it is decayed to the first half's end as it comes, and from there when their
     // own half begins.
-    const uint32_t half0 = w0 >= kHalf ? kHalf : 0;
+    const uint32_t half0 = CHUNK > kHalf && w0 >= kHalf ? kHalf : 0;
     const float half_end = SELECTIVE ? pws[kHalf - 1] : 0.0f;
     if (half0) {
         const float f = SELECTIVE ? expf(half_end) : pws[kHalf];
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int d = 0; d < 4; d++) o[b][d] *= f;
     }
-    float own[2];                                              // selective: the running sum at the lane's row
+    float sum_to[NB];                                          // selective: the running sum at the half's end, then at the lane's row
 #pragma unroll
-    for (int b = 0; b < 2; b++) own[b] = SELECTIVE ? pws[min(w0 + 16 * b + n, L - 1)] : 0.0f;
+    for (int b = 0; b < NB; b++) sum_to[b] = half_end;
     // the chunk's own rows, 32 at a time
 #pragma unroll 1
     for (uint32_t s0 = 0; s0 <= w0; s0 += 32) {
-        lh_f32x4 sc[2][2];
+        lh_f32x4 sc[NB][2];
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int b = 0; b < NB; b++)
 #pragma unroll
             for (int u = 0; u < 2; u++) {
                 sc[b][u] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
@@ -499,19 +512,20 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
             for (int i = 0; i < 4; i++) w[i] = pick(next.v[2 * i], next.v[2 * i + 1], d);
             vf[d] = bf8(w);
         }
-        if (s0 < w0) fetch(s0 + 32);
+        if (s0 + 32 <= w0) fetch(s0 + 32);
         const bool across = s0 < half0;
         if (s0 == half0)
 #pragma unroll
-            for (int b = 0; b < 2; b++) {
-                const float f = SELECTIVE ? expf(own[b]) : pws[min(w0 + 16 * b + n, L - 1) - half0 + 1];
+            for (int b = 0; b < NB; b++) {
+                const uint32_t tr = min(w0 + 16 * b + n, L - 1);
+                sum_to[b] = pws[SELECTIVE ? tr : 0];
+                const float f = SELECTIVE ? expf(sum_to[b]) : pws[tr - half0 + 1];
 #pragma unroll
                 for (int d = 0; d < 4; d++) o[b][d] *= f;
             }
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
+        for (int b = 0; b < NB; b++) {
             const uint32_t t = w0 + 16 * b + n, to = across ? kHalf - 1 : t;
-            const float sum_to = across ? half_end : own[b];
             uint32_t p[3][4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -520,7 +534,7 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
                 for (int y = 0; y < 2; y++) {
                     const int m = 2 * j + y;
                     const uint32_t s = s0 + (m >> 2) * 16 + g * 4 + (m & 3);
-                    const float f = SELECTIVE ? expf(fminf(sum_to - pws[s], 0.0f)) * sizes[s] : pws[min(to - s, kHalf)];
+                    const float f = SELECTIVE ? expf(fminf(sum_to[b] - pws[s], 0.0f)) * sizes[s] : pws[min(to - s, kHalf)];
                     // the product is made for rows after t as well (skipping it would take a branch for each) and left out whatever it is:
                     // a step size or a power there may be no finite number
                     const float x = sc[b][m >> 2][m & 3] * f;
@@ -537,7 +551,7 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
     // a lane holds 16 neighbouring value columns of its rows
     const float skip = SELECTIVE ? a.skip[h] : 0.0f;
 #pragma unroll
-    for (int b = 0; b < 2; b++) {
+    for (int b = 0; b < NB; b++) {
         const uint32_t t = w0 + 16 * b + n;
         if (t >= L) continue;
         float* out = a.out + ((size_t)(t0 + t) * a.heads + h) * a.vdim;
@@ -561,32 +575,37 @@ __global__ __launch_bounds__(256, DQ <= 128 ? 2 : 1) void chunk_output_kernel(co
     }
 }
 
-template <int DQ, bool SELECTIVE, Values VALUES>
+template <int DQ, uint32_t CHUNK, bool SELECTIVE, Values VALUES>
 int launch_chunked(lh_context* ctx, const ChunkArgs& a, const char* op) {
     const uint32_t grid = a.chunks * a.heads * ((a.vdim + 63) / 64), waves = grid * (DQ / 32);
-    hipLaunchKernelGGL((chunk_state_kernel<DQ, SELECTIVE, VALUES>), dim3((waves + 3) / 4), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL((chunk_state_kernel<DQ, CHUNK, SELECTIVE, VALUES>), dim3((waves + 3) / 4), dim3(256), 0, ctx->stream, a);
     int r = lh_check_launch(op);
     if (r != LH_OK) return r;
     const size_t total4 = (size_t)a.heads * a.vdim * DQ / 4;
     hipLaunchKernelGGL((chunk_scan_kernel<SELECTIVE>), dim3((uint32_t)((total4 + 255) / 256)), dim3(256), 0, ctx->stream, a, (uint32_t)DQ);
     r = lh_check_launch(op);
     if (r != LH_OK) return r;
-    hipLaunchKernelGGL((chunk_output_kernel<DQ, SELECTIVE, VALUES>), dim3(grid), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL((chunk_output_kernel<DQ, CHUNK, SELECTIVE, VALUES>), dim3(grid), dim3(256), 0, ctx->stream, a);
     return lh_check_launch(op);
 }
-template <bool SELECTIVE, Values VALUES>
+template <uint32_t CHUNK, bool SELECTIVE, Values VALUES>
 int launch_chunked_values(lh_context* ctx, const ChunkArgs& a, const char* op) {
     switch (lh_linear_attention_padded_dim(a.dim)) {
-        case 32: return launch_chunked<32, SELECTIVE, VALUES>(ctx, a, op);
-        case 64: return launch_chunked<64, SELECTIVE, VALUES>(ctx, a, op);
-        case 128: return launch_chunked<128, SELECTIVE, VALUES>(ctx, a, op);
-        default: return launch_chunked<256, SELECTIVE, VALUES>(ctx, a, op);
+        case 32: return launch_chunked<32, CHUNK, SELECTIVE, VALUES>(ctx, a, op);
+        case 64: return launch_chunked<64, CHUNK, SELECTIVE, VALUES>(ctx, a, op);
+        case 128: return launch_chunked<128, CHUNK, SELECTIVE, VALUES>(ctx, a, op);
+        default: return launch_chunked<256, CHUNK, SELECTIVE, VALUES>(ctx, a, op);
     }
 }
+template <uint32_t CHUNK, bool SELECTIVE>
+int launch_chunked_rows(lh_context* ctx, const ChunkArgs& a, const char* op) {
+    if (a.vdim % 4 == 0) return launch_chunked_values<CHUNK, SELECTIVE, kPieces>(ctx, a, op);
+    return a.vdim > 4 ? launch_chunked_values<CHUNK, SELECTIVE, kWords>(ctx, a, op) : launch_chunked_values<CHUNK, SELECTIVE, kSingles>(ctx, a, op);
+}
 template <bool SELECTIVE>
-int launch_chunked_dim(lh_context* ctx, const ChunkArgs& a, const char* op) {
-    if (a.vdim % 4 == 0) return launch_chunked_values<SELECTIVE, kPieces>(ctx, a, op);
-    return a.vdim > 4 ? launch_chunked_values<SELECTIVE, kWords>(ctx, a, op) : launch_chunked_values<SELECTIVE, kSingles>(ctx, a, op);
+int launch_chunked_dim(lh_context* ctx, ChunkArgs& a, const char* op) {
+    a.chunks = (a.rows + a.chunk - 1) / a.chunk;
+    return a.chunk == 64 ? launch_chunked_rows<64, SELECTIVE>(ctx, a, op) : launch_chunked_rows<128, SELECTIVE>(ctx, a, op);
 }
 
 template <typename T, bool SELECTIVE>
@@ -625,8 +644,9 @@ extern "C" {
 
 uint32_t lh_linear_attention_padded_dim(uint32_t dim) { return dim <= 32 ? 32u : dim <= 64 ? 64u : (dim + 127) / 128 * 128; }
 
+// (what is enough for `rows` is enough for fewer)
 size_t lh_linear_attention_workspace_bytes(uint32_t rows, uint32_t heads, uint32_t dim, uint32_t vdim) {
-    return (size_t)((rows + kChunk - 1) / kChunk) * heads * vdim * lh_linear_attention_padded_dim(dim) * 4;
+    return state_bytes(std::max((rows + 127) / 128, std::min((rows + 63) / 64, short_chunks(heads, vdim))), heads, dim, vdim);
 }
 
 int lh_linear_attention_recurrent_into(lh_batch* batch, const lh_buffer* q, const lh_buffer* k, const lh_buffer* v, int dtype, lh_buffer* state,
@@ -665,7 +685,7 @@ int lh_linear_attention_chunked_into(lh_batch* batch, const lh_buffer* q, const 
     LH_NEED(v, (size_t)rows * heads * vdim * 2, op, "v");
     LH_NEED(state, (size_t)heads * vdim * dq * 4, op, "state");
     LH_NEED(decay_powers, (size_t)heads * (kHalf + 1) * 4, op, "decay_powers");
-    LH_NEED(workspace, lh_linear_attention_workspace_bytes(rows, heads, dim, vdim), op, "workspace");
+    LH_NEED(workspace, state_bytes((rows + 127) / 128, heads, dim, vdim), op, "workspace");
     LH_NEED(output, (size_t)rows * heads * vdim * 4, op, "output");
     LH_REQUIRE((((uintptr_t)q->ptr | (uintptr_t)k->ptr | (uintptr_t)v->ptr | (uintptr_t)state->ptr | (uintptr_t)workspace->ptr | (uintptr_t)output->ptr) & 15) == 0,
                "%s: buffers must be 16-byte aligned", op);
@@ -681,8 +701,8 @@ int lh_linear_attention_chunked_into(lh_batch* batch, const lh_buffer* q, const 
     ChunkArgs a{};
     a.q = (const uint16_t*)q->ptr; a.k = (const uint16_t*)k->ptr; a.v = (const uint16_t*)v->ptr; a.state = (float*)state->ptr;
     a.powers = (const float*)decay_powers->ptr; a.chunk_state = (float*)workspace->ptr; a.out = (float*)output->ptr;
-    a.rows = rows; a.heads = a.key_heads = heads; a.dim = dim; a.vdim = vdim; a.chunks = (rows + kChunk - 1) / kChunk; a.halves = (rows + kHalf - 1) / kHalf; a.scale = scale;
-    LH_REQUIRE((uint64_t)a.chunks * heads * ((vdim + 63) / 64) * 8 < 0x7FFFFFFFull, "%s: %u rows", op, rows);
+    a.rows = rows; a.heads = a.key_heads = heads; a.dim = dim; a.vdim = vdim; a.chunk = chunk_in(workspace->len, rows, heads, dim, vdim); a.halves = (rows + kHalf - 1) / kHalf; a.scale = scale;
+    LH_REQUIRE((uint64_t)((rows + 63) / 64) * heads * ((vdim + 63) / 64) * 8 < 0x7FFFFFFFull, "%s: %u rows", op, rows);
     const int r = launch_chunked_dim<false>(batch->ctx, a, op);
     if (r == LH_OK) batch->dispatch_count += 3;
     return r;
@@ -738,7 +758,7 @@ int lh_selective_chunked_into(lh_batch* batch, const lh_buffer* x, const lh_buff
     LH_NEED(skip, (size_t)heads * 4, op, "skip");
     LH_NEED(memory, (size_t)heads * vdim * dq * 4, op, "memory");
     LH_NEED(steps, lh_selective_steps_bytes(rows, heads), op, "steps");
-    LH_NEED(workspace, lh_linear_attention_workspace_bytes(rows, heads, state, vdim), op, "workspace");
+    LH_NEED(workspace, state_bytes((rows + 127) / 128, heads, state, vdim), op, "workspace");
     LH_NEED(output, (size_t)rows * heads * vdim * 4, op, "output");
     LH_REQUIRE((((uintptr_t)x->ptr | (uintptr_t)b->ptr | (uintptr_t)c->ptr | (uintptr_t)memory->ptr | (uintptr_t)workspace->ptr | (uintptr_t)output->ptr) & 15) == 0,
                "%s: buffers must be 16-byte aligned", op);
@@ -746,8 +766,8 @@ int lh_selective_chunked_into(lh_batch* batch, const lh_buffer* x, const lh_buff
     ChunkArgs a{};
     a.q = (const uint16_t*)c->ptr; a.k = (const uint16_t*)b->ptr; a.v = (const uint16_t*)x->ptr; a.state = (float*)memory->ptr;
     a.chunk_state = (float*)workspace->ptr; a.out = (float*)output->ptr; a.skip = (const float*)skip->ptr;
-    a.rows = rows; a.heads = heads; a.key_heads = groups; a.dim = state; a.vdim = vdim; a.chunks = (rows + kChunk - 1) / kChunk; a.halves = (rows + kHalf - 1) / kHalf; a.scale = 1.0f;
-    LH_REQUIRE((uint64_t)a.chunks * heads * ((vdim + 63) / 64) * 8 < 0x7FFFFFFFull, "%s: %u rows", op, rows);
+    a.rows = rows; a.heads = heads; a.key_heads = groups; a.dim = state; a.vdim = vdim; a.chunk = chunk_in(workspace->len, rows, heads, state, vdim); a.halves = (rows + kHalf - 1) / kHalf; a.scale = 1.0f;
+    LH_REQUIRE((uint64_t)((rows + 63) / 64) * heads * ((vdim + 63) / 64) * 8 < 0x7FFFFFFFull, "%s: %u rows", op, rows);
     float* sums = (float*)steps->ptr;
     float* sizes = sums + (size_t)a.halves * kHalf * heads;
     a.sums = sums; a.sizes = sizes;

@@ -600,9 +600,11 @@ def test_linear_attention_forms(ai, gpu, heads, dim, vdim, cuts):
             at += n
 
 
-@pytest.mark.parametrize("heads,dim,vdim,rows", [(64, 64, 64, 1100), (8, 256, 100, 1153), (3, 128, 64, 127), (3, 128, 64, 128), (2, 40, 6, 129), (2, 128, 130, 193), (3, 20, 33, 129), (3, 20, 3, 70), (2, 200, 5, 64)])
+@pytest.mark.parametrize("heads,dim,vdim,rows", [(64, 64, 64, 1100), (8, 256, 100, 1153), (3, 128, 64, 127), (3, 128, 64, 128), (2, 40, 6, 129), (2, 128, 130, 193),
+                                                  (130, 20, 33, 127), (129, 32, 64, 128), (130, 64, 70, 193), (260, 8, 6, 129), (260, 40, 3, 130), (3, 20, 3, 70), (2, 200, 5, 64)])
 def test_linear_attention_chunks(ai, gpu, heads, dim, vdim, rows):
-    """Chunks of 128 rows: whole, one row short and over, ending in either half; one and several tiles of key and value columns."""
+    """Chunks of 128 rows (more than 256 workgroups with 64) and of 64: whole, one row short and over, ending in either half; one and several
+    tiles of key and value columns, widths of values of all remainders."""
     ctx, K = gpu
     g = np.random.default_rng(heads + dim + rows)
     decay, dq = np.linspace(0.6, 1.0, heads), K.linear_attention_padded_dim(dim)
@@ -622,13 +624,14 @@ def test_linear_attention_chunks(ai, gpu, heads, dim, vdim, rows):
 
 
 @pytest.mark.parametrize("decay,rows", [(2.0, 17), (2.0, 100), (2.0, 127), (2.0, 130), (1.25, 200), (3.0, 70)])
-def test_linear_attention_decays_above_one(ai, gpu, decay, rows):
+@pytest.mark.parametrize("heads", [2, 130])
+def test_linear_attention_decays_above_one(ai, gpu, decay, rows, heads):
     """Chunked: what is finite in steps of 64 rows is so; a row is judged against its own size, which grows with the decay's powers."""
     ctx, K = gpu
-    g, heads, dim, vdim = np.random.default_rng(rows), 2, 32, 48
+    g, dim, vdim = np.random.default_rng(rows), 32, 48
     q, k, v = (M.rounded(g.standard_normal(s)) for s in ((rows, heads, dim), (rows, heads, dim), (rows, heads, vdim)))
     k *= 2.0 ** -14
-    decays = np.array([decay, 0.5])
+    decays = np.array([decay, 0.5] * (heads // 2))
     state, out = ai.Buffer.empty(ctx, heads * vdim * dim * 4), empty(ai, ctx, rows * heads * vdim, ai.F32)
     pw = ai.Buffer.from_slice(ctx, (decays[:, None] ** np.arange(65)).astype(np.float32))
     work = ai.Buffer.empty(ctx, K.linear_attention_workspace_bytes(rows, heads, dim, vdim))
