@@ -297,6 +297,17 @@ class CommandBatch:
             pass
 
 
+def encoded_work_ran(ctx: Context, error: BaseException) -> bool:
+    """Whether what had been encoded when `error` came has run: waits for it, unless the error is what a wait reported."""
+    if isinstance(error, CommandBuffer):
+        return False
+    try:
+        CommandBatch(ctx).commit_and_wait()
+    except Error:
+        return False
+    return True
+
+
 class Graph:
     """A recorded batch: ``launch()`` enqueues one replay of every dispatch captured between
     ``CommandBatch.begin_capture`` and ``end_capture``."""

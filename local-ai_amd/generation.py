@@ -11,7 +11,7 @@ from typing import Deque, List, Optional, Sequence
 
 import numpy as np
 
-from . import CommandBatch, InvalidArgument
+from . import CommandBatch, InvalidArgument, encoded_work_ran
 from .kv_cache import SlotPool
 
 
@@ -145,19 +145,26 @@ class PipelineSequences:
         self.slots.release(seq)
 
     def step(self, seq, tokens, want=()) -> np.ndarray:
-        """Chunks of rows are only encoded: the token behind them, whose results are waited for, is on the same stream."""
+        """Chunks of rows are only encoded: the token behind them, whose results are waited for, is on the same stream.  If that wait
+        reports a fault, the sequence is where the last one that did not left it."""
         out = np.empty((len(want), self.vocab_size), np.float32)
-        last, lo = len(tokens) - 1, 0
-        while lo <= last:
-            if any(p == lo for p in want) or lo == last:
-                seq.decode_step(int(tokens[lo]))
-                for i, p in enumerate(want):
-                    if p == lo:
-                        seq.logits_buf.read_into(out[i])
-                lo += 1
-                continue
-            hi = min([p for p in want if p > lo] + [last, lo + seq.max_batch])
-            seq.forward_tokens_batch(list(tokens[lo:hi]), seq.position, batch=CommandBatch(seq.ctx))
-            seq.position += hi - lo
-            lo = hi
+        last, lo, sure = len(tokens) - 1, 0, seq.position
+        try:
+            while lo <= last:
+                if any(p == lo for p in want) or lo == last:
+                    seq.decode_step(int(tokens[lo]))
+                    sure = seq.position
+                    for i, p in enumerate(want):
+                        if p == lo:
+                            seq.logits_buf.read_into(out[i])
+                    lo += 1
+                    continue
+                hi = min([p for p in want if p > lo] + [last, lo + seq.max_batch])
+                seq.forward_tokens_batch(list(tokens[lo:hi]), seq.position, batch=CommandBatch(seq.ctx))
+                seq.position += hi - lo
+                lo = hi
+        except BaseException as e:
+            if seq.position != sure and not encoded_work_ran(seq.ctx, e):
+                seq.position = sure
+            raise
         return out

@@ -7,7 +7,7 @@ from typing import List, Optional, Sequence, Tuple, Type
 
 import numpy as np
 
-from . import BF16, F32, Buffer, CommandBatch, InvalidArgument, Kernels
+from . import BF16, F32, Buffer, CommandBatch, InvalidArgument, Kernels, encoded_work_ran
 from .kv_cache import SequenceSlot, SlotPool
 from .linear_weight import Segment, StackedLinear
 from .mixers import LatentAttentionSpec, LayerSpec, Norm, OutputNormLayer, PreNormLayer, Run, Workspace
@@ -103,7 +103,8 @@ class StackPipeline:
         self.slots.release(seq)
 
     def step(self, seq: SequenceSlot, tokens: Sequence[int], want: Sequence[int] = ()) -> np.ndarray:
-        """Runs `tokens` at the sequence's next positions; logits f32 [len(want), vocab] at those places among them."""
+        """Runs `tokens` at the sequence's next positions; logits f32 [len(want), vocab] at those places among them.  All pieces but
+        the last are only encoded: if the wait behind them reports a fault, the sequence is where it was."""
         n = len(tokens)
         if n == 0:
             raise InvalidArgument("a step needs at least one token")
@@ -114,13 +115,19 @@ class StackPipeline:
         if any(not 0 <= int(p) < n for p in want):
             raise InvalidArgument("wanted place outside the step")
         out = np.empty((len(want), self.vocab_size), np.float32)
-        for lo in range(0, n, self.max_rows):
-            hi = min(lo + self.max_rows, n)
-            at = [i for i, p in enumerate(want) if lo <= p < hi]
-            got = out if len(at) == len(want) else np.empty((len(at), self.vocab_size), np.float32)
-            self._forward(seq, tokens[lo:hi], [want[i] - lo for i in at], got, wait=hi == n)
-            if at and got is not out:
-                out[at] = got
+        begin = seq.position
+        try:
+            for lo in range(0, n, self.max_rows):
+                hi = min(lo + self.max_rows, n)
+                at = [i for i, p in enumerate(want) if lo <= p < hi]
+                got = out if len(at) == len(want) else np.empty((len(at), self.vocab_size), np.float32)
+                self._forward(seq, tokens[lo:hi], [want[i] - lo for i in at], got, wait=hi == n)
+                if at and got is not out:
+                    out[at] = got
+        except BaseException as e:
+            if seq.position != begin and not encoded_work_ran(self.ctx, e):
+                seq.position = begin
+            raise
         return out
 
     def greedy(self, seq: SequenceSlot, token: int) -> int:

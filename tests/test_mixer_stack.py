@@ -335,3 +335,93 @@ def test_trace_replay_orders_and_files(ai, tmp_path):
     a = np.fromfile(tmp_path / "0.f32", "<f4").reshape(2, 97)
     assert a.argmax(1).tolist() == [21, 5] and np.fromfile(tmp_path / "1.f32", "<f4").argmax() == 5
     assert not (tmp_path / "2.f32").exists()
+
+
+class _Batches:
+    """In place of CommandBatch: counts waits, and lets the `fault`-th report one."""
+    def __init__(self, ai, fault):
+        self.ai, self.fault, self.waits = ai, fault, 0
+
+    def __call__(self, ctx):
+        return self
+
+    def write(self, *a):
+        pass
+
+    def commit_and_wait(self):
+        self.waits += 1
+        if self.waits == self.fault:
+            raise self.ai.CommandBuffer("GPU error")
+
+
+def _pieces(ai, monkeypatch, fault, encode_fails=None):
+    """A stack pipeline in pieces of four rows whose device work is left out; the third piece may fail to encode."""
+    from local_ai_amd import stack_pipeline
+    from types import SimpleNamespace as Obj
+    batches = _Batches(ai, fault)
+    monkeypatch.setattr(stack_pipeline, "CommandBatch", batches)
+    monkeypatch.setattr(ai, "CommandBatch", batches)
+    p = object.__new__(stack_pipeline.StackPipeline)
+    p.ctx, p.kernels, p.config, p.vocab_size, p.max_rows, p.max_tokens = None, Obj(advance_position_into=lambda *a: None), Obj(width=2), 50, 4, 100
+    p.tokens_buf = p.observe = None
+    starts = []
+
+    def encode(batch, seq, n, max_position):
+        starts.append(seq.position)
+        if encode_fails is not None and len(starts) == 3:
+            raise encode_fails
+    p._encode_stack = encode
+    return p, Obj(position=10, position_buf=None), batches, starts
+
+
+def test_a_step_whose_wait_reports_a_fault_leaves_the_sequence_where_it_was(ai, monkeypatch):
+    p, seq, batches, starts = _pieces(ai, monkeypatch, fault=1)
+    with pytest.raises(ai.CommandBuffer):
+        p.step(seq, list(range(12)))
+    assert starts == [10, 14, 18] and batches.waits == 1 and seq.position == 10
+    p, seq, batches, starts = _pieces(ai, monkeypatch, fault=None)
+    p.step(seq, list(range(12)))
+    assert batches.waits == 1 and seq.position == 22                        # (a fault-free step: one wait for all pieces)
+
+
+def test_pieces_before_one_that_cannot_be_encoded_count_once_they_have_run(ai, monkeypatch):
+    p, seq, batches, starts = _pieces(ai, monkeypatch, fault=None, encode_fails=ai.InvalidArgument("no"))
+    with pytest.raises(ai.InvalidArgument):
+        p.step(seq, list(range(12)))
+    assert batches.waits == 1 and seq.position == 18
+    p, seq, batches, starts = _pieces(ai, monkeypatch, fault=1, encode_fails=ai.InvalidArgument("no"))
+    with pytest.raises(ai.InvalidArgument):
+        p.step(seq, list(range(12)))
+    assert batches.waits == 1 and seq.position == 10
+
+
+@pytest.mark.parametrize("fault,encode_fails,position", [(1, False, 5), (2, False, 9), (None, True, 11), (1, True, 5), (None, False, 12)])
+def test_chunks_of_the_quantized_decoder_count_once_they_have_run(ai, monkeypatch, fault, encode_fails, position):
+    """Tokens 5 .. 11: a chunk of three rows and a token, whose place is wanted, then a chunk of two and the last token."""
+    from local_ai_amd import generation
+    batches = _Batches(ai, fault)
+    monkeypatch.setattr(generation, "CommandBatch", batches)
+    monkeypatch.setattr(ai, "CommandBatch", batches)
+
+    class Decoder:
+        config, max_context, max_batch, ctx, position, tokens = type("C", (), {"vocab_size": 7}), 100, 8, None, 5, 0
+        logits_buf = type("B", (), {"read_into": lambda self, out: None})()
+
+        def forward_tokens_batch(self, tokens, start, batch=None):
+            assert start == self.position and batch is batches
+
+        def decode_step(self, token):
+            self.tokens += 1
+            if encode_fails and self.tokens == (1 if fault else 2):
+                raise ai.InvalidArgument("beyond the context")
+            batches.commit_and_wait()
+            self.position += 1
+    seq = Decoder()
+    model = generation.PipelineSequences(seq)
+    if position == 12:
+        model.step(seq, list(range(7)), [3])
+        assert batches.waits == 2
+    else:
+        with pytest.raises(ai.Error):
+            model.step(seq, list(range(7)), [3])
+    assert seq.position == position
