@@ -104,7 +104,8 @@ LH_API uint32_t lh_batch_dispatch_count(const lh_batch* batch);
 LH_API int lh_batch_blit_copy(lh_batch* batch, const lh_buffer* src, size_t src_offset, lh_buffer* dst,
                               size_t dst_offset, size_t len);
 /* Bytes of the host for `dst`, written in the order of the batch's dispatches; `src` may be reused on return.  Up to 2 KB travel as a
- * dispatch's arguments and up to 64 KB through staging memory, with no wait; more are copied as lh_buffer_write does.  Not while a graph is being captured. */
+ * dispatch's arguments, with no wait, and up to 64 KB through one of four staging blocks, with none but for the dispatches up to the block's
+ * last use; more are copied as lh_buffer_write does.  Not while a graph is being captured. */
 LH_API int lh_batch_write(lh_batch* batch, lh_buffer* dst, size_t offset, const void* src, size_t len);
 /* Waits for the stream.  Besides HIP errors this reports, as LH_ERR_COMMAND_BUFFER, a kernel of the batch that gave
  * up a bounded wait of its own (the split form of the TQ2_0 matvec polls an LDS word for the previous use of a ring

@@ -266,7 +266,8 @@ class CommandBatch:
                                         C.c_size_t(length)))
 
     def write(self, dst: Buffer, src, offset: int = 0) -> None:
-        """Host data for `dst` in the order of the batch's dispatches; no wait up to 64 KB."""
+        """Host data for `dst` in the order of the batch's dispatches; up to 2 KB no wait, up to 64 KB none while fewer
+        than four such writes are still to be carried out."""
         a = np.ascontiguousarray(src)
         _check(lib().lh_batch_write(self._h, dst._h, C.c_size_t(offset), C.c_void_p(a.ctypes.data), C.c_size_t(a.nbytes)))
 

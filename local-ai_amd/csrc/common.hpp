@@ -29,14 +29,15 @@ struct lh_context {
     std::vector<void*> deferred_free;
     // Graphs released while a capture is open; they go when it ends.
     std::vector<lh_graph*> deferred_graphs;
-    // Pinned staging for descriptor tables of grouped launches: a small ring of slots, each guarded by an event that is
-    // recorded behind the slot's copy, so a slot is rewritten only after the copy that read it has run.
+    // Pinned staging for descriptor tables of grouped launches and for host data of a batch: a small ring of slots, each guarded by an
+    // event that is recorded behind what reads the slot, so a slot is rewritten only after that has run.  One slot is filled at a time.
     static constexpr int kDescSlots = 4;
     static constexpr size_t kDescSlotBytes = 64 * 1024;
     void* desc_pinned;
     hipEvent_t desc_event[kDescSlots];
     bool desc_used[kDescSlots];
     unsigned desc_next;
+    std::mutex desc_mutex;
     // One word of pinned host memory that kernels can reach: a kernel that had to give up a bounded wait stores a code
     // here, and the next wait on the stream (lh_batch_commit_and_wait, lh_context_synchronize) reports it.
     uint32_t* fault_host;

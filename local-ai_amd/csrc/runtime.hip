@@ -84,11 +84,12 @@ int lh_raise_dynamic_lds(lh_context* ctx, const void* kernel, size_t bytes, cons
         if (rs__ != LH_OK) return rs__; \
     } while (0)
 
-// Puts up to kDescSlotBytes into the next slot of the pinned staging memory.  Whoever reads the slot on the stream records its event
-// behind that and marks it used.
+// Puts up to kDescSlotBytes into the next slot of the pinned staging memory.  The caller holds desc_mutex until it has launched what
+// reads the slot, recorded the slot's event behind that and marked it used.  Waits while four staged blocks are still to be read, as
+// when a prompt's fifth piece is encoded before the first has begun.
 static int stage_slot(lh_context* ctx, const void* host, size_t bytes, const char* op, unsigned& slot) {
     slot = ctx->desc_next++ % lh_context::kDescSlots;
-    if (ctx->desc_used[slot]) {   // what last read this slot must have run (it has, but for a very deep queue)
+    if (ctx->desc_used[slot]) {   // what last read this slot must have run
         const hipError_t e = hipEventSynchronize(ctx->desc_event[slot]);
         if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: %s: staging memory: %s", op, hipGetErrorString(e));
     }
@@ -101,6 +102,7 @@ int lh_upload_descriptors(lh_context* ctx, const void* host, size_t bytes, void*
     if (bytes == 0) return LH_OK;
     hipError_t e;
     if (bytes <= lh_context::kDescSlotBytes) {
+        std::lock_guard<std::mutex> lock(ctx->desc_mutex);
         unsigned slot;
         LH_TRY_STAGE(stage_slot(ctx, host, bytes, op, slot));
         e = hipMemcpyAsync(device_dst, static_cast<char*>(ctx->desc_pinned) + (size_t)slot * lh_context::kDescSlotBytes, bytes, hipMemcpyHostToDevice, ctx->stream);
@@ -493,6 +495,7 @@ int lh_batch_write(lh_batch* batch, lh_buffer* dst, size_t offset, const void* s
     if (dst->ctx == batch->ctx && len <= sizeof(SentWords<16>)) return send(SentWords<16>{});
     if (dst->ctx == batch->ctx && len <= sizeof(SentWords<512>)) return send(SentWords<512>{});
     if (dst->ctx == batch->ctx && len <= lh_context::kDescSlotBytes) {
+        std::lock_guard<std::mutex> lock(batch->ctx->desc_mutex);
         unsigned slot;
         LH_TRY_STAGE(stage_slot(batch->ctx, src, len, "batch_write", slot));
         void* from = nullptr;

@@ -204,3 +204,24 @@ def test_writes_in_stream_order(pkg, gpu, size, offset):
     for c, w in zip(copies, want):
         if offset % 16 == 0 or size % 4 == 0:
             assert np.array_equal(c.as_array(np.uint8, size), w)
+
+
+def test_writes_of_several_threads(pkg, gpu):
+    """Staged writes of threads that share a context each carry their own bytes."""
+    import threading
+    ctx, K = gpu
+    size, bad = 40000, []
+
+    def work(i):
+        g, batch, dst = np.random.default_rng(i), pkg.CommandBatch(ctx), pkg.Buffer.empty(ctx, 40000)
+        for _ in range(40):
+            src = g.integers(0, 256, size, dtype=np.uint8)
+            batch.write(dst, src)
+            if not np.array_equal(dst.as_array(np.uint8), src):
+                bad.append(i)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
