@@ -42,8 +42,9 @@ struct lh_context {
     // here, and the next wait on the stream (lh_batch_commit_and_wait, lh_context_synchronize) reports it.
     uint32_t* fault_host;
     uint32_t* fault_dev;   // the same word as the device addresses it
+    std::atomic<uint64_t> waited;   // launches that the last wait on the stream covers
     // Pinned memory through which lh_buffer_read brings what fits it to the host; one read at a time.
-    static constexpr size_t kReadBytes = (size_t)256 << 10;
+    static constexpr size_t kReadBytes = (size_t)256 << 10, kReadIdleBytes = (size_t)16 << 10;   // (see lh_buffer_read)
     void* read_host;
     void* read_dev;        // the same memory as the device addresses it
     std::mutex read_mutex;

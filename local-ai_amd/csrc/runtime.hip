@@ -57,7 +57,18 @@ int lh_fail(int code, const char* fmt, ...) {
     return code;
 }
 
+// Launches so far, of all contexts.  A context whose last wait began behind all of them has nothing to wait for; where another's launches
+// make it seem to have, a read takes a few microseconds longer.
+static std::atomic<uint64_t> g_launches{0};
+static hipError_t wait_for_stream(lh_context* ctx) {
+    const uint64_t n = g_launches.load(std::memory_order_relaxed);
+    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) ctx->waited.store(n, std::memory_order_relaxed);
+    return e;
+}
+
 int lh_check_launch(const char* what) {
+    g_launches.fetch_add(1, std::memory_order_relaxed);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: %s launch failed: %s", what, hipGetErrorString(e));
     return LH_OK;
@@ -218,6 +229,7 @@ int lh_context_create(int device_index, lh_context** out) {
         return lh_fail(LH_ERR_BUFFER_ALLOCATION, "size=%zu: pinned fault word", (size_t)64);
     }
     *ctx->fault_host = 0;
+    ctx->waited = 0;
     ctx->read_host = ctx->read_dev = nullptr;
     if (hipHostMalloc(&ctx->read_host, lh_context::kReadBytes, hipHostMallocDefault) != hipSuccess ||
         hipHostGetDevicePointer(&ctx->read_dev, ctx->read_host, 0) != hipSuccess) {
@@ -270,7 +282,7 @@ void* lh_context_stream(const lh_context* ctx) { return ctx ? (void*)ctx->stream
 int lh_context_synchronize(lh_context* ctx) {
     if (ctx && ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "context_synchronize: not while a graph is being captured");
     if (!ctx) return lh_fail(LH_ERR_INVALID_ARGUMENT, "synchronize: context is null");
-    hipError_t e = hipStreamSynchronize(ctx->stream);
+    hipError_t e = wait_for_stream(ctx);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: %s", hipGetErrorString(e));
     return lh_check_fault_word(ctx);
 }
@@ -340,7 +352,7 @@ int lh_buffer_from_bytes(lh_context* ctx, const void* src, size_t len, lh_buffer
     if (r != LH_OK) return r;
     hipError_t e = hipMemsetAsync((char*)(*out)->ptr + len, 0, 64, ctx->stream);
     if (e == hipSuccess && len) e = hipMemcpyAsync((*out)->ptr, src, len, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // src may be freed by the caller on return
+    if (e == hipSuccess) e = wait_for_stream(ctx);  // src may be freed by the caller on return
     if (e != hipSuccess) { lh_buffer_free(*out); *out = nullptr; return lh_fail(LH_ERR_BUFFER_ALLOCATION, "size=%zu: %s", len, hipGetErrorString(e)); }
     return LH_OK;
 }
@@ -393,13 +405,15 @@ int lh_buffer_write(lh_buffer* buf, size_t offset, const void* src, size_t len) 
         return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_write: range %zu+%zu exceeds %zu", offset, len, buf->len);
     if (!len) return LH_OK;
     hipError_t e = hipMemcpyAsync((char*)buf->ptr + offset, src, len, hipMemcpyHostToDevice, buf->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(buf->ctx->stream);
+    if (e == hipSuccess) e = wait_for_stream(buf->ctx);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_write: %s", hipGetErrorString(e));
     return LH_OK;
 }
 
-// Up to 256 KB a kernel writes the bytes into pinned memory and the host copies them from there: 128 KB behind a kernel 21 us until they
-// are there, through hipMemcpyAsync into memory that it has to pin first 30.  Of 1 MB the second copy takes longer than the pinning.
+// Behind work that is still to run, up to 256 KB are written into pinned memory by a kernel, and the host copies them from there: 4 KB behind a
+// kernel of 29 us are there after 31.4 us, 128 KB after 36.1; through hipMemcpyAsync, which begins when that work has ended, after 38.2 and 45.2.  (The kernel's
+// lead, 9 us, lasts at least to 512 KB; 256 KB is what a context is to hold for it.)  With nothing to wait for the copy is as good from 16 KB on, where
+// the runtime no longer copies twice: 4 KB 13.1 us with the kernel and 22.3 without, 16400 bytes 14.2 and 10.4, 128 KB 18.2 and 15.2.
 int lh_buffer_read(const lh_buffer* buf, size_t offset, void* dst, size_t len) {
     if (!buf || (!dst && len)) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_read: null argument");
     if (buf->ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_read: not while a graph is being captured");
@@ -408,19 +422,21 @@ int lh_buffer_read(const lh_buffer* buf, size_t offset, void* dst, size_t len) {
     if (!len) return LH_OK;
     lh_context* ctx = buf->ctx;
     const uint8_t* from = (const uint8_t*)buf->ptr + offset;
-    if (len <= lh_context::kReadBytes && ((uintptr_t)from & 15) == 0) {
+    const bool waiting = ctx->waited.load(std::memory_order_relaxed) != g_launches.load(std::memory_order_relaxed);
+    const bool through = len <= (waiting ? lh_context::kReadBytes : lh_context::kReadIdleBytes) && ((uintptr_t)from & 15) == 0;
+    if (through) {
         std::lock_guard<std::mutex> lock(ctx->read_mutex);
         const size_t grid = (len + 4095) / 4096;
         hipLaunchKernelGGL(read_out_kernel, dim3((uint32_t)(grid < 256 ? grid : 256)), dim3(256), 0, ctx->stream, from, (uint8_t*)ctx->read_dev, len);
         const int r = lh_check_launch("buffer_read");
         if (r != LH_OK) return r;
-        const hipError_t e = hipStreamSynchronize(ctx->stream);
+        const hipError_t e = wait_for_stream(ctx);
         if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_read: %s", hipGetErrorString(e));
         memcpy(dst, ctx->read_host, len);
         return LH_OK;
     }
     hipError_t e = hipMemcpyAsync(dst, (const char*)buf->ptr + offset, len, hipMemcpyDeviceToHost, buf->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(buf->ctx->stream);
+    if (e == hipSuccess) e = wait_for_stream(buf->ctx);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_read: %s", hipGetErrorString(e));
     return LH_OK;
 }
@@ -512,7 +528,7 @@ int lh_batch_write(lh_batch* batch, lh_buffer* dst, size_t offset, const void* s
         return LH_OK;
     }
     hipError_t e = hipMemcpyAsync(to, src, len, hipMemcpyHostToDevice, batch->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(batch->ctx->stream);
+    if (e == hipSuccess) e = wait_for_stream(batch->ctx);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: batch_write: %s", hipGetErrorString(e));
     return LH_OK;
 }
@@ -520,7 +536,7 @@ int lh_batch_write(lh_batch* batch, lh_buffer* dst, size_t offset, const void* s
 int lh_batch_commit_and_wait(lh_batch* batch) {
     if (!batch) return lh_fail(LH_ERR_INVALID_ARGUMENT, "commit_and_wait: batch is null");
     if (batch->ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "commit_and_wait: not while a graph is being captured");
-    hipError_t e = hipStreamSynchronize(batch->ctx->stream);
+    hipError_t e = wait_for_stream(batch->ctx);
     batch->dispatch_count = 0;
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: %s", hipGetErrorString(e));
     return lh_check_fault_word(batch->ctx);   // a kernel that gave up a bounded wait says so here (batch.rs:136-144: GPU errors surface at the wait)
@@ -595,6 +611,7 @@ int lh_batch_end_capture(lh_batch* batch, lh_graph** out) {
 int lh_graph_launch(lh_graph* graph) {
     if (!graph) return lh_fail(LH_ERR_INVALID_ARGUMENT, "graph_launch: graph is null");
     if (graph->ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "graph_launch: not while a graph is being captured");
+    g_launches.fetch_add(1, std::memory_order_relaxed);
     hipError_t e = hipGraphLaunch(graph->exec, graph->ctx->stream);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: graph_launch: %s", hipGetErrorString(e));
     return LH_OK;

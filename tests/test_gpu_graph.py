@@ -225,3 +225,20 @@ def test_writes_of_several_threads(pkg, gpu):
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("size", [1, 15, 4097, 16384, 16385, 131072, 262144, 262145])
+@pytest.mark.parametrize("offset", [0, 1, 4, 16])
+@pytest.mark.parametrize("behind", [False, True])
+def test_reads_of_every_route(pkg, gpu, size, offset, behind):
+    """Through pinned memory or by the runtime's copy, behind work that is still to run or with nothing to wait for: the bytes asked for, and
+    nothing around them."""
+    ctx, K = gpu
+    src = np.random.default_rng(size + offset).integers(0, 256, size + 64, dtype=np.uint8)
+    a, b, batch = pkg.Buffer.from_slice(ctx, src), pkg.Buffer.empty(ctx, size + 64), pkg.CommandBatch(ctx)
+    batch.blit_copy(a, 0, b, 0, size + 64)
+    if not behind:
+        batch.commit_and_wait()
+    out = np.full(size + 32, 7, np.uint8)
+    b.read_into(out[16:size + 16], offset)
+    assert np.array_equal(out[16:size + 16], src[offset:offset + size]) and (out[:16] == 7).all() and (out[size + 16:] == 7).all()
