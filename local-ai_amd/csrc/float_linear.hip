@@ -755,51 +755,50 @@ __global__ __launch_bounds__(256) void linear_plain_kernel(const LhLinear a) {
     constexpr int BK = 16;
     __shared__ float as[BK][64 + 4], bs[BK][64 + 4];
     const uint32_t tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const uint32_t bm = a.ex.tiles ? a.ex.tile_rows : 64u, nt_n = (a.N + 63) / 64, mt = blockIdx.x / nt_n, nt = blockIdx.x % nt_n;
-    const RowTile rt = row_tile(a, mt, bm);
+    const uint32_t nt_n = (a.N + 63) / 64, mt = blockIdx.x / nt_n, nt = blockIdx.x % nt_n;
+    const RowTile rt = row_tile(a, mt, 64);
+    if (rt.begin >= rt.end) return;
     const T* A = static_cast<const T*>(a.A);
     const uint16_t* W = a.W + (size_t)rt.expert * a.N * a.K;
     const uint32_t n0 = nt * 64, K = a.K, pos0 = a.seg.position ? *a.seg.position : 0u;
-    for (uint32_t begin = rt.begin; begin < rt.end; begin += 64) {
-        float acc[4][4] = {};
-        for (uint32_t k0 = 0; k0 < K; k0 += BK) {
-            for (uint32_t e = tid; e < 64 * BK; e += 256) {
-                const uint32_t r = e >> 4, k = k0 + (e & 15);
-                const bool ka = k < K;
-                as[e & 15][r] = ka && begin + r < rt.end ? lh_ld(A, (size_t)a_row(a, begin + r) * a.lda + k) : 0.0f;
-                bs[e & 15][r] = ka && n0 + r < a.N ? lh_bf2f(W[(size_t)(n0 + r) * K + k]) : 0.0f;
+    float acc[4][4] = {};
+    for (uint32_t k0 = 0; k0 < K; k0 += BK) {
+        for (uint32_t e = tid; e < 64 * BK; e += 256) {
+            const uint32_t r = e >> 4, k = k0 + (e & 15);
+            const bool ka = k < K;
+            as[e & 15][r] = ka && rt.begin + r < rt.end ? lh_ld(A, (size_t)a_row(a, rt.begin + r) * a.lda + k) : 0.0f;
+            bs[e & 15][r] = ka && n0 + r < a.N ? lh_bf2f(W[(size_t)(n0 + r) * K + k]) : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < BK; k++) {
+            float x[4], w[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) { x[i] = as[k][ty * 4 + i]; w[i] = bs[k][tx * 4 + i]; }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i][j] = __builtin_fmaf(x[i], w[j], acc[i][j]);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t slot = rt.begin + ty * 4 + i;
+        if (slot >= rt.end) continue;
+        const OutRow o = out_row(a, slot);
+        if (a.seg.pairs) {                                // (an expert's weight and a bias do not occur with pairs of a plain product)
+#pragma unroll
+            for (int j = 0; j < 4; j += 2) {
+                const uint32_t n = n0 + tx * 4 + j;
+                if (n < a.N) lh_segment_store_pair(a.seg, o.row, n, acc[i][j] + (a.bias ? a.bias[n] : 0.0f), acc[i][j + 1] + (a.bias ? a.bias[n + 1] : 0.0f), pos0);
             }
-            __syncthreads();
-#pragma unroll
-            for (int k = 0; k < BK; k++) {
-                float x[4], w[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) { x[i] = as[k][ty * 4 + i]; w[i] = bs[k][tx * 4 + i]; }
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) acc[i][j] = __builtin_fmaf(x[i], w[j], acc[i][j]);
-            }
-            __syncthreads();
+            continue;
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t slot = begin + ty * 4 + i;
-            if (slot >= rt.end) continue;
-            const OutRow o = out_row(a, slot);
-            if (a.seg.pairs) {                                // (an expert's weight and a bias do not occur with pairs of a plain product)
-#pragma unroll
-                for (int j = 0; j < 4; j += 2) {
-                    const uint32_t n = n0 + tx * 4 + j;
-                    if (n < a.N) lh_segment_store_pair(a.seg, o.row, n, acc[i][j] + (a.bias ? a.bias[n] : 0.0f), acc[i][j + 1] + (a.bias ? a.bias[n + 1] : 0.0f), pos0);
-                }
-                continue;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t n = n0 + tx * 4 + j;
-                if (n < a.N) lh_segment_store(a.seg, o.row, n, acc[i][j] * o.weight + (a.bias ? a.bias[n] : 0.0f), pos0);
-            }
+        for (int j = 0; j < 4; j++) {
+            const uint32_t n = n0 + tx * 4 + j;
+            if (n < a.N) lh_segment_store(a.seg, o.row, n, acc[i][j] * o.weight + (a.bias ? a.bias[n] : 0.0f), pos0);
         }
     }
 }
@@ -1245,7 +1244,8 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     }
     const bool mfma = !a.a_f32 && a.K % 8 == 0 && a.lda % 8 == 0 && (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0;
     if (!mfma) {
-        const uint64_t mt = a.ex.tiles ? a.ex.n_tiles : ((uint64_t)a.M + 63) / 64, grid = mt * ((a.N + 63) / 64);
+        // (a workgroup for every 64 rows of an expert's tile: 1030 -> 512 columns, 1024 rows with two of 8 experts, 128 rows a workgroup 325 us, 256 637, now 180)
+        const uint64_t mt = a.ex.tiles ? (uint64_t)a.ex.n_tiles * (a.ex.tile_rows / 64) : ((uint64_t)a.M + 63) / 64, grid = mt * ((a.N + 63) / 64);
         LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: %u x %u outputs", op, a.M, a.N);
         if (grid == 0) return LH_OK;
         if (a.a_f32) hipLaunchKernelGGL((linear_plain_kernel<float>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a);
