@@ -1228,6 +1228,39 @@ static int launch_phased(lh_context* ctx, const LhLinear& a, uint64_t grid, cons
     return r == LH_OK ? lh_check_launch(op) : r;
 }
 
+// The forms for the tiles of an expert plan, and what one is expected to take in microseconds: `start`, `step` for each 64 columns of k and, for
+// every further tile a CU has, `round` and `round_step`; in each round `through` where a lane cannot store its `lanes` columns as they are, and
+// `wide` for f32 results; `empty` for each round of tiles without rows, and `weights` for each 4 MB of them.  Fitted to 982 products (up to
+// 4096 rows, 8192 columns and 128 experts), of which a form's times lie within 10 to 19 % (r.m.s.), then weighed against each other: the choice
+// takes 2 % longer than the best form would, 64 x 64 for all 11 %.  Two of 16 experts a row, 2048 -> 1024 columns: 200 rows 18 us (64 x 64; 64 x 32
+// tiles that share out k 23), 4096 rows 45 (256 x 256; 128 x 128 of four waves 60).
+struct PlanForm {
+    uint32_t bm, bn, lanes;
+    bool phased;
+    float start, step, round, round_step, through, wide, empty, weights;
+    int (*launch)(lh_context*, const LhLinear&, uint64_t, const char*);
+};
+static const PlanForm kPlanForms[] = {
+    {256, 256, 16, true, 5.71f, 0.893f, 0.0f, 1.4f, 2.7f, 17.7f, 43.3f, 0.0f, launch_phased<256, 256>},
+    {256, 128, 16, true, 5.21f, 0.698f, 3.34f, 0.852f, 3.0f, 11.3f, 20.4f, 0.089f, launch_phased<256, 128>},
+    {128, 128, 16, true, 6.33f, 0.471f, 4.33f, 0.557f, 2.75f, 6.49f, 9.79f, 0.0858f, launch_phased<128, 128>},
+    {128, 128, 16, false, 4.58f, 0.6f, 0.242f, 0.375f, 6.51f, 4.51f, 11.7f, 0.0f, launch_mfma<128, 128, 2>},
+    {64, 64, 8, false, 4.09f, 0.328f, 1.0f, 0.162f, 1.4f, 0.7f, 1.7f, 0.089f, launch_mfma<64, 64, 3>},
+    {32, 32, 4, false, 4.12f, 0.066f, 1.37f, 0.076f, 0.5f, 0.4f, 1.1f, 0.324f, launch_sliced<32, 32, 2>},
+    {32, 32, 4, false, 3.89f, 0.223f, 0.514f, 0.0977f, 0.0735f, 0.263f, 0.735f, 0.338f, launch_mfma<32, 32, 4>},
+};
+static float plan_time(const PlanForm& f, const LhLinear& a, uint64_t steps, uint64_t tiles, uint64_t cus) {
+    // A plan has one tile more for each expert than can be full.  Every expert that is chosen has one with rows, and of the last ones about half.
+    const uint64_t used = std::min(a.ex.slots, a.ex.experts);
+    const uint64_t filled = std::max<uint64_t>(used, a.ex.slots / f.bm + a.ex.experts / 2) * ((a.N + f.bn - 1) / f.bn);
+    // Tiles without rows lie between them, so that a CU has one more than its share now and then: a tenth more of the large ones.
+    const uint64_t spread = f.bm >= 128 ? filled * 11 / 10 : filled;
+    const float rounds = (float)((spread + cus - 1) / cus), s = (float)steps, mb = (float)used * (float)a.N * (float)a.K * 2e-6f;
+    return f.start + f.step * s + (rounds - 1) * (f.round + f.round_step * s) +
+           rounds * ((epilogue_of(a.seg, f.lanes) == kThroughLds ? f.through : 0.0f) + (a.seg.f32[0] ? f.wide : 0.0f)) +
+           (tiles > filled ? f.empty * (float)(tiles - filled) / (float)cus : 0.0f) + f.weights * mb / 4;
+}
+
 int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     LhLinear a = given;
     if (a.lda == 0) a.lda = a.K;
@@ -1252,45 +1285,56 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
         else hipLaunchKernelGGL((linear_plain_kernel<uint16_t>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a);
         return lh_check_launch(op);
     }
-    const uint64_t want = (uint64_t)ctx->cu_count, steps = (uint64_t)a.K / 64 * a.parts;
+    const uint64_t want = (uint64_t)ctx->cu_count, steps = ((uint64_t)a.K + 63) / 64 * a.parts;
     auto tiles = [&](uint32_t bm, uint32_t bn) {
         return (a.ex.tiles ? (uint64_t)a.ex.n_tiles * (a.ex.tile_rows / bm) : ((uint64_t)a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
     };
     // Byte offsets of the phased kernels are 32 bits wide.
     const uint64_t a_bytes = (uint64_t)a_rows * a.lda * 2, w_bytes = (uint64_t)a.N * a.K * 2;
     const bool phased = a.K % 64 == 0 && a_bytes < (1ull << 32) && w_bytes < (1ull << 32);
-    // Of an expert plan about half the experts' last tiles count: the plan has one more for each than can be full.
-    auto filled = [&](uint32_t bm, uint32_t bn) {
-        return a.ex.tiles ? ((uint64_t)a.ex.slots / bm + a.ex.experts / 2 + 1) * ((a.N + bn - 1) / bn) : tiles(bm, bn);
-    };
-    if (phased && a.ex.tile_rows % 128 == 0 && 4 * filled(128, 128) >= 3 * want) {
+    if (a.ex.tiles) {
+        const PlanForm* best = nullptr;
+        float least = INFINITY;
+        for (const PlanForm& f : kPlanForms) {
+            if ((f.phased && !phased) || a.ex.tile_rows < f.bm) continue;
+            const float t = plan_time(f, a, steps, tiles(f.bm, f.bn), want);
+            if (t < least) { least = t; best = &f; }
+        }
+        return best->launch(ctx, a, tiles(best->bm, best->bn), op);
+    }
+    if (phased && 4 * tiles(128, 128) >= 3 * want) {
         // One workgroup fits a CU, so a launch takes whole rounds of them, and the form is the one whose rounds are the shortest.  A
         // round's time in nanoseconds, measured with 64 columns of k per step: 256 x 256 9000 + 1650 per step, 256 x 128 8000 + 800,
         // 128 x 128 7000 + 520.  Before / now, bf16 results: 2048 x 2048 x 8192 85 / 60 us (256 x 256; the matrix cores alone would take
         // 28 at 2.4 GHz; on random data the clock is 1.5 to 1.8 GHz and they are busy for 70 % of the cycles of such launches), 2048 x 2048 x 4096 39 / 34 and 2048 x 2048 x 3072 35 / 28
         // (256 x 128), 2048 x 8192 x 2048 90 / 74 (128 x 128).  With fewer than three tiles of 128 x 128 to four CUs the small tiles
         // win: 128 of them (953 x 2048 x 2048) 22 us against 18.
-        // The experts of a mixture, 4096 slots of 16: from 2048 to 1024 columns 42 -> 39.5 us (256 x 128), back 54 -> 48 (256 x 256; 60 with 256 x 128; both were on 128 x 128 tiles of four
-        // waves, whose last round is short of tiles).
-        auto rounds = [&](uint32_t bm, uint32_t bn) { return a.ex.tiles && a.ex.tile_rows < bm ? 1u << 20 : (filled(bm, bn) + want - 1) / want; };
+        auto rounds = [&](uint32_t bm, uint32_t bn) { return (tiles(bm, bn) + want - 1) / want; };
         const uint64_t t256 = rounds(256, 256) * (9000 + 1650 * steps), t384 = rounds(256, 128) * (8000 + 800 * steps), t128 = rounds(128, 128) * (7000 + 520 * steps);
         if (t256 <= t384 && t256 <= t128) return launch_phased<256, 256>(ctx, a, tiles(256, 256), op);
         if (t384 <= t128) return launch_phased<256, 128>(ctx, a, tiles(256, 128), op);
         return launch_phased<128, 128>(ctx, a, tiles(128, 128), op);
     }
-    if (a.ex.tile_rows % 128 == 0 && filled(128, 128) >= 2 * want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
-    // The rest by its expected time in nanoseconds, measured: 64 x 64 tiles of shared waves, up to three workgroups a CU; or waves that
-    // share out k, on 64 x 32 tiles (one workgroup a CU) or 32 x 32 (two).  Before / now, weights in the memory-side cache: 512 x 1024 x 4096 25.5 / 12.5 us
-    // and 200 x 2048 x 8192 46.7 / 19.2 (64 x 32), 512 x 1024 x 1024 9.6 / 6.5, 2048 x 16 x 2048 14.0 / 6.0 and 256 x 1024 x 4096 25.2 / 9.4
-    // (32 x 32), 953 x 2048 x 2048 21 / 17.9 and 300 x 6144 x 1536 19.5 / 15.3 (64 x 64, from 128 x 64), 333 x 1024 x 1024 with f32
-    // activations 20.3 / 9.6.
-    const uint64_t n64 = filled(64, 64), n32 = filled(32, 32);
-    const uint64_t t64 = n64 <= want ? 4000 + 345 * steps : n64 <= 2 * want ? 4600 + 430 * steps : (n64 + 3 * want - 1) / (3 * want) * (5000 + 600 * steps);
-    const uint64_t t64_32 = 1000 + (filled(64, 32) + want - 1) / want * (3500 + 100 * steps);
-    const uint64_t t32 = n32 <= want ? 4000 + 75 * steps : 1000 + (n32 + 2 * want - 1) / (2 * want) * (3500 + 150 * steps);
-    if (t64 <= t64_32 && t64 <= t32) return launch_mfma<64, 64, 3>(ctx, a, tiles(64, 64), op);
-    if (t64_32 <= t32) return launch_sliced<64, 32, 3>(ctx, a, tiles(64, 32), op);
-    return launch_sliced<32, 32, 2>(ctx, a, tiles(32, 32), op);
+    if (tiles(128, 128) >= 2 * want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
+    // The rest by its expected time in nanoseconds, measured: 64 x 64 or 32 x 32 tiles of shared waves, up to three or five workgroups a CU;
+    // waves that share out k, on 64 x 32 tiles (one workgroup a CU) or 32 x 32 (two); or 128 x 128 tiles of shared waves, where there is more than one a
+    // CU.  A lane that cannot store its columns as they are (bf16 rows that are no multiple of 16 bytes) costs the more the larger the tile.  Before / now,
+    // weights in the memory-side cache: 512 x 1024 x 4096 25.5 / 12.5 us and 200 x 2048 x 8192 46.7 / 19.2 (64 x 32), 512 x 1024 x 1024 9.6 / 6.5, 2048 x 16 x 2048 14.0 / 6.0
+    // and 256 x 1024 x 4096 25.2 / 9.4 (32 x 32, shared-out k), 953 x 2048 x 2048 21 / 17.9 and 300 x 6144 x 1536 19.5 / 15.3 (64 x 64, from 128 x 64), 333 x 1024 x 1024
+    // with f32 activations 20.3 / 9.6; short k: 287 x 1444 x 176 7.5 / 5.1, 25 x 620 x 136 5.2 / 4.7 (32 x 32, shared waves); ragged k: 3893 x 1504 x 4568 120 / 82 (128 x 128).
+    const uint64_t n64 = tiles(64, 64), n32 = tiles(32, 32), n128 = tiles(128, 128);
+    auto through = [&](uint32_t lanes, uint64_t t) { return epilogue_of(a.seg, lanes) == kThroughLds ? t : 0; };
+    auto per_cu = [&](uint64_t n) { return (n + want - 1) / want; };
+    const uint64_t t64 = (n64 <= want ? 4000 + 345 * steps : n64 <= 2 * want ? 4600 + 430 * steps : n64 <= 3 * want ? 5600 + 590 * steps : per_cu(n64) * (2100 + 190 * steps)) + through(8, 1700);
+    const uint64_t t64_32 = 1000 + per_cu(tiles(64, 32)) * (3500 + 100 * steps) + through(4, 900);
+    const uint64_t t32 = (n32 <= want ? 4000 + 75 * steps : 1000 + (n32 + 2 * want - 1) / (2 * want) * (3500 + 150 * steps)) + through(4, 700);
+    const uint64_t t32_shared = (n32 <= want ? 3700 + 240 * steps : n32 <= 2 * want ? 3900 + 280 * steps : n32 <= 3 * want ? 4300 + 360 * steps : per_cu(n32) * (1100 + 92 * steps)) + through(4, 200);
+    const uint64_t t128 = n128 > want ? 8000 + 870 * steps + through(16, 11000) : UINT64_MAX;
+    const uint64_t least = std::min({t64, t64_32, t32, t32_shared, t128});
+    if (t128 == least) return launch_mfma<128, 128, 2>(ctx, a, n128, op);
+    if (t64 == least) return launch_mfma<64, 64, 3>(ctx, a, n64, op);
+    if (t64_32 == least) return launch_sliced<64, 32, 3>(ctx, a, tiles(64, 32), op);
+    return t32 == least ? launch_sliced<32, 32, 2>(ctx, a, n32, op) : launch_mfma<32, 32, 4>(ctx, a, n32, op);
 }
 
 extern "C" {
