@@ -58,12 +58,13 @@ __global__ __launch_bounds__(256) void route_kernel(const float* __restrict__ lo
 }
 
 // A thread takes neighbouring slots, so that one scan over the workgroup orders them.  (256 slots at a time, with two barriers each: 16 us
-// for 4096 slots of 16 experts; now 6.)
-constexpr uint32_t kPlaceThreads = 1024;
-__global__ __launch_bounds__(kPlaceThreads) void place_kernel(uint32_t* __restrict__ plan, uint32_t rows, uint32_t experts, uint32_t top, uint32_t tile) {
-    __shared__ uint32_t less[kPlaceThreads / 64], same[kPlaceThreads / 64];
+// for 4096 slots of 16 experts; now 6.)  THREADS: 256 up to 256 slots, where what takes the time is to begin and end (128 slots, with the
+// routing before it, 5.8 us; 1024 threads 6.0).
+template <uint32_t THREADS>
+__global__ __launch_bounds__(THREADS) void place_kernel(uint32_t* __restrict__ plan, uint32_t rows, uint32_t experts, uint32_t top, uint32_t tile) {
+    __shared__ uint32_t less[THREADS / 64], same[THREADS / 64];
     const uint32_t e = blockIdx.x, S = rows * top, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t per = (S + kPlaceThreads - 1) / kPlaceThreads, i0 = min(threadIdx.x * per, S), i1 = min(i0 + per, S);
+    const uint32_t per = (S + THREADS - 1) / THREADS, i0 = min(threadIdx.x * per, S), i1 = min(i0 + per, S);
     uint32_t nl = 0, ns = 0;
 #pragma unroll 4
     for (uint32_t i = i0; i < i1; i++) { const uint32_t x = plan[i]; nl += x < e; ns += x == e; }
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(uint32_t* __restri
     __syncthreads();
     uint32_t base = 0, count = 0, before = 0;
 #pragma unroll
-    for (uint32_t w = 0; w < kPlaceThreads / 64; w++) {
+    for (uint32_t w = 0; w < THREADS / 64; w++) {
         base += less[w];
         before += w < wave ? same[w] : 0u;
         count += same[w];
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(uint32_t* __restri
         }
     // expert e's tiles start at base / tile + e: there is always room for its ceil(count / tile) before the next expert's
     const uint32_t t0 = base / tile + e, t1 = (base + count) / tile + e + 1;
-    for (uint32_t t = t0 + threadIdx.x; t < t1; t += kPlaceThreads) {
+    for (uint32_t t = t0 + threadIdx.x; t < t1; t += THREADS) {
         const uint32_t b = min(base + (t - t0) * tile, base + count);
         uint32_t* w = plan + 5 * S + 3 * t;
         w[0] = e; w[1] = b; w[2] = min(b + tile, base + count);
@@ -313,7 +314,8 @@ int lh_moe_route_into(lh_batch* batch, const lh_buffer* logits, lh_buffer* plan,
     LH_NEED(plan, (size_t)lh_moe_plan_words(rows, experts, top) * 4, op, "plan");
     hipLaunchKernelGGL(route_kernel, dim3((rows + 3) / 4), dim3(256), 0, batch->ctx->stream, (const float*)logits->ptr, (uint32_t*)plan->ptr, rows, experts, top);
     LH_TRY(lh_check_launch(op));
-    hipLaunchKernelGGL(place_kernel, dim3(experts), dim3(kPlaceThreads), 0, batch->ctx->stream, (uint32_t*)plan->ptr, rows, experts, top,
+    const bool few = rows * top <= 256;
+    hipLaunchKernelGGL((few ? place_kernel<256> : place_kernel<1024>), dim3(experts), dim3(few ? 256 : 1024), 0, batch->ctx->stream, (uint32_t*)plan->ptr, rows, experts, top,
                        lh_expert_tile_rows(rows * top, experts));
     LH_TRY(lh_check_launch(op));
     batch->dispatch_count += 2;
