@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256) void softcap_kernel(float* x, size_t n, float 
 __global__ void advance_position_kernel(uint32_t* position, uint32_t by) { *position += by; }
 
 // Index of the largest value of each row; `position`, if there is one, moves on behind it (a launch of its own for that: 2.5 us of a
-// token's chain).  What the threads find meets in one wave, behind one barrier: 5.1 us for 32000 values, with the position or without.
+// token's chain).
 __global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restrict__ x, uint32_t* __restrict__ index, uint32_t n, uint32_t* position, uint32_t by) {
     __shared__ float sv[1024];
     __shared__ uint32_t si[1024];
@@ -228,22 +228,16 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restri
     }
     sv[threadIdx.x] = best; si[threadIdx.x] = at;
     __syncthreads();
-    if (threadIdx.x >= 64) return;
-    struct Found { float v; uint32_t i; };
-    auto better = [](const Found& a, const Found& b) {
-        return b.i != 0xFFFFFFFFu && (a.i == 0xFFFFFFFFu || b.v > a.v || (b.v == a.v && b.i < a.i)) ? b : a;
-    };
-    Found f[16];
-#pragma unroll
-    for (uint32_t j = 0; j < 16; j++) f[j] = Found{sv[j * 64 + threadIdx.x], si[j * 64 + threadIdx.x]};
-#pragma unroll
-    for (uint32_t h = 8; h > 0; h >>= 1)
-#pragma unroll
-        for (uint32_t j = 0; j < h; j++) f[j] = better(f[j], f[j + h]);
-#pragma unroll
-    for (uint32_t h = 32; h > 0; h >>= 1) f[0] = better(f[0], Found{__shfl_down(f[0].v, h, 64), (uint32_t)__shfl_down((int)f[0].i, h, 64)});
+    for (uint32_t h = 512; h > 0; h >>= 1) {
+        if (threadIdx.x < h) {
+            const float v = sv[threadIdx.x + h];
+            const uint32_t i = si[threadIdx.x + h];
+            if (i != 0xFFFFFFFFu && (si[threadIdx.x] == 0xFFFFFFFFu || v > sv[threadIdx.x] || (v == sv[threadIdx.x] && i < si[threadIdx.x]))) { sv[threadIdx.x] = v; si[threadIdx.x] = i; }
+        }
+        __syncthreads();
+    }
     if (threadIdx.x != 0) return;
-    index[blockIdx.x] = f[0].i;
+    index[blockIdx.x] = si[0];
     if (position) *position += by;
 }
 
