@@ -378,15 +378,19 @@ int lh_gated_norm_rows_into(lh_batch* batch, const lh_buffer* input, const lh_bu
     if (group % 4 == 0 && group <= 4096 && (at & 15) == 0 && items < 0x7FFFFFFFull) {
         uint32_t threads = 8;
         while (threads < 64 && threads * 4 < group) threads *= 2;
-        const bool block = group > 256;
-        const uint32_t q = block ? (group + 1023) / 1024 : 1u, grid = block ? rows : (uint32_t)((items + 256 / threads - 1) / (256 / threads));
+        // Four parts and more a row, of up to 1024 columns: a wave each, four at a time (2048 rows of eight parts of 512: a workgroup one after the
+        // other 23.9 us, before these pieces 18.4, now 14.4).
+        const bool block = group > (dim / group >= 4 ? 1024u : 256u);
+        const uint32_t q = block ? (group + 1023) / 1024 : (group + 255) / 256, grid = block ? rows : (uint32_t)((items + 256 / threads - 1) / (256 / threads));
 #define LH_PIECES(T, Q, B)                                                                                                                              \
         hipLaunchKernelGGL((gated_norm_pieces_kernel<T, Q, B>), dim3(grid), dim3(256), 0, batch->ctx->stream, (const float*)input->ptr, (const T*)gate->ptr, \
                            weight ? (const float*)weight->ptr : nullptr, (T*)output->ptr, (uint32_t)items, dim, group, B ? 256u : threads, gate_act,    \
                            gate_first ? 1u : 0u, eps)
 #define LH_PIECES_OF(T)                                                                                                                                 \
         do {                                                                                                                                            \
-            if (!block) LH_PIECES(T, 1, false);                                                                                                         \
+            if (!block && q == 1) LH_PIECES(T, 1, false);                                                                                               \
+            else if (!block && q == 2) LH_PIECES(T, 2, false);                                                                                          \
+            else if (!block) LH_PIECES(T, 4, false);                                                                                                    \
             else if (q == 1) LH_PIECES(T, 1, true);                                                                                                     \
             else if (q == 2) LH_PIECES(T, 2, true);                                                                                                     \
             else LH_PIECES(T, 4, true);                                                                                                                 \

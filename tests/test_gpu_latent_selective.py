@@ -434,7 +434,7 @@ def test_destinations_of_mixed_types(ai, gpu):
 
 
 @pytest.mark.parametrize("first", [0, 1])
-@pytest.mark.parametrize("rows,dim,group", [(1, 4, 4), (37, 72, 36), (5, 256, 128), (9, 800, 200), (3, 512, 256), (2, 520, 260), (4, 1024, 1024), (3, 2056, 1028), (2, 4096, 4096),
+@pytest.mark.parametrize("rows,dim,group", [(1, 4, 4), (37, 72, 36), (5, 256, 128), (9, 800, 200), (3, 512, 256), (2, 520, 260), (4, 1024, 1024), (3, 2056, 1028), (2, 4096, 4096), (5, 1200, 300), (3, 3216, 804), (2, 6144, 1024),
                                             (2, 3000, 3000), (2, 4100, 4100), (3, 12288, 4096), (70, 33, 11)])
 def test_gated_norm_parts(ai, gpu, rows, dim, group, first):
     """Parts on a few lanes of a wave, on a workgroup, and those that are not made of whole pieces; with a weight and without."""
