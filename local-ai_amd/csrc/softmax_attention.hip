@@ -377,7 +377,9 @@ int launch_mfma(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const 
         a.splits = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(std::max(std::min<uint64_t>(cus / groups, max_blocks / (4 * NB)),
                                                                                std::min<uint64_t>(2 * cus / groups, max_blocks / (8 * NB))), room));
         LH_REQUIRE(groups * a.splits < 0x7FFFFFFFull, "%s: %u rows", op, a.rows);
-        a.resident = (uint32_t)cus;
+        // (one workgroup fits a CU where the sums of two maps take its registers: the longest first there, 2048 rows of 16 heads of 128 and 256
+        // columns 188 us; in the order for two a CU 230)
+        a.resident = MAPS * DV <= 256 ? (uint32_t)cus : UINT32_MAX;
         hipLaunchKernelGGL((attention_tile_kernel<DQ, DV, MAPS, NB, G>), dim3((uint32_t)(groups * a.splits)), dim3(256 * G), 0, ctx->stream, a);
         const int r = lh_check_launch(op);
         return r != LH_OK || a.splits == 1 ? r : merge();

@@ -21,7 +21,7 @@ struct AttentionArgs {
     float* partial;            // records [16-row tile][kv head][split][map][16] of dv unnormalised sums, maximum, sum of weights
     uint32_t splits;
     uint32_t parts;            // workgroups that share a row's columns in the merge (one map)
-    uint32_t resident;         // tiles: workgroups of a launch before any CU has two
+    uint32_t resident;         // tiles: workgroups of a launch before any CU has two (none has: all of them)
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
