@@ -819,7 +819,8 @@ LH_API int lh_selective_step_into(lh_batch* batch, const lh_buffer* input, lh_bu
 /* Mixture of experts: scores = sigmoid(router logits), each row takes the `top` largest (ties: the lower index), scaled
  * by the score itself on the way into the expert.  Experts are stacked, up [experts, ff, width]
  * and down [experts, width, ff], without biases.
- *   route   logits f32 [rows, experts] -> the rows grouped by expert: plan u32 [lh_moe_plan_words]
+ *   route   logits f32 [rows, experts] -> the rows grouped by expert: plan u32 [lh_moe_plan_words]; what is enough for some
+ *           rows is enough for fewer
  *   up      hidden[slot] = act(w * (up[e] . input[row])), one slot per (row, choice), in plan order
  *   down    residual[row] += sum over the row's slots of down[e] . hidden[slot]
  *   vector  both for one row: the selection is done by every workgroup from the logits; `input` is normed as in

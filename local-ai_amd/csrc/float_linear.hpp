@@ -5,7 +5,7 @@
 // Rows of an expert product: the plan's tiles (see float_moe.hip), each `tile_rows` plan slots of one expert.
 struct LhExpertRows {
     const uint32_t* tiles;          // null: an ordinary product.  [n_tiles][3]: expert, first slot, one past the last slot
-    uint32_t n_tiles, tile_rows;    // 64 or 128
+    uint32_t n_tiles, tile_rows;    // 64, 128 or 256
     const uint32_t* slot_row;       // slot -> row of the activations
     const float* slot_weight;       // slot -> weight of the expert's input (null: 1)
     uint32_t gather;                // activations are indexed by slot_row (else by the slot itself)

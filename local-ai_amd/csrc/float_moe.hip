@@ -274,6 +274,7 @@ int check_shape(const char* op, uint32_t rows, uint32_t experts, uint32_t top) {
     return LH_OK;
 }
 uint32_t plan_tiles(uint32_t slots, uint32_t experts) { return slots / lh_expert_tile_rows(slots, experts) + experts; }
+size_t plan_bytes(uint32_t rows, uint32_t experts, uint32_t top) { return ((size_t)5 * rows * top + (size_t)3 * plan_tiles(rows * top, experts)) * 4; }
 
 void expert_rows(LhExpertRows& x, const lh_buffer* plan, uint32_t rows, uint32_t experts, uint32_t top) {
     const uint32_t S = rows * top;
@@ -302,7 +303,7 @@ extern "C" {
 
 uint32_t lh_moe_plan_words(uint32_t rows, uint32_t experts, uint32_t top) {
     const uint32_t S = rows * top;
-    return 5 * S + 3 * plan_tiles(S, experts);
+    return 5 * S + 3 * (S / 64 + experts);                    // with the smallest tiles: what is enough for `rows` is enough for fewer
 }
 
 int lh_moe_route_into(lh_batch* batch, const lh_buffer* logits, lh_buffer* plan, uint32_t rows, uint32_t experts, uint32_t top) {
@@ -311,7 +312,7 @@ int lh_moe_route_into(lh_batch* batch, const lh_buffer* logits, lh_buffer* plan,
     LH_TRY(check_shape(op, rows, experts, top));
     if (rows == 0) return LH_OK;
     LH_NEED(logits, (size_t)rows * experts * 4, op, "logits");
-    LH_NEED(plan, (size_t)lh_moe_plan_words(rows, experts, top) * 4, op, "plan");
+    LH_NEED(plan, plan_bytes(rows, experts, top), op, "plan");
     hipLaunchKernelGGL(route_kernel, dim3((rows + 3) / 4), dim3(256), 0, batch->ctx->stream, (const float*)logits->ptr, (uint32_t*)plan->ptr, rows, experts, top);
     LH_TRY(lh_check_launch(op));
     const bool few = rows * top <= 256;
@@ -332,7 +333,7 @@ int lh_moe_up_into(lh_batch* batch, const lh_buffer* input, int dtype, const lh_
     if (rows == 0) return LH_OK;
     const size_t es = dtype == LH_F32 ? 4 : 2;
     LH_NEED(input, (size_t)rows * width * es, op, "input");
-    LH_NEED(plan, (size_t)lh_moe_plan_words(rows, experts, top) * 4, op, "plan");
+    LH_NEED(plan, plan_bytes(rows, experts, top), op, "plan");
     LH_NEED(up, (size_t)experts * ff * width * 2, op, "up");
     LH_NEED(hidden, (size_t)rows * top * ff * es, op, "hidden");
     LhLinear a;
@@ -360,7 +361,7 @@ int lh_moe_down_into(lh_batch* batch, const lh_buffer* hidden, int dtype, const 
     if (rows == 0) return LH_OK;
     const size_t es = dtype == LH_F32 ? 4 : 2;
     LH_NEED(hidden, (size_t)rows * top * ff * es, op, "hidden");
-    LH_NEED(plan, (size_t)lh_moe_plan_words(rows, experts, top) * 4, op, "plan");
+    LH_NEED(plan, plan_bytes(rows, experts, top), op, "plan");
     LH_NEED(down, (size_t)experts * ff * width * 2, op, "down");
     LH_NEED(residual, (size_t)rows * width * 4, op, "residual");
     const bool direct = top == 1;                            // one slot per row: add it where it belongs

@@ -425,3 +425,18 @@ def test_chunks_of_the_quantized_decoder_count_once_they_have_run(ai, monkeypatc
         with pytest.raises(ai.Error):
             model.step(seq, list(range(7)), [3])
     assert seq.position == position
+
+
+@pytest.mark.parametrize("experts,top", [(1, 1), (16, 2), (64, 4), (7, 3), (300, 8)])
+def test_a_plan_for_some_rows_is_enough_for_fewer(ai, experts, top):
+    """Also where the rows of a plan's tiles change."""
+    words = [ai.lib().lh_moe_plan_words(ai._u32(r), ai._u32(experts), ai._u32(top)) for r in range(1, 6000)]
+    assert all(a <= b for a, b in zip(words, words[1:])) and words[99] >= 5 * 100 * top + 3 * experts
+
+
+@pytest.mark.parametrize("heads,dim,vdim", [(16, 128, 128), (1, 32, 64), (300, 64, 64), (4, 200, 33)])
+def test_a_workspace_for_some_rows_is_enough_for_fewer(ai, heads, dim, vdim):
+    """Also where chunks change from 64 rows to 128; never less than chunks of 128 need."""
+    size = [ai.lib().lh_linear_attention_workspace_bytes(ai._u32(r), ai._u32(heads), ai._u32(dim), ai._u32(vdim)) for r in range(1, 6000)]
+    each = heads * vdim * ai.lib().lh_linear_attention_padded_dim(ai._u32(dim)) * 4
+    assert all(a <= b for a, b in zip(size, size[1:])) and all(s >= -(-r // 128) * each for r, s in enumerate(size, 1))
