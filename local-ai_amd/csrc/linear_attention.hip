@@ -464,10 +464,11 @@ __global__ __launch_bounds__(256, DQ <= 64 ? 3 : DQ <= 128 ? 2 : 1) void chunk_o
         }
         __syncthreads();
         if (!on) continue;
+        // (the small terms of all columns first: the large ones are then rounded once a product, not with each of their remainders as well)
 #pragma unroll
-        for (int i = 0; i < KB / 32; i++)
+        for (int z = 2; z >= 0; z--)
 #pragma unroll
-            for (int z = 2; z >= 0; z--) {
+            for (int i = 0; i < KB / 32; i++) {
                 lh_bf16x8 sf[4];
 #pragma unroll
                 for (int d = 0; d < 4; d++) sf[d] = __builtin_bit_cast(lh_bf16x8, terms[z][d][i][lane]);
@@ -542,10 +543,14 @@ __global__ __launch_bounds__(256, DQ <= 64 ? 3 : DQ <= 128 ? 2 : 1) void chunk_o
                 }
                 split3_pair(e[0], e[1], p[0][j], p[1][j], p[2][j]);
             }
+            // (a sum of its own for these rows: what was added up before is rounded once for them, not with each term)
 #pragma unroll
-            for (int z = 2; z >= 0; z--)
-#pragma unroll
-                for (int d = 0; d < 4; d++) o[b][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], bf8(p[z]), o[b][d], 0, 0, 0);
+            for (int d = 0; d < 4; d++) {
+                lh_f32x4 r = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], bf8(p[2]), (lh_f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                r = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], bf8(p[1]), r, 0, 0, 0);
+                r = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], bf8(p[0]), r, 0, 0, 0);
+                o[b][d] += r;
+            }
         }
     }
     // a lane holds 16 neighbouring value columns of its rows

@@ -646,6 +646,26 @@ def test_linear_attention_decays_above_one(ai, gpu, decay, rows, heads):
     close(got / size, end.transpose(0, 2, 1) / size, F32_TOL, "state")
 
 
+def test_linear_attention_sums_are_rounded_little(ai, gpu):
+    """Chunks of 128 rows against f64: no further off, in the 2-norm, than chunks of 64 rows with one running sum for all terms were (1.41e-7
+    at this size, and 1.62e-7 with 128 rows)."""
+    ctx, K = gpu
+    g, rows, heads, dim, vdim = np.random.default_rng(3), 1024, 40, 32, 64
+    q, k, v = (M.rounded(g.standard_normal((rows, heads, n))) for n in (dim, dim, vdim))
+    decay = np.linspace(0.6, 0.9995, heads).astype(np.float32).astype(np.float64)
+    state, out = ai.Buffer.empty(ctx, heads * vdim * dim * 4), empty(ai, ctx, rows * heads * vdim, ai.F32)
+    pw, work = ai.Buffer.from_slice(ctx, (decay[:, None] ** np.arange(65)).astype(np.float32)), ai.Buffer.empty(ctx, K.linear_attention_workspace_bytes(rows, heads, dim, vdim))
+    print("rounding of sums", flush=True)
+    batch = ai.CommandBatch(ctx)
+    K.linear_attention_chunked_into(batch, *(upload(ai, ctx, x, ai.BF16) for x in (q, k, v)), state, pw, work, out, rows, heads, dim, vdim)
+    batch.commit_and_wait()
+    t = np.arange(rows)
+    between = np.maximum(t[:, None] - t, 0)
+    want = np.stack([(q[:, h] @ k[:, h].T * np.tril(decay[h] ** between)) @ v[:, h] for h in range(heads)], 1)
+    err = np.linalg.norm(download(ai, out, rows * heads * vdim, ai.F32).reshape(want.shape) - want) / np.linalg.norm(want)
+    assert err <= 1.45e-7, err
+
+
 def test_linear_attention_of_very_wide_rows(ai, gpu):
     """Rows of 2^24 values, which a chunk's 32-bit offsets do not reach, and a state of more than 2^32 bytes a head, which they do."""
     ctx, K = gpu
