@@ -96,12 +96,12 @@ def test_latent_expand(ai, gpu, dtype, heads, dim, rot, vdim, rank):
     close(values_from_cache(download(ai, values, T * heads * dv, dt), heads * dv).reshape(T, heads, dv)[..., :vdim], (c @ uv.T).reshape(T, heads, vdim), tol, "values")
 
 
-def latent_case(ai, gpu, dtype, heads, rank, rot, start, rows, capacity, spike=None, stale=False, sink=0.5):
+def latent_case(ai, gpu, dtype, heads, rank, rot, start, rows, capacity, spike=None, stale=False, sink=0.5, scale=None):
     """`spike` (row, key): that row's queries match that key far better than any other."""
     ctx, K = gpu
     dt, g, T = ai.BF16 if dtype == "bf16" else ai.F32, np.random.default_rng(heads + rank + start + rows), start + rows
     c, kr = stored(g.standard_normal((T, rank)), ai, dt), stored(g.standard_normal((T, rot)), ai, dt)
-    q, scale = g.standard_normal((rows, heads, rank + rot)), 1.0 / np.sqrt(rank + rot)
+    q, scale = g.standard_normal((rows, heads, rank + rot)), 1.0 / np.sqrt(rank + rot) if scale is None else scale
     if spike:
         q[spike[0]] = np.concatenate([c[spike[1]], kr[spike[1]]]) * (12.0 / np.sqrt(rank + rot)) * np.linspace(1, 2, heads)[:, None]
         scale = 1.0
@@ -178,6 +178,13 @@ def test_latent_attention_long_context_splits(ai, gpu):
         latent_case(ai, gpu, "bf16", 2, 128, 16, 9000, rows, 9056, spike=(0, 37))
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("scale", [-0.05, 0.0])
+def test_latent_attention_scales_of_zero_and_below(ai, gpu, dtype, scale):
+    latent_case(ai, gpu, dtype, 5, 100, 20, 70, 40, 128, scale=scale)
+    latent_case(ai, gpu, dtype, 16, 256, 32, 600, 1, 640, scale=scale)
+
+
 def test_latent_attention_rejects(ai, gpu):
     ctx, K = gpu
     b, batch = ai.Buffer.empty(ctx, 1 << 16), ai.CommandBatch(ctx)
@@ -213,6 +220,12 @@ def test_softmax_attention_with_sink_and_gate(ai, gpu, dtype, heads, kv_heads, d
 
 
 # ---- selective state space --------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,start,rows", [(8, 2, 64, 64, 700, 200), (16, 4, 56, 33, 900, 150), (8, 8, 128, 250, 500, 130), (16, 2, 100, 120, 900, 65)])
+def test_sink_and_gate_of_many_rows_in_splits(ai, gpu, heads, kv_heads, dim, vdim, start, rows):
+    """1024 pairs of a row and a head and more, whose few splits are merged by a few lanes a pair."""
+    test_softmax_attention_with_sink_and_gate(ai, gpu, "bf16", heads, kv_heads, dim, vdim, start, rows)
+
+
 @pytest.mark.parametrize("heads,vdim,state,groups,taps", [(1, 3, 5, 1, 1), (4, 24, 20, 2, 4), (3, 33, 64, 3, 2), (2, 64, 128, 1, 3), (6, 16, 130, 2, 6), (2, 20, 300, 1, 4), (2, 8, 12, 1, 20)])
 @pytest.mark.parametrize("cuts", [[1, 1, 1, 1, 1], [2, 2, 1, 2], [17, 1, 65, 2, 130], [63, 1, 64, 1], [200]])
 def test_selective_state_space(ai, gpu, heads, vdim, state, groups, taps, cuts):

@@ -106,10 +106,13 @@ def test_large_products(ai, gpu, m, k, n, act):
     close(download(ai, res, m * n, ai.F32).reshape(m, n), want + 1, F32_TOL, "residual")
 
 
-@pytest.mark.parametrize("m,k,n", [(33, 8, 36), (64, 576, 512), (100, 4096, 260), (129, 200, 1000), (511, 1288, 1028), (512, 2048, 1024), (480, 712, 1536)])
+@pytest.mark.parametrize("m,k,n", [(33, 8, 36), (64, 576, 512), (100, 4096, 260), (129, 200, 1000), (511, 1288, 1028), (512, 2048, 1024), (480, 712, 1536),
+                                   (33, 72, 36), (33, 136, 36), (301, 1048, 712), (333, 1000, 1032), (190, 4104, 1500), (333, 2056, 1036), (287, 176, 1444), (2100, 2056, 2080)])
 @pytest.mark.parametrize("act", [0, 1, 2, 3])
 def test_products_of_few_tiles(ai, gpu, m, k, n, act):
-    """Waves that share out k: 32 x 32 tiles (the first four) and 64 x 32, fewer steps of k than waves, buffers used again, ragged steps."""
+    """By the rule for 256 CUs.  Waves that share out k on 32 x 32 tiles: 64 x 512 x 576, 100 x 260 x 4096, 129 x 1000 x 200, 301 x 712 x 1048
+    and, with f32 results, 33 rows of k 72 and 136, which leave waves without a step; on 64 x 32: 512 x 1024 x 2048 and, with ragged rows,
+    columns and last steps, those of k 1000, 4104 and 2056.  Shared waves: 32 x 32 for k 8, 176 and 1288, 64 x 64 for k 712, 128 x 128 for 2100 rows."""
     test_large_products(ai, gpu, m, k, n, act)
 
 
@@ -408,11 +411,11 @@ def test_row_norms_and_gather(ai, gpu, rows, dim):
 
 
 # ---- softmax attention -------------------------------------------------------------------------------------------------
-def attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows, cap, seed=0, spike=None, stale=False, lam=0.4, out_scale=0.7, poison=()):
+def attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows, cap, seed=0, spike=None, stale=False, lam=0.4, out_scale=0.7, poison=(), scale=None):
     """Caches filled as the projections fill them.  `spike` = (row, key): one key that takes nearly all of a row's weight."""
     ctx, K = gpu
     dt = ai.BF16 if dtype == "bf16" else ai.F32
-    g, eps, scale = np.random.default_rng(seed + start + rows + dim), 1e-5, dim ** -0.5
+    g, eps, scale = np.random.default_rng(seed + start + rows + dim), 1e-5, dim ** -0.5 if scale is None else scale
     L, dq, dv = start + rows, K.attention_padded_dim(dim), K.attention_padded_vdim(vdim)
     q, k, v = (stored(g.standard_normal(s), ai, dt) for s in ((rows, heads, maps, dim), (L, kv_heads, maps, dim), (L, kv_heads, vdim)))
     if spike is not None:
@@ -523,6 +526,15 @@ def test_attention_long_context_splits(ai, gpu):
 def test_attention_of_many_rows(ai, gpu, maps, dim, vdim, heads, start, rows):
     """A few splits of many rows, and launches whose workgroups are all on the chip at once, two a CU."""
     attention_case(ai, gpu, "bf16", maps, heads, 2 if heads < 16 else 4, dim, vdim, start, rows, (start + rows + 31) // 32 * 32)
+
+
+@pytest.mark.parametrize("scale", [-0.2, 0.0])
+@pytest.mark.parametrize("maps", [1, 2])
+@pytest.mark.parametrize("dtype,heads,kv_heads,dim,vdim,start,rows", [("bf16", 4, 2, 32, 64, 50, 20), ("bf16", 8, 2, 64, 128, 40, 150), ("bf16", 4, 4, 24, 40, 100, 90),
+                                                                     ("f32", 4, 2, 32, 64, 50, 20), ("f32", 4, 2, 64, 64, 40, 1)])
+def test_attention_scales_of_zero_and_below(ai, gpu, scale, maps, dtype, heads, kv_heads, dim, vdim, start, rows):
+    """Whose sign, or that they are zero, goes into the queries: up to 64 rows of a key head and tiles of more."""
+    attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows, (start + rows + 31) // 32 * 32, scale=scale)
 
 
 def test_attention_rejects(ai, gpu):
@@ -711,10 +723,13 @@ def test_mixture_of_odd_widths(ai, gpu, dtype, rows, experts, top, width, ff):
     test_mixture_of_experts(ai, gpu, dtype, rows, experts, top, width, ff)
 
 
-@pytest.mark.parametrize("rows,experts,top,width,ff", [(1000, 5, 1, 2048, 1024), (770, 6, 2, 1024, 2048), (1600, 3, 1, 192, 4096), (400, 2, 1, 2048, 2048)])
+@pytest.mark.parametrize("rows,experts,top,width,ff", [(1000, 5, 1, 2048, 1024), (770, 6, 2, 1024, 2048), (1600, 3, 1, 192, 4096), (400, 2, 1, 2048, 2048),
+                                                       (2000, 4, 2, 2048, 1024), (4000, 2, 1, 2048, 1024), (4000, 8, 1, 2048, 512), (3500, 3, 1, 2048, 1024), (2000, 12, 1, 72, 1040)])
 def test_mixture_of_large_experts(ai, gpu, rows, experts, top, width, ff):
-    """Expert plans with tiles of 256 rows through the kernels of large products: ragged last tiles, an expert with a few rows and one
-    with none.  The reference is f32 arithmetic on the CPU."""
+    """Expert plans through the kernels of large products, by the rule for 256 CUs (first product / second): 770, 1600 rows 256 x 128 phased
+    / 64 x 64 and 32 x 32; 2000 rows with two of four experts and 4000 with one of two 256 x 128 / 256 x 256 phased, the second added up from slots
+    and straight into the rows; 4000 with one of eight 128 x 128 / 256 x 256, 3500 128 x 128 / 256 x 128; 2000 of 12 128 x 128 of four waves / 32 x 32; the others 64 x 64.
+    Ragged last tiles, an expert with a few rows and one with none.  The reference is f32 arithmetic on the CPU."""
     ctx, K = gpu
     g = np.random.default_rng(rows + experts)
     x = M.rounded(g.standard_normal((rows, width))).astype(np.float32)
