@@ -1230,9 +1230,10 @@ static int launch_phased(lh_context* ctx, const LhLinear& a, uint64_t grid, cons
 
 // The forms for the tiles of an expert plan, and what one is expected to take in microseconds: `start`, `step` for each 64 columns of k and, for
 // every further tile a CU has, `round` and `round_step`; in each round `through` where a lane cannot store its `lanes` columns as they are, and
-// `wide` for f32 results; `empty` for each round of tiles without rows, and `weights` for each 4 MB of them.  Fitted to 982 products (up to
-// 4096 rows, 8192 columns and 128 experts), of which a form's times lie within 10 to 19 % (r.m.s.), then weighed against each other: the choice
-// takes 2 % longer than the best form would, 64 x 64 for all 11 %.  Two of 16 experts a row, 2048 -> 1024 columns: 200 rows 18 us (64 x 64; 64 x 32
+// `wide` for f32 results; `empty` for each round of tiles without rows, and `weights` for each 4 MB of them.  Fitted to 1004 products (up to
+// 4096 rows, 8192 columns and 128 experts; of 416 the weights came from memory, of the others from the memory-side cache) and then weighed against each
+// other: the choice takes 1 % longer than the best form would, on weights from memory 3 %.  64 x 64 tiles come with rings of
+// four buffers (up to two workgroups a CU) and of three (three a CU).  Two of 16 experts a row, 2048 -> 1024 columns: 200 rows 18 us (64 x 64; 64 x 32
 // tiles that share out k 23), 4096 rows 45 (256 x 256; 128 x 128 of four waves 60).
 struct PlanForm {
     uint32_t bm, bn, lanes;
@@ -1241,13 +1242,14 @@ struct PlanForm {
     int (*launch)(lh_context*, const LhLinear&, uint64_t, const char*);
 };
 static const PlanForm kPlanForms[] = {
-    {256, 256, 16, true, 5.71f, 0.893f, 0.0f, 1.4f, 2.7f, 17.7f, 43.3f, 0.0f, launch_phased<256, 256>},
-    {256, 128, 16, true, 5.21f, 0.698f, 3.34f, 0.852f, 3.0f, 11.3f, 20.4f, 0.089f, launch_phased<256, 128>},
-    {128, 128, 16, true, 6.33f, 0.471f, 4.33f, 0.557f, 2.75f, 6.49f, 9.79f, 0.0858f, launch_phased<128, 128>},
-    {128, 128, 16, false, 4.58f, 0.6f, 0.242f, 0.375f, 6.51f, 4.51f, 11.7f, 0.0f, launch_mfma<128, 128, 2>},
-    {64, 64, 8, false, 4.09f, 0.328f, 1.0f, 0.162f, 1.4f, 0.7f, 1.7f, 0.089f, launch_mfma<64, 64, 3>},
-    {32, 32, 4, false, 4.12f, 0.066f, 1.37f, 0.076f, 0.5f, 0.4f, 1.1f, 0.324f, launch_sliced<32, 32, 2>},
-    {32, 32, 4, false, 3.89f, 0.223f, 0.514f, 0.0977f, 0.0735f, 0.263f, 0.735f, 0.338f, launch_mfma<32, 32, 4>},
+    {256, 256, 16, true, 10.8f, 0.99f, 7.15f, 1.35f, 0.0f, 9.65f, 14.2f, 0.151f, launch_phased<256, 256>},
+    {256, 128, 16, true, 11.2f, 0.487f, 6.64f, 0.692f, 0.0f, 8.2f, 0.046f, 0.201f, launch_phased<256, 128>},
+    {128, 128, 16, true, 5.99f, 0.545f, 2.7f, 0.567f, 0.0f, 4.1f, 9.55f, 0.0f, launch_phased<128, 128>},
+    {128, 128, 16, false, 4.94f, 0.684f, 0.937f, 0.324f, 9.8f, 4.06f, 8.02f, 0.0947f, launch_mfma<128, 128, 2>},
+    {64, 64, 8, false, 4.14f, 0.33f, 0.795f, 0.239f, 0.178f, 0.916f, 2.1f, 0.123f, launch_mfma<64, 64, 4>},
+    {64, 64, 8, false, 4.04f, 0.366f, 0.49f, 0.204f, 0.0f, 0.984f, 1.71f, 0.115f, launch_mfma<64, 64, 3>},
+    {32, 32, 4, false, 5.15f, 0.0526f, 1.41f, 0.102f, 0.0f, 0.35f, 0.611f, 0.577f, launch_sliced<32, 32, 2>},
+    {32, 32, 4, false, 4.12f, 0.22f, 0.438f, 0.13f, 0.0f, 0.477f, 0.544f, 0.434f, launch_mfma<32, 32, 4>},
 };
 static float plan_time(const PlanForm& f, const LhLinear& a, uint64_t steps, uint64_t tiles, uint64_t cus) {
     // A plan has one tile more for each expert than can be full.  Every expert that is chosen has one with rows, and of the last ones about half.
@@ -1326,13 +1328,15 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     auto through = [&](uint32_t lanes, uint64_t t) { return epilogue_of(a.seg, lanes) == kThroughLds ? t : 0; };
     auto per_cu = [&](uint64_t n) { return (n + want - 1) / want; };
     const uint64_t t64 = (n64 <= want ? 4000 + 345 * steps : n64 <= 2 * want ? 4600 + 430 * steps : n64 <= 3 * want ? 5600 + 590 * steps : per_cu(n64) * (2100 + 190 * steps)) + through(8, 1700);
-    const uint64_t t64_32 = 1000 + per_cu(tiles(64, 32)) * (3500 + 100 * steps) + through(4, 900);
+    const uint64_t n6432 = tiles(64, 32), t64_32 = (n6432 <= want ? 4500 + 100 * steps : per_cu(n6432) * (3700 + 130 * steps)) + through(4, 900);
     const uint64_t t32 = (n32 <= want ? 4000 + 75 * steps : 1000 + (n32 + 2 * want - 1) / (2 * want) * (3500 + 150 * steps)) + through(4, 700);
-    const uint64_t t32_shared = (n32 <= want ? 3700 + 240 * steps : n32 <= 2 * want ? 3900 + 280 * steps : n32 <= 3 * want ? 4300 + 360 * steps : per_cu(n32) * (1100 + 92 * steps)) + through(4, 200);
+    // (with longer k it is the slower one on weights that come from memory: 200 x 4360 x 1024 18 us against 12 of 64 x 64)
+    const uint64_t t32_shared = steps > 4 ? UINT64_MAX : (n32 <= want ? 3700 + 240 * steps : n32 <= 2 * want ? 3900 + 280 * steps : n32 <= 3 * want ? 4300 + 360 * steps : per_cu(n32) * (1100 + 92 * steps)) + through(4, 200);
     const uint64_t t128 = n128 > want ? 8000 + 870 * steps + through(16, 11000) : UINT64_MAX;
     const uint64_t least = std::min({t64, t64_32, t32, t32_shared, t128});
     if (t128 == least) return launch_mfma<128, 128, 2>(ctx, a, n128, op);
-    if (t64 == least) return launch_mfma<64, 64, 3>(ctx, a, n64, op);
+    // (with a CU to itself a workgroup keeps four buffers in flight rather than three: 3 % faster, on weights from memory 6 %; from the third a CU on they do not fit, 18 to 30 % slower)
+    if (t64 == least) return n64 <= want ? launch_mfma<64, 64, 4>(ctx, a, n64, op) : launch_mfma<64, 64, 3>(ctx, a, n64, op);
     if (t64_32 == least) return launch_sliced<64, 32, 3>(ctx, a, tiles(64, 32), op);
     return t32 == least ? launch_sliced<32, 32, 2>(ctx, a, n32, op) : launch_mfma<32, 32, 4>(ctx, a, n32, op);
 }

@@ -107,12 +107,13 @@ def test_large_products(ai, gpu, m, k, n, act):
 
 
 @pytest.mark.parametrize("m,k,n", [(33, 8, 36), (64, 576, 512), (100, 4096, 260), (129, 200, 1000), (511, 1288, 1028), (512, 2048, 1024), (480, 712, 1536),
-                                   (33, 72, 36), (33, 136, 36), (301, 1048, 712), (333, 1000, 1032), (190, 4104, 1500), (333, 2056, 1036), (287, 176, 1444), (2100, 2056, 2080)])
+                                   (33, 72, 36), (33, 136, 36), (301, 1048, 712), (333, 1000, 1032), (190, 4104, 1500), (333, 2056, 1036), (287, 176, 1444), (2100, 2056, 2080), (1500, 712, 1512)])
 @pytest.mark.parametrize("act", [0, 1, 2, 3])
 def test_products_of_few_tiles(ai, gpu, m, k, n, act):
     """By the rule for 256 CUs.  Waves that share out k on 32 x 32 tiles: 64 x 512 x 576, 100 x 260 x 4096, 129 x 1000 x 200, 301 x 712 x 1048
     and, with f32 results, 33 rows of k 72 and 136, which leave waves without a step; on 64 x 32: 512 x 1024 x 2048 and, with ragged rows,
-    columns and last steps, those of k 1000, 4104 and 2056.  Shared waves: 32 x 32 for k 8, 176 and 1288, 64 x 64 for k 712, 128 x 128 for 2100 rows."""
+    columns and last steps, those of k 1000, 4104 and 2056 and f32 results of k 1288.  Shared waves: 32 x 32 for k 8 and 176 and bf16 results of k 72
+    and 136; 64 x 64 with four buffers for 480 rows of k 712 and bf16 results of k 1288, with three for 1500 rows; 128 x 128 for 2100 rows."""
     test_large_products(ai, gpu, m, k, n, act)
 
 
@@ -726,9 +727,9 @@ def test_mixture_of_odd_widths(ai, gpu, dtype, rows, experts, top, width, ff):
 @pytest.mark.parametrize("rows,experts,top,width,ff", [(1000, 5, 1, 2048, 1024), (770, 6, 2, 1024, 2048), (1600, 3, 1, 192, 4096), (400, 2, 1, 2048, 2048),
                                                        (2000, 4, 2, 2048, 1024), (4000, 2, 1, 2048, 1024), (4000, 8, 1, 2048, 512), (3500, 3, 1, 2048, 1024), (2000, 12, 1, 72, 1040)])
 def test_mixture_of_large_experts(ai, gpu, rows, experts, top, width, ff):
-    """Expert plans through the kernels of large products, by the rule for 256 CUs (first product / second): 770, 1600 rows 256 x 128 phased
-    / 64 x 64 and 32 x 32; 2000 rows with two of four experts and 4000 with one of two 256 x 128 / 256 x 256 phased, the second added up from slots
-    and straight into the rows; 4000 with one of eight 128 x 128 / 256 x 256, 3500 128 x 128 / 256 x 128; 2000 of 12 128 x 128 of four waves / 32 x 32; the others 64 x 64.
+    """Expert plans through the kernels of large products, by the rule for 256 CUs (first product / second): 1000 rows 64 x 64 / 128 x 128
+    phased; 770, 1600 rows 256 x 128 phased / 64 x 64 and 32 x 32; 400 rows 64 x 64 with four buffers; 2000 rows with two
+    of four experts and 4000 with one of two 256 x 128 / 256 x 256 phased, the second added up from slots and straight into the rows; 4000 with one of eight 128 x 128 / 256 x 256, 3500 128 x 128 / 256 x 128; 2000 of 12 128 x 128 of four waves / 32 x 32.
     Ragged last tiles, an expert with a few rows and one with none.  The reference is f32 arithmetic on the CPU."""
     ctx, K = gpu
     g = np.random.default_rng(rows + experts)
