@@ -24,18 +24,22 @@ constexpr uint32_t kHalf = 64;   // rows that the callers' powers, and the runni
 // What the step of a token is: fixed per head, or computed from the token (selective state space).
 __device__ __forceinline__ float softplus(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
 
+// Where the decay comes from is known when a kernel is compiled: a stride read from the arguments made each token's launch 0.4 us longer.
+enum Decay { kFixed, kPowers, kSelective };
+
 struct RecurrentArgs {
     const void *q, *k, *v;
     float* state;
-    const float* decay;                                     // [heads], `decay_step` apart
+    const float* decay;                                     // [heads], or [heads, kHalf + 1] powers of them
     const float *dt_raw, *dt_bias, *a_log, *skip;           // selective: [rows, heads], then [heads] each
     float* out;
-    uint32_t rows, heads, key_heads, dim, dq, vdim, decay_step;
+    uint32_t rows, heads, key_heads, dim, dq, vdim;
     float scale;
 };
 
-template <typename T, int NR, bool SELECTIVE>
+template <typename T, int NR, Decay DECAY>
 __global__ __launch_bounds__(256) void recurrent_kernel(const RecurrentArgs a) {
+    constexpr bool SELECTIVE = DECAY == kSelective;
     const T *q = static_cast<const T*>(a.q), *k = static_cast<const T*>(a.k), *v = static_cast<const T*>(a.v);
     const uint32_t dim = a.dim, dq = a.dq, vdim = a.vdim, heads = a.heads, rows = a.rows;
     const uint32_t vt = (vdim + 15) / 16, h = blockIdx.x / vt, col = (blockIdx.x % vt) * 16 + (threadIdx.x >> 4), part = threadIdx.x & 15;
@@ -46,7 +50,7 @@ __global__ __launch_bounds__(256) void recurrent_kernel(const RecurrentArgs a) {
     float s[NR];
 #pragma unroll
     for (int i = 0; i < NR; i++) s[i] = k0 + i < dq ? st[i] : 0.0f;
-    const float fixed = SELECTIVE ? 0.0f : a.decay[(size_t)h * a.decay_step], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
+    const float fixed = SELECTIVE ? 0.0f : a.decay[(size_t)h * (DECAY == kPowers ? kHalf + 1 : 1)], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
                 skip = SELECTIVE ? a.skip[h] : 0.0f;
     float kn[NR], qn[NR], vn, zn = 0.0f;
     auto fetch = [&](uint32_t t) {
@@ -108,8 +112,9 @@ template <int N> struct Packed<uint16_t, N> {
 
 // The same recurrence over many rows.  A step is a few dozen instructions behind its inputs, so the inputs of AHEAD rows are on their
 // way at any time, in whole pieces, and no load is conditional (one row ahead and a value at a time: 2 us a row; now 0.2).
-template <typename T, int NR, int AHEAD, bool SELECTIVE>
+template <typename T, int NR, int AHEAD, Decay DECAY>
 __global__ __launch_bounds__(256) void recurrent_rows_kernel(const RecurrentArgs a) {
+    constexpr bool SELECTIVE = DECAY == kSelective;
     const uint32_t dim = a.dim, dq = a.dq, vdim = a.vdim, heads = a.heads, rows = a.rows;
     const uint32_t vt = (vdim + 15) / 16, h = blockIdx.x / vt, col = (blockIdx.x % vt) * 16 + (threadIdx.x >> 4), part = threadIdx.x & 15;
     const bool on = col < vdim, has = part * NR < dq;             // (dq is a multiple of NR: a lane has all of its values, or none)
@@ -120,7 +125,7 @@ __global__ __launch_bounds__(256) void recurrent_rows_kernel(const RecurrentArgs
     float s[NR];
 #pragma unroll
     for (int i = 0; i < NR; i++) s[i] = has ? st[i] : 0.0f;
-    const float fixed = SELECTIVE ? 0.0f : a.decay[(size_t)h * a.decay_step], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
+    const float fixed = SELECTIVE ? 0.0f : a.decay[(size_t)h * (DECAY == kPowers ? kHalf + 1 : 1)], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
                 skip = SELECTIVE ? a.skip[h] : 0.0f;
     struct Row { Packed<T, NR> k, q; T v; float z; } next[AHEAD];
     auto fetch = [&](Row& r, uint32_t t) {
@@ -613,12 +618,12 @@ int launch_chunked_dim(lh_context* ctx, ChunkArgs& a, const char* op) {
     return a.chunk == 64 ? launch_chunked_rows<64, SELECTIVE>(ctx, a, op) : launch_chunked_rows<128, SELECTIVE>(ctx, a, op);
 }
 
-template <typename T, bool SELECTIVE>
+template <typename T, Decay DECAY>
 int launch_recurrent(lh_context* ctx, const RecurrentArgs& a, const char* op) {
     const uint64_t grid = (uint64_t)a.heads * ((a.vdim + 15) / 16);
     LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: heads %u, vdim %u", op, a.heads, a.vdim);
     if (a.rows >= 8 && (((uintptr_t)a.q | (uintptr_t)a.k) & 15) == 0) {        // (a row's keys and queries start at multiples of 32 values)
-#define LH_REC(NR_, AHEAD_) hipLaunchKernelGGL((recurrent_rows_kernel<T, NR_, AHEAD_, SELECTIVE>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a)
+#define LH_REC(NR_, AHEAD_) hipLaunchKernelGGL((recurrent_rows_kernel<T, NR_, AHEAD_, DECAY>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a)
         if (a.dq <= 32) LH_REC(2, 8);
         else if (a.dq <= 64) LH_REC(4, 8);
         else if (a.dq <= 128) LH_REC(8, 8);
@@ -628,7 +633,7 @@ int launch_recurrent(lh_context* ctx, const RecurrentArgs& a, const char* op) {
 #undef LH_REC
         return lh_check_launch(op);
     }
-#define LH_REC(NR_) hipLaunchKernelGGL((recurrent_kernel<T, NR_, SELECTIVE>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a)
+#define LH_REC(NR_) hipLaunchKernelGGL((recurrent_kernel<T, NR_, DECAY>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a)
     if (a.dq <= 32) LH_REC(2);
     else if (a.dq <= 64) LH_REC(4);
     else if (a.dq <= 128) LH_REC(8);
@@ -671,8 +676,8 @@ int lh_linear_attention_recurrent_into(lh_batch* batch, const lh_buffer* q, cons
     LH_NEED(output, (size_t)rows * heads * vdim * 4, op, "output");
     RecurrentArgs a{};
     a.q = q->ptr; a.k = k->ptr; a.v = v->ptr; a.state = (float*)state->ptr; a.decay = (const float*)decay->ptr; a.out = (float*)output->ptr;
-    a.rows = rows; a.heads = a.key_heads = heads; a.dim = dim; a.dq = dq; a.vdim = vdim; a.decay_step = 1; a.scale = scale;
-    const int r = dtype == LH_F32 ? launch_recurrent<float, false>(batch->ctx, a, op) : launch_recurrent<uint16_t, false>(batch->ctx, a, op);
+    a.rows = rows; a.heads = a.key_heads = heads; a.dim = dim; a.dq = dq; a.vdim = vdim; a.scale = scale;
+    const int r = dtype == LH_F32 ? launch_recurrent<float, kFixed>(batch->ctx, a, op) : launch_recurrent<uint16_t, kFixed>(batch->ctx, a, op);
     if (r == LH_OK) batch->dispatch_count++;
     return r;
 }
@@ -697,9 +702,9 @@ int lh_linear_attention_chunked_into(lh_batch* batch, const lh_buffer* q, const 
     if (!chunk_offsets_fit(heads, dq, vdim)) {
         RecurrentArgs r{};
         r.q = q->ptr; r.k = k->ptr; r.v = v->ptr; r.state = (float*)state->ptr; r.out = (float*)output->ptr;
-        r.decay = (const float*)decay_powers->ptr + 1; r.decay_step = kHalf + 1;
+        r.decay = (const float*)decay_powers->ptr + 1;
         r.rows = rows; r.heads = r.key_heads = heads; r.dim = dim; r.dq = dq; r.vdim = vdim; r.scale = scale;
-        const int rc = launch_recurrent<uint16_t, false>(batch->ctx, r, op);
+        const int rc = launch_recurrent<uint16_t, kPowers>(batch->ctx, r, op);
         if (rc == LH_OK) batch->dispatch_count++;
         return rc;
     }
@@ -740,7 +745,7 @@ int lh_selective_recurrent_into(lh_batch* batch, const lh_buffer* x, const lh_bu
     a.q = c->ptr; a.k = b->ptr; a.v = x->ptr; a.state = (float*)memory->ptr; a.out = (float*)output->ptr;
     a.dt_raw = (const float*)dt_raw->ptr; a.dt_bias = (const float*)dt_bias->ptr; a.a_log = (const float*)a_log->ptr; a.skip = (const float*)skip->ptr;
     a.rows = rows; a.heads = heads; a.key_heads = groups; a.dim = state; a.dq = dq; a.vdim = vdim; a.scale = 1.0f;
-    const int r = dtype == LH_F32 ? launch_recurrent<float, true>(batch->ctx, a, op) : launch_recurrent<uint16_t, true>(batch->ctx, a, op);
+    const int r = dtype == LH_F32 ? launch_recurrent<float, kSelective>(batch->ctx, a, op) : launch_recurrent<uint16_t, kSelective>(batch->ctx, a, op);
     if (r == LH_OK) batch->dispatch_count++;
     return r;
 }
