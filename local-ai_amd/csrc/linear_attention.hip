@@ -24,7 +24,7 @@ constexpr uint32_t kHalf = 64;   // rows that the callers' powers, and the runni
 // What the step of a token is: fixed per head, or computed from the token (selective state space).
 __device__ __forceinline__ float softplus(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
 
-// Where the decay comes from is known when a kernel is compiled: a stride read from the arguments made each token's launch 0.4 us longer.
+// Where the decay comes from is known when a kernel is compiled, so that a token's launch starts with no address to compute from a stride.
 enum Decay { kFixed, kPowers, kSelective };
 
 struct RecurrentArgs {
