@@ -96,7 +96,7 @@ typedef __attribute__((address_space(3))) void lvoid;
 // What binds is vector and matrix instructions at the clock that they leave (a step of 64 keys of two maps: 3600 cycles of matrix
 // instructions per SIMD and about 3000 of vector instructions, before two values were rounded and reduced by one instruction each 5000:
 // 2048 rows of 16 heads, two maps, at position 0 104 -> 95 us, at 2048 252 -> 216).  No product waits for the one before it: 95 -> 89.  With one map the two blocks of a step belong to two groups of four
-// waves, whose sums meet at the end: 2048 rows of 16 heads of 192 and 128 columns 75 -> 66 us.  With two maps the registers do not suffice for that.
+// waves, whose sums meet at the end: 2048 rows of 16 heads of 192 and 128 columns 75 -> 61 us.  With two maps the registers do not suffice for that.
 __device__ __forceinline__ uint32_t value_place(uint32_t col) { return ((col >> 2) & 1) * 2 + (((col >> 1) ^ (col >> 3)) & 1); }
 template <int DQ, int DV, int MAPS, int NB, int G>
 __global__ __launch_bounds__(256 * G, G == 2 ? 4 : MAPS * DV <= 256 ? 2 : 1) void attention_tile_kernel(const AttentionArgs a) {
