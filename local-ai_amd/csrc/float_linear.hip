@@ -1321,7 +1321,7 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     // The rest by its expected time in nanoseconds, measured: 64 x 64 or 32 x 32 tiles of shared waves, up to three or five workgroups a CU;
     // waves that share out k, on 64 x 32 tiles (one workgroup a CU) or 32 x 32 (two); or 128 x 128 tiles of shared waves, where there is more than one a
     // CU.  A lane that cannot store its columns as they are (bf16 rows that are no multiple of 16 bytes) costs the more the larger the tile.  Before / now,
-    // weights in the memory-side cache: 512 x 1024 x 4096 25.5 / 12.5 us and 200 x 2048 x 8192 46.7 / 19.2 (64 x 32), 512 x 1024 x 1024 9.6 / 6.5, 2048 x 16 x 2048 14.0 / 6.0
+    // weights in the memory-side cache: 512 x 1024 x 4096 25.5 / 12.5 us, 200 x 2048 x 8192 46.7 / 19.2 and 512 x 1024 x 1024 9.6 / 6.5 (64 x 32), 2048 x 16 x 2048 14.0 / 6.0
     // and 256 x 1024 x 4096 25.2 / 9.4 (32 x 32, shared-out k), 953 x 2048 x 2048 21 / 17.9 and 300 x 6144 x 1536 19.5 / 15.3 (64 x 64, from 128 x 64), 333 x 1024 x 1024
     // with f32 activations 20.3 / 9.6; short k: 287 x 1444 x 176 7.5 / 5.1, 25 x 620 x 136 5.2 / 4.7 (32 x 32, shared waves); ragged k: 3893 x 1504 x 4568 120 / 82 (128 x 128).
     const uint64_t n64 = tiles(64, 64), n32 = tiles(32, 32), n128 = tiles(128, 128);
