@@ -1319,21 +1319,23 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     }
     if (tiles(128, 128) >= 2 * want) return launch_mfma<128, 128, 2>(ctx, a, tiles(128, 128), op);
     // The rest by its expected time in nanoseconds, measured: 64 x 64 or 32 x 32 tiles of shared waves, up to three or five workgroups a CU;
-    // waves that share out k, on 64 x 32 tiles (one workgroup a CU) or 32 x 32 (two); or 128 x 128 tiles of shared waves, where there is more than one a
-    // CU.  A lane that cannot store its columns as they are (bf16 rows that are no multiple of 16 bytes) costs the more the larger the tile.  Before / now,
+    // waves that share out k, on 64 x 32 tiles (one workgroup a CU) or 32 x 32 (two); or 128 x 64 and 128 x 128 tiles of shared waves, where there is more than
+    // one a CU (1702 x 1880 x 2928 41 us on 128 x 64 tiles, weights from memory, 56 on 64 x 64).  A lane that cannot store its columns as they are (bf16 rows that are no multiple of 16 bytes) costs the more the larger the tile.  Before / now,
     // weights in the memory-side cache: 512 x 1024 x 4096 25.5 / 12.5 us, 200 x 2048 x 8192 46.7 / 19.2 and 512 x 1024 x 1024 9.6 / 6.5 (64 x 32), 2048 x 16 x 2048 14.0 / 6.0
     // and 256 x 1024 x 4096 25.2 / 9.4 (32 x 32, shared-out k), 953 x 2048 x 2048 21 / 17.9 and 300 x 6144 x 1536 19.5 / 15.3 (64 x 64, from 128 x 64), 333 x 1024 x 1024
     // with f32 activations 20.3 / 9.6; short k: 287 x 1444 x 176 7.5 / 5.1, 25 x 620 x 136 5.2 / 4.7 (32 x 32, shared waves); ragged k: 3893 x 1504 x 4568 120 / 82 (128 x 128).
-    const uint64_t n64 = tiles(64, 64), n32 = tiles(32, 32), n128 = tiles(128, 128);
+    const uint64_t n64 = tiles(64, 64), n32 = tiles(32, 32), n128 = tiles(128, 128), n128_64 = tiles(128, 64);
     auto through = [&](uint32_t lanes, uint64_t t) { return epilogue_of(a.seg, lanes) == kThroughLds ? t : 0; };
     auto per_cu = [&](uint64_t n) { return (n + want - 1) / want; };
     const uint64_t t64 = (n64 <= want ? 4000 + 345 * steps : n64 <= 2 * want ? 4600 + 430 * steps : n64 <= 3 * want ? 5600 + 590 * steps : per_cu(n64) * (2100 + 190 * steps)) + through(8, 1700);
-    const uint64_t n6432 = tiles(64, 32), t64_32 = (n6432 <= want ? 4500 + 100 * steps : per_cu(n6432) * (3700 + 130 * steps)) + through(4, 900);
+    const uint64_t n6432 = tiles(64, 32), t64_32 = (n6432 <= want ? 4500 + 100 * steps : per_cu(n6432) * (3550 + 148 * steps)) + through(4, 900);
     const uint64_t t32 = (n32 <= want ? 4000 + 75 * steps : 1000 + (n32 + 2 * want - 1) / (2 * want) * (3500 + 150 * steps)) + through(4, 700);
     // (with longer k it is the slower one on weights that come from memory: 200 x 4360 x 1024 18 us against 12 of 64 x 64)
     const uint64_t t32_shared = steps > 4 ? UINT64_MAX : (n32 <= want ? 3700 + 240 * steps : n32 <= 2 * want ? 3900 + 280 * steps : n32 <= 3 * want ? 4300 + 360 * steps : per_cu(n32) * (1100 + 92 * steps)) + through(4, 200);
     const uint64_t t128 = n128 > want ? 8000 + 870 * steps + through(16, 11000) : UINT64_MAX;
-    const uint64_t least = std::min({t64, t64_32, t32, t32_shared, t128});
+    const uint64_t t128_64 = n128_64 > want ? 5800 + 385 * steps + (per_cu(n128_64) - 1) * (1400 + 386 * steps) + through(8, 1700) : UINT64_MAX;
+    const uint64_t least = std::min({t64, t64_32, t32, t32_shared, t128_64, t128});
+    if (t128_64 == least) return launch_mfma<128, 64, 3>(ctx, a, n128_64, op);
     if (t128 == least) return launch_mfma<128, 128, 2>(ctx, a, n128, op);
     // (with a CU to itself a workgroup keeps four buffers in flight rather than three: 3 % faster, on weights from memory 6 %; from the third a CU on they do not fit, 18 to 30 % slower)
     if (t64 == least) return n64 <= want ? launch_mfma<64, 64, 4>(ctx, a, n64, op) : launch_mfma<64, 64, 3>(ctx, a, n64, op);

@@ -107,13 +107,14 @@ def test_large_products(ai, gpu, m, k, n, act):
 
 
 @pytest.mark.parametrize("m,k,n", [(33, 8, 36), (64, 576, 512), (100, 4096, 260), (129, 200, 1000), (511, 1288, 1028), (512, 2048, 1024), (480, 712, 1536),
-                                   (33, 72, 36), (33, 136, 36), (301, 1048, 712), (333, 1000, 1032), (190, 4104, 1500), (333, 2056, 1036), (287, 176, 1444), (2100, 2056, 2080), (1500, 712, 1512)])
+                                   (33, 72, 36), (33, 136, 36), (301, 1048, 712), (333, 1000, 1032), (190, 4104, 1500), (333, 2056, 1036), (287, 176, 1444), (2100, 2056, 2080), (1500, 712, 1512), (1490, 1096, 2308)])
 @pytest.mark.parametrize("act", [0, 1, 2, 3])
 def test_products_of_few_tiles(ai, gpu, m, k, n, act):
     """By the rule for 256 CUs.  Waves that share out k on 32 x 32 tiles: 64 x 512 x 576, 100 x 260 x 4096, 129 x 1000 x 200, 301 x 712 x 1048
     and, with f32 results, 33 rows of k 72 and 136, which leave waves without a step; on 64 x 32: 512 x 1024 x 2048 and, with ragged rows,
     columns and last steps, those of k 1000, 4104 and 2056 and f32 results of k 1288.  Shared waves: 32 x 32 for k 8 and 176 and bf16 results of k 72
-    and 136; 64 x 64 with four buffers for 480 rows of k 712 and bf16 results of k 1288, with three for 1500 rows; 128 x 128 for 2100 rows."""
+    and 136; 64 x 64 with four buffers for 480 rows of k 712 and bf16 results of k 1288, with three for 1500 rows; 128 x 64 for
+    1490 rows and 128 x 128 for 2100."""
     test_large_products(ai, gpu, m, k, n, act)
 
 
