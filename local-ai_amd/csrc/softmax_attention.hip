@@ -380,7 +380,11 @@ int launch_mfma(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const 
         // (one workgroup fits a CU where the sums of two maps take its registers: the longest first there, 2048 rows of 16 heads of 128 and 256
         // columns 188 us; in the order for two a CU 230)
         a.resident = MAPS * DV <= 256 ? (uint32_t)cus : UINT32_MAX;
-        hipLaunchKernelGGL((attention_tile_kernel<DQ, DV, MAPS, NB, G>), dim3((uint32_t)(groups * a.splits)), dim3(256 * G), 0, ctx->stream, a);
+        // One step of keys is all that there may be: the second group would only add its empty sums (rows of 1 to 64 keys, heads of 64 to 192: 6 % and at
+        // most 8 slower; from 65 keys on two groups take as long, from 129 on less).
+        const bool one = std::min<uint64_t>((uint64_t)max_position + a.rows, a.capacity) <= 32 * NB;
+        if (G == 2 && one) hipLaunchKernelGGL((attention_tile_kernel<DQ, DV, MAPS, NB, 1>), dim3((uint32_t)(groups * a.splits)), dim3(256), 0, ctx->stream, a);
+        else hipLaunchKernelGGL((attention_tile_kernel<DQ, DV, MAPS, NB, G>), dim3((uint32_t)(groups * a.splits)), dim3(256 * G), 0, ctx->stream, a);
         const int r = lh_check_launch(op);
         return r != LH_OK || a.splits == 1 ? r : merge();
     }

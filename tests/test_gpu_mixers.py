@@ -457,7 +457,7 @@ def attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("maps", [1, 2])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(3, 3, 32, 64), (6, 2, 24, 40), (8, 1, 64, 128), (3, 3, 8, 16), (4, 2, 128, 256), (5, 1, 20, 33), (34, 2, 16, 24)])
-@pytest.mark.parametrize("start,rows", [(0, 1), (31, 1), (32, 2), (95, 34), (0, 97), (63, 190)])
+@pytest.mark.parametrize("start,rows", [(0, 1), (31, 1), (32, 2), (95, 34), (0, 97), (63, 190), (0, 64), (1, 64)])
 def test_attention_shapes(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows):
     attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, rows, 256)
 
