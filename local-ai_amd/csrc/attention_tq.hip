@@ -75,8 +75,7 @@ __device__ __forceinline__ float reduce8(const float (&v)[8], int lane) {
     // complemented, so route through an xor-4 exchange instead.
     float c = keep + __shfl_xor(give, 4, 64);
     c += __shfl_xor(c, 8, 64);
-    c += lh_swap16_f(c);
-    c += lh_swap32_f(c);
+    c = lh_sum32_f(lh_sum16_f(c));
     return c;   // total of value index ((lane&1) | (lane&2) | (lane&4)) -> lane & 7
 }
 

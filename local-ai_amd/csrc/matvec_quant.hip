@@ -455,11 +455,11 @@ __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProble
             }
             if (red_width > 16) {
 #pragma unroll
-                for (int u = 0; u < U; u++) part[u] += lh_swap16_f(part[u]);
+                for (int u = 0; u < U; u++) part[u] = lh_sum16_f(part[u]);
             }
             if (red_width > 32) {
 #pragma unroll
-                for (int u = 0; u < U; u++) part[u] += lh_swap32_f(part[u]);
+                for (int u = 0; u < U; u++) part[u] = lh_sum32_f(part[u]);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {

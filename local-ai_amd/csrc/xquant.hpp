@@ -4,6 +4,7 @@
 // products with small unsigned weight codes are exact in v_dot4_i32_i8 / MFMA i8 arithmetic.
 #pragma once
 #include "common.hpp"
+#include <type_traits>
 
 template <int L> struct Limb;
 template <> struct Limb<2> { static constexpr float qmax = 32639.0f; };     // 127*256 + 127
@@ -74,14 +75,14 @@ __device__ __forceinline__ void xpro_rotate8_regs(float (&v)[8], const XPrologue
         }
     }
     const uint32_t lane = threadIdx.x & 63;
-    for (uint32_t m = 1; 8 * m < pro.head_dim; m <<= 1) {
-        const bool upper = (lane & m) != 0;
+    const auto stage = [&](auto far) {
+        constexpr int LEN = decltype(far)::value;
+        if (8 * LEN >= pro.head_dim) return;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float other = __shfl_xor(v[i], (int)m, 64);
-            v[i] = upper ? __fsub_rn(other, v[i]) : __fadd_rn(v[i], other);
-        }
-    }
+        for (int i = 0; i < 8; i++) v[i] = lh_fwht_lane_stage<LEN>(v[i], lane);
+    };
+    stage(std::integral_constant<int, 1>()); stage(std::integral_constant<int, 2>()); stage(std::integral_constant<int, 4>());
+    stage(std::integral_constant<int, 8>()); stage(std::integral_constant<int, 16>()); stage(std::integral_constant<int, 32>());
     const float sg[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = lh_h2f(lh_f2h_exact(__fmul_rn(__fmul_rn(v[i], pro.scale), sg[i])));
