@@ -208,6 +208,13 @@ LH_API int lh_matvec_quant_norm_chain_into(lh_batch* batch, lh_quant fmt, uint32
                                            const lh_buffer* vector, const lh_buffer* weight, const lh_buffer* residual,
                                            const lh_buffer* next_weight, lh_buffer* store, float eps,
                                            lh_buffer* const* outputs, uint32_t rows, uint32_t cols);
+/* The same with the GeGLU product behind it (layer.rs:476-482, 495-500), where the products' own launch can form it: with `up`, `out` holds
+ * gelu(gate's results) * up's results, as gelu_mul_into computes it from the f16 results; with `factor` (f16[rows], exactly one of the two),
+ * gelu(gate's results) * factor.  `*applied` says whether it did: if not, `out` and `up_out` hold the results themselves. */
+LH_API int lh_matvec_quant_norm_chain_gelu_into(lh_batch* batch, lh_quant fmt, const lh_buffer* gate, const lh_buffer* up,
+                                                const lh_buffer* factor, const lh_buffer* vector, const lh_buffer* weight,
+                                                const lh_buffer* residual, const lh_buffer* next_weight, lh_buffer* store, float eps,
+                                                lh_buffer* out, lh_buffer* up_out, uint32_t rows, uint32_t cols, int* applied);
 /* The chain across two layers (layer.rs:503-520 of one layer, 387-392 of the next): the staged vector is the layer
  * output that rms_norm_residual_scale_into would have written,
  *   t = f16(f16(f16(rms_norm(vector) * weight) + residual) * scale)     (the scale only with `apply_scale`),

@@ -431,6 +431,18 @@ class Kernels:
                                                        vector._h, weight._h, h(residual), h(next_weight), h(store),
                                                        C.c_float(eps), _handles(outputs), _u32(rows), _u32(cols)))
 
+    def matvec_quant_norm_chain_gelu_into(self, batch, fmt, gate, up, factor, vector, weight, residual, next_weight, store, eps, out, up_out,
+                                          rows, cols) -> bool:
+        """The norm chain with the GeGLU product behind it where its launch can form it: True, and `out` holds gelu(gate results) * (up
+        results, or `factor`); False, and `out` and `up_out` hold the products' results.  One of `up` and `factor` is None."""
+        def h(b):
+            return b._h if b is not None else None
+        applied = C.c_int(0)
+        _check(self._l.lh_matvec_quant_norm_chain_gelu_into(batch._h, C.c_int(fmt), gate._h, h(up), h(factor), vector._h, weight._h,
+                                                            h(residual), h(next_weight), h(store), C.c_float(eps), out._h, h(up_out),
+                                                            _u32(rows), _u32(cols), C.byref(applied)))
+        return applied.value != 0
+
     def matvec_quant_norm_chain_tail_into(self, batch, fmt, matrices, vector, weight, residual, scale, next_weight, store, eps,
                                           outputs, rows, cols):
         """Matvecs against the next layer's attention norm of t = (rms_norm(vector) * weight + residual) * scale, rounded as

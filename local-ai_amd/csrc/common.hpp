@@ -126,8 +126,10 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
                               void* const* outputs, lh_dtype xt, lh_dtype yt, uint32_t rows, uint32_t K, uint32_t xstride,
                               uint32_t ystride, const XPrologue& pro = XPrologue{kXProNone, nullptr, 0.0f}, uint64_t mstride = 0);
 // Up to eight TQ2_0 or Q4_0 matrices and one vector, or one matrix and a batch of vectors, f16 in (before a rotation: f32) and out (matvec_direct.hip); -1: not for this form.
+// Behind a norm: `gated`, two matrices whose results leave as gelu(first) * second in outputs[0]; `factor`, one whose results leave as
+// gelu(result) * factor.
 int lh_launch_matvec_direct(lh_context* ctx, lh_quant fmt, uint32_t count, const void* const* matrices, const void* vector, void* const* outputs, uint32_t rows,
-                                uint32_t K, const XPrologue& pro, uint32_t batch = 1, uint32_t xstride = 0, uint32_t ystride = 0);
+                                uint32_t K, const XPrologue& pro, uint32_t batch = 1, uint32_t xstride = 0, uint32_t ystride = 0, bool gated = false, const uint16_t* factor = nullptr);
 // The m rows of a small activation batch against one quantized matrix, as m matvecs in one launch (matvec_quant.hip).
 // Returns LH_OK, an error, or -1 when the fast kernels do not take the shape (the caller then uses its own kernel).
 int lh_matvec_rows(lh_batch* batch, lh_quant fmt, uint32_t m, const lh_buffer* weight, const lh_buffer* input, lh_dtype at,

@@ -672,10 +672,14 @@ bool fast_path_ok(lh_quant fmt, const void* matrix, const void* vector, uint32_t
     return ((uintptr_t)matrix & 1) == 0;
 }
 
+// What becomes of the results where the kernel can still change them: gelu(first matrix's) * second's, or gelu(the one matrix's) * factor.
+struct Gelu { const uint16_t* factor; int* applied; };
+
 // Validates and launches `count` matvecs of one shape.
 int matvec_dispatch(lh_batch* batch, lh_quant fmt, uint32_t count, const lh_buffer* const* matrices,
                     const lh_buffer* const* vectors, lh_dtype xt, lh_buffer* const* outputs, lh_dtype yt, uint32_t rows,
-                    uint32_t cols, const char* op, const XPrologue& pro = XPrologue{kXProNone, nullptr, 0.0f}) {
+                    uint32_t cols, const char* op, const XPrologue& pro = XPrologue{kXProNone, nullptr, 0.0f}, const Gelu* gelu = nullptr) {
+    if (gelu) *gelu->applied = 0;
     if (!batch) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: batch is null", op);
     if (xt == LH_BF16 || yt == LH_BF16) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: bf16 vectors are not supported", op);
     // kernels.rs:5720-5724, 5857-5861: block alignment is checked before anything is encoded.
@@ -732,9 +736,9 @@ int matvec_dispatch(lh_batch* batch, lh_quant fmt, uint32_t count, const lh_buff
     if (one_vector) {
         const void* pm[8]; void* py[8];
         for (uint32_t i = 0; i < count; i++) { pm[i] = matrices[i]->ptr; py[i] = outputs[i]->ptr; }
-        const int r = lh_launch_matvec_direct(ctx, fmt, count, pm, vectors[0]->ptr, py, rows, cols, pro);
+        const int r = lh_launch_matvec_direct(ctx, fmt, count, pm, vectors[0]->ptr, py, rows, cols, pro, 1, 0, 0, gelu && count == 2, gelu ? gelu->factor : nullptr);
         if (r != -1) {
-            if (r == LH_OK) batch->dispatch_count++;
+            if (r == LH_OK) { batch->dispatch_count++; if (gelu) *gelu->applied = 1; }
             return r;
         }
     }
@@ -906,9 +910,9 @@ int lh_matvec_quant_fused_into(lh_batch* b, lh_quant fmt, uint32_t count, const 
     return matvec_dispatch(b, fmt, count, ms, xs, LH_F16, ys, LH_F16, rows, cols, op, pro);
 }
 
-int lh_matvec_quant_norm_chain_into(lh_batch* b, lh_quant fmt, uint32_t count, const lh_buffer* const* ms, const lh_buffer* x,
-                                    const lh_buffer* weight, const lh_buffer* residual, const lh_buffer* next_weight, lh_buffer* store,
-                                    float eps, lh_buffer* const* ys, uint32_t rows, uint32_t cols) {
+static int norm_chain(lh_batch* b, lh_quant fmt, uint32_t count, const lh_buffer* const* ms, const lh_buffer* x,
+                      const lh_buffer* weight, const lh_buffer* residual, const lh_buffer* next_weight, lh_buffer* store,
+                      float eps, lh_buffer* const* ys, uint32_t rows, uint32_t cols, const Gelu* gelu) {
     const char* op = fmt == LH_Q4_0 ? "matvec_q4_0 (norm chain)" : "matvec_tq2_0 (norm chain)";
     if (fmt != LH_Q4_0 && fmt != LH_TQ2_0) return lh_fail(LH_ERR_INVALID_ARGUMENT, "matvec_quant: unknown weight format %d", (int)fmt);
     if (count == 0 || rows == 0 || cols == 0) return LH_OK;
@@ -935,7 +939,27 @@ int lh_matvec_quant_norm_chain_into(lh_batch* b, lh_quant fmt, uint32_t count, c
     pro.res = residual ? (const uint16_t*)residual->ptr : nullptr;
     pro.aux2 = next_weight ? (const uint16_t*)next_weight->ptr : nullptr;
     pro.store = store ? (uint16_t*)store->ptr : nullptr;
-    return matvec_dispatch(b, fmt, count, ms, xs, LH_F16, ys, LH_F16, rows, cols, op, pro);
+    return matvec_dispatch(b, fmt, count, ms, xs, LH_F16, ys, LH_F16, rows, cols, op, pro, gelu);
+}
+
+int lh_matvec_quant_norm_chain_into(lh_batch* b, lh_quant fmt, uint32_t count, const lh_buffer* const* ms, const lh_buffer* x,
+                                    const lh_buffer* weight, const lh_buffer* residual, const lh_buffer* next_weight, lh_buffer* store,
+                                    float eps, lh_buffer* const* ys, uint32_t rows, uint32_t cols) {
+    return norm_chain(b, fmt, count, ms, x, weight, residual, next_weight, store, eps, ys, rows, cols, nullptr);
+}
+
+int lh_matvec_quant_norm_chain_gelu_into(lh_batch* b, lh_quant fmt, const lh_buffer* gate, const lh_buffer* up, const lh_buffer* factor, const lh_buffer* x,
+                                         const lh_buffer* weight, const lh_buffer* residual, const lh_buffer* next_weight, lh_buffer* store,
+                                         float eps, lh_buffer* out, lh_buffer* up_out, uint32_t rows, uint32_t cols, int* applied) {
+    const char* op = "matvec (norm chain, gelu)";
+    if (!applied) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: applied is null", op);
+    *applied = 0;
+    if ((up != nullptr) == (factor != nullptr)) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: either an up projection or a factor", op);
+    if (factor) LH_NEED(factor, (size_t)rows * 2, op, "factor");
+    const lh_buffer* ms[2] = {gate, up};
+    lh_buffer* ys[2] = {out, up_out};
+    const Gelu gelu{factor ? (const uint16_t*)factor->ptr : nullptr, applied};
+    return norm_chain(b, fmt, up ? 2 : 1, ms, x, weight, residual, next_weight, store, eps, ys, rows, cols, &gelu);
 }
 
 int lh_matvec_quant_norm_chain_tail_into(lh_batch* b, lh_quant fmt, uint32_t count, const lh_buffer* const* ms, const lh_buffer* x,

@@ -63,7 +63,7 @@ __device__ __forceinline__ void xpro_norm_add8(const void* xv, const XPrologue& 
 // (the same butterflies in the same order of stages; a sum does not depend on which operand is named first).  Stages
 // 1, 2, 4 pair elements of one lane, the others pair the lanes of a head, head_dim / 8 <= 64 consecutive lanes of a wave.
 // Every lane of the wave calls it; lanes past the vector carry zeros.  s0, s1: the eight elements' signs.
-__device__ __forceinline__ void xpro_rotate8_regs(float (&v)[8], const XPrologue& pro, const float4 s0, const float4 s1) {
+__device__ __forceinline__ void xpro_rotate8_regs(float (&v)[8], uint32_t head_dim, float scale, const float4 s0, const float4 s1) {
 #pragma unroll
     for (int len = 1; len < 8; len <<= 1) {
 #pragma unroll
@@ -77,7 +77,7 @@ __device__ __forceinline__ void xpro_rotate8_regs(float (&v)[8], const XPrologue
     const uint32_t lane = threadIdx.x & 63;
     const auto stage = [&](auto far) {
         constexpr int LEN = decltype(far)::value;
-        if (8 * LEN >= pro.head_dim) return;
+        if (8 * LEN >= head_dim) return;
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] = lh_fwht_lane_stage<LEN>(v[i], lane);
     };
@@ -85,11 +85,11 @@ __device__ __forceinline__ void xpro_rotate8_regs(float (&v)[8], const XPrologue
     stage(std::integral_constant<int, 8>()); stage(std::integral_constant<int, 16>()); stage(std::integral_constant<int, 32>());
     const float sg[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = lh_h2f(lh_f2h_exact(__fmul_rn(__fmul_rn(v[i], pro.scale), sg[i])));
+    for (int i = 0; i < 8; i++) v[i] = lh_h2f(lh_f2h_exact(__fmul_rn(__fmul_rn(v[i], scale), sg[i])));
 }
 __device__ __forceinline__ void xpro_rotate8(float (&v)[8], const XPrologue& pro, uint32_t e0) {
     const float* s = pro.signs + (e0 & (pro.head_dim - 1));
-    xpro_rotate8_regs(v, pro, *reinterpret_cast<const float4*>(s), *reinterpret_cast<const float4*>(s + 4));
+    xpro_rotate8_regs(v, pro.head_dim, pro.scale, *reinterpret_cast<const float4*>(s), *reinterpret_cast<const float4*>(s + 4));
 }
 
 // Second level of the fixed point, for blocks whose first-level step would be too coarse.  A block with max|x| = m has

@@ -369,17 +369,20 @@ class TransformerLayer:
 
         # 4. GeGLU feed-forward -> post_feedforward_norm + residual #2
         inter = p.intermediate_size
+        multiplied = False
         if chain_ffn:   # residual #1 and the feed-forward pre-norm while gate / up stage their input; attn_resid kept
-            kernels.matvec_quant_norm_chain_into(batch, w.ffn_gate.ty, [w.ffn_gate.buf, w.ffn_up.buf], s.ffn_out,
-                                                 w.attn_post_norm, input, w.ffn_norm, s.attn_resid, eps, [s.gate, s.up],
-                                                 w.ffn_gate.rows, w.ffn_gate.cols)
+            multiplied = kernels.matvec_quant_norm_chain_gelu_into(batch, w.ffn_gate.ty, w.ffn_gate.buf, w.ffn_up.buf, None, s.ffn_out,
+                                                                   w.attn_post_norm, input, w.ffn_norm, s.attn_resid, eps, s.gate, s.up,
+                                                                   w.ffn_gate.rows, w.ffn_gate.cols)
         elif self._fusable(w.ffn_gate, w.ffn_up):
             self._fused_matvecs(batch, kernels, kernels.PROLOGUE_RMS_NORM, s.attn_resid, w.ffn_norm,
                                 [w.ffn_gate, w.ffn_up], [s.gate, s.up])
         else:
             kernels.rms_norm_into(batch, s.attn_resid, w.ffn_norm, s.normed, h, 1, eps)
             self._pair_matvec(batch, kernels, w.ffn_gate, w.ffn_up, s.normed, s.gate, s.up)
-        if self._fusable(w.ffn_down):
+        if multiplied:
+            w.ffn_down.matvec_into(batch, kernels, s.gate, s.ffn_out)
+        elif self._fusable(w.ffn_down):
             self._fused_matvecs(batch, kernels, kernels.PROLOGUE_GELU_MUL, s.gate, s.up, [w.ffn_down], [s.ffn_out])
         else:
             kernels.gelu_mul_into(batch, s.gate, s.up, s.gate, inter)
@@ -393,13 +396,17 @@ class TransformerLayer:
         # 5. per-layer input injection -> residual #3
         if has_ple:
             pld = p.per_layer_dim
+            multiplied = False
             if chain_ple:   # residual #2 while the per-layer gate stages its input; `output` written once by that kernel
                 g = w.per_layer_inp_gate
-                kernels.matvec_quant_norm_chain_into(batch, g.ty, [g.buf], s.ffn_out, w.ffn_post_norm, s.attn_resid, None,
-                                                     output, eps, [s.ple_h], g.rows, g.cols)
+                multiplied = kernels.matvec_quant_norm_chain_gelu_into(batch, g.ty, g.buf, None, self._ple_slice(per_layer_input), s.ffn_out,
+                                                                       w.ffn_post_norm, s.attn_resid, None, output, eps, s.ple_h, None,
+                                                                       g.rows, g.cols)
             else:
                 w.per_layer_inp_gate.matvec_into(batch, kernels, output, s.ple_h)
-            if self._fusable(w.per_layer_proj):
+            if multiplied:
+                w.per_layer_proj.matvec_into(batch, kernels, s.ple_h, s.ffn_out)
+            elif self._fusable(w.per_layer_proj):
                 # this layer's slice is read in place (no copy into scratch) while the projection stages its input
                 self._fused_matvecs(batch, kernels, kernels.PROLOGUE_GELU_MUL, s.ple_h, self._ple_slice(per_layer_input),
                                     [w.per_layer_proj], [s.ffn_out])

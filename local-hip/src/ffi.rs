@@ -92,6 +92,7 @@ extern "C" {
     pub fn lh_matvec_quant_typed_into(batch: *mut lh_batch, fmt: lh_quant, matrix: *const lh_buffer, vector: *const lh_buffer, vector_dtype: lh_dtype, output: *mut lh_buffer, output_dtype: lh_dtype, rows: u32, cols: u32) -> c_int;
     pub fn lh_matvec_quant_grouped_into(batch: *mut lh_batch, fmt: lh_quant, count: u32, matrices: *const *const lh_buffer, vectors: *const *const lh_buffer, vector_dtype: lh_dtype, outputs: *const *mut lh_buffer, output_dtype: lh_dtype, rows: u32, cols: u32) -> c_int;
     pub fn lh_matvec_quant_norm_chain_into(batch: *mut lh_batch, fmt: lh_quant, count: u32, matrices: *const *const lh_buffer, vector: *const lh_buffer, weight: *const lh_buffer, residual: *const lh_buffer, next_weight: *const lh_buffer, store: *mut lh_buffer, eps: f32, outputs: *const *mut lh_buffer, rows: u32, cols: u32) -> c_int;
+    pub fn lh_matvec_quant_norm_chain_gelu_into(batch: *mut lh_batch, fmt: lh_quant, gate: *const lh_buffer, up: *const lh_buffer, factor: *const lh_buffer, vector: *const lh_buffer, weight: *const lh_buffer, residual: *const lh_buffer, next_weight: *const lh_buffer, store: *mut lh_buffer, eps: f32, out: *mut lh_buffer, up_out: *mut lh_buffer, rows: u32, cols: u32, applied: *mut c_int) -> c_int;
     pub fn lh_matvec_quant_norm_chain_tail_into(batch: *mut lh_batch, fmt: lh_quant, count: u32, matrices: *const *const lh_buffer, vector: *const lh_buffer, weight: *const lh_buffer, residual: *const lh_buffer, apply_scale: c_int, scale: f32, next_weight: *const lh_buffer, store: *mut lh_buffer, eps: f32, outputs: *const *mut lh_buffer, rows: u32, cols: u32) -> c_int;
     pub fn lh_matvec_quant_rotated_into(batch: *mut lh_batch, fmt: lh_quant, matrix: *const lh_buffer, vector: *const lh_buffer, signs: *const lh_buffer, head_dim: u32, output: *mut lh_buffer, rows: u32, cols: u32) -> c_int;
     pub fn lh_matvec_quant_fused_into(batch: *mut lh_batch, fmt: lh_quant, count: u32, matrices: *const *const lh_buffer, vector: *const lh_buffer, prologue: c_int, aux: *const lh_buffer, eps: f32, outputs: *const *mut lh_buffer, rows: u32, cols: u32) -> c_int;

@@ -670,3 +670,32 @@ def test_matvec_tq2_split_wait_gives_up_loudly(pkg, gpu, oracle):
     got = yall.as_array(np.float32, count * rows).reshape(count, rows)
     for i in (0, count // 2, count - 1):
         refgen.assert_close(got[i], want, 1e-3, f"problem {i} after the budget was restored")
+
+
+@pytest.mark.parametrize("fmt,rows,cols,gated", [("tq2_0", 6144, 1536, True), ("tq2_0", 301, 2304, True), ("q4_0", 33, 320, True), ("tq2_0", 1, 256, True),
+                                                 ("q4_0", 256, 1536, False), ("q4_0", 7, 4160, False), ("tq2_0", 20000, 1536, True)])
+def test_matvec_norm_chain_gelu(pkg, gpu, fmt, rows, cols, gated):
+    """The GeGLU product formed by the launch of its factors has the bits of gelu_mul_into on the results of the plain chain, and a launch that
+    cannot form it (20000 pairs of rows) leaves those results."""
+    ctx, K = gpu
+    ty = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0
+    g = pkg.synth.rng(35, rows + cols)
+    make = refgen.q4_0_payload if fmt == "q4_0" else refgen.tq2_0_payload
+    ws = [pkg.QuantWeight.from_bytes(ctx, make(rows, cols, 0x51 + i), ty, rows, cols) for i in range(2 if gated else 1)]
+    x, res, w1, w2 = (pkg.Buffer.from_slice(ctx, (m + s * g.standard_normal(cols, dtype=np.float32)).astype(np.float16))
+                      for m, s in ((0, 0.7), (0, 1), (1, 0.2), (1, 0.2)))
+    factor = pkg.Buffer.from_slice(ctx, g.standard_normal(rows, dtype=np.float32).astype(np.float16))
+    stores, outs = ([pkg.Buffer.empty(ctx, n) for _ in range(4)] for n in (cols * 2, rows * 2))
+    batch = pkg.CommandBatch(ctx)
+    K.matvec_quant_norm_chain_into(batch, ty, [w.buf for w in ws], x, w1, res, w2, stores[0], 1e-6, outs[:len(ws)], rows, cols)
+    applied = K.matvec_quant_norm_chain_gelu_into(batch, ty, ws[0].buf, ws[1].buf if gated else None, None if gated else factor, x, w1, res, w2,
+                                                  stores[1], 1e-6, outs[2], outs[3] if gated else None, rows, cols)
+    assert applied == (rows < 20000) and batch.dispatch_count() == 2
+    if applied:
+        K.gelu_mul_into(batch, outs[0], outs[1] if gated else factor, outs[0], rows)
+    batch.commit_and_wait()
+    for a, b in [(stores[0], stores[1]), (outs[0], outs[2])] + ([] if applied else [(outs[1], outs[3])]):
+        assert np.array_equal(a.as_array(np.uint16), b.as_array(np.uint16))
+    for up, f in ((ws[0].buf, factor), (None, None)):        # exactly one of the two
+        with pytest.raises(pkg.InvalidArgument):
+            K.matvec_quant_norm_chain_gelu_into(pkg.CommandBatch(ctx), ty, ws[0].buf, up, f, x, w1, res, w2, stores[1], 1e-6, outs[2], outs[3], rows, cols)
