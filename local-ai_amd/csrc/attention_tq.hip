@@ -465,6 +465,9 @@ int attention_dispatch(lh_batch* batch, const char* op, const lh_buffer* rq, con
         }
         hipLaunchKernelGGL(attention_tq_split_kernel, dim3(p.num_splits, p.num_queries * p.num_kv_heads), dim3(kThreads), lds_bytes, ctx->stream,
                            ptrs.rq, ptrs.k_codes, ptrs.k_norms, ptrs.v_codes, ptrs.v_norms, ptrs.levels, ptrs.positions, ptrs.out, ptrs.ws, p);
+    } else if (short_supported(ctx, p, max_span)) {
+        const int rl = launch_short(ctx, op, ptrs, p, max_span);
+        if (rl != LH_OK) return rl;
     } else {
         const int rl = launch_mfma(ctx, op, ptrs, p, max_span, ws_avail);
         if (rl != LH_OK) return rl;

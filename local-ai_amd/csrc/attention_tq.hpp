@@ -55,6 +55,10 @@ bool mfma_supported(const AttnParams& p, const AttnPointers& a);
 // runs the merge kernel when p.num_splits > 1.
 int launch_mfma(lh_context* ctx, const char* op, const AttnPointers& a, AttnParams& p, uint64_t max_span, size_t ws_floats);
 
+// Queries that leave no CU with two, over a short span (attention_tq_short.hip; what mfma_supported takes, head_dim 256, spans of up to eleven groups of 64): the output is final.
+bool short_supported(const lh_context* ctx, const AttnParams& p, uint64_t max_span);
+int launch_short(lh_context* ctx, const char* op, const AttnPointers& a, AttnParams& p, uint64_t max_span);
+
 // The tiled prefill kernel (attention_tq_prefill_tile.hip): sixteen query rows per workgroup share one pass over the codes,
 // K and V levels as f16 through LDS, any level table.  Takes 2-bit codes, head_dim 256, at most 8 query heads per KV head,
 // ring absent or a multiple of 64 slots, two rows or more.

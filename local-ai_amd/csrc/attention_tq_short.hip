@@ -1,0 +1,359 @@
+// Attention over a short span of packed 2-bit TurboQuant codes: a sliding window's one token, or one token of each of some dozens of
+// sequences, or the rows of a prompt's chunk.
+//
+// Same contract and the same arithmetic as attention_tq_mfma.hip (stands in for shaders/attention_flash_tq.metal:154-690): the level table as bit
+// planes, queries and softmax weights in 16-bit fixed point as two int8 limbs, v_mfma_i32_16x16x64_i8.  What differs is who does what.  There a K wave
+// and a V wave walk a chunk of positions with a hand-over after each 64, which is what long spans want; over 512 positions the walk of three hand-overs is
+// a chain of 7 of the launch's 10.7 us, on one CU.  Here:
+//   * a wave takes an aligned group of 64 positions through both products, so that a window of 512 (nine groups) is one step of nine waves, and
+//     nothing is handed over: a wave's softmax reference, sums and fixed-point scales are its own and meet in LDS at the end;
+//   * a query's workgroups, four of them on four CUs, take 64 of the 256 output dims each (two with 128 where there are queries for that, or one with all).
+//     Each repeats the scores (half of the work), none waits for another, and the kernel's output is final: no partial records, no merge launch;
+//   * everything that comes from memory -- queries, codes of both kinds, norms -- is requested at the top, ahead of the level table, on which the
+//     rest depends.
+// Bound by the chain of one group and by a SIMD's two or three waves taking turns to issue.  From the first to the last instruction of one token over a
+// window of 512: 10.7 us there, 6.1 here; launches of 1 query 12.8 and 7.6, of 256 rows 14.3 and 10.2.
+#include "attention_tq.hpp"
+#include <algorithm>
+#include <cstdlib>
+
+namespace {
+using namespace lh_attn;
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef unsigned short us2_t __attribute__((ext_vector_type(2)));
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
+
+constexpr uint32_t kGroup = 64, kHeads = 8, kDim = 256, kMaxWaves = 12;
+constexpr float kLog2e = 1.4426950408889634f, kQmax = 32639.0f, kNoRef = -1.0e30f;
+
+__device__ __forceinline__ u32x4_t ld16(const uint8_t* p) {
+    typedef u32x4_t __attribute__((aligned(4))) u32x4_a4;
+    return *reinterpret_cast<const u32x4_a4*>(p);
+}
+
+struct ShortShared {
+    float q[4][kHeads][72];              // by field, head and code byte (a row in 72: a quarter wave's 16-byte reads on distinct banks)
+    uint8_t rqop[12][64][16];            // score operands per (plane, field) and lane
+    float maxabs[kHeads], sum[kHeads];
+    float fin_r[kMaxWaves][kHeads], fin_l[kMaxWaves][kHeads];
+};
+// S: workgroups of a query, 256 / S output dims each.
+template <int S>
+struct ShortWave {
+    float2 norm[kGroup];                 // (norm_k log2 e, norm_v) per position
+    union {
+        struct { uint8_t wx[3][1024], vt[4 / S][kGroup * 16]; };
+        float park[kHeads][kDim / S];    // the wave's sums, when it is done
+    };
+};
+
+// What a wave has requested of a group: see the loads in the kernel.
+template <int S>
+struct Group { u32x4_t k[4], v[4 / S]; uint32_t nk, nv; uint32_t lo, hi; };
+
+template <int NPL, int S, class Load>
+__device__ __forceinline__ void short_body(const AttnPointers& a, const AttnParams& p, ShortShared& sh, ShortWave<S>& mine, Group<S> gr, uint32_t G, uint32_t g_last, Load load,
+                                           float alpha, float beta, float gam, float delta, uint32_t qi, uint32_t kvh, uint32_t group) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6, pcol = lane & 15, g = lane >> 4;
+    constexpr int E = 4 / S;              // chunks of 16 code bytes, 64 dims
+    const float cmax = fmaxf(fmaxf(fabsf(beta), fabsf(0.5f * gam)), NPL == 3 ? fabsf(delta) : 0.0f), inv_cmax = cmax > 0.0f ? 1.0f / cmax : 0.0f;
+
+    // ---- score operands: row r of the product is head (r / 4) + 4 ((r / 2) % 2), limb r % 2; k slot (word m, byte e) of row group g is code byte
+    //      16 g + 4 m + e, i.e. dim 4 (16 g + 4 m + e) + f for field f.  The lanes of a head's two limbs quantise two of the four words each.
+    {
+        const uint32_t h = (pcol >> 2) + 4 * ((pcol >> 1) & 1), limb = pcol & 1;
+        const float ma = sh.maxabs[h], inv = (ma > 0.0f && cmax > 0.0f) ? kQmax / (ma * cmax) : 0.0f;
+        for (uint32_t unit = wave; unit < 4 * NPL; unit += nwaves) {
+            const uint32_t pl = unit >> 2, f = unit & 3;
+            const float mul = (pl == 0 ? beta : pl == 1 ? 0.5f * gam : delta) * inv;
+            uint32_t w[4];
+#pragma unroll
+            for (int mm = 0; mm < 2; mm++) {                  // word 2 mm + limb
+                const float4 x = *reinterpret_cast<const float4*>(&sh.q[f][h][16 * g + 4 * (2 * mm + limb)]);
+                const float xs[4] = {x.x, x.y, x.z, x.w};
+                uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int n = (int)fminf(fmaxf(__builtin_rintf(xs[e] * mul), -kQmax), kQmax), low = (int)(int8_t)(n & 0xFF);
+                    lo |= (uint32_t)(low & 0xFF) << (8 * e);
+                    hi |= (uint32_t)(((n - low) >> 8) & 0xFF) << (8 * e);
+                }
+                const uint32_t own = limb ? hi : lo, got = (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR1>((int)(limb ? lo : hi));
+                w[2 * mm] = limb ? got : own;
+                w[2 * mm + 1] = limb ? own : got;
+            }
+            *reinterpret_cast<u32x4_t*>(&sh.rqop[unit][lane][0]) = (u32x4_t){w[0], w[1], w[2], w[3]};
+        }
+    }
+    lh_lds_barrier();
+
+    float R[2] = {kNoRef, kNoRef}, l_run[2] = {0.f, 0.f}, w_run[2] = {0.f, 0.f}, sctr[2] = {0.f, 0.f}, out[E][4][2];
+#pragma unroll
+    for (int e = 0; e < E; e++)
+#pragma unroll
+        for (int f = 0; f < 4; f++) out[e][f][0] = out[e][f][1] = 0.0f;
+    const bool any = G <= g_last;
+    if (any) {
+        float cs[2], ca[2];              // logit (log2 domain) = norm_k log2 e (cs int + ca) for the lane's two heads g, g + 4
+#pragma unroll
+        for (int hs = 0; hs < 2; hs++) { cs[hs] = sh.maxabs[g + 4 * hs] * cmax * (0.25f / kQmax); ca[hs] = alpha * sh.sum[g + 4 * hs]; }
+        v4i kept[4];                     // plane 0's, where there is room for them
+#pragma unroll
+        for (int u = 0; u < 4; u++) if (E == 1) kept[u] = *reinterpret_cast<const v4i*>(&sh.rqop[u][lane][0]);
+        uint32_t from = lane;
+        auto rq = [&](int u) { return E == 1 && u < 4 ? kept[u & 3] : *reinterpret_cast<const v4i*>(&sh.rqop[u][from][0]); };
+        for (;;) {
+            asm volatile("" : "+v"(from));                       // (or the operands would be read ahead of the loop and spilled)
+            const bool valid = lane >= gr.lo && lane < gr.hi;
+            mine.norm[lane] = make_float2(lh_h2f((uint16_t)gr.nk) * kLog2e, valid ? lh_h2f((uint16_t)gr.nv) : 0.0f);
+#pragma unroll
+            for (int e = 0; e < E; e++) *reinterpret_cast<u32x4_t*>(&mine.vt[e][lane * 16]) = gr.v[e];
+            __builtin_amdgcn_wave_barrier();
+            // ---- scores of 4 tiles x (this lane's column position, heads g and g + 4)
+            float lg[4][2], vn[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                v4i acc1 = (v4i){0, 0, 0, 0}, acc4 = (v4i){0, 0, 0, 0};      // by mask scale: fields 0, 2 arrive x1, fields 1, 3 x4
+                const uint32_t w[4] = {gr.k[q].x, gr.k[q].y, gr.k[q].z, gr.k[q].w};
+#pragma unroll
+                for (int pl = 0; pl < NPL; pl++) {
+                    // plane 0 at bit 2 f of a field, plane 1 at bit 2 f + 1 (its coefficient is halved), plane 2 = bit0 & bit1 at bit 2 f
+                    const uint32_t bits = pl == 1 ? 0x02020202u : 0x01010101u;
+                    v4i b[4];
+#pragma unroll
+                    for (int m = 0; m < 4; m++) {
+                        const uint32_t t = pl == 2 ? w[m] & (w[m] >> 1) : w[m], u = t >> 4;
+                        b[0][m] = (int)(t & bits); b[1][m] = (int)(t & bits << 2); b[2][m] = (int)(u & bits); b[3][m] = (int)(u & bits << 2);
+                    }
+                    acc1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(rq(4 * pl), b[0], acc1, 0, 0, 0);
+                    acc4 = __builtin_amdgcn_mfma_i32_16x16x64_i8(rq(4 * pl + 1), b[1], acc4, 0, 0, 0);
+                    acc1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(rq(4 * pl + 2), b[2], acc1, 0, 0, 0);
+                    acc4 = __builtin_amdgcn_mfma_i32_16x16x64_i8(rq(4 * pl + 3), b[3], acc4, 0, 0, 0);
+                }
+                const float2 nrm = mine.norm[16 * q + pcol];
+                vn[q] = nrm.y;
+                const bool in = 16 * q + pcol >= gr.lo && 16 * q + pcol < gr.hi;
+#pragma unroll
+                for (int hs = 0; hs < 2; hs++) {
+                    const uint32_t t1 = ((uint32_t)acc1[2 * hs + 1] << 8) + (uint32_t)acc1[2 * hs], t4 = ((uint32_t)acc4[2 * hs + 1] << 8) + (uint32_t)acc4[2 * hs];
+                    lg[q][hs] = in ? nrm.x * ((float)(int)((t1 << 2) + t4) * cs[hs] + ca[hs]) : -INFINITY;
+                }
+                __builtin_amdgcn_sched_barrier(0);           // (four tiles' operands at a time would not fit the registers)
+            }
+            // (all dims of a query at once leave no registers for another group: launched only where a wave has one)
+            const bool more = S > 1 && G + nwaves <= g_last;
+            if (E == 1 && more) gr = load(G + nwaves);       // (with more dims only when the registers are free)
+            // ---- softmax weights relative to the wave's largest score so far, and as 16-bit fixed point relative to the head's largest weight of the group
+            float wm[2] = {0.f, 0.f}, un[2], ww[4][2];
+#pragma unroll
+            for (int hs = 0; hs < 2; hs++) {
+                const float r = fmaxf(R[hs], lh_group_max(fmaxf(fmaxf(lg[0][hs], lg[1][hs]), fmaxf(lg[2][hs], lg[3][hs])), 16)), fsc = __builtin_amdgcn_exp2f(R[hs] - r);
+                l_run[hs] *= fsc; w_run[hs] *= fsc; sctr[hs] *= fsc;
+#pragma unroll
+                for (int e = 0; e < E; e++)
+#pragma unroll
+                    for (int f = 0; f < 4; f++) out[e][f][hs] *= fsc;
+                R[hs] = r;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const float ew = __builtin_amdgcn_exp2f(lg[q][hs] - r);
+                    ww[q][hs] = ew * vn[q];
+                    l_run[hs] += ew;
+                    if constexpr (NPL == 3) w_run[hs] += ww[q][hs];
+                    wm[hs] = fmaxf(wm[hs], fabsf(ww[q][hs]));
+                }
+                // (zero, subnormal or non-finite maximum: scale and step 0, as in the other kernel)
+                const uint32_t e = lh_group_max_u(__float_as_uint(wm[hs]), 16) & 0x7F800000u;
+                const bool ok = e != 0u && e < (253u << 23);
+                const float sc = ok ? __uint_as_float((253u << 23) - e) : 0.0f;
+                un[hs] = ok ? __uint_as_float(e + (1u << 23)) * (cmax * (1.0f / kQmax)) : 0.0f;
+                const uint32_t A_ = pcol >> 2, B_ = ((pcol & 3) + 2 * (pcol >> 2)) & 3;      // k group and word: where the V codes of positions 16 q + pcol land
+#pragma unroll
+                for (int pl = 0; pl < NPL; pl++) {
+                    const float c = (pl == 0 ? beta : pl == 1 ? 0.5f * gam : delta) * inv_cmax * (kQmax / 32767.0f) * sc;
+                    const uint32_t p01 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_i16(ww[0][hs] * c, ww[1][hs] * c));
+                    const uint32_t p23 = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pknorm_i16(ww[2][hs] * c, ww[3][hs] * c));
+                    const uint32_t t01 = __builtin_bit_cast(uint32_t, (us2_t)(__builtin_bit_cast(us2_t, p01) + (us2_t){0x80, 0x80})) ^ 0x00800080u;
+                    const uint32_t t23 = __builtin_bit_cast(uint32_t, (us2_t)(__builtin_bit_cast(us2_t, p23) + (us2_t){0x80, 0x80})) ^ 0x00800080u;
+                    uint8_t* dst = &mine.wx[pl][(16 * A_ + 4 * g + 2 * hs) * 16 + 4 * B_];
+                    *reinterpret_cast<uint32_t*>(dst) = __builtin_amdgcn_perm(t23, t01, 0x06040200u);        // low limbs of tiles 0..3
+                    *reinterpret_cast<uint32_t*>(dst + 16) = __builtin_amdgcn_perm(t23, t01, 0x07050301u);   // high limbs
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            // ---- the values: one code byte over the positions of an operand word by transposing reads
+            typedef __attribute__((address_space(3))) uint8_t* lds8_t;
+            typedef __attribute__((address_space(3))) v2i* lds_v2i_t;
+            v4i wop[NPL], csum = (v4i){0, 0, 0, 0};
+#pragma unroll
+            for (int pl = 0; pl < NPL; pl++) {
+                wop[pl] = *reinterpret_cast<const v4i*>(&mine.wx[pl][lane * 16]);
+                const int cb = pl == 0 ? 0x02020202 : pl == 1 ? 0x04040404 : 0x01010101;
+                csum = __builtin_amdgcn_mfma_i32_16x16x64_i8(wop[pl], (v4i){cb, cb, cb, cb}, csum, 0, 0, 0);
+            }
+            const uint32_t i = lane & 15, A_ = lane >> 4, j = i >> 1;
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                const lds8_t vt = (lds8_t)&mine.vt[e][0];
+                uint32_t y[4];
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const uint32_t B_ = 2 * t + (j >> 2), src = 16 * (j & 3) + 4 * A_ + ((B_ + 2 * A_) & 3);
+                    const v2i r = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_t)(vt + src * 16 + 8 * (i & 1)));
+                    y[2 * t] = (uint32_t)r.x;
+                    y[2 * t + 1] = (uint32_t)r.y;
+                }
+                v4i acc[4];
+#pragma unroll
+                for (int f = 0; f < 4; f++) acc[f] = (v4i){0, 0, 0, 0};
+#pragma unroll
+                for (int pl = 0; pl < NPL; pl++)
+#pragma unroll
+                    for (int f = 0; f < 4; f++) {                            // field 3 is taken at field 2's place: 0x80 would be a negative int8
+                        const uint32_t mask = (pl == 1 ? 0x02020202u : 0x01010101u) << (f == 3 ? 4 : 2 * f);
+                        v4i b;
+#pragma unroll
+                        for (int m = 0; m < 4; m++) {
+                            const uint32_t yp = pl == 2 ? y[m] & (y[m] >> 1) : y[m];
+                            b[m] = (int)((f == 3 ? yp >> 2 : yp) & mask);
+                        }
+                        acc[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wop[pl], b, acc[f], 0, 0, 0);
+                    }
+#pragma unroll
+                for (int hs = 0; hs < 2; hs++)
+#pragma unroll
+                    for (int f = 0; f < 4; f++) {
+                        const int t = (int)(((uint32_t)acc[f][2 * hs + 1] << 8) + (uint32_t)acc[f][2 * hs]);
+                        out[e][f][hs] = __builtin_fmaf((float)t, un[hs] * (f == 0 ? 1.0f : f == 1 ? 0.25f : 0.0625f), out[e][f][hs]);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int hs = 0; hs < 2; hs++) {
+                const int t = (int)(((uint32_t)csum[2 * hs + 1] << 8) + (uint32_t)csum[2 * hs]);
+                sctr[hs] = __builtin_fmaf((float)t, 0.25f * un[hs], sctr[hs]);
+            }
+            if (!more) break;
+            G += nwaves;
+            if (E > 1) gr = load(G);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    // ---- the wave's sums (in place of its operands, which it has read), then all waves'
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int hs = 0; hs < 2; hs++) {
+        const uint32_t h = g + 4 * hs;
+        const float l = lh_group_sum(l_run[hs], 16), w = NPL == 3 ? lh_group_sum(w_run[hs], 16) : 0.0f;
+        if (pcol == 0) { sh.fin_l[wave][h] = l; sh.fin_r[wave][h] = R[hs] <= 0.5f * kNoRef ? -INFINITY : R[hs]; }
+        const float bias = NPL == 3 ? (alpha + 0.5f * (beta + gam) + 0.25f * delta) * w - sctr[hs] : -sctr[hs];
+#pragma unroll
+        for (int e = 0; e < E; e++)
+            *reinterpret_cast<float4*>(&mine.park[h][64 * e + 4 * pcol]) = make_float4(out[e][0][hs] + bias, out[e][1][hs] + bias, out[e][2][hs] + bias, out[e][3][hs] + bias);
+    }
+    lh_lds_barrier();
+    if (wave >= group) return;
+    const float r = lane < nwaves ? sh.fin_r[lane][wave] : -INFINITY, top = lh_group_max(r, 16);
+    const float f = r == -INFINITY ? 0.0f : exp2f(r - top), l = lh_group_sum(lane < nwaves ? f * sh.fin_l[lane][wave] : 0.0f, 16);
+    const ShortWave<S>* const all = &mine - wave;
+    float o[E] = {};
+    for (uint32_t w = 0; w < nwaves; w++) {
+        const float fw = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(f), (int)w));
+#pragma unroll
+        for (int e = 0; e < E; e++) o[e] = __builtin_fmaf(fw, all[w].park[wave][64 * e + lane], o[e]);
+    }
+    const float total = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(l)));
+    float* const dst = a.out + ((size_t)qi * p.num_q_heads + kvh * group + wave) * kDim + kDim / S * blockIdx.x + lane;
+#pragma unroll
+    for (int e = 0; e < E; e++) dst[64 * e] = total > 0.0f ? o[e] / total : 0.0f;
+}
+
+// The leading arguments arrive in registers with the wave (see the Makefile); the structures repeat them.
+template <int S>
+__global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_short_kernel(const float* queries, const float* levels, uint32_t q_heads, uint32_t kv_heads, const AttnPointers a,
+                                                                            const AttnParams p) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    ShortShared& sh = *reinterpret_cast<ShortShared*>(lds);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    ShortWave<S>& mine = reinterpret_cast<ShortWave<S>*>(lds + sizeof(ShortShared))[wave];
+    uint32_t qi = blockIdx.y, kvh = 0, group = q_heads;
+    if (kv_heads != 1) { qi = blockIdx.y / kv_heads; kvh = blockIdx.y - qi * kv_heads; group = q_heads / kv_heads; }
+    // ---- a wave has a head of the query
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (wave < group) x = reinterpret_cast<const float4*>(queries + ((size_t)qi * q_heads + kvh * group + wave) * kDim)[lane];
+    const float L0 = levels[0], L1 = levels[1], L2 = levels[2], L3 = levels[3];
+
+    // ---- the codes and norms of a group.  Lanes whose position is not visible read one that is: nothing of it is used (its weight is zero).
+    uint32_t lo, hi, lane_base;
+    query_range(p, a.positions, qi, lo, hi, lane_base);
+    const uint32_t stride = kv_heads * 64, G = (lo >> 6) + wave, g_last = hi > lo ? (hi - 1) >> 6 : 0u;
+    const bool none = hi <= lo;
+    auto load = [&](uint32_t G_) {
+        Group<S> r;
+        uint32_t at_lane = lane;
+        asm volatile("" : "+v"(at_lane));                       // (a second group's addresses are not to wait in registers for the rare loop that needs them)
+        const uint32_t start = G_ << 6, base = lane_base + (p.ring_capacity ? start % p.ring_capacity : start);
+        r.lo = lo > start ? lo - start : 0u;
+        r.hi = std::min(hi - start, kGroup);
+        auto at = [&](uint32_t i) { return (size_t)(base + std::min(std::max(i, r.lo), r.hi - 1)); };
+#pragma unroll
+        for (int q = 0; q < 4; q++) r.k[q] = ld16(a.k_codes + at(16 * q + (at_lane & 15)) * stride + kvh * 64 + 16 * (at_lane >> 4));
+        r.nk = a.k_norms[at(at_lane) * kv_heads + kvh];
+        r.nv = a.v_norms[at(at_lane) * kv_heads + kvh];
+#pragma unroll
+        for (int e = 0; e < 4 / S; e++) r.v[e] = ld16(a.v_codes + at(at_lane) * stride + kvh * 64 + 16 * (4 / S * blockIdx.x + e));
+        return r;
+    };
+    Group<S> first{};
+    if (!none && G <= g_last) first = load(G);
+
+    // ---- per head: max |q| (quantisation scale) and sum (constant term of the level table)
+    if (wave < kHeads) {
+        sh.q[0][wave][lane] = x.x; sh.q[1][wave][lane] = x.y; sh.q[2][wave][lane] = x.z; sh.q[3][wave][lane] = x.w;
+        const float m = lh_group_max(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))), 64), s = lh_group_sum((x.x + x.y) + (x.z + x.w), 64);
+        if (lane == 0) { sh.maxabs[wave] = m; sh.sum[wave] = s; }
+    }
+    lh_lds_barrier();
+
+    // L[c] = alpha + beta bit0 + gam bit1 + delta bit0 bit1: as in attention_tq_mfma_kernel
+    const float d_raw = (L3 - L2) - (L1 - L0), lmax = fmaxf(fmaxf(fabsf(L0), fabsf(L1)), fmaxf(fabsf(L2), fabsf(L3))), l_mean = 0.25f * ((L0 + L3) + (L1 + L2));
+    const uint32_t end = none ? 0u : g_last, begin = none ? 1u : G;
+    if (fabsf(d_raw) > 1e-5f * lmax || fabsf(l_mean) > 1e-6f * lmax) short_body<3, S>(a, p, sh, mine, first, begin, end, load, L0, L1 - L0, L2 - L0, d_raw, qi, kvh, group);
+    else short_body<2, S>(a, p, sh, mine, first, begin, end, load, L0 - 0.25f * d_raw, (L1 - L0) + 0.5f * d_raw, (L2 - L0) + 0.5f * d_raw, 0.0f, qi, kvh, group);
+}
+
+template <int S> constexpr size_t short_lds(uint32_t waves) { return sizeof(ShortShared) + waves * sizeof(ShortWave<S>); }
+
+template <int S>
+int launch(lh_context* ctx, const char* op, const AttnPointers& a, const AttnParams& p, uint32_t waves) {
+    hipLaunchKernelGGL(attention_tq_short_kernel<S>, dim3(S, p.num_queries * p.num_kv_heads), dim3(64 * waves), short_lds<S>(waves), ctx->stream, a.rq, a.levels,
+                       p.num_q_heads, p.num_kv_heads, a, p);
+    return lh_check_launch(op);
+}
+
+}  // namespace
+
+int lh_attention_short_init(lh_context* ctx) {
+    int r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<4>, short_lds<4>(kMaxWaves), "context_create");
+    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<2>, short_lds<2>(kMaxWaves), "context_create");
+    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<1>, short_lds<1>(kMaxWaves), "context_create");
+    return r;
+}
+
+namespace lh_attn {
+
+bool short_supported(const lh_context* ctx, const AttnParams& p, uint64_t max_span) {
+    static const bool off = [] { return getenv("LOCAL_HIP_ATTN_PAIR") != nullptr; }();      // (forces a form of the other kernel)
+    // A CU for each workgroup, a wave for each group that a span may touch.  (One workgroup a query where the host knows the spans: see `more`.)
+    return !off && p.head_dim == kDim && (uint64_t)p.num_queries * p.num_kv_heads * (p.mode == kBatched ? 2 : 1) <= (uint64_t)ctx->cu_count && (max_span + 62) / 64 + 1 <= kMaxWaves;
+}
+
+int launch_short(lh_context* ctx, const char* op, const AttnPointers& a, AttnParams& p, uint64_t max_span) {
+    p.num_splits = 1;
+    const uint32_t waves = std::max<uint32_t>(kHeads, (uint32_t)((max_span + 62) / 64 + 1)), queries = p.num_queries * p.num_kv_heads, cus = (uint32_t)ctx->cu_count;
+    return queries * 4 <= cus ? launch<4>(ctx, op, a, p, waves) : queries * 2 <= cus ? launch<2>(ctx, op, a, p, waves) : launch<1>(ctx, op, a, p, waves);
+}
+
+}  // namespace lh_attn

@@ -156,6 +156,45 @@ def test_attention_sink_with_flat_tail(pkg, gpu, oracle, T, sink):
     print(f"  err rotated {e1:.2e}, output {e2:.2e}")
 
 
+@pytest.mark.parametrize("mode,n,T,window,ring,nq,nkv,third", [
+    (0, 1, 1, 0, 0, 8, 1, False), (0, 1, 64, 0, 0, 8, 1, False), (0, 1, 705, 0, 0, 8, 1, False), (0, 1, 706, 0, 0, 8, 1, False),     # one group to eleven, and one more
+    (0, 1, 900, 512, 512, 8, 1, False), (0, 1, 3000, 705, 768, 4, 1, True), (0, 1, 500, 65, 0, 6, 2, False),                        # windows off the groups' grid
+    (1, 64, 576, 512, 0, 8, 1, False), (1, 65, 300, 0, 0, 8, 1, True), (1, 33, 200, 0, 0, 12, 2, False), (1, 129, 130, 0, 0, 8, 1, False),
+    (2, 64, 640, 512, 0, 8, 1, False), (2, 65, 200, 100, 0, 8, 1, False), (2, 129, 700, 512, 0, 8, 1, True), (2, 256, 600, 0, 0, 8, 1, False)])
+def test_short_spans(pkg, gpu, oracle, mode, n, T, window, ring, nq, nkv, third):
+    """Spans of one to eleven groups of 64 for queries that fill the chip with four, two and one workgroups each, and the calls next to them."""
+    ctx, K = gpu
+    hd, bits = 256, 2
+    g = np.random.default_rng(T * 7 + n)
+    levels = oracle.tq_levels(hd, bits)
+    if third:
+        levels = levels.copy(); levels[3] += 0.2
+    cap = T + 5 if mode == 1 else 0
+    positions = g.integers(0, T, n).astype(np.uint32); positions[0] = T - 1; positions[-1] = 0
+    if n == 1:
+        positions[0] = T - 1
+    phys = n * cap if mode == 1 else ring or T
+    kc, vc = (g.integers(0, 256, (phys, nkv, hd // 4), dtype=np.uint8) for _ in range(2))
+    kn, vn = ((g.random((phys, nkv), dtype=np.float32) * 4 + 14).astype(np.float16).view(np.uint16) for _ in range(2))
+    rq = g.standard_normal((n, nq * hd), dtype=np.float32) * (0.3 / 16)
+    b = upload(pkg, ctx, kc, kn, vc, vn, levels, rq, positions)
+    out = pkg.Buffer.empty(ctx, rq.nbytes)
+    batch = pkg.CommandBatch(ctx)
+    if mode == 0:
+        K.flash_attention_tq_into(batch, b[5], b[0], b[1], b[2], b[3], b[4], out, hd, T, T - 1, nq, nkv, window, bits, ring)
+    elif mode == 1:
+        K.flash_attention_tq_batched_into(batch, b[5], b[0], b[1], b[2], b[3], b[4], out, b[6], hd, cap, nq, nkv, window, bits, n, 0)
+    else:
+        K.flash_attention_tq_prefill_tiled_into(batch, b[5], b[0], b[1], b[2], b[3], b[4], out, hd, T, T - n, n, nq, nkv, window, bits, ring)
+    batch.commit_and_wait()
+    got = out.as_array(np.float32).reshape(n, nq * hd)
+    for i in sorted({0, n // 2, n - 1}):
+        pos = int(positions[i]) if mode == 1 else T - n + i
+        want = oracle.attention_tq_codespace(rq[i], kc, kn, vc, vn, levels, hd, pos + 1 if mode == 1 else T, pos, nq, nkv, window, bits, ring,
+                                             **({"lane_base": i * cap} if mode == 1 else {}))
+        check(got[i], want, f"query {i}")
+
+
 @pytest.mark.parametrize("seed", [1, 2, 3])
 def test_randomised_shapes_match_oracle(pkg, gpu, oracle, seed):
     """Sixty random shapes per seed -- decode, batched lanes and prefill rows; head_dim 256 / 512; 1, 4, 6 or 8 query heads
