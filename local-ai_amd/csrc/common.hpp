@@ -44,7 +44,7 @@ struct lh_context {
     uint32_t* fault_dev;   // the same word as the device addresses it
     std::atomic<uint64_t> waited;   // launches that the last wait on the stream covers
     // Pinned memory through which lh_buffer_read brings what fits it to the host; one read at a time.
-    static constexpr size_t kReadBytes = (size_t)256 << 10, kReadIdleBytes = (size_t)16 << 10;   // (see lh_buffer_read)
+    static constexpr size_t kReadBytes = (size_t)2 << 20, kReadIdleBytes = (size_t)16 << 10;   // (see lh_buffer_read)
     void* read_host;
     void* read_dev;        // the same memory as the device addresses it
     std::mutex read_mutex;

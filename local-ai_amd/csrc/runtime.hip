@@ -410,10 +410,11 @@ int lh_buffer_write(lh_buffer* buf, size_t offset, const void* src, size_t len) 
     return LH_OK;
 }
 
-// Behind work that is still to run, up to 256 KB are written into pinned memory by a kernel, and the host copies them from there: 4 KB behind a
+// Behind work that is still to run, up to 2 MB are written into pinned memory by a kernel, and the host copies them from there: 4 KB behind a
 // kernel of 29 us are there after 31.4 us, 128 KB after 36.1; through hipMemcpyAsync, which begins when that work has ended, after 38.2 and 45.2.  (The kernel's
-// lead, 9 us, lasts at least to 512 KB; 256 KB is what a context is to hold for it.)  With nothing to wait for the copy is as good from 16 KB on, where
-// the runtime no longer copies twice: 4 KB 13.1 us with the kernel and 22.3 without, 16400 bytes 14.2 and 10.4, 128 KB 18.2 and 15.2.
+// lead is 9 us at 512 KB, 11 at the 1 MB of a large vocabulary's logits -- 97 us and 86 behind a copy of 30 --, 19 at 2 MB, which is what a context holds for it.)
+// With nothing to wait for the copy is as good from 16 KB on, where the runtime no longer copies twice: 4 KB 13.1 us with the kernel and 22.3 without, 16400 bytes
+// 14.2 and 10.4, 128 KB 18.2 and 15.2.
 int lh_buffer_read(const lh_buffer* buf, size_t offset, void* dst, size_t len) {
     if (!buf || (!dst && len)) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_read: null argument");
     if (buf->ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_read: not while a graph is being captured");

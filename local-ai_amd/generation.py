@@ -152,11 +152,17 @@ class PipelineSequences:
         try:
             while lo <= last:
                 if any(p == lo for p in want) or lo == last:
-                    seq.decode_step(int(tokens[lo]))
+                    at = [i for i, p in enumerate(want) if p == lo]
+                    behind = getattr(seq, "decode_step_into", None) if at else None
+                    if behind is not None:
+                        behind(int(tokens[lo]), out[at[0]])
+                    else:
+                        seq.decode_step(int(tokens[lo]))
+                        if at:
+                            seq.logits_buf.read_into(out[at[0]])
                     sure = seq.position
-                    for i, p in enumerate(want):
-                        if p == lo:
-                            seq.logits_buf.read_into(out[i])
+                    for i in at[1:]:
+                        out[i] = out[at[0]]
                     lo += 1
                     continue
                 hi = min([p for p in want if p > lo] + [last, lo + seq.max_batch])

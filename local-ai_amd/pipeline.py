@@ -281,9 +281,18 @@ class DecodePipeline:
 
     def decode_step(self, token: int) -> None:
         """One generated token: forward_token at the current position and the logits tail in one batch, one wait."""
+        self._decode_step(token, None)
+
+    def decode_step_into(self, token: int, logits: np.ndarray) -> None:
+        """The same with the logits (f32[vocab]) read behind the work, in stream order, instead of after a wait for it."""
+        self._decode_step(token, logits)
+
+    def _decode_step(self, token: int, logits: Optional[np.ndarray]) -> None:
         batch = CommandBatch(self.ctx)
         final_in_a = self.forward_token(token, self.position, batch=batch)
         self.write_logits(final_in_a, batch=batch)
+        if logits is not None:
+            self.logits_buf.read_into(logits)
         batch.commit_and_wait()
         self.position += 1
 
