@@ -12,6 +12,7 @@
 // 4g + j - 4 of tile 1, which is the order of the value blocks.  Scores, weights and sums are f32; a weight enters the
 // product as the sum of three bf16 terms, which is all of its 24 bits.
 //   attention_tile_kernel   many rows: four waves share key and value blocks through LDS
+//   attention_one_kernel    one row over up to 640 keys: one workgroup per kv head
 //   attention_split_kernel  few rows: every wave walks its own share of the blocks straight from global memory; the
 //                           workgroup's four partial results are merged in LDS, the workgroups' by attention_merge_kernel
 //   attention_wide_kernel   f32 caches: f32 matrix instructions, 16 packed rows a workgroup
@@ -23,9 +24,7 @@ namespace {
 
 // The B operand of S^T: query values of packed row `row` (zero past the rows and past dim).
 template <int DQ, int MAPS>
-__device__ __forceinline__ void load_queries(lh_bf16x8 (&qf)[MAPS][DQ / 32], const AttentionArgs& a, uint32_t g, uint32_t row, uint32_t lane) {
-    const uint32_t R = a.heads / a.kv_heads, t = row / R, h = g * R + (row - t * R);
-    const bool on = t < a.rows;
+__device__ __forceinline__ void load_queries(lh_bf16x8 (&qf)[MAPS][DQ / 32], const AttentionArgs& a, const void* q, uint32_t th, bool on, uint32_t lane) {
 #pragma unroll
     for (int mp = 0; mp < MAPS; mp++)
 #pragma unroll
@@ -33,7 +32,7 @@ __device__ __forceinline__ void load_queries(lh_bf16x8 (&qf)[MAPS][DQ / 32], con
             const uint32_t k = c * 32 + (lane >> 4) * 8;
             u32x4 v = {0u, 0u, 0u, 0u};
             if (on && k < a.dim) {
-                v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.q) + (((size_t)t * a.heads + h) * MAPS + mp) * DQ + k);
+                v = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(q) + ((size_t)th * MAPS + mp) * DQ + k);
                 if (!(a.scale > 0.0f)) {
 #pragma unroll
                     for (int j = 0; j < 4; j++) v[j] = a.scale < 0.0f ? v[j] ^ 0x80008000u : 0u;      // (no number: scale2 is none either)
@@ -46,6 +45,12 @@ __device__ __forceinline__ void load_queries(lh_bf16x8 (&qf)[MAPS][DQ / 32], con
             }
             qf[mp][c] = __builtin_bit_cast(lh_bf16x8, v);
         }
+}
+
+template <int DQ, int MAPS>
+__device__ __forceinline__ void load_queries(lh_bf16x8 (&qf)[MAPS][DQ / 32], const AttentionArgs& a, uint32_t g, uint32_t row, uint32_t lane) {
+    const uint32_t R = a.heads / a.kv_heads, t = row / R;
+    load_queries<DQ, MAPS>(qf, a, a.q, t * a.heads + g * R + (row - t * R), t < a.rows, lane);
 }
 
 // A finished row: o[i][r] holds value 16 i + 4g + r of packed row (lane & 15), for every map unnormalised with sum l.
@@ -356,6 +361,118 @@ __global__ __launch_bounds__(256) void attention_split_kernel(const AttentionArg
     }
 }
 
+// One row (a decoded token) over a context that one workgroup per kv head gets through: its waves take blocks of 32 keys in turn and meet in LDS, where the rows are
+// finished.  Bound by the chain from the launch to the row and by the 65 GB/s or so that one CU reads, so everything that does not depend on the position is
+// requested ahead of it -- the queries, and a wave's first block whether or not it is visible (it is in the cache) -- and there is no division and no second launch.
+// 16 heads of 64 and 128 over 4 kv heads, two maps, recorded launches: 32 keys 5.6 us, 256 7.9, 512 10.4, 640 11.7, 768 13.1; in the split form with its merge 10.8,
+// 12.2, 12.3, 12.4 and 12.4, and the other way round from kOneBlocks on for 13 heads over one and 16 over 2 or 16 as well.  The leading arguments arrive in registers
+// with the wave; the structure repeats them.
+constexpr int kOneWaves = 8;
+constexpr uint32_t kOneBlocks = 20;
+template <int DQ, int DV, int MAPS>
+__global__ __launch_bounds__(64 * kOneWaves) void attention_one_kernel(const uint16_t* queries, const uint16_t* keys, const uint16_t* values, const uint32_t* position, uint32_t kv_heads,
+                                                                       uint32_t R, uint32_t blocks, const AttentionArgs a) {
+    extern __shared__ __align__(16) float merge[];                          // [waves][MAPS][R rows][DV + 4]: values, maximum, sum
+    constexpr uint32_t kRow = DV + 4;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = kOneWaves, g = blockIdx.x, row = lane & 15;
+    const uint16_t* K = keys + (size_t)g * MAPS * DQ + (lane >> 4) * 8;
+    const uint16_t* V = values + (size_t)g * DV * 32 + ((lane & 15) * 4 + (lane >> 4)) * 8;
+    const size_t krow = (size_t)kv_heads * MAPS * DQ, vblock = (size_t)kv_heads * DV * 32;
+    struct Block { u32x4 k[2][MAPS][DQ / 32], v[DV / 16]; };
+    auto issue = [&](Block& f, uint32_t b) {
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int mp = 0; mp < MAPS; mp++)
+#pragma unroll
+                for (int c = 0; c < DQ / 32; c++) f.k[t][mp][c] = *reinterpret_cast<const u32x4*>(K + (b * 32 + t * 16 + row) * krow + mp * DQ + c * 32);
+#pragma unroll
+        for (int d = 0; d < DV / 16; d++) f.v[d] = *reinterpret_cast<const u32x4*>(V + b * vblock + d * 512);
+    };
+    const uint32_t start = *position;
+    lh_bf16x8 qf[MAPS][DQ / 32];
+    load_queries<DQ, MAPS>(qf, a, queries, g * R + row, row < R, lane);
+    Block x;
+    issue(x, min(wave, blocks - 1));
+    lh_f32x4 o[MAPS][DV / 16];
+    RowState st[MAPS];
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++) {
+        st[mp] = RowState{-INFINITY, 0.0f};
+#pragma unroll
+        for (int d = 0; d < DV / 16; d++) o[mp][d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
+    }
+    const float scale2 = score_scale2(a.scale);
+    const uint32_t limit = min(start, 32 * blocks - 1), nb = limit / 32 + 1;
+    for (uint32_t b = wave; b < nb; b += nwaves) {
+        const bool bound = b * 32 + 31 > limit, more = b + nwaves < nb;
+        lh_bf16x8 w[MAPS][1][3];
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            lh_f32x4 s[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                s[t] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < DQ / 32; c++) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lh_bf16x8, x.k[t][mp][c]), qf[mp][c], s[t], 0, 0, 0);
+            }
+            const float alpha = softmax_step<1>(s, st[mp], scale2, b * 32, limit, bound, lane, w[mp]);
+            if (__ballot(alpha != 1.0f)) {
+#pragma unroll
+                for (int d = 0; d < DV / 16; d++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) o[mp][d][r] *= alpha;
+            }
+        }
+#pragma unroll
+        for (int z = 2; z >= 0; z--)                          // (no product waits for the one before it)
+#pragma unroll
+            for (int d = 0; d < DV / 16; d++)
+#pragma unroll
+                for (int mp = 0; mp < MAPS; mp++) o[mp][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(lh_bf16x8, x.v[d]), w[mp][0][z], o[mp][d], 0, 0, 0);
+        if (more) issue(x, b + nwaves);
+    }
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++) {
+        const float l = lh_column_sum(st[mp].l);
+        float* d0 = merge + ((wave * MAPS + mp) * R + row) * kRow;
+        if (row < R) {
+            if (lane < 16) { d0[DV] = st[mp].m; d0[DV + 1] = l; }
+#pragma unroll
+            for (int d = 0; d < DV / 16; d++) *reinterpret_cast<float4*>(d0 + d * 16 + (lane >> 4) * 4) = make_float4(o[mp][d][0], o[mp][d][1], o[mp][d][2], o[mp][d][3]);
+        }
+    }
+    lh_lds_barrier();
+    constexpr int C = (DV + 63) / 64;                         // a wave finishes a head, C columns a lane
+    for (uint32_t r = wave; r < R; r += nwaves) {
+        const uint32_t h = g * R + r;
+        float v[C];
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            const float2 ml = lane < nwaves ? *reinterpret_cast<const float2*>(merge + ((lane * MAPS + mp) * R + r) * kRow + DV) : make_float2(-INFINITY, 0.0f);
+            const float sink = MAPS == 1 && a.sink ? a.sink[h] * kLog2e : -INFINITY, top = fmaxf(lh_group_max(ml.x, 64), sink);
+            const float f = __builtin_amdgcn_exp2f(ml.x - top), inv = 1.0f / (lh_group_sum(f * ml.y, 64) + __builtin_amdgcn_exp2f(sink - top));
+            float acc[C] = {};
+#pragma unroll
+            for (uint32_t w = 0; w < nwaves; w++) {
+                const float fw = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), (int)w));
+                const float* s = merge + ((w * MAPS + mp) * R + r) * kRow + lane;
+#pragma unroll
+                for (int c = 0; c < C; c++) acc[c] += fw * (DV >= 64 || lane < DV ? s[64 * c] : 0.0f);
+            }
+#pragma unroll
+            for (int c = 0; c < C; c++) v[c] = mp == 0 ? acc[c] * inv : v[c] - a.lambda * (acc[c] * inv);
+        }
+        float ss = 0.0f, f = 1.0f;
+#pragma unroll
+        for (int c = 0; c < C; c++) ss += 64 * c + lane < a.vdim ? v[c] * v[c] : 0.0f;
+        if constexpr (MAPS == 2) f = rsqrtf(lh_group_sum(ss, 64) / (float)a.vdim + a.eps) * a.out_scale;
+        if (MAPS == 1 && a.gate) f = lh_sigmoid(a.gate[h]);
+#pragma unroll
+        for (int c = 0; c < C; c++) if (64 * c + lane < a.vdim) static_cast<uint16_t*>(a.out)[(size_t)h * a.vdim + 64 * c + lane] = lh_f2bf(v[c] * f);
+    }
+}
+
 template <int DQ, int DV, int MAPS>
 int launch_mfma(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const char* op, uint32_t& launches) {
     const uint32_t R = a.heads / a.kv_heads;
@@ -387,6 +504,18 @@ int launch_mfma(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const 
         else hipLaunchKernelGGL((attention_tile_kernel<DQ, DV, MAPS, NB, G>), dim3((uint32_t)(groups * a.splits)), dim3(256 * G), 0, ctx->stream, a);
         const int r = lh_check_launch(op);
         return r != LH_OK || a.splits == 1 ? r : merge();
+    }
+    if constexpr (MAPS * DV <= 256 && DQ + DV <= 448) {       // (what the registers hold)
+        constexpr size_t per_row = (size_t)kOneWaves * MAPS * (DV + 4) * 4;
+        if (a.rows == 1 && R <= 16 && max_blocks <= kOneBlocks && R * per_row <= 160 * 1024) {
+            if (R * per_row > 64 * 1024) {
+                const int r = lh_raise_dynamic_lds(ctx, (const void*)attention_one_kernel<DQ, DV, MAPS>, R * per_row, op);
+                if (r != LH_OK) return r;
+            }
+            hipLaunchKernelGGL((attention_one_kernel<DQ, DV, MAPS>), dim3(a.kv_heads), dim3(64 * kOneWaves), R * per_row, ctx->stream, (const uint16_t*)a.q,
+                               (const uint16_t*)a.keys, (const uint16_t*)a.values, a.position, a.kv_heads, R, a.capacity / 32, a);
+            return lh_check_launch(op);
+        }
     }
     // one block per wave at least, no more workgroups than one per CU
     const uint64_t groups = tiles16 * a.kv_heads;

@@ -477,6 +477,14 @@ def test_attention_finds_one_key_far_away(ai, gpu, dtype, rows, key):
     attention_case(ai, gpu, dtype, 2, 4, 2, 32, 64, 1023, rows, 1344, spike=(0, key))
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("heads,kv_heads,maps,dim,vdim", [(16, 1, 2, 64, 128), (17, 1, 1, 64, 128), (4, 4, 1, 192, 256), (6, 3, 2, 40, 30)])
+@pytest.mark.parametrize("start", [0, 255, 256, 638, 639, 640])
+def test_attention_of_one_row(ai, gpu, dtype, heads, kv_heads, maps, dim, vdim, start):
+    """One block of keys, one and two a wave, the longest context that a workgroup takes and the next; sixteen heads a kv head and seventeen."""
+    attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, 1, (start + 32) // 32 * 32)
+
+
 @pytest.mark.parametrize("rows", [1, 40, 200])
 def test_attention_ignores_what_lies_behind_the_last_position(ai, gpu, rows):
     """Stale rows and block entries past the last position (a slot that is used again) must not change a bit."""
