@@ -16,6 +16,7 @@
 //   attention_split_kernel  few rows: every wave walks its own share of the blocks straight from global memory; the
 //                           workgroup's four partial results are merged in LDS, the workgroups' by attention_merge_kernel
 //   attention_wide_kernel   f32 caches: f32 matrix instructions, 16 packed rows a workgroup
+//   attention_vector_kernel f32 caches, a few rows: the vector ALU, a workgroup per row and head
 // Plain form (any dtype, any dim): attention_plain_kernel, one workgroup per query row and head.
 #include "softmax_attention.hpp"
 #include <type_traits>
@@ -551,8 +552,7 @@ int launch_dv(lh_context* ctx, AttentionArgs& a, uint32_t mp, const char* op, ui
 // A matrix instruction takes one value of k per lane, and which one is free as long as both operands agree: over the dimensions of a
 // head lane group g has its g-th quarter of 16, over the keys of a tile its keys 4 g .. 4 g + 3, which is where S^T leaves the weights
 // and what a value block keeps side by side.  (attention_plain_kernel reads keys a value at a time, every thread its own row: 333 rows
-// of 8 heads with two maps over 64 dimensions, values of 128: 380 us; this form 27 us.  One row as well, though its workgroups are one per
-// kv head: 8 heads of 128 over 1 or 8, 64, 4096 and 16384 keys 9, 165 to 178 and 735 us, in the plain form 21, 665 and 2690.)
+// of 8 heads with two maps over 64 dimensions, values of 128: 380 us; this form 27 us.)
 constexpr uint32_t kWideMaxDim = 256;      // of a key, per map
 template <int DV, int MAPS>
 __global__ __launch_bounds__(256) void attention_wide_kernel(const AttentionArgs a) {
@@ -725,8 +725,127 @@ __global__ __launch_bounds__(256) void attention_wide_kernel(const AttentionArgs
     for (int i = 0; i < TD; i++) if (i * 16 + lr < a.vdim) out[i * 16 + lr] = v[i] * z;
 }
 
+// f32 queries, keys and values of a few rows on the vector ALU: a workgroup per row and head, its waves the blocks of 32 keys in turn.  Every load covers consecutive
+// memory: sixteen lanes a key row, four dimensions each, whose products are added between lanes; eight lanes a column of the value block, four entries each, whose sums
+// stay in the lanes until the end.  (With a key and a column a lane the 64 cache lines of every load bound it: 337 keys 15.5 us.)  Products and sums are FMA.
+// (The matrix form fills 16 rows whether or not there are any and walks a context on four waves of one CU per kv head: 16 heads over 4 kv heads, two maps, 1 row of 337
+// keys 25.7 us, 9.6 here; 16 rows of 1024 keys 66 and 17, one row of 4096 241 and 53.)
+template <int DV, int MAPS>
+__global__ __launch_bounds__(512) void attention_vector_kernel(const float* queries, const float* keys, const float* values, const uint32_t* position, uint32_t kv_heads, uint32_t heads,
+                                                               uint32_t dq, const AttentionArgs a) {
+    constexpr int WAVES = 8, NV = DV / 8;                     // loads of a value block
+    __shared__ __align__(16) float ps[WAVES][MAPS][32], sums[WAVES][MAPS][DV];
+    __shared__ float ms[WAVES][MAPS], ls[WAVES][MAPS], scratch[WAVES];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, key = lane & 31, part = lane & 15;
+    const uint32_t h = blockIdx.x % heads, t = blockIdx.x / heads, g = h / (heads / kv_heads);
+    const size_t th = (size_t)t * heads + h;
+    const uint32_t limit = min(*position + t, a.capacity - 1), nb = limit / 32 + 1;
+    const size_t krow = (size_t)kv_heads * MAPS * dq, vblock = (size_t)kv_heads * DV * 32;
+    const float *V = values + (size_t)g * DV * 32 + 4 * lane, *K = keys + (size_t)g * MAPS * dq;
+    float m = -INFINITY, l = 0.0f, acc[MAPS][NV] = {};
+    const uint32_t mp_of = MAPS == 2 ? half : 0u;
+    for (uint32_t b = wave; b < nb; b += WAVES) {
+        const bool bound = b * 32 + 31 > limit;
+        lh_f32x4 v[NV];
+#pragma unroll
+        for (int i = 0; i < NV; i++) v[i] = *reinterpret_cast<const lh_f32x4*>(V + b * vblock + 256 * i);
+        float s = 0.0f;                                       // of key `key`, map mp_of
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            float sum[8] = {};                                // of key 4 i + lane / 16
+            for (uint32_t c = part; c < dq / 4 + part; c += 16) {
+                const uint32_t at = 4 * min(c, dq / 4 - 1);
+                lh_f32x4 x[8], q4 = *reinterpret_cast<const lh_f32x4*>(queries + (th * MAPS + mp) * dq + at);
+#pragma unroll
+                for (int i = 0; i < 8; i++) x[i] = *reinterpret_cast<const lh_f32x4*>(K + min(b * 32 + 4 * i + (lane >> 4), limit) * krow + mp * dq + at);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const bool in = c < dq / 4 && 4 * c + j < a.dim;    // (what pads a key row may be anything)
+                    q4[j] = in ? q4[j] : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 8; i++) sum[i] = __builtin_fmaf(in ? x[i][j] : 0.0f, q4[j], sum[i]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) sum[i] = lh_group_sum(sum[i], 16);
+            __builtin_amdgcn_wave_barrier();
+            if (part == 0)
+#pragma unroll
+                for (int i = 0; i < 8; i++) ps[wave][mp][4 * i + (lane >> 4)] = sum[i];
+            __builtin_amdgcn_wave_barrier();
+        }
+        s = ps[wave][mp_of][key] * a.scale;
+        if (b * 32 + key > limit) s = -INFINITY;
+        const float nm = fmaxf(m, lh_group_max(s, 32)), base = nm == -INFINITY ? 0.0f : nm, alpha = expf(m - base), p = expf(s - base);
+        l = l * alpha + lh_group_sum(p, 32);
+        m = nm;
+        __builtin_amdgcn_wave_barrier();
+        if (MAPS == 2 || half == 0) ps[wave][mp_of][lh_block_slot(key)] = p;
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t slot = 4 * (lane & 7);                 // the lane's four entries of every column: keys 4 (slot / 8) + 16 (slot / 4 % 2) + 0 .. 3
+        if (bound) {                                          // entries behind the row's last key may be anything
+            const uint32_t first = b * 32 + 4 * (slot >> 3) + 16 * ((slot >> 2) & 1);
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[i][j] = first + j > limit ? 0.0f : v[i][j];
+        }
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            const float al = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, alpha), 32 * mp));
+            const lh_f32x4 w4 = *reinterpret_cast<const lh_f32x4*>(&ps[wave][mp][slot]);
+#pragma unroll
+            for (int i = 0; i < NV; i++) {
+                acc[mp][i] *= al;
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[mp][i] = __builtin_fmaf(v[i][j], w4[j], acc[mp][i]);
+            }
+        }
+    }
+    if (key == 0 && (MAPS == 2 || half == 0)) { ms[wave][mp_of] = m; ls[wave][mp_of] = l; }
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++)
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const float x = lh_group_sum(acc[mp][i], 8);
+            if ((lane & 7) == 0) sums[wave][mp][8 * i + (lane >> 3)] = x;
+        }
+    __syncthreads();
+    float out = 0.0f;
+    if (tid < DV) {
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            const float sink = MAPS == 1 && a.sink ? a.sink[h] : -INFINITY;
+            float top = sink;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) top = fmaxf(top, ms[w][mp]);
+            float total = expf(sink - top), x = 0.0f;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
+                const float f = expf(ms[w][mp] - top);
+                total += f * ls[w][mp];
+                x += f * sums[w][mp][tid];
+            }
+            x /= total;
+            out = mp == 0 ? x : out - a.lambda * x;
+        }
+        if (tid >= a.vdim) out = 0.0f;
+    }
+    float z = 1.0f;
+    if constexpr (MAPS == 2) z = rsqrtf(lh_block_sum(out * out, scratch) / (float)a.vdim + a.eps) * a.out_scale;
+    if (MAPS == 1 && a.gate) z = lh_sigmoid(a.gate[th]);
+    if (tid < a.vdim) static_cast<float*>(a.out)[th * a.vdim + tid] = out * z;
+}
+
 template <int DV, int MAPS>
 int launch_wide(lh_context* ctx, const AttentionArgs& a, const char* op) {
+    // Up to a workgroup a CU of the vector form, which is the faster one at every context and head measured there (16 rows of 16 heads over 4 kv heads, two maps: 32 keys
+    // 13.3 us and 6.2, 337 27.0 and 9.8, 4096 242 and 49); two maps of 256 columns would not fit its registers.
+    if constexpr (MAPS * DV <= 256) if ((uint64_t)a.rows * a.heads <= (uint64_t)ctx->cu_count) {
+        hipLaunchKernelGGL((attention_vector_kernel<DV, MAPS>), dim3(a.rows * a.heads), dim3(512), 0, ctx->stream, (const float*)a.q, (const float*)a.keys, (const float*)a.values,
+                           a.position, a.kv_heads, a.heads, a.dq, a);
+        return lh_check_launch(op);
+    }
     const uint64_t grid = ((uint64_t)a.rows * (a.heads / a.kv_heads) + 15) / 16 * a.kv_heads;
     LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: %u rows", op, a.rows);
     const size_t lds = std::max<size_t>((size_t)MAPS * 16 * (a.dq + 4), (size_t)4 * MAPS * 16 * (DV + 4)) * 4;
