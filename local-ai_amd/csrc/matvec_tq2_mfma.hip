@@ -71,6 +71,8 @@ struct Tq2Base {
     uint32_t xstride, ystride;   // bytes
     uint64_t mstride = 0;        // bytes between the matrices of consecutive problems (0: one matrix for all of them)
     uint32_t split_waves = 0;    // split form: waves that share the block groups of one tile (0: all waves of the workgroup)
+    uint32_t share = 0, left = 0;   // slots of a workgroup, and how many workgroups have one more
+    uint32_t runs = 0;           // a workgroup's slots lie side by side (0: dealt one by one)
     // A pair of unrelated problems (gate and up) also travels here, so the common grouped launch needs no
     // descriptor upload ahead of it.
     Tq2Problem second = {nullptr, nullptr, nullptr};
@@ -144,8 +146,13 @@ __global__ __launch_bounds__(MAXT, MAXT == 256 ? 2 : 1) void matvec_tq2_mfma_ker
     uint32_t slot_seq = 0;                                                      // tiles this wave has completed (split form)
     uint8_t* image = lds + zero_off + 128 + (size_t)wave * kImageBytes;         // this wave's tile image
 
-    // Work order: "slots" of nwaves consecutive tiles, dealt round-robin to the workgroups, so that at any moment
-    // the whole grid reads one compact, advancing window of the weight stream.
+    // Work order: "slots" of nwaves consecutive tiles.  Problems of one vector, and one matrix's several vectors, are dealt
+    // round-robin to the workgroups, so that at any moment the whole grid reads one compact, advancing window of the weight
+    // stream.  Problems with a vector each are dealt in runs, a workgroup's slots side by side: it stages a vector once or
+    // twice instead of with almost every slot, and a staging waits for all loads of the workgroup and lets none out behind
+    // it.  (128 products of 8192 x 2048: 127 us round-robin, 112 in runs, 105 with one vector for all; 128 of 2048 x 8192:
+    // 173, 116, 111; 100 of 2048 x 6144: 102, 76, 74.  In runs with one vector for all, 105 -> 107, 111 -> 112.5 and
+    // 64 of 8192 x 4096 114 -> 116; eight vectors and one matrix of 262144 x 2048, 180 -> 195.)
     const uint32_t tiles_per_problem = (rows + 15) >> 4;
     // Normally a slot is nwaves consecutive tiles, one per wave, each wave walking all block groups of its tile.  With
     // `splitk` (few tiles, long rows) a slot is ONE tile whose block groups are dealt to the waves (nwaves divides their
@@ -156,11 +163,11 @@ __global__ __launch_bounds__(MAXT, MAXT == 256 ? 2 : 1) void matvec_tq2_mfma_ker
     const uint32_t tps = splitk ? (uint32_t)nwaves / sw : (uint32_t)nwaves;                          // tiles per slot
     const uint32_t tsub = splitk ? (uint32_t)wave / sw : (uint32_t)wave;                             // this wave's tile of the slot
     const uint32_t slots_per_problem = (tiles_per_problem + tps - 1) / tps;
-    const uint64_t total_slots = (uint64_t)slots_per_problem * count;
     const uint32_t ngroups = (nb + 7) >> 3;
-    const uint64_t my_slots = blockIdx.x < total_slots ? (total_slots - blockIdx.x + gridDim.x - 1) / gridDim.x : 0;
+    const uint32_t my_slots = single.share + (blockIdx.x < single.left ? 1u : 0u);
+    const uint32_t first_slot = single.runs ? blockIdx.x * single.share + min(blockIdx.x, single.left) : blockIdx.x;
     const uint32_t grp0 = splitk ? (uint32_t)wave % sw : 0u, grp_step = sw;
-    const uint32_t nitems = (uint32_t)(my_slots * (ngroups / grp_step));   // one item = one (tile, block group); the host keeps a launch's total under 2^32
+    const uint32_t nitems = my_slots * (ngroups / grp_step);   // one item = one (tile, block group); the host keeps a workgroup's total under 2^32
 
     // Chunk -> (row, chunk-in-row) of the lane's staging loads.  Full groups of 8 blocks (33 chunks per row): the global
     // offsets live in registers and the image offsets are linear in the chunk index.  The trailing group of nb % 8
@@ -178,7 +185,7 @@ __global__ __launch_bounds__(MAXT, MAXT == 256 ? 2 : 1) void matvec_tq2_mfma_ker
         pro_words[threadIdx.x] = reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(&cold_kernargs()->single.pro)[threadIdx.x];
     // Position in the work order, advanced incrementally (all scalar, no division in the loop).
     struct Item { uint32_t grp, sip, prob; };                       // block group, slot within the problem, problem
-    const uint32_t step_prob = gridDim.x / slots_per_problem, step_sip = gridDim.x % slots_per_problem;
+    const uint32_t step_prob = single.runs ? 0u : gridDim.x / slots_per_problem, step_sip = single.runs ? 1u : gridDim.x % slots_per_problem;
     auto advance = [&](Item it) {
         it.grp += grp_step;
         if (it.grp >= ngroups) {
@@ -197,7 +204,7 @@ __global__ __launch_bounds__(MAXT, MAXT == 256 ? 2 : 1) void matvec_tq2_mfma_ker
         else pb = Tq2Problem{single.p.matrix + (size_t)it.prob * single.mstride, (const char*)single.p.vector + (size_t)it.prob * single.xstride,
                              (char*)single.p.output + (size_t)it.prob * single.ystride};
     };
-    Item cur{grp0, blockIdx.x % slots_per_problem, blockIdx.x / slots_per_problem};
+    Item cur{grp0, first_slot % slots_per_problem, first_slot / slots_per_problem};
 
     u32x4_t pre[kStageLoads];
     // `offs`: the lane's nine chunk offsets of a full group, read from full_tab by the caller ahead of the call (at the top of
@@ -524,6 +531,11 @@ int lh_launch_matvec_tq2_mfma(lh_context* ctx, uint32_t count, const void* const
     Tq2Base single{Tq2Problem{(const uint8_t*)matrices[0], vectors[0], outputs[0]}, xstride, ystride};
     single.mstride = mstride;
     single.split_waves = wide_split;
+    single.share = (uint32_t)(slots / grid);
+    single.left = (uint32_t)(slots % grid);
+    bool own_vectors = strided && mstride != 0 && xstride != 0;   // a matrix and a vector a problem
+    for (uint32_t i = 1; !strided && i < count && !own_vectors; i++) own_vectors = vectors[i] != vectors[0];
+    single.runs = own_vectors && slots <= 0xFFFFFFFFull ? 1u : 0u;
     single.pro = pro;
     single.spin_limit = g_tq2_spin_limit.load(std::memory_order_relaxed);
     single.fault = ctx->fault_dev;

@@ -559,6 +559,35 @@ def test_grouped_long_f16_problems_with_their_own_vectors(pkg, gpu, oracle, rows
         refgen.assert_close(y.as_array(np.float16, rows).astype(np.float32), oracle.matvec_quant_ref("tq2_0", r, x.astype(np.float32), rows, cols, threads=8), 2e-3, f"{rows} x{count}")
 
 
+@pytest.mark.parametrize("rows,cols,count,apart", [(100, 2048, 300, True), (1000, 2048, 100, False), (2064, 2048, 29, True), (1, 256, 5, True),
+                                                   (17, 1536, 1000, False), (2040, 8192, 49, True), (70, 4096, 3, False)])
+def test_grouped_problems_with_a_vector_each(pkg, gpu, oracle, rows, cols, count, apart):
+    """Each problem its own matrix and vector: a workgroup takes a run of neighbouring slots, which may begin and end inside
+    a problem and span several; fewer slots than workgroups, one more here and there, partial tiles, surplus waves; wherever
+    the problems lie or evenly spaced."""
+    ctx, K = gpu
+    g, wb = pkg.synth.rng(61, rows + cols), pkg.synth.weight_bytes("tq2_0", rows, cols)
+    raws = [pkg.synth.weights("tq2_0", rows, cols, g) for _ in range(3)]
+    hosts = [pkg.synth.activations(1, cols, g)[0] for _ in range(4)]
+    wants = {(i, j): oracle.matvec_quant_ref("tq2_0", raws[i], hosts[j], rows, cols, threads=8) for i in range(3) for j in range(4)}
+    gap = 64 if apart else 0
+    big, xs = pkg.Buffer.empty(ctx, (wb + gap) * count), pkg.Buffer.empty(ctx, (cols * 4 + gap) * count)
+    yall = pkg.Buffer.from_slice(ctx, np.full(count * rows, np.nan, np.float32))
+    order = list(range(count))
+    if apart:
+        order = [int(i) for i in g.permutation(count)]
+    for n, at in enumerate(order):
+        big.copy_from_bytes(raws[n % 3], at * (wb + gap))
+        xs.copy_from_bytes(hosts[n % 4], at * (cols * 4 + gap))
+    batch = pkg.CommandBatch(ctx)
+    K.matvec_quant_grouped_into(batch, pkg.TQ2_0, [big.view(at * (wb + gap), wb) for at in order], [xs.view(at * (cols * 4 + gap), cols * 4) for at in order],
+                                pkg.F32, [yall.view(n * rows * 4, rows * 4) for n in range(count)], pkg.F32, rows, cols)
+    batch.commit_and_wait()
+    got = yall.as_array(np.float32, count * rows).reshape(count, rows)
+    for n in range(count):
+        refgen.assert_close(got[n], wants[n % 3, n % 4], 1e-3, f"{rows}x{cols} x{count} problem {n}")
+
+
 @pytest.mark.parametrize("rows,cols,count,shared_x,half", [(2048, 8192, 52, True, False), (1024, 4096, 100, False, False),
                                                            (2032, 8192, 52, True, False), (2048, 8192, 52, False, True)])
 def test_grouped_long_rows_many_tiles(pkg, gpu, oracle, rows, cols, count, shared_x, half):
