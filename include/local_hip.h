@@ -661,6 +661,9 @@ LH_API uint32_t lh_flash_split_count(uint32_t eff_seq_len);
 /* output[r] = table[rows[r]] as f32 (row index clamped to the last row) */
 LH_API int lh_embed_rows_bf16_into(lh_batch* batch, const lh_buffer* table, uint32_t table_rows, uint32_t cols,
                                    const lh_buffer* rows, uint32_t n_rows, lh_buffer* output);
+/* output = table[token] as f32 (clamped to the last row); *at = position and *next = position + 1 (u32) */
+LH_API int lh_embed_token_bf16_into(lh_batch* batch, const lh_buffer* table, uint32_t table_rows, uint32_t cols,
+                                    uint32_t token, uint32_t position, lh_buffer* output, lh_buffer* at, lh_buffer* next);
 /* t = input[row] (+ add[row]), stored to `store` when given (may be `input`); output = t / sqrt(mean(t^2) + eps) * weight.
  * `row_index` (device u32, may be null) picks the input rows. */
 LH_API int lh_norm_rows_f32_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* add, const lh_buffer* weight,

@@ -824,6 +824,10 @@ class Kernels:
     def embed_rows_bf16_into(self, batch, table, table_rows, cols, rows, n_rows, output):
         _check(self._l.lh_embed_rows_bf16_into(batch._h, table._h, _u32(table_rows), _u32(cols), rows._h, _u32(n_rows), output._h))
 
+    def embed_token_bf16_into(self, batch, table, table_rows, cols, token, position, output, at, next):
+        _check(self._l.lh_embed_token_bf16_into(batch._h, table._h, _u32(table_rows), _u32(cols), _u32(token), _u32(position), output._h, at._h,
+                                                next._h))
+
     def norm_rows_f32_into(self, batch, input, add, weight, store, row_index, output, output_dtype, dim, rows, eps):
         _check(self._l.lh_norm_rows_f32_into(batch._h, input._h, _opt(add), weight._h, _opt(store), _opt(row_index), output._h,
                                              C.c_int(output_dtype), _u32(dim), _u32(rows), C.c_float(eps)))

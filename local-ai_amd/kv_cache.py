@@ -365,8 +365,14 @@ class SequenceSlot:
         self.memories = memories
         self.position_buf = Buffer.empty(ctx, 4)
         self.position = 0
-        # the slot's recorded decode step, the scratch it was recorded with, and whether a step has run unrecorded
-        self.graph, self.graph_version, self.graph_ready = None, -1, False
+        # the slot's recorded decode steps, with the pick of the next token and without, each with the version of the scratch it was
+        # recorded with; and whether a step has run unrecorded
+        self.graphs, self.graph_ready = {}, False
+
+    @property
+    def graph(self):
+        """The recorded step: the one that picks, if there is one."""
+        return next((self.graphs[pick][0] for pick in (True, False) if pick in self.graphs), None)
 
     def reset(self) -> None:
         for m in {id(m): m for m in self.memories}.values():      # layers may share one

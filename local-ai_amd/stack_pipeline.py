@@ -84,6 +84,7 @@ class StackPipeline:
         self.tokens_buf = Buffer.empty(ctx, 4 * max_rows)
         self.logits_buf = Buffer.empty(ctx, 4 * config.vocab)
         self.next_buf = Buffer.empty(ctx, 4)
+        self.at_buf = Buffer.empty(ctx, 4)                # where the token of a step stands
         self.slots = SlotPool(self._new_slot, max_sequences)
         self.observe = None          # called with (run index, residual stream buffer, rows) after every layer run
 
@@ -134,7 +135,7 @@ class StackPipeline:
         """One decoded token whose successor is picked on the device."""
         if seq.position + 1 > self.max_tokens:
             raise InvalidArgument(f"position {seq.position + 1} beyond the {self.max_tokens} tokens of a sequence")
-        batch = self._decode(seq, token)
+        batch = self._decode(seq, token, pick=True)
         picked = int(self.next_buf.as_array(np.uint32, 1)[0])
         self._finish(batch, seq, 1)
         return picked
@@ -144,11 +145,14 @@ class StackPipeline:
         """Embedding and all layer runs of the n tokens in tokens_buf; returns the residual stream.  The embedding output
         stays as it is (later passes of a loop add it): the first norm leaves the stream in a buffer of its own.  For one
         token a norm may not write what other workgroups still read, so the stream alternates between two buffers."""
+        x0 = self.ws.get("embedded", n * self.config.width * 4)
+        self.kernels.embed_rows_bf16_into(batch, self.embed, self.vocab_size, self.config.width, self.tokens_buf, n, x0)
+        return self._encode_layers(batch, seq, n, max_position, x0, seq.position_buf)
+
+    def _encode_layers(self, batch, seq: SequenceSlot, n: int, max_position: int, x0: Buffer, position: Buffer) -> Buffer:
         K, width = self.kernels, self.config.width
-        x0 = self.ws.get("embedded", n * width * 4)
         x, y = self.ws.get("stream", n * width * 4), self.ws.get("stream.other", width * 4)
-        K.embed_rows_bf16_into(batch, self.embed, self.vocab_size, width, self.tokens_buf, n, x0)
-        r = Run(K, batch, n, self.ws, self.dtype, seq.position_buf, max_position, x0, None, x)
+        r = Run(K, batch, n, self.ws, self.dtype, position, max_position, x0, None, x)
         for i, ((layer, add), memory) in enumerate(zip(self.runs, seq.memories)):
             if add:
                 r.add = x0
@@ -164,7 +168,7 @@ class StackPipeline:
         """Results are read behind the work, in stream order: one wait for both, and for all pieces of a step."""
         n = len(tokens)
         if n == 1 and self.observe is None:
-            batch = self._decode(seq, int(tokens[0]))
+            batch = self._decode(seq, int(tokens[0]), pick=False)
             if want:
                 self.logits_buf.read_into(out[0])
                 out[1:] = out[0]
@@ -209,29 +213,49 @@ class StackPipeline:
         if self.config.softcap is not None:
             self.kernels.softcap_f32_into(batch, logits, rows * self.vocab_size, self.config.softcap)
 
-    def _encode_decode(self, batch, seq: SequenceSlot, max_position: int) -> None:
-        self._encode_head(batch, self._encode_stack(batch, seq, 1, max_position))
-        self.kernels.argmax_advance_f32_into(batch, self.logits_buf, self.next_buf, self.vocab_size, seq.position_buf, 1)
-
-    def _decode(self, seq: SequenceSlot, token: int) -> CommandBatch:
-        """One token, encoded: logits in logits_buf, the largest one's index in next_buf.  The first decoded token of a slot runs
-        dispatch by dispatch, the next one records the step into a graph that later ones replay as long as the scratch buffers
-        stay where they are (everything that changes from step to step is in device memory)."""
-        batch = CommandBatch(self.ctx)
-        batch.write(self.tokens_buf, np.asarray([token], np.uint32))
-        if seq.graph is not None and seq.graph_version == self.ws.version:
-            seq.graph.launch()
-        elif self.graphs and seq.graph_ready:
-            seq.graph = None
-            batch.begin_capture()
-            try:
-                self._encode_decode(batch, seq, self.max_tokens - 1)
-            except BaseException:
-                batch.end_capture()
-                raise
-            seq.graph, seq.graph_version = batch.end_capture(), self.ws.version
-            seq.graph.launch()
+    def _encode_decode(self, batch, seq: SequenceSlot, max_position: int, pick: bool) -> None:
+        if pick:
+            self._encode_head(batch, self._encode_stack(batch, seq, 1, max_position))
+            self.kernels.argmax_advance_f32_into(batch, self.logits_buf, self.next_buf, self.vocab_size, seq.position_buf, 1)
         else:
-            self._encode_decode(batch, seq, seq.position)
-            seq.graph_ready = True
+            x0 = self.ws.get("embedded", self.config.width * 4)
+            self._encode_head(batch, self._encode_layers(batch, seq, 1, max_position, x0, self.at_buf))
+
+    def _decode(self, seq: SequenceSlot, token: int, pick: bool) -> CommandBatch:
+        """One token, encoded: logits in logits_buf and, where asked, the largest one's index in next_buf.  The first decoded token of a
+        slot runs dispatch by dispatch, the next one records the step into a graph that later ones replay as long as the scratch buffers
+        stay where they are (everything that changes from step to step is in device memory).  Without the pick a launch ahead of the
+        recorded ones brings the token's row and position, by value, and counts the sequence on."""
+        batch = CommandBatch(self.ctx)
+        if pick:
+            batch.write(self.tokens_buf, np.asarray([token], np.uint32))
+        else:
+            width = self.config.width
+            self.kernels.embed_token_bf16_into(batch, self.embed, self.vocab_size, width, token, seq.position,
+                                               self.ws.get("embedded", width * 4), self.at_buf, seq.position_buf)
+        try:
+            self._launch_decode(batch, seq, pick)
+        except BaseException:
+            if not pick:
+                batch.write(seq.position_buf, np.asarray([seq.position], np.uint32))
+            raise
         return batch
+
+    def _launch_decode(self, batch, seq: SequenceSlot, pick: bool) -> None:
+        graph, version = seq.graphs.get(pick, (None, -1))
+        if graph is not None and version == self.ws.version:
+            return graph.launch()
+        if not (self.graphs and seq.graph_ready):
+            self._encode_decode(batch, seq, seq.position, pick)
+            seq.graph_ready = True
+            return
+        seq.graphs.pop(pick, None)
+        batch.begin_capture()
+        try:
+            self._encode_decode(batch, seq, self.max_tokens - 1, pick)
+        except BaseException:
+            batch.end_capture()
+            raise
+        graph = batch.end_capture()
+        seq.graphs[pick] = graph, self.ws.version
+        graph.launch()

@@ -170,6 +170,7 @@ extern "C" {
     pub fn lh_flash_attention_windowed_split_into(batch: *mut lh_batch, q: *const lh_buffer, k: *const lh_buffer, v: *const lh_buffer, output: *mut lh_buffer, partial_max: *mut lh_buffer, partial_sum: *mut lh_buffer, partial_acc: *mut lh_buffer, head_dim: u32, kv_len: u32, current_pos: u32, num_q_heads: u32, num_kv_heads: u32, window: u32, num_splits: u32) -> c_int;
     pub fn lh_flash_split_count(eff_seq_len: u32) -> u32;
     pub fn lh_embed_rows_bf16_into(batch: *mut lh_batch, table: *const lh_buffer, table_rows: u32, cols: u32, rows: *const lh_buffer, n_rows: u32, output: *mut lh_buffer) -> c_int;
+    pub fn lh_embed_token_bf16_into(batch: *mut lh_batch, table: *const lh_buffer, table_rows: u32, cols: u32, token: u32, position: u32, output: *mut lh_buffer, at: *mut lh_buffer, next: *mut lh_buffer) -> c_int;
     pub fn lh_norm_rows_f32_into(batch: *mut lh_batch, input: *const lh_buffer, add: *const lh_buffer, weight: *const lh_buffer, store: *mut lh_buffer, row_index: *const lh_buffer, output: *mut lh_buffer, output_dtype: c_int, dim: u32, rows: u32, eps: f32) -> c_int;
     pub fn lh_residual_rows_into(batch: *mut lh_batch, input: *const lh_buffer, branch: *const lh_buffer, weight: *const lh_buffer, store: *mut lh_buffer, output: *mut lh_buffer, output_dtype: c_int, dim: u32, rows: u32, eps: f32) -> c_int;
     pub fn lh_gated_norm_rows_into(batch: *mut lh_batch, input: *const lh_buffer, gate: *const lh_buffer, gate_act: u32, gate_first: c_int, weight: *const lh_buffer, output: *mut lh_buffer, dtype: c_int, dim: u32, group: u32, rows: u32, eps: f32) -> c_int;

@@ -524,6 +524,13 @@ impl Kernels {
         check(unsafe { ffi::lh_embed_rows_bf16_into(batch.as_ptr(), table.as_ptr(), table_rows, cols, rows.as_ptr(), n_rows, output.as_ptr()) })
     }
 
+    /// `lh_embed_token_bf16_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn embed_token_bf16_into(&self, batch: &mut CommandBatch, table: &Buffer, table_rows: u32, cols: u32, token: u32, position: u32, output: &Buffer, at: &Buffer, next: &Buffer) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_embed_token_bf16_into(batch.as_ptr(), table.as_ptr(), table_rows, cols, token, position, output.as_ptr(), at.as_ptr(), next.as_ptr()) })
+    }
+
     /// `lh_norm_rows_f32_into` (include/local_hip.h).
     #[allow(clippy::too_many_arguments)]
     pub fn norm_rows_f32_into(&self, batch: &mut CommandBatch, input: &Buffer, add: &Buffer, weight: &Buffer, store: &Buffer, row_index: &Buffer, output: &Buffer, output_dtype: c_int, dim: u32, rows: u32, eps: f32) -> Result<()> {

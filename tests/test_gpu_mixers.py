@@ -53,6 +53,20 @@ def values_from_cache(flat, cols):
 
 
 # ---- products ----------------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("cols,shift", [(1, 0), (4, 0), (7, 0), (1023, 0), (1024, 0), (1028, 0), (2048, 1), (5000, 0)])
+def test_embed_token(ai, gpu, cols, shift):
+    ctx, K = gpu
+    table = M.rounded(np.random.default_rng(cols).standard_normal((5, cols)))
+    tb = ai.Buffer.from_slice(ctx, np.concatenate([np.zeros(shift, np.uint16), M.bf16_bits(table).reshape(-1)])).view(2 * shift, 10 * cols)
+    out, at, then, batch = ai.Buffer.from_slice(ctx, np.full(cols + 4, 7, np.float32)), ai.Buffer.empty(ctx, 4), ai.Buffer.empty(ctx, 4), ai.CommandBatch(ctx)
+    for token in (3, 0, 4, 9):
+        K.embed_token_bf16_into(batch, tb, 5, cols, token, 40 + token, out, at, then)
+        batch.commit_and_wait()
+        got = out.as_array(np.float32, cols + 4)
+        assert np.array_equal(got[:cols], table[min(token, 4)]) and (got[cols:] == 7).all()
+        assert at.as_array(np.uint32, 1)[0] == 40 + token and then.as_array(np.uint32, 1)[0] == 41 + token
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("m,k,n", [(1, 64, 48), (2, 256, 200), (31, 72, 33), (33, 40, 70), (64, 520, 130), (65, 64, 64), (129, 200, 257),
                                    (300, 136, 2052), (7, 60, 45), (140, 7, 9), (2100, 128, 2048),

@@ -296,6 +296,33 @@ def test_recorded_decoding_equals_unrecorded_bit_for_bit(ai, gpu, name, n, capac
     assert rec_a and not rec_b and np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("name", ["both", "latent_and_states"])
+def test_steps_and_picks_in_turn(ai, gpu, name):
+    """Portions, single tokens and picks in any order, two sequences in turn: the three keep one count of positions, and the two recorded
+    steps of a slot do not disturb each other.  Against the same calls unrecorded."""
+    cfg, _, m = build(ai, gpu, name, "bfloat16", max_tokens=63, max_sequences=2)
+    _, _, plain = build(ai, gpu, name, "bfloat16", max_tokens=63, max_sequences=2, graphs=False)
+    tokens = [int(t) for t in np.random.default_rng(13).integers(0, cfg["vocab"], 64)]
+    calls = [5, 1, 1, "pick", "pick", "pick", 1, 3, "pick", 1, 1, 2, 1, "pick"]
+
+    def run(model):
+        live, out = [[model.new_sequence(), 0], [model.new_sequence(), 0]], []
+        for call in calls:
+            for l in live:
+                s, at = l
+                if call == "pick":
+                    out.append(np.array([model.greedy(s, tokens[at])]))
+                else:
+                    out.append(model.step(s, tokens[at:at + call], [call - 1]))
+                l[1] += 1 if call == "pick" else call
+                assert s.position == l[1] and s.position_buf.as_array(np.uint32, 1)[0] == l[1]
+        for s, _ in live:
+            model.end_sequence(s)
+        return out
+    for i, (a, b) in enumerate(zip(run(m), run(plain))):
+        assert np.array_equal(a, b), i
+
+
 @pytest.mark.parametrize("name", ["loop_all", "latent_and_states"])
 def test_long_decoding(ai, gpu, name):
     cfg, w, m = build(ai, gpu, name, max_tokens=700)
