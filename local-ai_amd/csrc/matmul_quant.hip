@@ -955,6 +955,96 @@ __global__ __launch_bounds__(256, 2) void matmul_skinny_kernel(const uint16_t* _
     }
 }
 
+// ---- a few weight rows behind many: the gate of the per-layer inputs with its GeGLU ------------------------------------------------
+// out = half(gelu(half(X . W^T)) * gate), gate read out of longer rows.  256 weight rows leave the chip idle whichever way they are cut,
+// and what counts is the length of one chain: the product split over k with its partial tiles through memory was one launch of 5 us, their
+// sum and the GeGLU one of 4.8.  Here a workgroup owns 32 weight rows and 16 activation rows and all of k: a wave per split, every operand
+// of a pass over four units requested at once, the codes along the rows (each lane's own eight bytes and scale straight from memory: 6.0 and,
+// at eight waves, 8.8, bound by the cache lines a load touches), and the partial tiles meet in LDS.  Quarters, splits and their order are those of matmul_skinny_kernel: the same bits.
+constexpr uint32_t kGatedWaves = 12;
+template <int FMT>
+__global__ __launch_bounds__(64 * kGatedWaves) void matmul_gated_kernel(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W, const uint16_t* gate, uint16_t* out,
+                                                                        uint32_t M, uint32_t K, uint32_t N, uint32_t units_per_quarter, uint32_t gate_stride, uint32_t gate_off) {
+    constexpr int UK = Skinny<FMT>::unit_k, NF = Skinny<FMT>::frags;
+    // Four units of a row lie side by side: 144 bytes (Q4_0) or 132 (TQ2_0).  They come in along the rows, 8 bytes a lane, and a lane takes
+    // its own from the wave's area (rows an odd number of words apart); later the area holds the wave's partial tiles.
+    constexpr uint32_t BYTES = FMT == kQ4 ? 144 : 132, PIECES = (BYTES + 7) / 8, PITCH = FMT == kQ4 ? 148 : 132, LOADS = (32 * PIECES + 63) / 64;
+    __shared__ __align__(16) uint8_t area[kGatedWaves][32 * 148];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
+    const uint32_t r = lane & 15, g = lane >> 4, n0 = blockIdx.x * 32, m = blockIdx.y * 16 + r;
+    const size_t row_bytes = FMT == kQ4 ? (size_t)(K >> 5) * 18 : (size_t)(K >> 8) * 66;
+    const uint32_t k_begin = wave * 4 * units_per_quarter * UK;
+    const uint8_t* codes = W + (size_t)n0 * row_bytes + (FMT == kQ4 ? (size_t)(k_begin >> 6) * 36 : (size_t)(k_begin >> 8) * 66);
+    const uint16_t* xrow = X + (size_t)(m < M ? m : M - 1) * K + k_begin;
+    uint8_t* mine = area[wave];
+    uint32_t from[LOADS], to[LOADS];
+#pragma unroll
+    for (uint32_t i = 0; i < LOADS; i++) {
+        const uint32_t at = std::min(64 * i + lane, 32 * PIECES - 1), row = at / PIECES, piece = std::min(8 * (at - row * PIECES), BYTES - 8);
+        from[i] = row * (uint32_t)row_bytes + piece;
+        to[i] = row * PITCH + piece;
+    }
+    f32x4 sum[2], acc[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) sum[t] = acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    uint32_t done = 0, quarter = 0;
+    for (uint32_t pass = 0; pass < units_per_quarter; pass++) {
+        f16x8 x[4][NF];
+        uint2 raw[LOADS];
+#pragma unroll
+        for (uint32_t i = 0; i < LOADS; i++) raw[i] = ld8_align2(codes + pass * BYTES + from[i]);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int f = 0; f < NF; f++)
+                x[q][f] = *reinterpret_cast<const f16x8*>(xrow + (pass * 4 + q) * UK + (FMT == kQ4 ? 32 * (g >> 1) + 8 * (g & 1) + 16 * f : 32 * f + 8 * g));
+#pragma unroll
+        for (uint32_t i = 0; i < LOADS; i++) { *reinterpret_cast<lds_word_t*>(mine + to[i]) = raw[i].x; *reinterpret_cast<lds_word_t*>(mine + to[i] + 4) = raw[i].y; }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            SkinnyRaw w[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const uint8_t* p = mine + (16 * t + r) * PITCH;
+                if constexpr (FMT == kQ4) w[t] = skinny_take<kQ4>(p + 36 * q, g);
+                else {
+                    const uint32_t o = 66 * (q >> 1) + 32 * (q & 1) + 8 * g;          // a block begins on a half word where q is 2 or 3
+                    const lds_word_t* c = reinterpret_cast<const lds_word_t*>(p + (o & ~3u));
+                    const uint32_t d = *reinterpret_cast<const lds_half_t*>(p + 66 * (q >> 1) + 64) * 0x10001u;
+                    if (q < 2) w[t] = {c[0], c[1], d};
+                    else w[t] = {__builtin_amdgcn_alignbit(c[1], c[0], 16), __builtin_amdgcn_alignbit(c[2], c[1], 16), d};
+                }
+            }
+#pragma unroll
+            for (int f = 0; f < NF; f++)
+#pragma unroll
+                for (int t = 0; t < 2; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(skinny_fragment<FMT>(w[t], f), x[q][f], acc[t], 0, 0, 0);
+            if (++done == units_per_quarter) {
+                done = 0;
+#pragma unroll
+                for (int t = 0; t < 2; t++) { sum[t] = quarter ? sum[t] + acc[t] : acc[t]; acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f}; }
+                quarter++;
+            }
+        }
+    }
+    const auto part = [&](uint32_t z, uint32_t t) { return reinterpret_cast<f32x4*>(area[z] + 1024 * t) + lane; };
+#pragma unroll
+    for (int t = 0; t < 2; t++) *part(wave, t) = sum[t];
+    lh_lds_barrier();
+    for (uint32_t t = wave; t < 2; t += nwaves) {
+        f32x4 v = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (uint32_t z = 0; z < nwaves; z++) v += *part(z, t);
+        if (m >= M) continue;
+        const uint32_t n = n0 + 16 * t + 4 * g;               // D[row 4g + i of tile t][activation row r]
+        const uint2 b = *reinterpret_cast<const uint2*>(gate + (size_t)m * gate_stride + gate_off + n);
+        const uint32_t bw[2] = {b.x, b.y};
+        uint16_t h[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) h[i] = lh_gelu_mul_h(lh_f2h(v[i]), (uint16_t)(bw[i >> 1] >> (16 * (i & 1))));
+        *reinterpret_cast<uint2*>(out + (size_t)m * N + n) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+    }
+}
+
 // An address in global memory that is the same in all lanes, kept in scalar registers: a load at it plus 32 bits of offset of the lane's own
 // needs no vector registers for addresses.  (The builtin gives a signed word: it must not be widened as one.)
 typedef const __attribute__((address_space(1))) uint8_t* GlobalBytes;
@@ -1363,6 +1453,26 @@ bool try_skinny(lh_context* ctx, const void* A, const uint8_t* W, void* C, lh_dt
     return false;
 }
 
+// matmul_gated_kernel where try_skinny would take the rows, up to a workgroup a CU, and two of up to 2048 columns: each reads its codes and
+// activations for itself.  (Q4_0, us, split and summed -> this: 64 x 1536 x 256 8.5 -> 5.5, 256 x 1536 x 1024, two a CU, 10.3 -> 7.4; beyond:
+// 160 x 1536 x 2048 12.0 -> 10.9, 256 x 1536 x 2048 11.7 -> 15.3, 160 x 4096 x 1024 12.4 -> 13.7.)
+template <int FMT>
+bool try_gated(lh_context* ctx, const lh_buffer* X, const lh_buffer* W, const lh_buffer* gate, lh_buffer* out, uint32_t m, uint32_t k, uint32_t n,
+               uint32_t gate_stride, uint32_t gate_off) {
+    if (m < skinny_min_m(FMT) || m > skinny_max_m() || (FMT == kQ4 && m <= (uint32_t)kMaxMultivecM) || n % BN != 0 || k % (4 * Skinny<FMT>::unit_k) != 0) return false;
+    const uint64_t workgroups = (uint64_t)(n / 32) * ((m + 15) / 16);
+    if (workgroups > (k <= 2048 ? 2 : 1) * (uint64_t)ctx->cu_count) return false;
+    const auto apart = [&](const lh_buffer* b, size_t len) {          // the rows are read while others are written
+        return (uintptr_t)b->ptr + len <= (uintptr_t)out->ptr || (uintptr_t)out->ptr + (size_t)m * n * 2 <= (uintptr_t)b->ptr;
+    };
+    if (!apart(X, (size_t)m * k * 2) || !apart(W, (size_t)n * (FMT == kQ4 ? (size_t)(k / 32) * 18 : (size_t)(k / 256) * 66))) return false;
+    const uint32_t per_wg = k / Skinny<FMT>::unit_k / 4, splits = skinny_splits(ctx, m, n / 64 * ((m + 63) / 64), per_wg);
+    if (splits > kGatedWaves) return false;
+    hipLaunchKernelGGL(matmul_gated_kernel<FMT>, dim3(n / 32, (m + 15) / 16), dim3(64 * splits), 0, ctx->stream, (const uint16_t*)X->ptr, (const uint8_t*)W->ptr,
+                       (const uint16_t*)gate->ptr, (uint16_t*)out->ptr, m, k, n, per_wg / splits, gate_stride, gate_off);
+    return true;
+}
+
 // The 64-row-tile kernel over `tiles_n` column tiles (one matrix, or the matrices of `grp` side by side).  Few output
 // tiles (a decode batch of some tens of rows): k is split so that every CU gets a workgroup, at least two k steps per
 // split, partial tiles within the lower half of the context workspace, summed by splitk_reduce_kernel.
@@ -1632,6 +1742,12 @@ int lh_matmul_nt_quant_gelu_mul_strided_into(lh_batch* b, lh_quant fmt, const lh
     LH_NEED(out, (size_t)m * n * 2, op, "output");
     LH_REQUIRE((((uintptr_t)in->ptr | (uintptr_t)gate_rows->ptr | (uintptr_t)out->ptr) & 15) == 0, "%s: buffers must be 16-byte aligned", op);
     LH_REQUIRE(((uintptr_t)w->ptr & 1) == 0, "%s: weight must be 2-byte aligned", op);
+    if (fmt == LH_Q4_0 ? try_gated<kQ4>(ctx, in, w, gate_rows, out, m, k, n, row_stride, row_offset)
+                       : try_gated<kTQ2>(ctx, in, w, gate_rows, out, m, k, n, row_stride, row_offset)) {
+        int r = lh_check_launch(op);
+        if (r == LH_OK) b->dispatch_count++;
+        return r;
+    }
     const ClipArgs none{nullptr, 0.f, 0.f, 0.f, 0.f, 0u};
     SkinnyPartials kept{nullptr, 0, 0};
     const uint8_t* W = (const uint8_t*)w->ptr;

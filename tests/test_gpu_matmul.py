@@ -473,6 +473,32 @@ def test_many_query_heads_prepared_with_their_product(pkg, gpu, fmt):
         assert np.array_equal(one, other)
 
 
+@pytest.mark.parametrize("fmt,m,k,n", [("q4_0", 17, 256, 128), ("q4_0", 256, 1536, 1024), ("q4_0", 65, 2048, 256), ("q4_0", 100, 6144, 512), ("q4_0", 48, 768, 384),
+                                       ("tq2_0", 2, 512, 128), ("tq2_0", 256, 1536, 256), ("tq2_0", 129, 3072, 128), ("tq2_0", 15, 6144, 512), ("tq2_0", 77, 1024, 384)])
+def test_few_gated_rows_in_one_launch(pkg, gpu, fmt, m, k, n):
+    """The product whose GeGLU follows in the same launch (one to twelve waves, one or more units a quarter, one and two workgroups a
+    CU, partial groups of rows) against the two separate ones, bit for bit; a result over its own input takes the separate way."""
+    ctx, K = gpu
+    ty = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0
+    g = pkg.synth.rng(83, m + k + n)
+    w = pkg.QuantWeight.from_bytes(ctx, pkg.synth.weights(fmt, n, k, g), ty, n, k)
+    host = (g.standard_normal((m, k), dtype=np.float32) * 0.5).astype(np.float16)
+    stride, off = n + 264, 256
+    rows = pkg.Buffer.from_slice(ctx, g.standard_normal(m * stride + n, dtype=np.float32).astype(np.float16))
+    x, tmp, want = pkg.Buffer.from_slice(ctx, host), pkg.Buffer.empty(ctx, m * n * 2), pkg.Buffer.empty(ctx, m * n * 2)
+    got = pkg.Buffer.from_slice(ctx, np.full(m * n + 64, 7, np.uint16))
+    batch = pkg.CommandBatch(ctx)
+    w.matmul_nt_into(batch, K, x, tmp, m)
+    K.gelu_mul_strided_into(batch, tmp, rows, stride, off, want, n, m)
+    K.matmul_nt_quant_gelu_mul_strided_into(batch, ty, x, w.buf, m, k, n, rows, stride, off, got)
+    over = pkg.Buffer.from_slice(ctx, np.concatenate([host.reshape(-1), np.zeros(max(0, m * n - m * k), np.float16)]))
+    K.matmul_nt_quant_gelu_mul_strided_into(batch, ty, over, w.buf, m, k, n, rows, stride, off, over)
+    batch.commit_and_wait()
+    one = got.as_array(np.uint16)
+    assert np.array_equal(one[:m * n], want.as_array(np.uint16)) and (one[m * n:] == 7).all()
+    assert np.array_equal(over.as_array(np.uint16, m * n), want.as_array(np.uint16))
+
+
 @pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
 def test_matmul_gelu_mul_strided_fused_equals_separate_kernels(pkg, gpu, fmt):
     """matmul_nt_quant_gelu_mul_strided_into against matmul_nt + gelu_mul_strided (itself gather_strided + gelu_mul), bit for
