@@ -758,6 +758,8 @@ LH_API int lh_attention_rows_into(lh_batch* batch, const lh_buffer* q, const lh_
  *   rows     attention of queries that the key projection has been applied to, in the latent space: q f32 [rows, heads,
  *            lh_latent_row], output [rows, heads, rank] of `dtype`, of which the value projection is then taken.  sink and
  *            gate as above.
+ *   values   rows, and the value projection (weight [heads, vdim, rank]) of what they leave: output [rows, heads, vdim] of
+ *            `dtype`.  `latent` [rows, heads, rank] is scratch.
  *   queries  prepare and the key projection of q [rows, heads, dim] (weight [heads, rank, dim]) into the queries of rows */
 LH_API uint32_t lh_latent_padded_rank(uint32_t rank);
 LH_API uint32_t lh_latent_row(uint32_t rank, uint32_t rot);
@@ -774,6 +776,11 @@ LH_API int lh_latent_attention_rows_into(lh_batch* batch, const lh_buffer* q, co
                                          int dtype, const lh_buffer* position, uint32_t max_position, uint32_t rows,
                                          uint32_t heads, uint32_t rank, uint32_t rot, uint32_t capacity, float scale,
                                          const lh_buffer* sink, const lh_buffer* gate);
+LH_API int lh_latent_attention_values_into(lh_batch* batch, const lh_buffer* q, const lh_buffer* cache, lh_buffer* latent,
+                                           int dtype, const lh_buffer* position, uint32_t max_position, uint32_t rows,
+                                           uint32_t heads, uint32_t rank, uint32_t rot, uint32_t capacity, float scale,
+                                           const lh_buffer* sink, const lh_buffer* gate, const lh_buffer* value_weight,
+                                           uint32_t vdim, lh_buffer* output);
 LH_API int lh_latent_queries_into(lh_batch* batch, const lh_buffer* q, const lh_buffer* key_weight, const lh_buffer* q_rot,
                                   const lh_buffer* down, const lh_buffer* norm_weight, const lh_buffer* frequencies,
                                   const lh_buffer* position, lh_buffer* output, lh_buffer* cache, int dtype, uint32_t rows,

@@ -941,6 +941,13 @@ class Kernels:
                                                      _u32(max_position), _u32(rows), _u32(heads), _u32(rank), _u32(rot),
                                                      _u32(capacity), C.c_float(scale), _opt(sink), _opt(gate)))
 
+    def latent_attention_values_into(self, batch, q, cache, latent, dtype, position, max_position, rows, heads, rank, rot, capacity,
+                                     scale, sink, gate, value_weight, vdim, output):
+        _check(self._l.lh_latent_attention_values_into(batch._h, q._h, cache._h, latent._h, C.c_int(dtype), position._h,
+                                                       _u32(max_position), _u32(rows), _u32(heads), _u32(rank), _u32(rot),
+                                                       _u32(capacity), C.c_float(scale), _opt(sink), _opt(gate), value_weight._h,
+                                                       _u32(vdim), output._h))
+
     def latent_queries_into(self, batch, q, key_weight, q_rot, down, norm_weight, frequencies, position, output, cache, dtype, rows,
                             heads, dim, rank, rot, capacity, eps):
         _check(self._l.lh_latent_queries_into(batch._h, q._h, key_weight._h, q_rot._h, _opt(down), _opt(norm_weight),

@@ -266,8 +266,43 @@ __global__ __launch_bounds__(256) void latent_split_kernel(const AttentionArgs a
     if (tid < 16) { rec[DV] = st.m; rec[DV + 1] = l; }
 }
 
+// A token's splits merged and the value projection of the result, which the merge's launch handed to a second one: every workgroup of 16
+// columns of a head merges all of the head's latent columns for itself, its weights already on their way.  Quarters of K and their order as in
+// head_tile.  (Attention and projection, rank 512, warm: 8 heads and 256 keys 11.8 us with a launch of its own and 10.0 with this, 16 heads
+// 12.2 and 10.7, 32 heads and 1024 keys 15.2 and 13.9.)  Up to 24 splits: then reading all of them in every workgroup costs what the launch
+// does (8 heads: 512 keys 11.8 and 10.8, 1024 12.5 and 12.4, 1500 12.5 and 13.7; 16 heads, 1024: 13.3 and 13.5).
+constexpr uint32_t kValueSplits = 24;
+__global__ __launch_bounds__(kMergeThreads) void latent_values_kernel(const AttentionArgs a, const HeadArgs v) {
+    __shared__ MergeSpace<1> space;
+    __shared__ __align__(16) uint16_t x[512];
+    __shared__ lh_f32x4 part[4][64];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, h = blockIdx.y, n0 = blockIdx.x * 16;
+    const uint32_t steps = (v.K + 31) / 32, per = (steps + 3) / 4, s0 = min(wave * per, steps), s1 = min(s0 + per, steps);        // K <= 512: at most four
+    const uint16_t* w = v.W + ((size_t)h * v.N + min(n0 + (lane & 15), v.N - 1)) * v.K;
+    lh_bf16x8 weights[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) weights[i] = operand8(w, s0 + i < s1 ? (s0 + i) * 32 + (lane >> 4) * 8 : v.K, v.K, v.vec);
+    const float gate = a.gate ? a.gate[h] : 0.0f;
+    const float merged = merge_columns<1>(a, 0, h, 0, a.dv, space);
+    x[threadIdx.x] = threadIdx.x < v.K ? lh_f2bf(a.gate ? merged * lh_sigmoid(gate) : merged) : 0;
+    __syncthreads();
+    if (wave < 4) {
+        lh_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            if (s0 + i >= s1) break;
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(weights[i], *reinterpret_cast<const lh_bf16x8*>(x + (s0 + i) * 32 + (lane >> 4) * 8), acc, 0, 0, 0);
+        }
+        part[wave][lane] = acc;
+    }
+    __syncthreads();
+    const uint32_t n = n0 + threadIdx.x, l = threadIdx.x / 4 * 16, r = threadIdx.x & 3;           // thread: one output, of the tile's first row
+    if (threadIdx.x < 16 && n < v.N)
+        lh_st(static_cast<uint16_t*>(v.out), (size_t)h * v.ld + n, (part[0][l][r] + part[1][l][r]) + (part[2][l][r] + part[3][l][r]));
+}
+
 template <int DV>
-int launch_split(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const char* op, uint32_t& launches) {
+int launch_split(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const char* op, uint32_t& launches, const HeadArgs* values, bool& projected) {
     constexpr size_t lds = 2 * 32 * (DV + kRotPad) * 2 + 4 * 2 * 64 * 16;
     const uint64_t tiles = ((uint64_t)a.rows * a.heads + 15) / 16, want = (uint64_t)ctx->cu_count * (tiles > 2 ? 2 : 1);
     const uint32_t max_blocks = (uint32_t)std::min<uint64_t>((uint64_t)max_position + a.rows, a.capacity) / 32 + 1;
@@ -287,7 +322,10 @@ int launch_split(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const
     int r = lh_check_launch(op);
     if (r != LH_OK) return r;
     launches = 2;
-    return launch_merge<1>(ctx, a, op);
+    projected = values && a.rows == 1 && a.splits <= kValueSplits;
+    if (!projected) return launch_merge<1>(ctx, a, op);
+    hipLaunchKernelGGL(latent_values_kernel, dim3((values->N + 15) / 16, a.heads), dim3(kMergeThreads), 0, ctx->stream, a, *values);
+    return lh_check_launch(op);
 }
 
 // Checks and arguments of an attention over cache rows; the output is the caller's.
@@ -313,11 +351,11 @@ int latent_args(AttentionArgs& a, const char* op, const lh_buffer* q, const lh_b
 bool tiled(const AttentionArgs& a, int dtype, uint32_t rot) {
     return dtype == LH_BF16 && (((uintptr_t)a.q | (uintptr_t)a.keys) & 15) == 0 && rot <= kRotPad && a.dv <= 512;
 }
-int launch_tiled(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const char* op, uint32_t& launches) {
-    if (a.dv == 64) return launch_split<64>(ctx, a, max_position, op, launches);
-    if (a.dv == 128) return launch_split<128>(ctx, a, max_position, op, launches);
-    if (a.dv == 256) return launch_split<256>(ctx, a, max_position, op, launches);
-    return launch_split<512>(ctx, a, max_position, op, launches);
+int launch_tiled(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const char* op, uint32_t& launches, const HeadArgs* values, bool& projected) {
+    if (a.dv == 64) return launch_split<64>(ctx, a, max_position, op, launches, values, projected);
+    if (a.dv == 128) return launch_split<128>(ctx, a, max_position, op, launches, values, projected);
+    if (a.dv == 256) return launch_split<256>(ctx, a, max_position, op, launches, values, projected);
+    return launch_split<512>(ctx, a, max_position, op, launches, values, projected);
 }
 
 int prepare_args(PrepareArgs& a, uint32_t& pieces, const char* op, const lh_buffer* q_rot, const lh_buffer* down, const lh_buffer* norm_weight,
@@ -447,19 +485,16 @@ int lh_latent_expand_into(lh_batch* batch, const lh_buffer* cache, int dtype, co
     return r;
 }
 
-int lh_latent_attention_rows_into(lh_batch* batch, const lh_buffer* q, const lh_buffer* cache, lh_buffer* output, int dtype, const lh_buffer* position,
-                                  uint32_t max_position, uint32_t rows, uint32_t heads, uint32_t rank, uint32_t rot, uint32_t capacity, float scale,
-                                  const lh_buffer* sink, const lh_buffer* gate) {
-    const char* op = "latent_attention_rows";
-    LH_REQUIRE(batch, "%s: batch is null", op);
-    if (rows == 0) return LH_OK;
+static int attention_rows(lh_batch* batch, const char* op, const lh_buffer* q, const lh_buffer* cache, lh_buffer* output, int dtype, const lh_buffer* position,
+                          uint32_t max_position, uint32_t rows, uint32_t heads, uint32_t rank, uint32_t rot, uint32_t capacity, float scale,
+                          const lh_buffer* sink, const lh_buffer* gate, const HeadArgs* values, bool& projected) {
     AttentionArgs a;
     int r = latent_args(a, op, q, cache, dtype, position, max_position, rows, heads, rank, rot, capacity, scale, sink, gate);
     if (r != LH_OK) return r;
     LH_NEED(output, (size_t)rows * heads * rank * (dtype == LH_F32 ? 4 : 2), op, "output");
     a.out = output->ptr;
     uint32_t launches = 1;
-    if (tiled(a, dtype, rot)) r = launch_tiled(batch->ctx, a, max_position, op, launches);
+    if (tiled(a, dtype, rot)) r = launch_tiled(batch->ctx, a, max_position, op, launches, values, projected);
     else {
         LH_REQUIRE((uint64_t)rows * heads < 0x7FFFFFFFull, "%s: %u rows", op, rows);
         if (dtype == LH_F32) hipLaunchKernelGGL((attention_plain_kernel<float, float>), dim3(rows * heads), dim3(256), (size_t)a.dim * 4, batch->ctx->stream, a);
@@ -468,6 +503,32 @@ int lh_latent_attention_rows_into(lh_batch* batch, const lh_buffer* q, const lh_
     }
     batch->dispatch_count += launches;
     return r;
+}
+
+int lh_latent_attention_rows_into(lh_batch* batch, const lh_buffer* q, const lh_buffer* cache, lh_buffer* output, int dtype, const lh_buffer* position,
+                                  uint32_t max_position, uint32_t rows, uint32_t heads, uint32_t rank, uint32_t rot, uint32_t capacity, float scale,
+                                  const lh_buffer* sink, const lh_buffer* gate) {
+    const char* op = "latent_attention_rows";
+    LH_REQUIRE(batch, "%s: batch is null", op);
+    if (rows == 0) return LH_OK;
+    bool projected = false;
+    return attention_rows(batch, op, q, cache, output, dtype, position, max_position, rows, heads, rank, rot, capacity, scale, sink, gate, nullptr, projected);
+}
+
+int lh_latent_attention_values_into(lh_batch* batch, const lh_buffer* q, const lh_buffer* cache, lh_buffer* latent, int dtype, const lh_buffer* position,
+                                    uint32_t max_position, uint32_t rows, uint32_t heads, uint32_t rank, uint32_t rot, uint32_t capacity, float scale,
+                                    const lh_buffer* sink, const lh_buffer* gate, const lh_buffer* value_weight, uint32_t vdim, lh_buffer* output) {
+    const char* op = "latent_attention_values";
+    LH_REQUIRE(batch, "%s: batch is null", op);
+    if (rows == 0) return LH_OK;
+    LH_NEED(latent, (size_t)rows * heads * rank * (dtype == LH_F32 ? 4 : 2), op, "latent");
+    HeadArgs v;
+    int r = head_args(v, op, latent, dtype, value_weight, output, dtype, rows, heads, vdim, rank, vdim);
+    if (r != LH_OK) return r;
+    bool projected = false;
+    r = attention_rows(batch, op, q, cache, latent, dtype, position, max_position, rows, heads, rank, rot, capacity, scale, sink, gate, &v, projected);
+    if (r != LH_OK || projected) return r;
+    return lh_head_linear_into(batch, latent, dtype, value_weight, output, dtype, rows, heads, vdim, rank, vdim);
 }
 
 int lh_latent_queries_into(lh_batch* batch, const lh_buffer* q, const lh_buffer* key_weight, const lh_buffer* q_rot, const lh_buffer* down,

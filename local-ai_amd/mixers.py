@@ -273,9 +273,8 @@ class LatentAttention:
             K.latent_queries_into(b, q, self.key_up, q_rot, down, self.latent_norm, self.frequencies, r.position, ql, memory.rows, r.dtype,
                                   n, H, s.dim, s.kv_rank, s.rot_dim, memory.capacity, self.eps)
             ol = r.scratch("latent.out", n * H * s.kv_rank)
-            K.latent_attention_rows_into(b, ql, memory.rows, ol, r.dtype, r.position, r.max_position, n, H, s.kv_rank, s.rot_dim,
-                                         memory.capacity, s.scale, self.sink, gate)
-            K.head_linear_into(b, ol, r.dtype, self.value_up, mixed, r.dtype, n, H, s.vdim, s.kv_rank, s.vdim)
+            K.latent_attention_values_into(b, ql, memory.rows, ol, r.dtype, r.position, r.max_position, n, H, s.kv_rank, s.rot_dim,
+                                           memory.capacity, s.scale, self.sink, gate, self.value_up, s.vdim, mixed)
         norm.finish(r, self.out, mixed, r.dtype)
 
 

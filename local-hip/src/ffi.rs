@@ -191,6 +191,7 @@ extern "C" {
     pub fn lh_head_linear_into(batch: *mut lh_batch, input: *const lh_buffer, dtype: c_int, weight: *const lh_buffer, output: *mut lh_buffer, output_dtype: c_int, rows: u32, heads: u32, n: u32, k: u32, output_ld: u32) -> c_int;
     pub fn lh_latent_expand_into(batch: *mut lh_batch, cache: *const lh_buffer, dtype: c_int, weight: *const lh_buffer, keys: *mut lh_buffer, values: *mut lh_buffer, positions: u32, heads: u32, dim: u32, rot: u32, vdim: u32, rank: u32) -> c_int;
     pub fn lh_latent_attention_rows_into(batch: *mut lh_batch, q: *const lh_buffer, cache: *const lh_buffer, output: *mut lh_buffer, dtype: c_int, position: *const lh_buffer, max_position: u32, rows: u32, heads: u32, rank: u32, rot: u32, capacity: u32, scale: f32, sink: *const lh_buffer, gate: *const lh_buffer) -> c_int;
+    pub fn lh_latent_attention_values_into(batch: *mut lh_batch, q: *const lh_buffer, cache: *const lh_buffer, latent: *mut lh_buffer, dtype: c_int, position: *const lh_buffer, max_position: u32, rows: u32, heads: u32, rank: u32, rot: u32, capacity: u32, scale: f32, sink: *const lh_buffer, gate: *const lh_buffer, value_weight: *const lh_buffer, vdim: u32, output: *mut lh_buffer) -> c_int;
     pub fn lh_latent_queries_into(batch: *mut lh_batch, q: *const lh_buffer, key_weight: *const lh_buffer, q_rot: *const lh_buffer, down: *const lh_buffer, norm_weight: *const lh_buffer, frequencies: *const lh_buffer, position: *const lh_buffer, output: *mut lh_buffer, cache: *mut lh_buffer, dtype: c_int, rows: u32, heads: u32, dim: u32, rank: u32, rot: u32, capacity: u32, eps: f32) -> c_int;
     pub fn lh_linear_attention_padded_dim(dim: u32) -> u32;
     pub fn lh_linear_attention_workspace_bytes(rows: u32, heads: u32, dim: u32, vdim: u32) -> usize;

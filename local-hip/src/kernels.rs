@@ -640,6 +640,13 @@ impl Kernels {
         check(unsafe { ffi::lh_latent_attention_rows_into(batch.as_ptr(), q.as_ptr(), cache.as_ptr(), output.as_ptr(), dtype, position.as_ptr(), max_position, rows, heads, rank, rot, capacity, scale, sink.as_ptr(), gate.as_ptr()) })
     }
 
+    /// `lh_latent_attention_values_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn latent_attention_values_into(&self, batch: &mut CommandBatch, q: &Buffer, cache: &Buffer, latent: &Buffer, dtype: c_int, position: &Buffer, max_position: u32, rows: u32, heads: u32, rank: u32, rot: u32, capacity: u32, scale: f32, sink: &Buffer, gate: &Buffer, value_weight: &Buffer, vdim: u32, output: &Buffer) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_latent_attention_values_into(batch.as_ptr(), q.as_ptr(), cache.as_ptr(), latent.as_ptr(), dtype, position.as_ptr(), max_position, rows, heads, rank, rot, capacity, scale, sink.as_ptr(), gate.as_ptr(), value_weight.as_ptr(), vdim, output.as_ptr()) })
+    }
+
     /// `lh_latent_queries_into` (include/local_hip.h).
     #[allow(clippy::too_many_arguments)]
     pub fn latent_queries_into(&self, batch: &mut CommandBatch, q: &Buffer, key_weight: &Buffer, q_rot: &Buffer, down: &Buffer, norm_weight: &Buffer, frequencies: &Buffer, position: &Buffer, output: &Buffer, cache: &Buffer, dtype: c_int, rows: u32, heads: u32, dim: u32, rank: u32, rot: u32, capacity: u32, eps: f32) -> Result<()> {

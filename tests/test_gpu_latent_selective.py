@@ -126,6 +126,32 @@ def latent_case(ai, gpu, dtype, heads, rank, rot, start, rows, capacity, spike=N
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("rows,heads,rank,rot,vdim,start", [(1, 1, 5, 2, 3, 0), (1, 8, 512, 64, 128, 257), (1, 16, 512, 64, 130, 31), (1, 17, 100, 16, 40, 700), (1, 3, 128, 20, 16, 767),
+                                                            (1, 4, 256, 64, 64, 768), (1, 2, 500, 64, 17, 64), (3, 8, 512, 64, 128, 90)])
+def test_latent_attention_with_the_value_projection(ai, gpu, dtype, rows, heads, rank, rot, vdim, start):
+    """One launch for the merge and the projection of a token of up to 24 splits, else the two steps: against those."""
+    ctx, K = gpu
+    dt, g = ai.BF16 if dtype == "bf16" else ai.F32, np.random.default_rng(heads + rank)
+    row, capacity = K.latent_row(rank, rot), (start + rows + 31) // 32 * 32
+    qp = np.zeros((rows, heads, row))
+    qp[..., :rank + rot] = g.standard_normal((rows, heads, rank + rot))
+    cache = upload(ai, ctx, cache_rows(K, g.standard_normal((capacity, rank)), g.standard_normal((capacity, rot))), dt)
+    q, sink, gate, uv = f32(ai, ctx, qp), f32(ai, ctx, g.standard_normal(heads)), f32(ai, ctx, g.standard_normal((rows, heads))), g.standard_normal((heads, vdim, rank))
+    uv, pos, batch = ai.Buffer.from_slice(ctx, M.bf16_bits(uv / np.sqrt(rank))), ai.Buffer.from_slice(ctx, np.array([start], np.uint32)), ai.CommandBatch(ctx)
+    latent, scratch, want, got = empty(ai, ctx, rows * heads * rank, dt), empty(ai, ctx, rows * heads * rank, dt), empty(ai, ctx, rows * heads * vdim, dt), empty(ai, ctx, rows * heads * vdim + 8, dt)
+    got.fill_zero()
+    args = (pos, start, rows, heads, rank, rot, capacity, 1.0 / np.sqrt(rank + rot))
+    print(f"values {dtype} {rows} {heads} {rank} {rot} {vdim} {start}", flush=True)
+    K.latent_attention_rows_into(batch, q, cache, latent, dt, *args, sink, gate)
+    K.head_linear_into(batch, latent, dt, uv, want, dt, rows, heads, vdim, rank, vdim)
+    K.latent_attention_values_into(batch, q, cache, scratch, dt, *args, sink, gate, uv, vdim, got)
+    batch.commit_and_wait()
+    one = download(ai, got, rows * heads * vdim + 8, dt)
+    close(one[:-8], download(ai, want, rows * heads * vdim, dt), F32_TOL if dt == ai.F32 else BF16_TOL, "values")
+    assert not one[-8:].any()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("rows,heads,dim,rank,rot,own", [(1, 1, 3, 5, 2, True), (1, 6, 64, 128, 16, False), (1, 16, 128, 512, 64, True), (40, 3, 40, 96, 20, True)])
 def test_latent_queries_equal_the_two_steps(ai, gpu, dtype, rows, heads, dim, rank, rot, own):
     ctx, K = gpu
