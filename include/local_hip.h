@@ -512,6 +512,13 @@ LH_API int lh_matmul_nt_qkv_prepare_rows_into(lh_batch* batch, lh_quant fmt, con
                                               uint32_t n_kv_heads, uint32_t rows, float eps, uint32_t start_position,
                                               float theta, float partial_rotary_factor, uint32_t bits, uint32_t ring_capacity,
                                               uint32_t lane_capacity);
+/* The same for a layer that shares another layer's cache: its Q projection and the preparation of the queries alone (the
+ * preparation above with k and v null), with the same results bit for bit.  w_q [n_q_heads * head_dim, k_dim] in `fmt`. */
+LH_API int lh_matmul_nt_q_prepare_rows_into(lh_batch* batch, lh_quant fmt, const lh_buffer* input, const lh_buffer* w_q,
+                                            uint32_t k_dim, lh_buffer* q, const lh_buffer* q_norm, const lh_buffer* signs,
+                                            lh_buffer* rq, const lh_buffer* positions, uint32_t head_dim, uint32_t n_q_heads,
+                                            uint32_t rows, float eps, uint32_t start_position, float theta,
+                                            float partial_rotary_factor, uint32_t lane_capacity);
 /* kernels.rs:5032-5163 hadamard_rotate{,_hf,_fh}_into,
  * shaders/attention_flash_tq.metal:58-139: per head optional sign flip, FWHT,
  * 1/sqrt(d), optional sign flip.  f32->f32, f16->f32, f32->f16. */

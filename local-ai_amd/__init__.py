@@ -714,6 +714,14 @@ class Kernels:
                                                           C.c_float(partial_rotary_factor), _u32(bits), _u32(ring_capacity),
                                                           _u32(lane_capacity)))
 
+    def matmul_nt_q_prepare_rows_into(self, batch, weight_type, input, w_q, k_dim, q, q_norm, signs, rq, positions, head_dim, n_q_heads,
+                                      rows, eps, start_position, theta, partial_rotary_factor, lane_capacity):
+        """The Q product alone and the queries' part of decode_qkv_prepare_rows_into (a layer that shares its cache)."""
+        _check(self._l.lh_matmul_nt_q_prepare_rows_into(batch._h, C.c_int(weight_type), input._h, w_q._h, _u32(k_dim), q._h, _opt(q_norm),
+                                                        signs._h, rq._h, _opt(positions), _u32(head_dim), _u32(n_q_heads), _u32(rows),
+                                                        C.c_float(eps), _u32(start_position), C.c_float(theta),
+                                                        C.c_float(partial_rotary_factor), _u32(lane_capacity)))
+
     def hadamard_rotate_into(self, batch, input, signs, output, head_dim, num_heads, pre_sign, post_sign):
         _check(self._l.lh_hadamard_rotate_into(batch._h, input._h, signs._h, output._h, _u32(head_dim),
                                                _u32(num_heads), C.c_int(bool(pre_sign)), C.c_int(bool(post_sign))))

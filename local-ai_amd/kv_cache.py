@@ -167,6 +167,12 @@ class QuantizedKvCache:
                                                 eps, start_pos, theta, partial_rotary_factor, self.bits,
                                                 self.ring_capacity(), 0)
 
+    def project_queries_rows_into(self, batch, kernels: Kernels, w_q, x: Buffer, q: Buffer, q_norm, rq: Buffer, start_pos: int, n_rows: int,
+                                  n_q_heads: int, eps: float, theta: float, partial_rotary_factor: float) -> None:
+        """The Q projection of a chunk's rows and ``prepare_rows_into`` of the queries alone (a KV-shared layer) as one encoded step."""
+        kernels.matmul_nt_q_prepare_rows_into(batch, w_q.ty, x, w_q.buf, w_q.cols, q, q_norm, self.signs, rq, None, self.head_dim, n_q_heads,
+                                              n_rows, eps, start_pos, theta, partial_rotary_factor, 0)
+
     def attention_rows_from_rotated_into(self, batch, kernels: Kernels, rq: Buffer, vacc: Buffer, attn_out: Buffer,
                                          kv_len: int, start_pos: int, n_rows: int, n_q_heads: int, window: int) -> None:
         """quant_cache.rs:660-700: the attend and rotate-back steps of ``fused_attention_batch_into``."""
@@ -262,6 +268,12 @@ class QuantizedUnifiedKvPool:
                                                 self.value_norms, positions, self.head_dim, n_q_heads, self.n_kv_heads,
                                                 lanes, eps, 0, theta, partial_rotary_factor, self.bits,
                                                 self.lane_ring_capacity, self.lane_stride())
+
+    def project_queries_lanes_into(self, batch, kernels: Kernels, w_q, x: Buffer, q: Buffer, q_norm, rq: Buffer, positions: Buffer,
+                                   active_lanes: int, n_q_heads: int, eps: float, theta: float, partial_rotary_factor: float) -> None:
+        """The Q projection of every lane and ``prepare_lanes_into`` of the queries alone (a KV-shared layer) as one encoded step."""
+        kernels.matmul_nt_q_prepare_rows_into(batch, w_q.ty, x, w_q.buf, w_q.cols, q, q_norm, self.signs, rq, positions, self.head_dim, n_q_heads,
+                                              min(active_lanes, self.n_lanes), eps, 0, theta, partial_rotary_factor, self.lane_stride())
 
     def attention_from_rotated_into(self, batch, kernels: Kernels, rq: Buffer, vacc: Buffer, attn_out: Buffer,
                                     positions: Buffer, n_q_heads: int, window: int, active_lanes: int) -> None:

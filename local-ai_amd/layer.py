@@ -250,6 +250,9 @@ class TransformerLayer:
         return (self.group_projections and self.fuse_norm_chain and q.ty != W_F16 and q.ty == k.ty == v.ty
                 and q.cols == k.cols == v.cols)
 
+    def _queries_as_one(self) -> bool:
+        return self.group_projections and self.fuse_norm_chain and self.weights.attn_q.ty != W_F16
+
     def _one_prepare(self) -> bool:
         hd = self.params.head_dim
         return self.fuse_prologues and 64 <= hd <= 512 and hd & (hd - 1) == 0
@@ -515,6 +518,13 @@ class TransformerLayer:
                                                       n_head, p.sliding_window)
             self._attention_tail(kernels, batch, rows, input, output, bs, ple_all, next_norm)
             return
+        if not own_kv and one_prepare and self._queries_as_one():
+            kv_cache.project_queries_rows_into(batch, kernels, w.attn_q, bs.normed, bs.q, w.q_norm, bs.rq, start_pos, n_rows, n_head, eps,
+                                               p.rope_theta, p.partial_rotary_factor)
+            kv_cache.attention_rows_from_rotated_into(batch, kernels, bs.rq, bs.vacc, bs.attn_out, kv_len, start_pos, rows,
+                                                      n_head, p.sliding_window)
+            self._attention_tail(kernels, batch, rows, input, output, bs, ple_all, next_norm)
+            return
         if own_kv:
             self._matmuls(batch, kernels, [w.attn_q, w.attn_k, w.attn_v], bs.normed, [bs.q, bs.k, bs.v], rows)
         else:
@@ -559,6 +569,13 @@ class TransformerLayer:
             pool.project_and_prepare_lanes_into(batch, kernels, w.attn_q.ty, bs.normed, w.attn_q.buf, w.attn_k.buf,
                                                 w.attn_v.buf, w.attn_q.cols, bs.q, bs.k, bs.v, w.q_norm, w.k_norm, bs.rq,
                                                 positions, n_lanes, n_head, eps, p.rope_theta, p.partial_rotary_factor)
+            pool.attention_from_rotated_into(batch, kernels, bs.rq, bs.vacc, bs.attn_out, positions, n_head,
+                                             p.sliding_window, n_lanes)
+            self._attention_tail(kernels, batch, rows, input, output, bs, ple_all, next_norm)
+            return
+        if not own_kv and one_prepare and self._queries_as_one():
+            pool.project_queries_lanes_into(batch, kernels, w.attn_q, bs.normed, bs.q, w.q_norm, bs.rq, positions, n_lanes, n_head, eps,
+                                            p.rope_theta, p.partial_rotary_factor)
             pool.attention_from_rotated_into(batch, kernels, bs.rq, bs.vacc, bs.attn_out, positions, n_head,
                                              p.sliding_window, n_lanes)
             self._attention_tail(kernels, batch, rows, input, output, bs, ple_all, next_norm)

@@ -155,6 +155,7 @@ extern "C" {
     pub fn lh_decode_qkv_prepare_into(batch: *mut lh_batch, q: *mut lh_buffer, k: *mut lh_buffer, v: *mut lh_buffer, q_norm: *const lh_buffer, k_norm: *const lh_buffer, levels: *const lh_buffer, signs: *const lh_buffer, rq: *mut lh_buffer, k_codes: *mut lh_buffer, k_norms: *mut lh_buffer, v_codes: *mut lh_buffer, v_norms: *mut lh_buffer, head_dim: u32, n_q_heads: u32, n_kv_heads: u32, eps: f32, position: u32, theta: f32, partial_rotary_factor: f32, bits: u32, ring_capacity: u32) -> c_int;
     pub fn lh_decode_qkv_prepare_rows_into(batch: *mut lh_batch, q: *mut lh_buffer, k: *mut lh_buffer, v: *mut lh_buffer, q_norm: *const lh_buffer, k_norm: *const lh_buffer, levels: *const lh_buffer, signs: *const lh_buffer, rq: *mut lh_buffer, k_codes: *mut lh_buffer, k_norms: *mut lh_buffer, v_codes: *mut lh_buffer, v_norms: *mut lh_buffer, positions: *const lh_buffer, head_dim: u32, n_q_heads: u32, n_kv_heads: u32, rows: u32, eps: f32, start_position: u32, theta: f32, partial_rotary_factor: f32, bits: u32, ring_capacity: u32, lane_capacity: u32) -> c_int;
     pub fn lh_matmul_nt_qkv_prepare_rows_into(batch: *mut lh_batch, fmt: lh_quant, input: *const lh_buffer, w_q: *const lh_buffer, w_k: *const lh_buffer, w_v: *const lh_buffer, k_dim: u32, q: *mut lh_buffer, k: *mut lh_buffer, v: *mut lh_buffer, q_norm: *const lh_buffer, k_norm: *const lh_buffer, levels: *const lh_buffer, signs: *const lh_buffer, rq: *mut lh_buffer, k_codes: *mut lh_buffer, k_norms: *mut lh_buffer, v_codes: *mut lh_buffer, v_norms: *mut lh_buffer, positions: *const lh_buffer, head_dim: u32, n_q_heads: u32, n_kv_heads: u32, rows: u32, eps: f32, start_position: u32, theta: f32, partial_rotary_factor: f32, bits: u32, ring_capacity: u32, lane_capacity: u32) -> c_int;
+    pub fn lh_matmul_nt_q_prepare_rows_into(batch: *mut lh_batch, fmt: lh_quant, input: *const lh_buffer, w_q: *const lh_buffer, k_dim: u32, q: *mut lh_buffer, q_norm: *const lh_buffer, signs: *const lh_buffer, rq: *mut lh_buffer, positions: *const lh_buffer, head_dim: u32, n_q_heads: u32, rows: u32, eps: f32, start_position: u32, theta: f32, partial_rotary_factor: f32, lane_capacity: u32) -> c_int;
     pub fn lh_hadamard_rotate_into(batch: *mut lh_batch, input: *const lh_buffer, signs: *const lh_buffer, output: *mut lh_buffer, head_dim: u32, num_heads: u32, pre_sign: c_int, post_sign: c_int) -> c_int;
     pub fn lh_hadamard_rotate_hf_into(batch: *mut lh_batch, input: *const lh_buffer, signs: *const lh_buffer, output: *mut lh_buffer, head_dim: u32, num_heads: u32, pre_sign: c_int, post_sign: c_int) -> c_int;
     pub fn lh_hadamard_rotate_fh_into(batch: *mut lh_batch, input: *const lh_buffer, signs: *const lh_buffer, output: *mut lh_buffer, head_dim: u32, num_heads: u32, pre_sign: c_int, post_sign: c_int) -> c_int;

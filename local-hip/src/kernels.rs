@@ -434,6 +434,13 @@ impl Kernels {
         check(unsafe { ffi::lh_matmul_nt_qkv_prepare_rows_into(batch.as_ptr(), fmt, input.as_ptr(), w_q.as_ptr(), w_k.as_ptr(), w_v.as_ptr(), k_dim, q.as_ptr(), k.as_ptr(), v.as_ptr(), q_norm.as_ptr(), k_norm.as_ptr(), levels.as_ptr(), signs.as_ptr(), rq.as_ptr(), k_codes.as_ptr(), k_norms.as_ptr(), v_codes.as_ptr(), v_norms.as_ptr(), positions.as_ptr(), head_dim, n_q_heads, n_kv_heads, rows, eps, start_position, theta, partial_rotary_factor, bits, ring_capacity, lane_capacity) })
     }
 
+    /// `lh_matmul_nt_q_prepare_rows_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn matmul_nt_q_prepare_rows_into(&self, batch: &mut CommandBatch, fmt: ffi::lh_quant, input: &Buffer, w_q: &Buffer, k_dim: u32, q: &Buffer, q_norm: &Buffer, signs: &Buffer, rq: &Buffer, positions: &Buffer, head_dim: u32, n_q_heads: u32, rows: u32, eps: f32, start_position: u32, theta: f32, partial_rotary_factor: f32, lane_capacity: u32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_matmul_nt_q_prepare_rows_into(batch.as_ptr(), fmt, input.as_ptr(), w_q.as_ptr(), k_dim, q.as_ptr(), q_norm.as_ptr(), signs.as_ptr(), rq.as_ptr(), positions.as_ptr(), head_dim, n_q_heads, rows, eps, start_position, theta, partial_rotary_factor, lane_capacity) })
+    }
+
     /// `lh_hadamard_rotate_into` (include/local_hip.h).
     #[allow(clippy::too_many_arguments)]
     pub fn hadamard_rotate_into(&self, batch: &mut CommandBatch, input: &Buffer, signs: &Buffer, output: &Buffer, head_dim: u32, num_heads: u32, pre_sign: c_int, post_sign: c_int) -> Result<()> {

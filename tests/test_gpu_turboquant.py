@@ -381,3 +381,30 @@ def test_qkv_product_and_prepare_as_one_step_equals_the_two_calls(pkg, gpu, orac
         K.matmul_nt_qkv_prepare_rows_into(pkg.CommandBatch(ctx), ty, x, ws[0], ws[1], ws[2], k_dim, a["q"], a["k"], a["v"], qwb, kwb,
                                           lv, sg, pkg.Buffer.empty(ctx, 64), a["kc"], a["kn"], a["vc"], a["vn"], pos_buf, hd, n_q,
                                           n_kv, rows, eps, start, theta, prf, bits, 0, lane_cap)
+
+
+@pytest.mark.parametrize("fmt,rows,hd,n_q,k_dim,lanes_mode", [("q4_0", 64, 256, 8, 1536, True), ("q4_0", 200, 256, 8, 1536, False), ("q4_0", 12, 64, 6, 512, True),
+                                                              ("q4_0", 17, 128, 4, 768, False), ("tq2_0", 33, 512, 8, 2048, True), ("tq2_0", 2, 64, 2, 512, False),
+                                                              ("q4_0", 1, 256, 8, 2048, True), ("tq2_0", 257, 256, 4, 1024, False), ("q4_0", 40, 64, 3, 320, True)])
+def test_query_product_and_prepare_as_one_step_equals_the_two_calls(pkg, gpu, oracle, fmt, rows, hd, n_q, k_dim, lanes_mode):
+    """lh_matmul_nt_q_prepare_rows_into (split and not split, every product kernel, whole tiles and not) against the product
+    and the preparation of the queries alone, bit for bit."""
+    print(f"case {fmt} rows={rows} hd={hd} n_q={n_q} k={k_dim} lanes={lanes_mode}", flush=True)
+    ctx, K = gpu
+    ty, g, n = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, pkg.synth.rng(67, rows * 7 + hd), n_q * hd
+    lane_cap, start = (300, 0) if lanes_mode else (0, 41)
+    pos = pkg.Buffer.from_slice(ctx, g.integers(0, lane_cap, rows).astype(np.uint32)) if lanes_mode else None
+    w, x = pkg.Buffer.from_slice(ctx, pkg.synth.weights(fmt, n, k_dim, g)), pkg.Buffer.from_slice(ctx, pkg.synth.activations(rows, k_dim, g).astype(np.float16))
+    qw = pkg.Buffer.from_slice(ctx, (0.25 * (1 + 0.1 * g.standard_normal(hd, dtype=np.float32))).astype(np.float16))
+    sg, batch = pkg.Buffer.from_slice(ctx, oracle.rotation_signs(hd)), pkg.CommandBatch(ctx)
+    out = [[pkg.Buffer.from_slice(ctx, np.full(rows * n + 8, 7, t)) for t in (np.uint16, np.float32)] for _ in range(2)]
+    K.matmul_nt_q_prepare_rows_into(batch, ty, x, w, k_dim, out[0][0], qw, sg, out[0][1], pos, hd, n_q, rows, 1e-6, start, 1e4, 0.5, lane_cap)
+    K.matmul_nt_quant_typed_into(batch, ty, x, pkg.F16, w, out[1][0], pkg.F16, rows, k_dim, n)
+    K.decode_qkv_prepare_rows_into(batch, out[1][0], None, None, qw, None, sg, sg, out[1][1], None, None, None, None, pos, hd, n_q, 1, rows, 1e-6, start, 1e4, 0.5,
+                                   2, 0, lane_cap)
+    batch.commit_and_wait()
+    for a, b in zip(*out):
+        assert np.array_equal(a.as_array(np.uint8), b.as_array(np.uint8))
+    assert out[0][1].as_array(np.float32)[:rows * n].any()
+    with pytest.raises(pkg.InvalidArgument):               # a too-small output is refused before anything is launched
+        K.matmul_nt_q_prepare_rows_into(batch, ty, x, w, k_dim, out[0][0], qw, sg, pkg.Buffer.empty(ctx, 64), pos, hd, n_q, rows, 1e-6, start, 1e4, 0.5, lane_cap)
