@@ -1239,9 +1239,7 @@ __global__ __launch_bounds__(256, 2) void matmul_wide_kernel(const uint16_t* __r
 // fewer, k split over the waves is the shorter way (256 rows, gate and up of 6144 x 1536: 192 workgroups, 21.7 us split).
 bool wide_pays(const lh_context* ctx, uint32_t blocks, uint32_t mgroups) { return (uint64_t)((blocks + 3) / 4) * mgroups >= (uint64_t)ctx->cu_count; }
 
-// Most activation rows the skinny kernel takes (256: a prefill chunk).  Beyond 64 rows
-// every group of 64 gets workgroups of its own, which re-read the codes from L2 while the activation traffic grows with
-// rows x weight rows; measured on a 256-row chunk of the layer bench: 197 -> 163 us per layer, no gain at 512 rows.
+// Most activation rows of the pair and the gated forms (256: a prefill chunk).
 uint32_t skinny_max_m() {
     return 256u;
 }
@@ -1370,6 +1368,17 @@ uint32_t skinny_max_blocks(const lh_context* ctx) {
     return 64u * (uint32_t)ctx->cu_count;
 }
 
+// Whether `m` rows against `blocks` 64-row blocks are the skinny kernel's.  Beyond 64 activation rows every group of 64 gets workgroups of its
+// own, which re-read the codes from L2 while the activation traffic grows with rows x weight rows: up to a chunk's 256 rows it is the shortest way
+// up to 8 workgroups a CU (a 256-row chunk of the layer bench: 197 -> 163 us per layer), and with more rows up to 2, where the LDS-tiled kernels
+// leave CUs idle or split k (TQ2_0, us, tiled -> this: 257 x 1536 x 2048 19.1 -> 9.0, 512 x 2048 x 2048 21.7 -> 12.0, 512 x 1536 x 1024 16.9 -> 9.0,
+// 512 x 6144 x 4096 47.0 -> 42.1, 1024 x 2048 x 2048 20.7 -> 18.5, 2048 x 1536 x 1024 17.6 -> 16.4; Q4_0 512 x 1536 x 1536 21.9 -> 15.6.  Beyond: TQ2_0
+// 257 x 2048 x 8192 20.6 -> 24.1, 384 x 1536 x 6144 17.0 -> 18.7, 2048 x 1536 x 1536 19.1 -> 21.3).
+bool skinny_fits(const lh_context* ctx, uint32_t m, uint32_t blocks) {
+    const uint64_t workgroups = (uint64_t)blocks * ((m + 63) / 64), cus = (uint64_t)ctx->cu_count;
+    return blocks <= skinny_max_blocks(ctx) && (m <= 64 || workgroups <= (m <= 256 ? 8 : 2) * cus);
+}
+
 // k splits of the skinny kernel over `workgroups` (64-row blocks x groups of 64 activation rows): enough workgroups for every CU, a whole number of units
 // per wave, partial tiles within half the workspace.
 uint32_t skinny_splits(const lh_context* ctx, uint32_t m, uint32_t workgroups, uint32_t units_per_wg) {
@@ -1383,8 +1392,7 @@ uint32_t skinny_splits(const lh_context* ctx, uint32_t m, uint32_t workgroups, u
     return splits;
 }
 
-// The skinny kernel when the shape allows it (f16 activations, 17 .. skinny_max_m() rows, whole 128-row tiles, at least one unit of k
-// per wave; at most 64 workgroups per CU, far above any shape here); false
+// The skinny kernel when the shape allows it (f16 activations, whole 128-row tiles, at least one unit of k per wave, skinny_fits); false
 // leaves the launch to the LDS-tiled kernels.  With `keep` the f32 partial
 // tiles (one split included) stay in the workspace for a consumer that sums them itself.
 struct SkinnyPartials { const float* partial; uint32_t splits, cols; };
@@ -1419,8 +1427,7 @@ bool try_skinny(lh_context* ctx, const void* A, const uint8_t* W, void* C, lh_dt
         bool whole = grp.count ? true : n % BN == 0;          // every matrix fills its 128-row tiles
         for (uint32_t i = 0; i < grp.count; i++) whole = whole && grp.N[i] % BN == 0;
         const uint32_t units = k / Skinny<FMT>::unit_k;
-        if (!clip.enabled && m >= skinny_min_m(FMT) && m <= skinny_max_m() && whole && k % (4 * Skinny<FMT>::unit_k) == 0 &&
-            2 * tiles_n <= skinny_max_blocks(ctx) && (m <= 64 || 2 * tiles_n * ((m + 63) / 64) <= 8 * (uint32_t)ctx->cu_count)) {
+        if (!clip.enabled && m >= skinny_min_m(FMT) && whole && k % (4 * Skinny<FMT>::unit_k) == 0 && skinny_fits(ctx, m, 2 * tiles_n)) {
             // k splits: enough workgroups for every CU, a whole number of units per wave, partial tiles within half the workspace
             const uint32_t blocks = 2 * tiles_n, per_wg = units / 4;
             const uint64_t fit = (ctx->workspace_bytes / 2) / ((uint64_t)m * blocks * 64 * 4);

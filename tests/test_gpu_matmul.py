@@ -78,6 +78,25 @@ def test_small_batch_q4_kernel_keeps_f32_weights(pkg, gpu, oracle):
         refgen.assert_close(outs[i].as_array(np.float16).astype(np.float32), want, 1e-3, f"small q4 grouped #{i}")
 
 
+@pytest.mark.parametrize("fmt,m,k,n", [("q4_0", 257, 1536, 2048), ("tq2_0", 257, 512, 8192), ("tq2_0", 512, 2048, 2048), ("q4_0", 512, 256, 4096), ("tq2_0", 513, 1536, 1536),
+                                       ("q4_0", 1000, 768, 1536), ("tq2_0", 1025, 512, 1920), ("q4_0", 2049, 512, 1024), ("tq2_0", 4100, 512, 384)])
+def test_many_rows_against_few_weight_rows(pkg, gpu, oracle, fmt, m, k, n):
+    """f16 rows beyond a chunk of 256 on both sides of the line of two workgroups a CU, split and not: the weights are the f16
+    values of the blocks in either kernel, so only f32 summation error is left."""
+    ctx, K = gpu
+    print(f"case {fmt} m={m} k={k} n={n}", flush=True)
+    raw = payload(fmt, n, k, 0x51 + m)
+    weights = expand(oracle, fmt, raw, n, k).astype(np.float16).astype(np.float64)
+    a16 = (pkg.synth.rng(4, m + k).standard_normal((m, k), dtype=np.float32) * 0.5).astype(np.float16)
+    w = pkg.QuantWeight.from_bytes(ctx, raw, pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, n, k)
+    c, batch = pkg.Buffer.from_slice(ctx, np.full(m * n + 16, 7, np.float32)), pkg.CommandBatch(ctx)
+    w.matmul_nt_typed_into(batch, K, pkg.Buffer.from_slice(ctx, a16), pkg.F16, c, pkg.F32, m)
+    batch.commit_and_wait()
+    got = c.as_array(np.float32)
+    refgen.assert_close(got[:m * n].reshape(m, n), (a16.astype(np.float64) @ weights.T).astype(np.float32), 2e-5, f"{fmt} {m}x{k}x{n}")
+    assert (got[m * n:] == 7).all()
+
+
 @pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
 def test_mfma_matmul_tile_boundaries(pkg, gpu, oracle, fmt):
     """kernels.rs:9551: M = 70 with N, K spanning several tiles and ragged edges."""
