@@ -1518,6 +1518,19 @@ int launch_by_out(bool mfma, lh_context* ctx, const void* A, const uint8_t* W, v
     const int cus = ctx->cu_count;
     if (mfma) {
         if (try_skinny<FMT, ADT>(ctx, A, W, C, ct, m, k, n, clip, GroupArgs{})) return LH_OK;
+        if constexpr (ADT == LH_BF16 && FMT != kF16W) {
+            // Up to one and a half workgroups a CU the decode-batch kernel is worth a pass that makes f16 rows of bf16 ones, the same values that the
+            // tiled kernels make of them (TQ2_0, f32 out, us, tiled -> this: 65 x 2048 x 8192 19.9 -> 14.6, 256 x 1536 x 2048 16.7 -> 12.6, 384 x 1536 x 4096 18.9 ->
+            // 17.0, 512 x 2048 x 2048 22.8 -> 16.9; with two, 256 x 2048 x 8192 21.3 -> 22.1, 512 x 1536 x 4096 18.1 -> 18.6).  They lie in the workspace's third quarter.
+            const size_t half = ctx->workspace_bytes / 2;
+            if (!clip.enabled && n % BN == 0 && k % (4 * Skinny<FMT>::unit_k) == 0 && skinny_fits(ctx, m, n / 64) && (size_t)m * k * 2 <= half / 2 &&
+                (uint64_t)(n / 64) * ((m + 63) / 64) * 2 <= 3 * (uint64_t)cus) {
+                uint16_t* a16 = reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(ctx->workspace) + half);
+                const size_t n8 = (size_t)m * k / 8;
+                hipLaunchKernelGGL((convert_to_f16_kernel<LH_BF16>), dim3((uint32_t)((n8 + 255) / 256)), dim3(256), 0, s, A, a16, n8);
+                if (try_skinny<FMT, LH_F16>(ctx, a16, W, C, ct, m, k, n, clip, GroupArgs{})) return LH_OK;
+            }
+        }
         // 128-row tiles reuse each dequantised weight tile twice as often; 64-row tiles when that would leave most CUs idle
         const uint64_t tiles128 = (uint64_t)((n + BN - 1) / BN) * ((m + 127) / 128);
         const bool big = m > 64 && tiles128 * 2 >= (uint64_t)cus;

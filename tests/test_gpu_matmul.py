@@ -97,6 +97,26 @@ def test_many_rows_against_few_weight_rows(pkg, gpu, oracle, fmt, m, k, n):
     assert (got[m * n:] == 7).all()
 
 
+@pytest.mark.parametrize("fmt,m,k,n", [("q4_0", 17, 256, 128), ("tq2_0", 65, 512, 8192), ("q4_0", 200, 1536, 2048), ("tq2_0", 384, 512, 4096), ("tq2_0", 385, 512, 4096),
+                                       ("q4_0", 600, 2048, 1024)])
+def test_bf16_rows_made_f16_for_the_decode_batch_kernel(pkg, gpu, oracle, fmt, m, k, n):
+    """bf16 rows on both sides of the line up to which they are made f16 ahead of the product (every value here is one of both)."""
+    ctx, K = gpu
+    print(f"case {fmt} m={m} k={k} n={n}", flush=True)
+    raw = payload(fmt, n, k, 0x61 + m)
+    weights = expand(oracle, fmt, raw, n, k).astype(np.float16).astype(np.float64)
+    bits = ((pkg.synth.rng(4, m + k).standard_normal((m, k), dtype=np.float32) * 0.5).view(np.uint32) >> 16).astype(np.uint16)
+    a = (bits.astype(np.uint32) << 16).view(np.float32)
+    a = np.where(np.abs(a) < 1e-4, np.float32(0), a)
+    w = pkg.QuantWeight.from_bytes(ctx, raw, pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0, n, k)
+    c, batch = pkg.Buffer.from_slice(ctx, np.full(m * n + 16, 7, np.float32)), pkg.CommandBatch(ctx)
+    w.matmul_nt_typed_into(batch, K, pkg.Buffer.from_slice(ctx, (a.view(np.uint32) >> 16).astype(np.uint16)), pkg.BF16, c, pkg.F32, m)
+    batch.commit_and_wait()
+    got = c.as_array(np.float32)
+    refgen.assert_close(got[:m * n].reshape(m, n), (a.astype(np.float64) @ weights.T).astype(np.float32), 2e-5, f"{fmt} {m}x{k}x{n}")
+    assert (got[m * n:] == 7).all()
+
+
 @pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
 def test_mfma_matmul_tile_boundaries(pkg, gpu, oracle, fmt):
     """kernels.rs:9551: M = 70 with N, K spanning several tiles and ragged edges."""
