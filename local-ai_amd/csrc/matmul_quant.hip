@@ -659,7 +659,8 @@ __global__ __launch_bounds__(256 + 64 * PW) void matmul_mfma128_kernel(const uin
     }
 }
 
-// ---- a decode batch of 17 .. 64 rows, a prefill chunk of up to 256: weights straight from global memory into MFMA operands ----
+// ---- a decode batch of 17 .. 64 rows, a prefill chunk of up to 256, more rows where few weight rows meet them (skinny_fits): weights straight
+// from global memory into MFMA operands ----
 // At these row counts a product is a few microseconds of matrix-core time and what counts is latency, so this kernel
 // has no workgroup-wide staging phase and one barrier.  A workgroup owns 64 weight rows (four 16-row MFMA tiles) and a
 // k range; its four waves split that range in quarters, every wave multiplying all four tiles against all activation
