@@ -28,7 +28,15 @@ template <class A>
 __device__ __forceinline__ float lh_dot2h(A a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), c, false);
 }
-constexpr uint32_t kOnes = 0x3C003C00u;
+// Two codes of a word, where `mask` has them in the low bytes of its halves, less their zero point (`zero`, at the codes' place): exact, as the f16 value
+// 1024 + code less 1024 + zero.  `base`: 1024 twice, in a vector register, so that taking and setting the bits is one instruction.  A word of sixteen TQ2_0
+// codes takes 37 instructions with its products.  (Codes as they are, the vector's sum taken off in the end: 36, but the two sums nearly cancel, with 2 to 4 times
+// the f32 error for vectors of one sign or with a large element, and weights of zero did not give zero; byte permutes: 39.  46 shapes of one f16 vector: 4 % longer
+// with the sums.)
+__device__ __forceinline__ f16x2 code_values(uint32_t word, uint32_t mask, uint32_t base, uint32_t zero) {
+    const _Float16 less = (_Float16)(float)(1024u + zero);
+    return __builtin_bit_cast(f16x2, (word & mask) | base) - (f16x2){less, less};
+}
 
 struct DirectArgs {
     const uint8_t* m[8];       // `count` matrices of [rows][K / 256] blocks of 66 bytes or [rows][K / 32] of 18, all for the one vector
@@ -242,49 +250,33 @@ __global__ __launch_bounds__(64 * direct_waves(NG)) void matvec_direct_kernel(co
             const uint4 t = *reinterpret_cast<const uint4*>(xs + (((j * NG + grp) * 8 + c) * 32 + l) * 2);
             x[j][c][0] = t.x; x[j][c][1] = t.y; x[j][c][2] = t.z; x[j][c][3] = t.w;
         }
-    // What the codes' zero point takes off: the sum of the lane's elements (TQ2_0), eight times that of each block's (Q4_0).
-    float zero[V][2];
-#pragma unroll
-    for (int j = 0; j < V; j++) {
-        float s[8];
-#pragma unroll
-        for (int c = 0; c < 8; c++) s[c] = lh_dot2h(kOnes, x[j][c][0], lh_dot2h(kOnes, x[j][c][1], 0.0f)) + lh_dot2h(kOnes, x[j][c][2], lh_dot2h(kOnes, x[j][c][3], 0.0f));
-        const float lo = (s[0] + s[1]) + (s[2] + s[3]), hi = (s[4] + s[5]) + (s[6] + s[7]);
-        zero[j][0] = FMT == LH_TQ2_0 ? -(lo + hi) : -8.0f * lo;
-        zero[j][1] = -8.0f * hi;
-    }
-
     float mine[V];                                            // lane 32 h + i: row h of the wave's pair i (32 of them at most)
 #pragma unroll
     for (int j = 0; j < V; j++) mine[j] = 0.0f;
-    // Two codes of a word come apart by a shift and an AND: with its highest bit at bit 10 and nothing else in the 16 bits a code is the f16
-    // value code * 2^-15 (TQ2_0; Q4_0: 2^-17), subnormal or in the first binade above, and the product with the vector is exact.  (Further down, where
-    // the AND alone would do, v_dot2 cuts ten bits more off: it aligns a subnormal's products by the exponent of the smallest normal value.  As f16 values
-    // of code - 1 by byte permutes a word of sixteen TQ2_0 codes took 32 instructions, most of them in the long encoding; now 28.  Infinite vectors give
-    // NaN where codes are above their zero point.)
+    uint32_t base = 0x64006400u;
+    asm("" : "+v"(base));
     lh_walk_rows(v, count, issue, [&](const Pair& p, uint32_t i) {
         float part[V];
         if constexpr (FMT == LH_TQ2_0) {
             float acc[V][4];
 #pragma unroll
-            for (int j = 0; j < V; j++)
-#pragma unroll
-                for (int f = 0; f < 4; f++) acc[j][f] = 0.0f;
-#pragma unroll
             for (int m = 0; m < 4; m++) {
-                const uint32_t c = p.w[m];
-                const uint32_t even[4] = {c << 9, c << 7, c << 5, c << 3}, odd[4] = {c << 1, c >> 1, c >> 3, c >> 5};      // fields of bytes 0, 2 and 1, 3
+                const uint32_t c = p.w[m], c8 = c >> 8;
 #pragma unroll
-                for (int f = 0; f < 4; f++)
+                for (int f = 0; f < 4; f++) {
+                    const uint32_t mask = 0x00030003u << (2 * f), zero = 1u << (2 * f);
+                    const f16x2 even = code_values(c, mask, base, zero), odd = code_values(c8, mask, base, zero);      // bytes 0, 2 and 1, 3
 #pragma unroll
                     for (int j = 0; j < V; j++) {
                         const uint32_t* xc = &x[j][2 * f + (m >> 1)][2 * (m & 1)];
-                        acc[j][f] += lh_dot2h(even[f] & 0x06000600u, xc[0], lh_dot2h(odd[f] & 0x06000600u, xc[1], 0.0f));
+                        const float four = lh_dot2h(even, xc[0], lh_dot2h(odd, xc[1], 0.0f));
+                        acc[j][f] = m ? acc[j][f] + four : four;
                     }
+                }
             }
 #pragma unroll
             for (int j = 0; j < V; j++) {
-                part[j] = __builtin_fmaf((acc[j][0] + acc[j][1]) + (acc[j][2] + acc[j][3]), 32768.0f, zero[j][0]) * lh_h2f((uint16_t)p.d);
+                part[j] = (__builtin_fmaf(acc[j][1], 0.25f, acc[j][0]) + __builtin_fmaf(acc[j][3], 0.015625f, acc[j][2] * 0.0625f)) * lh_h2f((uint16_t)p.d);
                 asm volatile("" : "+v"(part[j]));             // rounded here, not in an addition of the sum over the lanes: in every variant the same
             }
         } else {
@@ -296,21 +288,21 @@ __global__ __launch_bounds__(64 * direct_waves(NG)) void matvec_direct_kernel(co
             for (int b = 0; b < 2; b++) {
                 float acc[V][2];
 #pragma unroll
-                for (int j = 0; j < V; j++) acc[j][0] = acc[j][1] = 0.0f;
-#pragma unroll
                 for (int m = 0; m < 4; m++) {
-                    const uint32_t c = b ? w[5 + m] : __builtin_amdgcn_alignbit(w[m + 1], w[m], 16);
+                    const uint32_t c = b ? w[5 + m] : __builtin_amdgcn_alignbit(w[m + 1], w[m], 16), c8 = c >> 8;
+                    const f16x2 lo0 = code_values(c, 0x000F000Fu, base, 8), lo1 = code_values(c8, 0x000F000Fu, base, 8);
+                    const f16x2 hi0 = code_values(c, 0x00F000F0u, base, 128), hi1 = code_values(c8, 0x00F000F0u, base, 128);
 #pragma unroll
                     for (int j = 0; j < V; j++) {
                         const uint32_t *xl = &x[j][4 * b + (m >> 1)][2 * (m & 1)], *xh = &x[j][4 * b + 2 + (m >> 1)][2 * (m & 1)];
-                        acc[j][0] += lh_dot2h((c << 7) & 0x07800780u, xl[0], lh_dot2h((c >> 1) & 0x07800780u, xl[1], 0.0f));
-                        acc[j][1] += lh_dot2h((c << 3) & 0x07800780u, xh[0], lh_dot2h((c >> 5) & 0x07800780u, xh[1], 0.0f));
+                        const float lo = lh_dot2h(lo0, xl[0], lh_dot2h(lo1, xl[1], 0.0f)), hi = lh_dot2h(hi0, xh[0], lh_dot2h(hi1, xh[1], 0.0f));
+                        acc[j][0] = m ? acc[j][0] + lo : lo;
+                        acc[j][1] = m ? acc[j][1] + hi : hi;
                     }
                 }
 #pragma unroll
                 for (int j = 0; j < V; j++)
-                    part[j] = __builtin_fmaf(__builtin_fmaf(acc[j][0] + acc[j][1], 131072.0f, zero[j][b]),
-                                             lh_h2f((uint16_t)(b ? w[4] >> 16 : w[0] & 0xFFFFu)), part[j]);
+                    part[j] = __builtin_fmaf(__builtin_fmaf(acc[j][1], 0.0625f, acc[j][0]), lh_h2f((uint16_t)(b ? w[4] >> 16 : w[0] & 0xFFFFu)), part[j]);
             }
         }
 #pragma unroll

@@ -728,3 +728,45 @@ def test_matvec_norm_chain_gelu(pkg, gpu, fmt, rows, cols, gated):
     for up, f in ((ws[0].buf, factor), (None, None)):        # exactly one of the two
         with pytest.raises(pkg.InvalidArgument):
             K.matvec_quant_norm_chain_gelu_into(pkg.CommandBatch(ctx), ty, ws[0].buf, up, f, x, w1, res, w2, stores[1], 1e-6, outs[2], outs[3], rows, cols)
+
+
+@pytest.mark.parametrize("fmt", ["tq2_0", "q4_0"])
+@pytest.mark.parametrize("kind", ["signs", "one_sign", "one_large"])
+@pytest.mark.parametrize("rows,cols,batch", [(33, 1536, 1), (65, 6144, 1), (4609, 1536, 2), (4609, 1536, 8), (50, 512, 3)])
+def test_products_of_few_signs_and_large_elements(pkg, gpu, oracle, fmt, kind, rows, cols, batch):
+    """Vectors whose elements do not cancel, or one of which is a thousand times the others, f16 in and out, alone and two and four to a workgroup: codes at
+    their zero point take no part, so that weights of zero give exactly zero, and other weights are no further from the product in 64 bits than f16 rounding and
+    the sums' f32 rounding: four products of a group truncated (4 * 2^-24), at most 20 more additions of what all parts add up to."""
+    ctx, K = gpu
+    ty = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0
+    g = pkg.synth.rng(71, rows + cols)
+    x = g.standard_normal((batch, cols), dtype=np.float32)
+    if kind == "one_sign":
+        x = np.abs(x) + np.float32(0.25)
+    if kind == "one_large":
+        x[np.arange(batch), g.integers(0, cols, batch)] *= 1000
+    x = x.astype(np.float16)
+    raw = pkg.synth.weights(fmt, rows, cols, g)
+    zeros = raw.reshape(-1, 18 if fmt == "q4_0" else 66).copy()
+    if fmt == "q4_0":
+        zeros[:, 2:] = 0x88
+    else:
+        zeros[:, :64] = 0x55
+    xb = pkg.Buffer.from_slice(ctx, x)
+    print(f"case {fmt} {kind} {rows}x{cols} x{batch}", flush=True)
+    got = []
+    for r in (zeros.reshape(-1), raw):
+        w, yb = pkg.QuantWeight.from_bytes(ctx, r, ty, rows, cols), pkg.Buffer.empty(ctx, batch * rows * 2)
+        b = pkg.CommandBatch(ctx)
+        if batch == 1:
+            w.matvec_typed_into(b, K, xb, pkg.F16, yb, pkg.F16)
+        else:
+            w.matmul_nt_typed_into(b, K, xb, pkg.F16, yb, pkg.F16, batch)
+        b.commit_and_wait()
+        got.append(yb.as_array(np.float16, batch * rows).reshape(batch, rows).astype(np.float64))
+    assert not got[0].any(), f"{np.count_nonzero(got[0])} of {got[0].size} products with zeros are not zero, up to {np.abs(got[0]).max()}"
+    expand = oracle.expand_q4_0_f32 if fmt == "q4_0" else oracle.expand_tq2_0_f32
+    w64, x64 = np.asarray(expand(raw, rows, cols), np.float64).reshape(rows, cols), x.astype(np.float64)
+    want = x64 @ w64.T
+    half = np.exp2(np.maximum(np.floor(np.log2(np.maximum(np.abs(want), 1e-30))), -14) - 11)
+    assert np.all(np.abs(got[1] - want) <= 1.001 * half + 24 * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T))
