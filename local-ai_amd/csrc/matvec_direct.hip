@@ -71,6 +71,14 @@ __device__ __forceinline__ Elements<E> load_elements(const uint16_t* p) {
     return r;
 }
 
+// A use of what a load brings, without an instruction.
+template <int E>
+__device__ __forceinline__ void keep(const Elements<E>& v) {
+#pragma unroll
+    for (int j = 0; j < E / 2; j++) asm volatile("" :: "v"(v.w[j]));
+}
+__device__ __forceinline__ void keep(const float4& v) { asm volatile("" :: "v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w)); }
+
 // A workgroup of TEAMS x NG waves: wave w takes the block group w % NG of the row pairs of team w / NG.  V: vectors V blockIdx.y .. of a
 // batch that the workgroup multiplies each code with once it is apart (the last ones may repeat the last vector); what a vector gives does
 // not depend on V.
@@ -224,6 +232,10 @@ __global__ __launch_bounds__(64 * direct_waves(NG)) void matvec_direct_kernel(co
             if (e >= K)
 #pragma unroll
                 for (int j = 0; j < W; j++) w[j] = 0u;
+        } else {                                              // (or the compiler would request them here, behind the weights)
+            if constexpr (KIND == kXProRotate) { keep(fa[i]); keep(fb[i]); keep(sa[i]); keep(sb[i]); }
+            else keep(va[p]);
+            if constexpr (KIND == kXProGeluMul) keep(vb[i]);
         }
         // TQ2_0: element e of a block is in half e / 128, field e / 32 % 4, byte 16 (e / 16 % 2) + e % 16: lane 4 b + 2 half + e / 16 % 2, chunk
         // 2 field + e / 8 % 2.  Q4_0: chunk e / 8 % 8 of lane e / 64.  Four elements in the order 0 2 1 3 in which a word's codes come apart.
