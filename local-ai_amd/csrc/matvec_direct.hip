@@ -213,7 +213,7 @@ __global__ __launch_bounds__(64 * direct_waves(NG)) void matvec_direct_kernel(co
         if (has(i)) {
             if constexpr (KIND == kXProRotate) {
                 float t[8] = {fa[i].x, fa[i].y, fa[i].z, fa[i].w, fb[i].x, fb[i].y, fb[i].z, fb[i].w};
-                xpro_rotate8_regs(t, a.head_dim, a.scale, sa[i], sb[i]);
+                xpro_rotate8_regs<false>(t, a.head_dim, a.scale, sa[i], sb[i]);
 #pragma unroll
                 for (int j = 0; j < W; j++) w[j] = (uint32_t)lh_f2h(t[2 * j]) | (uint32_t)lh_f2h(t[2 * j + 1]) << 16;
             } else
