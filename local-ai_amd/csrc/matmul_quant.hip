@@ -1369,15 +1369,22 @@ uint32_t skinny_max_blocks(const lh_context* ctx) {
     return 64u * (uint32_t)ctx->cu_count;
 }
 
-// Whether `m` rows against `blocks` 64-row blocks are the skinny kernel's.  Beyond 64 activation rows every group of 64 gets workgroups of its
+// Whether `m` rows of `k` against `blocks` 64-row blocks are the skinny kernel's.  Beyond 64 activation rows every group of 64 gets workgroups of its
 // own, which re-read the codes from L2 while the activation traffic grows with rows x weight rows: up to a chunk's 256 rows it is the shortest way
 // up to 8 workgroups a CU (a 256-row chunk of the layer bench: 197 -> 163 us per layer), and with more rows up to 2, where the LDS-tiled kernels
 // leave CUs idle or split k (TQ2_0, us, tiled -> this: 257 x 1536 x 2048 19.1 -> 9.0, 512 x 2048 x 2048 21.7 -> 12.0, 512 x 1536 x 1024 16.9 -> 9.0,
 // 512 x 6144 x 4096 47.0 -> 42.1, 1024 x 2048 x 2048 20.7 -> 18.5, 2048 x 1536 x 1024 17.6 -> 16.4; Q4_0 512 x 1536 x 1536 21.9 -> 15.6.  Beyond: TQ2_0
-// 257 x 2048 x 8192 20.6 -> 24.1, 384 x 1536 x 6144 17.0 -> 18.7, 2048 x 1536 x 1536 19.1 -> 21.3).
-bool skinny_fits(const lh_context* ctx, uint32_t m, uint32_t blocks) {
+// 257 x 2048 x 8192 20.6 -> 24.1, 384 x 1536 x 6144 17.0 -> 18.7, 2048 x 1536 x 1536 19.1 -> 21.3).  Fewer blocks stand against more rows, which every XCD
+// reads for itself: with less than 16 up to 1.5 workgroups a CU (TQ2_0 3072 x 512 x 512 8.9 -> 6.9, Q4_0 3072 x 4096 x 512 44.2 -> 35.7; with two, TQ2_0
+// 4096 x 2048 x 512 20.6 -> 25.3, 4096 x 4096 x 512 33.3 -> 42.7), with less than 8 up to one (TQ2_0 4096 x 1536 x 256 19.0 -> 13.7; with 1.5, 4096 x 1024 x 384 behind
+// a norm 19.0 -> 20.2).  TQ2_0 rows longer than 2048 against less than 16 up to a half: its tiled kernel splits such k finer (1100 x 4096 x 512 23.5 -> 25.0).
+template <int FMT>
+bool skinny_fits(const lh_context* ctx, uint32_t m, uint32_t k, uint32_t blocks) {
     const uint64_t workgroups = (uint64_t)blocks * ((m + 63) / 64), cus = (uint64_t)ctx->cu_count;
-    return blocks <= skinny_max_blocks(ctx) && (m <= 64 || workgroups <= (m <= 256 ? 8 : 2) * cus);
+    if (blocks > skinny_max_blocks(ctx)) return false;
+    if (m <= 256) return m <= 64 || workgroups <= 8 * cus;
+    const uint32_t halves = blocks >= 16 ? 4 : FMT == kTQ2 && k > 2048 ? 1 : blocks >= 8 ? 3 : 2;
+    return 2 * workgroups <= halves * cus;
 }
 
 // k splits of the skinny kernel over `workgroups` (64-row blocks x groups of 64 activation rows): enough workgroups for every CU, a whole number of units
@@ -1395,7 +1402,7 @@ uint32_t skinny_splits(const lh_context* ctx, uint32_t m, uint32_t workgroups, u
 
 // The skinny kernel when the shape allows it (f16 activations, whole 128-row tiles, at least one unit of k per wave, skinny_fits); false
 // leaves the launch to the LDS-tiled kernels.  With `keep` the f32 partial
-// tiles (one split included) stay in the workspace for a consumer that sums them itself.
+// tiles (up to 256 rows one split included) stay in the workspace for a consumer that sums them itself.
 struct SkinnyPartials { const float* partial; uint32_t splits, cols; };
 template <int FMT, int ADT>
 bool try_skinny(lh_context* ctx, const void* A, const uint8_t* W, void* C, lh_dtype ct, uint32_t m, uint32_t k, uint32_t n, const ClipArgs& clip,
@@ -1428,13 +1435,16 @@ bool try_skinny(lh_context* ctx, const void* A, const uint8_t* W, void* C, lh_dt
         bool whole = grp.count ? true : n % BN == 0;          // every matrix fills its 128-row tiles
         for (uint32_t i = 0; i < grp.count; i++) whole = whole && grp.N[i] % BN == 0;
         const uint32_t units = k / Skinny<FMT>::unit_k;
-        if (!clip.enabled && m >= skinny_min_m(FMT) && whole && k % (4 * Skinny<FMT>::unit_k) == 0 && skinny_fits(ctx, m, 2 * tiles_n)) {
+        if (!clip.enabled && m >= skinny_min_m(FMT) && whole && k % (4 * Skinny<FMT>::unit_k) == 0 && skinny_fits<FMT>(ctx, m, k, 2 * tiles_n)) {
             // k splits: enough workgroups for every CU, a whole number of units per wave, partial tiles within half the workspace
             const uint32_t blocks = 2 * tiles_n, per_wg = units / 4;
             const uint64_t fit = (ctx->workspace_bytes / 2) / ((uint64_t)m * blocks * 64 * 4);
             if (keep && fit == 0) return false;
             const uint32_t mgroups = (m + 63) / 64;
             const uint32_t splits = skinny_splits(ctx, m, blocks * mgroups, per_wg);
+            // (Of many rows a finished f16 product costs its reader less than one f32 tile: TQ2_0, us, 448 x 1024 x 4096 and a norm 19.9 and 18.8,
+            // 1280 x 1024 x 1536 and the queries' preparation 37.9 and 34.3.)
+            if (keep && splits == 1 && m > 256) return false;
             float* partial = (splits > 1 || keep) ? static_cast<float*>(ctx->workspace) : nullptr;
             const dim3 grid(blocks, mgroups, splits);
             const uint16_t* X = static_cast<const uint16_t*>(A);
@@ -1524,7 +1534,7 @@ int launch_by_out(bool mfma, lh_context* ctx, const void* A, const uint8_t* W, v
             // tiled kernels make of them (TQ2_0, f32 out, us, tiled -> this: 65 x 2048 x 8192 19.9 -> 14.6, 256 x 1536 x 2048 16.7 -> 12.6, 384 x 1536 x 4096 18.9 ->
             // 17.0, 512 x 2048 x 2048 22.8 -> 16.9; with two, 256 x 2048 x 8192 21.3 -> 22.1, 512 x 1536 x 4096 18.1 -> 18.6).  They lie in the workspace's third quarter.
             const size_t half = ctx->workspace_bytes / 2;
-            if (!clip.enabled && n % BN == 0 && k % (4 * Skinny<FMT>::unit_k) == 0 && skinny_fits(ctx, m, n / 64) && (size_t)m * k * 2 <= half / 2 &&
+            if (!clip.enabled && n % BN == 0 && k % (4 * Skinny<FMT>::unit_k) == 0 && skinny_fits<FMT>(ctx, m, k, n / 64) && (size_t)m * k * 2 <= half / 2 &&
                 (uint64_t)(n / 64) * ((m + 63) / 64) * 2 <= 3 * (uint64_t)cus) {
                 uint16_t* a16 = reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(ctx->workspace) + half);
                 const size_t n8 = (size_t)m * k / 8;

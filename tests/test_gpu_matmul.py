@@ -566,6 +566,62 @@ def test_matmul_gelu_mul_strided_fused_equals_separate_kernels(pkg, gpu, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
+@pytest.mark.parametrize("m,k,n", [(257, 1536, 1536), (400, 1024, 4096), (1100, 512, 1024), (3000, 512, 512), (4096, 512, 512), (4100, 512, 256), (300, 512, 128)])
+def test_products_behind_many_rows_with_their_readers(pkg, gpu, fmt, m, k, n):
+    """More rows than a chunk, with k split (the readers sum the partial tiles) and not (they read the finished product), on both sides of the lines
+    for few weight rows: product and norm, product and strided GeGLU, a group of two, and the queries' product with their preparation,
+    alone and in a group, against the separate calls, bit for bit."""
+    ctx, K = gpu
+    ty = pkg.Q4_0 if fmt == "q4_0" else pkg.TQ2_0
+    g = pkg.synth.rng(84, m + k + n)
+    w = pkg.QuantWeight.from_bytes(ctx, pkg.synth.weights(fmt, n, k, g), ty, n, k)
+    half = lambda *s: pkg.Buffer.from_slice(ctx, (g.standard_normal(s, dtype=np.float32) * 0.5).astype(np.float16))
+    x, res, nw, gate = half(m, k), half(m, n), half(n), half(m, n + 64)
+    tmp, want, got, gwant, ggot = (pkg.Buffer.empty(ctx, m * n * 2) for _ in range(5))
+    hd, nq, nk = 128, n // 128, 1
+    levels, signs, norm = pkg.Buffer.from_slice(ctx, np.linspace(-1, 1, 4).astype(np.float32)), pkg.Buffer.from_slice(ctx, np.ones(hd, np.float32)), pkg.Buffer.from_slice(ctx, np.ones(hd, np.float16))
+    rqs = [pkg.Buffer.empty(ctx, m * n * 4) for _ in range(2)]
+    print(f"case {fmt} m={m} k={k} n={n}", flush=True)
+    batch = pkg.CommandBatch(ctx)
+    w.matmul_nt_into(batch, K, x, tmp, m)
+    batch.commit_and_wait()
+    alone = tmp.as_array(np.float16).astype(np.float32)
+    batch = pkg.CommandBatch(ctx)
+    K.rms_norm_add_into(batch, tmp, nw, res, want, n, m, 1e-6)
+    K.gelu_mul_strided_into(batch, tmp, gate, n + 64, 64, gwant, n, m)
+    K.matmul_nt_quant_norm_into(batch, ty, x, w.buf, m, k, n, nw, res, got, 1e-6)
+    K.matmul_nt_quant_gelu_mul_strided_into(batch, ty, x, w.buf, m, k, n, gate, n + 64, 64, ggot)
+    K.decode_qkv_prepare_rows_into(batch, tmp, None, None, norm, None, levels, signs, rqs[0], None, None, None, None, None, hd, nq, 0, m, 1e-6, 3, 1e4, 1.0, 2, 0, 0)
+    q = pkg.Buffer.empty(ctx, m * n * 2)
+    K.matmul_nt_q_prepare_rows_into(batch, ty, x, w.buf, k, q, norm, signs, rqs[1], None, hd, nq, m, 1e-6, 3, 1e4, 1.0, 0)
+    batch.commit_and_wait()
+    assert np.array_equal(got.as_array(np.uint16), want.as_array(np.uint16))
+    assert np.array_equal(ggot.as_array(np.uint16), gwant.as_array(np.uint16))
+    assert np.array_equal(rqs[0].as_array(np.uint32), rqs[1].as_array(np.uint32))
+    # the group: against the product on its own only as far as another split of k rounds
+    wk, wv = (pkg.QuantWeight.from_bytes(ctx, pkg.synth.weights(fmt, hd, k, g), ty, hd, k) for _ in range(2))
+    results = []
+    for fused in (False, True):
+        qkv = [pkg.Buffer.empty(ctx, m * c * 2) for c in (n, hd, hd)]
+        rq, kc, kn, vc, vn = (pkg.Buffer.empty(ctx, c) for c in (m * n * 4, m * hd // 4, m * 2, m * hd // 4, m * 2))
+        rest = (norm, norm, levels, signs, rq, kc, kn, vc, vn, None, hd, nq, nk, m, 1e-6, 0, 1e4, 1.0, 2, 0, 0)
+        batch = pkg.CommandBatch(ctx)
+        if fused:
+            K.matmul_nt_qkv_prepare_rows_into(batch, ty, x, w.buf, wk.buf, wv.buf, k, *qkv, *rest)
+        else:
+            K.matmul_nt_quant_grouped_into(batch, ty, x, [w.buf, wk.buf, wv.buf], qkv, m, k, [n, hd, hd])
+            batch.commit_and_wait()
+            grouped = qkv[0].as_array(np.float16).astype(np.float32)
+            batch = pkg.CommandBatch(ctx)
+            K.decode_qkv_prepare_rows_into(batch, *qkv, *rest)
+        batch.commit_and_wait()
+        results.append([b.as_array(np.uint8) for b in (rq, kc, kn, vc, vn)])
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
+    refgen.assert_close(grouped, alone, 1e-3, f"{fmt} grouped {m}x{k}x{n}")
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "tq2_0"])
 def test_mfma_matmul_split_k(pkg, gpu, oracle, fmt):
     """A decode batch of some tens of rows against the layer's projections: few output tiles, so the k range is split
     over several workgroups whose partial tiles a second kernel sums -- even and odd numbers of k steps per split, a
