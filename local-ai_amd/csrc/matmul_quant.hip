@@ -1532,10 +1532,15 @@ int launch_by_out(bool mfma, lh_context* ctx, const void* A, const uint8_t* W, v
         if constexpr (ADT == LH_BF16 && FMT != kF16W) {
             // Up to one and a half workgroups a CU the decode-batch kernel is worth a pass that makes f16 rows of bf16 ones, the same values that the
             // tiled kernels make of them (TQ2_0, f32 out, us, tiled -> this: 65 x 2048 x 8192 19.9 -> 14.6, 256 x 1536 x 2048 16.7 -> 12.6, 384 x 1536 x 4096 18.9 ->
-            // 17.0, 512 x 2048 x 2048 22.8 -> 16.9; with two, 256 x 2048 x 8192 21.3 -> 22.1, 512 x 1536 x 4096 18.1 -> 18.6).  They lie in the workspace's third quarter.
+            // 17.0, 512 x 2048 x 2048 22.8 -> 16.9; with two, 256 x 2048 x 8192 21.3 -> 22.1, 512 x 1536 x 4096 18.1 -> 18.6).  Beyond 64 rows the pass and the
+            // tiles of a split k weigh more the fewer weight rows there are: below 2048 it is worth them from 1024 on, up to one workgroup a CU and with k beyond 2048
+            // from 0.75 on (1024 x 1024 x 1024 18.2 -> 13.8, 1024 x 4096 x 1024 30.2 -> 26.6, but 1500 x 1024 x 1024 14.6 -> 17.9, 512 x 4096 x 1024 19.2 -> 21.6,
+            // 128 x 12288 x 1536 24.7 -> 26.7, 1024 x 2048 x 512 16.6 -> 19.8).  They lie in the workspace's third quarter.
             const size_t half = ctx->workspace_bytes / 2;
+            const uint64_t workgroups = (uint64_t)(n / 64) * ((m + 63) / 64);
+            const bool enough = m <= 64 || n >= 2048 || (n >= 1024 && workgroups <= (uint64_t)cus && (k <= 2048 || 4 * workgroups >= 3 * (uint64_t)cus));
             if (!clip.enabled && n % BN == 0 && k % (4 * Skinny<FMT>::unit_k) == 0 && skinny_fits<FMT>(ctx, m, k, n / 64) && (size_t)m * k * 2 <= half / 2 &&
-                (uint64_t)(n / 64) * ((m + 63) / 64) * 2 <= 3 * (uint64_t)cus) {
+                2 * workgroups <= 3 * (uint64_t)cus && enough) {
                 uint16_t* a16 = reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(ctx->workspace) + half);
                 const size_t n8 = (size_t)m * k / 8;
                 hipLaunchKernelGGL((convert_to_f16_kernel<LH_BF16>), dim3((uint32_t)((n8 + 255) / 256)), dim3(256), 0, s, A, a16, n8);

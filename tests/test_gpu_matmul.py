@@ -98,7 +98,7 @@ def test_many_rows_against_few_weight_rows(pkg, gpu, oracle, fmt, m, k, n):
 
 
 @pytest.mark.parametrize("fmt,m,k,n", [("q4_0", 17, 256, 128), ("tq2_0", 65, 512, 8192), ("q4_0", 200, 1536, 2048), ("tq2_0", 384, 512, 4096), ("tq2_0", 385, 512, 4096),
-                                       ("q4_0", 600, 2048, 1024)])
+                                       ("q4_0", 600, 2048, 1024), ("tq2_0", 64, 512, 256), ("tq2_0", 65, 512, 256), ("q4_0", 384, 4096, 1024), ("q4_0", 769, 4096, 1024)])
 def test_bf16_rows_made_f16_for_the_decode_batch_kernel(pkg, gpu, oracle, fmt, m, k, n):
     """bf16 rows on both sides of the line up to which they are made f16 ahead of the product (every value here is one of both)."""
     ctx, K = gpu
