@@ -15,6 +15,7 @@ toolchain exists where this library is built, so the file is generated and check
 from __future__ import annotations
 
 import os
+import re
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -22,6 +23,7 @@ sys.path.insert(0, HERE)
 import gen_ffi  # noqa: E402  (the header parser)
 
 OUT = os.path.join(HERE, "src", "kernels.rs")
+BY_HAND = os.path.join(HERE, "src", "lib.rs")
 
 # C parameter type -> (Rust parameter type, expression passed to the raw function)
 SCALAR = {"uint32_t": "u32", "uint64_t": "u64", "size_t": "usize", "float": "f32", "int": "c_int",
@@ -78,6 +80,8 @@ def wrap(name, ret, params):
 
 def generate(text: str) -> str:
     fns = gen_ffi.parse_header(text)
+    with open(BY_HAND) as f:
+        by_hand = set(re.findall(r"ffi::(lh_\w+)\(", f.read()))
     methods, skipped = [], []
     for name, ret, params in fns:
         src = wrap(name, ret, params)
@@ -85,11 +89,14 @@ def generate(text: str) -> str:
             methods.append(src)
         elif not name.startswith(NOT_OPS):
             skipped.append(name)
+            if params and squeeze(params[0][0]) in ("lh_batch*", "lh_context*") and name not in by_hand:
+                raise SystemExit(f"{name} is a dispatch operation that the header's types alone do not wrap: it needs a wrapper in src/lib.rs")
     lines = [
         "// The kernel-dispatch layer: `Kernels`, one method per operation of liblocal_hip.so, with the names and the argument",
         "// order that local-engine calls on local-metal (local-metal/src/kernels.rs).  GENERATED by gen_safe.py from",
-        "// include/local_hip.h: do not edit.  Host-side helpers that take plain pointers are not dispatch operations and are",
-        "// wrapped by hand in lib.rs: " + ", ".join(skipped) + ".",
+        "// include/local_hip.h: do not edit.  Operations with host pointers and the helpers of the codec are wrapped by hand in lib.rs: " +
+        ", ".join(n for n in skipped if n in by_hand) + ".",
+        "// Other host-side helpers are reached through `ffi`: " + ", ".join(n for n in skipped if n not in by_hand) + ".",
         "use core::ffi::c_int;",
         "",
         "use crate::batch::CommandBatch;",

@@ -77,3 +77,26 @@ pub fn flash_attention_tq_rotated_lazy_into(batch: &mut CommandBatch, rq: &Buffe
     })?;
     Ok(rotated != 0)
 }
+
+/// The pointer of a buffer that a call may go without.
+fn opt(buffer: Option<&Buffer>) -> *mut ffi::lh_buffer {
+    buffer.map_or(core::ptr::null_mut(), Buffer::as_ptr)
+}
+
+/// `lh_matvec_quant_norm_chain_gelu_into` (include/local_hip.h): gate and up projection (or, with `factor` instead of `up`, one
+/// projection) behind a chain of norms, and the GeGLU product of their results where the launch can form it (layer.rs:476-482,
+/// 495-500).  `Ok(true)`: `out` holds the product.  `Ok(false)`: `out` and `up_out` hold the projections' results.
+#[allow(clippy::too_many_arguments)]
+pub fn matvec_quant_norm_chain_gelu_into(batch: &mut CommandBatch, fmt: ffi::lh_quant, gate: &Buffer, up: Option<&Buffer>,
+                                         factor: Option<&Buffer>, vector: &Buffer, weight: &Buffer, residual: Option<&Buffer>,
+                                         next_weight: Option<&Buffer>, store: Option<&Buffer>, eps: f32, out: &Buffer,
+                                         up_out: Option<&Buffer>, rows: u32, cols: u32) -> Result<bool> {
+    let mut applied: core::ffi::c_int = 0;
+    // SAFETY: every pointer is null or comes from a live handle of this crate or from a local; the library validates sizes and shapes.
+    error::check(unsafe {
+        ffi::lh_matvec_quant_norm_chain_gelu_into(batch.as_ptr(), fmt, gate.as_ptr(), opt(up), opt(factor), vector.as_ptr(),
+                                                  weight.as_ptr(), opt(residual), opt(next_weight), opt(store), eps,
+                                                  out.as_ptr(), opt(up_out), rows, cols, &mut applied)
+    })?;
+    Ok(applied != 0)
+}

@@ -155,6 +155,22 @@ def test_safe_layer_methods_follow_the_header():
         assert (name in wrapped) == is_op, name
 
 
+def test_operations_without_a_generated_method_are_wrapped_by_hand():
+    """Dispatch operations with arguments that the generator does not take (an `int*` result) have a wrapper in lib.rs, and what
+    kernels.rs says is wrapped there is."""
+    lib = open(os.path.join(ROOT, "local-hip", "src", "lib.rs")).read()
+    text = open(KERNELS_RS).read()
+    generated = {raw for _, _, raw, _ in safe_methods()}
+    others = {name for name, _, cparams in c_functions() if cparams and cparams[0][0] in ("lh_batch*", "lh_context*") and name not in generated
+              and not name.startswith(("lh_context_", "lh_buffer_", "lh_batch_", "lh_event_", "lh_graph_", "lh_debug_"))}
+    assert "lh_matvec_quant_norm_chain_gelu_into" in others
+    for name in others:
+        assert re.search(rf"pub fn {name[3:]}\(", lib) and f"ffi::{name}(" in lib, name
+    named, = re.findall(r"wrapped by hand in lib\.rs: ([^.]*)\.", text)
+    for name in named.split(", "):
+        assert f"ffi::{name}(" in lib, name
+
+
 def test_safe_layer_argument_order_of_the_reference():
     """Three methods whose parameter lists were read off the reference (local-metal/src/kernels.rs:4819-4834, 5176-5193,
     5434-5452; kept here as data): the generated methods take exactly these parameters in exactly this order."""
