@@ -12,7 +12,7 @@
 // 4g + j - 4 of tile 1, which is the order of the value blocks.  Scores, weights and sums are f32; a weight enters the
 // product as the sum of three bf16 terms, which is all of its 24 bits.
 //   attention_tile_kernel   many rows: four waves share key and value blocks through LDS
-//   attention_one_kernel    one row over up to 640 keys: one workgroup per kv head
+//   attention_one_kernel    one row over a few hundred keys (one_blocks): one workgroup per kv head
 //   attention_split_kernel  few rows: every wave walks its own share of the blocks straight from global memory; the
 //                           workgroup's four partial results are merged in LDS, the workgroups' by attention_merge_kernel
 //   attention_wide_kernel   f32 caches: f32 matrix instructions, 16 packed rows a workgroup
@@ -365,11 +365,15 @@ __global__ __launch_bounds__(256) void attention_split_kernel(const AttentionArg
 // One row (a decoded token) over a context that one workgroup per kv head gets through: its waves take blocks of 32 keys in turn and meet in LDS, where the rows are
 // finished.  Bound by the chain from the launch to the row and by the 65 GB/s or so that one CU reads, so everything that does not depend on the position is
 // requested ahead of it -- the queries, and a wave's first block whether or not it is visible (it is in the cache) -- and there is no division and no second launch.
-// 16 heads of 64 and 128 over 4 kv heads, two maps, recorded launches: 32 keys 5.6 us, 256 7.9, 512 10.4, 640 11.7, 768 13.1; in the split form with its merge 10.8,
-// 12.2, 12.3, 12.4 and 12.4, and the other way round from kOneBlocks on for 13 heads over one and 16 over 2 or 16 as well.  The leading arguments arrive in registers
-// with the wave; the structure repeats them.
+// 16 heads of 64 and 128 over 4 kv heads, two maps, recorded launches: 32 keys 5.6 us, 256 7.9, 512 10.4; in the split form with its merge 10.8, 12.2 and 12.3.  The
+// leading arguments arrive in registers with the wave; the structure repeats them.
 constexpr int kOneWaves = 8;
-constexpr uint32_t kOneBlocks = 20;
+// Most blocks that the caller may ask of it, by the columns of a position that a CU reads: `values` of all maps' key and the value.  The split form takes a round of
+// blocks for every four, so that it is the shorter way first where their number is a multiple of four.  (Times of this one over the split one's at 8, 11, 12, 15, 16, 19
+// and 20 blocks, geometric means over up to six shapes: 192 columns 0.66, 0.68, 0.76, 0.77, 0.85, 0.86, 0.95; 256 0.68, 0.69, 0.79, 0.80, 0.90, 0.88, 0.97, up to 1.04;
+// 320 0.83, 0.82, 0.99, 0.95, 1.13, 1.09, 1.30; 384 and 448 0.86, 0.86, 1.04, 1.04, 1.24, 1.15, 1.38.  The line is that of the positions a recorded step may reach.)
+constexpr uint32_t one_blocks(uint32_t values) { return values <= 192 ? 20 : values <= 256 ? 19 : values <= 320 ? 15 : 11; }
+constexpr bool one_fits(uint32_t values, uint32_t blocks) { return blocks <= (values > 256 && blocks % 4 == 0 ? 8 : one_blocks(values)); }
 template <int DQ, int DV, int MAPS>
 __global__ __launch_bounds__(64 * kOneWaves) void attention_one_kernel(const uint16_t* queries, const uint16_t* keys, const uint16_t* values, const uint32_t* position, uint32_t kv_heads,
                                                                        uint32_t R, uint32_t blocks, const AttentionArgs a) {
@@ -508,7 +512,7 @@ int launch_mfma(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const 
     }
     if constexpr (MAPS * DV <= 256 && DQ + DV <= 448) {       // (what the registers hold)
         constexpr size_t per_row = (size_t)kOneWaves * MAPS * (DV + 4) * 4;
-        if (a.rows == 1 && R <= 16 && max_blocks <= kOneBlocks && R * per_row <= 160 * 1024) {
+        if (a.rows == 1 && R <= 16 && one_fits(MAPS * DQ + DV, max_blocks) && R * per_row <= 160 * 1024) {
             if (R * per_row > 64 * 1024) {
                 const int r = lh_raise_dynamic_lds(ctx, (const void*)attention_one_kernel<DQ, DV, MAPS>, R * per_row, op);
                 if (r != LH_OK) return r;

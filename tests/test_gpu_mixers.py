@@ -499,6 +499,22 @@ def test_attention_of_one_row(ai, gpu, dtype, heads, kv_heads, maps, dim, vdim, 
     attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, 1, (start + 32) // 32 * 32)
 
 
+@pytest.mark.parametrize("heads,kv_heads,maps,dim,vdim,alone,split", [(8, 2, 1, 64, 64, [638], [639]), (16, 4, 2, 64, 128, [606], [607]), (8, 2, 1, 128, 128, [606], [607]),
+                                                                      (8, 2, 1, 192, 128, [350, 383, 478], [351, 382, 479]), (4, 2, 2, 128, 128, [350], [351, 382, 511]),
+                                                                      (8, 1, 1, 192, 256, [255, 350], [351, 638])])
+def test_attention_of_one_row_by_the_columns_of_a_position(ai, gpu, heads, kv_heads, maps, dim, vdim, alone, split):
+    """Wide rows are read by many workgroups from fewer keys on: one launch up to a line, two behind it."""
+    ctx, K = gpu
+    b = ai.Buffer.empty(ctx, 672 * kv_heads * (maps * 192 + 256) * 2)
+    b.fill_zero()
+    for start in alone + split:
+        attention_case(ai, gpu, "bf16", maps, heads, kv_heads, dim, vdim, start, 1, (start + 32) // 32 * 32)
+        batch = ai.CommandBatch(ctx)
+        K.attention_rows_into(batch, b, b, b, ai.Buffer.empty(ctx, heads * vdim * 2), ai.BF16, b, start, 1, heads, kv_heads, maps, dim, vdim, 672, 1.0, 0.4, 0.7, 1e-5)
+        assert batch.dispatch_count() == (1 if start in alone else 2), start
+        batch.commit_and_wait()
+
+
 @pytest.mark.parametrize("rows", [1, 40, 200])
 def test_attention_ignores_what_lies_behind_the_last_position(ai, gpu, rows):
     """Stale rows and block entries past the last position (a slot that is used again) must not change a bit."""
