@@ -155,24 +155,31 @@ __device__ __forceinline__ s16x4 transposed4(const void* lds) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)lds);
 }
 
-// grid: row tiles x splits; packed row r = head r % heads of query row r / heads.  The splits of a row tile take the blocks of 32 positions of
-// the visible range in turn.  The four waves share a block in LDS, in tiles of 8 key rows x 8
+// grid: row tiles x splits; packed row r = head r % heads of query row r / heads.  The blocks of 32 positions of the visible range are dealt out
+// to the splits of a row tile, in turn or in contiguous runs.  The four waves share a block in LDS, in tiles of 8 key rows x 8
 // chunks of 16 bytes, chunk c of row k at place c ^ k of its row (a load fills one tile, and every address is one of a few per
 // lane plus a constant), while the next block is on its way into a second buffer.  A wave takes every fourth 32 columns of the
 // scores' sums, which meet in LDS, and a quarter of the value columns, which it reads through the transposing LDS read.  A query
 // value enters as the sum of two bf16 terms.
-template <int DV>
+// ONE: a token, whose chain is without divisions by the heads and has the first block requested ahead of the queries.
+// The blocks go in turn to splits with a CU each, where each walks as few as there can be, and in runs to more than that: what a split of the first then has
+// no block for costs no CU its time.  (Rank 512, 2000 keys, with the merge: 8 rows of 8 heads, 124 workgroups, 14.5 us in turn and 15.7 in runs; 5 of 64, 520,
+// 26.7 and 23.2; 16 of 16, 496, 22.7 and 20.4.)
+template <int DV, bool ONE>
 __global__ __launch_bounds__(256) void latent_split_kernel(const AttentionArgs a) {
     constexpr int DQ = DV + kRotPad, KT = DQ / 64, NC = (DQ / 32 + 3) / 4, ND = DV / 64, kBlock = 4 * KT * 64;
     extern __shared__ __align__(16) uint4 sm[];             // two blocks, then the partial scores [4 waves][2 tiles][64 lanes]
     lh_f32x4* sums = reinterpret_cast<lh_f32x4*>(sm + 2 * kBlock);
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, lc = lane & 15;
-    uint32_t split = blockIdx.x, tile = 0, t_first = 0, t_last = 0, t_row = 0;     // of the packed rows: the query rows of the first, the last and this lane's
-    const uint32_t start = *a.position, packed = a.rows * a.heads;
-    if (packed > 16) { tile = split / a.splits; split -= tile * a.splits; }
+    const uint32_t start = *a.position, packed = ONE ? a.heads : a.rows * a.heads;
+    uint32_t split = blockIdx.x, tile = 0;
+    if (!ONE || packed > 16) { tile = split / a.splits; split -= tile * a.splits; }
     const uint32_t row0 = tile * 16, row_last = min(row0 + 16, packed) - 1, row = row0 + lc;
-    if (a.rows > 1) { t_first = row0 / a.heads; t_last = row_last / a.heads; t_row = row / a.heads; }     // (a token's chain is without the divisions)
-    const uint32_t last_key = min(start + t_last, a.capacity - 1), nb = last_key / 32 + 1, limit = min(start + t_row, last_key), first_limit = start + t_first;
+    const uint32_t last_key = min(start + (ONE ? 0u : row_last / a.heads), a.capacity - 1), nb = last_key / 32 + 1;
+    const uint32_t limit = min(start + (ONE ? 0u : row / a.heads), last_key), first_limit = start + (ONE ? 0u : row0 / a.heads);
+    const bool turns = ONE || gridDim.x <= a.resident;
+    const uint32_t per = (nb + a.splits - 1) / a.splits, step = turns ? a.splits : 1u;
+    const uint32_t b0 = turns ? split : min(split * per, nb), b1 = turns ? nb : min(b0 + per, nb);
     const uint16_t* cache = static_cast<const uint16_t*>(a.keys) + ((lane & 7) ^ (lane >> 3)) * 8;
     auto load_block = [&](uint32_t b, uint32_t buf) {         // a wave brings in eight key rows
         const uint16_t* key = cache + (size_t)min(b * 32 + wave * 8 + (lane >> 3), last_key) * DQ;               // keys past the last are masked
@@ -181,7 +188,7 @@ __global__ __launch_bounds__(256) void latent_split_kernel(const AttentionArgs a
         for (int i = 0; i < KT; i++) __builtin_amdgcn_global_load_lds((gvoid*)(key + i * 64), (lvoid*)(to + i * 64), 16, 0, 0);
     };
     uint32_t buf = 0;
-    if (split < nb) load_block(split, 0);                     // ahead of the queries, which are converted below
+    if (ONE && b0 < b1) load_block(b0, 0);
     lh_bf16x8 qh[NC], ql[NC];
 #pragma unroll
     for (int i = 0; i < NC; i++) {
@@ -203,6 +210,7 @@ __global__ __launch_bounds__(256) void latent_split_kernel(const AttentionArgs a
         qh[i] = __builtin_bit_cast(lh_bf16x8, (u32x4){h[0], h[1], h[2], h[3]});
         ql[i] = __builtin_bit_cast(lh_bf16x8, (u32x4){l[0], l[1], l[2], l[3]});
     }
+    if (!ONE && b0 < b1) load_block(b0, 0);
     lh_f32x4 o[ND];
 #pragma unroll
     for (int d = 0; d < ND; d++) o[d] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
@@ -213,10 +221,10 @@ __global__ __launch_bounds__(256) void latent_split_kernel(const AttentionArgs a
     const uint32_t vk = g * 4 + (lc >> 2);
     const char* vp = reinterpret_cast<const char*>(sm + (vk >> 3) * (KT * 64) + (vk & 7) * 8) + (lane & 1) * 8;
 
-    for (uint32_t b = split; b < nb; b += a.splits, buf ^= kBlock) {
+    for (uint32_t b = b0; b < b1; b += step, buf ^= kBlock) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         lh_lds_barrier();                                     // the block has arrived, and the one before has been read by all
-        if (b + a.splits < nb) load_block(b + a.splits, buf ^ kBlock);
+        if (b + step < b1) load_block(b + step, buf ^ kBlock);
         lh_f32x4 s[2], low[2];                                // four sums that do not wait for each other
 #pragma unroll
         for (int t = 0; t < 2; t++) s[t] = low[t] = (lh_f32x4){0.f, 0.f, 0.f, 0.f};
@@ -314,11 +322,12 @@ int launch_split(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const
     a.splits = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({tiles == 1 && max_blocks <= 48 ? max_blocks : max_blocks / 2, (want + tiles - 1) / tiles, room}));
     LH_REQUIRE(tiles * a.splits < 0x7FFFFFFFull && (uint64_t)a.rows * a.heads < 0x7FFFFFFFull, "%s: %u rows", op, a.rows);
     a.partial = (float*)ctx->workspace;
+    a.resident = (uint32_t)ctx->cu_count;
     if (lds > 64 * 1024) {
-        const int r = lh_raise_dynamic_lds(ctx, (const void*)latent_split_kernel<DV>, lds, op);
+        const int r = lh_raise_dynamic_lds(ctx, a.rows == 1 ? (const void*)latent_split_kernel<DV, true> : (const void*)latent_split_kernel<DV, false>, lds, op);
         if (r != LH_OK) return r;
     }
-    hipLaunchKernelGGL((latent_split_kernel<DV>), dim3((uint32_t)(tiles * a.splits)), dim3(256), lds, ctx->stream, a);
+    hipLaunchKernelGGL((a.rows == 1 ? latent_split_kernel<DV, true> : latent_split_kernel<DV, false>), dim3((uint32_t)(tiles * a.splits)), dim3(256), lds, ctx->stream, a);
     int r = lh_check_launch(op);
     if (r != LH_OK) return r;
     launches = 2;

@@ -125,6 +125,13 @@ def latent_case(ai, gpu, dtype, heads, rank, rot, start, rows, capacity, spike=N
     return got
 
 
+@pytest.mark.parametrize("rows,heads,rank,start", [(5, 64, 64, 1995), (16, 16, 128, 1000), (16, 16, 64, 497), (8, 8, 512, 1990), (2, 40, 256, 2047), (1, 40, 256, 2047)])
+def test_latent_attention_of_a_few_rows_in_turn_and_in_runs(ai, gpu, rows, heads, rank, start):
+    """Up to a workgroup a CU the splits take blocks in turn, beyond in runs: blocks that do not fill the splits, splits without any."""
+    latent_case(ai, gpu, "bf16", heads, rank, 16, start, rows, (start + rows + 31) // 32 * 32)
+    latent_case(ai, gpu, "bf16", heads, rank, 16, start, rows, (start + rows + 31) // 32 * 32, spike=(rows - 1, 3))
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("rows,heads,rank,rot,vdim,start", [(1, 1, 5, 2, 3, 0), (1, 8, 512, 64, 128, 257), (1, 16, 512, 64, 130, 31), (1, 17, 100, 16, 40, 700), (1, 3, 128, 20, 16, 767),
                                                             (1, 4, 256, 64, 64, 768), (1, 2, 500, 64, 17, 64), (3, 8, 512, 64, 128, 90)])
