@@ -278,8 +278,11 @@ __global__ __launch_bounds__(256) void latent_split_kernel(const AttentionArgs a
 // columns of a head merges all of the head's latent columns for itself, its weights already on their way.  Quarters of K and their order as in
 // head_tile.  (Attention and projection, rank 512, warm: 8 heads and 256 keys 11.8 us with a launch of its own and 10.0 with this, 16 heads
 // 12.2 and 10.7, 32 heads and 1024 keys 15.2 and 13.9.)  Up to 24 splits: then reading all of them in every workgroup costs what the launch
-// does (8 heads: 512 keys 11.8 and 10.8, 1024 12.5 and 12.4, 1500 12.5 and 13.7; 16 heads, 1024: 13.3 and 13.5).
+// does (8 heads: 512 keys 11.8 and 10.8, 1024, 33 splits, 12.5 and 12.4, 1500, 47, 12.5 and 13.7; 16 heads, 1024: 13.3 and 13.5).  And while all
+// workgroups read up to 12 MB: with many heads that is the longer way from fewer splits on (128 heads, 6 splits, 12 MB: 18.1 and 17.2; 8, 16 MB: 16.9 and 17.6;
+// 16, 32 MB: 18.4 and 22.0; 64 heads, 12, 12 MB: 15.9 and 15.1; 23, 23 MB: 18.7 and 19.6).
 constexpr uint32_t kValueSplits = 24;
+constexpr uint64_t kValueBytes = 12ull << 20;
 __global__ __launch_bounds__(kMergeThreads) void latent_values_kernel(const AttentionArgs a, const HeadArgs v) {
     __shared__ MergeSpace<1> space;
     __shared__ __align__(16) uint16_t x[512];
@@ -317,9 +320,12 @@ int launch_split(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const
     const size_t rec = (size_t)tiles * 16 * (DV + 4) * 4;
     const uint32_t room = (uint32_t)std::min<size_t>(ctx->workspace_bytes / rec, kMaxSplits);
     LH_REQUIRE(room >= 1, "%s: %u rows of %u heads exceed the workspace", op, a.rows, a.heads);
-    // A block a split for one row tile, until merging them costs what the second block of a split does (with the merge, 8 heads: 256 keys 10.4 us with two and 8.9
-    // with one, 1024 10.5 and 9.5, 2048 10.8 and 10.5, 16 heads there 11.4 and 11.5, 8192 13.6 and 16.5).
-    a.splits = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({tiles == 1 && max_blocks <= 48 ? max_blocks : max_blocks / 2, (want + tiles - 1) / tiles, room}));
+    // A block a split for one row tile, until merging them costs what the second block of a split does (with a merge of its own, 8 heads: 256 keys 10.4 us with two and 8.9
+    // with one, 1024 10.5 and 9.5, 2048 10.8 and 10.5, 16 heads there 11.4 and 11.5, 8192 13.6 and 16.5), or where the projection takes them, until those are too many for
+    // it (with the projection, 8 heads: 1024 keys 12.4 with two, 12.7 with one; where 1530 may come and 300 have, 11.7 and 12.7, as most of them have no block).
+    const bool token = values && a.rows == 1;
+    const uint32_t one_each = token ? kValueSplits : 48;
+    a.splits = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({tiles == 1 && max_blocks <= one_each ? max_blocks : max_blocks / 2, (want + tiles - 1) / tiles, room}));
     LH_REQUIRE(tiles * a.splits < 0x7FFFFFFFull && (uint64_t)a.rows * a.heads < 0x7FFFFFFFull, "%s: %u rows", op, a.rows);
     a.partial = (float*)ctx->workspace;
     a.resident = (uint32_t)ctx->cu_count;
@@ -331,7 +337,7 @@ int launch_split(lh_context* ctx, AttentionArgs& a, uint32_t max_position, const
     int r = lh_check_launch(op);
     if (r != LH_OK) return r;
     launches = 2;
-    projected = values && a.rows == 1 && a.splits <= kValueSplits;
+    projected = token && a.splits <= kValueSplits && (uint64_t)a.heads * ((values->N + 15) / 16) * a.splits * DV * 4 <= kValueBytes;
     if (!projected) return launch_merge<1>(ctx, a, op);
     hipLaunchKernelGGL(latent_values_kernel, dim3((values->N + 15) / 16, a.heads), dim3(kMergeThreads), 0, ctx->stream, a, *values);
     return lh_check_launch(op);

@@ -158,6 +158,28 @@ def test_latent_attention_with_the_value_projection(ai, gpu, dtype, rows, heads,
     assert not one[-8:].any()
 
 
+@pytest.mark.parametrize("heads,vdim,limit,launches", [(128, 128, 414, 2), (128, 128, 415, 3), (64, 128, 767, 2), (64, 128, 831, 3), (128, 130, 350, 2), (128, 130, 383, 3),
+                                                       (8, 128, 766, 2), (8, 128, 1534, 2), (8, 128, 1599, 3)])
+def test_latent_value_projection_by_what_its_workgroups_read(ai, gpu, heads, vdim, limit, launches):
+    """A merge of its own for more than 24 splits and where the workgroups of the projection would read more than 12 MB.  `limit`: the position that the launch may meet, with
+    the token there and far in front of it."""
+    ctx, K = gpu
+    rank, rot, g = 512, 64, np.random.default_rng(heads)
+    capacity = (limit + 32) // 32 * 32
+    cache = upload(ai, ctx, cache_rows(K, g.standard_normal((capacity, rank)), g.standard_normal((capacity, rot))), ai.BF16)
+    q, uv = f32(ai, ctx, g.standard_normal((heads, K.latent_row(rank, rot)))), ai.Buffer.from_slice(ctx, M.bf16_bits(g.standard_normal((heads, vdim, rank)) / np.sqrt(rank)))
+    latent, want, got = empty(ai, ctx, heads * rank, ai.BF16), empty(ai, ctx, heads * vdim, ai.BF16), empty(ai, ctx, heads * vdim, ai.BF16)
+    for at in (limit, 40):
+        pos, batch = ai.Buffer.from_slice(ctx, np.array([at], np.uint32)), ai.CommandBatch(ctx)
+        args = (ai.BF16, pos, limit, 1, heads, rank, rot, capacity, 1.0 / np.sqrt(rank + rot))
+        K.latent_attention_values_into(batch, q, cache, latent, *args, None, None, uv, vdim, got)
+        assert batch.dispatch_count() == launches
+        K.latent_attention_rows_into(batch, q, cache, latent, *args)
+        K.head_linear_into(batch, latent, ai.BF16, uv, want, ai.BF16, 1, heads, vdim, rank, vdim)
+        batch.commit_and_wait()
+        close(download(ai, got, heads * vdim, ai.BF16), download(ai, want, heads * vdim, ai.BF16), BF16_TOL, "values")
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("rows,heads,dim,rank,rot,own", [(1, 1, 3, 5, 2, True), (1, 6, 64, 128, 16, False), (1, 16, 128, 512, 64, True), (40, 3, 40, 96, 20, True)])
 def test_latent_queries_equal_the_two_steps(ai, gpu, dtype, rows, heads, dim, rank, rot, own):
