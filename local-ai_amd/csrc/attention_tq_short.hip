@@ -12,7 +12,7 @@
 //   * everything that comes from memory -- queries, codes of both kinds, norms -- is requested at the top, ahead of the level table, on which the
 //     rest depends.
 // Bound by the chain of one group and by a SIMD's two or three waves taking turns to issue.  From the first to the last instruction of one token over a
-// window of 512: 10.7 us there, 6.1 here; launches of 1 query 12.8 and 7.6, of 256 rows 14.3 and 10.2.
+// window of 512: 10.7 us there, 6.1 here.  Recorded launches one after the other, a window of 512: 1 query 10.1 us there and 7.2, 64 lanes 11.9 and 8.1, 256 rows 11.2 and 9.8.
 #include "attention_tq.hpp"
 #include <algorithm>
 #include <cstdlib>

@@ -11,8 +11,8 @@
 //   * the vector after its prologue consists of f16 values, and a code less its zero point is exact in f16 too: v_dot2_f32_f16
 //     multiplies them exactly (subnormal values included) and adds in f32; it truncates, so its sums stay short (four products).
 // (Per launch in a token, weights cold: TQ2_0 2 x 6144 x 1536 behind the norms of a layer's end 10.2 us in the matrix-core form; with 2 x 12288 x 1536
-// 8.5 on average in this one at first, and 7.2 since the first loads' arguments arrive with the wave, all waves share the prologue and a shift and an AND take
-// codes apart; 1536 x 6144 behind GeGLU 12.2, 6.1 and now 5.1, 1536 x 12288 14.2, 7.5 and 6.6, that product being formed by the launch in front.  Q4_0,
+// 8.5 on average in this one at first, and 7.2 since the first loads' arguments arrive with the wave, all waves share the prologue and the vector is requested ahead
+// of the weights; 1536 x 6144 behind GeGLU 12.2, 6.1 and now 4.5, 1536 x 12288 14.2, 7.5 and 5.7, that product being formed by the launch in front.  Q4_0,
 // against the form with v_dot4, one launch after the other: 2048 x 2048 5.0 and 3.6, 2 x 6144 x 1536 behind a norm 8.0 and 6.8; in a token 1536 x 2048
 // behind a rotation 5.4 and now 4.0.)
 #include "common.hpp"
@@ -59,7 +59,8 @@ constexpr int direct_elements(int ng, int kind) { return ng == 1 && kind != (int
 // The matrices of a launch: one; several, each with results of its own; or a gate and an up projection whose rows of one index are the two
 // halves of a wave, which leaves gelu(gate) * up of the two f16 results; or one whose results leave as gelu(result) * factor.  (The product
 // behind them would make the same of them in its prologue, but each of its workgroups again: a quantized token of ten
-// layers 659 us with those prologues, 640 without.)
+// layers 659 us with those prologues, 640 without.  Both launches, with the prologue and without, TQ2_0: two of 1024 rows, four to six groups of columns,
+// 8192 12.6 us and 10.9, 10240 14.4 and 12.6, 12288 15.1 and 13.2; one of 512 rows 11.0 and 9.7, 12.4 and 11.1, 12.9 and 11.6; Q4_0 alike, 164 shapes 0.84.)
 enum : int { kOne = 0, kSeveral = 1, kGated = 2, kFactor = 3 };
 
 template <int E> struct Elements { uint32_t w[E / 2]; };
