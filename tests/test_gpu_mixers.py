@@ -495,7 +495,8 @@ def test_attention_finds_one_key_far_away(ai, gpu, dtype, rows, key):
 @pytest.mark.parametrize("heads,kv_heads,maps,dim,vdim", [(16, 1, 2, 64, 128), (17, 1, 1, 64, 128), (4, 4, 1, 192, 256), (6, 3, 2, 40, 30)])
 @pytest.mark.parametrize("start", [0, 255, 256, 638, 639, 640])
 def test_attention_of_one_row(ai, gpu, dtype, heads, kv_heads, maps, dim, vdim, start):
-    """One block of keys, one and two a wave, the longest context that a workgroup takes and the next; sixteen heads a kv head and seventeen."""
+    """One block of keys, one and two a wave, the longest context that a workgroup takes of narrow positions and the next (of wide ones: the test below);
+    sixteen heads a kv head and seventeen."""
     attention_case(ai, gpu, dtype, maps, heads, kv_heads, dim, vdim, start, 1, (start + 32) // 32 * 32)
 
 
