@@ -166,7 +166,8 @@ class PipelineSequences:
                     lo += 1
                     continue
                 hi = min([p for p in want if p > lo] + [last, lo + seq.max_batch])
-                seq.forward_tokens_batch(list(tokens[lo:hi]), seq.position, batch=CommandBatch(seq.ctx))
+                fill = getattr(seq, "fill_caches_batch", None) or seq.forward_tokens_batch
+                fill(list(tokens[lo:hi]), seq.position, batch=CommandBatch(seq.ctx))
                 seq.position += hi - lo
                 lo = hi
         except BaseException as e:

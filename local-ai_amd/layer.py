@@ -250,6 +250,10 @@ class TransformerLayer:
         return (self.group_projections and self.fuse_norm_chain and q.ty != W_F16 and q.ty == k.ty == v.ty
                 and q.cols == k.cols == v.cols)
 
+    def owns_cache(self) -> bool:
+        """Whether the layer writes keys and values (it reads another's otherwise)."""
+        return not self.params.is_kv_shared and self.weights.attn_k is not None and self.weights.attn_v is not None
+
     def _queries_as_one(self) -> bool:
         return self.group_projections and self.fuse_norm_chain and self.weights.attn_q.ty != W_F16
 
@@ -494,18 +498,20 @@ class TransformerLayer:
     # -------------------------------------- n consecutive rows of one sequence
     def forward_batch(self, kernels: Kernels, batch, n_rows: int, start_pos: int, input: Buffer, output: Buffer,
                       bs: BatchScratch, ones: Buffer, kv_cache: QuantizedKvCache, ple_all=None, prenormed: bool = False,
-                      next_norm: Optional[Buffer] = None) -> None:
+                      next_norm: Optional[Buffer] = None, cache_only: bool = False) -> None:
         """layer.rs:542-718: rows at positions ``start_pos .. start_pos + n_rows``; ``ple_all`` is
         ``(buffer [n_rows, n_layer_total, per_layer_dim] f16, n_layer_total)``.  ``prenormed``: ``bs.normed`` already
         holds this layer's attention norm of ``input`` (the previous layer was given this layer's norm weight as its
-        ``next_norm``)."""
+        ``next_norm``).  ``cache_only``: the layer ends where the rows' keys and values are in its cache; ``output`` is not written."""
         self._check_rows(n_rows, bs)
         p, w = self.params, self.weights
         rows, h, hd, n_head, n_kv, eps = n_rows, p.hidden_size, p.head_dim, p.num_attention_heads, \
             p.num_key_value_heads, p.rms_norm_eps
         kv_len = start_pos + n_rows
 
-        own_kv = not p.is_kv_shared and w.attn_k is not None and w.attn_v is not None
+        own_kv = self.owns_cache()
+        if cache_only and not own_kv:
+            return
         one_prepare = self._one_prepare()
         if not prenormed:
             kernels.rms_norm_into(batch, input, w.attn_norm, bs.normed, h, rows, eps)
@@ -514,6 +520,8 @@ class TransformerLayer:
             kv_cache.project_and_prepare_rows_into(batch, kernels, w.attn_q.ty, bs.normed, w.attn_q.buf, w.attn_k.buf,
                                                    w.attn_v.buf, w.attn_q.cols, bs.q, bs.k, bs.v, w.q_norm, w.k_norm, bs.rq,
                                                    start_pos, n_rows, n_head, eps, p.rope_theta, p.partial_rotary_factor)
+            if cache_only:
+                return
             kv_cache.attention_rows_from_rotated_into(batch, kernels, bs.rq, bs.vacc, bs.attn_out, kv_len, start_pos, rows,
                                                       n_head, p.sliding_window)
             self._attention_tail(kernels, batch, rows, input, output, bs, ple_all, next_norm)
@@ -533,6 +541,8 @@ class TransformerLayer:
             kv_cache.prepare_rows_into(batch, kernels, bs.q, bs.k if own_kv else None, bs.v if own_kv else None, w.q_norm,
                                        w.k_norm, bs.rq, start_pos, n_rows, n_head, eps, p.rope_theta,
                                        p.partial_rotary_factor)
+            if cache_only:
+                return
             kv_cache.attention_rows_from_rotated_into(batch, kernels, bs.rq, bs.vacc, bs.attn_out, kv_len, start_pos, rows,
                                                       n_head, p.sliding_window)
         else:
@@ -545,6 +555,8 @@ class TransformerLayer:
                 kernels.rms_norm_into(batch, bs.v, ones, bs.v, hd, rows * n_kv, eps)
                 kernels.rope_batch_into(batch, bs.k, start_pos, p.rope_theta, hd, n_kv, rows, p.partial_rotary_factor)
                 kv_cache.write_kv_gpu_into(batch, kernels, bs.k, bs.v, start_pos, n_rows)
+            if cache_only:
+                return
             kv_cache.fused_attention_batch_into(batch, kernels, bs.q, bs.rq, bs.vacc, bs.attn_out, kv_len, start_pos, rows,
                                                 n_head, p.sliding_window)
         self._attention_tail(kernels, batch, rows, input, output, bs, ple_all, next_norm)

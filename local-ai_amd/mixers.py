@@ -26,6 +26,7 @@ CHUNKED_MIN_ROWS = 17      # below this a portion walks the recurrence
 MAX_CHUNKED_DIM = 256
 GATED_IN_PRODUCT = 2048    # longer gated norms are a step of their own: every wave of the product would repeat them
 EXPANDED_MIN_ROWS = 65     # from here on latent attention makes keys and values of every head out of its cache
+NO_ROW = -1                # of a pass: it runs for what it leaves in caches and states
 
 
 class Workspace:
@@ -58,6 +59,21 @@ class Run:
     store: Optional[Buffer] = None   # where the next norm leaves the (summed) stream; None: x stays as it is
     other: Optional[Buffer] = None   # norms behind the branches: the stream's second buffer
     pending: Optional[tuple] = None  # norms behind the branches: (branch output, its norm) still to be added to x
+    only: Optional[int] = None       # last layer: the one row that is read behind it, or NO_ROW; None: every row
+
+    def leaves(self, width: int, *rows) -> Optional[list]:
+        """The (buffer, bytes a row) of `rows` as the rest of the layer reads them: from here on the pass is the wanted row alone.  The other
+        rows of a prompt have left what they leave for later tokens -- keys, values, states -- and nothing reads their stream behind the
+        last layer.  None where no row is wanted; all rows where one does not begin at 16 bytes, as a single row's kernels read it."""
+        if self.only is not None and self.only != NO_ROW and any(n % 16 for n in [width * 4] + [n for _, n in rows]):
+            self.only = None
+        if self.only is None:
+            return [b for b, _ in rows]
+        if self.only == NO_ROW:
+            return None
+        row, self.only, self.rows = self.only, None, 1
+        self.x = self.x.view(row * width * 4, width * 4)
+        return [b.view(row * n, n) for b, n in rows]
 
     @property
     def size(self) -> int:
@@ -196,11 +212,13 @@ class SoftmaxAttention:
         q = r.scratch("q", r.rows * s.heads * s.maps * self.dq)
         outputs = [q, memory.keys, memory.values]
         norm.project(r, self.qkv, outputs, r.dtype)
+        if r.only == NO_ROW:
+            return
         mixed = r.scratch("mixed", r.rows * s.heads * s.vdim)
         r.kernels.attention_rows_into(r.batch, q, memory.keys, memory.values, mixed, r.dtype, r.position, r.max_position, r.rows,
                                       s.heads, s.kv_heads, s.maps, s.dim, s.vdim, memory.capacity, s.scale, self.lam,
                                       self.out_scale, self.eps)
-        norm.finish(r, self.out, mixed, r.dtype)
+        norm.finish(r, self.out, *r.leaves(norm.dim, (mixed, s.heads * s.vdim * r.size)), r.dtype)
 
 
 # ---- latent attention ---------------------------------------------------------------------------------------------------
@@ -255,6 +273,8 @@ class LatentAttention:
     def run(self, r: Run, norm: Norm, memory: LatentCache) -> None:
         s, K, b, n = self.spec, r.kernels, r.batch, r.rows
         H, expanded = s.heads, n >= EXPANDED_MIN_ROWS
+        if r.only == NO_ROW and self.source is not None:      # it leaves nothing of its own
+            return
         q_rot, gate = r.scratch("latent.rot", n * H * s.rot_dim, f32=True), r.scratch("latent.gate", n * H, f32=True)
         down = r.scratch("latent.down", n * (s.kv_rank + s.rot_dim), f32=True) if self.source is None else None
         q = r.scratch("q", n * H * (self.dq if expanded else s.dim))
@@ -263,6 +283,8 @@ class LatentAttention:
         if expanded:
             K.latent_prepare_into(b, q_rot, down, self.latent_norm, self.frequencies, r.position, q, r.dtype, memory.rows, r.dtype, n, H,
                                   s.kv_rank, s.rot_dim, self.dq, s.dim, s.dim, memory.capacity, self.eps)
+            if r.only == NO_ROW:
+                return
             positions = (r.max_position + n + 31) // 32 * 32
             keys, values = r.scratch("latent.keys", positions * H * self.dq), r.scratch("latent.values", positions * H * self.dv)
             K.latent_expand_into(b, memory.rows, r.dtype, self.up, keys, values, positions, H, s.dim, s.rot_dim, s.vdim, s.kv_rank)
@@ -272,10 +294,12 @@ class LatentAttention:
             ql = r.scratch("latent.q", n * H * self.row, f32=True)
             K.latent_queries_into(b, q, self.key_up, q_rot, down, self.latent_norm, self.frequencies, r.position, ql, memory.rows, r.dtype,
                                   n, H, s.dim, s.kv_rank, s.rot_dim, memory.capacity, self.eps)
+            if r.only == NO_ROW:
+                return
             ol = r.scratch("latent.out", n * H * s.kv_rank)
             K.latent_attention_values_into(b, ql, memory.rows, ol, r.dtype, r.position, r.max_position, n, H, s.kv_rank, s.rot_dim,
                                            memory.capacity, s.scale, self.sink, gate, self.value_up, s.vdim, mixed)
-        norm.finish(r, self.out, mixed, r.dtype)
+        norm.finish(r, self.out, *r.leaves(norm.dim, (mixed, H * s.vdim * r.size)), r.dtype)
 
 
 # ---- linear attention with a fixed decay per head -----------------------------------------------------------------------
@@ -295,6 +319,10 @@ def finish_gated(r: Run, norm: Norm, out: StackedLinear, o: Buffer, gate: Buffer
                  act: int, gate_first: bool) -> None:
     """Norm in parts of `group` values and gate of o (f32), then the branch's last product."""
     K, b, k = r.kernels, r.batch, out.k
+    wanted = r.leaves(norm.dim, (o, k * 4), (gate, k * (4 if gate_dtype == F32 else 2)))
+    if wanted is None:
+        return
+    o, gate = wanted
     if r.rows == 1 and k <= GATED_IN_PRODUCT and K.gated_vector_fits(k, group):
         dest, add = norm.destination(r)
         K.linear_gated_vector_into(b, o, gate, gate_dtype, weight, eps, out.weight, None, k, out.segments, [dest], F32, add, None, group,
@@ -507,7 +535,7 @@ class PreNormLayer:
 
     def run(self, r: Run, memory) -> None:
         self.mixer.run(r, self.norm1, memory)
-        if self.ff is not None:
+        if self.ff is not None and r.only != NO_ROW:
             self.ff.run(r, self.norm2)
 
 

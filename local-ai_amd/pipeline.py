@@ -328,6 +328,18 @@ class DecodePipeline:
     def forward_tokens_batch(self, tokens, start_pos: int, ple_tokens=None, batch=None) -> bool:
         """pipeline.rs:969-1100: one prefill chunk, rows at positions start_pos .. start_pos + len(tokens), through every
         layer's batch path into the single-sequence caches.  Returns True when the result is in batch_scratch.hidden_a."""
+        return self._forward_rows(tokens, start_pos, ple_tokens, batch, len(self.layers), False)
+
+    def fill_caches_batch(self, tokens, start_pos: int, ple_tokens=None, batch=None) -> None:
+        """``forward_tokens_batch`` for what it leaves in the caches: it ends at the keys and values of the last layer that has any.  What the
+        rows would be behind that, in layers that read another's cache and in the last one's attention and feed-forward, nothing reads:
+        the token behind a prompt's chunks meets the chunks in the caches alone.  (256 rows at 16000 and a token, five of ten layers with caches of
+        their own: 2139 us with everything, 1102 so.)"""
+        own = [i for i, layer in enumerate(self.layers) if layer.owns_cache()]
+        self._forward_rows(tokens, start_pos, ple_tokens, batch, own[-1] + 1 if own else 0, True)
+
+    def _forward_rows(self, tokens, start_pos: int, ple_tokens, batch, n_layers: int, cache_only: bool) -> bool:
+        """The first `n_layers` layers, the last of them only as far as its cache where `cache_only`."""
         n = len(tokens)
         ple_tokens = tokens if ple_tokens is None else ple_tokens
         if len(ple_tokens) != n:
@@ -341,11 +353,11 @@ class DecodePipeline:
         bs = self.batch_scratch
         ple_arg = (bs.ple_all, self.config.num_hidden_layers) if self._embed_rows(batch, tokens, ple_tokens) else None
         cur_in_a, prenormed = True, False
-        for i, layer in enumerate(self.layers):
+        for i, layer in enumerate(self.layers[:n_layers]):
             inp, out = (bs.hidden_a, bs.hidden_b) if cur_in_a else (bs.hidden_b, bs.hidden_a)
             next_norm = self._next_norm(i)
-            layer.forward_batch(self.kernels, batch, n, start_pos, inp, out, bs, self.scratch.ones,
-                                self.kv_caches[self.kv_index_map[i]], ple_arg, prenormed, next_norm)
+            layer.forward_batch(self.kernels, batch, n, start_pos, inp, out, bs, self.scratch.ones, self.kv_caches[self.kv_index_map[i]],
+                                ple_arg, prenormed, next_norm, cache_only and i == n_layers - 1)
             cur_in_a, prenormed = not cur_in_a, next_norm is not None
         if own:
             batch.commit_and_wait()
@@ -361,7 +373,7 @@ class DecodePipeline:
         pos = 0
         while pos < last_idx:
             chunk = tokens[pos:min(pos + chunk_len, last_idx)]
-            self.forward_tokens_batch(chunk, pos)
+            self.fill_caches_batch(chunk, pos)
             pos += len(chunk)
         self.position = last_idx
         return self.forward_token(tokens[last_idx], last_idx)

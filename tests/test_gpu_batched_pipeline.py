@@ -210,3 +210,27 @@ def test_batched_step_arguments(pkg, gpu):
         pipe.prefill_lane(state, 0, [1] * 601)
     with pytest.raises(pkg.InvalidArgument):
         pipe.forward_tokens_batch([1] * 9, 0)
+
+
+@pytest.mark.parametrize("shared,pld,options", [(3, 64, {}), (0, 64, {}), (3, 0, {"fuse_norm_chain": False}), (0, 0, {"fuse_prologues": False}), (3, 64, {"group_projections": False})])
+def test_a_chunk_for_the_caches_leaves_what_a_whole_one_does(pkg, gpu, shared, pld, options):
+    """It ends at the keys and values of the last layer that has any: the same bytes in every cache, the same token behind them."""
+    ctx, K = gpu
+    cfg = _config(pkg, pld)
+    cfg.num_kv_shared_layers = shared
+    g = pkg.synth.rng(17, shared + pld)
+    pipe = pkg.pipeline.DecodePipeline.from_host(ctx, K, cfg, pkg.synth.decode_model_tensors(cfg, g, [512, 512, 512, 1024, 1024, 1024]), 1024, max_batch=64, **options)
+    assert len(pipe.kv_caches) == 6 - shared
+    tokens, out = [int(v) for v in g.integers(0, cfg.vocab_size, 90)], []
+    for run in (pipe.forward_tokens_batch, pipe.fill_caches_batch):
+        pipe.reset()
+        for lo, hi in ((0, 19), (19, 20), (20, 84), (84, 89)):
+            run(tokens[lo:hi], lo)
+        pipe.write_logits(pipe.forward_token(tokens[89], 89))
+        out.append([b.as_array(np.uint8, b.length()).copy() for c in pipe.kv_caches for b in (c.keys_q, c.key_norms, c.values_q, c.value_norms)] + [pipe.logits().copy()])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    with pytest.raises(pkg.InvalidArgument):
+        pipe.fill_caches_batch([1] * 65, 0)
+    with pytest.raises(pkg.InvalidArgument):
+        pipe.fill_caches_batch([1] * 5, 1020)

@@ -94,6 +94,25 @@ def test_prompt_portions_and_decoding_agree_with_the_plain_statement(ai, gpu, na
         check(feed(m, tokens, cuts), want, dtype, f"{name} {what}")
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", sorted(CONFIGS))
+def test_portions_of_which_one_row_or_none_is_wanted(ai, gpu, name, dtype):
+    """Their last layer ends early for the other rows; what those leave for the tokens behind them is all there."""
+    cfg, w, m = build(ai, gpu, name, dtype, max_rows=80)           # the longest portion takes two passes
+    tokens = [int(t) for t in np.random.default_rng(15).integers(0, cfg["vocab"], 301)]
+    want = O.forward(cfg, w, tokens)
+    for wanted in (lambda c: [c - 1], lambda c: [], lambda c: [c // 2], lambda c: [0]):
+        s, at, got, where = m.new_sequence(), 0, [], []
+        for c in [70, 2, 100, 17, 1, 1, 1, 66, 3, 40]:
+            p = wanted(c) if c > 1 else [0]
+            got.append(m.step(s, tokens[at:at + c], p))
+            where += [at + i for i in p]
+            at += c
+        assert at == len(tokens)
+        m.end_sequence(s)
+        check(np.concatenate(got), want[where], dtype, f"{name} {wanted(10)}")
+
+
 @pytest.mark.parametrize("name", ["both", "loop_all", "latent_and_states", "latent_shared"])
 def test_residual_stream_after_every_layer_run(ai, gpu, name):
     cfg, w, m = build(ai, gpu, name)
