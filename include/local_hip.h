@@ -619,6 +619,20 @@ LH_API int lh_flash_attention_tq_rotated_lazy_into(lh_batch* batch, const lh_buf
                                                    uint32_t head_dim, uint32_t kv_len, uint32_t current_pos,
                                                    uint32_t num_q_heads, uint32_t num_kv_heads, uint32_t window,
                                                    uint32_t bits, uint32_t ring_capacity, int* rotated);
+/* lh_decode_qkv_prepare_into and lh_flash_attention_tq_rotated_lazy_into (with `rotated` NULL: _rotated_into) of a decoded
+ * token at `position` as one step, which is one launch where the span is short (a sliding window): the heads are
+ * taken from q_raw / k_raw / v_raw and left behind norm and rotary embedding in q / k / v (the same buffers, or NULL for
+ * the raw ones: prepared in place, in a launch of its own).  k = v = NULL for a layer that shares another's cache.  `rq`
+ * holds the rotated query only where the preparation was a launch of its own.  Codes, norms and prepared rows are
+ * those of the separate steps, the heads theirs to within their rounding. */
+LH_API int lh_token_attention_tq_into(lh_batch* batch, const lh_buffer* q_raw, const lh_buffer* k_raw, const lh_buffer* v_raw,
+                                      lh_buffer* q, lh_buffer* k, lh_buffer* v, const lh_buffer* q_norm,
+                                      const lh_buffer* k_norm, const lh_buffer* levels, const lh_buffer* signs,
+                                      lh_buffer* rq, lh_buffer* k_codes, lh_buffer* k_norms, lh_buffer* v_codes,
+                                      lh_buffer* v_norms, lh_buffer* out, lh_buffer* out_f16, uint32_t head_dim,
+                                      uint32_t num_q_heads, uint32_t num_kv_heads, float eps, uint32_t position,
+                                      float theta, float partial_rotary_factor, uint32_t window, uint32_t bits,
+                                      uint32_t ring_capacity, int* rotated);
 LH_API int lh_flash_attention_tq_batched_rotated_into(lh_batch* batch, const lh_buffer* rq, const lh_buffer* k_codes,
                                                       const lh_buffer* k_norms, const lh_buffer* v_codes,
                                                       const lh_buffer* v_norms, const lh_buffer* levels,

@@ -801,6 +801,23 @@ class Kernels:
                                                                _u32(bits), _u32(ring_capacity), C.byref(rotated)))
         return bool(rotated.value)
 
+    def token_attention_tq_into(self, batch, raw, q, k, v, q_norm, k_norm, levels, signs, rq, k_codes, k_norms, v_codes, v_norms, out,
+                                out_f16, head_dim, num_q_heads, num_kv_heads, eps, position, theta, partial_rotary_factor, window, bits,
+                                ring_capacity, lazy) -> bool:
+        """``decode_qkv_prepare_into`` and ``flash_attention_tq_rotated_into`` (``lazy``: ``_rotated_lazy_into``) of one decoded token,
+        as one launch where its span is short.  ``raw``: the (q, k, v) rows to prepare into q, k, v; k = v = None for a layer that reads
+        another's cache.  True: ``out_f16`` holds the rotated heads."""
+        def h(b):
+            return b._h if b is not None else None
+        rotated = C.c_int(0)
+        kv = k is not None
+        _check(self._l.lh_token_attention_tq_into(batch._h, raw[0]._h, h(raw[1] if kv else None), h(raw[2] if kv else None), q._h, h(k), h(v), h(q_norm),
+                                                  h(k_norm), levels._h, signs._h, rq._h, k_codes._h, k_norms._h, v_codes._h, v_norms._h, out._h,
+                                                  out_f16._h, _u32(head_dim), _u32(num_q_heads), _u32(num_kv_heads), C.c_float(eps), _u32(position),
+                                                  C.c_float(theta), C.c_float(partial_rotary_factor), _u32(window), _u32(bits), _u32(ring_capacity),
+                                                  C.byref(rotated) if lazy else None))
+        return bool(rotated.value) or not lazy
+
     def flash_attention_tq_batched_rotated_into(self, batch, rq, k_codes, k_norms, v_codes, v_norms, levels, signs, out,
                                                 out_f16, positions, head_dim, lane_capacity, num_q_heads, num_kv_heads,
                                                 window, bits, n_lanes, ring_capacity):

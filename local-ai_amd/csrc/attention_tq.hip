@@ -405,10 +405,41 @@ struct RotateBack {
     int* rotated = nullptr;
 };
 
+// What comes ahead of the attention and may ride in its launch: the queries' (keys', values') preparation.
+struct Preparation {
+    const LhPrepareRows& rows;
+    const float* partial;               // as lh_prepare_rows_launch takes them
+    uint32_t splits, part_cols;
+};
+
+bool apart(const lh_buffer* raw, const lh_buffer* out, size_t bytes) {
+    return raw && out && ((uintptr_t)raw->ptr + bytes <= (uintptr_t)out->ptr || (uintptr_t)out->ptr + bytes <= (uintptr_t)raw->ptr);
+}
+
+// The preparation as attention_tq_token_kernel takes it; false: it has to run by itself.
+bool token_preparation(const lh_context* ctx, const AttnParams& p, const AttnPointers& ptrs, const Preparation& prep, uint64_t max_span, TokenPrep& t) {
+    const LhPrepareRows& a = prep.rows;
+    const bool kv = a.k && a.v && a.n_kv_heads != 0;
+    const auto ptr = [](const lh_buffer* b) { return b ? (uint16_t*)b->ptr : nullptr; };
+    t = TokenPrep{ptr(a.q_raw), kv ? ptr(a.k_raw) : nullptr, kv ? ptr(a.v_raw) : nullptr, prep.partial, prep.splits, a.rows, prep.part_cols, ptr(a.q), kv ? ptr(a.k) : nullptr,
+                  kv ? ptr(a.v) : nullptr, ptr(a.q_norm), kv ? ptr(a.k_norm) : nullptr, (const float*)a.signs->ptr, kv ? (uint8_t*)a.k_codes->ptr : nullptr,
+                  kv ? (uint8_t*)a.v_codes->ptr : nullptr, kv ? ptr(a.k_norms) : nullptr, kv ? ptr(a.v_norms) : nullptr, a.eps, a.theta, a.partial_rotary_factor,
+                  1.0f / std::sqrt((float)p.head_dim)};
+    if (p.mode == kPrefill || p.head_dim != a.head_dim || p.num_q_heads != a.n_q_heads || (kv && p.num_kv_heads != a.n_kv_heads) || p.num_queries != a.rows) return false;
+    // Every workgroup of a query reads its raw rows while the first one stores the prepared ones.
+    const size_t q_bytes = (size_t)a.rows * a.n_q_heads * a.head_dim * 2, kv_bytes = (size_t)a.rows * a.n_kv_heads * a.head_dim * 2;
+    if (!prep.partial) {
+        const std::pair<const lh_buffer*, size_t> in[3] = {{a.q_raw, q_bytes}, {a.k_raw, kv_bytes}, {a.v_raw, kv_bytes}}, out[3] = {{a.q, q_bytes}, {a.k, kv_bytes}, {a.v, kv_bytes}};
+        for (int i = 0; i < (kv ? 3 : 1); i++)
+            for (int o = 0; o < (kv ? 3 : 1); o++) if (!apart(in[i].first, out[o].first, std::max(in[i].second, out[o].second))) return false;
+    }
+    return max_span != 0 && mfma_supported(p, ptrs) && token_supported(ctx, p, t, max_span);
+}
+
 int attention_dispatch(lh_batch* batch, const char* op, const lh_buffer* rq, const lh_buffer* k_codes, const lh_buffer* k_norms,
                        const lh_buffer* v_codes, const lh_buffer* v_norms, const lh_buffer* levels, lh_buffer* out,
                        const lh_buffer* positions, AttnParams p, uint64_t max_span, uint64_t phys_slots, const RotateBack* rot = nullptr,
-                       float* ws_override = nullptr, size_t ws_override_floats = 0) {
+                       float* ws_override = nullptr, size_t ws_override_floats = 0, const Preparation* prep = nullptr) {
     if (!batch) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: batch is null", op);
     if (p.bits < 2 || p.bits > 4) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: TurboQuant bits must be 2..=4, got %u", op, p.bits);
     if (p.head_dim == 0 || (p.head_dim & (p.head_dim - 1)) || p.head_dim > 512)
@@ -438,6 +469,12 @@ int attention_dispatch(lh_batch* batch, const char* op, const lh_buffer* rq, con
     const AttnPointers ptrs{(const float*)rq->ptr, (const uint8_t*)k_codes->ptr, (const uint16_t*)k_norms->ptr,
                             (const uint8_t*)v_codes->ptr, (const uint16_t*)v_norms->ptr, (const float*)levels->ptr,
                             positions ? (const uint32_t*)positions->ptr : nullptr, (float*)out->ptr, ws, ctx->fault_dev};
+    TokenPrep token{};
+    const bool in_one = prep && token_preparation(ctx, p, ptrs, *prep, max_span, token);
+    if (prep && !in_one) {
+        const int rp = lh_prepare_rows_launch(batch, prep->rows, prep->partial, prep->splits, prep->part_cols);
+        if (rp != LH_OK) return rp;
+    }
     // Prefill entries with more than one row.  Sixteen rows sharing a pass over the codes (the tiled kernel) pay when there
     // is enough work to keep its eight-wave workgroups busy: measured against one query row per workgroup it wins from about
     // 1.5 M (row, position) pairs on (256 rows over 8k positions: 50 against 60 us; over 32k: 118 against 192) and loses
@@ -446,7 +483,10 @@ int attention_dispatch(lh_batch* batch, const char* op, const lh_buffer* rq, con
     // form for every launch it supports (each is validated against the oracle that way).
     static const int prefill_env = [] { const char* e = getenv("LOCAL_HIP_ATTN_PREFILL"); return !e ? 0 : e[0] == 'r' ? 1 : e[0] == 't' ? 2 : 0; }();
     const bool tiled_pays = (uint64_t)p.num_queries * max_span >= 1500000ull;
-    if (max_span != 0 && prefill_env != 1 && (prefill_env == 2 || tiled_pays) && prefill_tile_supported(p, ptrs)) {
+    if (in_one) {
+        const int rl = launch_token(ctx, op, ptrs, p, token, max_span);
+        if (rl != LH_OK) return rl;
+    } else if (max_span != 0 && prefill_env != 1 && (prefill_env == 2 || tiled_pays) && prefill_tile_supported(p, ptrs)) {
         const int rl = launch_prefill_tile(ctx, op, ptrs, p, max_span, ws_avail);
         if (rl != LH_OK) return rl;
     } else if (max_span == 0 || !mfma_supported(p, ptrs)) {
@@ -596,6 +636,29 @@ int lh_flash_attention_tq_rotated_lazy_into(lh_batch* batch, const lh_buffer* rq
     RotateBack rot{signs, out_f16};
     rot.rotated = rotated;
     return attention_dispatch(batch, "flash_attention_tq_rotated_lazy", rq, k_codes, k_norms, v_codes, v_norms, levels, out, nullptr, p, span, phys, &rot);
+}
+
+int lh_token_attention_tq_into(lh_batch* batch, const lh_buffer* q_raw, const lh_buffer* k_raw, const lh_buffer* v_raw, lh_buffer* q, lh_buffer* k, lh_buffer* v,
+                               const lh_buffer* q_norm, const lh_buffer* k_norm, const lh_buffer* levels, const lh_buffer* signs, lh_buffer* rq, lh_buffer* k_codes,
+                               lh_buffer* k_norms, lh_buffer* v_codes, lh_buffer* v_norms, lh_buffer* out, lh_buffer* out_f16, uint32_t head_dim, uint32_t num_q_heads,
+                               uint32_t num_kv_heads, float eps, uint32_t position, float theta, float partial_rotary_factor, uint32_t window, uint32_t bits,
+                               uint32_t ring_capacity, int* rotated) {
+    if (rotated) *rotated = 0;
+    const bool kv = k != nullptr && v != nullptr;
+    LhPrepareRows a{q, kv ? k : nullptr, kv ? v : nullptr, q_norm, kv ? k_norm : nullptr, levels, signs, rq, kv ? k_codes : nullptr, kv ? k_norms : nullptr, kv ? v_codes : nullptr,
+                    kv ? v_norms : nullptr, nullptr, head_dim, num_q_heads, kv ? num_kv_heads : 0u, 1, eps, position, theta, partial_rotary_factor, bits, ring_capacity, 0};
+    a.q_raw = q_raw; a.k_raw = kv ? k_raw : nullptr; a.v_raw = kv ? v_raw : nullptr;
+    int r = lh_prepare_rows_launch(batch, a, nullptr, 0, 0, true);          // its arguments, before anything is launched
+    if (r != LH_OK) return r;
+    AttnParams p{};
+    p.head_dim = head_dim; p.bits = bits; p.num_q_heads = num_q_heads; p.num_kv_heads = num_kv_heads; p.kv_len = position + 1;
+    p.pos0 = position; p.window = window; p.ring_capacity = ring_capacity; p.mode = kSingle; p.num_queries = 1;
+    const uint64_t seq = (uint64_t)position + 1, lo = (window > 0 && seq > window) ? seq - window : 0;
+    const uint64_t phys = (ring_capacity ? std::min<uint64_t>(ring_capacity, seq) : seq) * num_kv_heads;
+    RotateBack rot{signs, out_f16};
+    rot.rotated = rotated;
+    const Preparation prep{a, nullptr, 0, 0};
+    return attention_dispatch(batch, "token_attention_tq", rq, k_codes, k_norms, v_codes, v_norms, levels, out, nullptr, p, seq - lo, phys, &rot, nullptr, 0, &prep);
 }
 
 static int prefill_common(const char* op, lh_batch* batch, const lh_buffer* rq, const lh_buffer* k_codes, const lh_buffer* k_norms,

@@ -59,6 +59,24 @@ int launch_mfma(lh_context* ctx, const char* op, const AttnPointers& a, AttnPara
 bool short_supported(const lh_context* ctx, const AttnParams& p, uint64_t max_span);
 int launch_short(lh_context* ctx, const char* op, const AttnPointers& a, AttnParams& p, uint64_t max_span);
 
+// A query whose preparation rides in the same launch: what decode_qkv_prepare_kernel does for it (turboquant_kv.hip), on heads that lie as
+// raw f16 rows ([query][head][256], apart from where the prepared ones go) or as the f32 partial tiles of a k-split product.
+struct TokenPrep {
+    const uint16_t *q, *k, *v;           // raw rows
+    const float* partial;                // [splits][rows][part_cols], the query, key and value heads side by side; null: the rows above
+    uint32_t splits, rows, part_cols;
+    uint16_t *q_out, *k_out, *v_out;     // the heads as f16 behind norm and rotary embedding
+    const uint16_t *q_norm, *k_norm;     // may be null
+    const float* signs;
+    uint8_t *k_codes, *v_codes;          // null: the query alone, on a cache that has the position already
+    uint16_t *k_norms, *v_norms;
+    float eps, theta, prf, inv_sqrt_d;
+};
+// What short_supported takes, with room for the two waves that bring in the query's own key and value, on a cache where that position's slot is
+// no other's of the span.
+bool token_supported(const lh_context* ctx, const AttnParams& p, const TokenPrep& t, uint64_t max_span);
+int launch_token(lh_context* ctx, const char* op, const AttnPointers& a, AttnParams& p, const TokenPrep& t, uint64_t max_span);
+
 // The tiled prefill kernel (attention_tq_prefill_tile.hip): sixteen query rows per workgroup share one pass over the codes,
 // K and V levels as f16 through LDS, any level table.  Takes 2-bit codes, head_dim 256, at most 8 query heads per KV head,
 // ring absent or a multiple of 64 slots, two rows or more.

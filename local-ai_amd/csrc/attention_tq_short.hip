@@ -34,7 +34,8 @@ __device__ __forceinline__ u32x4_t ld16(const uint8_t* p) {
 }
 
 struct ShortShared {
-    float q[4][kHeads][72];              // by field, head and code byte (a row in 72: a quarter wave's 16-byte reads on distinct banks)
+    float queries[4][kHeads * 72 + 16];  // by field, head and code byte (a row in 72: a quarter wave's 16-byte reads on distinct banks; 16 more: the fields of a byte too)
+    __device__ __forceinline__ float& q(uint32_t field, uint32_t head, uint32_t byte) { return queries[field][head * 72 + byte]; }
     uint8_t rqop[12][64][16];            // score operands per (plane, field) and lane
     float maxabs[kHeads], sum[kHeads];
     float fin_r[kMaxWaves][kHeads], fin_l[kMaxWaves][kHeads];
@@ -55,8 +56,8 @@ struct Group { u32x4_t k[4], v[4 / S]; uint32_t nk, nv; uint32_t lo, hi; };
 
 template <int NPL, int S, class Load>
 __device__ __forceinline__ void short_body(const AttnPointers& a, const AttnParams& p, ShortShared& sh, ShortWave<S>& mine, Group<S> gr, uint32_t G, uint32_t g_last, Load load,
-                                           float alpha, float beta, float gam, float delta, uint32_t qi, uint32_t kvh, uint32_t group) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6, pcol = lane & 15, g = lane >> 4;
+                                           float alpha, float beta, float gam, float delta, uint32_t qi, uint32_t kvh, uint32_t group, uint32_t nwaves, uint32_t parts) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), pcol = lane & 15, g = lane >> 4;
     constexpr int E = 4 / S;              // chunks of 16 code bytes, 64 dims
     const float cmax = fmaxf(fmaxf(fabsf(beta), fabsf(0.5f * gam)), NPL == 3 ? fabsf(delta) : 0.0f), inv_cmax = cmax > 0.0f ? 1.0f / cmax : 0.0f;
 
@@ -71,7 +72,7 @@ __device__ __forceinline__ void short_body(const AttnPointers& a, const AttnPara
             uint32_t w[4];
 #pragma unroll
             for (int mm = 0; mm < 2; mm++) {                  // word 2 mm + limb
-                const float4 x = *reinterpret_cast<const float4*>(&sh.q[f][h][16 * g + 4 * (2 * mm + limb)]);
+                const float4 x = *reinterpret_cast<const float4*>(&sh.q(f, h, 16 * g + 4 * (2 * mm + limb)));
                 const float xs[4] = {x.x, x.y, x.z, x.w};
                 uint32_t lo = 0u, hi = 0u;
 #pragma unroll
@@ -257,14 +258,22 @@ __device__ __forceinline__ void short_body(const AttnPointers& a, const AttnPara
     }
     lh_lds_barrier();
     if (wave >= group) return;
-    const float r = lane < nwaves ? sh.fin_r[lane][wave] : -INFINITY, top = lh_group_max(r, 16);
-    const float f = r == -INFINITY ? 0.0f : exp2f(r - top), l = lh_group_sum(lane < nwaves ? f * sh.fin_l[lane][wave] : 0.0f, 16);
+    const float r = lane < parts ? sh.fin_r[lane][wave] : -INFINITY, top = lh_group_max(r, 16);
+    const float f = r == -INFINITY ? 0.0f : exp2f(r - top), l = lh_group_sum(lane < parts ? f * sh.fin_l[lane][wave] : 0.0f, 16);
     const ShortWave<S>* const all = &mine - wave;
     float o[E] = {};
-    for (uint32_t w = 0; w < nwaves; w++) {
-        const float fw = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(f), (int)w));
+    for (uint32_t w0 = 0; w0 < parts; w0 += 4) {                // (one at a time each is a trip to LDS; past the last: its values, with weight 0)
+        float x[4][E];
 #pragma unroll
-        for (int e = 0; e < E; e++) o[e] = __builtin_fmaf(fw, all[w].park[wave][64 * e + lane], o[e]);
+        for (uint32_t u = 0; u < 4; u++)
+#pragma unroll
+            for (int e = 0; e < E; e++) x[u][e] = all[std::min(w0 + u, parts - 1)].park[wave][64 * e + lane];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) {
+            const float fw = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(f), (int)(w0 + u)));
+#pragma unroll
+            for (int e = 0; e < E; e++) o[e] = __builtin_fmaf(fw, x[u][e], o[e]);
+        }
     }
     const float total = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(l)));
     float* const dst = a.out + ((size_t)qi * p.num_q_heads + kvh * group + wave) * kDim + kDim / S * blockIdx.x + lane;
@@ -272,58 +281,310 @@ __device__ __forceinline__ void short_body(const AttnPointers& a, const AttnPara
     for (int e = 0; e < E; e++) dst[64 * e] = total > 0.0f ? o[e] / total : 0.0f;
 }
 
+// The codes and norms of group G_ of positions [lo, hi).  Lanes whose position is not visible read one that is: nothing of it is used (its weight is zero).
+template <int S>
+__device__ __forceinline__ Group<S> load_group(const AttnPointers& a, const AttnParams& p, uint32_t G_, uint32_t lo, uint32_t hi, uint32_t lane_base, uint32_t kv_heads, uint32_t kvh) {
+    Group<S> r;
+    const uint32_t stride = kv_heads * 64;
+    uint32_t at_lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(at_lane));                           // (a second group's addresses are not to wait in registers for the rare loop that needs them)
+    const uint32_t start = G_ << 6, base = lane_base + (p.ring_capacity ? start % p.ring_capacity : start);
+    r.lo = lo > start ? lo - start : 0u;
+    r.hi = std::min(hi - start, kGroup);
+    auto at = [&](uint32_t i) { return (size_t)(base + std::min(std::max(i, r.lo), r.hi - 1)); };
+#pragma unroll
+    for (int q = 0; q < 4; q++) r.k[q] = ld16(a.k_codes + at(16 * q + (at_lane & 15)) * stride + kvh * 64 + 16 * (at_lane >> 4));
+    r.nk = a.k_norms[at(at_lane) * kv_heads + kvh];
+    r.nv = a.v_norms[at(at_lane) * kv_heads + kvh];
+#pragma unroll
+    for (int e = 0; e < 4 / S; e++) r.v[e] = ld16(a.v_codes + at(at_lane) * stride + kvh * 64 + 16 * (4 / S * blockIdx.x + e));
+    return r;
+}
+
+// L[c] = alpha + beta bit0 + gam bit1 + delta bit0 bit1: as in attention_tq_mfma_kernel
+template <int S, class Load>
+__device__ __forceinline__ void short_by_levels(const AttnPointers& a, const AttnParams& p, ShortShared& sh, ShortWave<S>& mine, const Group<S>& first, uint32_t begin, uint32_t end, Load load,
+                                                float L0, float L1, float L2, float L3, uint32_t qi, uint32_t kvh, uint32_t group, uint32_t nwaves, uint32_t parts) {
+    const float d_raw = (L3 - L2) - (L1 - L0), lmax = fmaxf(fmaxf(fabsf(L0), fabsf(L1)), fmaxf(fabsf(L2), fabsf(L3))), l_mean = 0.25f * ((L0 + L3) + (L1 + L2));
+    if (fabsf(d_raw) > 1e-5f * lmax || fabsf(l_mean) > 1e-6f * lmax) short_body<3, S>(a, p, sh, mine, first, begin, end, load, L0, L1 - L0, L2 - L0, d_raw, qi, kvh, group, nwaves, parts);
+    else short_body<2, S>(a, p, sh, mine, first, begin, end, load, L0 - 0.25f * d_raw, (L1 - L0) + 0.5f * d_raw, (L2 - L0) + 0.5f * d_raw, 0.0f, qi, kvh, group, nwaves, parts);
+}
+
+__device__ __forceinline__ float level_of(float table, int i) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(table), i)); }
+
 // The leading arguments arrive in registers with the wave (see the Makefile); the structures repeat them.
 template <int S>
 __global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_short_kernel(const float* queries, const float* levels, uint32_t q_heads, uint32_t kv_heads, const AttnPointers a,
                                                                             const AttnParams p) {
     extern __shared__ __align__(16) uint8_t lds[];
     ShortShared& sh = *reinterpret_cast<ShortShared*>(lds);
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
     ShortWave<S>& mine = reinterpret_cast<ShortWave<S>*>(lds + sizeof(ShortShared))[wave];
     uint32_t qi = blockIdx.y, kvh = 0, group = q_heads;
     if (kv_heads != 1) { qi = blockIdx.y / kv_heads; kvh = blockIdx.y - qi * kv_heads; group = q_heads / kv_heads; }
     // ---- a wave has a head of the query
     float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
     if (wave < group) x = reinterpret_cast<const float4*>(queries + ((size_t)qi * q_heads + kvh * group + wave) * kDim)[lane];
-    const float L0 = levels[0], L1 = levels[1], L2 = levels[2], L3 = levels[3];
+    const float table = levels[lane & 3];                       // (as a scalar load every argument behind it would wait for it)
 
-    // ---- the codes and norms of a group.  Lanes whose position is not visible read one that is: nothing of it is used (its weight is zero).
     uint32_t lo, hi, lane_base;
     query_range(p, a.positions, qi, lo, hi, lane_base);
-    const uint32_t stride = kv_heads * 64, G = (lo >> 6) + wave, g_last = hi > lo ? (hi - 1) >> 6 : 0u;
+    const uint32_t G = (lo >> 6) + wave, g_last = hi > lo ? (hi - 1) >> 6 : 0u;
     const bool none = hi <= lo;
-    auto load = [&](uint32_t G_) {
-        Group<S> r;
-        uint32_t at_lane = lane;
-        asm volatile("" : "+v"(at_lane));                       // (a second group's addresses are not to wait in registers for the rare loop that needs them)
-        const uint32_t start = G_ << 6, base = lane_base + (p.ring_capacity ? start % p.ring_capacity : start);
-        r.lo = lo > start ? lo - start : 0u;
-        r.hi = std::min(hi - start, kGroup);
-        auto at = [&](uint32_t i) { return (size_t)(base + std::min(std::max(i, r.lo), r.hi - 1)); };
-#pragma unroll
-        for (int q = 0; q < 4; q++) r.k[q] = ld16(a.k_codes + at(16 * q + (at_lane & 15)) * stride + kvh * 64 + 16 * (at_lane >> 4));
-        r.nk = a.k_norms[at(at_lane) * kv_heads + kvh];
-        r.nv = a.v_norms[at(at_lane) * kv_heads + kvh];
-#pragma unroll
-        for (int e = 0; e < 4 / S; e++) r.v[e] = ld16(a.v_codes + at(at_lane) * stride + kvh * 64 + 16 * (4 / S * blockIdx.x + e));
-        return r;
-    };
+    auto load = [&](uint32_t G_) { return load_group<S>(a, p, G_, lo, hi, lane_base, kv_heads, kvh); };
     Group<S> first{};
     if (!none && G <= g_last) first = load(G);
 
     // ---- per head: max |q| (quantisation scale) and sum (constant term of the level table)
     if (wave < kHeads) {
-        sh.q[0][wave][lane] = x.x; sh.q[1][wave][lane] = x.y; sh.q[2][wave][lane] = x.z; sh.q[3][wave][lane] = x.w;
+        sh.q(0, wave, lane) = x.x; sh.q(1, wave, lane) = x.y; sh.q(2, wave, lane) = x.z; sh.q(3, wave, lane) = x.w;
         const float m = lh_group_max(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))), 64), s = lh_group_sum((x.x + x.y) + (x.z + x.w), 64);
         if (lane == 0) { sh.maxabs[wave] = m; sh.sum[wave] = s; }
     }
     lh_lds_barrier();
+    short_by_levels<S>(a, p, sh, mine, first, none ? 1u : G, none ? 0u : g_last, load, level_of(table, 0), level_of(table, 1), level_of(table, 2), level_of(table, 3), qi, kvh, group,
+                       nwaves, nwaves);
+}
 
-    // L[c] = alpha + beta bit0 + gam bit1 + delta bit0 bit1: as in attention_tq_mfma_kernel
-    const float d_raw = (L3 - L2) - (L1 - L0), lmax = fmaxf(fmaxf(fabsf(L0), fabsf(L1)), fmaxf(fabsf(L2), fabsf(L3))), l_mean = 0.25f * ((L0 + L3) + (L1 + L2));
-    const uint32_t end = none ? 0u : g_last, begin = none ? 1u : G;
-    if (fabsf(d_raw) > 1e-5f * lmax || fabsf(l_mean) > 1e-6f * lmax) short_body<3, S>(a, p, sh, mine, first, begin, end, load, L0, L1 - L0, L2 - L0, d_raw, qi, kvh, group);
-    else short_body<2, S>(a, p, sh, mine, first, begin, end, load, L0 - 0.25f * d_raw, (L1 - L0) + 0.5f * d_raw, (L2 - L0) + 0.5f * d_raw, 0.0f, qi, kvh, group);
+// ---- the query's own preparation in the same launch -------------------------------------------------------------------------------
+// A token's preparation (6.7 us; 5.0 without a key and a value) and its attention over a window (7.3) are two chains on a few CUs, one behind
+// the other, and each begins with a trip to memory.  In one launch 9.5 us (9.2), a token at 32768 positions with eight such layers 577 -> 547.  Here a workgroup prepares its query itself: the head that a wave stages it also norms,
+// turns and transforms, in registers (a lane has dims lane + 64 j: a rotary pair is one lane's, and so are the transform's last two
+// stages).  The position's own key and value need a chain of 256 dependent additions for their codes: two more waves walk it while
+// the others are at the groups before it, and leave their one position as a partial result of its own (its score, the value's levels,
+// weight 1) that the last step merges with the rest; they walk it between the others' barriers, and store behind the last one (with all of it behind
+// the score operands they were 1.6 us longer than the groups).  Every workgroup of a query repeats this; the first one also stores what the
+// preparation leaves: f16 heads, codes, norms.  Same operations in the same order as decode_qkv_prepare_kernel: the same bits.
+struct TokenShared {
+    float2 turn[kDim / 2];               // cosine and sine of a rotary pair
+    float square[2][kDim];
+};
+
+// One head in a wave: out[j] becomes the f16 value of dim lane + 64 j behind the norm (`normalise`).
+__device__ __forceinline__ void norm_head(uint16_t (&h)[4], const uint16_t (&w)[4], bool weighted, float eps) {
+    float s[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float x = lh_h2f(h[j]);
+        float sq = x * x;
+        asm volatile("" : "+v"(sq));                            // (rounded before it is added)
+        s[j] = lh_group_sum(sq, 64);
+    }
+    const float rms = rsqrtf((((0.0f + s[0]) + s[1]) + s[2] + s[3]) / (float)kDim + eps);
+#pragma unroll
+    for (int j = 0; j < 4; j++) h[j] = lh_f2h_exact(lh_norm_product(lh_h2f(h[j]), rms, weighted ? lh_h2f(w[j]) : 1.0f));
+}
+__device__ __forceinline__ void turn_head(uint16_t (&h)[4], const float2* turn, uint32_t angles, uint32_t lane) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        if (lane + 64 * j >= angles) continue;
+        const float2 t = turn[lane + 64 * j];
+        lh_rope_apply(lh_h2f(h[j]), lh_h2f(h[j + 2]), t.x, t.y, h[j], h[j + 2]);
+    }
+}
+// Walsh-Hadamard transform of a head, pairs as in lh_fwht_lds.
+__device__ __forceinline__ void transform_head(float (&v)[4], uint32_t lane) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        v[j] = lh_fwht_lane_stage<1>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<2>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<4>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<8>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<16>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<32>(v[j], lane);
+    }
+    const float a = __fadd_rn(v[0], v[1]), b = __fsub_rn(v[0], v[1]), c = __fadd_rn(v[2], v[3]), d = __fsub_rn(v[2], v[3]);
+    v[0] = __fadd_rn(a, c); v[2] = __fsub_rn(a, c);
+    v[1] = __fadd_rn(b, d); v[3] = __fsub_rn(b, d);
+}
+// The codes of a head and its norm, as encode_vector makes them (turboquant_kv.hip): the squares, their sum from left to right as the CPU
+// encoder has it, the rest.
+__device__ __forceinline__ void place_squares(const uint16_t (&h)[4], float* square, uint32_t lane) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) square[lane + 64 * j] = lh_h2f(h[j]) * lh_h2f(h[j]);
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ float add_squares(float sum, const float* square, uint32_t first) {       // half of them
+#pragma unroll 8
+    for (uint32_t i = first; i < first + kDim / 2; i += 4) {
+        const float4 q = *reinterpret_cast<const float4*>(&square[i]);
+        sum += q.x; sum += q.y; sum += q.z; sum += q.w;
+    }
+    return sum;
+}
+__device__ __forceinline__ uint16_t encode_head(const uint16_t (&h)[4], float sum, const float (&sign)[4], const float (&level)[4], float inv_sqrt_d, uint32_t lane, uint32_t (&code)[4]) {
+    const float norm = __fsqrt_rn(sum), inv = __fdiv_rn(1.0f, norm);
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        v[j] = lh_h2f(h[j]);
+        if (norm > 0.0f) v[j] = __fmul_rn(v[j], inv);
+        v[j] = __fmul_rn(v[j], sign[j]);
+        asm volatile("" : "+v"(v[j]));
+    }
+    transform_head(v, lane);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        float y = __fmul_rn(v[j], inv_sqrt_d), best = INFINITY;
+        asm volatile("" : "+v"(y));                             // (rounded before the levels are taken off)
+        code[j] = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            const float d = fabsf(__fsub_rn(y, level[i]));
+            if (d < best) { best = d; code[j] = i; }
+        }
+    }
+    return lh_f2h_exact(norm);
+}
+
+// The leading arguments arrive in registers with the wave (see the Makefile); the structures repeat them.
+template <int S, bool OWN>
+__global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_token_kernel(const float* levels, const float* signs, uint32_t q_heads, uint32_t kv_heads, const AttnPointers a,
+                                                                            const AttnParams p, const TokenPrep t) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    ShortShared& sh = *reinterpret_cast<ShortShared*>(lds);
+    TokenShared& ts = *reinterpret_cast<TokenShared*>(lds + sizeof(ShortShared));
+    ShortWave<S>* const all = reinterpret_cast<ShortWave<S>*>(lds + sizeof(ShortShared) + sizeof(TokenShared));
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nall = blockDim.x >> 6, nwaves = OWN ? nall - 2 : nall;
+    uint32_t qi = blockIdx.y, kvh = 0, group = q_heads;
+    if (kv_heads != 1) { qi = blockIdx.y / kv_heads; kvh = blockIdx.y - qi * kv_heads; group = q_heads / kv_heads; }
+    const bool own = OWN && wave >= nwaves, is_v = own && wave > nwaves, is_q = wave < group, works = is_q || own;      // (the first eight waves are no `own`)
+    const float table = levels[lane & 3];                       // (as a scalar load every argument behind it would wait for it)
+
+    // ---- the rotary pairs by two waves, the value's and the last of the others (a window's ninth has no head), ahead of what they wait for
+    const uint32_t position = p.mode == kBatched ? a.positions[qi] : p.pos0, angles = (uint32_t)((float)kDim * t.prf) / 2;
+    const uint32_t second = OWN ? nwaves - 1 : nall - 2;
+    if (wave == nall - 1 || wave == second) {
+        const uint32_t i = lane + (wave == second ? 64 : 0);
+        float c = 1.0f, s = 0.0f;
+        if (i < angles) lh_rope_cos_sin(i, kDim, position, t.theta, c, s);
+        ts.turn[i] = make_float2(c, s);
+    }
+
+    // ---- the wave's head: raw values, norm weights, signs
+    const uint32_t head = is_q ? kvh * group + wave : kvh, column = (is_q ? head : is_v ? q_heads + kv_heads + kvh : q_heads + kvh) * kDim;
+    const size_t row_at = ((size_t)qi * (is_q ? q_heads : kv_heads) + head) * kDim + lane;
+    const uint16_t* const norm_w = is_q ? t.q_norm : own && !is_v ? t.k_norm : nullptr;
+    uint16_t h[4] = {0, 0, 0, 0}, w[4] = {0, 0, 0, 0};
+    float sign[4];
+    if (works) {
+        if (t.partial) {                                        // the splits in order, in f32, rounded to f16: as decode_qkv_prepare_kernel
+            const size_t zstride = (size_t)t.rows * t.part_cols;
+            const float* part = t.partial + (size_t)qi * t.part_cols + column + lane;
+            float acc[4] = {0.f, 0.f, 0.f, 0.f};
+            for (uint32_t z0 = 0; z0 < t.splits; z0 += 8) {
+                float x[8][4];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) x[u][j] = part[(size_t)(z0 + u < t.splits ? z0 + u : t.splits - 1) * zstride + 64 * j];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) if (z0 + u < t.splits) acc[j] += x[u][j];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) h[j] = lh_f2h(acc[j]);
+        } else {
+            const uint16_t* const raw = (is_q ? t.q : is_v ? t.v : t.k) + row_at;
+#pragma unroll
+            for (int j = 0; j < 4; j++) h[j] = raw[64 * j];
+        }
+        if (norm_w)
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[j] = norm_w[lane + 64 * j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) sign[j] = signs[lane + 64 * j];
+
+    uint32_t lo, hi, lane_base;
+    query_range(p, a.positions, qi, lo, hi, lane_base);
+    if (OWN) hi = hi > lo ? hi - 1 : hi;                        // the position itself comes from its own two waves
+    const uint32_t G = (lo >> 6) + wave, g_last = hi > lo ? (hi - 1) >> 6 : 0u;
+    const bool none = hi <= lo;
+    auto load = [&](uint32_t G_) { return load_group<S>(a, p, G_, lo, hi, lane_base, kv_heads, kvh); };
+    Group<S> first{};
+    if (!own && !none && G <= g_last) first = load(G);
+
+    if (works && (is_v || norm_w)) norm_head(h, w, !is_v, t.eps);
+    lh_lds_barrier();
+    if (works && !is_v) turn_head(h, ts.turn, angles, lane);
+    if (works && blockIdx.x == 0) {
+        uint16_t* const to = (is_q ? t.q_out : is_v ? t.v_out : t.k_out) + row_at;
+#pragma unroll
+        for (int j = 0; j < 4; j++) to[64 * j] = h[j];
+    }
+    if (wave < kHeads) {
+        float x[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) { x[j] = is_q ? __fmul_rn(lh_h2f(h[j]), sign[j]) : 0.0f; asm volatile("" : "+v"(x[j])); }
+        transform_head(x, lane);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            x[j] = __fmul_rn(x[j], t.inv_sqrt_d);
+            asm volatile("" : "+v"(x[j]));
+            sh.q(lane & 3, wave, (lane >> 2) + 16 * j) = x[j];
+        }
+        const float m = lh_group_max(fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))), 64), s = lh_group_sum((x[0] + x[1]) + (x[2] + x[3]), 64);
+        if (lane == 0) { sh.maxabs[wave] = m; sh.sum[wave] = s; }
+    }
+    // The position's own waves walk their sums while the others are between barriers.
+    float* const square = ts.square[is_v ? 1 : 0];
+    float squares = 0.0f;
+    if (OWN && own) { place_squares(h, square, lane); squares = add_squares(0.0f, square, 0); }
+    lh_lds_barrier();
+    const float L0 = level_of(table, 0), L1 = level_of(table, 1), L2 = level_of(table, 2), L3 = level_of(table, 3);
+    if (!own) {
+        short_by_levels<S>(a, p, sh, all[wave], first, none ? 1u : G, none ? 0u : g_last, load, L0, L1, L2, L3, qi, kvh, group, nwaves, OWN ? nwaves + 1 : nwaves);
+        return;
+    }
+    if constexpr (OWN) {
+        squares = add_squares(squares, square, kDim / 2);
+        lh_lds_barrier();                                       // short_body's, behind the score operands
+        const float level[4] = {L0, L1, L2, L3};
+        uint32_t code[4];
+        const uint16_t norm = encode_head(h, squares, sign, level, t.inv_sqrt_d, lane, code);
+        float x[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = code[j] == 0 ? L0 : code[j] == 1 ? L1 : code[j] == 2 ? L2 : L3;
+        if (is_v) {
+            constexpr uint32_t E = 4 / S;
+            const float n = lh_h2f(norm);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (j / E == blockIdx.x)
+#pragma unroll
+                    for (uint32_t i = 0; i < kHeads; i++) all[nwaves].park[i][64 * (j % E) + lane] = x[j] * n;
+            if (lane < kHeads) sh.fin_l[nwaves][lane] = 1.0f;
+        } else {                                                // eight lanes a head, eight code bytes each: the levels in the queries' order by way of LDS
+            const uint32_t i = lane >> 3, byte = 8 * (lane & 7);
+#pragma unroll
+            for (int j = 0; j < 4; j++) square[(lane & 3) * 64 + (lane >> 2) + 16 * j] = x[j];
+            __builtin_amdgcn_wave_barrier();
+            float d = 0.0f;
+#pragma unroll
+            for (int f = 0; f < 4; f++)
+#pragma unroll
+                for (int c = 0; c < 8; c += 4) {
+                    const float4 q = *reinterpret_cast<const float4*>(&sh.q(f, i, byte + c)), l = *reinterpret_cast<const float4*>(&square[f * 64 + byte + c]);
+                    d = __builtin_fmaf(q.x, l.x, d); d = __builtin_fmaf(q.y, l.y, d); d = __builtin_fmaf(q.z, l.z, d); d = __builtin_fmaf(q.w, l.w, d);
+                }
+            d = lh_group_sum(d, 8);
+            if ((lane & 7) == 0) sh.fin_r[nwaves][i] = d * (lh_h2f(norm) * kLog2e);
+        }
+        lh_lds_barrier();                                       // short_body's, ahead of the merge
+        if (blockIdx.x != 0) return;
+        const size_t slot = ((size_t)lane_base + (p.ring_capacity ? position % p.ring_capacity : position)) * kv_heads + kvh;
+        uint8_t* const bytes = (is_v ? t.v_codes : t.k_codes) + slot * (kDim / 4);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            uint32_t b = code[j] << 2 * (lane & 3);
+            b |= (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR1>((int)b);
+            b |= (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR2>((int)b);
+            if ((lane & 3) == 0) bytes[(lane >> 2) + 16 * j] = (uint8_t)b;
+        }
+        if (lane == 0) (is_v ? t.v_norms : t.k_norms)[slot] = norm;
+    }
 }
 
 template <int S> constexpr size_t short_lds(uint32_t waves) { return sizeof(ShortShared) + waves * sizeof(ShortWave<S>); }
@@ -335,12 +596,28 @@ int launch(lh_context* ctx, const char* op, const AttnPointers& a, const AttnPar
     return lh_check_launch(op);
 }
 
+template <int S> constexpr size_t token_lds(uint32_t waves) { return sizeof(TokenShared) + short_lds<S>(waves); }
+
+template <int S>
+int launch_token_form(lh_context* ctx, const char* op, const AttnPointers& a, const AttnParams& p, const TokenPrep& t, uint32_t waves) {
+    const dim3 grid(S, p.num_queries * p.num_kv_heads);
+    if (t.k_codes) hipLaunchKernelGGL((attention_tq_token_kernel<S, true>), grid, dim3(64 * (waves + 2)), token_lds<S>(waves + 2), ctx->stream, a.levels, t.signs, p.num_q_heads, p.num_kv_heads, a, p, t);
+    else hipLaunchKernelGGL((attention_tq_token_kernel<S, false>), grid, dim3(64 * waves), token_lds<S>(waves), ctx->stream, a.levels, t.signs, p.num_q_heads, p.num_kv_heads, a, p, t);
+    return lh_check_launch(op);
+}
+
 }  // namespace
 
 int lh_attention_short_init(lh_context* ctx) {
     int r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<4>, short_lds<4>(kMaxWaves), "context_create");
     if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<2>, short_lds<2>(kMaxWaves), "context_create");
     if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<1>, short_lds<1>(kMaxWaves), "context_create");
+    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<4, true>, token_lds<4>(kMaxWaves), "context_create");
+    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<4, false>, token_lds<4>(kMaxWaves), "context_create");
+    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<2, true>, token_lds<2>(kMaxWaves), "context_create");
+    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<2, false>, token_lds<2>(kMaxWaves), "context_create");
+    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<1, true>, token_lds<1>(kMaxWaves), "context_create");
+    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<1, false>, token_lds<1>(kMaxWaves), "context_create");
     return r;
 }
 
@@ -356,6 +633,23 @@ int launch_short(lh_context* ctx, const char* op, const AttnPointers& a, AttnPar
     p.num_splits = 1;
     const uint32_t waves = std::max<uint32_t>(kHeads, (uint32_t)((max_span + 62) / 64 + 1)), queries = p.num_queries * p.num_kv_heads, cus = (uint32_t)ctx->cu_count;
     return queries * 4 <= cus ? launch<4>(ctx, op, a, p, waves) : queries * 2 <= cus ? launch<2>(ctx, op, a, p, waves) : launch<1>(ctx, op, a, p, waves);
+}
+
+// Waves for the groups that `positions` in a row may touch, one for each head at least.
+static uint32_t group_waves(uint64_t positions) { return std::max<uint32_t>(kHeads, (uint32_t)((positions + 62) / 64 + 1)); }
+
+bool token_supported(const lh_context* ctx, const AttnParams& p, const TokenPrep& t, uint64_t max_span) {
+    if (max_span == 0 || !short_supported(ctx, p, max_span)) return false;
+    if (t.k_codes && group_waves(max_span - 1) + 2 > kMaxWaves) return false;
+    // The position's slot is written while the positions before it are read: on a ring it has to be none of theirs.
+    const uint64_t most = p.mode != kBatched ? max_span : p.window ? p.window : p.ring_capacity ? UINT64_MAX : max_span;
+    return !t.k_codes || p.ring_capacity == 0 || most <= p.ring_capacity;
+}
+
+int launch_token(lh_context* ctx, const char* op, const AttnPointers& a, AttnParams& p, const TokenPrep& t, uint64_t max_span) {
+    p.num_splits = 1;
+    const uint32_t waves = group_waves(t.k_codes ? max_span - 1 : max_span), queries = p.num_queries * p.num_kv_heads, cus = (uint32_t)ctx->cu_count;
+    return queries * 4 <= cus ? launch_token_form<4>(ctx, op, a, p, t, waves) : queries * 2 <= cus ? launch_token_form<2>(ctx, op, a, p, t, waves) : launch_token_form<1>(ctx, op, a, p, t, waves);
 }
 
 }  // namespace lh_attn

@@ -157,10 +157,10 @@ struct PrepareParams {
     // heads, the value heads, side by side) instead of f16 rows in q / k / v; nullptr: the rows are read from q / k / v.
     const float* partial;
     uint32_t splits, part_cols, rows;
+    const uint16_t *q_raw, *k_raw, *v_raw;          // the rows to prepare: q, k, v themselves where they are prepared in place
 };
 
-__global__ __launch_bounds__(kMaxHeadDim) void decode_qkv_prepare_kernel(uint16_t* __restrict__ q, uint16_t* __restrict__ k,
-                                                                        uint16_t* __restrict__ v, const uint16_t* __restrict__ q_norm_w,
+__global__ __launch_bounds__(kMaxHeadDim) void decode_qkv_prepare_kernel(uint16_t* q, uint16_t* k, uint16_t* v, const uint16_t* __restrict__ q_norm_w,
                                                                         const uint16_t* __restrict__ k_norm_w, const float* __restrict__ signs,
                                                                         const float* __restrict__ levels, float* __restrict__ rq,
                                                                         uint8_t* __restrict__ k_codes, uint16_t* __restrict__ k_norms,
@@ -176,7 +176,8 @@ __global__ __launch_bounds__(kMaxHeadDim) void decode_qkv_prepare_kernel(uint16_
     const uint32_t position = positions ? positions[row] : p.position + row;
     const bool is_q = b < p.n_q_heads, is_k = !is_q && b < p.n_q_heads + p.n_kv_heads;
     const uint32_t head = is_q ? b : (is_k ? b - p.n_q_heads : b - p.n_q_heads - p.n_kv_heads);
-    uint16_t* vec = (is_q ? q : (is_k ? k : v)) + ((size_t)row * (is_q ? p.n_q_heads : p.n_kv_heads) + head) * d;
+    const size_t vec_at = ((size_t)row * (is_q ? p.n_q_heads : p.n_kv_heads) + head) * d;
+    uint16_t* vec = (is_q ? q : (is_k ? k : v)) + vec_at;
     const uint16_t* norm_w = is_q ? q_norm_w : (is_k ? k_norm_w : nullptr);
     const bool normalise = !(is_q || is_k) || norm_w != nullptr;          // V always (unit weight); Q / K when the layer has the weight
 
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(kMaxHeadDim) void decode_qkv_prepare_kernel(uint16_
         }
         raw = lh_f2h(acc);
     } else {
-        raw = vec[lane];
+        raw = ((is_q ? p.q_raw : (is_k ? p.k_raw : p.v_raw)) + vec_at)[lane];
     }
     const float norm_weight = norm_w ? lh_h2f(norm_w[lane]) : 1.0f;
     const float sign = signs[lane];
@@ -510,6 +511,7 @@ int lh_prepare_rows_launch(lh_batch* batch, const LhPrepareRows& a, const float*
     const bool write_kv = k != nullptr && v != nullptr && n_kv_heads != 0;
     const uint32_t cb = lh_turboquant_code_bytes(head_dim, bits);
     LH_NEED(q, (size_t)rows * n_q_heads * head_dim * 2, op, "q");
+    if (a.q_raw) LH_NEED(a.q_raw, (size_t)rows * n_q_heads * head_dim * 2, op, "raw q");
     LH_NEED(rq, (size_t)rows * n_q_heads * head_dim * 4, op, "rq");
     LH_NEED(signs, (size_t)head_dim * 4, op, "signs");
     if (q_norm) LH_NEED(q_norm, (size_t)head_dim * 2, op, "q_norm");
@@ -521,6 +523,8 @@ int lh_prepare_rows_launch(lh_batch* batch, const LhPrepareRows& a, const float*
         const uint64_t phys = lane_capacity ? (uint64_t)rows * lane_capacity : (ring_capacity ? std::min<uint64_t>(ring_capacity, last) : last);
         LH_NEED(k, (size_t)rows * n_kv_heads * head_dim * 2, op, "k");
         LH_NEED(v, (size_t)rows * n_kv_heads * head_dim * 2, op, "v");
+        if (a.k_raw) LH_NEED(a.k_raw, (size_t)rows * n_kv_heads * head_dim * 2, op, "raw k");
+        if (a.v_raw) LH_NEED(a.v_raw, (size_t)rows * n_kv_heads * head_dim * 2, op, "raw v");
         LH_NEED(levels, (size_t)4 << bits, op, "levels");
         if (k_norm) LH_NEED(k_norm, (size_t)head_dim * 2, op, "k_norm");
         LH_NEED(k_codes, (size_t)phys * n_kv_heads * cb, op, "k_codes");
@@ -529,7 +533,9 @@ int lh_prepare_rows_launch(lh_batch* batch, const LhPrepareRows& a, const float*
         LH_NEED(v_norms, (size_t)phys * n_kv_heads * 2, op, "v_norms");
     }
     PrepareParams p{head_dim, n_q_heads, write_kv ? n_kv_heads : 0u, bits, cb, start_position, ring_capacity, write_kv ? 1u : 0u, lane_capacity,
-                    eps, theta, partial_rotary_factor, host_inv_sqrt(head_dim), partial, splits, part_cols, rows};
+                    eps, theta, partial_rotary_factor, host_inv_sqrt(head_dim), partial, splits, part_cols, rows,
+                    (const uint16_t*)(a.q_raw ? a.q_raw : q)->ptr, write_kv ? (const uint16_t*)(a.k_raw ? a.k_raw : k)->ptr : nullptr,
+                    write_kv ? (const uint16_t*)(a.v_raw ? a.v_raw : v)->ptr : nullptr};
     const uint64_t groups = (uint64_t)rows * (n_q_heads + (write_kv ? 2 * n_kv_heads : 0));
     LH_REQUIRE(groups <= 0x7FFFFFFFull, "%s: %u rows are too many for one launch", op, rows);
     if (partial) LH_REQUIRE(splits >= 1 && (uint64_t)(n_q_heads + (write_kv ? 2 * n_kv_heads : 0)) * head_dim <= part_cols,

@@ -144,6 +144,16 @@ class QuantizedKvCache:
                                                             self.head_dim, seq_len, current_pos, n_q_heads,
                                                             self.n_kv_heads, window, self.bits, self.ring_capacity())
 
+    def attend_token_into(self, batch, kernels: Kernels, raw, q: Buffer, k, v, q_norm, k_norm, rq: Buffer, vacc: Buffer, attn_out: Buffer, position: int,
+                          n_q_heads: int, window: int, eps: float, theta: float, partial_rotary_factor: float, lazy: bool) -> bool:
+        """``prepare_token_into`` on the rows ``raw`` (q, k, v), then ``attention_from_rotated_into`` or, ``lazy``, its lazy form, as one
+        step; True: ``attn_out`` holds the rotated f16 heads."""
+        if k is not None and position + 1 > self.max_positions:
+            raise InvalidArgument(f"KV write [{position}..{position + 1}) exceeds capacity {self.max_positions}")
+        return kernels.token_attention_tq_into(batch, raw, q, k, v, q_norm, k_norm, self.levels, self.signs, rq, self.keys_q, self.key_norms, self.values_q,
+                                               self.value_norms, vacc, attn_out, self.head_dim, n_q_heads, self.n_kv_heads, eps, position, theta,
+                                               partial_rotary_factor, window, self.bits, self.ring_capacity(), lazy)
+
     def prepare_rows_into(self, batch, kernels: Kernels, q: Buffer, k, v, q_norm, k_norm, rq: Buffer, start_pos: int,
                           n_rows: int, n_q_heads: int, eps: float, theta: float, partial_rotary_factor: float) -> None:
         """``prepare_token_into`` for the ``n_rows`` consecutive tokens of a prefill chunk."""

@@ -100,6 +100,8 @@ class ScratchBuffers:
         self.q = self.qkv.view(0, q_elems * 2)
         self.k = self.qkv.view(q_elems * 2, kv_elems * 2)
         self.v = self.qkv.view((q_elems + kv_elems) * 2, kv_elems * 2)
+        # the projections' rows, where the preparation leaves its own in q, k, v
+        self.raw_qkv = _alloc_f16(ctx, q_elems + 2 * kv_elems)
         self.rq = _alloc_f32(ctx, q_elems)
         self.vacc = _alloc_f32(ctx, q_elems)
         self.attn_out = _alloc_f16(ctx, q_elems)
@@ -204,13 +206,13 @@ class TransformerLayer:
         self._qkv = QuantWeight.quantized(stacked, q.ty, q.rows + k.rows + v.rows, q.cols)
 
     def _qkv_views(self, scratch: "ScratchBuffers"):
-        """(q, k, v) views of scratch.qkv at this layer's sizes, consecutive (cached per scratch object)."""
+        """(q, k, v, all three) views of scratch.qkv at this layer's sizes, consecutive, and the same of scratch.raw_qkv (cached per scratch
+        object)."""
         cached = getattr(self, "_qkv_view_cache", None)
         if cached is None or cached[0] is not scratch:
             p = self.params
             nq, nkv = p.num_attention_heads * p.head_dim * 2, p.num_key_value_heads * p.head_dim * 2
-            cached = (scratch, scratch.qkv.view(0, nq), scratch.qkv.view(nq, nkv), scratch.qkv.view(nq + nkv, nkv),
-                      scratch.qkv.view(0, nq + 2 * nkv))
+            cached = (scratch, *([b.view(0, nq), b.view(nq, nkv), b.view(nq + nkv, nkv), b.view(0, nq + 2 * nkv)] for b in (scratch.qkv, scratch.raw_qkv)))
             self._qkv_view_cache = cached
         return cached[1:]
 
@@ -309,13 +311,17 @@ class TransformerLayer:
         # 1. input_layernorm -> Q projection -> q_norm -> RoPE
         own_kv = not p.is_kv_shared and w.attn_k is not None and w.attn_v is not None
         fused_in = self._fusable(w.attn_q) and (not own_kv or self._fusable(w.attn_k, w.attn_v))
+        one_prepare = self._one_prepare()
         q_buf, k_buf, v_buf = s.q, s.k, s.v
         stacked = fused_in and own_kv and self._qkv is not None
+        prepared, raw = self._qkv_views(s)
+        if stacked:
+            q_buf, k_buf, v_buf = prepared[:3]
+        raw_q, raw_k, raw_v, qkv_out = raw if one_prepare else (q_buf, k_buf, v_buf, prepared[3])      # where the projections go
         if pending is not None and not fused_in:   # nothing here can take it along: the previous layer's last step by itself
             kernels.rms_norm_residual_scale_into(batch, pending.x, pending.weight, pending.residual, input, h, 1, eps, pending.scale)
             pending = None
         if stacked:   # one matvec over the stacked [Wq; Wk; Wv] writes q | k | v side by side
-            q_buf, k_buf, v_buf, qkv_out = self._qkv_views(s)
             if pending is not None:
                 kernels.matvec_quant_norm_chain_tail_into(batch, self._qkv.ty, [self._qkv.buf], pending.x, pending.weight,
                                                           pending.residual, pending.scale, w.attn_norm, input, eps, [qkv_out],
@@ -325,14 +331,13 @@ class TransformerLayer:
         elif fused_in:
             if pending is not None:   # (the K / V launch below then finds `input` written)
                 kernels.matvec_quant_norm_chain_tail_into(batch, w.attn_q.ty, [w.attn_q.buf], pending.x, pending.weight,
-                                                          pending.residual, pending.scale, w.attn_norm, input, eps, [s.q],
+                                                          pending.residual, pending.scale, w.attn_norm, input, eps, [raw_q],
                                                           w.attn_q.rows, w.attn_q.cols)
             else:
-                self._fused_matvecs(batch, kernels, kernels.PROLOGUE_RMS_NORM, input, w.attn_norm, [w.attn_q], [s.q])
+                self._fused_matvecs(batch, kernels, kernels.PROLOGUE_RMS_NORM, input, w.attn_norm, [w.attn_q], [raw_q])
         else:
             kernels.rms_norm_into(batch, input, w.attn_norm, s.normed, h, 1, eps)
-            w.attn_q.matvec_into(batch, kernels, s.normed, s.q)
-        one_prepare = self._one_prepare()
+            w.attn_q.matvec_into(batch, kernels, s.normed, raw_q)
         rotate_in_o = (one_prepare and self.fuse_rotation and self._fusable(w.attn_output)
                        and w.attn_output.cols == n_head * hd)
         if not one_prepare:
@@ -342,19 +347,15 @@ class TransformerLayer:
         if own_kv and not stacked:
             if fused_in:
                 self._fused_matvecs(batch, kernels, kernels.PROLOGUE_RMS_NORM, input, w.attn_norm,
-                                    [w.attn_k, w.attn_v], [s.k, s.v])
+                                    [w.attn_k, w.attn_v], [raw_k, raw_v])
             else:
-                self._pair_matvec(batch, kernels, w.attn_k, w.attn_v, s.normed, s.k, s.v)
-        if one_prepare:   # head norms, RoPE, V norm, both encodes and the query rotation in one dispatch
-            kv_cache.prepare_token_into(batch, kernels, q_buf, k_buf if own_kv else None, v_buf if own_kv else None,
-                                        w.q_norm, w.k_norm, s.rq, position, n_head, eps, p.rope_theta,
-                                        p.partial_rotary_factor)
-            if rotate_in_o:   # where the rotation would be a launch of its own, step 3 does it while it stages the heads
-                rotate_in_o = not kv_cache.attention_from_rotated_lazy_into(batch, kernels, s.rq, s.vacc, s.attn_out,
-                                                                            seq_len, pos, n_head, p.sliding_window)
-            else:
-                kv_cache.attention_from_rotated_into(batch, kernels, s.rq, s.vacc, s.attn_out, seq_len, pos, n_head,
-                                                     p.sliding_window)
+                self._pair_matvec(batch, kernels, w.attn_k, w.attn_v, s.normed, raw_k, raw_v)
+        if one_prepare:   # head norms, RoPE, V norm, both encodes, the query rotation and attention: over a window one dispatch
+            # (where the rotation back would be a launch of its own, step 3 does it while it stages the heads)
+            rotated = kv_cache.attend_token_into(batch, kernels, (raw_q, raw_k, raw_v), q_buf, k_buf if own_kv else None, v_buf if own_kv else None,
+                                                 w.q_norm, w.k_norm, s.rq, s.vacc, s.attn_out, pos, n_head, p.sliding_window, eps,
+                                                 p.rope_theta, p.partial_rotary_factor, rotate_in_o)
+            rotate_in_o = rotate_in_o and not rotated
         elif own_kv:
             kernels.rms_norm_into(batch, v_buf, s.ones, v_buf, hd, n_kv, eps)   # V: RMS norm with unit weight
             self._norm_rope(batch, kernels, k_buf, w.k_norm, n_kv, pos)

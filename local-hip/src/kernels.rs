@@ -1,6 +1,6 @@
 // The kernel-dispatch layer: `Kernels`, one method per operation of liblocal_hip.so, with the names and the argument
 // order that local-engine calls on local-metal (local-metal/src/kernels.rs).  GENERATED by gen_safe.py from
-// include/local_hip.h: do not edit.  Operations with host pointers and the helpers of the codec are wrapped by hand in lib.rs: lh_matvec_quant_norm_chain_gelu_into, lh_turboquant_levels, lh_turboquant_signs, lh_turboquant_code_bytes, lh_swa_ring_capacity, lh_flash_attention_tq_rotated_lazy_into, lh_flash_split_count.
+// include/local_hip.h: do not edit.  Operations with host pointers and the helpers of the codec are wrapped by hand in lib.rs: lh_matvec_quant_norm_chain_gelu_into, lh_turboquant_levels, lh_turboquant_signs, lh_turboquant_code_bytes, lh_swa_ring_capacity, lh_flash_attention_tq_rotated_lazy_into, lh_token_attention_tq_into, lh_flash_split_count.
 // Other host-side helpers are reached through `ffi`: lh_qk_norm_rope_available, lh_smallm_max_m, lh_batchm_max_m, lh_multivec_max_m, lh_batchm_enabled, lh_mma_enabled, lh_smallm_enabled, lh_kv_bits_from_env, lh_gated_vector_fits, lh_attention_padded_dim, lh_attention_padded_vdim, lh_latent_padded_rank, lh_latent_row, lh_linear_attention_padded_dim, lh_linear_attention_workspace_bytes, lh_selective_steps_bytes, lh_moe_plan_words.
 use core::ffi::c_int;
 

@@ -83,6 +83,30 @@ fn opt(buffer: Option<&Buffer>) -> *mut ffi::lh_buffer {
     buffer.map_or(core::ptr::null_mut(), Buffer::as_ptr)
 }
 
+/// `lh_token_attention_tq_into` (include/local_hip.h): a decoded token's preparation (layer.rs:393-450) and its attention over the
+/// codes as one step.  The first three of `raw` and `rows` are the query, key and value rows before and behind norm and
+/// rotary embedding; without key and value rows the layer reads another's cache.  `lazy`, `Ok`: as for
+/// `flash_attention_tq_rotated_lazy_into` (`Ok(true)` wherever `lazy` is not asked for).
+#[allow(clippy::too_many_arguments)]
+pub fn token_attention_tq_into(batch: &mut CommandBatch, q_raw: Option<&Buffer>, k_raw: Option<&Buffer>, v_raw: Option<&Buffer>,
+                               q: &Buffer, k: Option<&Buffer>, v: Option<&Buffer>, q_norm: Option<&Buffer>,
+                               k_norm: Option<&Buffer>, levels: &Buffer, signs: &Buffer, rq: &Buffer, k_codes: &Buffer,
+                               k_norms: &Buffer, v_codes: &Buffer, v_norms: &Buffer, out: &Buffer, out_f16: &Buffer,
+                               head_dim: u32, num_q_heads: u32, num_kv_heads: u32, eps: f32, position: u32, theta: f32,
+                               partial_rotary_factor: f32, window: u32, bits: u32, ring_capacity: u32, lazy: bool) -> Result<bool> {
+    let mut rotated: core::ffi::c_int = 1;
+    let asked = if lazy { &mut rotated as *mut core::ffi::c_int } else { core::ptr::null_mut() };
+    // SAFETY: every pointer is null or comes from a live handle of this crate or from a local; the library validates sizes and shapes.
+    error::check(unsafe {
+        ffi::lh_token_attention_tq_into(batch.as_ptr(), opt(q_raw), opt(k_raw), opt(v_raw), q.as_ptr(), opt(k), opt(v), opt(q_norm),
+                                        opt(k_norm), levels.as_ptr(), signs.as_ptr(), rq.as_ptr(), k_codes.as_ptr(),
+                                        k_norms.as_ptr(), v_codes.as_ptr(), v_norms.as_ptr(), out.as_ptr(), out_f16.as_ptr(),
+                                        head_dim, num_q_heads, num_kv_heads, eps, position, theta, partial_rotary_factor, window,
+                                        bits, ring_capacity, asked)
+    })?;
+    Ok(rotated != 0)
+}
+
 /// `lh_matvec_quant_norm_chain_gelu_into` (include/local_hip.h): gate and up projection (or, with `factor` instead of `up`, one
 /// projection) behind a chain of norms, and the GeGLU product of their results where the launch can form it (layer.rs:476-482,
 /// 495-500).  `Ok(true)`: `out` holds the product.  `Ok(false)`: `out` and `up_out` hold the projections' results.

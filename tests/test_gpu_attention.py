@@ -710,3 +710,65 @@ def test_rotated_entry_arguments(pkg, gpu, oracle):
         K.flash_attention_tq_rotated_into(batch, rqb, kcb, knb, vcb, vnb, lvb, pkg.Buffer.empty(ctx, hd * 2), acc, o16, hd, T,
                                           T - 1, nq, nkv, 0, bits, 0)
     batch.commit_and_wait()
+
+
+@pytest.mark.parametrize("n_q,n_kv,window,ring,position", [
+    (8, 1, 512, 1024, 0), (8, 1, 512, 1024, 1), (8, 1, 512, 1024, 63), (8, 1, 512, 1024, 64), (8, 1, 512, 1024, 511), (8, 1, 512, 1024, 512), (8, 1, 512, 1024, 2000),
+    (8, 1, 512, 512, 700), (4, 1, 32, 64, 70), (8, 2, 300, 512, 900), (3, 3, 0, 0, 200), (8, 1, 1, 64, 129), (8, 1, 0, 0, 577), (8, 1, 0, 0, 578), (8, 1, 0, 256, 700)])
+@pytest.mark.parametrize("own,with_norms,asymmetric", [(True, True, False), (False, True, False), (True, False, True)])
+def test_token_in_one_step_equals_preparation_and_attention(pkg, gpu, oracle, n_q, n_kv, window, ring, position, own, with_norms, asymmetric):
+    """A token's preparation in the attention's launch (where the span is short and the position's slot is no other's: a window of 512, a
+    few positions, not the last two cases' 579 positions and wrapped ring) leaves the caches and heads of the separate steps bit for
+    bit; its own position's weight is summed in f32 instead of 16-bit fixed point, so the heads differ by that."""
+    ctx, K = gpu
+    hd, bits, eps, theta = 256, 2, 1e-6, 1e4
+    g = pkg.synth.rng(71, position + n_q + window)
+    slots = ring or position + 5
+    levels, signs = oracle.tq_levels(hd, bits), oracle.rotation_signs(hd)
+    if asymmetric:
+        levels = (levels + np.float32(0.3 * levels.max())).astype(np.float32)
+    lv, sg = pkg.Buffer.from_slice(ctx, levels), pkg.Buffer.from_slice(ctx, signs)
+    # (scores of a few units: beyond, the old steps' 16-bit scores are what the two would differ by)
+    rows = {n: (g.standard_normal(c * hd, dtype=np.float32) * (2 if with_norms or n == "v" else 0.25)).astype(np.float16) for n, c in (("q", n_q), ("k", n_kv), ("v", n_kv))}
+    qw, kw = ((0.25 * (1 + 0.1 * g.standard_normal(hd, dtype=np.float32))).astype(np.float16) for _ in range(2))
+    qwb, kwb = (pkg.Buffer.from_slice(ctx, w) if with_norms else None for w in (qw, kw))
+    codes = [g.integers(0, 256, slots * n_kv * hd // 4, dtype=np.uint8) for _ in range(2)]
+    norms = [(14 * (0.8 + 0.4 * g.random(slots * n_kv))).astype(np.float16) for _ in range(2)]
+
+    def fresh():
+        b = {n: pkg.Buffer.from_slice(ctx, x) for n, x in rows.items()}
+        b.update({"raw_" + n: pkg.Buffer.from_slice(ctx, x) for n, x in rows.items()})
+        b.update(kc=pkg.Buffer.from_slice(ctx, codes[0]), vc=pkg.Buffer.from_slice(ctx, codes[1]), kn=pkg.Buffer.from_slice(ctx, norms[0]),
+                 vn=pkg.Buffer.from_slice(ctx, norms[1]), rq=pkg.Buffer.empty(ctx, n_q * hd * 4), out=pkg.Buffer.empty(ctx, n_q * hd * 4),
+                 o16=pkg.Buffer.empty(ctx, n_q * hd * 2))
+        return b
+    a = fresh()
+    batch = pkg.CommandBatch(ctx)
+    K.decode_qkv_prepare_into(batch, a["q"], a["k"] if own else None, a["v"] if own else None, qwb, kwb if own else None, lv, sg, a["rq"], a["kc"], a["kn"], a["vc"],
+                              a["vn"], hd, n_q, n_kv, eps, position, theta, 0.5, bits, ring)
+    K.flash_attention_tq_rotated_into(batch, a["rq"], a["kc"], a["kn"], a["vc"], a["vn"], lv, sg, a["out"], a["o16"], hd, position + 1, position, n_q, n_kv, window,
+                                      bits, ring)
+    batch.commit_and_wait()
+    want = a["out"].as_array(np.float32)
+    span = min(position + 1, window or position + 1)
+    one = span + 1 <= 579 and (not ring or span <= ring) and not (not own and span > 641)
+    for raw, lazy in ((True, False), (True, True), (False, False)):
+        b = fresh()
+        batch = pkg.CommandBatch(ctx)
+        src = [b["raw_" + n] if raw else b[n] for n in "qkv"]
+        done = K.token_attention_tq_into(batch, src, b["q"], b["k"] if own else None, b["v"] if own else None, qwb, kwb if own else None, lv, sg,
+                                         b["rq"], b["kc"], b["kn"], b["vc"], b["vn"], b["out"], b["o16"], hd, n_q, n_kv, eps, position, theta, 0.5, window,
+                                         bits, ring, lazy)
+        launches = batch.dispatch_count()
+        batch.commit_and_wait()
+        if own and raw and one:
+            assert launches == (1 if lazy else 2) and done == (not lazy)
+        if not raw:
+            assert launches >= 3
+        for n in ("q", "k", "v", "kc", "kn", "vc", "vn"):
+            if own or n == "q":
+                assert np.array_equal(a[n].as_array(np.uint8), b[n].as_array(np.uint8)), n
+        got = b["out"].as_array(np.float32)
+        assert np.abs(got - want).max() <= 2e-4 * np.abs(want).max() + 1e-30, (raw, np.abs(got - want).max(), np.abs(want).max())
+        if not lazy:
+            assert np.abs(b["o16"].as_array(np.float16).astype(np.float32) - a["o16"].as_array(np.float16).astype(np.float32)).max() <= 1e-3 * np.abs(want).max()
