@@ -220,8 +220,10 @@ __device__ __forceinline__ u32x4_t ld16_stream(gptr_t p) {
     return __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) u32x4_a4*>(p));
 }
 
-// One launch serves `count` problems of the same shape (count == 1 for the plain matvec).
-template <int FMT, int L, int NPOS, typename XT, typename YT, bool IMG = false>
+// One launch serves `count` problems of the same shape (count == 1 for the plain matvec).  PRO: the vector may stand behind a prologue.
+// (Streaming launches without one have a form of their own: with the prologues' code in it a 1536-column launch keeps 76 bytes a lane in scratch memory,
+// without 24: the 262144 rows of a token's logits 47-50 us, 42.7.  2048 and more columns: the same time in both.)
+template <int FMT, int L, int NPOS, typename XT, typename YT, bool IMG = false, bool PRO = true>
 __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProblem* __restrict__ problems, MatvecBase single,
                                                              uint32_t count, uint32_t rows, uint32_t K, uint32_t lpr_log2,
                                                              uint32_t steps_per_wg) {
@@ -326,7 +328,8 @@ __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProble
         }
         if (pb.vector != staged_vector) {
             __syncthreads();   // every wave is done reading the previous vector's limbs
-            quantize_x_to_lds<L, G, XT>(static_cast<const XT*>(pb.vector), K, xq, xs, nullptr, kWG, single.pro, L == 2 ? &resid : nullptr);
+            if constexpr (PRO) quantize_x_to_lds<L, G, XT>(static_cast<const XT*>(pb.vector), K, xq, xs, nullptr, kWG, single.pro, L == 2 ? &resid : nullptr);
+            else quantize_x_to_lds<L, G, XT>(static_cast<const XT*>(pb.vector), K, xq, xs, nullptr, kWG, XPrologue{kXProNone, nullptr, 0.0f}, L == 2 ? &resid : nullptr);
             __syncthreads();
             if constexpr (L == 2) {
                 bool mine = false;
@@ -626,7 +629,8 @@ int launch_typed(lh_context* ctx, const MatvecProblem* dev_problems, const Matve
 #define LH_LAUNCH(XT, YT)                                                                                                   \
     do {                                                                                                                    \
         if constexpr (FMT == LH_Q4_0 && L == 2) {                                                                           \
-            if (g.img) LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, true>));                                      \
+            if (g.img && single.pro.kind == kXProNone) LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, true, false>)); \
+            else if (g.img) LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, true>));                                 \
             else LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, false>));                                           \
         } else LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, false>));                                             \
     } while (0)
