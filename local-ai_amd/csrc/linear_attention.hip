@@ -3,8 +3,8 @@
 // a multiple of v is added to y).  The state M is f32,
 // kept as [head][value column][DQ key columns] (the key columns that exist, then zeros).
 //
-// Recurrent form: one workgroup per head and 16 value columns; a row of 16 lanes holds one value column's state in
-// registers (DQ / 16 values each) and walks the rows.  From eight rows on the inputs come in several rows ahead.
+// Recurrent form: a wave (65 to 512 key columns) or a row of 16 lanes holds one value column's state in registers and walks the
+// rows, whose inputs come in several rows ahead.
 //
 // Chunked form (64 or 128 rows a chunk, bf16 inputs on the matrix cores, everything else f32; with 128 the states, which every step
 // writes or reads, are half as many):
@@ -161,6 +161,92 @@ __global__ __launch_bounds__(256) void recurrent_rows_kernel(const RecurrentArgs
     if (on && has) {
 #pragma unroll
         for (int i = 0; i < NR; i++) st[i] = s[i];
+    }
+}
+
+// The same with a wave a value column: four times as many waves, a quarter of the state in each.  Where columns are few the form above has a
+// wave on every fourth SIMD, and a row is the instructions of one wave one behind the other: 333 rows of 8 heads, 128 x 128, in 32 bits
+// 62 us there (450 cycles a row), 31 here.  Four rows' sums over the lanes share their steps -- a lane keeps the row of its two lowest bits --
+// and leave in one store; what a selective state space computes for a row is computed for AHEAD rows at a time, a lane each.
+template <typename T, int NR, int AHEAD, Decay DECAY>
+__global__ __launch_bounds__(256) void recurrent_wide_kernel(const RecurrentArgs a) {
+    static_assert(AHEAD % 4 == 0 && AHEAD <= 64, "rows in fours, a lane each");
+    constexpr bool SELECTIVE = DECAY == kSelective;
+    const uint32_t lane = threadIdx.x & 63, column = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), dim = a.dim, dq = a.dq, vdim = a.vdim, heads = a.heads, rows = a.rows;
+    if (column >= heads * vdim) return;
+    const uint32_t h = column / vdim;
+    const bool has = lane * NR < dq;                              // (dq is a multiple of NR: a lane has all of its values, or none)
+    const uint32_t k0 = has ? lane * NR : 0u, in = !has ? 0u : k0 < dim ? min(dim - k0, (uint32_t)NR) : 0u;
+    const size_t step = (size_t)a.key_heads * dq, first = (size_t)(h / (heads / a.key_heads)) * dq, across = (size_t)heads * vdim;
+    const T *q = static_cast<const T*>(a.q) + first, *k = static_cast<const T*>(a.k) + first, *v = static_cast<const T*>(a.v) + column;
+    float* st = a.state + (size_t)column * dq;
+    float s[NR];
+#pragma unroll
+    for (int i = 0; i < NR; i++) s[i] = has ? st[k0 + i] : 0.0f;
+    const float fixed = SELECTIVE ? 0.0f : a.decay[(size_t)h * (DECAY == kPowers ? kHalf + 1 : 1)], rate = SELECTIVE ? -expf(a.a_log[h]) : 0.0f, bias = SELECTIVE ? a.dt_bias[h] : 0.0f,
+                skip = SELECTIVE ? a.skip[h] : 0.0f;
+    struct Row { Packed<T, NR> k, q; T v; } next[AHEAD];
+    auto fetch = [&](Row& r, uint32_t t) {
+        const size_t u = min(t, rows - 1);
+        r.k.load(k + u * step + k0);
+        r.q.load(q + u * step + k0);
+        r.v = v[u * across];
+    };
+    auto raw = [&](uint32_t t) { return SELECTIVE ? a.dt_raw[(size_t)min(t + min(lane, (uint32_t)AHEAD - 1), rows - 1) * heads + h] : 0.0f; };
+    float z = raw(0), dts = 1.0f, ds = 1.0f;                        // lane j: what row t + j has
+    auto steps = [&](uint32_t t) {                                  // of rows t .. t + AHEAD - 1; the next ones' are requested
+        if constexpr (SELECTIVE) {
+            dts = softplus(z + bias);
+            ds = expf(rate * dts);
+            z = raw(t + AHEAD);
+        }
+    };
+    auto at_row = [&](float x, int j) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), j)); };
+    auto four = [&](const Row* r, int j0, uint32_t t, uint32_t count) {
+        float o[4], x[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            o[j] = 0.0f;
+            x[j] = lh_ld(&r[j].v, 0);
+            if ((uint32_t)j >= count) continue;
+            const float dt = SELECTIVE ? at_row(dts, j0 + j) : 1.0f, d = SELECTIVE ? at_row(ds, j0 + j) : fixed, vc = SELECTIVE ? dt * x[j] : x[j];
+#pragma unroll
+            for (int i = 0; i < NR; i++) {
+                s[i] = __builtin_fmaf((uint32_t)i < in ? r[j].k.get(i) : 0.0f, vc, d * s[i]);
+                o[j] = __builtin_fmaf(s[i], (uint32_t)i < in ? r[j].q.get(i) : 0.0f, o[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[j] += lh_dpp_f<LH_DPP_QUAD_XOR1>(o[j]);
+        float e = lane & 1 ? o[1] : o[0], f = lane & 1 ? o[3] : o[2];
+        e += lh_dpp_f<LH_DPP_QUAD_XOR2>(e);
+        f += lh_dpp_f<LH_DPP_QUAD_XOR2>(f);
+        float y = lane & 2 ? f : e;
+        y += lh_lane_xor_f<4>(y);
+        y += lh_lane_xor_f<8>(y);
+        y = lh_sum32_f(lh_sum16_f(y));
+        if (SELECTIVE) y = __builtin_fmaf(skip, lane & 2 ? (lane & 1 ? x[3] : x[2]) : (lane & 1 ? x[1] : x[0]), y);
+        else y *= a.scale;
+        if (lane < count) a.out[(size_t)(t + lane) * across + column] = y;
+    };
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) fetch(next[j], j);
+    uint32_t t = 0;
+    for (; t + AHEAD <= rows; t += AHEAD) {
+        steps(t);
+#pragma unroll
+        for (int j = 0; j < AHEAD; j += 4) {
+            four(next + j, j, t + j, 4);
+#pragma unroll
+            for (int i = 0; i < 4; i++) fetch(next[j + i], t + AHEAD + j + i);
+        }
+    }
+    steps(t);
+#pragma unroll
+    for (int j = 0; j < AHEAD; j += 4) if (t + j < rows) four(next + j, j, t + j, min(rows - t - j, 4u));
+    if (has) {
+#pragma unroll
+        for (int i = 0; i < NR; i++) st[k0 + i] = s[i];
     }
 }
 
@@ -622,13 +708,26 @@ template <typename T, Decay DECAY>
 int launch_recurrent(lh_context* ctx, const RecurrentArgs& a, const char* op) {
     const uint64_t grid = (uint64_t)a.heads * ((a.vdim + 15) / 16);
     LH_REQUIRE(grid < 0x7FFFFFFFull, "%s: heads %u, vdim %u", op, a.heads, a.vdim);
-    if (a.rows >= 8 && (((uintptr_t)a.q | (uintptr_t)a.k) & 15) == 0) {        // (a row's keys and queries start at multiples of 32 values)
+    const bool whole = (((uintptr_t)a.q | (uintptr_t)a.k) & 15) == 0;          // (a row's keys and queries start at multiples of 32 values)
+    const uint64_t columns = (uint64_t)a.heads * a.vdim;
+    // A wave a column from 65 key columns on (below, half its lanes would have none): few rows always (us of 1, 2 and 7 rows of 16 heads, bf16, then so: 128 x 128 5.4,
+    // 6.4, 12.1 and 4.8, 4.6, 4.9; 256 x 128 10.7, 14.6, 33.2 and 4.7, 4.6, 4.8), and of many rows where a lane of the other form would hold
+    // more than eight values or compute the rows' steps (200 rows of 48 heads, f32: 256 x 128 189 and 99, selective 128 x 128 186 and 98);
+    // else up to two waves a SIMD (128 x 128, 8, 16 and 24 heads: 39, 40, 40 and 21, 33, 47).
+    if (whole && a.dq > 64 && a.dq <= 512 && (a.rows < 8 || a.dq > 128 || DECAY == kSelective || columns <= 8ull * (uint64_t)ctx->cu_count)) {
+        const dim3 blocks((uint32_t)((columns + 3) / 4));
+#define LH_REC(NR_, AHEAD_) hipLaunchKernelGGL((recurrent_wide_kernel<T, NR_, AHEAD_, DECAY>), blocks, dim3(256), 0, ctx->stream, a)
+        if (a.dq <= 128) { if (a.rows < 8) LH_REC(2, 4); else LH_REC(2, 16); }
+        else if (a.dq <= 256) { if (a.rows < 8) LH_REC(4, 4); else LH_REC(4, 8); }
+        else LH_REC(8, 4);
+#undef LH_REC
+        return lh_check_launch(op);
+    }
+    if (a.rows >= 8 && whole) {
 #define LH_REC(NR_, AHEAD_) hipLaunchKernelGGL((recurrent_rows_kernel<T, NR_, AHEAD_, DECAY>), dim3((uint32_t)grid), dim3(256), 0, ctx->stream, a)
         if (a.dq <= 32) LH_REC(2, 8);
         else if (a.dq <= 64) LH_REC(4, 8);
-        else if (a.dq <= 128) LH_REC(8, 8);
-        else if (a.dq <= 256) LH_REC(16, 4);
-        else if (a.dq <= 512) LH_REC(32, 2);
+        else if (a.dq <= 128) { if constexpr (DECAY != kSelective) LH_REC(8, 8); }
         else LH_REC(64, 1);
 #undef LH_REC
         return lh_check_launch(op);
