@@ -619,6 +619,19 @@ LH_API int lh_flash_attention_tq_rotated_lazy_into(lh_batch* batch, const lh_buf
                                                    uint32_t head_dim, uint32_t kv_len, uint32_t current_pos,
                                                    uint32_t num_q_heads, uint32_t num_kv_heads, uint32_t window,
                                                    uint32_t bits, uint32_t ring_capacity, int* rotated);
+/* lh_matmul_nt_qkv_prepare_rows_into for `lanes` tokens at positions[lane] (without key and value projections:
+ * lh_matmul_nt_q_prepare_rows_into) and lh_flash_attention_tq_batched_rotated_into behind it as one step: over a short span
+ * (a sliding window) preparation, attention and rotation are one launch.  q, k, v are left prepared, `rq` and `out` hold
+ * the rotated queries and the heads in code space only where those are launches of their own. */
+LH_API int lh_matmul_nt_qkv_attention_lanes_into(lh_batch* batch, lh_quant fmt, const lh_buffer* input, const lh_buffer* w_q,
+                                                 const lh_buffer* w_k, const lh_buffer* w_v, uint32_t k_dim, lh_buffer* q,
+                                                 lh_buffer* k, lh_buffer* v, const lh_buffer* q_norm, const lh_buffer* k_norm,
+                                                 const lh_buffer* levels, const lh_buffer* signs, lh_buffer* rq,
+                                                 lh_buffer* k_codes, lh_buffer* k_norms, lh_buffer* v_codes, lh_buffer* v_norms,
+                                                 const lh_buffer* positions, lh_buffer* out, lh_buffer* out_f16,
+                                                 uint32_t head_dim, uint32_t n_q_heads, uint32_t n_kv_heads, uint32_t lanes,
+                                                 float eps, float theta, float partial_rotary_factor, uint32_t window,
+                                                 uint32_t bits, uint32_t ring_capacity, uint32_t lane_capacity);
 /* lh_decode_qkv_prepare_into and lh_flash_attention_tq_rotated_lazy_into (with `rotated` NULL: _rotated_into) of a decoded
  * token at `position` as one step, which is one launch where the span is short (a sliding window): the heads are
  * taken from q_raw / k_raw / v_raw and left behind norm and rotary embedding in q / k / v (the same buffers, or NULL for

@@ -801,6 +801,18 @@ class Kernels:
                                                                _u32(bits), _u32(ring_capacity), C.byref(rotated)))
         return bool(rotated.value)
 
+    def matmul_nt_qkv_attention_lanes_into(self, batch, weight_type, input, w_q, w_k, w_v, k_dim, q, k, v, q_norm, k_norm, levels, signs, rq, k_codes, k_norms,
+                                           v_codes, v_norms, positions, out, out_f16, head_dim, n_q_heads, n_kv_heads, lanes, eps, theta,
+                                           partial_rotary_factor, window, bits, ring_capacity, lane_capacity):
+        """The projections of one token of every lane, their preparation, the attention over the lanes' codes and the rotation of the heads to
+        f16 as one step; w_k = w_v = k = v = None for a layer that reads another's cache."""
+        def h(b):
+            return b._h if b is not None else None
+        _check(self._l.lh_matmul_nt_qkv_attention_lanes_into(
+            batch._h, C.c_int(weight_type), input._h, w_q._h, h(w_k), h(w_v), _u32(k_dim), q._h, h(k), h(v), h(q_norm), h(k_norm), levels._h, signs._h, rq._h,
+            k_codes._h, k_norms._h, v_codes._h, v_norms._h, positions._h, out._h, out_f16._h, _u32(head_dim), _u32(n_q_heads), _u32(n_kv_heads), _u32(lanes),
+            C.c_float(eps), C.c_float(theta), C.c_float(partial_rotary_factor), _u32(window), _u32(bits), _u32(ring_capacity), _u32(lane_capacity)))
+
     def token_attention_tq_into(self, batch, raw, q, k, v, q_norm, k_norm, levels, signs, rq, k_codes, k_norms, v_codes, v_norms, out,
                                 out_f16, head_dim, num_q_heads, num_kv_heads, eps, position, theta, partial_rotary_factor, window, bits,
                                 ring_capacity, lazy) -> bool:

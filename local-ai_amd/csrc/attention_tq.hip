@@ -424,7 +424,7 @@ bool token_preparation(const lh_context* ctx, const AttnParams& p, const AttnPoi
     t = TokenPrep{ptr(a.q_raw), kv ? ptr(a.k_raw) : nullptr, kv ? ptr(a.v_raw) : nullptr, prep.partial, prep.splits, a.rows, prep.part_cols, ptr(a.q), kv ? ptr(a.k) : nullptr,
                   kv ? ptr(a.v) : nullptr, ptr(a.q_norm), kv ? ptr(a.k_norm) : nullptr, (const float*)a.signs->ptr, kv ? (uint8_t*)a.k_codes->ptr : nullptr,
                   kv ? (uint8_t*)a.v_codes->ptr : nullptr, kv ? ptr(a.k_norms) : nullptr, kv ? ptr(a.v_norms) : nullptr, a.eps, a.theta, a.partial_rotary_factor,
-                  1.0f / std::sqrt((float)p.head_dim)};
+                  1.0f / std::sqrt((float)p.head_dim), nullptr};
     if (p.mode == kPrefill || p.head_dim != a.head_dim || p.num_q_heads != a.n_q_heads || (kv && p.num_kv_heads != a.n_kv_heads) || p.num_queries != a.rows) return false;
     // Every workgroup of a query reads its raw rows while the first one stores the prepared ones.
     const size_t q_bytes = (size_t)a.rows * a.n_q_heads * a.head_dim * 2, kv_bytes = (size_t)a.rows * a.n_kv_heads * a.head_dim * 2;
@@ -471,6 +471,7 @@ int attention_dispatch(lh_batch* batch, const char* op, const lh_buffer* rq, con
                             positions ? (const uint32_t*)positions->ptr : nullptr, (float*)out->ptr, ws, ctx->fault_dev};
     TokenPrep token{};
     const bool in_one = prep && token_preparation(ctx, p, ptrs, *prep, max_span, token);
+    if (in_one && rot && !rot->rotated) token.rotated = (uint16_t*)rot->out16->ptr;
     if (prep && !in_one) {
         const int rp = lh_prepare_rows_launch(batch, prep->rows, prep->partial, prep->splits, prep->part_cols);
         if (rp != LH_OK) return rp;
@@ -515,6 +516,7 @@ int attention_dispatch(lh_batch* batch, const char* op, const lh_buffer* rq, con
     int r = lh_check_launch(op);
     if (r != LH_OK) return r;
     batch->dispatch_count++;
+    if (token.rotated) return r;
     if (rot && p.num_splits > 1 && p.num_splits <= 2 * kReduceBatch) {
         hipLaunchKernelGGL(attention_tq_reduce_rotate_kernel, dim3(p.num_queries * p.num_q_heads), dim3(p.head_dim), 0, ctx->stream,
                            (const float*)ws, (const float*)rot->signs->ptr, (uint16_t*)rot->out16->ptr, p.head_dim, p.num_splits,
@@ -695,7 +697,7 @@ static int batched_common(const char* op, lh_batch* batch, const lh_buffer* rq, 
                           const lh_buffer* v_codes, const lh_buffer* v_norms, const lh_buffer* levels, lh_buffer* out,
                           const lh_buffer* positions, uint32_t head_dim, uint32_t lane_capacity, uint32_t num_q_heads,
                           uint32_t num_kv_heads, uint32_t window, uint32_t bits, uint32_t n_lanes, uint32_t ring_capacity,
-                          const RotateBack* rot) {
+                          const RotateBack* rot, const Preparation* prep = nullptr) {
     AttnParams p{};
     p.head_dim = head_dim; p.bits = bits; p.num_q_heads = num_q_heads; p.num_kv_heads = num_kv_heads;
     p.window = window; p.ring_capacity = ring_capacity; p.lane_capacity = lane_capacity; p.mode = kBatched; p.num_queries = n_lanes;
@@ -705,7 +707,7 @@ static int batched_common(const char* op, lh_batch* batch, const lh_buffer* rq, 
     const uint64_t cap = ring_capacity ? ring_capacity : lane_capacity;
     const uint64_t span = window ? std::min<uint64_t>(window, cap) : cap;
     const uint64_t phys = (uint64_t)n_lanes * lane_capacity * num_kv_heads;
-    return attention_dispatch(batch, op, rq, k_codes, k_norms, v_codes, v_norms, levels, out, positions, p, span, phys, rot);
+    return attention_dispatch(batch, op, rq, k_codes, k_norms, v_codes, v_norms, levels, out, positions, p, span, phys, rot, nullptr, 0, prep);
 }
 
 int lh_flash_attention_tq_batched_into(lh_batch* batch, const lh_buffer* rq, const lh_buffer* k_codes, const lh_buffer* k_norms,
@@ -727,3 +729,10 @@ int lh_flash_attention_tq_batched_rotated_into(lh_batch* batch, const lh_buffer*
 }
 
 }  // extern "C"
+
+int lh_attend_lanes(lh_batch* batch, const LhPrepareRows& a, const float* partial, uint32_t splits, uint32_t part_cols, const LhAttendLanes& t, const char* op) {
+    const RotateBack rot{a.signs, t.out_f16};
+    const Preparation prep{a, partial, splits, part_cols};
+    return batched_common(op, batch, a.rq, t.k_codes, t.k_norms, t.v_codes, t.v_norms, t.levels, t.out, a.positions, a.head_dim, a.lane_capacity, a.n_q_heads,
+                          t.n_kv_heads, t.window, a.bits, a.rows, a.ring_capacity, &rot, &prep);
+}

@@ -71,6 +71,7 @@ struct TokenPrep {
     uint8_t *k_codes, *v_codes;          // null: the query alone, on a cache that has the position already
     uint16_t *k_norms, *v_norms;
     float eps, theta, prf, inv_sqrt_d;
+    uint16_t* rotated;                   // not null: the heads as f16 behind the rotation out of code space, instead of `out`
 };
 // What short_supported takes, with room for the two waves that bring in the query's own key and value, on a cache where that position's slot is
 // no other's of the span.

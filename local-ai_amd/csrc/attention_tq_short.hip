@@ -16,6 +16,7 @@
 #include "attention_tq.hpp"
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace {
 using namespace lh_attn;
@@ -54,9 +55,29 @@ struct ShortWave {
 template <int S>
 struct Group { u32x4_t k[4], v[4 / S]; uint32_t nk, nv; uint32_t lo, hi; };
 
-template <int NPL, int S, class Load>
+// Walsh-Hadamard transform of a head in a wave, a lane with dims lane + 64 j, pairs as in lh_fwht_lds.
+__device__ __forceinline__ void transform_head(float (&v)[4], uint32_t lane) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        v[j] = lh_fwht_lane_stage<1>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<2>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<4>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<8>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<16>(v[j], lane);
+        v[j] = lh_fwht_lane_stage<32>(v[j], lane);
+    }
+    const float a = __fadd_rn(v[0], v[1]), b = __fsub_rn(v[0], v[1]), c = __fadd_rn(v[2], v[3]), d = __fsub_rn(v[2], v[3]);
+    v[0] = __fadd_rn(a, c); v[2] = __fsub_rn(a, c);
+    v[1] = __fadd_rn(b, d); v[3] = __fsub_rn(b, d);
+}
+
+// Where finished heads go as f16 behind the rotation out of code space, as hadamard_rotate_kernel makes it (a workgroup with all dims of a query).
+struct RotateOut { uint16_t* out; const float (&sign)[4]; float inv_sqrt_d; };
+struct NoRotation {};
+
+template <int NPL, int S, class Load, class Rotation>
 __device__ __forceinline__ void short_body(const AttnPointers& a, const AttnParams& p, ShortShared& sh, ShortWave<S>& mine, Group<S> gr, uint32_t G, uint32_t g_last, Load load,
-                                           float alpha, float beta, float gam, float delta, uint32_t qi, uint32_t kvh, uint32_t group, uint32_t nwaves, uint32_t parts) {
+                                           float alpha, float beta, float gam, float delta, uint32_t qi, uint32_t kvh, uint32_t group, uint32_t nwaves, uint32_t parts, const Rotation& rotation) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), pcol = lane & 15, g = lane >> 4;
     constexpr int E = 4 / S;              // chunks of 16 code bytes, 64 dims
     const float cmax = fmaxf(fmaxf(fabsf(beta), fabsf(0.5f * gam)), NPL == 3 ? fabsf(delta) : 0.0f), inv_cmax = cmax > 0.0f ? 1.0f / cmax : 0.0f;
@@ -276,9 +297,18 @@ __device__ __forceinline__ void short_body(const AttnPointers& a, const AttnPara
         }
     }
     const float total = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(l)));
-    float* const dst = a.out + ((size_t)qi * p.num_q_heads + kvh * group + wave) * kDim + kDim / S * blockIdx.x + lane;
+    const size_t at = ((size_t)qi * p.num_q_heads + kvh * group + wave) * kDim + kDim / S * blockIdx.x + lane;
 #pragma unroll
-    for (int e = 0; e < E; e++) dst[64 * e] = total > 0.0f ? o[e] / total : 0.0f;
+    for (int e = 0; e < E; e++) o[e] = total > 0.0f ? o[e] / total : 0.0f;
+    if constexpr (std::is_same_v<Rotation, RotateOut>) {
+        static_assert(E == 4, "all dims of a head");
+        transform_head(o, lane);
+#pragma unroll
+        for (int e = 0; e < E; e++) rotation.out[at + 64 * e] = lh_f2h_exact(__fmul_rn(__fmul_rn(o[e], rotation.inv_sqrt_d), rotation.sign[e]));
+    } else {
+#pragma unroll
+        for (int e = 0; e < E; e++) a.out[at + 64 * e] = o[e];
+    }
 }
 
 // The codes and norms of group G_ of positions [lo, hi).  Lanes whose position is not visible read one that is: nothing of it is used (its weight is zero).
@@ -302,12 +332,12 @@ __device__ __forceinline__ Group<S> load_group(const AttnPointers& a, const Attn
 }
 
 // L[c] = alpha + beta bit0 + gam bit1 + delta bit0 bit1: as in attention_tq_mfma_kernel
-template <int S, class Load>
+template <int S, class Load, class Rotation>
 __device__ __forceinline__ void short_by_levels(const AttnPointers& a, const AttnParams& p, ShortShared& sh, ShortWave<S>& mine, const Group<S>& first, uint32_t begin, uint32_t end, Load load,
-                                                float L0, float L1, float L2, float L3, uint32_t qi, uint32_t kvh, uint32_t group, uint32_t nwaves, uint32_t parts) {
+                                                float L0, float L1, float L2, float L3, uint32_t qi, uint32_t kvh, uint32_t group, uint32_t nwaves, uint32_t parts, const Rotation& rotation) {
     const float d_raw = (L3 - L2) - (L1 - L0), lmax = fmaxf(fmaxf(fabsf(L0), fabsf(L1)), fmaxf(fabsf(L2), fabsf(L3))), l_mean = 0.25f * ((L0 + L3) + (L1 + L2));
-    if (fabsf(d_raw) > 1e-5f * lmax || fabsf(l_mean) > 1e-6f * lmax) short_body<3, S>(a, p, sh, mine, first, begin, end, load, L0, L1 - L0, L2 - L0, d_raw, qi, kvh, group, nwaves, parts);
-    else short_body<2, S>(a, p, sh, mine, first, begin, end, load, L0 - 0.25f * d_raw, (L1 - L0) + 0.5f * d_raw, (L2 - L0) + 0.5f * d_raw, 0.0f, qi, kvh, group, nwaves, parts);
+    if (fabsf(d_raw) > 1e-5f * lmax || fabsf(l_mean) > 1e-6f * lmax) short_body<3, S>(a, p, sh, mine, first, begin, end, load, L0, L1 - L0, L2 - L0, d_raw, qi, kvh, group, nwaves, parts, rotation);
+    else short_body<2, S>(a, p, sh, mine, first, begin, end, load, L0 - 0.25f * d_raw, (L1 - L0) + 0.5f * d_raw, (L2 - L0) + 0.5f * d_raw, 0.0f, qi, kvh, group, nwaves, parts, rotation);
 }
 
 __device__ __forceinline__ float level_of(float table, int i) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(table), i)); }
@@ -343,7 +373,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_short_kernel(cons
     }
     lh_lds_barrier();
     short_by_levels<S>(a, p, sh, mine, first, none ? 1u : G, none ? 0u : g_last, load, level_of(table, 0), level_of(table, 1), level_of(table, 2), level_of(table, 3), qi, kvh, group,
-                       nwaves, nwaves);
+                       nwaves, nwaves, NoRotation{});
 }
 
 // ---- the query's own preparation in the same launch -------------------------------------------------------------------------------
@@ -381,21 +411,6 @@ __device__ __forceinline__ void turn_head(uint16_t (&h)[4], const float2* turn, 
         const float2 t = turn[lane + 64 * j];
         lh_rope_apply(lh_h2f(h[j]), lh_h2f(h[j + 2]), t.x, t.y, h[j], h[j + 2]);
     }
-}
-// Walsh-Hadamard transform of a head, pairs as in lh_fwht_lds.
-__device__ __forceinline__ void transform_head(float (&v)[4], uint32_t lane) {
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        v[j] = lh_fwht_lane_stage<1>(v[j], lane);
-        v[j] = lh_fwht_lane_stage<2>(v[j], lane);
-        v[j] = lh_fwht_lane_stage<4>(v[j], lane);
-        v[j] = lh_fwht_lane_stage<8>(v[j], lane);
-        v[j] = lh_fwht_lane_stage<16>(v[j], lane);
-        v[j] = lh_fwht_lane_stage<32>(v[j], lane);
-    }
-    const float a = __fadd_rn(v[0], v[1]), b = __fsub_rn(v[0], v[1]), c = __fadd_rn(v[2], v[3]), d = __fsub_rn(v[2], v[3]);
-    v[0] = __fadd_rn(a, c); v[2] = __fsub_rn(a, c);
-    v[1] = __fadd_rn(b, d); v[3] = __fsub_rn(b, d);
 }
 // The codes of a head and its norm, as encode_vector makes them (turboquant_kv.hip): the squares, their sum from left to right as the CPU
 // encoder has it, the rest.
@@ -438,7 +453,7 @@ __device__ __forceinline__ uint16_t encode_head(const uint16_t (&h)[4], float su
 }
 
 // The leading arguments arrive in registers with the wave (see the Makefile); the structures repeat them.
-template <int S, bool OWN>
+template <int S, bool OWN, bool ROTATE>
 __global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_token_kernel(const float* levels, const float* signs, uint32_t q_heads, uint32_t kv_heads, const AttnPointers a,
                                                                             const AttnParams p, const TokenPrep t) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -535,7 +550,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_token_kernel(cons
     lh_lds_barrier();
     const float L0 = level_of(table, 0), L1 = level_of(table, 1), L2 = level_of(table, 2), L3 = level_of(table, 3);
     if (!own) {
-        short_by_levels<S>(a, p, sh, all[wave], first, none ? 1u : G, none ? 0u : g_last, load, L0, L1, L2, L3, qi, kvh, group, nwaves, OWN ? nwaves + 1 : nwaves);
+        const uint32_t parts = OWN ? nwaves + 1 : nwaves;
+        if constexpr (ROTATE) short_by_levels<S>(a, p, sh, all[wave], first, none ? 1u : G, none ? 0u : g_last, load, L0, L1, L2, L3, qi, kvh, group, nwaves, parts, RotateOut{t.rotated, sign, t.inv_sqrt_d});
+        else short_by_levels<S>(a, p, sh, all[wave], first, none ? 1u : G, none ? 0u : g_last, load, L0, L1, L2, L3, qi, kvh, group, nwaves, parts, NoRotation{});
         return;
     }
     if constexpr (OWN) {
@@ -598,11 +615,11 @@ int launch(lh_context* ctx, const char* op, const AttnPointers& a, const AttnPar
 
 template <int S> constexpr size_t token_lds(uint32_t waves) { return sizeof(TokenShared) + short_lds<S>(waves); }
 
-template <int S>
+template <int S, bool ROTATE = false>
 int launch_token_form(lh_context* ctx, const char* op, const AttnPointers& a, const AttnParams& p, const TokenPrep& t, uint32_t waves) {
     const dim3 grid(S, p.num_queries * p.num_kv_heads);
-    if (t.k_codes) hipLaunchKernelGGL((attention_tq_token_kernel<S, true>), grid, dim3(64 * (waves + 2)), token_lds<S>(waves + 2), ctx->stream, a.levels, t.signs, p.num_q_heads, p.num_kv_heads, a, p, t);
-    else hipLaunchKernelGGL((attention_tq_token_kernel<S, false>), grid, dim3(64 * waves), token_lds<S>(waves), ctx->stream, a.levels, t.signs, p.num_q_heads, p.num_kv_heads, a, p, t);
+    if (t.k_codes) hipLaunchKernelGGL((attention_tq_token_kernel<S, true, ROTATE>), grid, dim3(64 * (waves + 2)), token_lds<S>(waves + 2), ctx->stream, a.levels, t.signs, p.num_q_heads, p.num_kv_heads, a, p, t);
+    else hipLaunchKernelGGL((attention_tq_token_kernel<S, false, ROTATE>), grid, dim3(64 * waves), token_lds<S>(waves), ctx->stream, a.levels, t.signs, p.num_q_heads, p.num_kv_heads, a, p, t);
     return lh_check_launch(op);
 }
 
@@ -612,12 +629,15 @@ int lh_attention_short_init(lh_context* ctx) {
     int r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<4>, short_lds<4>(kMaxWaves), "context_create");
     if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<2>, short_lds<2>(kMaxWaves), "context_create");
     if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_short_kernel<1>, short_lds<1>(kMaxWaves), "context_create");
-    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<4, true>, token_lds<4>(kMaxWaves), "context_create");
-    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<4, false>, token_lds<4>(kMaxWaves), "context_create");
-    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<2, true>, token_lds<2>(kMaxWaves), "context_create");
-    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<2, false>, token_lds<2>(kMaxWaves), "context_create");
-    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<1, true>, token_lds<1>(kMaxWaves), "context_create");
-    if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)attention_tq_token_kernel<1, false>, token_lds<1>(kMaxWaves), "context_create");
+    const auto raise = [&](auto kernel, size_t bytes) { if (r == LH_OK) r = lh_raise_dynamic_lds(ctx, (const void*)kernel, bytes, "context_create"); };
+    raise(attention_tq_token_kernel<4, true, false>, token_lds<4>(kMaxWaves));
+    raise(attention_tq_token_kernel<4, false, false>, token_lds<4>(kMaxWaves));
+    raise(attention_tq_token_kernel<2, true, false>, token_lds<2>(kMaxWaves));
+    raise(attention_tq_token_kernel<2, false, false>, token_lds<2>(kMaxWaves));
+    raise(attention_tq_token_kernel<1, true, false>, token_lds<1>(kMaxWaves));
+    raise(attention_tq_token_kernel<1, false, false>, token_lds<1>(kMaxWaves));
+    raise(attention_tq_token_kernel<1, true, true>, token_lds<1>(kMaxWaves));
+    raise(attention_tq_token_kernel<1, false, true>, token_lds<1>(kMaxWaves));
     return r;
 }
 
@@ -649,6 +669,9 @@ bool token_supported(const lh_context* ctx, const AttnParams& p, const TokenPrep
 int launch_token(lh_context* ctx, const char* op, const AttnPointers& a, AttnParams& p, const TokenPrep& t, uint64_t max_span) {
     p.num_splits = 1;
     const uint32_t waves = group_waves(t.k_codes ? max_span - 1 : max_span), queries = p.num_queries * p.num_kv_heads, cus = (uint32_t)ctx->cu_count;
+    // A workgroup with all dims of a query can rotate its heads, which is worth the other dims' products in it: 64 lanes, window of 512, 14.5 us in one launch (14.2 on
+    // another layer's cache) against 20.6 (18.3) for preparation, attention on four CUs a lane and rotation, two gaps not counted.
+    if (t.rotated) return launch_token_form<1, true>(ctx, op, a, p, t, waves);
     return queries * 4 <= cus ? launch_token_form<4>(ctx, op, a, p, t, waves) : queries * 2 <= cus ? launch_token_form<2>(ctx, op, a, p, t, waves) : launch_token_form<1>(ctx, op, a, p, t, waves);
 }
 

@@ -1663,6 +1663,47 @@ int matmul_dispatch(lh_batch* batch, const char* op, int kind, const lh_buffer* 
     return r;
 }
 
+// The Q, K and V projections of rows where lh_matmul_nt_quant_grouped_into sends them to the decode-batch kernel as one launch: their partial tiles
+// stay in the workspace for the preparation.  False: nothing is launched.
+bool keep_qkv(lh_context* ctx, lh_quant fmt, const lh_buffer* in, const lh_buffer* const (&ws)[3], const uint32_t (&ns)[3], uint32_t m, uint32_t k, SkinnyPartials& kept) {
+    const int kind = fmt == LH_Q4_0 ? kQ4 : kTQ2;
+    const uint32_t blk = fmt == LH_Q4_0 ? 32 : 256;
+    uint64_t tiles_n = 0;
+    bool whole = true;
+    for (uint32_t i = 0; i < 3; i++) { tiles_n += (ns[i] + BN - 1) / BN; whole = whole && ns[i] % BN == 0; }
+    const uint64_t tiles128 = tiles_n * ((m + 127) / 128);
+    const bool small = m <= (uint32_t)kMaxMultivecM;
+    const bool together = (!small || m >= skinny_min_m(kind)) && !(m > 64 && tiles128 * 2 >= (uint64_t)ctx->cu_count);
+    if (!together || !whole || k % blk != 0 || ((uintptr_t)in->ptr & 15) != 0 || in->len < (size_t)m * k * 2) return false;
+    GroupArgs grp{};
+    grp.count = 3;
+    uint32_t tile = 0;
+    for (uint32_t i = 0; i < 3; i++) {
+        const size_t wbytes = fmt == LH_Q4_0 ? (size_t)ns[i] * (k / 32) * 18 : (size_t)ns[i] * (k / 256) * 66;
+        if (ws[i]->len < wbytes || ((uintptr_t)ws[i]->ptr & 1) != 0) return false;
+        grp.W[i] = (const uint8_t*)ws[i]->ptr; grp.N[i] = ns[i];
+        grp.tile0[i] = tile;
+        tile += ns[i] / BN;
+    }
+    for (uint32_t i = 3; i <= 4; i++) grp.tile0[i] = tile;
+    const ClipArgs none{nullptr, 0.f, 0.f, 0.f, 0.f, 0u};
+    return fmt == LH_Q4_0 ? try_skinny<kQ4, LH_F16>(ctx, in->ptr, grp.W[0], nullptr, LH_F16, m, k, grp.N[0], none, grp, &kept)
+                          : try_skinny<kTQ2, LH_F16>(ctx, in->ptr, grp.W[0], nullptr, LH_F16, m, k, grp.N[0], none, grp, &kept);
+}
+
+// The same for the queries alone: the shapes whose product matmul_dispatch gives the decode-batch kernel, and only where that splits k.
+bool keep_queries(lh_context* ctx, lh_quant fmt, const lh_buffer* in, const lh_buffer* w_q, uint32_t n, uint32_t m, uint32_t k, SkinnyPartials& kept) {
+    const int kind = fmt == LH_Q4_0 ? kQ4 : kTQ2;
+    const uint32_t unit = fmt == LH_Q4_0 ? Skinny<kQ4>::unit_k : Skinny<kTQ2>::unit_k;
+    const size_t wbytes = fmt == LH_Q4_0 ? (size_t)n * (k / 32) * 18 : (size_t)n * (k / 256) * 66;
+    if (m < skinny_min_m(kind) || n % BN != 0 || k % (4 * unit) != 0 || ((uintptr_t)in->ptr & 15) != 0 || in->len < (size_t)m * k * 2 || ((uintptr_t)w_q->ptr & 1) != 0 ||
+        w_q->len < wbytes || skinny_splits(ctx, m, n / 64 * ((m + 63) / 64), k / unit / 4) <= 1) return false;
+    const ClipArgs none{nullptr, 0.f, 0.f, 0.f, 0.f, 0u};
+    const uint8_t* W = (const uint8_t*)w_q->ptr;
+    return kind == kQ4 ? try_skinny<kQ4, LH_F16>(ctx, in->ptr, W, nullptr, LH_F16, m, k, n, none, GroupArgs{}, &kept)
+                       : try_skinny<kTQ2, LH_F16>(ctx, in->ptr, W, nullptr, LH_F16, m, k, n, none, GroupArgs{}, &kept);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1886,37 +1927,8 @@ int lh_matmul_nt_qkv_prepare_rows_into(lh_batch* b, lh_quant fmt, const lh_buffe
     const lh_buffer* const ws[3] = {w_q, w_k, w_v};
     lh_buffer* const outs[3] = {q, k, v};
     const uint32_t ns[3] = {n_q_heads * head_dim, n_kv_heads * head_dim, n_kv_heads * head_dim};
-    lh_context* ctx = b->ctx;
-    const int kind = fmt == LH_Q4_0 ? kQ4 : kTQ2;
-    const uint32_t blk = fmt == LH_Q4_0 ? 32 : 256, m = rows;
-    // The shapes that lh_matmul_nt_quant_grouped_into sends to the decode-batch kernel as one launch can leave their partial
-    // tiles to the preparation; every other shape runs as that entry point followed by the preparation.
-    uint64_t tiles_n = 0;
-    bool whole = true;
-    for (uint32_t i = 0; i < 3; i++) { tiles_n += (ns[i] + BN - 1) / BN; whole = whole && ns[i] % BN == 0; }
-    const uint64_t tiles128 = tiles_n * ((m + 127) / 128);
-    const bool small = m <= (uint32_t)kMaxMultivecM;
-    const bool together = (!small || m >= skinny_min_m(kind)) && !(m > 64 && tiles128 * 2 >= (uint64_t)ctx->cu_count);
-    bool fused = false;
     SkinnyPartials kept{nullptr, 0, 0};
-    if (together && whole && k_dim % blk == 0 && ((uintptr_t)in->ptr & 15) == 0 && in->len >= (size_t)m * k_dim * 2) {
-        GroupArgs grp{};
-        grp.count = 3;
-        uint32_t tile = 0;
-        bool fits = true;
-        for (uint32_t i = 0; i < 3; i++) {
-            const size_t wbytes = fmt == LH_Q4_0 ? (size_t)ns[i] * (k_dim / 32) * 18 : (size_t)ns[i] * (k_dim / 256) * 66;
-            fits = fits && ws[i]->len >= wbytes && ((uintptr_t)ws[i]->ptr & 1) == 0;
-            grp.W[i] = (const uint8_t*)ws[i]->ptr; grp.C[i] = outs[i]->ptr; grp.N[i] = ns[i];
-            grp.tile0[i] = tile;
-            tile += ns[i] / BN;
-        }
-        for (uint32_t i = 3; i <= 4; i++) grp.tile0[i] = tile;
-        const ClipArgs none{nullptr, 0.f, 0.f, 0.f, 0.f, 0u};
-        if (fits)
-            fused = fmt == LH_Q4_0 ? try_skinny<kQ4, LH_F16>(ctx, in->ptr, grp.W[0], grp.C[0], LH_F16, m, k_dim, grp.N[0], none, grp, &kept)
-                                   : try_skinny<kTQ2, LH_F16>(ctx, in->ptr, grp.W[0], grp.C[0], LH_F16, m, k_dim, grp.N[0], none, grp, &kept);
-    }
+    const bool fused = keep_qkv(b->ctx, fmt, in, ws, ns, rows, k_dim, kept);
     if (fused) {
         r = lh_check_launch(op);
         if (r != LH_OK) return r;
@@ -1941,24 +1953,64 @@ int lh_matmul_nt_q_prepare_rows_into(lh_batch* b, lh_quant fmt, const lh_buffer*
     int r = lh_prepare_rows_launch(b, a, nullptr, 0, 0, true);   // the second half's arguments, before anything is launched
     if (r != LH_OK) return r;
     if (rows == 0 || k_dim == 0) return LH_OK;
-    lh_context* ctx = b->ctx;
     const int kind = fmt == LH_Q4_0 ? kQ4 : kTQ2;
-    const uint32_t n = n_q_heads * head_dim, unit = fmt == LH_Q4_0 ? Skinny<kQ4>::unit_k : Skinny<kTQ2>::unit_k;
-    const size_t wbytes = fmt == LH_Q4_0 ? (size_t)n * (k_dim / 32) * 18 : (size_t)n * (k_dim / 256) * 66;
-    // the shapes whose product matmul_dispatch gives the decode-batch kernel, and only where that splits k
-    if (rows >= skinny_min_m(kind) && n % BN == 0 && k_dim % (4 * unit) == 0 && ((uintptr_t)in->ptr & 15) == 0 && in->len >= (size_t)rows * k_dim * 2 &&
-        ((uintptr_t)w_q->ptr & 1) == 0 && w_q->len >= wbytes && skinny_splits(ctx, rows, n / 64 * ((rows + 63) / 64), k_dim / unit / 4) > 1) {
-        SkinnyPartials kept{nullptr, 0, 0};
-        const ClipArgs none{nullptr, 0.f, 0.f, 0.f, 0.f, 0u};
-        const uint8_t* W = (const uint8_t*)w_q->ptr;
-        if (kind == kQ4 ? try_skinny<kQ4, LH_F16>(ctx, in->ptr, W, nullptr, LH_F16, rows, k_dim, n, none, GroupArgs{}, &kept)
-                        : try_skinny<kTQ2, LH_F16>(ctx, in->ptr, W, nullptr, LH_F16, rows, k_dim, n, none, GroupArgs{}, &kept)) {
-            r = lh_check_launch(op);
-            return r != LH_OK ? r : lh_prepare_rows_launch(b, a, kept.partial, kept.splits, kept.cols);
-        }
+    const uint32_t n = n_q_heads * head_dim;
+    SkinnyPartials kept{nullptr, 0, 0};
+    if (keep_queries(b->ctx, fmt, in, w_q, n, rows, k_dim, kept)) {
+        r = lh_check_launch(op);
+        return r != LH_OK ? r : lh_prepare_rows_launch(b, a, kept.partial, kept.splits, kept.cols);
     }
     r = matmul_dispatch(b, op, kind, in, LH_F16, w_q, q, LH_F16, rows, k_dim, n, false);
     return r != LH_OK ? r : lh_prepare_rows_launch(b, a, nullptr, 0, 0);
+}
+
+// A step of several sequences was the product, its tiles' preparation (7.6 us; 5.3 without keys and values), the attention (10.2) and the rotation of the
+// heads (2.8), each waiting for the one before; over a window the last three are one launch now.
+int lh_matmul_nt_qkv_attention_lanes_into(lh_batch* b, lh_quant fmt, const lh_buffer* in, const lh_buffer* w_q, const lh_buffer* w_k, const lh_buffer* w_v, uint32_t k_dim,
+                                          lh_buffer* q, lh_buffer* k, lh_buffer* v, const lh_buffer* q_norm, const lh_buffer* k_norm, const lh_buffer* levels,
+                                          const lh_buffer* signs, lh_buffer* rq, lh_buffer* k_codes, lh_buffer* k_norms, lh_buffer* v_codes, lh_buffer* v_norms,
+                                          const lh_buffer* positions, lh_buffer* out, lh_buffer* out_f16, uint32_t head_dim, uint32_t n_q_heads, uint32_t n_kv_heads,
+                                          uint32_t lanes, float eps, float theta, float partial_rotary_factor, uint32_t window, uint32_t bits, uint32_t ring_capacity,
+                                          uint32_t lane_capacity) {
+    const char* op = fmt == LH_Q4_0 ? "matmul_nt_q4_0 (Q, K, V) + attention of lanes" : "matmul_nt_tq2_0 (Q, K, V) + attention of lanes";
+    if (!b) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: batch is null", op);
+    if (fmt != LH_Q4_0 && fmt != LH_TQ2_0) return lh_fail(LH_ERR_INVALID_ARGUMENT, "matmul_nt_quant: unknown weight format %d", (int)fmt);
+    const bool kv = w_k && w_v && k && v;
+    if (!in || !w_q || !q || !positions || n_q_heads == 0 || n_kv_heads == 0 || (!kv && (w_k || w_v || k || v)))
+        return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: needs the query projection, its output and the lanes' positions; the key and value projections and theirs, or none of them", op);
+    LhPrepareRows a{q, kv ? k : nullptr, kv ? v : nullptr, q_norm, kv ? k_norm : nullptr, kv ? levels : nullptr, signs, rq, kv ? k_codes : nullptr, kv ? k_norms : nullptr,
+                    kv ? v_codes : nullptr, kv ? v_norms : nullptr, positions, head_dim, n_q_heads, kv ? n_kv_heads : 0u, lanes, eps, 0, theta, partial_rotary_factor, bits,
+                    ring_capacity, lane_capacity};
+    int r = lh_prepare_rows_launch(b, a, nullptr, 0, 0, true);   // the second half's arguments, before anything is launched
+    if (r != LH_OK) return r;
+    if (lanes == 0 || k_dim == 0) return LH_OK;
+    const LhAttendLanes t{k_codes, k_norms, v_codes, v_norms, levels, out, out_f16, n_kv_heads, window};
+    const uint32_t ns[3] = {n_q_heads * head_dim, n_kv_heads * head_dim, n_kv_heads * head_dim};
+    const lh_buffer* const ws[3] = {w_q, w_k, w_v};
+    SkinnyPartials kept{nullptr, 0, 0};
+    if (kv ? keep_qkv(b->ctx, fmt, in, ws, ns, lanes, k_dim, kept) : keep_queries(b->ctx, fmt, in, w_q, ns[0], lanes, k_dim, kept)) {
+        r = lh_check_launch(op);
+        if (r != LH_OK) return r;
+        b->dispatch_count++;
+        return lh_attend_lanes(b, a, kept.partial, kept.splits, kept.cols, t, op);
+    }
+    // The rows of a finished product in the third quarter of the workspace, apart from where the prepared ones go.
+    lh_buffer raw[3] = {}, *outs[3] = {q, k, v};
+    size_t at = b->ctx->workspace_bytes / 2;
+    const size_t end = at + b->ctx->workspace_bytes / 4;
+    for (int i = 0; i < (kv ? 3 : 1); i++) {
+        raw[i].ctx = b->ctx;
+        raw[i].ptr = static_cast<uint8_t*>(b->ctx->workspace) + at;
+        raw[i].len = (size_t)lanes * ns[i] * 2;
+        at += (raw[i].len + 255) & ~(size_t)255;
+    }
+    if (at <= end) {
+        for (int i = 0; i < (kv ? 3 : 1); i++) outs[i] = &raw[i];
+        a.q_raw = &raw[0];
+        if (kv) { a.k_raw = &raw[1]; a.v_raw = &raw[2]; }
+    }
+    r = kv ? lh_matmul_nt_quant_grouped_into(b, fmt, 3, in, ws, outs, ns, lanes, k_dim) : matmul_dispatch(b, op, fmt == LH_Q4_0 ? kQ4 : kTQ2, in, LH_F16, w_q, outs[0], LH_F16, lanes, k_dim, ns[0], false);
+    return r != LH_OK ? r : lh_attend_lanes(b, a, nullptr, 0, 0, t, op);
 }
 
 int lh_matmul_nt_quant_gelu_mul_into(lh_batch* b, lh_quant fmt, const lh_buffer* in, const lh_buffer* w_gate, const lh_buffer* w_up,

@@ -295,6 +295,16 @@ class QuantizedUnifiedKvPool:
                                                         positions, hd, self.lane_stride(), n_q_heads, self.n_kv_heads,
                                                         window, self.bits, lanes, self.lane_ring_capacity)
 
+    def project_and_attend_lanes_into(self, batch, kernels: Kernels, w_q, w_k, w_v, x: Buffer, q: Buffer, k, v, q_norm, k_norm, rq: Buffer, vacc: Buffer,
+                                      attn_out: Buffer, positions: Buffer, active_lanes: int, n_q_heads: int, window: int, eps: float, theta: float,
+                                      partial_rotary_factor: float) -> None:
+        """``project_and_prepare_lanes_into`` (without key and value projections: ``project_queries_lanes_into``) and
+        ``attention_from_rotated_into`` as one encoded step."""
+        kernels.matmul_nt_qkv_attention_lanes_into(batch, w_q.ty, x, w_q.buf, w_k and w_k.buf, w_v and w_v.buf, w_q.cols, q, k, v, q_norm, k_norm, self.levels,
+                                                   self.signs, rq, self.keys_q, self.key_norms, self.values_q, self.value_norms, positions, vacc, attn_out,
+                                                   self.head_dim, n_q_heads, self.n_kv_heads, min(active_lanes, self.n_lanes), eps, theta,
+                                                   partial_rotary_factor, window, self.bits, self.lane_ring_capacity, self.lane_stride())
+
     def copy_prefill_from(self, batch, cache: QuantizedKvCache, lane: int, positions: int) -> None:
         """quant_unified_pool.rs:269-315: seed ``lane`` with the first ``positions`` rows of a single-sequence
         cache that shares the codec (a ringed pair copies the whole physical ring once it has wrapped).  Both

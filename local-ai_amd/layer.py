@@ -577,20 +577,11 @@ class TransformerLayer:
         one_prepare = self._one_prepare()
         if not prenormed:
             kernels.rms_norm_into(batch, input, w.attn_norm, bs.normed, h, rows, eps)
-        if own_kv and one_prepare and self._qkv_as_one():
-            # the three projections and the preparation as one step: the preparation sums the product's k-split tiles
-            pool.project_and_prepare_lanes_into(batch, kernels, w.attn_q.ty, bs.normed, w.attn_q.buf, w.attn_k.buf,
-                                                w.attn_v.buf, w.attn_q.cols, bs.q, bs.k, bs.v, w.q_norm, w.k_norm, bs.rq,
-                                                positions, n_lanes, n_head, eps, p.rope_theta, p.partial_rotary_factor)
-            pool.attention_from_rotated_into(batch, kernels, bs.rq, bs.vacc, bs.attn_out, positions, n_head,
-                                             p.sliding_window, n_lanes)
-            self._attention_tail(kernels, batch, rows, input, output, bs, ple_all, next_norm)
-            return
-        if not own_kv and one_prepare and self._queries_as_one():
-            pool.project_queries_lanes_into(batch, kernels, w.attn_q, bs.normed, bs.q, w.q_norm, bs.rq, positions, n_lanes, n_head, eps,
-                                            p.rope_theta, p.partial_rotary_factor)
-            pool.attention_from_rotated_into(batch, kernels, bs.rq, bs.vacc, bs.attn_out, positions, n_head,
-                                             p.sliding_window, n_lanes)
+        if one_prepare and (self._qkv_as_one() if own_kv else self._queries_as_one()):
+            # projections, preparation and attention as one step: what follows the product sums its k-split tiles
+            pool.project_and_attend_lanes_into(batch, kernels, w.attn_q, w.attn_k if own_kv else None, w.attn_v if own_kv else None, bs.normed, bs.q,
+                                               bs.k if own_kv else None, bs.v if own_kv else None, w.q_norm, w.k_norm, bs.rq, bs.vacc, bs.attn_out,
+                                               positions, n_lanes, n_head, p.sliding_window, eps, p.rope_theta, p.partial_rotary_factor)
             self._attention_tail(kernels, batch, rows, input, output, bs, ple_all, next_norm)
             return
         if own_kv:

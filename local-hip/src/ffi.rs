@@ -166,6 +166,7 @@ extern "C" {
     pub fn lh_flash_attention_tq_batched_into(batch: *mut lh_batch, rq: *const lh_buffer, k_codes: *const lh_buffer, k_norms: *const lh_buffer, v_codes: *const lh_buffer, v_norms: *const lh_buffer, levels: *const lh_buffer, out: *mut lh_buffer, positions: *const lh_buffer, head_dim: u32, lane_capacity: u32, num_q_heads: u32, num_kv_heads: u32, window: u32, bits: u32, n_lanes: u32, ring_capacity: u32) -> c_int;
     pub fn lh_flash_attention_tq_rotated_into(batch: *mut lh_batch, rq: *const lh_buffer, k_codes: *const lh_buffer, k_norms: *const lh_buffer, v_codes: *const lh_buffer, v_norms: *const lh_buffer, levels: *const lh_buffer, signs: *const lh_buffer, out: *mut lh_buffer, out_f16: *mut lh_buffer, head_dim: u32, kv_len: u32, current_pos: u32, num_q_heads: u32, num_kv_heads: u32, window: u32, bits: u32, ring_capacity: u32) -> c_int;
     pub fn lh_flash_attention_tq_rotated_lazy_into(batch: *mut lh_batch, rq: *const lh_buffer, k_codes: *const lh_buffer, k_norms: *const lh_buffer, v_codes: *const lh_buffer, v_norms: *const lh_buffer, levels: *const lh_buffer, signs: *const lh_buffer, out: *mut lh_buffer, out_f16: *mut lh_buffer, head_dim: u32, kv_len: u32, current_pos: u32, num_q_heads: u32, num_kv_heads: u32, window: u32, bits: u32, ring_capacity: u32, rotated: *mut c_int) -> c_int;
+    pub fn lh_matmul_nt_qkv_attention_lanes_into(batch: *mut lh_batch, fmt: lh_quant, input: *const lh_buffer, w_q: *const lh_buffer, w_k: *const lh_buffer, w_v: *const lh_buffer, k_dim: u32, q: *mut lh_buffer, k: *mut lh_buffer, v: *mut lh_buffer, q_norm: *const lh_buffer, k_norm: *const lh_buffer, levels: *const lh_buffer, signs: *const lh_buffer, rq: *mut lh_buffer, k_codes: *mut lh_buffer, k_norms: *mut lh_buffer, v_codes: *mut lh_buffer, v_norms: *mut lh_buffer, positions: *const lh_buffer, out: *mut lh_buffer, out_f16: *mut lh_buffer, head_dim: u32, n_q_heads: u32, n_kv_heads: u32, lanes: u32, eps: f32, theta: f32, partial_rotary_factor: f32, window: u32, bits: u32, ring_capacity: u32, lane_capacity: u32) -> c_int;
     pub fn lh_token_attention_tq_into(batch: *mut lh_batch, q_raw: *const lh_buffer, k_raw: *const lh_buffer, v_raw: *const lh_buffer, q: *mut lh_buffer, k: *mut lh_buffer, v: *mut lh_buffer, q_norm: *const lh_buffer, k_norm: *const lh_buffer, levels: *const lh_buffer, signs: *const lh_buffer, rq: *mut lh_buffer, k_codes: *mut lh_buffer, k_norms: *mut lh_buffer, v_codes: *mut lh_buffer, v_norms: *mut lh_buffer, out: *mut lh_buffer, out_f16: *mut lh_buffer, head_dim: u32, num_q_heads: u32, num_kv_heads: u32, eps: f32, position: u32, theta: f32, partial_rotary_factor: f32, window: u32, bits: u32, ring_capacity: u32, rotated: *mut c_int) -> c_int;
     pub fn lh_flash_attention_tq_batched_rotated_into(batch: *mut lh_batch, rq: *const lh_buffer, k_codes: *const lh_buffer, k_norms: *const lh_buffer, v_codes: *const lh_buffer, v_norms: *const lh_buffer, levels: *const lh_buffer, signs: *const lh_buffer, out: *mut lh_buffer, out_f16: *mut lh_buffer, positions: *const lh_buffer, head_dim: u32, lane_capacity: u32, num_q_heads: u32, num_kv_heads: u32, window: u32, bits: u32, n_lanes: u32, ring_capacity: u32) -> c_int;
     pub fn lh_flash_decoding_into(batch: *mut lh_batch, q: *const lh_buffer, k: *const lh_buffer, v: *const lh_buffer, output: *mut lh_buffer, head_dim: u32, kv_len: u32, current_pos: u32, num_q_heads: u32, num_kv_heads: u32) -> c_int;

@@ -504,6 +504,13 @@ impl Kernels {
         check(unsafe { ffi::lh_flash_attention_tq_rotated_into(batch.as_ptr(), rq.as_ptr(), k_codes.as_ptr(), k_norms.as_ptr(), v_codes.as_ptr(), v_norms.as_ptr(), levels.as_ptr(), signs.as_ptr(), out.as_ptr(), out_f16.as_ptr(), head_dim, kv_len, current_pos, num_q_heads, num_kv_heads, window, bits, ring_capacity) })
     }
 
+    /// `lh_matmul_nt_qkv_attention_lanes_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn matmul_nt_qkv_attention_lanes_into(&self, batch: &mut CommandBatch, fmt: ffi::lh_quant, input: &Buffer, w_q: &Buffer, w_k: &Buffer, w_v: &Buffer, k_dim: u32, q: &Buffer, k: &Buffer, v: &Buffer, q_norm: &Buffer, k_norm: &Buffer, levels: &Buffer, signs: &Buffer, rq: &Buffer, k_codes: &Buffer, k_norms: &Buffer, v_codes: &Buffer, v_norms: &Buffer, positions: &Buffer, out: &Buffer, out_f16: &Buffer, head_dim: u32, n_q_heads: u32, n_kv_heads: u32, lanes: u32, eps: f32, theta: f32, partial_rotary_factor: f32, window: u32, bits: u32, ring_capacity: u32, lane_capacity: u32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_matmul_nt_qkv_attention_lanes_into(batch.as_ptr(), fmt, input.as_ptr(), w_q.as_ptr(), w_k.as_ptr(), w_v.as_ptr(), k_dim, q.as_ptr(), k.as_ptr(), v.as_ptr(), q_norm.as_ptr(), k_norm.as_ptr(), levels.as_ptr(), signs.as_ptr(), rq.as_ptr(), k_codes.as_ptr(), k_norms.as_ptr(), v_codes.as_ptr(), v_norms.as_ptr(), positions.as_ptr(), out.as_ptr(), out_f16.as_ptr(), head_dim, n_q_heads, n_kv_heads, lanes, eps, theta, partial_rotary_factor, window, bits, ring_capacity, lane_capacity) })
+    }
+
     /// `lh_flash_attention_tq_batched_rotated_into` (include/local_hip.h).
     #[allow(clippy::too_many_arguments)]
     pub fn flash_attention_tq_batched_rotated_into(&self, batch: &mut CommandBatch, rq: &Buffer, k_codes: &Buffer, k_norms: &Buffer, v_codes: &Buffer, v_norms: &Buffer, levels: &Buffer, signs: &Buffer, out: &Buffer, out_f16: &Buffer, positions: &Buffer, head_dim: u32, lane_capacity: u32, num_q_heads: u32, num_kv_heads: u32, window: u32, bits: u32, n_lanes: u32, ring_capacity: u32) -> Result<()> {
