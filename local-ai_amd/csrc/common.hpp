@@ -149,7 +149,6 @@ struct LhNormFused {
     float eps;
     uint32_t apply_scale;
     float scale;
-    uint32_t tail;            // 0 here: the residual is added in f32 (rms_norm_add); passed through to the shared chunk arithmetic
     const uint16_t* w2;       // null: no second norm
     uint16_t* out2;
 };

@@ -7,19 +7,23 @@
 #include "common.hpp"
 #include "xquant.hpp"
 #include <cstdlib>
+#include <type_traits>
 
 namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float h_at(const uint16_t* p, size_t i) { return lh_h2f(p[i]); }
 
 // Sum over a workgroup of up to 256 threads (4 waves).
-__device__ __forceinline__ float block_sum(float v, float* scratch) {
+__device__ __forceinline__ float block_sum(float v, float* scratch, uint32_t threads) {
     v = lh_group_sum(v, 64);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = (blockDim.x + 63) >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = (threads + 63) >> 6;
     if (lane == 0) scratch[wave] = v;
     __syncthreads();
     float t = 0.0f;
-    for (int w = 0; w < nwaves; w++) t += scratch[w];
+#pragma unroll
+    for (int w = 0; w < 4; w++) t = w < nwaves ? t + scratch[w] : t;
     __syncthreads();
     return t;
 }
@@ -80,7 +84,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* in, const
     } else {
         for (uint32_t i = threadIdx.x; i < dim; i += blockDim.x) { const float v = value(i); s += v * v; }
     }
-    const float rms = rsqrtf(block_sum(s, scratch) / (float)dim + eps);
+    const float rms = rsqrtf(block_sum(s, scratch, blockDim.x) / (float)dim + eps);
     if constexpr (VEC == 8) {
         for (uint32_t i = threadIdx.x * 8; i < dim; i += blockDim.x * 8) {
             const uint4 g = *reinterpret_cast<const uint4*>(w + i);
@@ -115,57 +119,63 @@ void launch_rms_norm(hipStream_t stream, const void* in, const void* w, const vo
 // followed by the output scale (scale_in_place.metal:5-14) and by a second plain norm of the row just produced
 // (layer.rs:640-652: post-attention norm + residual, then the feed-forward norm): up to four dispatches of a decode
 // batch's layer in one.  Same thread count, accumulation order and rounding points as the separate kernels, so the
-// results are theirs bit for bit.  A thread keeps its (up to four) 8-element chunks in registers between the passes.
-template <bool PART, bool ADD>
-__global__ __launch_bounds__(256) void rms_norm_fused_kernel(const LhNormFused a) {
+// results are theirs bit for bit.  A thread keeps its (two, or up to four) 8-element chunks in registers between the passes.
+// A chain on one CU, bound by its trips to memory: with the loads under conditions the compiler had put five of them one behind the other,
+// and code for four chunks and every tail took more instruction fetches.  64 rows of 1536, three splits, two norms: 5.4 us, now 4.0; 256 rows 4.6 and 4.1.
+template <bool PART, bool ADD, int CHUNKS>
+__global__ __launch_bounds__(256) void rms_norm_fused_kernel(const uint16_t* nw, const uint16_t* res, const uint16_t* nw2, const float* partial, uint32_t dim, uint32_t splits,
+                                                            uint32_t part_rows, uint32_t part_cols, uint32_t threads, const LhNormFused a) {
     __shared__ float scratch[4];
-    const uint32_t dim = a.dim, rowi = blockIdx.x;
+    const uint32_t rowi = blockIdx.x;
     const size_t row = (size_t)rowi * dim;
-    uint4 x[4], o[4];
+    uint4 x[CHUNKS], o[CHUNKS];
     // The norm weights, the residual and the second norm's weights are requested here, with the row itself: read where they
-    // are used, each waits for memory again behind the barrier of the pass before.
-    uint4 gw[4], rr[4], gw2[4];
+    // are used, each waits for memory again behind the barrier of the pass before.  A thread without a chunk reads its row's
+    // first: with a branch around them, the values it would leave alone are put in place behind the loads, and those waited for.
+    const uint16_t* const second = nw2 != nullptr ? nw2 : nw;
+    bool has[CHUNKS];
+    uint32_t at[CHUNKS];
+    uint4 gw[CHUNKS], rr[CHUNKS], gw2[CHUNKS];
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const uint32_t i = (threadIdx.x + it * blockDim.x) * 8;
-        gw[it] = rr[it] = gw2[it] = make_uint4(0u, 0u, 0u, 0u);
-        if (i >= dim) break;
-        gw[it] = *reinterpret_cast<const uint4*>(a.w + i);
-        if (ADD) rr[it] = *reinterpret_cast<const uint4*>(a.res + row + i);
-        if (a.w2 != nullptr) gw2[it] = *reinterpret_cast<const uint4*>(a.w2 + i);
+    for (int it = 0; it < CHUNKS; it++) {
+        const uint32_t i = (threadIdx.x + it * threads) * 8;
+        has[it] = i < dim;
+        at[it] = has[it] ? i : 0u;
+        gw[it] = *reinterpret_cast<const uint4*>(nw + at[it]);
+        if (ADD) rr[it] = *reinterpret_cast<const uint4*>(res + row + at[it]);
+        gw2[it] = *reinterpret_cast<const uint4*>(second + at[it]);
     }
-    float s = 0.0f;
     if constexpr (PART) {
-        // the splits of two chunks, eight at a time, are all requested before the first is added (in split order)
-        const size_t zstride = (size_t)a.part_rows * a.part_cols;
+        // the splits of two chunks, three at a time (a product has two or three in most layers), are all requested before the first is added (in split order);
+        // past the last split its values are requested again and not added
+        const size_t zstride = (size_t)part_rows * part_cols;
 #pragma unroll
-        for (int it0 = 0; it0 < 4; it0 += 2) {
+        for (int it0 = 0; it0 < CHUNKS; it0 += 2) {
             float v[2][8];
 #pragma unroll
             for (int c = 0; c < 2; c++)
 #pragma unroll
                 for (int e = 0; e < 8; e++) v[c][e] = 0.0f;
-            const uint32_t i0 = (threadIdx.x + it0 * blockDim.x) * 8, i1 = (threadIdx.x + (it0 + 1) * blockDim.x) * 8;
-            if (i0 >= dim) break;
-            const bool two = i1 < dim;
-            const float* p0 = a.partial + (size_t)rowi * a.part_cols + i0;
-            const float* p1 = a.partial + (size_t)rowi * a.part_cols + (two ? i1 : i0);
-            for (uint32_t z0 = 0; z0 < a.splits; z0 += 8) {
-                float4 lo[2][8], hi[2][8];
+            const float* p0 = partial + (size_t)rowi * part_cols + at[it0];
+            const float* p1 = partial + (size_t)rowi * part_cols + at[it0 + 1];
+            for (uint32_t z0 = 0; z0 < splits; z0 += 3) {
+                f32x4 lo[2][3], hi[2][3];
 #pragma unroll
-                for (uint32_t u = 0; u < 8; u++) {
-                    const size_t zo = (size_t)(z0 + u < a.splits ? z0 + u : a.splits - 1) * zstride;
-                    lo[0][u] = *reinterpret_cast<const float4*>(p0 + zo); hi[0][u] = *reinterpret_cast<const float4*>(p0 + zo + 4);
-                    lo[1][u] = *reinterpret_cast<const float4*>(p1 + zo); hi[1][u] = *reinterpret_cast<const float4*>(p1 + zo + 4);
+                for (uint32_t u = 0; u < 3; u++) {
+                    const size_t zo = (size_t)(z0 + u < splits ? z0 + u : splits - 1) * zstride;
+                    lo[0][u] = *reinterpret_cast<const f32x4*>(p0 + zo); hi[0][u] = *reinterpret_cast<const f32x4*>(p0 + zo + 4);
+                    lo[1][u] = *reinterpret_cast<const f32x4*>(p1 + zo); hi[1][u] = *reinterpret_cast<const f32x4*>(p1 + zo + 4);
                 }
+                // All of them before the first addition: left to itself the compiler puts a split's loads behind the additions of the one before.
+                asm volatile("" : "+v"(lo[0][0]), "+v"(hi[0][0]), "+v"(lo[1][0]), "+v"(hi[1][0]), "+v"(lo[0][1]), "+v"(hi[0][1]), "+v"(lo[1][1]), "+v"(hi[1][1]), "+v"(lo[0][2]),
+                             "+v"(hi[0][2]), "+v"(lo[1][2]), "+v"(hi[1][2]));
 #pragma unroll
-                for (uint32_t u = 0; u < 8; u++) {
-                    if (z0 + u >= a.splits) break;
+                for (uint32_t u = 0; u < 3; u++) {
+                    const bool in = z0 + u < splits;
 #pragma unroll
-                    for (int c = 0; c < 2; c++) {
-                        v[c][0] += lo[c][u].x; v[c][1] += lo[c][u].y; v[c][2] += lo[c][u].z; v[c][3] += lo[c][u].w;
-                        v[c][4] += hi[c][u].x; v[c][5] += hi[c][u].y; v[c][6] += hi[c][u].z; v[c][7] += hi[c][u].w;
-                    }
+                    for (int c = 0; c < 2; c++)
+#pragma unroll
+                        for (int e = 0; e < 8; e++) v[c][e] = in ? v[c][e] + (e < 4 ? lo : hi)[c][u][e & 3] : v[c][e];
                 }
             }
 #pragma unroll
@@ -173,43 +183,33 @@ __global__ __launch_bounds__(256) void rms_norm_fused_kernel(const LhNormFused a
                 x[it0 + c] = make_uint4((uint32_t)lh_f2h(v[c][0]) | ((uint32_t)lh_f2h(v[c][1]) << 16), (uint32_t)lh_f2h(v[c][2]) | ((uint32_t)lh_f2h(v[c][3]) << 16),
                                         (uint32_t)lh_f2h(v[c][4]) | ((uint32_t)lh_f2h(v[c][5]) << 16), (uint32_t)lh_f2h(v[c][6]) | ((uint32_t)lh_f2h(v[c][7]) << 16));
         }
-    }
+    } else {
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const uint32_t i = (threadIdx.x + it * blockDim.x) * 8;
-        if (i >= dim) break;
-        if constexpr (!PART) x[it] = *reinterpret_cast<const uint4*>(a.in + row + i);
-        rms_sumsq8(x[it], s);
+        for (int it = 0; it < CHUNKS; it++) x[it] = *reinterpret_cast<const uint4*>(a.in + row + at[it]);
     }
-    const float rms = rsqrtf(block_sum(s, scratch) / (float)dim + a.eps);
+    float s = 0.0f;
+#pragma unroll
+    for (int it = 0; it < CHUNKS; it++) {
+        float t = s;
+        rms_sumsq8(x[it], t);
+        s = has[it] ? t : s;
+    }
+    const float rms = rsqrtf(block_sum(s, scratch, threads) / (float)dim + a.eps);
     float s2 = 0.0f;
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const uint32_t i = (threadIdx.x + it * blockDim.x) * 8;
-        if (i >= dim) break;
-        const uint4 g = gw[it];
-        uint4 r = x[it];
-        if (ADD) r = rr[it];
-        uint4 w = rms_apply8<ADD>(x[it], g, r, rms, a.tail, 1.0f);
-        if (a.apply_scale) {
-            uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                ws[j] = (uint32_t)lh_f2h(lh_h2f((uint16_t)(ws[j] & 0xFFFF)) * a.scale) | ((uint32_t)lh_f2h(lh_h2f((uint16_t)(ws[j] >> 16)) * a.scale) << 16);
-            w = make_uint4(ws[0], ws[1], ws[2], ws[3]);
-        }
-        o[it] = w;
-        rms_sumsq8(w, s2);
-        *reinterpret_cast<uint4*>(a.out + row + i) = w;
+    for (int it = 0; it < CHUNKS; it++) {
+        o[it] = rms_apply8<ADD>(x[it], gw[it], ADD ? rr[it] : x[it], rms, 0u, 1.0f);
+        if (a.apply_scale) o[it] = scale8(o[it], a.scale);
+        float t = s2;
+        rms_sumsq8(o[it], t);
+        s2 = has[it] ? t : s2;
+        if (has[it]) *reinterpret_cast<uint4*>(a.out + row + at[it]) = o[it];
     }
-    if (a.w2 == nullptr) return;
-    const float rms2 = rsqrtf(block_sum(s2, scratch) / (float)dim + a.eps);
+    if (nw2 == nullptr) return;
+    const float rms2 = rsqrtf(block_sum(s2, scratch, threads) / (float)dim + a.eps);
 #pragma unroll
-    for (int it = 0; it < 4; it++) {
-        const uint32_t i = (threadIdx.x + it * blockDim.x) * 8;
-        if (i >= dim) break;
-        *reinterpret_cast<uint4*>(a.out2 + row + i) = rms_apply8<false>(o[it], gw2[it], o[it], rms2, a.tail, 1.0f);
-    }
+    for (int it = 0; it < CHUNKS; it++)
+        if (has[it]) *reinterpret_cast<uint4*>(a.out2 + row + at[it]) = rms_apply8<false>(o[it], gw2[it], o[it], rms2, 0u, 1.0f);
 }
 
 // qk_norm.metal:6-56 (in place; head h of `qk`), and 70-140 with the NEOX rotation fused: the normalised values are
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256) void qk_norm_kernel(const uint16_t* in, uint16
     const size_t base = (size_t)blockIdx.x * head_dim;
     float s = 0.0f;
     for (uint32_t j = threadIdx.x; j < head_dim; j += blockDim.x) { const float v = h_at(in, base + j); s += v * v; }
-    const float rms = rsqrtf(block_sum(s, scratch) / (float)head_dim + eps);
+    const float rms = rsqrtf(block_sum(s, scratch, blockDim.x) / (float)head_dim + eps);
     if (!ROPE) {
         for (uint32_t j = threadIdx.x; j < head_dim; j += blockDim.x) out[base + j] = lh_f2h_exact(lh_norm_product(h_at(in, base + j), rms, h_at(w, j)));
         return;
@@ -419,14 +419,16 @@ void lh_launch_gelu_mul_strided(hipStream_t stream, const void* a, const float* 
 void lh_launch_norm_fused(hipStream_t stream, const LhNormFused& a) {
     // the thread count launch_rms_norm picks for 16-byte accesses: the partial sums of the squares add up in the same order
     const uint32_t threads = a.dim >= 2048 ? 256u : (a.dim >= 1024 ? 128u : 64u);
-    const bool part = a.partial != nullptr, add = a.res != nullptr;
-    if (part) {
-        if (add) hipLaunchKernelGGL((rms_norm_fused_kernel<true, true>), dim3(a.rows), dim3(threads), 0, stream, a);
-        else hipLaunchKernelGGL((rms_norm_fused_kernel<true, false>), dim3(a.rows), dim3(threads), 0, stream, a);
-    } else {
-        if (add) hipLaunchKernelGGL((rms_norm_fused_kernel<false, true>), dim3(a.rows), dim3(threads), 0, stream, a);
-        else hipLaunchKernelGGL((rms_norm_fused_kernel<false, false>), dim3(a.rows), dim3(threads), 0, stream, a);
-    }
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(a.rows), dim3(threads), 0, stream, a.w, a.res, a.w2, a.partial, a.dim, a.splits, a.part_rows, a.part_cols, threads, a);
+    };
+    const auto by_rows = [&](auto chunks) {
+        constexpr int C = decltype(chunks)::value;
+        if (a.partial) launch(a.res ? rms_norm_fused_kernel<true, true, C> : rms_norm_fused_kernel<true, false, C>);
+        else launch(a.res ? rms_norm_fused_kernel<false, true, C> : rms_norm_fused_kernel<false, false, C>);
+    };
+    if (a.dim <= 16 * threads) by_rows(std::integral_constant<int, 2>{});
+    else by_rows(std::integral_constant<int, 4>{});
 }
 
 extern "C" {
