@@ -87,6 +87,9 @@ LH_API int lh_event_elapsed_ms(lh_event* start, lh_event* stop, float* ms); /* w
  *      work already enqueued on the context. ---- */
 LH_API int lh_buffer_from_bytes(lh_context* ctx, const void* src, size_t len, lh_buffer** out);
 LH_API int lh_buffer_empty(lh_context* ctx, size_t len, lh_buffer** out);      /* zero-filled */
+/* Zero-filled pinned host memory, which kernels reach over the bus: for results that the host reads behind the work (lh_buffer_read waits
+ * for the stream and copies). */
+LH_API int lh_buffer_pinned(lh_context* ctx, size_t len, lh_buffer** out);
 LH_API int lh_buffer_view(lh_buffer* parent, size_t offset, size_t len, lh_buffer** out); /* non-owning */
 LH_API int lh_buffer_wrap(lh_context* ctx, void* device_ptr, size_t len, lh_buffer** out); /* non-owning */
 LH_API void lh_buffer_free(lh_buffer* buf);
@@ -163,6 +166,10 @@ LH_API int lh_matvec_q4_0_f32out(lh_context* ctx, const lh_buffer* matrix, const
                                  lh_buffer* output, uint32_t rows, uint32_t cols);
 LH_API int lh_matvec_q4_0_f32out_into(lh_batch* batch, const lh_buffer* matrix, const lh_buffer* vector,
                                       lh_buffer* output, uint32_t rows, uint32_t cols);
+/* cap * tanh(y / cap) of lh_matvec_q4_0_f32out_into's results (as they are where cap is 0), in `output` and in `copy` (pinned memory that
+ * the host reads once it has waited), apart from each other. */
+LH_API int lh_matvec_q4_0_copied_into(lh_batch* batch, const lh_buffer* matrix, const lh_buffer* vector, lh_buffer* output,
+                                      lh_buffer* copy, uint32_t rows, uint32_t cols, float cap);
 LH_API int lh_matvec_tq2_0(lh_context* ctx, const lh_buffer* matrix, const lh_buffer* vector, lh_buffer* output,
                            uint32_t rows, uint32_t cols);
 LH_API int lh_matvec_tq2_0_into(lh_batch* batch, const lh_buffer* matrix, const lh_buffer* vector, lh_buffer* output,
@@ -745,6 +752,11 @@ LH_API int lh_linear_norm_vector_into(lh_batch* batch, const lh_buffer* input, c
 LH_API int lh_linear_norm_vector_capped_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps,
                                              const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t n,
                                              lh_buffer* output, float cap);
+/* the same, capped where cap is not 0, with the results in `copy` too (pinned memory that the host reads once it has waited), apart
+ * from each other */
+LH_API int lh_linear_norm_vector_copied_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps,
+                                             const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t n,
+                                             lh_buffer* output, lh_buffer* copy, float cap);
 LH_API int lh_linear_residual_vector_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* branch,
                                           lh_buffer* store, const lh_buffer* norm_weight, float eps,
                                           const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t count,

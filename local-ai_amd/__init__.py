@@ -200,6 +200,13 @@ class Buffer:
         return cls(h, ctx)
 
     @classmethod
+    def pinned(cls, ctx: Context, byte_len: int) -> "Buffer":
+        """Pinned host memory that kernels write: its bytes are read with a wait and no launch."""
+        h = C.c_void_p()
+        _check(lib().lh_buffer_pinned(ctx._h, C.c_size_t(byte_len), C.byref(h)))
+        return cls(h, ctx)
+
+    @classmethod
     def wrap(cls, ctx: Context, device_ptr: int, byte_len: int, owner=None) -> "Buffer":
         """Non-owning handle over device memory allocated elsewhere (e.g. a torch tensor)."""
         h = C.c_void_p()
@@ -381,6 +388,9 @@ class Kernels:
 
     def matvec_q4_0_f32out_into(self, batch, matrix, vector, output, rows, cols):
         _check(self._l.lh_matvec_q4_0_f32out_into(batch._h, matrix._h, vector._h, output._h, _u32(rows), _u32(cols)))
+
+    def matvec_q4_0_copied_into(self, batch, matrix, vector, output, copy, rows, cols, cap):
+        _check(self._l.lh_matvec_q4_0_copied_into(batch._h, matrix._h, vector._h, output._h, copy._h, _u32(rows), _u32(cols), C.c_float(cap)))
 
     def matvec_tq2_0(self, ctx, matrix, vector, output, rows, cols):
         _check(self._l.lh_matvec_tq2_0(ctx._h, matrix._h, vector._h, output._h, _u32(rows), _u32(cols)))
@@ -902,6 +912,10 @@ class Kernels:
     def linear_norm_vector_capped_into(self, batch, input, norm_weight, eps, weight, bias, k, n, output, cap):
         _check(self._l.lh_linear_norm_vector_capped_into(batch._h, input._h, norm_weight._h, C.c_float(eps), weight._h, _opt(bias),
                                                          _u32(k), _u32(n), output._h, C.c_float(cap)))
+
+    def linear_norm_vector_copied_into(self, batch, input, norm_weight, eps, weight, bias, k, n, output, copy, cap):
+        _check(self._l.lh_linear_norm_vector_copied_into(batch._h, input._h, norm_weight._h, C.c_float(eps), weight._h, _opt(bias),
+                                                         _u32(k), _u32(n), output._h, copy._h, C.c_float(cap)))
 
     def linear_residual_vector_into(self, batch, input, branch, store, norm_weight, eps, weight, bias, k, segments, outputs,
                                     output_dtype, accumulate=False, position=None):

@@ -9,6 +9,7 @@
 #include "../../include/local_hip.h"
 
 struct lh_graph;
+struct LhMemory { void* ptr; bool pinned; };   // an allocation of a buffer's
 struct lh_context {
     int device;
     hipStream_t stream;
@@ -26,7 +27,7 @@ struct lh_context {
     bool capturing;
     // Owning buffers released while a capture is open.  A recorded dispatch may reference them, so they live as long as
     // the graph the capture produces (lh_graph_free releases them); when the capture fails they go when it ends.
-    std::vector<void*> deferred_free;
+    std::vector<LhMemory> deferred_free;
     // Graphs released while a capture is open; they go when it ends.
     std::vector<lh_graph*> deferred_graphs;
     // Pinned staging for descriptor tables of grouped launches and for host data of a batch: a small ring of slots, each guarded by an
@@ -60,6 +61,7 @@ struct lh_buffer {
     size_t len;
     bool owns;
     size_t slack;   // readable bytes behind ptr + len (allocation padding, or the rest of a viewed parent)
+    void* host;     // pinned memory: the same bytes as the host addresses them; null for device memory
 };
 
 struct lh_batch {
@@ -71,6 +73,8 @@ struct lh_batch {
 int lh_fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 // Post-launch check: converts a pending HIP launch error into LH_ERR_COMMAND_BUFFER.
 int lh_check_launch(const char* what);
+// `len` bytes between two places, either of which may be pinned host memory
+void lh_launch_copy_out(hipStream_t stream, const void* src, void* dst, size_t len);
 
 #define LH_HIP_TRY(expr, code, what)                                                        \
     do {                                                                                    \
@@ -158,6 +162,7 @@ bool lh_norm_fused_supported(uint32_t dim);
 void lh_launch_gelu_mul_strided(hipStream_t stream, const void* a, const float* partial, uint32_t splits, uint32_t part_cols, const void* b,
                                 uint32_t b_row_stride, uint32_t b_off, void* out, uint32_t dim, uint32_t rows);
 void lh_launch_logit_softcap(hipStream_t stream, float* data, float cap, uint32_t count);                  // logit_softcap_gpu_into's kernel
+void lh_launch_logit_softcap_copied(hipStream_t stream, float* data, float* copy, float cap, uint32_t count);   // with the results in `copy` too
 void lh_launch_gelu_mul(hipStream_t stream, const void* a, const void* b, void* out, uint32_t count);   // gelu_mul_into's kernel
 void lh_launch_norm_fused(hipStream_t stream, const LhNormFused& a);
 

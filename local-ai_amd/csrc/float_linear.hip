@@ -991,10 +991,13 @@ __global__ __launch_bounds__(256) void matvec_bf16_kernel(const VectorStage st, 
 // requested right behind it and every wait leaves the younger loads on their way.  What bounds it is the length of one such chain, not
 // the bytes.  (Four waves, each with the vector for itself and one row ahead: 10.0 us a launch on average over the products of a step
 // behind a norm, 2048 columns and 2048 to 32000 rows, 10.6 behind a gate, 5.9 with neither; with eight waves 8.9, 5.8 and 4.0.)
-template <int STAGE, int NL, int WAVES>
+// COPY: one plain row of values, which also goes to `copy` (memory of the host, as a rule); the sums of a workgroup meet in LDS and leave in
+// runs of a row a wave, 32 bytes, not in single words.  (32000 x 2048 22.4 us, 21.8 without; a copy over the bus behind it took 4.7 and the step to it.)
+template <int STAGE, int NL, int WAVES, bool COPY = false>
 __global__ __launch_bounds__(64 * WAVES) void matvec_bf16_reg_kernel(const VectorStage st, const uint16_t* __restrict__ W, const float* __restrict__ bias, const LhSegments seg,
-                                                             uint32_t N, uint32_t K) {
+                                                             uint32_t N, uint32_t K, float* __restrict__ copy) {
     __shared__ LhVectorSpace<WAVES> space;
+    __shared__ float results[COPY ? WAVES : 1][65];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), last = (K >> 3) - 1;
     const RowWalk walk{blockIdx.x * WAVES + wave, gridDim.x * WAVES, seg.pairs};
     const uint32_t rows = walk.rows(N);
@@ -1010,15 +1013,25 @@ __global__ __launch_bounds__(64 * WAVES) void matvec_bf16_reg_kernel(const Vecto
     RowSums sums{seg, bias, walk, lane};
     float xr[NL][8];
     x.finish(st, K, lane, wave, blockIdx.x == 0 && st.store != nullptr, space, xr);
-    if (rows == 0) return;
-    sums.request(rows);
+    if (!COPY && rows == 0) return;
+    if constexpr (!COPY) sums.request(rows);
     lh_walk_rows(v, rows, issue, [&](const Row& r, uint32_t) {
         float acc = 0.0f;
 #pragma unroll
         for (int c = 0; c < NL; c++) acc = lh_dot8(r.w[c], xr[c], acc);
         sums.keep(lh_group_sum(acc, 64));
     });
-    sums.flush();
+    if constexpr (COPY) {
+        results[wave][lane] = sums.mine;                      // rows: at most 64 a wave
+        lh_lds_barrier();
+        const uint32_t row = walk.first - wave + threadIdx.x % WAVES + threadIdx.x / WAVES * walk.count;
+        if (row >= N) return;
+        float v = results[threadIdx.x % WAVES][threadIdx.x / WAVES];
+        if (bias) v += bias[row];
+        if (seg.cap != 0.0f) v = seg.cap * tanhf(v / seg.cap);
+        static_cast<float*>(seg.out[0])[row] = v;
+        copy[row] = v;
+    } else sums.flush();
 }
 
 // Rows longer than a wave's registers: the eight waves of a workgroup take an eighth of the columns each, and the parts of up to 64
@@ -1072,7 +1085,15 @@ __global__ __launch_bounds__(512) void matvec_bf16_part_kernel(const VectorStage
 constexpr uint32_t kMaxVectorK = 36864;   // 144 KB of staged f32 activations
 
 template <int STAGE>
-int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, const float* bias, const LhSegments& seg, uint32_t N, uint32_t K, const char* op) {
+int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, const float* bias, const LhSegments& seg, uint32_t N, uint32_t K, const char* op,
+                  float* copy = nullptr) {
+    // `copy` of the one plain f32 row of results: by the launch itself, or by one behind it.
+    const auto copied = [&]() {
+        const int r = lh_check_launch(op);
+        if (r != LH_OK || !copy) return r;
+        lh_launch_copy_out(ctx->stream, seg.out[0], copy, (size_t)N * 4);
+        return lh_check_launch(op);
+    };
     LH_REQUIRE(K > 0 && K <= kMaxVectorK, "%s: k %u outside 1..=%u", op, K, kMaxVectorK);
     const size_t lds = (size_t)(K + 511) / 512 * 512 * 4;
     const uint32_t takes = seg.pairs ? N / 2 : N;             // rows, or pairs of rows
@@ -1090,7 +1111,14 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
         const uint32_t each = seg.pairs ? 32 : 64;           // a wave's sums fit its lanes
         const uint32_t grid = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(((uint64_t)takes + w - 1) / w, most),
                                                            ((uint64_t)takes + w * each - 1) / (w * each));
-#define LH_MVR(NLOADS, WAVES) hipLaunchKernelGGL((matvec_bf16_reg_kernel<STAGE, NLOADS, WAVES>), dim3(grid), dim3(64 * WAVES), 0, ctx->stream, st, W, bias, seg, N, K)
+#define LH_MVC(NLOADS, WAVES, COPY) hipLaunchKernelGGL((matvec_bf16_reg_kernel<STAGE, NLOADS, WAVES, COPY>), dim3(grid), dim3(64 * WAVES), 0, ctx->stream, st, W, bias, seg, N, K, copy)
+#define LH_MVR(NLOADS, WAVES) LH_MVC(NLOADS, WAVES, false)
+        if constexpr (STAGE == kNorm) if (copy && w == 8 && K <= 2048) {
+            if (K <= 512) LH_MVC(1, 8, true);
+            else if (K <= 1024) LH_MVC(2, 8, true);
+            else LH_MVC(4, 8, true);
+            return lh_check_launch(op);
+        }
         if (w == 4) {
             if (K <= 512) LH_MVR(1, 4);
             else if (K <= 1024) LH_MVR(2, 4);
@@ -1100,7 +1128,8 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
         else if (K <= 2048) LH_MVR(4, 8);
         else LH_MVR(8, 8);
 #undef LH_MVR
-        return lh_check_launch(op);
+#undef LH_MVC
+        return copied();
     }
     if constexpr (STAGE == kPlain) if (vec && K <= 16384 && lh_stage_aligned(st)) {
         const uint32_t part = ((K + 7) / 8 + 7) / 8 * 8, each = seg.pairs ? 32 : 64;
@@ -1108,7 +1137,7 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
         if (part <= 512) hipLaunchKernelGGL((matvec_bf16_part_kernel<1, 4>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
         else if (part <= 1024) hipLaunchKernelGGL((matvec_bf16_part_kernel<2, 4>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
         else hipLaunchKernelGGL((matvec_bf16_part_kernel<4, 2>), dim3(grid), dim3(64 * kVectorWaves), 0, ctx->stream, st, W, bias, seg, N, K, part);
-        return lh_check_launch(op);
+        return copied();
     }
     const uint32_t grid = (uint32_t)std::min<uint64_t>(((uint64_t)takes + 3) / 4, (uint64_t)ctx->cu_count * 4);
 #define LH_MV(NLOADS, V)                                                                                                               \
@@ -1124,7 +1153,7 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
     else if (K <= 1024) LH_MV(2, true);
     else LH_MV(4, true);
 #undef LH_MV
-    return lh_check_launch(op);
+    return copied();
 }
 
 int check_common(lh_batch* batch, const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint64_t n, const char* op) {
@@ -1141,7 +1170,7 @@ int check_common(lh_batch* batch, const lh_buffer* weight, const lh_buffer* bias
 
 int vector_entry(lh_batch* batch, const char* op, int stage, const VectorStage& st, const lh_buffer* weight, const lh_buffer* bias, uint32_t k,
                  uint32_t count, const uint32_t* ns, const uint32_t* acts, const uint32_t* heads, const uint32_t* padded, const uint32_t* layouts,
-                 lh_buffer* const* outputs, int output_dtype, int accumulate, const lh_buffer* position, float cap = 0.0f) {
+                 lh_buffer* const* outputs, int output_dtype, int accumulate, const lh_buffer* position, float cap = 0.0f, lh_buffer* copy = nullptr) {
     LhSegments seg;
     LH_TRY(lh_make_segments(seg, op, 1, 0, count, ns, acts, heads, padded, layouts, outputs, output_dtype, accumulate, position));
     seg.cap = cap;
@@ -1153,7 +1182,7 @@ int vector_entry(lh_batch* batch, const char* op, int stage, const VectorStage& 
     int r;
     if (stage == kResidual) r = launch_vector<kResidual>(batch->ctx, st, W, b, seg, n, k, op);
     else if (stage == kPlain) r = launch_vector<kPlain>(batch->ctx, st, W, b, seg, n, k, op);
-    else if (stage == kNorm) r = launch_vector<kNorm>(batch->ctx, st, W, b, seg, n, k, op);
+    else if (stage == kNorm) r = launch_vector<kNorm>(batch->ctx, st, W, b, seg, n, k, op, copy ? static_cast<float*>(copy->ptr) : nullptr);
     else r = launch_vector<kGated>(batch->ctx, st, W, b, seg, n, k, op);
     if (r == LH_OK) batch->dispatch_count++;
     return r;
@@ -1386,7 +1415,7 @@ int lh_linear_vector_into(lh_batch* batch, const lh_buffer* input, int input_dty
 static int norm_vector(lh_batch* batch, const char* op, const lh_buffer* input, const lh_buffer* add, lh_buffer* store, const lh_buffer* norm_weight, float eps,
                        const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t count, const uint32_t* ns, const uint32_t* acts,
                        const uint32_t* heads, const uint32_t* padded, const uint32_t* layouts, lh_buffer* const* outputs, int output_dtype,
-                       int accumulate, const lh_buffer* position, float cap) {
+                       int accumulate, const lh_buffer* position, float cap, lh_buffer* copy = nullptr) {
     LH_REQUIRE(batch, "%s: batch is null", op);
     LH_NEED(input, (size_t)k * 4, op, "input");
     LH_NEED(norm_weight, (size_t)k * 4, op, "norm_weight");
@@ -1398,7 +1427,7 @@ static int norm_vector(lh_batch* batch, const char* op, const lh_buffer* input, 
     VectorStage st{};
     st.x = input->ptr; st.x_f32 = 1; st.add = add ? (const float*)add->ptr : nullptr; st.store = store ? (float*)store->ptr : nullptr;
     st.norm_weight = (const float*)norm_weight->ptr; st.eps = eps;
-    return vector_entry(batch, op, kNorm, st, weight, bias, k, count, ns, acts, heads, padded, layouts, outputs, output_dtype, accumulate, position, cap);
+    return vector_entry(batch, op, kNorm, st, weight, bias, k, count, ns, acts, heads, padded, layouts, outputs, output_dtype, accumulate, position, cap, copy);
 }
 
 int lh_linear_norm_vector_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* add, lh_buffer* store, const lh_buffer* norm_weight, float eps,
@@ -1415,6 +1444,16 @@ int lh_linear_norm_vector_capped_into(lh_batch* batch, const lh_buffer* input, c
     LH_REQUIRE(cap > 0.0f, "%s: cap %g", op, (double)cap);
     const uint32_t act = LH_ACT_NONE, layout = LH_ROWS;
     return norm_vector(batch, op, input, nullptr, nullptr, norm_weight, eps, weight, bias, k, 1, &n, &act, &n, &n, &layout, &output, LH_F32, 0, nullptr, cap);
+}
+
+int lh_linear_norm_vector_copied_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps, const lh_buffer* weight,
+                                      const lh_buffer* bias, uint32_t k, uint32_t n, lh_buffer* output, lh_buffer* copy, float cap) {
+    const char* op = "linear_norm_vector_copied";
+    LH_REQUIRE(cap >= 0.0f, "%s: cap %g", op, (double)cap);
+    LH_NEED(output, (size_t)n * 4, op, "output");
+    LH_NEED(copy, (size_t)n * 4, op, "copy");
+    const uint32_t act = LH_ACT_NONE, layout = LH_ROWS;
+    return norm_vector(batch, op, input, nullptr, nullptr, norm_weight, eps, weight, bias, k, 1, &n, &act, &n, &n, &layout, &output, LH_F32, 0, nullptr, cap, copy);
 }
 
 int lh_linear_residual_vector_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* branch, lh_buffer* store, const lh_buffer* norm_weight,

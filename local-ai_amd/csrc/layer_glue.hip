@@ -388,6 +388,11 @@ __global__ __launch_bounds__(256) void logit_softcap_kernel(float* __restrict__ 
     if (i < count) data[i] = cap * tanhf(data[i] / cap);
 }
 
+__global__ __launch_bounds__(256) void logit_softcap_copied_kernel(float* __restrict__ data, float* __restrict__ copy, float cap, uint32_t count) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) copy[i] = data[i] = cap * tanhf(data[i] / cap);
+}
+
 inline uint32_t blocks_for(uint64_t n) { return (uint32_t)((n + 255) / 256); }
 inline uint32_t norm_threads(uint32_t dim) { return dim >= 256 ? 256u : (dim > 64 ? 128u : 64u); }
 
@@ -399,6 +404,9 @@ int finish(lh_batch* batch, const char* op) {
 
 }  // namespace
 
+void lh_launch_logit_softcap_copied(hipStream_t stream, float* data, float* copy, float cap, uint32_t count) {
+    hipLaunchKernelGGL(logit_softcap_copied_kernel, dim3(blocks_for(count)), dim3(256), 0, stream, data, copy, cap, count);
+}
 void lh_launch_logit_softcap(hipStream_t stream, float* data, float cap, uint32_t count) {
     hipLaunchKernelGGL(logit_softcap_kernel, dim3(blocks_for(count)), dim3(256), 0, stream, data, cap, count);
 }

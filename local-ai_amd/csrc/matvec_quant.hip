@@ -223,10 +223,15 @@ __device__ __forceinline__ u32x4_t ld16_stream(gptr_t p) {
 // One launch serves `count` problems of the same shape (count == 1 for the plain matvec).  PRO: the vector may stand behind a prologue.
 // (Streaming launches without one have a form of their own: with the prologues' code in it a 1536-column launch keeps 76 bytes a lane in scratch memory,
 // without 24: the 262144 rows of a token's logits 47-50 us, 42.7.  2048 and more columns: the same time in both.)
-template <int FMT, int L, int NPOS, typename XT, typename YT, bool IMG = false, bool PRO = true>
+// COPY (staged form, one problem, f32): results are capped and go to a second place too.  A wave takes `copy.run` batches of consecutive rows,
+// whose results meet in LDS and leave together, up to 32 of them, 128 bytes: what the host reads is written over the bus in pieces of that size.
+struct MatvecCopy { float* to; float cap; uint32_t run; };
+template <int FMT, int L, int NPOS, typename XT, typename YT, bool IMG = false, bool PRO = true, bool COPY = false>
 __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProblem* __restrict__ problems, MatvecBase single,
                                                              uint32_t count, uint32_t rows, uint32_t K, uint32_t lpr_log2,
-                                                             uint32_t steps_per_wg) {
+                                                             uint32_t steps_per_wg, MatvecCopy copy) {
+    __shared__ float results[COPY ? kWaves : 1][64];
+    [[maybe_unused]] uint32_t in_run = 0;
     extern __shared__ __align__(16) uint8_t lds[];
     constexpr int G = FMT == LH_TQ2_0 ? 256 : 32;
     constexpr int U = steps_in_flight<FMT>(NPOS);
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProble
     // that the grid reads one compact, advancing window of the matrix instead of one stream per workgroup (the
     // 262144 x 1536 logits product: 0.64 -> 0.67 of the HBM rate).  Several problems keep a contiguous share per
     // workgroup: a workgroup then stages one or two vectors, not one per batch.
-    const bool grid_window = count == 1 && steps_per_wg >= 8u * kWaves * U;
+    const bool grid_window = COPY || (count == 1 && steps_per_wg >= 8u * kWaves * U);
     uint64_t g0 = grid_window ? 0 : (uint64_t)blockIdx.x * steps_per_wg;
     const uint64_t g1 = grid_window ? total_steps : (g0 + steps_per_wg < total_steps ? g0 + steps_per_wg : total_steps);
 
@@ -275,10 +280,14 @@ __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProble
         // 2048 x 2048 launch against 0.80-0.81) and a segment of few steps is not loaded once per wave: a wave always
         // requests U steps' rows, and with a contiguous share of one step each the four waves of a small launch requested
         // the same rows four times (a single-token decode layer: 66.6 -> 64.5 us).
-        uint32_t st = s_begin + (grid_window ? blockIdx.x * kWaves + wave : wave) * U;
+        uint32_t st = s_begin + (grid_window ? blockIdx.x * kWaves + wave : wave) * U * (COPY ? copy.run : 1u);
         const uint32_t st_end = s_end;
         if (st > s_end) st = s_end;
         const uint32_t kStride = (grid_window ? gridDim.x * kWaves : kWaves) * U;
+        const auto behind = [&](uint32_t s) {              // the wave's step behind step s
+            if constexpr (COPY) return in_run + 1 < copy.run ? s + U : s + U + (kStride - U) * copy.run;
+            return s + kStride;
+        };
 
         YT* y = static_cast<YT*>(pb.output);
         gptr_t mat = (gptr_t)pb.matrix;
@@ -361,7 +370,8 @@ __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProble
             staged_vector = pb.vector;
         }
 
-        for (; st < st_end; st += kStride) {
+        for (uint32_t next; st < st_end; st = next) {
+            next = behind(st);
             float part[U];
             if constexpr (IMG) {
                 __builtin_amdgcn_s_setprio(0);        // (raised below, once the step's data is in the image)
@@ -370,7 +380,7 @@ __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProble
                 for (int i = 0; i < kImgLoads; i++)
                     if ((uint32_t)lane + 64 * i < step_chunks) *reinterpret_cast<u32x4_t*>(image + ((uint32_t)lane + 64 * i) * 16) = pre[i];
                 __builtin_amdgcn_wave_barrier();
-                if (st + kStride < st_end) prefetch(st + kStride);
+                if (next < st_end) prefetch(next);
                 // The wave has what it needs for this step and runs it at a raised priority: of the waves of a SIMD the one
                 // that can finish a step does, and reaches its next wait, and the loads behind it, sooner.
                 __builtin_amdgcn_s_setprio(1);
@@ -464,6 +474,23 @@ __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProble
 #pragma unroll
                 for (int u = 0; u < U; u++) part[u] = lh_sum32_f(part[u]);
             }
+            if constexpr (COPY) {
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (writer) results[wave][(in_run * U + u) * rpw + rsub] = part[u];
+                if (++in_run == copy.run || next >= st_end) {
+                    __builtin_amdgcn_wave_barrier();
+                    const uint32_t row = (st + U - in_run * U) * rpw + lane;
+                    if ((uint32_t)lane < in_run * U * rpw && row < rows) {
+                        float v = results[wave][lane];
+                        if (copy.cap != 0.0f) v = copy.cap * tanhf(v / copy.cap);
+                        y[row] = v;
+                        copy.to[row] = v;
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    in_run = 0;
+                }
+            } else
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const uint32_t row = (st + u) * rpw + rsub;
@@ -613,7 +640,7 @@ LaunchGeom plan(lh_quant fmt, uint32_t count, uint32_t rows, uint32_t K, int cu_
 
 template <int FMT, int L, int NPOS>
 int launch_typed(lh_context* ctx, const MatvecProblem* dev_problems, const MatvecBase& single, uint32_t count, lh_dtype xt,
-                 lh_dtype yt, uint32_t rows, uint32_t K, const LaunchGeom& g) {
+                 lh_dtype yt, uint32_t rows, uint32_t K, const LaunchGeom& g, const MatvecCopy& copy) {
 #define LH_LAUNCH_K(KERNEL)                                                                                                 \
     do {                                                                                                                    \
         if (g.lds_bytes > kMaxDynamicLds)                                                                                   \
@@ -624,7 +651,7 @@ int launch_typed(lh_context* ctx, const MatvecProblem* dev_problems, const Matve
             if (rl != LH_OK) return rl;                                                                                     \
         }                                                                                                                   \
         hipLaunchKernelGGL(KERNEL, dim3(g.grid), dim3(kWG), g.lds_bytes, ctx->stream,                                       \
-                           dev_problems, single, count, rows, K, g.lpr_log2, g.steps_per_wg);                               \
+                           dev_problems, single, count, rows, K, g.lpr_log2, g.steps_per_wg, copy);                         \
     } while (0)
 #define LH_LAUNCH(XT, YT)                                                                                                   \
     do {                                                                                                                    \
@@ -634,7 +661,9 @@ int launch_typed(lh_context* ctx, const MatvecProblem* dev_problems, const Matve
             else LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, false>));                                           \
         } else LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, false>));                                             \
     } while (0)
-    if (xt == LH_F32 && yt == LH_F32) LH_LAUNCH(float, float);
+    if (copy.to) {
+        if constexpr (FMT == LH_Q4_0 && L == 2) LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, uint16_t, float, true, false, true>));
+    } else if (xt == LH_F32 && yt == LH_F32) LH_LAUNCH(float, float);
     else if (xt == LH_F16 && yt == LH_F16) LH_LAUNCH(uint16_t, uint16_t);
     else if (xt == LH_F16 && yt == LH_F32) LH_LAUNCH(uint16_t, float);
     else LH_LAUNCH(float, uint16_t);
@@ -645,12 +674,12 @@ int launch_typed(lh_context* ctx, const MatvecProblem* dev_problems, const Matve
 
 template <int FMT, int L>
 int launch_npos(lh_context* ctx, const MatvecProblem* p, const MatvecBase& single, uint32_t count, lh_dtype xt, lh_dtype yt,
-                uint32_t rows, uint32_t K, const LaunchGeom& g) {
+                uint32_t rows, uint32_t K, const LaunchGeom& g, const MatvecCopy& copy = MatvecCopy{nullptr, 0.0f, 1}) {
     switch (g.npos) {
-        case 1: return launch_typed<FMT, L, 1>(ctx, p, single, count, xt, yt, rows, K, g);
-        case 2: return launch_typed<FMT, L, 2>(ctx, p, single, count, xt, yt, rows, K, g);
-        case 3: return launch_typed<FMT, L, 3>(ctx, p, single, count, xt, yt, rows, K, g);
-        default: return launch_typed<FMT, L, 4>(ctx, p, single, count, xt, yt, rows, K, g);
+        case 1: return launch_typed<FMT, L, 1>(ctx, p, single, count, xt, yt, rows, K, g, copy);
+        case 2: return launch_typed<FMT, L, 2>(ctx, p, single, count, xt, yt, rows, K, g, copy);
+        case 3: return launch_typed<FMT, L, 3>(ctx, p, single, count, xt, yt, rows, K, g, copy);
+        default: return launch_typed<FMT, L, 4>(ctx, p, single, count, xt, yt, rows, K, g, copy);
     }
 }
 
@@ -881,6 +910,38 @@ int lh_matvec_tq2_0_f32out(lh_context* ctx, const lh_buffer* m, const lh_buffer*
 }
 int lh_matvec_tq2_0_f32out_into(lh_batch* b, const lh_buffer* m, const lh_buffer* x, lh_buffer* y, uint32_t rows, uint32_t cols) {
     return matvec_one(b, LH_TQ2_0, m, x, LH_F16, y, LH_F32, rows, cols);
+}
+
+// The logits of a token: the launch of the product caps them and leaves them where the host reads them (262144 x 1536: 42.7 us, a cap of 4.7 and a copy
+// of 1 MB over the bus of 19.7 behind it; now 57.7; runs of 8, 16 and 64 rows 62.8, 59.6 and 58.5).  Where the product has no staged form (few rows), the cap's launch does both.
+int lh_matvec_q4_0_copied_into(lh_batch* b, const lh_buffer* m, const lh_buffer* x, lh_buffer* y, lh_buffer* copy, uint32_t rows, uint32_t cols, float cap) {
+    const char* op = "matvec_q4_0_copied";
+    LH_NEED(y, (size_t)rows * 4, op, "output");
+    LH_NEED(copy, (size_t)rows * 4, op, "copy");
+    if (!(cap >= 0.0f)) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: cap %g", op, (double)cap);
+    if (b && rows && cols && cols % 32 == 0 && m && x && fast_path_ok(LH_Q4_0, m->ptr, x->ptr, cols)) {
+        const size_t wbytes = (size_t)rows * (cols / 32) * 18;
+        LH_NEED(m, wbytes, op, "matrix");
+        LH_NEED(x, (size_t)cols * 2, op, "vector");
+        LaunchGeom g = plan(LH_Q4_0, 1, rows, cols, b->ctx->cu_count, x_limbs(LH_Q4_0), m->len - wbytes + m->slack);
+        const uint32_t batch_rows = (g.npos == 1 ? 4u : g.npos == 2 ? 2u : 1u) * g.rpw;   // steps_in_flight<LH_Q4_0>(npos) steps
+        if (g.img && x_limbs(LH_Q4_0) == 2 && batch_rows <= 64) {
+            // Runs as long as every wave of the grid still has two.
+            uint32_t run = 1;
+            while (2 * run * batch_rows <= 32 && (uint64_t)rows >= 4ull * run * batch_rows * kWaves * g.grid) run *= 2;
+            const MatvecBase single{MatvecProblem{(const uint8_t*)m->ptr, x->ptr, y->ptr}, 0, 0};
+            const int r = launch_npos<LH_Q4_0, 2>(b->ctx, nullptr, single, 1, LH_F16, LH_F32, rows, cols, g, MatvecCopy{(float*)copy->ptr, cap, run});
+            if (r == LH_OK) b->dispatch_count++;
+            return r;
+        }
+    }
+    const int r = matvec_one(b, LH_Q4_0, m, x, LH_F16, y, LH_F32, rows, cols);
+    if (r != LH_OK || rows == 0 || cols == 0) return r;
+    if (cap != 0.0f) lh_launch_logit_softcap_copied(b->ctx->stream, (float*)y->ptr, (float*)copy->ptr, cap, rows);
+    else lh_launch_copy_out(b->ctx->stream, y->ptr, copy->ptr, (size_t)rows * 4);
+    const int rc = lh_check_launch(op);
+    if (rc == LH_OK) b->dispatch_count++;
+    return rc;
 }
 
 int lh_matvec_quant_typed_into(lh_batch* b, lh_quant fmt, const lh_buffer* m, const lh_buffer* x, lh_dtype xt, lh_buffer* y,

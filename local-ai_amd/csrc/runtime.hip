@@ -30,6 +30,14 @@ __global__ __launch_bounds__(256) void read_out_kernel(const uint8_t* __restrict
     if (blockIdx.x == 0 && threadIdx.x < len % 16) dst[n16 * 16 + threadIdx.x] = src[n16 * 16 + threadIdx.x];
 }
 
+void lh_launch_copy_out(hipStream_t stream, const void* src, void* dst, size_t len) {
+    const size_t grid = (len + 4095) / 4096;
+    if ((((uintptr_t)src | (uintptr_t)dst) & 15) == 0)
+        hipLaunchKernelGGL(read_out_kernel, dim3((uint32_t)(grid < 256 ? grid : 256)), dim3(256), 0, stream, (const uint8_t*)src, (uint8_t*)dst, len);
+    else
+        hipLaunchKernelGGL(blit_copy1_kernel, dim3((uint32_t)(grid < 256 ? grid : 256)), dim3(256), 0, stream, (const uint8_t*)src, (uint8_t*)dst, len);
+}
+
 static const char* status_prefix(int code) {
     switch (code) {  // Display strings of local_metal::Error (error.rs:1-32)
         case LH_ERR_NO_DEVICE: return "No Metal device found";
@@ -345,6 +353,26 @@ int lh_buffer_empty(lh_context* ctx, size_t len, lh_buffer** out) {
     return LH_OK;
 }
 
+// Results that a kernel leaves here need no launch behind it to reach the host, which reads them once it has waited.
+int lh_buffer_pinned(lh_context* ctx, size_t len, lh_buffer** out) {
+    if (!ctx || !out) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_pinned: null argument");
+    *out = nullptr;
+    if (ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_pinned: not while a graph is being captured");
+    lh_buffer* b = new (std::nothrow) lh_buffer();
+    if (!b) return lh_fail(LH_ERR_BUFFER_ALLOCATION, "size=%zu: host allocation", len);
+    b->ctx = ctx; b->len = len; b->owns = true; b->slack = 64;
+    hipError_t e = hipHostMalloc(&b->host, len + 64, hipHostMallocDefault);
+    if (e == hipSuccess) {
+        e = hipHostGetDevicePointer(&b->ptr, b->host, 0);
+        if (e != hipSuccess) (void)hipHostFree(b->host);
+    }
+    if (e != hipSuccess) { delete b; return lh_fail(LH_ERR_BUFFER_ALLOCATION, "size=%zu: pinned memory: %s", len, hipGetErrorString(e)); }
+    memset(b->host, 0, len + 64);
+    ctx_retain(ctx);
+    *out = b;
+    return LH_OK;
+}
+
 int lh_buffer_from_bytes(lh_context* ctx, const void* src, size_t len, lh_buffer** out) {
     if (ctx && ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_from_bytes: not while a graph is being captured");
     if (!src && len) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_from_bytes: src is null");
@@ -364,6 +392,7 @@ int lh_buffer_view(lh_buffer* parent, size_t offset, size_t len, lh_buffer** out
     lh_buffer* b = new (std::nothrow) lh_buffer();
     if (!b) return lh_fail(LH_ERR_BUFFER_ALLOCATION, "size=%zu: host allocation", len);
     b->ctx = parent->ctx; b->ptr = (char*)parent->ptr + offset; b->len = len; b->owns = false;
+    b->host = parent->host ? (char*)parent->host + offset : nullptr;
     b->slack = parent->len - offset - len + parent->slack;
     ctx_retain(b->ctx);
     *out = b;
@@ -380,15 +409,18 @@ int lh_buffer_wrap(lh_context* ctx, void* device_ptr, size_t len, lh_buffer** ou
     return LH_OK;
 }
 
+static void release(const LhMemory& m) { (void)(m.pinned ? hipHostFree(m.ptr) : hipFree(m.ptr)); }
 void lh_buffer_free(lh_buffer* buf) {
     if (!buf) return;
     if (buf->owns && buf->ptr) {
         lh_context* ctx = buf->ctx;
+        const LhMemory memory{buf->host ? buf->host : buf->ptr, buf->host != nullptr};
         if (ctx->capturing) {
-            ctx->deferred_free.push_back(buf->ptr);   // neither a wait nor a free may happen inside a capture
+            // neither a wait nor a free may happen inside a capture
+            ctx->deferred_free.push_back(memory);
         } else {
             (void)hipStreamSynchronize(ctx->stream);
-            (void)hipFree(buf->ptr);
+            release(memory);
         }
     }
     ctx_release(buf->ctx);
@@ -404,9 +436,10 @@ int lh_buffer_write(lh_buffer* buf, size_t offset, const void* src, size_t len) 
     if (offset > buf->len || len > buf->len - offset)
         return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_write: range %zu+%zu exceeds %zu", offset, len, buf->len);
     if (!len) return LH_OK;
-    hipError_t e = hipMemcpyAsync((char*)buf->ptr + offset, src, len, hipMemcpyHostToDevice, buf->ctx->stream);
+    hipError_t e = buf->host ? hipSuccess : hipMemcpyAsync((char*)buf->ptr + offset, src, len, hipMemcpyHostToDevice, buf->ctx->stream);
     if (e == hipSuccess) e = wait_for_stream(buf->ctx);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_write: %s", hipGetErrorString(e));
+    if (buf->host) memcpy((char*)buf->host + offset, src, len);
     return LH_OK;
 }
 
@@ -422,13 +455,18 @@ int lh_buffer_read(const lh_buffer* buf, size_t offset, void* dst, size_t len) {
         return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_read: range %zu+%zu exceeds %zu", offset, len, buf->len);
     if (!len) return LH_OK;
     lh_context* ctx = buf->ctx;
+    if (buf->host) {
+        const hipError_t e = wait_for_stream(ctx);
+        if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_read: %s", hipGetErrorString(e));
+        memcpy(dst, (const char*)buf->host + offset, len);
+        return LH_OK;
+    }
     const uint8_t* from = (const uint8_t*)buf->ptr + offset;
     const bool waiting = ctx->waited.load(std::memory_order_relaxed) != g_launches.load(std::memory_order_relaxed);
     const bool through = len <= (waiting ? lh_context::kReadBytes : lh_context::kReadIdleBytes) && ((uintptr_t)from & 15) == 0;
     if (through) {
         std::lock_guard<std::mutex> lock(ctx->read_mutex);
-        const size_t grid = (len + 4095) / 4096;
-        hipLaunchKernelGGL(read_out_kernel, dim3((uint32_t)(grid < 256 ? grid : 256)), dim3(256), 0, ctx->stream, from, (uint8_t*)ctx->read_dev, len);
+        lh_launch_copy_out(ctx->stream, from, ctx->read_dev, len);
         const int r = lh_check_launch("buffer_read");
         if (r != LH_OK) return r;
         const hipError_t e = wait_for_stream(ctx);
@@ -446,6 +484,12 @@ int lh_buffer_fill_zero(lh_buffer* buf) {
     if (!buf) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_fill_zero: buffer is null");
     if (!buf->len) return LH_OK;
     if (buf->ctx->capturing) return lh_fail(LH_ERR_INVALID_ARGUMENT, "buffer_fill_zero: not while a graph is being captured");
+    if (buf->host) {
+        const hipError_t e = wait_for_stream(buf->ctx);
+        if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_fill_zero: %s", hipGetErrorString(e));
+        memset(buf->host, 0, buf->len);
+        return LH_OK;
+    }
     hipError_t e = hipMemsetAsync(buf->ptr, 0, buf->len, buf->ctx->stream);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: buffer_fill_zero: %s", hipGetErrorString(e));
     return LH_OK;
@@ -553,7 +597,7 @@ int lh_batch_commit_and_renew(lh_batch* batch) { return lh_batch_commit_and_wait
 // ---- recorded batches ----------------------------------------------------------
 struct lh_graph {
     lh_context* ctx; hipGraph_t graph; hipGraphExec_t exec; uint32_t dispatch_count;
-    std::vector<void*> owned;   // allocations released while the graph was recorded: its dispatches may still use them
+    std::vector<LhMemory> owned;   // allocations released while the graph was recorded: its dispatches may still use them
 };
 
 int lh_batch_begin_capture(lh_batch* batch) {
@@ -578,12 +622,12 @@ int lh_batch_end_capture(lh_batch* batch, lh_graph** out) {
     std::vector<lh_graph*> graphs;
     graphs.swap(ctx->deferred_graphs);
     for (lh_graph* old : graphs) lh_graph_free(old);
-    std::vector<void*> released;
+    std::vector<LhMemory> released;
     released.swap(ctx->deferred_free);
     auto drop_released = [&]() {   // no graph will replay: nothing can reference them once the stream is idle
         if (released.empty()) return;
         (void)hipStreamSynchronize(ctx->stream);
-        for (void* p : released) (void)hipFree(p);
+        for (const LhMemory& m : released) release(m);
         released.clear();
     };
     if (e != hipSuccess || !graph) { drop_released(); return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: end_capture: %s", hipGetErrorString(e)); }
@@ -626,7 +670,7 @@ void lh_graph_free(lh_graph* graph) {
     (void)hipStreamSynchronize(graph->ctx->stream);   // a replay may still be running
     (void)hipGraphExecDestroy(graph->exec);
     (void)hipGraphDestroy(graph->graph);
-    for (void* p : graph->owned) (void)hipFree(p);
+    for (const LhMemory& m : graph->owned) release(m);
     ctx_release(graph->ctx);
     delete graph;
 }

@@ -156,6 +156,7 @@ class DecodePipeline:
         h, pld = config.hidden_size, config.hidden_size_per_layer_input
         self.hidden_a, self.hidden_b = Buffer.empty(ctx, h * 2), Buffer.empty(ctx, h * 2)
         self.logits_buf = Buffer.empty(ctx, config.vocab_size * 4)
+        self.logits_host = Buffer.pinned(ctx, config.vocab_size * 4)   # the same for the host, behind a step that was asked for them
         self.scratch = ScratchBuffers(ctx, h, max(l.params.intermediate_size for l in layers), config.num_attention_heads,
                                       config.num_key_value_heads, max(l.params.head_dim for l in layers), pld)
         ple_total = pld * config.num_hidden_layers
@@ -265,19 +266,22 @@ class DecodePipeline:
             batch.commit_and_wait()
         return cur_in_a
 
-    def write_logits(self, final_in_a: bool, batch=None) -> None:
-        """pipeline.rs:914-953: output norm, tied-embedding logits (f32), soft cap."""
+    def write_logits(self, final_in_a: bool, batch=None, copy: Optional[Buffer] = None) -> bool:
+        """pipeline.rs:914-953: output norm, tied-embedding logits (f32), soft cap.  True where they went to `copy` too."""
         own = batch is None
         batch = batch or CommandBatch(self.ctx)
         cfg, K = self.config, self.kernels
         final_hidden = self.hidden_a if final_in_a else self.hidden_b
         # the reference norms into hidden_b even when hidden_b is the input (the kernel is safe in place)
         K.rms_norm_into(batch, final_hidden, self.output_norm, self.hidden_b, cfg.hidden_size, 1, cfg.rms_norm_eps)
-        self.token_embd.matvec_f32out_into(batch, K, self.hidden_b, self.logits_buf)
-        if self.logit_softcap > 0.0:
-            K.logit_softcap_gpu_into(batch, self.logits_buf, self.logit_softcap, cfg.vocab_size)
+        copied = copy is not None and self.token_embd.matvec_copied_into(batch, K, self.hidden_b, self.logits_buf, copy, max(self.logit_softcap, 0.0))
+        if not copied:
+            self.token_embd.matvec_f32out_into(batch, K, self.hidden_b, self.logits_buf)
+            if self.logit_softcap > 0.0:
+                K.logit_softcap_gpu_into(batch, self.logits_buf, self.logit_softcap, cfg.vocab_size)
         if own:
             batch.commit_and_wait()
+        return copied
 
     def decode_step(self, token: int) -> None:
         """One generated token: forward_token at the current position and the logits tail in one batch, one wait."""
@@ -290,9 +294,9 @@ class DecodePipeline:
     def _decode_step(self, token: int, logits: Optional[np.ndarray]) -> None:
         batch = CommandBatch(self.ctx)
         final_in_a = self.forward_token(token, self.position, batch=batch)
-        self.write_logits(final_in_a, batch=batch)
+        copied = self.write_logits(final_in_a, batch, None if logits is None else self.logits_host)
         if logits is not None:
-            self.logits_buf.read_into(logits)
+            (self.logits_host if copied else self.logits_buf).read_into(logits)
         batch.commit_and_wait()
         self.position += 1
 

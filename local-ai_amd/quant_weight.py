@@ -64,6 +64,13 @@ class QuantWeight:
         else:
             kernels.matvec_f32out_offset_into(batch, self.buf, 0, x, out, self.rows, self.cols)
 
+    def matvec_copied_into(self, batch, kernels: Kernels, x: Buffer, out: Buffer, copy: Buffer, cap: float) -> bool:
+        """f32 results, capped where cap is not 0, in `out` and in pinned memory; False where the format has no such product."""
+        if self.ty != Q4_0:
+            return False
+        kernels.matvec_q4_0_copied_into(batch, self.buf, x, out, copy, self.rows, self.cols, cap)
+        return True
+
     def matvec_typed_into(self, batch, kernels: Kernels, x: Buffer, x_dtype: int, out: Buffer, out_dtype: int) -> None:
         kernels.matvec_quant_typed_into(batch, self.ty, self.buf, x, x_dtype, out, out_dtype, self.rows, self.cols)
 

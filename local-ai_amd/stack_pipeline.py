@@ -83,6 +83,7 @@ class StackPipeline:
         self.ws = Workspace(ctx)
         self.tokens_buf = Buffer.empty(ctx, 4 * max_rows)
         self.logits_buf = Buffer.empty(ctx, 4 * config.vocab)
+        self.logits_host = Buffer.pinned(ctx, 4 * config.vocab)   # one row, behind a step
         self.next_buf = Buffer.empty(ctx, 4)
         self.at_buf = Buffer.empty(ctx, 4)                # where the token of a step stands
         self.slots = SlotPool(self._new_slot, max_sequences)
@@ -177,7 +178,7 @@ class StackPipeline:
         if n == 1 and self.observe is None:
             batch = self._decode(seq, int(tokens[0]), pick=False)
             if want:
-                self.logits_buf.read_into(out[0])
+                self.logits_host.read_into(out[0])
                 out[1:] = out[0]
             return self._finish(batch, seq, 1, wait)
         K, width = self.kernels, self.config.width
@@ -188,8 +189,8 @@ class StackPipeline:
         K.advance_position_into(batch, seq.position_buf, n)
         logits = None
         if len(want) == 1:
-            logits = self.logits_buf
-            self._encode_head(batch, x if only is not None else x.view(want[0] * width * 4, width * 4))
+            logits = self.logits_host
+            self._encode_head(batch, x if only is not None else x.view(want[0] * width * 4, width * 4), logits)
         elif want:
             m = len(want)
             index = self.ws.get("want", 4 * self.max_rows)
@@ -209,9 +210,12 @@ class StackPipeline:
             batch.commit_and_wait()
         seq.position += n
 
-    def _encode_head(self, batch, row: Buffer) -> None:
+    def _encode_head(self, batch, row: Buffer, copy: Optional[Buffer] = None) -> None:
         norm, eps, cap = self.final_norm.weight, self.config.eps, self.config.softcap
-        if cap is None:
+        if copy is not None:
+            self.kernels.linear_norm_vector_copied_into(batch, row, norm, eps, self.head.weight, self.head.bias, self.head.k, self.vocab_size,
+                                                        self.logits_buf, copy, 0.0 if cap is None else cap)
+        elif cap is None:
             self.head.normed_vector_into(batch, self.kernels, row, norm, eps, [self.logits_buf], F32)
         else:
             self.kernels.linear_norm_vector_capped_into(batch, row, norm, eps, self.head.weight, self.head.bias, self.head.k, self.vocab_size,
@@ -227,7 +231,7 @@ class StackPipeline:
             self.kernels.argmax_advance_f32_into(batch, self.logits_buf, self.next_buf, self.vocab_size, seq.position_buf, 1)
         else:
             x0 = self.ws.get("embedded", self.config.width * 4)
-            self._encode_head(batch, self._encode_layers(batch, seq, 1, max_position, x0, self.at_buf))
+            self._encode_head(batch, self._encode_layers(batch, seq, 1, max_position, x0, self.at_buf), self.logits_host)
 
     def _decode(self, seq: SequenceSlot, token: int, pick: bool) -> CommandBatch:
         """One token, encoded: logits in logits_buf and, where asked, the largest one's index in next_buf.  The first decoded token of a

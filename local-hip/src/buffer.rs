@@ -32,6 +32,14 @@ impl Buffer {
         Ok(Buffer { raw })
     }
 
+    /// Zero-filled pinned host memory, which kernels write: for results that are read behind the work.
+    pub fn pinned(ctx: &Context, byte_len: usize) -> Result<Self> {
+        let mut raw = ptr::null_mut();
+        // SAFETY: valid out pointer.
+        check(unsafe { ffi::lh_buffer_pinned(ctx.as_ptr(), byte_len, &mut raw) })?;
+        Ok(Buffer { raw })
+    }
+
     /// A non-owning window of `len` bytes at `offset` (the reference passes byte offsets into one large buffer where this
     /// API takes a buffer; a view gives such a call its operand).
     pub fn view(&self, offset: usize, len: usize) -> Result<Buffer> {

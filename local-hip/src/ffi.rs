@@ -57,6 +57,7 @@ extern "C" {
     pub fn lh_event_elapsed_ms(start: *mut lh_event, stop: *mut lh_event, ms: *mut f32) -> c_int;
     pub fn lh_buffer_from_bytes(ctx: *mut lh_context, src: *const c_void, len: usize, out: *mut *mut lh_buffer) -> c_int;
     pub fn lh_buffer_empty(ctx: *mut lh_context, len: usize, out: *mut *mut lh_buffer) -> c_int;
+    pub fn lh_buffer_pinned(ctx: *mut lh_context, len: usize, out: *mut *mut lh_buffer) -> c_int;
     pub fn lh_buffer_view(parent: *mut lh_buffer, offset: usize, len: usize, out: *mut *mut lh_buffer) -> c_int;
     pub fn lh_buffer_wrap(ctx: *mut lh_context, device_ptr: *mut c_void, len: usize, out: *mut *mut lh_buffer) -> c_int;
     pub fn lh_buffer_free(buf: *mut lh_buffer);
@@ -84,6 +85,7 @@ extern "C" {
     pub fn lh_matvec_q4_0_into(batch: *mut lh_batch, matrix: *const lh_buffer, vector: *const lh_buffer, output: *mut lh_buffer, rows: u32, cols: u32) -> c_int;
     pub fn lh_matvec_q4_0_f32out(ctx: *mut lh_context, matrix: *const lh_buffer, vector: *const lh_buffer, output: *mut lh_buffer, rows: u32, cols: u32) -> c_int;
     pub fn lh_matvec_q4_0_f32out_into(batch: *mut lh_batch, matrix: *const lh_buffer, vector: *const lh_buffer, output: *mut lh_buffer, rows: u32, cols: u32) -> c_int;
+    pub fn lh_matvec_q4_0_copied_into(batch: *mut lh_batch, matrix: *const lh_buffer, vector: *const lh_buffer, output: *mut lh_buffer, copy: *mut lh_buffer, rows: u32, cols: u32, cap: f32) -> c_int;
     pub fn lh_matvec_tq2_0(ctx: *mut lh_context, matrix: *const lh_buffer, vector: *const lh_buffer, output: *mut lh_buffer, rows: u32, cols: u32) -> c_int;
     pub fn lh_matvec_tq2_0_into(batch: *mut lh_batch, matrix: *const lh_buffer, vector: *const lh_buffer, output: *mut lh_buffer, rows: u32, cols: u32) -> c_int;
     pub fn lh_matvec_tq2_0_f32out(ctx: *mut lh_context, matrix: *const lh_buffer, vector: *const lh_buffer, output: *mut lh_buffer, rows: u32, cols: u32) -> c_int;
@@ -182,6 +184,7 @@ extern "C" {
     pub fn lh_linear_vector_into(batch: *mut lh_batch, input: *const lh_buffer, input_dtype: c_int, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
     pub fn lh_linear_norm_vector_into(batch: *mut lh_batch, input: *const lh_buffer, add: *const lh_buffer, store: *mut lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
     pub fn lh_linear_norm_vector_capped_into(batch: *mut lh_batch, input: *const lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, n: u32, output: *mut lh_buffer, cap: f32) -> c_int;
+    pub fn lh_linear_norm_vector_copied_into(batch: *mut lh_batch, input: *const lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, n: u32, output: *mut lh_buffer, copy: *mut lh_buffer, cap: f32) -> c_int;
     pub fn lh_linear_residual_vector_into(batch: *mut lh_batch, input: *const lh_buffer, branch: *const lh_buffer, store: *mut lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
     pub fn lh_gated_vector_fits(k: u32, group: u32) -> u32;
     pub fn lh_linear_gated_vector_into(batch: *mut lh_batch, input: *const lh_buffer, gate: *const lh_buffer, gate_dtype: c_int, gate_act: u32, gate_first: c_int, norm_weight: *const lh_buffer, group: u32, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;

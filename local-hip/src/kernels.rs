@@ -45,6 +45,13 @@ impl Kernels {
         check(unsafe { ffi::lh_matvec_q4_0_f32out_into(batch.as_ptr(), matrix.as_ptr(), vector.as_ptr(), output.as_ptr(), rows, cols) })
     }
 
+    /// `lh_matvec_q4_0_copied_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn matvec_q4_0_copied_into(&self, batch: &mut CommandBatch, matrix: &Buffer, vector: &Buffer, output: &Buffer, copy: &Buffer, rows: u32, cols: u32, cap: f32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_matvec_q4_0_copied_into(batch.as_ptr(), matrix.as_ptr(), vector.as_ptr(), output.as_ptr(), copy.as_ptr(), rows, cols, cap) })
+    }
+
     /// `lh_matvec_tq2_0` (include/local_hip.h).
     pub fn matvec_tq2_0(&self, ctx: &Context, matrix: &Buffer, vector: &Buffer, output: &Buffer, rows: u32, cols: u32) -> Result<()> {
         // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
@@ -601,6 +608,13 @@ impl Kernels {
     pub fn linear_norm_vector_capped_into(&self, batch: &mut CommandBatch, input: &Buffer, norm_weight: &Buffer, eps: f32, weight: &Buffer, bias: &Buffer, k: u32, n: u32, output: &Buffer, cap: f32) -> Result<()> {
         // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
         check(unsafe { ffi::lh_linear_norm_vector_capped_into(batch.as_ptr(), input.as_ptr(), norm_weight.as_ptr(), eps, weight.as_ptr(), bias.as_ptr(), k, n, output.as_ptr(), cap) })
+    }
+
+    /// `lh_linear_norm_vector_copied_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn linear_norm_vector_copied_into(&self, batch: &mut CommandBatch, input: &Buffer, norm_weight: &Buffer, eps: f32, weight: &Buffer, bias: &Buffer, k: u32, n: u32, output: &Buffer, copy: &Buffer, cap: f32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_linear_norm_vector_copied_into(batch.as_ptr(), input.as_ptr(), norm_weight.as_ptr(), eps, weight.as_ptr(), bias.as_ptr(), k, n, output.as_ptr(), copy.as_ptr(), cap) })
     }
 
     /// `lh_linear_residual_vector_into` (include/local_hip.h).

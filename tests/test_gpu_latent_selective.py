@@ -540,6 +540,29 @@ def test_capped_products(ai, gpu):
         K.linear_norm_vector_capped_into(batch, x, norm, 1e-6, w, bias, k, n, b, 0.0)
 
 
+@pytest.mark.parametrize("cap", [0.0, 15.5])
+@pytest.mark.parametrize("k,n", [(64, 300), (512, 40000), (1024, 33001), (2048, 2049), (2048, 131071), (2048, 5000), (3072, 9000), (6000, 70), (20, 9)])
+def test_copied_products(ai, gpu, k, n, cap):
+    """Results that also go to pinned memory are those of the product alone, in both places and behind the last one nothing is written."""
+    ctx, K = gpu
+    g, batch = np.random.default_rng(k), ai.CommandBatch(ctx)
+    x, w = upload(ai, ctx, g.standard_normal(k) * 3, ai.F32), upload(ai, ctx, g.standard_normal((n, k), np.float32), ai.BF16)
+    norm, a, b, c = upload(ai, ctx, np.full(k, 0.5), ai.F32), *(ai.Buffer.empty(ctx, n * 4 + 64) for _ in range(2)), ai.Buffer.pinned(ctx, n * 4 + 64)
+    for bias in (None, upload(ai, ctx, g.standard_normal(n), ai.F32)):
+        K.linear_norm_vector_into(batch, x, None, None, norm, 1e-6, w, bias, k, ai.linear_weight.Segments([ai.linear_weight.Segment(n)]), [a], ai.F32)
+        if cap:
+            K.softcap_f32_into(batch, a, n, cap)
+        for at in (0, 4):                                      # a place that only single words reach
+            b.fill_zero()
+            c.fill_zero()
+            K.linear_norm_vector_copied_into(batch, x, norm, 1e-6, w, bias, k, n, b.view(at, n * 4), c.view(at, n * 4), cap)
+            want, device, host = (v.as_array(np.uint8) for v in (a, b, c))
+            assert (device == host).all() and not device[:at].any() and not device[at + 4 * n:].any()
+            assert (device[at:at + 4 * n] == want[:4 * n]).all()
+    with pytest.raises(ai.InvalidArgument):
+        K.linear_norm_vector_copied_into(batch, x, norm, 1e-6, w, bias, k, n, b.view(0, n * 4 - 4), c, cap)
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 1000, 16384, 16385, 40000])
 def test_argmax_and_position(ai, gpu, n):
     """The first of several largest values, wherever they lie, and the position moved on behind it."""

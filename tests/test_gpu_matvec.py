@@ -770,3 +770,27 @@ def test_products_of_few_signs_and_large_elements(pkg, gpu, oracle, fmt, kind, r
     want = x64 @ w64.T
     half = np.exp2(np.maximum(np.floor(np.log2(np.maximum(np.abs(want), 1e-30))), -14) - 11)
     assert np.all(np.abs(got[1] - want) <= 1.001 * half + 24 * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T))
+
+
+@pytest.mark.parametrize("cap", [0.0, 30.0])
+@pytest.mark.parametrize("rows,cols", [(262144 - 37, 1536), (66001, 2048), (33003, 4096), (20000, 8192), (70007, 1024), (300001, 256), (200000, 64), (32000, 1536), (300, 1536), (7, 96)])
+def test_matvec_q4_0_results_in_pinned_memory_too(pkg, gpu, rows, cols, cap):
+    """One to three batches of rows in a wave's run, ragged ends, and shapes without the staged form: both places hold the product's bits, capped."""
+    ctx, K = gpu
+    g = pkg.synth.rng(3, rows)
+    w = pkg.QuantWeight.from_bytes(ctx, pkg.synth.weights("q4_0", rows, cols, g), pkg.Q4_0, rows, cols)
+    x = pkg.Buffer.from_slice(ctx, pkg.synth.activations(1, cols, g)[0].astype(np.float16))
+    a, b, c = pkg.Buffer.empty(ctx, rows * 4), pkg.Buffer.empty(ctx, rows * 4 + 64), pkg.Buffer.pinned(ctx, rows * 4 + 64)
+    batch = pkg.CommandBatch(ctx)
+    w.matvec_f32out_into(batch, K, x, a)
+    if cap:
+        K.logit_softcap_gpu_into(batch, a, cap, rows)
+    for at in (0, 4):                                          # a place that only single words reach
+        b.fill_zero()
+        c.fill_zero()
+        assert w.matvec_copied_into(batch, K, x, b.view(at, rows * 4), c.view(at, rows * 4), cap)
+        want, device, host = (v.as_array(np.uint8) for v in (a, b, c))
+        assert (device == host).all() and not device[:at].any() and not device[at + 4 * rows:].any()
+        assert (device[at:at + 4 * rows] == want).all()
+    with pytest.raises(pkg.InvalidArgument):
+        K.matvec_q4_0_copied_into(batch, w.buf, x, b, c.view(0, rows * 4 - 4), rows, cols, cap)
