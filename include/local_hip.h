@@ -900,6 +900,11 @@ LH_API int lh_moe_down_into(lh_batch* batch, const lh_buffer* hidden, int dtype,
 LH_API int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps,
                                  const lh_buffer* logits, const lh_buffer* up, lh_buffer* hidden, uint32_t experts,
                                  uint32_t top, uint32_t width, uint32_t ff, uint32_t act);
+/* lh_linear_norm_vector_into of the router's rows (bf16, no bias) into `logits`, then lh_moe_vector_up_into, in one launch where a
+ * workgroup's waves have at most four rows of it each */
+LH_API int lh_moe_vector_routed_up_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps,
+                                        const lh_buffer* router, lh_buffer* logits, const lh_buffer* up, lh_buffer* hidden,
+                                        uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act);
 LH_API int lh_moe_vector_down_into(lh_batch* batch, const lh_buffer* hidden, const lh_buffer* logits, const lh_buffer* down,
                                    lh_buffer* residual, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff);
 

@@ -1046,6 +1046,10 @@ class Kernels:
         _check(self._l.lh_moe_down_into(batch._h, hidden._h, C.c_int(dtype), plan._h, down._h, _opt(slots), residual._h,
                                         _u32(rows), _u32(experts), _u32(top), _u32(width), _u32(ff)))
 
+    def moe_vector_routed_up_into(self, batch, input, norm_weight, eps, router, logits, up, hidden, experts, top, width, ff, act):
+        _check(self._l.lh_moe_vector_routed_up_into(batch._h, input._h, norm_weight._h, C.c_float(eps), router._h, logits._h, up._h, hidden._h,
+                                                    _u32(experts), _u32(top), _u32(width), _u32(ff), _u32(act)))
+
     def moe_vector_up_into(self, batch, input, norm_weight, eps, logits, up, hidden, experts, top, width, ff, act):
         _check(self._l.lh_moe_vector_up_into(batch._h, input._h, norm_weight._h, C.c_float(eps), logits._h, up._h, hidden._h,
                                              _u32(experts), _u32(top), _u32(width), _u32(ff), _u32(act)))

@@ -177,28 +177,51 @@ __global__ __launch_bounds__(256) void vector_up_kernel(const float* __restrict_
 
 // The same with the normed vector in registers (width a multiple of 8, up to 512 * NL), brought in by the waves together: a
 // workgroup keeps to one expert's rows (blockIdx.y: the choice), and the weights of two rows are requested as soon as the selection is known.
-template <int NL, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void vector_up_reg_kernel(const VectorStage st, const float* __restrict__ logits, const uint16_t* __restrict__ up,
+// ROUTE: the logits come from the router's rows (at most kRouted a wave), which every workgroup multiplies for itself, requested with the vector; what they cost
+// there is less than the launch that they had (two of 16 experts, 2048 -> 1024 columns: 4.5 us and 3.2 with the step between them, 6.2 now; 8 experts, 1024 -> 512: 3.4 and 3.3, 4.1).
+constexpr int kRouted = 4;
+template <int NL, int WAVES, int ROUTE>
+__global__ __launch_bounds__(64 * WAVES) void vector_up_reg_kernel(const VectorStage st, float* __restrict__ logits, const uint16_t* __restrict__ router, const uint16_t* __restrict__ up,
                                                            float* __restrict__ hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act) {
     __shared__ uint32_t ids[WAVES][kMaxTop];
     __shared__ float weights[WAVES][kMaxTop];
     __shared__ LhVectorSpace<WAVES> space;
+    __shared__ float routed[ROUTE ? WAVES * ROUTE : 1];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = blockIdx.y, last = (width >> 3) - 1;
     LhSharedVector<kNorm, NL, WAVES> x;
     x.fetch(st, width, lane, wave);
-    select_experts(logits, experts, c + 1, lane, ids[wave], weights[wave]);    // every wave for itself: no barrier
+    float xr[NL][8];
+    struct Row { uint4 w[NL]; } v[2];
+    if constexpr (ROUTE > 0) {
+        Row t[ROUTE];
+#pragma unroll
+        for (int i = 0; i < ROUTE; i++)
+#pragma unroll
+            for (int j = 0; j < NL; j++) t[i].w[j] = *reinterpret_cast<const uint4*>(router + (size_t)min(wave + i * WAVES, experts - 1) * width + 8 * min(64u * j + lane, last));
+        x.finish(st, width, lane, wave, false, space, xr);
+#pragma unroll
+        for (int i = 0; i < ROUTE; i++) {
+            float acc = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NL; j++) acc = lh_dot8(t[i].w[j], xr[j], acc);
+            acc = lh_group_sum(acc, 64);
+            const uint32_t e = wave + i * WAVES;
+            if (lane == 0) routed[e] = acc;
+            if (blockIdx.x == 0 && c == 0 && lane == 0 && e < experts) logits[e] = acc;
+        }
+        lh_lds_barrier();
+        select_experts_of<1>(routed, experts, c + 1, lane, ids[wave], weights[wave]);
+    } else select_experts(logits, experts, c + 1, lane, ids[wave], weights[wave]);    // every wave for itself: no barrier
     const uint32_t e = __builtin_amdgcn_readfirstlane(ids[wave][c]);
     const float weight = weights[wave][c];
     const uint16_t* base = up + (size_t)e * ff * width;
     const uint32_t first = blockIdx.x * WAVES + wave, step = gridDim.x * WAVES, rows = first < ff ? (ff - first - 1) / step + 1 : 0u;
-    struct Row { uint4 w[NL]; } v[2];
     auto issue = [&](Row& x, uint32_t i) {
 #pragma unroll
         for (int j = 0; j < NL; j++) x.w[j] = lh_ld16_stream(base + (size_t)(first + i * step) * width + 8 * min(64u * j + lane, last));
     };
     if (rows) lh_first_rows(v, rows, issue);
-    float xr[NL][8];
-    x.finish(st, width, lane, wave, false, space, xr);
+    if constexpr (ROUTE == 0) x.finish(st, width, lane, wave, false, space, xr);
     if (rows == 0) return;
     lh_walk_rows(v, rows, issue, [&](const Row& r, uint32_t i) {
         float acc = 0.0f;
@@ -386,9 +409,16 @@ int lh_moe_down_into(lh_batch* batch, const lh_buffer* hidden, int dtype, const 
     return LH_OK;
 }
 
-int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps, const lh_buffer* logits, const lh_buffer* up,
-                          lh_buffer* hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act) {
-    const char* op = "moe_vector_up";
+static int route_vector(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps, const lh_buffer* router, lh_buffer* logits, uint32_t experts,
+                        uint32_t width) {
+    const uint32_t act = LH_ACT_NONE, layout = LH_ROWS;
+    return lh_linear_norm_vector_into(batch, input, nullptr, nullptr, norm_weight, eps, router, nullptr, width, 1, &experts, &act, &experts, &experts, &layout, &logits, LH_F32, 0,
+                                      nullptr);
+}
+
+// router: null where the logits are there
+static int vector_up(lh_batch* batch, const char* op, const lh_buffer* input, const lh_buffer* norm_weight, float eps, const lh_buffer* router, lh_buffer* logits,
+                     const lh_buffer* up, lh_buffer* hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act) {
     LH_REQUIRE(batch, "%s: batch is null", op);
     LH_TRY(check_shape(op, 1, experts, top));
     LH_REQUIRE(width > 0 && ff > 0 && act <= LH_ACT_SIGMOID, "%s: width %u, ff %u, activation %u", op, width, ff, act);
@@ -397,14 +427,19 @@ int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const lh_buff
     LH_NEED(logits, (size_t)experts * 4, op, "logits");
     LH_NEED(up, (size_t)experts * ff * width * 2, op, "up");
     LH_NEED(hidden, (size_t)top * ff * 4, op, "hidden");
+    if (router) LH_NEED(router, (size_t)experts * width * 2, op, "router");
     VectorStage st{};
     st.x = input->ptr; st.x_f32 = 1; st.norm_weight = (const float*)norm_weight->ptr; st.eps = eps;
     if (width % 8 == 0 && width <= 4096 && ((uintptr_t)up->ptr & 15) == 0 && lh_stage_aligned(st)) {
-        // (four waves where all rows are at most eight per CU, as the one-row products)
-        const uint32_t cus = (uint32_t)batch->ctx->cu_count, w = width <= 2048 && (uint64_t)ff * top <= 8ull * cus ? 4 : kVectorWaves;
+        // (four waves where all rows are at most eight per CU, as the one-row products; with the router and more than 1024 columns eight, so that half as many
+        // workgroups read it: 16 experts, 2048 columns 6.2 us and 7.0; 8 experts, 1024 columns 4.5 and 4.1)
+        const uint32_t cus = (uint32_t)batch->ctx->cu_count, w = width <= (router ? 1024u : 2048u) && (uint64_t)ff * top <= 8ull * cus ? 4 : kVectorWaves;
+        const bool route = router && experts <= kRouted * w && ((uintptr_t)router->ptr & 15) == 0;
+        if (router && !route) LH_TRY(route_vector(batch, input, norm_weight, eps, router, logits, experts, width));
         const dim3 grid(std::min<uint32_t>((ff + w - 1) / w, std::max<uint32_t>(1, (w == 4 ? 2 : 1) * cus / top)), top);
-#define LH_UP(NL, WAVES) hipLaunchKernelGGL((vector_up_reg_kernel<NL, WAVES>), grid, dim3(64 * WAVES), 0, batch->ctx->stream, st, (const float*)logits->ptr, \
-                                            (const uint16_t*)up->ptr, (float*)hidden->ptr, experts, top, width, ff, act)
+#define LH_UP_R(NL, WAVES, R) hipLaunchKernelGGL((vector_up_reg_kernel<NL, WAVES, R>), grid, dim3(64 * WAVES), 0, batch->ctx->stream, st, (float*)logits->ptr, \
+                                                 route ? (const uint16_t*)router->ptr : nullptr, (const uint16_t*)up->ptr, (float*)hidden->ptr, experts, top, width, ff, act)
+#define LH_UP(NL, WAVES) do { if (!route) LH_UP_R(NL, WAVES, 0); else if (experts <= WAVES) LH_UP_R(NL, WAVES, 1); else if (experts <= 2 * WAVES) LH_UP_R(NL, WAVES, 2); else LH_UP_R(NL, WAVES, kRouted); } while (0)
         if (w == 4) {
             if (width <= 512) LH_UP(1, 4);
             else if (width <= 1024) LH_UP(2, 4);
@@ -414,10 +449,12 @@ int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const lh_buff
         else if (width <= 2048) LH_UP(4, 8);
         else LH_UP(8, 8);
 #undef LH_UP
+#undef LH_UP_R
         LH_TRY(lh_check_launch(op));
         batch->dispatch_count++;
         return LH_OK;
     }
+    if (router) LH_TRY(route_vector(batch, input, norm_weight, eps, router, logits, experts, width));
     const size_t lds = (size_t)width * 4;
     LH_TRY(vector_lds(batch->ctx, (const void*)vector_up_kernel, lds, op));
     const uint32_t grid = (uint32_t)std::min<uint64_t>(((uint64_t)top * ff + 3) / 4, (uint64_t)batch->ctx->cu_count * 4);
@@ -427,6 +464,18 @@ int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const lh_buff
     LH_TRY(lh_check_launch(op));
     batch->dispatch_count++;
     return LH_OK;
+}
+
+int lh_moe_vector_up_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps, const lh_buffer* logits, const lh_buffer* up,
+                          lh_buffer* hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act) {
+    return vector_up(batch, "moe_vector_up", input, norm_weight, eps, nullptr, const_cast<lh_buffer*>(logits), up, hidden, experts, top, width, ff, act);
+}
+
+int lh_moe_vector_routed_up_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* norm_weight, float eps, const lh_buffer* router, lh_buffer* logits,
+                                 const lh_buffer* up, lh_buffer* hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act) {
+    const char* op = "moe_vector_routed_up";
+    LH_REQUIRE(router, "%s: router is null", op);
+    return vector_up(batch, op, input, norm_weight, eps, router, logits, up, hidden, experts, top, width, ff, act);
 }
 
 int lh_moe_vector_down_into(lh_batch* batch, const lh_buffer* hidden, const lh_buffer* logits, const lh_buffer* down, lh_buffer* residual, uint32_t experts,

@@ -494,9 +494,12 @@ class MoeFeedForward:
         s, K, b, n = self.spec, r.kernels, r.batch, r.rows
         logits = r.scratch("router", n * s.experts, f32=True)
         if n == 1:
-            norm.vector_into(r, self.router, [logits], F32)
             h = r.scratch("expert", s.top * s.ff, f32=True)
-            K.moe_vector_up_into(b, r.x, norm.weight, norm.eps, logits, self.up, h, s.experts, s.top, self.width, s.ff, s.act)
+            if r.add is None and r.store is None:
+                K.moe_vector_routed_up_into(b, r.x, norm.weight, norm.eps, self.router.weight, logits, self.up, h, s.experts, s.top, self.width, s.ff, s.act)
+            else:
+                norm.vector_into(r, self.router, [logits], F32)
+                K.moe_vector_up_into(b, r.x, norm.weight, norm.eps, logits, self.up, h, s.experts, s.top, self.width, s.ff, s.act)
             K.moe_vector_down_into(b, h, logits, self.down, r.x, s.experts, s.top, self.width, s.ff)
             return
         x = norm.rows(r)

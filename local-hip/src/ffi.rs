@@ -213,6 +213,7 @@ extern "C" {
     pub fn lh_moe_up_into(batch: *mut lh_batch, input: *const lh_buffer, dtype: c_int, plan: *const lh_buffer, up: *const lh_buffer, hidden: *mut lh_buffer, rows: u32, experts: u32, top: u32, width: u32, ff: u32, act: u32) -> c_int;
     pub fn lh_moe_down_into(batch: *mut lh_batch, hidden: *const lh_buffer, dtype: c_int, plan: *const lh_buffer, down: *const lh_buffer, slots: *mut lh_buffer, residual: *mut lh_buffer, rows: u32, experts: u32, top: u32, width: u32, ff: u32) -> c_int;
     pub fn lh_moe_vector_up_into(batch: *mut lh_batch, input: *const lh_buffer, norm_weight: *const lh_buffer, eps: f32, logits: *const lh_buffer, up: *const lh_buffer, hidden: *mut lh_buffer, experts: u32, top: u32, width: u32, ff: u32, act: u32) -> c_int;
+    pub fn lh_moe_vector_routed_up_into(batch: *mut lh_batch, input: *const lh_buffer, norm_weight: *const lh_buffer, eps: f32, router: *const lh_buffer, logits: *mut lh_buffer, up: *const lh_buffer, hidden: *mut lh_buffer, experts: u32, top: u32, width: u32, ff: u32, act: u32) -> c_int;
     pub fn lh_moe_vector_down_into(batch: *mut lh_batch, hidden: *const lh_buffer, logits: *const lh_buffer, down: *const lh_buffer, residual: *mut lh_buffer, experts: u32, top: u32, width: u32, ff: u32) -> c_int;
     pub fn lh_advance_position_into(batch: *mut lh_batch, position: *mut lh_buffer, by: u32) -> c_int;
     pub fn lh_argmax_rows_f32_into(batch: *mut lh_batch, logits: *const lh_buffer, index: *mut lh_buffer, rows: u32, n: u32) -> c_int;

@@ -751,6 +751,13 @@ impl Kernels {
         check(unsafe { ffi::lh_moe_vector_up_into(batch.as_ptr(), input.as_ptr(), norm_weight.as_ptr(), eps, logits.as_ptr(), up.as_ptr(), hidden.as_ptr(), experts, top, width, ff, act) })
     }
 
+    /// `lh_moe_vector_routed_up_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn moe_vector_routed_up_into(&self, batch: &mut CommandBatch, input: &Buffer, norm_weight: &Buffer, eps: f32, router: &Buffer, logits: &Buffer, up: &Buffer, hidden: &Buffer, experts: u32, top: u32, width: u32, ff: u32, act: u32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_moe_vector_routed_up_into(batch.as_ptr(), input.as_ptr(), norm_weight.as_ptr(), eps, router.as_ptr(), logits.as_ptr(), up.as_ptr(), hidden.as_ptr(), experts, top, width, ff, act) })
+    }
+
     /// `lh_moe_vector_down_into` (include/local_hip.h).
     #[allow(clippy::too_many_arguments)]
     pub fn moe_vector_down_into(&self, batch: &mut CommandBatch, hidden: &Buffer, logits: &Buffer, down: &Buffer, residual: &Buffer, experts: u32, top: u32, width: u32, ff: u32) -> Result<()> {

@@ -876,6 +876,27 @@ def test_mixture_of_experts(ai, gpu, dtype, rows, experts, top, width, ff):
     close(download(ai, rb0, width, ai.F32), res[0] + one, F32_TOL, "one row")
 
 
+@pytest.mark.parametrize("experts,top,width,ff", [(16, 2, 2048, 1024), (8, 2, 1024, 512), (17, 3, 2048, 1024), (5, 5, 512, 40), (32, 4, 1536, 1536), (33, 1, 4096, 900), (1, 1, 64, 8),
+                                                  (6, 2, 100, 24), (16, 2, 1368, 688)])
+def test_router_in_the_launch_of_the_experts(ai, gpu, experts, top, width, ff):
+    """The bits of the router's product and of the experts' own launch behind it, with and without room for the router."""
+    ctx, K = gpu
+    g = np.random.default_rng(experts * width)
+    x, nw = upload(ai, ctx, g.standard_normal(width) * 2, ai.F32), upload(ai, ctx, 1 + 0.1 * g.standard_normal(width), ai.F32)
+    router, up = upload(ai, ctx, g.standard_normal((experts, width)) / width ** 0.5, ai.BF16), upload(ai, ctx, g.standard_normal((experts, ff, width)) / width ** 0.5, ai.BF16)
+    got = []
+    for form in range(2):
+        lb, hid, batch = empty(ai, ctx, experts, ai.F32), empty(ai, ctx, top * ff, ai.F32), ai.CommandBatch(ctx)
+        if form:
+            K.moe_vector_routed_up_into(batch, x, nw, 1e-5, router, lb, up, hid, experts, top, width, ff, ai.ACT_RELU_SQUARED)
+        else:
+            K.linear_norm_vector_into(batch, x, None, None, nw, 1e-5, router, None, width, ai.linear_weight.Segments([ai.linear_weight.Segment(experts)]), [lb], ai.F32)
+            K.moe_vector_up_into(batch, x, nw, 1e-5, lb, up, hid, experts, top, width, ff, ai.ACT_RELU_SQUARED)
+        batch.commit_and_wait()
+        got.append((lb.as_array(np.uint32), hid.as_array(np.uint32)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][1].any()
+
+
 def test_equal_scores_go_to_the_lower_expert(ai, gpu):
     ctx, K = gpu
     logits = np.zeros((3, 9), np.float32)
