@@ -917,6 +917,11 @@ class Kernels:
         _check(self._l.lh_linear_norm_vector_copied_into(batch._h, input._h, norm_weight._h, C.c_float(eps), weight._h, _opt(bias),
                                                          _u32(k), _u32(n), output._h, copy._h, C.c_float(cap)))
 
+    def linear_residual_norm_vector_copied_into(self, batch, input, branch, branch_weight, branch_eps, norm_weight, eps, weight, bias, k, n, output, copy, cap):
+        _check(self._l.lh_linear_residual_norm_vector_copied_into(batch._h, input._h, branch._h, branch_weight._h, C.c_float(branch_eps),
+                                                                  norm_weight._h, C.c_float(eps), weight._h, _opt(bias), _u32(k), _u32(n),
+                                                                  output._h, copy._h, C.c_float(cap)))
+
     def linear_residual_vector_into(self, batch, input, branch, store, norm_weight, eps, weight, bias, k, segments, outputs,
                                     output_dtype, accumulate=False, position=None):
         _check(self._l.lh_linear_residual_vector_into(batch._h, input._h, branch._h, _opt(store), norm_weight._h, C.c_float(eps),

@@ -1082,6 +1082,13 @@ __global__ __launch_bounds__(512) void matvec_bf16_part_kernel(const VectorStage
     total.flush();
 }
 
+// A workgroup for every CU first; a second one where rows are short and each of its waves still has two (32000 x 1024: 11.9 us
+// against 12.5; 8192 x 2048: 7.8 against 7.65).  A wave's sums (`each`) fit its lanes.
+uint32_t one_row_grid(uint64_t takes, uint32_t K, uint32_t waves, uint32_t each, uint64_t cus) {
+    const uint64_t most = std::max(cus, K <= 1024 ? std::min<uint64_t>(2 * cus, (takes + 15) / 16) : 0);
+    return (uint32_t)std::max<uint64_t>(std::min<uint64_t>((takes + waves - 1) / waves, most), (takes + waves * each - 1) / (waves * each));
+}
+
 constexpr uint32_t kMaxVectorK = 36864;   // 144 KB of staged f32 activations
 
 template <int STAGE>
@@ -1105,12 +1112,7 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
     const bool few = takes <= 8 * cus;
     if (vec && K <= 4096 && lh_stage_aligned(st) && !(STAGE == kPlain && K > 2048 && few)) {
         const uint32_t w = K <= 2048 && few ? 4 : kVectorWaves;
-        // A workgroup for every CU first; a second one where rows are short and each of its waves still has two (32000 x 1024: 11.9 us
-        // against 12.5; 8192 x 2048: 7.8 against 7.65).
-        const uint64_t most = std::max(cus, K <= 1024 ? std::min<uint64_t>(2 * cus, ((uint64_t)takes + 15) / 16) : 0);
-        const uint32_t each = seg.pairs ? 32 : 64;           // a wave's sums fit its lanes
-        const uint32_t grid = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(((uint64_t)takes + w - 1) / w, most),
-                                                           ((uint64_t)takes + w * each - 1) / (w * each));
+        const uint32_t grid = one_row_grid(takes, K, w, seg.pairs ? 32 : 64, cus);
 #define LH_MVC(NLOADS, WAVES, COPY) hipLaunchKernelGGL((matvec_bf16_reg_kernel<STAGE, NLOADS, WAVES, COPY>), dim3(grid), dim3(64 * WAVES), 0, ctx->stream, st, W, bias, seg, N, K, copy)
 #define LH_MVR(NLOADS, WAVES) LH_MVC(NLOADS, WAVES, false)
         if constexpr (STAGE == kNorm) if (copy && w == 8 && K <= 2048) {
@@ -1454,6 +1456,43 @@ int lh_linear_norm_vector_copied_into(lh_batch* batch, const lh_buffer* input, c
     LH_NEED(copy, (size_t)n * 4, op, "copy");
     const uint32_t act = LH_ACT_NONE, layout = LH_ROWS;
     return norm_vector(batch, op, input, nullptr, nullptr, norm_weight, eps, weight, bias, k, 1, &n, &act, &n, &n, &layout, &output, LH_F32, 0, nullptr, cap, copy);
+}
+
+int lh_linear_residual_norm_vector_copied_into(lh_batch* batch, lh_buffer* input, const lh_buffer* branch, const lh_buffer* branch_weight, float branch_eps,
+                                               const lh_buffer* norm_weight, float eps, const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t n,
+                                               lh_buffer* output, lh_buffer* copy, float cap) {
+    const char* op = "linear_residual_norm_vector_copied";
+    LH_REQUIRE(batch, "%s: batch is null", op);
+    LH_REQUIRE(cap >= 0.0f, "%s: cap %g", op, (double)cap);
+    LH_NEED(input, (size_t)k * 4, op, "input");
+    LH_NEED(branch, (size_t)k * 4, op, "branch");
+    LH_NEED(branch_weight, (size_t)k * 4, op, "branch_weight");
+    LH_NEED(norm_weight, (size_t)k * 4, op, "norm_weight");
+    LH_NEED(output, (size_t)n * 4, op, "output");
+    LH_NEED(copy, (size_t)n * 4, op, "copy");
+    VectorStage st{};
+    st.x = input->ptr; st.x_f32 = 1; st.add = (const float*)branch->ptr; st.norm_weight = (const float*)branch_weight->ptr; st.eps = branch_eps;
+    st.outer_weight = (const float*)norm_weight->ptr; st.outer_eps = eps;
+    const uint64_t cus = (uint64_t)batch->ctx->cu_count;
+    if (k % 8 == 0 && k > 0 && k <= 2048 && n > 8 * cus && weight && ((uintptr_t)weight->ptr & 15) == 0 && lh_stage_aligned(st)) {
+        LH_TRY(check_common(batch, weight, bias, k, n, op));
+        LhSegments seg;
+        const uint32_t act = LH_ACT_NONE, layout = LH_ROWS;
+        LH_TRY(lh_make_segments(seg, op, 1, 0, 1, &n, &act, &n, &n, &layout, &output, LH_F32, 0, nullptr));
+        seg.cap = cap;
+        const uint32_t grid = one_row_grid(n, k, 8, 64, cus);
+#define LH_MVC(NLOADS) hipLaunchKernelGGL((matvec_bf16_reg_kernel<kResidualNorm, NLOADS, 8, true>), dim3(grid), dim3(512), 0, batch->ctx->stream, st, (const uint16_t*)weight->ptr, \
+                                          bias ? (const float*)bias->ptr : nullptr, seg, n, k, (float*)copy->ptr)
+        if (k <= 512) LH_MVC(1);
+        else if (k <= 1024) LH_MVC(2);
+        else LH_MVC(4);
+#undef LH_MVC
+        const int r = lh_check_launch(op);
+        if (r == LH_OK) batch->dispatch_count++;
+        return r;
+    }
+    LH_TRY(lh_residual_rows_into(batch, input, branch, branch_weight, input, nullptr, LH_F32, k, 1, branch_eps));
+    return lh_linear_norm_vector_copied_into(batch, input, norm_weight, eps, weight, bias, k, n, output, copy, cap);
 }
 
 int lh_linear_residual_vector_into(lh_batch* batch, const lh_buffer* input, const lh_buffer* branch, lh_buffer* store, const lh_buffer* norm_weight,

@@ -29,7 +29,7 @@ uint32_t lh_expert_tile_rows(uint32_t slots, uint32_t experts);
 // ---- one row: the activation vector in registers -------------------------------------------------------------------------
 // Up to 4096 columns a wave keeps the vector itself: lane l holds the NL chunks of eight elements 8 (64 c + l), which is what
 // it multiplies in every row.
-enum { kPlain = 0, kNorm = 1, kGated = 2, kResidual = 3 };
+enum { kPlain = 0, kNorm = 1, kGated = 2, kResidual = 3, kResidualNorm = 4 };   // the last: a residual, and the norm of it
 struct VectorStage {
     const void* x;             // plain: x_f32 ? f32 : bf16; the others: f32
     uint32_t x_f32;
@@ -39,6 +39,8 @@ struct VectorStage {
     const void* gate;          // gated
     uint32_t gate_f32, gate_act, gate_first, group;   // gated: the gate multiplies before the norm; elements per normed part
     float eps;
+    const float* outer_weight; // residual and norm: of the norm
+    float outer_eps;
 };
 
 __device__ __forceinline__ void lh_ld8(const float* p, float (&v)[8]) {
@@ -62,7 +64,7 @@ __device__ __forceinline__ void lh_ld8(const uint16_t* p, float (&v)[8]) {
 // rows, then `finish`.  And behind a load that not every path makes the compiler waits for all there are, so every load here is
 // made: lanes and waves without a chunk load one that exists, and an operand that is not there is read from x.
 constexpr int kVectorWaves = 8;
-template <int W = kVectorWaves> struct LhVectorSpace { float4 x[2 * W][64]; float part[W]; };
+template <int W = kVectorWaves> struct LhVectorSpace { float4 x[2 * W][64]; float part[W], outer[W]; };
 
 // Eight values at element k, stored as f32 or bf16.
 struct LhEither8 {
@@ -83,10 +85,11 @@ template <int STAGE, int NL, int W = kVectorWaves>
 struct LhSharedVector {
     static_assert(NL <= W, "a chunk per wave");
     static constexpr bool kAlone = NL == 1;
-    static constexpr bool kNormed = STAGE == kNorm || STAGE == kGated || STAGE == kResidual;
-    static constexpr bool kAdds = STAGE == kNorm || STAGE == kResidual;
+    static constexpr bool kAround = STAGE == kResidualNorm, kBranch = STAGE == kResidual || kAround;
+    static constexpr bool kNormed = STAGE == kNorm || STAGE == kGated || kBranch;
+    static constexpr bool kAdds = STAGE == kNorm || kBranch;
     LhEither8 x, gate;
-    float w[8], more[8];
+    float w[8], more[8], around[8];
 
     __device__ __forceinline__ void fetch(const VectorStage& st, uint32_t K, uint32_t lane, uint32_t wave) {
         const uint32_t k = kAlone ? min(lane * 8, K - 8) : wave < NL ? min((64 * wave + lane) * 8, K - 8) : 0u;
@@ -94,6 +97,7 @@ struct LhSharedVector {
         if constexpr (kNormed) lh_ld8((st.norm_weight ? st.norm_weight : static_cast<const float*>(st.x)) + k, w);
         if constexpr (kAdds) lh_ld8((st.add ? st.add : static_cast<const float*>(st.x)) + k, more);
         if constexpr (STAGE == kGated) gate.load(st.gate, st.gate_f32, k);
+        if constexpr (kAround) lh_ld8(st.outer_weight + k, around);
     }
     __device__ __forceinline__ void finish(const VectorStage& st, uint32_t K, uint32_t lane, uint32_t wave, bool store, LhVectorSpace<W>& sp, float (&xr)[NL][8]) {
         const uint32_t k = (64 * (kAlone ? 0u : wave) + lane) * 8;
@@ -116,7 +120,7 @@ struct LhSharedVector {
         if constexpr (kNormed) {
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                if constexpr (STAGE == kResidual) { sum += more[j] * more[j]; w[j] *= more[j]; }      // the weighted branch
+                if constexpr (kBranch) { sum += more[j] * more[j]; w[j] *= more[j]; }      // the weighted branch
                 else sum += v[j] * v[j];
             }
             sum = in ? sum : 0.0f;
@@ -132,16 +136,32 @@ struct LhSharedVector {
                 for (int e = 0; e < W; e++) sum += (uint32_t)e / per == w0 ? sp.part[e] : 0.0f;
             }
             const float r = rsqrtf(sum / (float)(parts ? st.group : K) + st.eps);
-            if constexpr (STAGE == kResidual)
+            if constexpr (kBranch)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = __builtin_fmaf(w[j], r, v[j]);
             if (STAGE != kGated && store && in && (!kAlone || wave == 0)) {
                 *reinterpret_cast<float4*>(st.store + k) = make_float4(v[0], v[1], v[2], v[3]);
                 *reinterpret_cast<float4*>(st.store + k + 4) = make_float4(v[4], v[5], v[6], v[7]);
             }
-            if constexpr (STAGE != kResidual)
+            if constexpr (!kBranch)
 #pragma unroll
                 for (int j = 0; j < 8; j++) v[j] = v[j] * r * w[j];
+            if constexpr (kAround) {
+                float s = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) s += v[j] * v[j];
+                s = lh_group_sum(in ? s : 0.0f, 64);
+                if constexpr (!kAlone) {
+                    if (lane == 0) sp.outer[wave] = s;
+                    lh_lds_barrier();
+                    s = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < W; e++) s += sp.outer[e];
+                }
+                const float f = rsqrtf(s / (float)K + st.outer_eps);
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = v[j] * f * around[j];
+            }
         }
         if constexpr (kAlone) {
 #pragma unroll
@@ -164,7 +184,7 @@ struct LhSharedVector {
 };
 
 static inline bool lh_stage_aligned(const VectorStage& st) {
-    return (((uintptr_t)st.x | (uintptr_t)st.add | (uintptr_t)st.store | (uintptr_t)st.norm_weight | (uintptr_t)st.gate) & 15) == 0;
+    return (((uintptr_t)st.x | (uintptr_t)st.add | (uintptr_t)st.store | (uintptr_t)st.norm_weight | (uintptr_t)st.gate | (uintptr_t)st.outer_weight) & 15) == 0;
 }
 
 // Weights are read once per launch: streaming loads.

@@ -142,16 +142,16 @@ class StackPipeline:
         return picked
 
     # ---- encoding -------------------------------------------------------------------------------------------------------
-    def _encode_stack(self, batch, seq: SequenceSlot, n: int, max_position: int, only: Optional[int] = NO_ROW) -> Buffer:
+    def _encode_stack(self, batch, seq: SequenceSlot, n: int, max_position: int, only: Optional[int] = NO_ROW):
         """Embedding and all layer runs of the n tokens in tokens_buf; returns the residual stream: of several tokens that of row `only`,
-        where it names one, and nothing to be read where it is NO_ROW.  The embedding output
+        where it names one, and nothing to be read where it is NO_ROW; and, of one row, what `_encode_head` has still to add to it.  The embedding output
         stays as it is (later passes of a loop add it): the first norm leaves the stream in a buffer of its own.  For one
         token a norm may not write what other workgroups still read, so the stream alternates between two buffers."""
         x0 = self.ws.get("embedded", n * self.config.width * 4)
         self.kernels.embed_rows_bf16_into(batch, self.embed, self.vocab_size, self.config.width, self.tokens_buf, n, x0)
         return self._encode_layers(batch, seq, n, max_position, x0, seq.position_buf, only if n > 1 and self.observe is None else None)
 
-    def _encode_layers(self, batch, seq: SequenceSlot, n: int, max_position: int, x0: Buffer, position: Buffer, only: Optional[int] = None) -> Buffer:
+    def _encode_layers(self, batch, seq: SequenceSlot, n: int, max_position: int, x0: Buffer, position: Buffer, only: Optional[int] = None):
         """With `only` the last layer ends where the rows' keys, values and states are written for all rows but that one: the final norm
         and the head read no other (two passes of 2048 rows, four layers with a routed feed-forward last: 2768 us for all rows, 2501 so)."""
         K, width = self.kernels, self.config.width
@@ -167,10 +167,12 @@ class StackPipeline:
             if self.observe is not None:
                 Norm.flush(r)
                 self.observe(i, r.x, n)
-        Norm.flush(r)
+        pending = r.pending if r.rows == 1 and self.observe is None else None
+        if pending is None:
+            Norm.flush(r)
         if only is None or only == NO_ROW or r.rows < n:
-            return r.x
-        return r.x.view(only * width * 4, width * 4)
+            return r.x, pending
+        return r.x.view(only * width * 4, width * 4), None
 
     def _forward(self, seq: SequenceSlot, tokens, want, out: np.ndarray, wait: bool) -> None:
         """Results are read behind the work, in stream order: one wait for both, and for all pieces of a step."""
@@ -190,7 +192,8 @@ class StackPipeline:
         logits = None
         if len(want) == 1:
             logits = self.logits_host
-            self._encode_head(batch, x if only is not None else x.view(want[0] * width * 4, width * 4), logits)
+            row, pending = x
+            self._encode_head(batch, row if only is not None else row.view(want[0] * width * 4, width * 4), pending, logits)
         elif want:
             m = len(want)
             index = self.ws.get("want", 4 * self.max_rows)
@@ -198,7 +201,7 @@ class StackPipeline:
             logits = self.ws.get("logits", m * self.vocab_size * 4)
             size = 4 if self.dtype == F32 else 2
             h = self.ws.get("wanted", m * width * size)
-            K.norm_rows_f32_into(batch, x, None, self.final_norm.weight, None, index, h, self.dtype, width, m, self.config.eps)
+            K.norm_rows_f32_into(batch, x[0], None, self.final_norm.weight, None, index, h, self.dtype, width, m, self.config.eps)
             self.head.rows_into(batch, K, h, self.dtype, m, [logits], F32)
             self._encode_cap(batch, logits, m)
         if want:
@@ -210,8 +213,15 @@ class StackPipeline:
             batch.commit_and_wait()
         seq.position += n
 
-    def _encode_head(self, batch, row: Buffer, copy: Optional[Buffer] = None) -> None:
+    def _encode_head(self, batch, row: Buffer, pending: Optional[tuple], copy: Optional[Buffer] = None) -> None:
         norm, eps, cap = self.final_norm.weight, self.config.eps, self.config.softcap
+        if pending is not None and copy is not None:
+            branch, outer = pending
+            return self.kernels.linear_residual_norm_vector_copied_into(batch, row, branch, outer.weight, outer.eps, norm, eps, self.head.weight, self.head.bias,
+                                                                        self.head.k, self.vocab_size, self.logits_buf, copy, 0.0 if cap is None else cap)
+        if pending is not None:
+            branch, outer = pending
+            self.kernels.residual_rows_into(batch, row, branch, outer.weight, row, None, F32, outer.dim, 1, outer.eps)
         if copy is not None:
             self.kernels.linear_norm_vector_copied_into(batch, row, norm, eps, self.head.weight, self.head.bias, self.head.k, self.vocab_size,
                                                         self.logits_buf, copy, 0.0 if cap is None else cap)
@@ -227,11 +237,11 @@ class StackPipeline:
 
     def _encode_decode(self, batch, seq: SequenceSlot, max_position: int, pick: bool) -> None:
         if pick:
-            self._encode_head(batch, self._encode_stack(batch, seq, 1, max_position))
+            self._encode_head(batch, *self._encode_stack(batch, seq, 1, max_position))
             self.kernels.argmax_advance_f32_into(batch, self.logits_buf, self.next_buf, self.vocab_size, seq.position_buf, 1)
         else:
             x0 = self.ws.get("embedded", self.config.width * 4)
-            self._encode_head(batch, self._encode_layers(batch, seq, 1, max_position, x0, self.at_buf), self.logits_host)
+            self._encode_head(batch, *self._encode_layers(batch, seq, 1, max_position, x0, self.at_buf), self.logits_host)
 
     def _decode(self, seq: SequenceSlot, token: int, pick: bool) -> CommandBatch:
         """One token, encoded: logits in logits_buf and, where asked, the largest one's index in next_buf.  The first decoded token of a

@@ -185,6 +185,7 @@ extern "C" {
     pub fn lh_linear_norm_vector_into(batch: *mut lh_batch, input: *const lh_buffer, add: *const lh_buffer, store: *mut lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
     pub fn lh_linear_norm_vector_capped_into(batch: *mut lh_batch, input: *const lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, n: u32, output: *mut lh_buffer, cap: f32) -> c_int;
     pub fn lh_linear_norm_vector_copied_into(batch: *mut lh_batch, input: *const lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, n: u32, output: *mut lh_buffer, copy: *mut lh_buffer, cap: f32) -> c_int;
+    pub fn lh_linear_residual_norm_vector_copied_into(batch: *mut lh_batch, input: *mut lh_buffer, branch: *const lh_buffer, branch_weight: *const lh_buffer, branch_eps: f32, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, n: u32, output: *mut lh_buffer, copy: *mut lh_buffer, cap: f32) -> c_int;
     pub fn lh_linear_residual_vector_into(batch: *mut lh_batch, input: *const lh_buffer, branch: *const lh_buffer, store: *mut lh_buffer, norm_weight: *const lh_buffer, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;
     pub fn lh_gated_vector_fits(k: u32, group: u32) -> u32;
     pub fn lh_linear_gated_vector_into(batch: *mut lh_batch, input: *const lh_buffer, gate: *const lh_buffer, gate_dtype: c_int, gate_act: u32, gate_first: c_int, norm_weight: *const lh_buffer, group: u32, eps: f32, weight: *const lh_buffer, bias: *const lh_buffer, k: u32, count: u32, ns: *const u32, acts: *const u32, heads: *const u32, padded: *const u32, layouts: *const u32, outputs: *const *mut lh_buffer, output_dtype: c_int, accumulate: c_int, position: *const lh_buffer) -> c_int;

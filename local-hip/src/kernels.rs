@@ -617,6 +617,13 @@ impl Kernels {
         check(unsafe { ffi::lh_linear_norm_vector_copied_into(batch.as_ptr(), input.as_ptr(), norm_weight.as_ptr(), eps, weight.as_ptr(), bias.as_ptr(), k, n, output.as_ptr(), copy.as_ptr(), cap) })
     }
 
+    /// `lh_linear_residual_norm_vector_copied_into` (include/local_hip.h).
+    #[allow(clippy::too_many_arguments)]
+    pub fn linear_residual_norm_vector_copied_into(&self, batch: &mut CommandBatch, input: &Buffer, branch: &Buffer, branch_weight: &Buffer, branch_eps: f32, norm_weight: &Buffer, eps: f32, weight: &Buffer, bias: &Buffer, k: u32, n: u32, output: &Buffer, copy: &Buffer, cap: f32) -> Result<()> {
+        // SAFETY: every pointer comes from a live handle of this crate; the library validates sizes and shapes.
+        check(unsafe { ffi::lh_linear_residual_norm_vector_copied_into(batch.as_ptr(), input.as_ptr(), branch.as_ptr(), branch_weight.as_ptr(), branch_eps, norm_weight.as_ptr(), eps, weight.as_ptr(), bias.as_ptr(), k, n, output.as_ptr(), copy.as_ptr(), cap) })
+    }
+
     /// `lh_linear_residual_vector_into` (include/local_hip.h).
     #[allow(clippy::too_many_arguments)]
     pub fn linear_residual_vector_into(&self, batch: &mut CommandBatch, input: &Buffer, branch: &Buffer, store: &Buffer, norm_weight: &Buffer, eps: f32, weight: &Buffer, bias: &Buffer, k: u32, count: u32, ns: &[u32], acts: &[u32], heads: &[u32], padded: &[u32], layouts: &[u32], outputs: &[&Buffer], output_dtype: c_int, accumulate: c_int, position: &Buffer) -> Result<()> {

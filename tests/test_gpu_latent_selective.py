@@ -563,6 +563,26 @@ def test_copied_products(ai, gpu, k, n, cap):
         K.linear_norm_vector_copied_into(batch, x, norm, 1e-6, w, bias, k, n, b.view(0, n * 4 - 4), c, cap)
 
 
+@pytest.mark.parametrize("k,n", [(64, 3000), (512, 2049), (768, 5000), (1024, 32000), (2048, 4111), (2048, 300), (2056, 5000), (20, 9)])
+def test_copied_products_of_a_residual(ai, gpu, k, n):
+    """A branch's norm, the norm of the sum and the product in one launch, against the three: f32 sums in another order."""
+    ctx, K = gpu
+    g, batch = np.random.default_rng(k), ai.CommandBatch(ctx)
+    x, y = (g.standard_normal(k).astype(np.float32) * s for s in (3, 40))
+    w, bw, nw = upload(ai, ctx, g.standard_normal((n, k), np.float32), ai.BF16), *(upload(ai, ctx, 1 + 0.1 * g.standard_normal(k), ai.F32) for _ in range(2))
+    bias, branch = upload(ai, ctx, g.standard_normal(n), ai.F32), upload(ai, ctx, y, ai.F32)
+    a, b, c, d = *(ai.Buffer.empty(ctx, n * 4) for _ in range(2)), *(ai.Buffer.pinned(ctx, n * 4) for _ in range(2))
+    one, two = upload(ai, ctx, x, ai.F32), upload(ai, ctx, x, ai.F32)
+    K.residual_rows_into(batch, one, branch, bw, one, None, ai.F32, k, 1, 1e-6)
+    K.linear_norm_vector_copied_into(batch, one, nw, 1e-5, w, bias, k, n, a, c, 30.0)
+    K.linear_residual_norm_vector_copied_into(batch, two, branch, bw, 1e-6, nw, 1e-5, w, bias, k, n, b, d, 30.0)
+    batch.commit_and_wait()
+    want, device, host = a.as_array(np.float32), b.as_array(np.float32), d.as_array(np.float32)
+    assert (device == host).all()
+    # two sums of squares in another order: each factor within (log2 k + 2) roundings of the other's, and as much again for what is multiplied
+    assert np.abs(host - want).max() <= (np.log2(k) + 8) * 2.0 ** -23 * 30.0 and np.abs(want).max() > 1
+
+
 @pytest.mark.parametrize("n", [1, 63, 64, 1000, 16384, 16385, 40000])
 def test_argmax_and_position(ai, gpu, n):
     """The first of several largest values, wherever they lie, and the position moved on behind it."""
