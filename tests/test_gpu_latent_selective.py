@@ -281,7 +281,8 @@ def test_sink_and_gate_of_many_rows_in_splits(ai, gpu, heads, kv_heads, dim, vdi
     test_softmax_attention_with_sink_and_gate(ai, gpu, "bf16", heads, kv_heads, dim, vdim, start, rows)
 
 
-@pytest.mark.parametrize("heads,vdim,state,groups,taps", [(1, 3, 5, 1, 1), (4, 24, 20, 2, 4), (3, 33, 64, 3, 2), (2, 64, 128, 1, 3), (6, 16, 130, 2, 6), (2, 20, 300, 1, 4), (2, 8, 12, 1, 20)])
+@pytest.mark.parametrize("heads,vdim,state,groups,taps", [(1, 3, 5, 1, 1), (4, 24, 20, 2, 4), (3, 33, 64, 3, 2), (2, 64, 128, 1, 3), (6, 16, 130, 2, 6), (2, 20, 300, 1, 4), (2, 8, 12, 1, 20),
+                                                          (3, 17, 33, 3, 4), (2, 64, 128, 1, 4), (4, 15, 127, 2, 4), (1, 1, 1, 1, 4)])
 @pytest.mark.parametrize("cuts", [[1, 1, 1, 1, 1], [2, 2, 1, 2], [17, 1, 65, 2, 130], [63, 1, 64, 1], [200]])
 def test_selective_state_space(ai, gpu, heads, vdim, state, groups, taps, cuts):
     """The kernels from the projections to the recurrence's output, in portions, and the states left behind: all f32, and bf16
