@@ -55,10 +55,11 @@ struct ShortWave {
 template <int S>
 struct Group { u32x4_t k[4], v[4 / S]; uint32_t nk, nv; uint32_t lo, hi; };
 
-// Walsh-Hadamard transform of a head in a wave, a lane with dims lane + 64 j, pairs as in lh_fwht_lds.
-__device__ __forceinline__ void transform_head(float (&v)[4], uint32_t lane) {
+// Walsh-Hadamard transform of a head of 64 N dims in a wave, a lane with dims lane + 64 j, pairs as in lh_fwht_lds.
+template <int N>
+__device__ __forceinline__ void transform_head(float (&v)[N], uint32_t lane) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < N; j++) {
         v[j] = lh_fwht_lane_stage<1>(v[j], lane);
         v[j] = lh_fwht_lane_stage<2>(v[j], lane);
         v[j] = lh_fwht_lane_stage<4>(v[j], lane);
@@ -66,9 +67,15 @@ __device__ __forceinline__ void transform_head(float (&v)[4], uint32_t lane) {
         v[j] = lh_fwht_lane_stage<16>(v[j], lane);
         v[j] = lh_fwht_lane_stage<32>(v[j], lane);
     }
-    const float a = __fadd_rn(v[0], v[1]), b = __fsub_rn(v[0], v[1]), c = __fadd_rn(v[2], v[3]), d = __fsub_rn(v[2], v[3]);
-    v[0] = __fadd_rn(a, c); v[2] = __fsub_rn(a, c);
-    v[1] = __fadd_rn(b, d); v[3] = __fsub_rn(b, d);
+#pragma unroll
+    for (int s = 1; s < N; s *= 2)
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            if (j & s) continue;
+            const float a = v[j], b = v[j | s];
+            v[j] = __fadd_rn(a, b);
+            v[j | s] = __fsub_rn(a, b);
+        }
 }
 
 // Where finished heads go as f16 behind the rotation out of code space, as hadamard_rotate_kernel makes it (a workgroup with all dims of a query).
@@ -342,6 +349,43 @@ __device__ __forceinline__ void short_by_levels(const AttnPointers& a, const Att
 
 __device__ __forceinline__ float level_of(float table, int i) { return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(table), i)); }
 
+// The raw values of a head: the splits in order, in f32, rounded to f16 as decode_qkv_prepare_kernel does, or finished rows (a lane's first value at `raw`).
+template <int N>
+__device__ __forceinline__ void raw_head(uint16_t (&h)[N], const TokenPrep& t, uint32_t row, uint32_t column, const uint16_t* raw, uint32_t lane) {
+    if (t.partial) {
+        const size_t zstride = (size_t)t.rows * t.part_cols;
+        const float* part = t.partial + (size_t)row * t.part_cols + column + lane;
+        float acc[N] = {};
+        for (uint32_t z0 = 0; z0 < t.splits; z0 += 8) {
+            float x[8][N];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; u++)
+#pragma unroll
+                for (int j = 0; j < N; j++) x[u][j] = part[(size_t)(z0 + u < t.splits ? z0 + u : t.splits - 1) * zstride + 64 * j];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; u++)
+#pragma unroll
+                for (int j = 0; j < N; j++) if (z0 + u < t.splits) acc[j] += x[u][j];
+        }
+#pragma unroll
+        for (int j = 0; j < N; j++) h[j] = lh_f2h(acc[j]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; j++) h[j] = raw[64 * j];
+    }
+}
+// The codes of a head, four to a byte.
+template <int N>
+__device__ __forceinline__ void store_codes(uint8_t* bytes, const uint32_t (&code)[N], uint32_t lane) {
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        uint32_t b = code[j] << 2 * (lane & 3);
+        b |= (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR1>((int)b);
+        b |= (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR2>((int)b);
+        if ((lane & 3) == 0) bytes[(lane >> 2) + 16 * j] = (uint8_t)b;
+    }
+}
+
 // The leading arguments arrive in registers with the wave (see the Makefile); the structures repeat them.
 template <int S>
 __global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_short_kernel(const float* queries, const float* levels, uint32_t q_heads, uint32_t kv_heads, const AttnPointers a,
@@ -390,48 +434,54 @@ struct TokenShared {
     float square[2][kDim];
 };
 
-// One head in a wave: out[j] becomes the f16 value of dim lane + 64 j behind the norm (`normalise`).
-__device__ __forceinline__ void norm_head(uint16_t (&h)[4], const uint16_t (&w)[4], bool weighted, float eps) {
-    float s[4];
+// One head in a wave: h[j] becomes the f16 value of dim lane + 64 j behind the norm.
+template <int N>
+__device__ __forceinline__ void norm_head(uint16_t (&h)[N], const uint16_t (&w)[N], bool weighted, float eps) {
+    float total = 0.0f, s[N];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < N; j++) {
         const float x = lh_h2f(h[j]);
         float sq = x * x;
         asm volatile("" : "+v"(sq));                            // (rounded before it is added)
         s[j] = lh_group_sum(sq, 64);
     }
-    const float rms = rsqrtf((((0.0f + s[0]) + s[1]) + s[2] + s[3]) / (float)kDim + eps);
 #pragma unroll
-    for (int j = 0; j < 4; j++) h[j] = lh_f2h_exact(lh_norm_product(lh_h2f(h[j]), rms, weighted ? lh_h2f(w[j]) : 1.0f));
+    for (int j = 0; j < N; j++) total += s[j];
+    const float rms = rsqrtf(total / (float)(64 * N) + eps);
+#pragma unroll
+    for (int j = 0; j < N; j++) h[j] = lh_f2h_exact(lh_norm_product(lh_h2f(h[j]), rms, weighted ? lh_h2f(w[j]) : 1.0f));
 }
-__device__ __forceinline__ void turn_head(uint16_t (&h)[4], const float2* turn, uint32_t angles, uint32_t lane) {
+template <int N>
+__device__ __forceinline__ void turn_head(uint16_t (&h)[N], const float2* turn, uint32_t angles, uint32_t lane) {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
+    for (int j = 0; j < N / 2; j++) {
         if (lane + 64 * j >= angles) continue;
         const float2 t = turn[lane + 64 * j];
-        lh_rope_apply(lh_h2f(h[j]), lh_h2f(h[j + 2]), t.x, t.y, h[j], h[j + 2]);
+        lh_rope_apply(lh_h2f(h[j]), lh_h2f(h[j + N / 2]), t.x, t.y, h[j], h[j + N / 2]);
     }
 }
 // The codes of a head and its norm, as encode_vector makes them (turboquant_kv.hip): the squares, their sum from left to right as the CPU
 // encoder has it, the rest.
-__device__ __forceinline__ void place_squares(const uint16_t (&h)[4], float* square, uint32_t lane) {
+template <int N>
+__device__ __forceinline__ void place_squares(const uint16_t (&h)[N], float* square, uint32_t lane) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) square[lane + 64 * j] = lh_h2f(h[j]) * lh_h2f(h[j]);
+    for (int j = 0; j < N; j++) square[lane + 64 * j] = lh_h2f(h[j]) * lh_h2f(h[j]);
     __builtin_amdgcn_wave_barrier();
 }
-__device__ __forceinline__ float add_squares(float sum, const float* square, uint32_t first) {       // half of them
+__device__ __forceinline__ float add_squares(float sum, const float* square, uint32_t first, uint32_t count = kDim / 2) {       // half of them
 #pragma unroll 8
-    for (uint32_t i = first; i < first + kDim / 2; i += 4) {
+    for (uint32_t i = first; i < first + count; i += 4) {
         const float4 q = *reinterpret_cast<const float4*>(&square[i]);
         sum += q.x; sum += q.y; sum += q.z; sum += q.w;
     }
     return sum;
 }
-__device__ __forceinline__ uint16_t encode_head(const uint16_t (&h)[4], float sum, const float (&sign)[4], const float (&level)[4], float inv_sqrt_d, uint32_t lane, uint32_t (&code)[4]) {
+template <int N>
+__device__ __forceinline__ uint16_t encode_head(const uint16_t (&h)[N], float sum, const float (&sign)[N], const float (&level)[4], float inv_sqrt_d, uint32_t lane, uint32_t (&code)[N]) {
     const float norm = __fsqrt_rn(sum), inv = __fdiv_rn(1.0f, norm);
-    float v[4];
+    float v[N];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < N; j++) {
         v[j] = lh_h2f(h[j]);
         if (norm > 0.0f) v[j] = __fmul_rn(v[j], inv);
         v[j] = __fmul_rn(v[j], sign[j]);
@@ -439,7 +489,7 @@ __device__ __forceinline__ uint16_t encode_head(const uint16_t (&h)[4], float su
     }
     transform_head(v, lane);
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < N; j++) {
         float y = __fmul_rn(v[j], inv_sqrt_d), best = INFINITY;
         asm volatile("" : "+v"(y));                             // (rounded before the levels are taken off)
         code[j] = 0;
@@ -483,28 +533,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_token_kernel(cons
     uint16_t h[4] = {0, 0, 0, 0}, w[4] = {0, 0, 0, 0};
     float sign[4];
     if (works) {
-        if (t.partial) {                                        // the splits in order, in f32, rounded to f16: as decode_qkv_prepare_kernel
-            const size_t zstride = (size_t)t.rows * t.part_cols;
-            const float* part = t.partial + (size_t)qi * t.part_cols + column + lane;
-            float acc[4] = {0.f, 0.f, 0.f, 0.f};
-            for (uint32_t z0 = 0; z0 < t.splits; z0 += 8) {
-                float x[8][4];
-#pragma unroll
-                for (uint32_t u = 0; u < 8; u++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) x[u][j] = part[(size_t)(z0 + u < t.splits ? z0 + u : t.splits - 1) * zstride + 64 * j];
-#pragma unroll
-                for (uint32_t u = 0; u < 8; u++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) if (z0 + u < t.splits) acc[j] += x[u][j];
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) h[j] = lh_f2h(acc[j]);
-        } else {
-            const uint16_t* const raw = (is_q ? t.q : is_v ? t.v : t.k) + row_at;
-#pragma unroll
-            for (int j = 0; j < 4; j++) h[j] = raw[64 * j];
-        }
+        raw_head(h, t, qi, column, (is_q ? t.q : is_v ? t.v : t.k) + row_at, lane);
         if (norm_w)
 #pragma unroll
             for (int j = 0; j < 4; j++) w[j] = norm_w[lane + 64 * j];
@@ -592,16 +621,67 @@ __global__ __launch_bounds__(64 * kMaxWaves) void attention_tq_token_kernel(cons
         lh_lds_barrier();                                       // short_body's, ahead of the merge
         if (blockIdx.x != 0) return;
         const size_t slot = ((size_t)lane_base + (p.ring_capacity ? position % p.ring_capacity : position)) * kv_heads + kvh;
-        uint8_t* const bytes = (is_v ? t.v_codes : t.k_codes) + slot * (kDim / 4);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            uint32_t b = code[j] << 2 * (lane & 3);
-            b |= (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR1>((int)b);
-            b |= (uint32_t)lh_dpp_i<LH_DPP_QUAD_XOR2>((int)b);
-            if ((lane & 3) == 0) bytes[(lane >> 2) + 16 * j] = (uint8_t)b;
-        }
+        store_codes((is_v ? t.v_codes : t.k_codes) + slot * (kDim / 4), code, lane);
         if (lane == 0) (is_v ? t.v_norms : t.k_norms)[slot] = norm;
     }
+}
+
+// The preparation by itself: a wave a head, in registers as above, a workgroup some heads of a row, or all of them, with the rotary pairs once.  What bounds many rows is
+// vector instructions: with a workgroup a head and the pairs' cosines and sines in each of them decode_qkv_prepare_kernel took 13.0 us for 256 rows of 10 heads of 256 dims and 18.3
+// of 512; now 7.3 and 10.0.  Few rows are bound by what a CU reads of the partial tiles, so that a
+// workgroup takes fewer heads there (64 rows of 512 dims, with keys and values and without: 9.2 us on average with all heads, 7.8).  The same bits.
+struct RowsPrep { float* rq; const float* levels; const uint32_t* positions; uint32_t position, ring_capacity, lane_capacity, q_heads, kv_heads; };
+constexpr uint32_t kRowHeads = 16;
+template <int N>
+__global__ __launch_bounds__(64 * kRowHeads) void prepare_rows_kernel(const RowsPrep r, const TokenPrep t) {
+    constexpr uint32_t D = 64 * N;
+    __shared__ float2 turn[D / 2];
+    extern __shared__ __align__(16) float squares[];            // [waves][D]
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = blockIdx.x, b = blockIdx.y * (blockDim.x >> 6) + wave;
+    const bool is_q = b < r.q_heads, is_v = b >= r.q_heads + r.kv_heads, works = b < r.q_heads + 2 * r.kv_heads;
+    const uint32_t head = is_q ? b : is_v ? b - r.q_heads - r.kv_heads : b - r.q_heads;
+    const size_t row_at = ((size_t)row * (is_q ? r.q_heads : r.kv_heads) + head) * D + lane;
+    const uint16_t* const norm_w = is_q ? t.q_norm : is_v ? nullptr : t.k_norm;
+    uint16_t h[N] = {}, w[N] = {};
+    float sign[N];
+    if (works) raw_head(h, t, row, b * D, (is_q ? t.q : is_v ? t.v : t.k) + row_at, lane);
+    if (norm_w)
+#pragma unroll
+        for (int j = 0; j < N; j++) w[j] = norm_w[lane + 64 * j];
+#pragma unroll
+    for (int j = 0; j < N; j++) sign[j] = t.signs[lane + 64 * j];
+    const float table = works && !is_q ? r.levels[lane & 3] : 0.0f;        // (null where there are queries alone)
+    const uint32_t position = r.positions ? r.positions[row] : r.position + row, angles = (uint32_t)((float)D * t.prf) / 2;
+    for (uint32_t i = tid; i < D / 2; i += blockDim.x) {
+        float c = 1.0f, s = 0.0f;
+        if (i < angles) lh_rope_cos_sin(i, D, position, t.theta, c, s);
+        turn[i] = make_float2(c, s);
+    }
+    if (is_v || norm_w) norm_head(h, w, !is_v, t.eps);
+    lh_lds_barrier();
+    if (!works) return;
+    if (!is_v) turn_head(h, turn, angles, lane);
+    uint16_t* const to = (is_q ? t.q_out : is_v ? t.v_out : t.k_out) + row_at;
+#pragma unroll
+    for (int j = 0; j < N; j++) to[64 * j] = h[j];
+    if (is_q) {
+        float x[N];
+#pragma unroll
+        for (int j = 0; j < N; j++) { x[j] = __fmul_rn(lh_h2f(h[j]), sign[j]); asm volatile("" : "+v"(x[j])); }
+        transform_head(x, lane);
+#pragma unroll
+        for (int j = 0; j < N; j++) r.rq[row_at + 64 * j] = __fmul_rn(x[j], t.inv_sqrt_d);
+        return;
+    }
+    float* const square = squares + wave * D;
+    place_squares(h, square, lane);
+    const float sum = add_squares(0.0f, square, 0, D);
+    const float level[4] = {level_of(table, 0), level_of(table, 1), level_of(table, 2), level_of(table, 3)};
+    uint32_t code[N];
+    const uint16_t norm = encode_head(h, sum, sign, level, t.inv_sqrt_d, lane, code);
+    const size_t slot = ((size_t)row * r.lane_capacity + (r.ring_capacity ? position % r.ring_capacity : position)) * r.kv_heads + head;
+    store_codes((is_v ? t.v_codes : t.k_codes) + slot * (D / 4), code, lane);
+    if (lane == 0) (is_v ? t.v_norms : t.k_norms)[slot] = norm;
 }
 
 template <int S> constexpr size_t short_lds(uint32_t waves) { return sizeof(ShortShared) + waves * sizeof(ShortWave<S>); }
@@ -642,6 +722,22 @@ int lh_attention_short_init(lh_context* ctx) {
 }
 
 namespace lh_attn {
+
+bool prepare_rows_supported(const lh_context* ctx, uint32_t head_dim, uint32_t bits, uint32_t heads, uint32_t rows) {
+    // Heads of 512 dims that have a CU each are the shorter way with a workgroup each (10 heads: one row 7.8 and 7.0 us, 8 rows 8.1 and 7.3, 64 rows 7.4 and 10.1).
+    return bits == 2 && heads <= kRowHeads && (head_dim == kDim || (head_dim == 2 * kDim && (uint64_t)rows * heads > (uint64_t)ctx->cu_count));
+}
+
+int launch_prepare_rows(lh_context* ctx, const char* op, const TokenPrep& t, uint32_t head_dim, uint32_t rows, float* rq, const float* levels, const uint32_t* positions, uint32_t position,
+                        uint32_t ring_capacity, uint32_t lane_capacity, uint32_t q_heads, uint32_t kv_heads) {
+    const RowsPrep r{rq, levels, positions, position, ring_capacity, lane_capacity, q_heads, kv_heads};
+    const auto kernel = head_dim == kDim ? prepare_rows_kernel<4> : prepare_rows_kernel<8>;
+    // As many heads a workgroup as leave every CU one.
+    const uint32_t heads = q_heads + 2 * kv_heads, cus = (uint32_t)ctx->cu_count, each = (uint32_t)std::min<uint64_t>(((uint64_t)rows * heads + cus - 1) / cus, kRowHeads);
+    const uint32_t groups = (heads + each - 1) / each, waves = (heads + groups - 1) / groups;
+    hipLaunchKernelGGL(kernel, dim3(rows, groups), dim3(64 * waves), (size_t)waves * head_dim * 4, ctx->stream, r, t);
+    return lh_check_launch(op);
+}
 
 bool short_supported(const lh_context* ctx, const AttnParams& p, uint64_t max_span) {
     static const bool off = [] { return getenv("LOCAL_HIP_ATTN_PAIR") != nullptr; }();      // (forces a form of the other kernel)

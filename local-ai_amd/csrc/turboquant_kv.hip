@@ -16,6 +16,7 @@
 //   - nearest level with strict '<' from index 0 (lowest index wins ties).
 // This file is compiled with -ffp-contract=off: no product may be fused into a sum.
 #include "common.hpp"
+#include "attention_tq.hpp"
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -541,6 +542,17 @@ int lh_prepare_rows_launch(lh_batch* batch, const LhPrepareRows& a, const float*
     if (partial) LH_REQUIRE(splits >= 1 && (uint64_t)(n_q_heads + (write_kv ? 2 * n_kv_heads : 0)) * head_dim <= part_cols,
                             "%s: partial tiles of %u columns do not hold the heads", op, part_cols);
     if (check_only) return LH_OK;
+    if (lh_attn::prepare_rows_supported(batch->ctx, head_dim, bits, n_q_heads + 2 * p.n_kv_heads, rows)) {
+        lh_attn::TokenPrep t{p.q_raw, p.k_raw, p.v_raw, partial, splits, rows, part_cols, (uint16_t*)q->ptr, write_kv ? (uint16_t*)k->ptr : nullptr,
+                             write_kv ? (uint16_t*)v->ptr : nullptr, q_norm ? (const uint16_t*)q_norm->ptr : nullptr,
+                             (write_kv && k_norm) ? (const uint16_t*)k_norm->ptr : nullptr, (const float*)signs->ptr, write_kv ? (uint8_t*)k_codes->ptr : nullptr,
+                             write_kv ? (uint8_t*)v_codes->ptr : nullptr, write_kv ? (uint16_t*)k_norms->ptr : nullptr, write_kv ? (uint16_t*)v_norms->ptr : nullptr,
+                             eps, theta, partial_rotary_factor, p.inv_sqrt_d, nullptr};
+        r = lh_attn::launch_prepare_rows(batch->ctx, op, t, head_dim, rows, (float*)rq->ptr, write_kv ? (const float*)levels->ptr : nullptr,
+                                         positions ? (const uint32_t*)positions->ptr : nullptr, start_position, ring_capacity, lane_capacity, n_q_heads, p.n_kv_heads);
+        if (r == LH_OK) batch->dispatch_count++;
+        return r;
+    }
     hipLaunchKernelGGL(decode_qkv_prepare_kernel, dim3((uint32_t)groups), dim3(head_dim), 0, batch->ctx->stream, (uint16_t*)q->ptr,
                        write_kv ? (uint16_t*)k->ptr : nullptr, write_kv ? (uint16_t*)v->ptr : nullptr,
                        q_norm ? (const uint16_t*)q_norm->ptr : nullptr, (write_kv && k_norm) ? (const uint16_t*)k_norm->ptr : nullptr,

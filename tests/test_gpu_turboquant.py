@@ -267,6 +267,36 @@ def test_decode_qkv_prepare_equals_the_separate_kernels(pkg, gpu, oracle, hd, n_
     assert not c["kc"].as_array(np.uint8).any()
 
 
+@pytest.mark.parametrize("hd,rows,prf,mode", [(256, 1, 1.0, "ring"), (256, 300, 0.25, "ring"), (256, 5, 1.0, "lanes"), (256, 9, 0.0, "query"), (512, 1, 0.25, "ring"), (512, 70, 1.0, "plain"),
+                                              (512, 5, 0.25, "lanes"), (512, 33, 0.25, "query")])
+@pytest.mark.parametrize("weighted", [True, False])
+def test_prepared_rows_of_few_and_of_many_heads_are_the_same(pkg, gpu, oracle, hd, rows, prf, mode, weighted):
+    """Heads that a workgroup's sixteen waves take and the same ones beside more than it can take (the general kernel): all bits, also of heads
+    of zeros and of large values."""
+    ctx, K = gpu
+    g = np.random.default_rng(hd + rows)
+    own, cb, cap = mode != "query", oracle.tq_code_bytes(hd, 2), 640
+    ring, lane_cap = {"ring": (512, 0), "plain": (0, 0), "lanes": (600, cap), "query": (0, 0)}[mode]
+    pos = pkg.Buffer.from_slice(ctx, g.integers(0, 5000, rows).astype(np.uint32)) if mode == "lanes" else None
+    raw = (g.standard_normal((rows, 17, hd)) * 2).astype(np.float16)
+    raw[0, 3], raw[-1, 5], raw[0, 15], raw[-1, 16, :3] = 0, 40000, 0, -65504
+    kv = [raw[:, 15:16].copy(), raw[:, 16:17].copy()]
+    lv, sg = pkg.Buffer.from_slice(ctx, oracle.tq_levels(hd, 2)), pkg.Buffer.from_slice(ctx, oracle.rotation_signs(hd))
+    qw, kw = (pkg.Buffer.from_slice(ctx, (0.25 * (1 + 0.1 * g.standard_normal(hd))).astype(np.float16)) if weighted else None for _ in range(2))
+    slots, got = max(rows * lane_cap, 1000), []
+    for n_q in ((14, 15) if own else (16, 17)):
+        heads = np.ascontiguousarray(raw[:, :n_q])
+        q, k, v = (pkg.Buffer.from_slice(ctx, x) for x in (heads, *kv))
+        rq, kc, vc, kn, vn = (pkg.Buffer.empty(ctx, n) for n in (rows * n_q * hd * 4, slots * cb, slots * cb, slots * 2, slots * 2))
+        batch, only = pkg.CommandBatch(ctx), lambda b: b if own else None
+        K.decode_qkv_prepare_rows_into(batch, q, only(k), only(v), qw, only(kw), lv, sg, rq, only(kc), only(kn), only(vc), only(vn), pos, hd, n_q, 1, rows, 1e-6, 0 if mode == "plain" else 400,
+                                       1e4, prf, 2, ring, lane_cap)
+        batch.commit_and_wait()
+        first = [b.as_array(np.uint8).reshape(rows, n_q, -1)[:, :14] for b in (q, rq)]
+        got.append(first + [b.as_array(np.uint8) for b in (k, v, kc, vc, kn, vn)])
+    assert all(np.array_equal(x, y) for x, y in zip(*got)) and got[0][1].any()
+
+
 @pytest.mark.parametrize("lanes_mode", [False, True])
 def test_decode_qkv_prepare_rows_equals_row_by_row(pkg, gpu, oracle, lanes_mode):
     """Several tokens in one dispatch -- consecutive positions of one sequence on a ring that wraps inside the call, or
