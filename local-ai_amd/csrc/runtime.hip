@@ -572,8 +572,9 @@ int lh_batch_write(lh_batch* batch, lh_buffer* dst, size_t offset, const void* s
         batch->ctx->desc_used[slot] = true;
         return LH_OK;
     }
-    hipError_t e = hipMemcpyAsync(to, src, len, hipMemcpyHostToDevice, batch->ctx->stream);
+    hipError_t e = dst->host ? hipSuccess : hipMemcpyAsync(to, src, len, hipMemcpyHostToDevice, batch->ctx->stream);
     if (e == hipSuccess) e = wait_for_stream(batch->ctx);
+    if (e == hipSuccess && dst->host) memcpy((char*)dst->host + offset, src, len);
     if (e != hipSuccess) return lh_fail(LH_ERR_COMMAND_BUFFER, "GPU error: batch_write: %s", hipGetErrorString(e));
     return LH_OK;
 }

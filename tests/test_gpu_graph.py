@@ -242,3 +242,49 @@ def test_reads_of_every_route(pkg, gpu, size, offset, behind):
     out = np.full(size + 32, 7, np.uint8)
     b.read_into(out[16:size + 16], offset)
     assert np.array_equal(out[16:size + 16], src[offset:offset + size]) and (out[:16] == 7).all() and (out[size + 16:] == 7).all()
+
+
+def test_pinned_buffers_take_what_device_buffers_take(pkg, gpu):
+    """Writes of every size and way, views, copies from and to device memory, zeros."""
+    ctx, K = gpu
+    data = np.random.default_rng(5).integers(0, 256, 200003, dtype=np.uint8)
+    p, d = pkg.Buffer.pinned(ctx, data.size), pkg.Buffer.empty(ctx, data.size)
+    assert not p.as_array(np.uint8).any()
+    p.copy_from_bytes(data)
+    assert np.array_equal(p.as_array(np.uint8), data) and np.array_equal(p.view(77, 1000).as_array(np.uint8), data[77:1077])
+    batch = pkg.CommandBatch(ctx)
+    batch.blit_copy(p, 16, d, 0, 100000)
+    for at, n in ((3, 60), (100, 2000), (4096, 5000), (20000, 100000)):
+        batch.write(p.view(at, n), data[:n])
+        assert np.array_equal(p.as_array(np.uint8)[at:at + n], data[:n]), n
+    assert np.array_equal(d.as_array(np.uint8)[:100000], data[16:100016])
+    batch.blit_copy(d, 0, p, 0, data.size)
+    assert np.array_equal(p.as_array(np.uint8)[:100000], data[16:100016])
+    p.fill_zero()
+    assert not p.as_array(np.uint8).any()
+
+
+def test_replays_write_a_pinned_buffer_and_keep_one_that_was_freed(pkg, gpu):
+    """A recorded product with results in pinned memory, replayed on new inputs between eager work; a buffer that went while it was recorded lives as long."""
+    ctx, K = gpu
+    g = pkg.synth.rng(8, 1)
+    rows, cols = 66001, 2048
+    w = pkg.QuantWeight.from_bytes(ctx, pkg.synth.weights("q4_0", rows, cols, g), pkg.Q4_0, rows, cols)
+    xs = [pkg.synth.activations(1, cols, g)[0].astype(np.float16) for _ in range(4)]
+    x, y, eager = pkg.Buffer.from_slice(ctx, xs[0]), pkg.Buffer.empty(ctx, rows * 4), pkg.Buffer.empty(ctx, rows * 4)
+    kept, gone = pkg.Buffer.pinned(ctx, rows * 4), pkg.Buffer.pinned(ctx, rows * 4)
+    batch = pkg.CommandBatch(ctx)
+    w.matvec_copied_into(batch, K, x, y, kept, 0.0)
+    batch.commit_and_wait()
+    batch.begin_capture()
+    w.matvec_copied_into(batch, K, x, y, gone, 30.0)
+    w.matvec_copied_into(batch, K, x, y, kept, 0.0)
+    gone.free()
+    graph = batch.end_capture()
+    for v in xs:
+        x.copy_from_bytes(v)
+        graph.launch()
+        got = kept.as_array(np.uint32)
+        w.matvec_f32out_into(batch, K, x, eager)
+        batch.commit_and_wait()
+        assert np.array_equal(got, eager.as_array(np.uint32)) and np.array_equal(got, y.as_array(np.uint32))
