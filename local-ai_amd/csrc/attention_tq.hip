@@ -439,7 +439,7 @@ bool token_preparation(const lh_context* ctx, const AttnParams& p, const AttnPoi
 int attention_dispatch(lh_batch* batch, const char* op, const lh_buffer* rq, const lh_buffer* k_codes, const lh_buffer* k_norms,
                        const lh_buffer* v_codes, const lh_buffer* v_norms, const lh_buffer* levels, lh_buffer* out,
                        const lh_buffer* positions, AttnParams p, uint64_t max_span, uint64_t phys_slots, const RotateBack* rot = nullptr,
-                       float* ws_override = nullptr, size_t ws_override_floats = 0, const Preparation* prep = nullptr) {
+                       float* ws_override = nullptr, size_t ws_override_floats = 0, const Preparation* prep = nullptr, bool check_only = false) {
     if (!batch) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: batch is null", op);
     if (p.bits < 2 || p.bits > 4) return lh_fail(LH_ERR_INVALID_ARGUMENT, "%s: TurboQuant bits must be 2..=4, got %u", op, p.bits);
     if (p.head_dim == 0 || (p.head_dim & (p.head_dim - 1)) || p.head_dim > 512)
@@ -463,6 +463,7 @@ int attention_dispatch(lh_batch* batch, const char* op, const lh_buffer* rq, con
         LH_NEED(rot->signs, (size_t)p.head_dim * 4, op, "signs");
         LH_NEED(rot->out16, qbytes / 2, op, "out_f16");
     }
+    if (check_only) return LH_OK;
 
     float* const ws = ws_override ? ws_override : (float*)ctx->workspace;
     const size_t ws_avail = ws_override ? ws_override_floats : (ctx->workspace_bytes / 2) / 4;   // floats; the lower half of the workspace
@@ -697,7 +698,7 @@ static int batched_common(const char* op, lh_batch* batch, const lh_buffer* rq, 
                           const lh_buffer* v_codes, const lh_buffer* v_norms, const lh_buffer* levels, lh_buffer* out,
                           const lh_buffer* positions, uint32_t head_dim, uint32_t lane_capacity, uint32_t num_q_heads,
                           uint32_t num_kv_heads, uint32_t window, uint32_t bits, uint32_t n_lanes, uint32_t ring_capacity,
-                          const RotateBack* rot, const Preparation* prep = nullptr) {
+                          const RotateBack* rot, const Preparation* prep = nullptr, bool check_only = false) {
     AttnParams p{};
     p.head_dim = head_dim; p.bits = bits; p.num_q_heads = num_q_heads; p.num_kv_heads = num_kv_heads;
     p.window = window; p.ring_capacity = ring_capacity; p.lane_capacity = lane_capacity; p.mode = kBatched; p.num_queries = n_lanes;
@@ -707,7 +708,7 @@ static int batched_common(const char* op, lh_batch* batch, const lh_buffer* rq, 
     const uint64_t cap = ring_capacity ? ring_capacity : lane_capacity;
     const uint64_t span = window ? std::min<uint64_t>(window, cap) : cap;
     const uint64_t phys = (uint64_t)n_lanes * lane_capacity * num_kv_heads;
-    return attention_dispatch(batch, op, rq, k_codes, k_norms, v_codes, v_norms, levels, out, positions, p, span, phys, rot, nullptr, 0, prep);
+    return attention_dispatch(batch, op, rq, k_codes, k_norms, v_codes, v_norms, levels, out, positions, p, span, phys, rot, nullptr, 0, prep, check_only);
 }
 
 int lh_flash_attention_tq_batched_into(lh_batch* batch, const lh_buffer* rq, const lh_buffer* k_codes, const lh_buffer* k_norms,
@@ -730,9 +731,10 @@ int lh_flash_attention_tq_batched_rotated_into(lh_batch* batch, const lh_buffer*
 
 }  // extern "C"
 
-int lh_attend_lanes(lh_batch* batch, const LhPrepareRows& a, const float* partial, uint32_t splits, uint32_t part_cols, const LhAttendLanes& t, const char* op) {
+int lh_attend_lanes(lh_batch* batch, const LhPrepareRows& a, const float* partial, uint32_t splits, uint32_t part_cols, const LhAttendLanes& t, const char* op,
+                    bool check_only) {
     const RotateBack rot{a.signs, t.out_f16};
     const Preparation prep{a, partial, splits, part_cols};
     return batched_common(op, batch, a.rq, t.k_codes, t.k_norms, t.v_codes, t.v_norms, t.levels, t.out, a.positions, a.head_dim, a.lane_capacity, a.n_q_heads,
-                          t.n_kv_heads, t.window, a.bits, a.rows, a.ring_capacity, &rot, &prep);
+                          t.n_kv_heads, t.window, a.bits, a.rows, a.ring_capacity, &rot, &prep, check_only);
 }

@@ -184,12 +184,13 @@ struct LhPrepareRows {
 };
 int lh_prepare_rows_launch(lh_batch* batch, const LhPrepareRows& a, const float* partial, uint32_t splits, uint32_t part_cols, bool check_only = false);
 // The attention of a by-lane pool behind the preparation `a` (or around it, where one launch does both), heads rotated to f16; defined in attention_tq.hip.
+// check_only validates the arguments and launches nothing.
 struct LhAttendLanes {
     const lh_buffer *k_codes, *k_norms, *v_codes, *v_norms, *levels;
     lh_buffer *out, *out_f16;
     uint32_t n_kv_heads, window;
 };
-int lh_attend_lanes(lh_batch* batch, const LhPrepareRows& a, const float* partial, uint32_t splits, uint32_t part_cols, const LhAttendLanes& t, const char* op);
+int lh_attend_lanes(lh_batch* batch, const LhPrepareRows& a, const float* partial, uint32_t splits, uint32_t part_cols, const LhAttendLanes& t, const char* op, bool check_only = false);
 int lh_launch_hadamard_fh(lh_context* ctx, const float* input, const float* signs, uint16_t* output, uint32_t head_dim, uint32_t num_heads);
 
 // Stream-ordered copy of a host-built descriptor table to device memory.  The host block may be freed as soon as this

@@ -1981,10 +1981,12 @@ int lh_matmul_nt_qkv_attention_lanes_into(lh_batch* b, lh_quant fmt, const lh_bu
     LhPrepareRows a{q, kv ? k : nullptr, kv ? v : nullptr, q_norm, kv ? k_norm : nullptr, kv ? levels : nullptr, signs, rq, kv ? k_codes : nullptr, kv ? k_norms : nullptr,
                     kv ? v_codes : nullptr, kv ? v_norms : nullptr, positions, head_dim, n_q_heads, kv ? n_kv_heads : 0u, lanes, eps, 0, theta, partial_rotary_factor, bits,
                     ring_capacity, lane_capacity};
-    int r = lh_prepare_rows_launch(b, a, nullptr, 0, 0, true);   // the second half's arguments, before anything is launched
+    int r = lh_prepare_rows_launch(b, a, nullptr, 0, 0, true);   // what comes behind the product: its arguments, before anything is launched
     if (r != LH_OK) return r;
     if (lanes == 0 || k_dim == 0) return LH_OK;
     const LhAttendLanes t{k_codes, k_norms, v_codes, v_norms, levels, out, out_f16, n_kv_heads, window};
+    r = lh_attend_lanes(b, a, nullptr, 0, 0, t, op, true);
+    if (r != LH_OK) return r;
     const uint32_t ns[3] = {n_q_heads * head_dim, n_kv_heads * head_dim, n_kv_heads * head_dim};
     const lh_buffer* const ws[3] = {w_q, w_k, w_v};
     SkinnyPartials kept{nullptr, 0, 0};

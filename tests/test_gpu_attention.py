@@ -830,3 +830,43 @@ def test_lanes_in_one_step_equal_product_preparation_and_attention(pkg, gpu, ora
     with pytest.raises(pkg.InvalidArgument):
         K.matmul_nt_qkv_attention_lanes_into(pkg.CommandBatch(ctx), ty, x, ws[0], ws[1], None, k_dim, b["q"], b["k"], b["v"], qw, kw, lv, sg, rq, b["kc"], b["kn"],
                                              b["vc"], b["vn"], pos, out, o16, hd, n_q, n_kv, lanes, eps, theta, 1.0, window, bits, ring, cap)
+
+
+@pytest.mark.parametrize("lanes,window,ring,cap", [(64, 512, 1024, 1024), (3, 0, 0, 700)])
+@pytest.mark.parametrize("own", [True, False])
+def test_lanes_in_one_step_refuses_before_anything_runs(pkg, gpu, oracle, lanes, window, ring, cap, own):
+    """Arguments of the attention, which comes last: nothing is launched, and the outputs of the products are as they were."""
+    ctx, K = gpu
+    hd, n_q, n_kv, k_dim = 256, 8, 1, 1536
+    g = pkg.synth.rng(79, lanes)
+    ws = [pkg.Buffer.from_slice(ctx, pkg.synth.weights("q4_0", n, k_dim, g)) for n in (n_q * hd, hd, hd)]
+    x = pkg.Buffer.from_slice(ctx, g.standard_normal(lanes * k_dim, dtype=np.float32).astype(np.float16))
+    slots = lanes * cap * n_kv
+    args = dict(levels=pkg.Buffer.from_slice(ctx, oracle.tq_levels(hd, 2)), kc=pkg.Buffer.empty(ctx, slots * hd // 4), kn=pkg.Buffer.empty(ctx, slots * 2),
+                vc=pkg.Buffer.empty(ctx, slots * hd // 4), vn=pkg.Buffer.empty(ctx, slots * 2), out=pkg.Buffer.empty(ctx, lanes * n_q * hd * 4),
+                o16=pkg.Buffer.empty(ctx, lanes * n_q * hd * 2))
+    sg, rq = pkg.Buffer.from_slice(ctx, oracle.rotation_signs(hd)), pkg.Buffer.empty(ctx, lanes * n_q * hd * 4)
+    w, pos = pkg.Buffer.from_slice(ctx, np.ones(hd, np.float16)), pkg.Buffer.from_slice(ctx, np.full(lanes, 3, np.uint32))
+    q, k, v = (pkg.Buffer.from_slice(ctx, np.full(lanes * n * hd, 7, np.float16)) for n in (n_q, n_kv, n_kv))
+
+    def step(batch, n_kv=n_kv, **other):
+        a = {**args, **other}
+        K.matmul_nt_qkv_attention_lanes_into(batch, pkg.Q4_0, x, ws[0], ws[1] if own else None, ws[2] if own else None, k_dim, q, k if own else None, v if own else None, w,
+                                             w, a["levels"], sg, rq, a["kc"], a["kn"], a["vc"], a["vn"], pos, a["out"], a["o16"], hd, n_q, n_kv, lanes, 1e-6, 1e4, 1.0,
+                                             window, 2, ring, cap)
+    for name in args:
+        batch = pkg.CommandBatch(ctx)
+        with pytest.raises(pkg.InvalidArgument):
+            step(batch, **{name: args[name].view(0, args[name].length() - 2)})
+        assert batch.dispatch_count() == 0, name
+    batch = pkg.CommandBatch(ctx)
+    if not own:                                                # (three heads of another's cache: eight queries are no multiple)
+        with pytest.raises(pkg.InvalidArgument):
+            step(batch, n_kv=3)
+    assert batch.dispatch_count() == 0
+    batch.commit_and_wait()
+    assert all((b.as_array(np.float16) == 7).all() for b in (q, k, v))
+    step(batch)
+    assert batch.dispatch_count() > 0
+    batch.commit_and_wait()
+    assert not (q.as_array(np.float16) == 7).all()
