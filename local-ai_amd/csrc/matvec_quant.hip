@@ -29,6 +29,7 @@ constexpr int kWG = 256;          // threads per workgroup (4 waves)
 constexpr int kWaves = kWG / 64;
 constexpr uint32_t kMaxFastCols = 16384;  // 4 unit columns per lane at most
 constexpr size_t kMaxDynamicLds = 96 * 1024;   // what launch_typed raises a kernel's dynamic LDS limit to
+constexpr size_t kStaticLds = 2048;            // more than a kernel has beside it (the copying form: 1 KB of results)
 
 struct MatvecProblem {
     const uint8_t* matrix;
@@ -224,7 +225,8 @@ __device__ __forceinline__ u32x4_t ld16_stream(gptr_t p) {
 // (Streaming launches without one have a form of their own: with the prologues' code in it a 1536-column launch keeps 76 bytes a lane in scratch memory,
 // without 24: the 262144 rows of a token's logits 47-50 us, 42.7.  2048 and more columns: the same time in both.)
 // COPY (staged form, one problem, f32): results are capped and go to a second place too.  A wave takes `copy.run` batches of consecutive rows,
-// whose results meet in LDS and leave together, up to 32 of them, 128 bytes: what the host reads is written over the bus in pieces of that size.
+// whose results meet in LDS and leave together, so that what the host reads is written over the bus in pieces of 128 bytes: a run is as many batches as
+// have up to 32 rows, and one batch where that has more (up to 64, of 256 columns and fewer: the size of `results`).
 struct MatvecCopy { float* to; float cap; uint32_t run; };
 template <int FMT, int L, int NPOS, typename XT, typename YT, bool IMG = false, bool PRO = true, bool COPY = false>
 __global__ __launch_bounds__(kWG, 2) void matvec_quant_kernel(const MatvecProblem* __restrict__ problems, MatvecBase single,
@@ -646,7 +648,7 @@ int launch_typed(lh_context* ctx, const MatvecProblem* dev_problems, const Matve
         if (g.lds_bytes > kMaxDynamicLds)                                                                                   \
             return lh_fail(LH_ERR_INVALID_ARGUMENT, "matvec_quant: %zu bytes of LDS needed, limit %zu", g.lds_bytes,        \
                            (size_t)kMaxDynamicLds);                                                                         \
-        if (g.lds_bytes > 64 * 1024) {   /* long rows: more than the 64 KB a kernel gets without asking */                  \
+        if (g.lds_bytes + kStaticLds > 64 * 1024) {   /* long rows: more than the 64 KB a kernel gets without asking */     \
             const int rl = lh_raise_dynamic_lds(ctx, (const void*)KERNEL, kMaxDynamicLds, "matvec_quant");                  \
             if (rl != LH_OK) return rl;                                                                                     \
         }                                                                                                                   \

@@ -773,7 +773,7 @@ def test_products_of_few_signs_and_large_elements(pkg, gpu, oracle, fmt, kind, r
 
 
 @pytest.mark.parametrize("cap", [0.0, 30.0])
-@pytest.mark.parametrize("rows,cols", [(262144 - 37, 1536), (66001, 2048), (33003, 4096), (20000, 8192), (70007, 1024), (300001, 256), (200000, 64), (32000, 1536), (300, 1536), (7, 96)])
+@pytest.mark.parametrize("rows,cols", [(262144 - 37, 1536), (66001, 2048), (33003, 4096), (20000, 8192), (20000, 6464), (20000, 6528), (20000, 6656), (70007, 1024), (300001, 256), (200000, 64), (32000, 1536), (300, 1536), (7, 96)])
 def test_matvec_q4_0_results_in_pinned_memory_too(pkg, gpu, rows, cols, cap):
     """One to three batches of rows in a wave's run, ragged ends, and shapes without the staged form: both places hold the product's bits, capped."""
     ctx, K = gpu
