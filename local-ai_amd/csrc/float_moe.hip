@@ -181,8 +181,9 @@ __global__ __launch_bounds__(256) void vector_up_kernel(const float* __restrict_
 // there is less than the launch that they had (two of 16 experts, 2048 -> 1024 columns: 4.5 us and 3.2 with the step between them, 6.2 now; 8 experts, 1024 -> 512: 3.4 and 3.3, 4.1).
 constexpr int kRouted = 4;
 template <int NL, int WAVES, int ROUTE>
-__global__ __launch_bounds__(64 * WAVES) void vector_up_reg_kernel(const VectorStage st, float* __restrict__ logits, const uint16_t* __restrict__ router, const uint16_t* __restrict__ up,
-                                                           float* __restrict__ hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act) {
+__global__ __launch_bounds__(64 * WAVES) void vector_up_reg_kernel(const VectorStage st, const float* __restrict__ logits, const uint16_t* __restrict__ up,
+                                                           float* __restrict__ hidden, uint32_t experts, uint32_t top, uint32_t width, uint32_t ff, uint32_t act,
+                                                           const uint16_t* __restrict__ router, float* __restrict__ left) {
     __shared__ uint32_t ids[WAVES][kMaxTop];
     __shared__ float weights[WAVES][kMaxTop];
     __shared__ LhVectorSpace<WAVES> space;
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(64 * WAVES) void vector_up_reg_kernel(const VectorS
             acc = lh_group_sum(acc, 64);
             const uint32_t e = wave + i * WAVES;
             if (lane == 0) routed[e] = acc;
-            if (blockIdx.x == 0 && c == 0 && lane == 0 && e < experts) logits[e] = acc;
+            if (blockIdx.x == 0 && c == 0 && lane == 0 && e < experts) left[e] = acc;
         }
         lh_lds_barrier();
         select_experts_of<1>(routed, experts, c + 1, lane, ids[wave], weights[wave]);
@@ -431,14 +432,16 @@ static int vector_up(lh_batch* batch, const char* op, const lh_buffer* input, co
     VectorStage st{};
     st.x = input->ptr; st.x_f32 = 1; st.norm_weight = (const float*)norm_weight->ptr; st.eps = eps;
     if (width % 8 == 0 && width <= 4096 && ((uintptr_t)up->ptr & 15) == 0 && lh_stage_aligned(st)) {
-        // (four waves where all rows are at most eight per CU, as the one-row products; with the router and more than 1024 columns eight, so that half as many
-        // workgroups read it: 16 experts, 2048 columns 6.2 us and 7.0; 8 experts, 1024 columns 4.5 and 4.1)
-        const uint32_t cus = (uint32_t)batch->ctx->cu_count, w = width <= (router ? 1024u : 2048u) && (uint64_t)ff * top <= 8ull * cus ? 4 : kVectorWaves;
-        const bool route = router && experts <= kRouted * w && ((uintptr_t)router->ptr & 15) == 0;
+        // (four waves where all rows are at most eight per CU, as the one-row products; with the router in the launch and more than 1024 columns eight, so that
+        // half as many workgroups read it: 16 experts, 2048 columns 6.2 us and 7.0; 8 experts, 1024 columns 4.5 and 4.1.  Behind a
+        // router of its own launch four are the better ones again: both launches of 33 experts, 2 x 256 rows of 2048 columns 6.7 us, with eight 7.0)
+        const uint32_t cus = (uint32_t)batch->ctx->cu_count, alone = width <= 2048 && (uint64_t)ff * top <= 8ull * cus ? 4 : kVectorWaves, beside = width > 1024 ? kVectorWaves : alone;
+        const bool route = router && experts <= kRouted * beside && ((uintptr_t)router->ptr & 15) == 0;
+        const uint32_t w = route ? beside : alone;
         if (router && !route) LH_TRY(route_vector(batch, input, norm_weight, eps, router, logits, experts, width));
         const dim3 grid(std::min<uint32_t>((ff + w - 1) / w, std::max<uint32_t>(1, (w == 4 ? 2 : 1) * cus / top)), top);
-#define LH_UP_R(NL, WAVES, R) hipLaunchKernelGGL((vector_up_reg_kernel<NL, WAVES, R>), grid, dim3(64 * WAVES), 0, batch->ctx->stream, st, (float*)logits->ptr, \
-                                                 route ? (const uint16_t*)router->ptr : nullptr, (const uint16_t*)up->ptr, (float*)hidden->ptr, experts, top, width, ff, act)
+#define LH_UP_R(NL, WAVES, R) hipLaunchKernelGGL((vector_up_reg_kernel<NL, WAVES, R>), grid, dim3(64 * WAVES), 0, batch->ctx->stream, st, route ? nullptr : (const float*)logits->ptr, \
+                                                 (const uint16_t*)up->ptr, (float*)hidden->ptr, experts, top, width, ff, act, route ? (const uint16_t*)router->ptr : nullptr, (float*)logits->ptr)
 #define LH_UP(NL, WAVES) do { if (!route) LH_UP_R(NL, WAVES, 0); else if (experts <= WAVES) LH_UP_R(NL, WAVES, 1); else if (experts <= 2 * WAVES) LH_UP_R(NL, WAVES, 2); else LH_UP_R(NL, WAVES, kRouted); } while (0)
         if (w == 4) {
             if (width <= 512) LH_UP(1, 4);

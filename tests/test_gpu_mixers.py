@@ -877,7 +877,7 @@ def test_mixture_of_experts(ai, gpu, dtype, rows, experts, top, width, ff):
 
 
 @pytest.mark.parametrize("experts,top,width,ff", [(16, 2, 2048, 1024), (8, 2, 1024, 512), (17, 3, 2048, 1024), (5, 5, 512, 40), (32, 4, 1536, 1536), (33, 1, 4096, 900), (1, 1, 64, 8),
-                                                  (6, 2, 100, 24), (16, 2, 1368, 688)])
+                                                  (6, 2, 100, 24), (16, 2, 1368, 688), (33, 2, 1536, 256), (64, 4, 2048, 512), (32, 4, 1032, 512), (17, 2, 1024, 512)])
 def test_router_in_the_launch_of_the_experts(ai, gpu, experts, top, width, ff):
     """The bits of the router's product and of the experts' own launch behind it, with and without room for the router."""
     ctx, K = gpu
