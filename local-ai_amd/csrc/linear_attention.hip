@@ -712,13 +712,16 @@ int launch_recurrent(lh_context* ctx, const RecurrentArgs& a, const char* op) {
     const uint64_t columns = (uint64_t)a.heads * a.vdim;
     // A wave a column from 65 key columns on (below, half its lanes would have none): few rows always (us of 1, 2 and 7 rows of 16 heads, bf16, then so: 128 x 128 5.4,
     // 6.4, 12.1 and 4.8, 4.6, 4.9; 256 x 128 10.7, 14.6, 33.2 and 4.7, 4.6, 4.8), and of many rows where a lane of the other form would hold
-    // more than eight values or compute the rows' steps (200 rows of 48 heads, f32: 256 x 128 189 and 99, selective 128 x 128 186 and 98);
-    // else up to two waves a SIMD (128 x 128, 8, 16 and 24 heads: 39, 40, 40 and 21, 33, 47).
-    if (whole && a.dq > 64 && a.dq <= 512 && (a.rows < 8 || a.dq > 128 || DECAY == kSelective || columns <= 8ull * (uint64_t)ctx->cu_count)) {
+    // more than eight 32-bit values or compute the rows' steps (200 rows of 48 heads, f32: 256 x 128 189 and 99, selective 128 x 128 186 and 98);
+    // else up to two waves a SIMD (128 x 128, 8, 16 and 24 heads: 39, 40, 40 and 21, 33, 47), of bf16 with 129 to 256 key columns, whose two values share a
+    // register there, up to five (200 rows of 256 x 128 with 32, 40, 48 and 64 heads: 66, 88, 88 and 88 us, and 63, 78, 91 and 119).
+    const uint64_t cus = (uint64_t)ctx->cu_count;
+    const bool few = a.rows < 8, wide = few || DECAY == kSelective || (a.dq <= 128 ? columns <= 8 * cus : sizeof(T) == 4 || a.dq > 256 || columns <= 20 * cus);
+    if (whole && a.dq > 64 && a.dq <= 512 && wide) {
         const dim3 blocks((uint32_t)((columns + 3) / 4));
 #define LH_REC(NR_, AHEAD_) hipLaunchKernelGGL((recurrent_wide_kernel<T, NR_, AHEAD_, DECAY>), blocks, dim3(256), 0, ctx->stream, a)
-        if (a.dq <= 128) { if (a.rows < 8) LH_REC(2, 4); else LH_REC(2, 16); }
-        else if (a.dq <= 256) { if (a.rows < 8) LH_REC(4, 4); else LH_REC(4, 8); }
+        if (a.dq <= 128) { if (few) LH_REC(2, 4); else LH_REC(2, 16); }
+        else if (a.dq <= 256) { if (few) LH_REC(4, 4); else LH_REC(4, 8); }
         else LH_REC(8, 4);
 #undef LH_REC
         return lh_check_launch(op);
@@ -728,6 +731,7 @@ int launch_recurrent(lh_context* ctx, const RecurrentArgs& a, const char* op) {
         if (a.dq <= 32) LH_REC(2, 8);
         else if (a.dq <= 64) LH_REC(4, 8);
         else if (a.dq <= 128) { if constexpr (DECAY != kSelective) LH_REC(8, 8); }
+        else if (a.dq <= 256) { if constexpr (DECAY != kSelective && sizeof(T) == 2) LH_REC(16, 4); }
         else LH_REC(64, 1);
 #undef LH_REC
         return lh_check_launch(op);

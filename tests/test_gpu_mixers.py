@@ -617,7 +617,7 @@ def test_recurrence_over_rows(ai, gpu, dtype, dim, rows):
     assert not got[:, :, dim:].any()
 
 
-@pytest.mark.parametrize("heads,vdim,dim", [(16, 128, 128), (41, 50, 128), (41, 50, 100), (33, 64, 65), (17, 128, 160)])
+@pytest.mark.parametrize("heads,vdim,dim", [(16, 128, 128), (41, 50, 128), (41, 50, 100), (33, 64, 65), (17, 128, 160), (40, 128, 160), (81, 64, 256), (44, 117, 129), (3, 50, 300)])
 @pytest.mark.parametrize("rows", [1, 7, 8, 33])
 def test_recurrence_of_many_columns(ai, gpu, heads, vdim, dim, rows):
     """Around the columns beyond which many rows share a wave's lanes, with fixed decays and with a head's steps computed from the token."""
@@ -626,21 +626,29 @@ def test_recurrence_of_many_columns(ai, gpu, heads, vdim, dim, rows):
     dq = K.linear_attention_padded_dim(dim)
     q, k, v = (M.rounded(g.standard_normal(s) / np.sqrt(dim)) for s in ((rows, heads, dim), (rows, heads, dim), (rows, heads, vdim)))
     decay, S = np.linspace(0.4, 1.0, heads).astype(np.float32), g.standard_normal((heads, dim, vdim)).astype(np.float32)
+    raw, (dt_bias, a_log, skip) = g.standard_normal((rows, heads)).astype(np.float32), g.standard_normal((3, heads)).astype(np.float32)
     qp, kp = np.full((rows, heads, dq), 3.0), np.full((rows, heads, dq), 3.0)
     qp[..., :dim], kp[..., :dim] = q, k
     state = np.zeros((heads, vdim, dq), np.float32)
     state[:, :, :dim] = S.transpose(0, 2, 1)
     for dt in (ai.BF16, ai.F32):
-        st, out = ai.Buffer.from_slice(ctx, state), empty(ai, ctx, rows * heads * vdim, ai.F32)
-        batch = ai.CommandBatch(ctx)
-        K.linear_attention_recurrent_into(batch, upload(ai, ctx, qp, dt), upload(ai, ctx, kp, dt), upload(ai, ctx, v, dt), dt, st, ai.Buffer.from_slice(ctx, decay), out,
-                                          rows, heads, dim, vdim, 0.5)
-        batch.commit_and_wait()
-        want, end = O.lightning_recurrence(q, k, v, decay.astype(np.float64), S.astype(np.float64))
-        close(download(ai, out, rows * heads * vdim, ai.F32).reshape(rows, heads, vdim), 0.5 * want, F32_TOL, "output")
-        got = st.as_array(np.float32, heads * vdim * dq).reshape(heads, vdim, dq)
-        close(got[:, :, :dim], end.transpose(0, 2, 1), F32_TOL, "state")
-        assert not got[:, :, dim:].any()
+        buffers = [upload(ai, ctx, x, dt) for x in (qp, kp, v)]
+        for selective in (False, True):
+            st, out = ai.Buffer.from_slice(ctx, state), empty(ai, ctx, rows * heads * vdim, ai.F32)
+            batch = ai.CommandBatch(ctx)
+            if selective:
+                K.selective_recurrent_into(batch, buffers[2], buffers[1], buffers[0], dt, *(ai.Buffer.from_slice(ctx, x) for x in (raw, dt_bias, a_log, skip)), st, out,
+                                           rows, heads, vdim, heads, dim)
+                want, end = O.selective_recurrence(v, k, q, O.softplus(raw.astype(np.float64) + dt_bias), a_log.astype(np.float64), skip.astype(np.float64), S.astype(np.float64))
+            else:
+                K.linear_attention_recurrent_into(batch, *buffers, dt, st, ai.Buffer.from_slice(ctx, decay), out, rows, heads, dim, vdim, 0.5)
+                want, end = O.lightning_recurrence(q, k, v, decay.astype(np.float64), S.astype(np.float64))
+                want = 0.5 * want
+            batch.commit_and_wait()
+            close(download(ai, out, rows * heads * vdim, ai.F32).reshape(rows, heads, vdim), want, F32_TOL, "output")
+            got = st.as_array(np.float32, heads * vdim * dq).reshape(heads, vdim, dq)
+            close(got[:, :, :dim], end.transpose(0, 2, 1), F32_TOL, "state")
+            assert not got[:, :, dim:].any()
 
 
 @pytest.mark.parametrize("heads,dim,vdim", [(4, 32, 48), (3, 20, 33), (2, 64, 128), (1, 128, 80), (2, 200, 48), (2, 8, 100)])
