@@ -618,9 +618,10 @@ def test_recurrence_over_rows(ai, gpu, dtype, dim, rows):
 
 
 @pytest.mark.parametrize("heads,vdim,dim", [(16, 128, 128), (41, 50, 128), (41, 50, 100), (33, 64, 65), (17, 128, 160), (40, 128, 160), (81, 64, 256), (44, 117, 129), (3, 50, 300)])
-@pytest.mark.parametrize("rows", [1, 7, 8, 33])
+@pytest.mark.parametrize("rows", [1, 7, 8, 11, 12, 23, 24, 33])
 def test_recurrence_of_many_columns(ai, gpu, heads, vdim, dim, rows):
-    """Around the columns beyond which many rows share a wave's lanes, with fixed decays and with a head's steps computed from the token."""
+    """Around the columns beyond which many rows share a wave's lanes, and the rows at which it has more of them ahead, with fixed decays and with a
+    head's steps computed from the token."""
     ctx, K = gpu
     g = np.random.default_rng(heads + dim + rows)
     dq = K.linear_attention_padded_dim(dim)
