@@ -73,8 +73,9 @@ struct TokenPrep {
     float eps, theta, prf, inv_sqrt_d;
     uint16_t* rotated;                   // not null: the heads as f16 behind the rotation out of code space, instead of `out`
 };
-// Rows prepared without their attention (decode_qkv_prepare_kernel's other form): heads of 256 or 512 dims and 2-bit codes, as many as a workgroup has waves.
-bool prepare_rows_supported(const lh_context* ctx, uint32_t head_dim, uint32_t bits, uint32_t heads, uint32_t rows);
+// Rows prepared without their attention (decode_qkv_prepare_kernel's other form): heads of 256 or 512 dims and 2-bit codes, as many as a workgroup has waves;
+// `own`: keys and values among them.
+bool prepare_rows_supported(const lh_context* ctx, uint32_t head_dim, uint32_t bits, uint32_t heads, uint32_t rows, bool own);
 int launch_prepare_rows(lh_context* ctx, const char* op, const TokenPrep& t, uint32_t head_dim, uint32_t rows, float* rq, const float* levels, const uint32_t* positions, uint32_t position,
                         uint32_t ring_capacity, uint32_t lane_capacity, uint32_t q_heads, uint32_t kv_heads);
 // What short_supported takes, with room for the two waves that bring in the query's own key and value, on a cache where that position's slot is

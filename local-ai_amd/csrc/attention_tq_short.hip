@@ -723,9 +723,15 @@ int lh_attention_short_init(lh_context* ctx) {
 
 namespace lh_attn {
 
-bool prepare_rows_supported(const lh_context* ctx, uint32_t head_dim, uint32_t bits, uint32_t heads, uint32_t rows) {
-    // Heads of 512 dims that have a CU each are the shorter way with a workgroup each (10 heads: one row 7.8 and 7.0 us, 8 rows 8.1 and 7.3, 64 rows 7.4 and 10.1).
-    return bits == 2 && heads <= kRowHeads && (head_dim == kDim || (head_dim == 2 * kDim && (uint64_t)rows * heads > (uint64_t)ctx->cu_count));
+bool prepare_rows_supported(const lh_context* ctx, uint32_t head_dim, uint32_t bits, uint32_t heads, uint32_t rows, bool own) {
+    // Heads that have a CU each, or are one of a few there, are the shorter way with a workgroup each (four or eight waves instead of one).  Us, that form and this one:
+    // queries alone of 256 dims up to four a CU (8 x 1 3.3 and 3.6; 8 x 64 3.9 and 3.5, but with the attention behind them, from partial tiles, 38.0 and 38.6; 8 x 200 so 69.3 and
+    // 67.9), of 512 dims, whose four a workgroup share their pairs from three a CU on, up to there (8 x 64 36.7 and 37.7, 8 x 100 43.8 and 43.0; 5 x 180 alone 16.4 and 17.4);
+    // with keys and values, whose chain of additions the others wait for, of 512 dims up to two a CU (10 x 1 6.7 and 8.4, 10 x 32 with product and attention 35.3 and 36.1, 10 x 64
+    // 41.3 and 41.6, 10 x 100 49.6 and 48.5).
+    const uint64_t all = (uint64_t)rows * heads, cus = (uint64_t)ctx->cu_count;
+    return bits == 2 && heads <= kRowHeads && (head_dim == kDim || head_dim == 2 * kDim) &&
+           all > (own ? (head_dim == kDim ? 0 : 2 * cus) : (head_dim == kDim || heads % 4 ? 4 : 3) * cus);
 }
 
 int launch_prepare_rows(lh_context* ctx, const char* op, const TokenPrep& t, uint32_t head_dim, uint32_t rows, float* rq, const float* levels, const uint32_t* positions, uint32_t position,

@@ -545,7 +545,7 @@ int lh_prepare_rows_launch(lh_batch* batch, const LhPrepareRows& a, const float*
     if (partial) LH_REQUIRE(splits >= 1 && (uint64_t)(n_q_heads + (write_kv ? 2 * n_kv_heads : 0)) * head_dim <= part_cols,
                             "%s: partial tiles of %u columns do not hold the heads", op, part_cols);
     if (check_only) return LH_OK;
-    if (lh_attn::prepare_rows_supported(batch->ctx, head_dim, bits, n_q_heads + 2 * p.n_kv_heads, rows)) {
+    if (lh_attn::prepare_rows_supported(batch->ctx, head_dim, bits, n_q_heads + 2 * p.n_kv_heads, rows, write_kv)) {
         lh_attn::TokenPrep t{p.q_raw, p.k_raw, p.v_raw, partial, splits, rows, part_cols, (uint16_t*)q->ptr, write_kv ? (uint16_t*)k->ptr : nullptr,
                              write_kv ? (uint16_t*)v->ptr : nullptr, q_norm ? (const uint16_t*)q_norm->ptr : nullptr,
                              (write_kv && k_norm) ? (const uint16_t*)k_norm->ptr : nullptr, (const float*)signs->ptr, write_kv ? (uint8_t*)k_codes->ptr : nullptr,
