@@ -5,68 +5,19 @@
 // in local-metal/src/kernels.rs.  At decode these touch a few KB per call: they are latency bound, one small
 // workgroup per row / head, f32 math, f16 storage with the same rounding points as the reference kernels.
 #include "common.hpp"
+#include "row_norms.hpp"
 #include "xquant.hpp"
 #include <cstdlib>
-#include <type_traits>
 
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ float h_at(const uint16_t* p, size_t i) { return lh_h2f(p[i]); }
-
-// Sum over a workgroup of up to 256 threads (4 waves).
-__device__ __forceinline__ float block_sum(float v, float* scratch, uint32_t threads) {
-    v = lh_group_sum(v, 64);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = (threads + 63) >> 6;
-    if (lane == 0) scratch[wave] = v;
-    __syncthreads();
-    float t = 0.0f;
-#pragma unroll
-    for (int w = 0; w < 4; w++) t = w < nwaves ? t + scratch[w] : t;
-    __syncthreads();
-    return t;
-}
 
 // rms_norm.metal:4-46 / 48-88: out[r, i] = in[r, i] * rsqrt(mean(in[r]^2) + eps) * w[i] (+ residual[r, i]).
 // VEC = 8: 16-byte accesses (dim a multiple of 8, 16-byte aligned rows); VEC = 1 otherwise.
 // ADD with `tail` != 0 is the three-kernel tail of the single-token layer in one dispatch (layer.rs:507-520: rms_norm,
 // residual_add, scale_in_place): the normalised value is rounded to f16, added to the residual as an f16 addition, and,
 // with tail == 2, scaled and rounded once more -- the roundings of the three separate kernels.
-__device__ __forceinline__ float norm_tail(float normed, float res, uint32_t tail, float scale) { return lh_norm_tail(normed, res, tail, scale); }
-
-// The arithmetic of one 8-element chunk, shared by every kernel that must reproduce the stand-alone norm bit for bit.
-__device__ __forceinline__ void rms_sumsq8(const uint4& v, float& s) {
-    const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int j = 0; j < 4; j++) { const float a = lh_h2f((uint16_t)(wv[j] & 0xFFFF)), b = lh_h2f((uint16_t)(wv[j] >> 16)); s += a * a; s += b * b; }
-}
-template <bool ADD>
-__device__ __forceinline__ uint4 rms_apply8(const uint4& v, const uint4& g, const uint4& r, float rms, uint32_t tail, float scale) {
-    const uint32_t wv[4] = {v.x, v.y, v.z, v.w}, wg[4] = {g.x, g.y, g.z, g.w}, wr[4] = {r.x, r.y, r.z, r.w};
-    uint32_t wo[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        float lo = lh_norm_product(lh_h2f((uint16_t)(wv[j] & 0xFFFF)), rms, lh_h2f((uint16_t)(wg[j] & 0xFFFF)));
-        float hi = lh_norm_product(lh_h2f((uint16_t)(wv[j] >> 16)), rms, lh_h2f((uint16_t)(wg[j] >> 16)));
-        if (ADD) {
-            const float rlo = lh_h2f((uint16_t)(wr[j] & 0xFFFF)), rhi = lh_h2f((uint16_t)(wr[j] >> 16));
-            if (tail) { lo = norm_tail(lo, rlo, tail, scale); hi = norm_tail(hi, rhi, tail, scale); }
-            else { lo += rlo; hi += rhi; }
-        }
-        wo[j] = (uint32_t)lh_f2h_exact(lo) | ((uint32_t)lh_f2h_exact(hi) << 16);
-    }
-    return make_uint4(wo[0], wo[1], wo[2], wo[3]);
-}
-
-// Eight values as scale_in_place_gpu_into leaves them.
-__device__ __forceinline__ uint4 scale8(uint4 v, float by) {
-    uint32_t* w = &v.x;
-#pragma unroll
-    for (int j = 0; j < 4; j++) w[j] = (uint32_t)lh_f2h(lh_h2f((uint16_t)(w[j] & 0xFFFF)) * by) | ((uint32_t)lh_f2h(lh_h2f((uint16_t)(w[j] >> 16)) * by) << 16);
-    return v;
-}
-
 // SCALED: the input is what scale_in_place_gpu_into would have made of it.  (Asked at run time, 2560 rows of 2048 with a residual 6.6 -> 7.0 us.)
 template <bool ADD, int VEC, bool SCALED = false>
 __global__ __launch_bounds__(256) void rms_norm_kernel(const uint16_t* in, const uint16_t* __restrict__ w, const uint16_t* res, uint16_t* out,   // out may be in or res
@@ -112,104 +63,6 @@ void launch_rms_norm(hipStream_t stream, const void* in, const void* w, const vo
     };
     if (ADD && before != 1.0f) launch(vec ? rms_norm_kernel<ADD, 8, ADD> : rms_norm_kernel<ADD, 1, ADD>);
     else launch(vec ? rms_norm_kernel<ADD, 8> : rms_norm_kernel<ADD, 1>);
-}
-
-// rms_norm_kernel<ADD, 8> with its input taken either from f16 rows or from the f32 partial tiles of a k-split product
-// (summed in split order and rounded to f16, which is what the product's own reduction would have stored), optionally
-// followed by the output scale (scale_in_place.metal:5-14) and by a second plain norm of the row just produced
-// (layer.rs:640-652: post-attention norm + residual, then the feed-forward norm): up to four dispatches of a decode
-// batch's layer in one.  Same thread count, accumulation order and rounding points as the separate kernels, so the
-// results are theirs bit for bit.  A thread keeps its (two, or up to four) 8-element chunks in registers between the passes.
-// A chain on one CU, bound by its trips to memory: with the loads under conditions the compiler had put five of them one behind the other,
-// and code for four chunks and every tail took more instruction fetches.  64 rows of 1536, three splits, two norms: 5.4 us, now 4.0; 256 rows 4.6 and 4.1.
-template <bool PART, bool ADD, int CHUNKS>
-__global__ __launch_bounds__(256) void rms_norm_fused_kernel(const uint16_t* nw, const uint16_t* res, const uint16_t* nw2, const float* partial, uint32_t dim, uint32_t splits,
-                                                            uint32_t part_rows, uint32_t part_cols, uint32_t threads, const LhNormFused a) {
-    __shared__ float scratch[4];
-    const uint32_t rowi = blockIdx.x;
-    const size_t row = (size_t)rowi * dim;
-    uint4 x[CHUNKS], o[CHUNKS];
-    // The norm weights, the residual and the second norm's weights are requested here, with the row itself: read where they
-    // are used, each waits for memory again behind the barrier of the pass before.  A thread without a chunk reads its row's
-    // first: with a branch around them, the values it would leave alone are put in place behind the loads, and those waited for.
-    const uint16_t* const second = nw2 != nullptr ? nw2 : nw;
-    bool has[CHUNKS];
-    uint32_t at[CHUNKS];
-    uint4 gw[CHUNKS], rr[CHUNKS], gw2[CHUNKS];
-#pragma unroll
-    for (int it = 0; it < CHUNKS; it++) {
-        const uint32_t i = (threadIdx.x + it * threads) * 8;
-        has[it] = i < dim;
-        at[it] = has[it] ? i : 0u;
-        gw[it] = *reinterpret_cast<const uint4*>(nw + at[it]);
-        if (ADD) rr[it] = *reinterpret_cast<const uint4*>(res + row + at[it]);
-        gw2[it] = *reinterpret_cast<const uint4*>(second + at[it]);
-    }
-    if constexpr (PART) {
-        // the splits of two chunks, three at a time (a product has two or three in most layers), are all requested before the first is added (in split order);
-        // past the last split its values are requested again and not added
-        const size_t zstride = (size_t)part_rows * part_cols;
-#pragma unroll
-        for (int it0 = 0; it0 < CHUNKS; it0 += 2) {
-            float v[2][8];
-#pragma unroll
-            for (int c = 0; c < 2; c++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[c][e] = 0.0f;
-            const float* p0 = partial + (size_t)rowi * part_cols + at[it0];
-            const float* p1 = partial + (size_t)rowi * part_cols + at[it0 + 1];
-            for (uint32_t z0 = 0; z0 < splits; z0 += 3) {
-                f32x4 lo[2][3], hi[2][3];
-#pragma unroll
-                for (uint32_t u = 0; u < 3; u++) {
-                    const size_t zo = (size_t)(z0 + u < splits ? z0 + u : splits - 1) * zstride;
-                    lo[0][u] = *reinterpret_cast<const f32x4*>(p0 + zo); hi[0][u] = *reinterpret_cast<const f32x4*>(p0 + zo + 4);
-                    lo[1][u] = *reinterpret_cast<const f32x4*>(p1 + zo); hi[1][u] = *reinterpret_cast<const f32x4*>(p1 + zo + 4);
-                }
-                // All of them before the first addition: left to itself the compiler puts a split's loads behind the additions of the one before.
-                asm volatile("" : "+v"(lo[0][0]), "+v"(hi[0][0]), "+v"(lo[1][0]), "+v"(hi[1][0]), "+v"(lo[0][1]), "+v"(hi[0][1]), "+v"(lo[1][1]), "+v"(hi[1][1]), "+v"(lo[0][2]),
-                             "+v"(hi[0][2]), "+v"(lo[1][2]), "+v"(hi[1][2]));
-#pragma unroll
-                for (uint32_t u = 0; u < 3; u++) {
-                    const bool in = z0 + u < splits;
-#pragma unroll
-                    for (int c = 0; c < 2; c++)
-#pragma unroll
-                        for (int e = 0; e < 8; e++) v[c][e] = in ? v[c][e] + (e < 4 ? lo : hi)[c][u][e & 3] : v[c][e];
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 2; c++)
-                x[it0 + c] = make_uint4((uint32_t)lh_f2h(v[c][0]) | ((uint32_t)lh_f2h(v[c][1]) << 16), (uint32_t)lh_f2h(v[c][2]) | ((uint32_t)lh_f2h(v[c][3]) << 16),
-                                        (uint32_t)lh_f2h(v[c][4]) | ((uint32_t)lh_f2h(v[c][5]) << 16), (uint32_t)lh_f2h(v[c][6]) | ((uint32_t)lh_f2h(v[c][7]) << 16));
-        }
-    } else {
-#pragma unroll
-        for (int it = 0; it < CHUNKS; it++) x[it] = *reinterpret_cast<const uint4*>(a.in + row + at[it]);
-    }
-    float s = 0.0f;
-#pragma unroll
-    for (int it = 0; it < CHUNKS; it++) {
-        float t = s;
-        rms_sumsq8(x[it], t);
-        s = has[it] ? t : s;
-    }
-    const float rms = rsqrtf(block_sum(s, scratch, threads) / (float)dim + a.eps);
-    float s2 = 0.0f;
-#pragma unroll
-    for (int it = 0; it < CHUNKS; it++) {
-        o[it] = rms_apply8<ADD>(x[it], gw[it], ADD ? rr[it] : x[it], rms, 0u, 1.0f);
-        if (a.apply_scale) o[it] = scale8(o[it], a.scale);
-        float t = s2;
-        rms_sumsq8(o[it], t);
-        s2 = has[it] ? t : s2;
-        if (has[it]) *reinterpret_cast<uint4*>(a.out + row + at[it]) = o[it];
-    }
-    if (nw2 == nullptr) return;
-    const float rms2 = rsqrtf(block_sum(s2, scratch, threads) / (float)dim + a.eps);
-#pragma unroll
-    for (int it = 0; it < CHUNKS; it++)
-        if (has[it]) *reinterpret_cast<uint4*>(a.out2 + row + at[it]) = rms_apply8<false>(o[it], gw2[it], o[it], rms2, 0u, 1.0f);
 }
 
 // qk_norm.metal:6-56 (in place; head h of `qk`), and 70-140 with the NEOX rotation fused: the normalised values are
@@ -411,8 +264,6 @@ void lh_launch_logit_softcap(hipStream_t stream, float* data, float cap, uint32_
     hipLaunchKernelGGL(logit_softcap_kernel, dim3(blocks_for(count)), dim3(256), 0, stream, data, cap, count);
 }
 
-bool lh_norm_fused_supported(uint32_t dim) { return (dim & 7) == 0 && dim <= 8192; }
-
 void lh_launch_gelu_mul(hipStream_t stream, const void* a, const void* b, void* out, uint32_t count) {
     launch_elementwise<kGeluMul>(stream, a, b, out, 0.0f, count);
 }
@@ -422,21 +273,6 @@ void lh_launch_gelu_mul_strided(hipStream_t stream, const void* a, const float* 
     const uint32_t items = rows * (dim / 8);
     hipLaunchKernelGGL(gelu_mul_strided_kernel<8>, dim3((items + 255) / 256), dim3(256), 0, stream, (const uint16_t*)a, (const uint16_t*)b,
                        (uint16_t*)out, dim, rows, b_row_stride, b_off, GeluPartials{partial, splits, part_cols});
-}
-
-void lh_launch_norm_fused(hipStream_t stream, const LhNormFused& a) {
-    // the thread count launch_rms_norm picks for 16-byte accesses: the partial sums of the squares add up in the same order
-    const uint32_t threads = a.dim >= 2048 ? 256u : (a.dim >= 1024 ? 128u : 64u);
-    const auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(a.rows), dim3(threads), 0, stream, a.w, a.res, a.w2, a.partial, a.dim, a.splits, a.part_rows, a.part_cols, threads, a);
-    };
-    const auto by_rows = [&](auto chunks) {
-        constexpr int C = decltype(chunks)::value;
-        if (a.partial) launch(a.res ? rms_norm_fused_kernel<true, true, C> : rms_norm_fused_kernel<true, false, C>);
-        else launch(a.res ? rms_norm_fused_kernel<false, true, C> : rms_norm_fused_kernel<false, false, C>);
-    };
-    if (a.dim <= 16 * threads) by_rows(std::integral_constant<int, 2>{});
-    else by_rows(std::integral_constant<int, 4>{});
 }
 
 extern "C" {
