@@ -223,7 +223,8 @@ __device__ __forceinline__ u32x4_t ld16_stream(gptr_t p) {
 
 // One launch serves `count` problems of the same shape (count == 1 for the plain matvec).  PRO: the vector may stand behind a prologue.
 // (Streaming launches without one have a form of their own: with the prologues' code in it a 1536-column launch keeps 76 bytes a lane in scratch memory,
-// without 24: the 262144 rows of a token's logits 47-50 us, 42.7.  2048 and more columns: the same time in both.)
+// without 24: the 262144 rows of a token's logits 47.9 us, 43.2; 65536 x 3072 29.2 and 26.2, x 6144 49.8 and 45.2, x 2048 18.6 and 18.1, x 8192 57.9 and 56.5.  Not for a
+// whole wave a row and a long walk, where it is the longer way: 65536 x 4096 30.8 and 32.1, 131072 54.5 and 56.8; 16384 x 4096 12.1 and 11.8.)
 // COPY (staged form, one problem, f32): results are capped and go to a second place too.  A wave takes `copy.run` batches of consecutive rows,
 // whose results meet in LDS and leave together, so that what the host reads is written over the bus in pieces of 128 bytes: a run is as many batches as
 // have up to 32 rows, and one batch where that has more (up to 64, of 256 columns and fewer: the size of `results`).
@@ -655,10 +656,12 @@ int launch_typed(lh_context* ctx, const MatvecProblem* dev_problems, const Matve
         hipLaunchKernelGGL(KERNEL, dim3(g.grid), dim3(kWG), g.lds_bytes, ctx->stream,                                       \
                            dev_problems, single, count, rows, K, g.lpr_log2, g.steps_per_wg, copy);                         \
     } while (0)
+    // (see the kernel: the form without the prologues' code)
+    const bool bare = single.pro.kind == kXProNone && !(NPOS == 1 && g.lpr_log2 == 6 && g.steps_per_wg >= 64);
 #define LH_LAUNCH(XT, YT)                                                                                                   \
     do {                                                                                                                    \
         if constexpr (FMT == LH_Q4_0 && L == 2) {                                                                           \
-            if (g.img && single.pro.kind == kXProNone) LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, true, false>)); \
+            if (g.img && bare) LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, true, false>));                       \
             else if (g.img) LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, true>));                                 \
             else LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, false>));                                           \
         } else LH_LAUNCH_K((matvec_quant_kernel<FMT, L, NPOS, XT, YT, false>));                                             \
