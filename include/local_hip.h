@@ -758,7 +758,7 @@ LH_API int lh_linear_norm_vector_copied_into(lh_batch* batch, const lh_buffer* i
                                              const lh_buffer* weight, const lh_buffer* bias, uint32_t k, uint32_t n,
                                              lh_buffer* output, lh_buffer* copy, float cap);
 /* lh_residual_rows_into of one row in place, then lh_linear_norm_vector_copied_into of it, in one launch where the product takes
- * eight waves; `input` may hold the sum afterwards or not */
+ * eight waves and leaves the copy itself (more than 1024 columns, or up to 65536 results); `input` may hold the sum afterwards or not */
 LH_API int lh_linear_residual_norm_vector_copied_into(lh_batch* batch, lh_buffer* input, const lh_buffer* branch,
                                                       const lh_buffer* branch_weight, float branch_eps,
                                                       const lh_buffer* norm_weight, float eps, const lh_buffer* weight,

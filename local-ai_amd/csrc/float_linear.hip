@@ -1089,6 +1089,11 @@ uint32_t one_row_grid(uint64_t takes, uint32_t K, uint32_t waves, uint32_t each,
     return (uint32_t)std::max<uint64_t>(std::min<uint64_t>((takes + waves - 1) / waves, most), (takes + waves * each - 1) / (waves * each));
 }
 
+// Results that also go to pinned memory: by the product's own launch, in pieces of 32 bytes, as long as the product is what takes the time.  Many results of
+// short rows are bound by the bus, where a copy behind the product is faster (us for the host, so and with the copy: 1024 columns, 32000 rows 28 and 30,
+// 65536 45 and 45, 262144 153 and 149; 256 columns 24 and 26, 34 and 34, 105 and 98; 1536 columns, 128000 rows 92 and 94).
+bool copied_in_product(uint32_t K, uint32_t N) { return K <= 2048 && (K > 1024 || N <= 65536); }
+
 constexpr uint32_t kMaxVectorK = 36864;   // 144 KB of staged f32 activations
 
 template <int STAGE>
@@ -1115,7 +1120,7 @@ int launch_vector(lh_context* ctx, const VectorStage& st, const uint16_t* W, con
         const uint32_t grid = one_row_grid(takes, K, w, seg.pairs ? 32 : 64, cus);
 #define LH_MVC(NLOADS, WAVES, COPY) hipLaunchKernelGGL((matvec_bf16_reg_kernel<STAGE, NLOADS, WAVES, COPY>), dim3(grid), dim3(64 * WAVES), 0, ctx->stream, st, W, bias, seg, N, K, copy)
 #define LH_MVR(NLOADS, WAVES) LH_MVC(NLOADS, WAVES, false)
-        if constexpr (STAGE == kNorm) if (copy && w == 8 && K <= 2048) {
+        if constexpr (STAGE == kNorm) if (copy && w == 8 && copied_in_product(K, N)) {
             if (K <= 512) LH_MVC(1, 8, true);
             else if (K <= 1024) LH_MVC(2, 8, true);
             else LH_MVC(4, 8, true);
@@ -1474,7 +1479,7 @@ int lh_linear_residual_norm_vector_copied_into(lh_batch* batch, lh_buffer* input
     st.x = input->ptr; st.x_f32 = 1; st.add = (const float*)branch->ptr; st.norm_weight = (const float*)branch_weight->ptr; st.eps = branch_eps;
     st.outer_weight = (const float*)norm_weight->ptr; st.outer_eps = eps;
     const uint64_t cus = (uint64_t)batch->ctx->cu_count;
-    if (k % 8 == 0 && k > 0 && k <= 2048 && n > 8 * cus && weight && ((uintptr_t)weight->ptr & 15) == 0 && lh_stage_aligned(st)) {
+    if (k % 8 == 0 && k > 0 && copied_in_product(k, n) && n > 8 * cus && weight && ((uintptr_t)weight->ptr & 15) == 0 && lh_stage_aligned(st)) {
         LH_TRY(check_common(batch, weight, bias, k, n, op));
         LhSegments seg;
         const uint32_t act = LH_ACT_NONE, layout = LH_ROWS;
