@@ -95,7 +95,7 @@ class ScratchBuffers:
         kv_elems = num_key_value_heads * head_dim
         self.normed = _alloc_f16(ctx, hidden_size)
         # q, k, v are consecutive pieces of one allocation: a layer whose three projections were stacked into one
-        # matrix writes them with a single matvec (at that layer's own sizes, see TransformerLayer._qkv_views)
+        # matrix writes them with a single matvec (at that layer's own sizes, see qkv_views)
         self.qkv = _alloc_f16(ctx, q_elems + 2 * kv_elems)
         self.q = self.qkv.view(0, q_elems * 2)
         self.k = self.qkv.view(q_elems * 2, kv_elems * 2)
@@ -115,6 +115,17 @@ class ScratchBuffers:
         self.fa_pmax = _alloc_f32(ctx, num_attention_heads * MAX_FLASH_SPLITS)
         self.fa_psum = _alloc_f32(ctx, num_attention_heads * MAX_FLASH_SPLITS)
         self.fa_pacc = _alloc_f32(ctx, num_attention_heads * MAX_FLASH_SPLITS * head_dim)
+        self._qkv_views = {}
+
+    def qkv_views(self, q_elems: int, kv_elems: int):
+        """(q, k, v, all three) views of ``qkv`` for a layer of these sizes, consecutive, and the same of ``raw_qkv``; made once for all layers of a
+        size (the first token of a pipeline waits for each of them)."""
+        views = self._qkv_views.get((q_elems, kv_elems))
+        if views is None:
+            nq, nkv = q_elems * 2, kv_elems * 2
+            views = self._qkv_views[q_elems, kv_elems] = tuple([b.view(0, nq), b.view(nq, nkv), b.view(nq + nkv, nkv), b.view(0, nq + 2 * nkv)]
+                                                               for b in (self.qkv, self.raw_qkv))
+        return views
 
 
 class BatchScratch:
@@ -204,17 +215,6 @@ class TransformerLayer:
             x.buf = stacked.view(off, n)
             off += n
         self._qkv = QuantWeight.quantized(stacked, q.ty, q.rows + k.rows + v.rows, q.cols)
-
-    def _qkv_views(self, scratch: "ScratchBuffers"):
-        """(q, k, v, all three) views of scratch.qkv at this layer's sizes, consecutive, and the same of scratch.raw_qkv (cached per scratch
-        object)."""
-        cached = getattr(self, "_qkv_view_cache", None)
-        if cached is None or cached[0] is not scratch:
-            p = self.params
-            nq, nkv = p.num_attention_heads * p.head_dim * 2, p.num_key_value_heads * p.head_dim * 2
-            cached = (scratch, *([b.view(0, nq), b.view(nq, nkv), b.view(nq + nkv, nkv), b.view(0, nq + 2 * nkv)] for b in (scratch.qkv, scratch.raw_qkv)))
-            self._qkv_view_cache = cached
-        return cached[1:]
 
     # ------------------------------------------------------------------ helpers
     def _pair_matvec(self, batch, kernels: Kernels, wa: QuantWeight, wb: QuantWeight, x: Buffer, out_a: Buffer,
@@ -314,7 +314,7 @@ class TransformerLayer:
         one_prepare = self._one_prepare()
         q_buf, k_buf, v_buf = s.q, s.k, s.v
         stacked = fused_in and own_kv and self._qkv is not None
-        prepared, raw = self._qkv_views(s)
+        prepared, raw = s.qkv_views(n_head * hd, n_kv * hd)
         if stacked:
             q_buf, k_buf, v_buf = prepared[:3]
         raw_q, raw_k, raw_v, qkv_out = raw if one_prepare else (q_buf, k_buf, v_buf, prepared[3])      # where the projections go

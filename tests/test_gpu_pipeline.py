@@ -73,3 +73,16 @@ def test_decode_steps_match_oracle(pkg, gpu, oracle, pld, fused, head_dims, defe
     assert pipe.position == 0 and not pipe.kv_caches[0].keys_q.as_array(np.uint8).any()
     with pytest.raises(pkg.InvalidArgument):
         pipe.forward_token(1, max_ctx)
+
+
+def test_a_first_token_makes_the_views_of_its_rows_once_for_each_size(pkg, gpu, monkeypatch):
+    """Handles cost host time ahead of the first launches: eight for each of the two sizes of layers and one each for the layers' own inputs, none later."""
+    ctx, K = gpu
+    cfg = _config(pkg, 64)
+    pipe = pkg.pipeline.DecodePipeline.from_host(ctx, K, cfg, pkg.synth.decode_model_tensors(cfg, pkg.synth.rng(5, 1), [512, 512, 512, 1024, 1024, 1024]), 256)
+    made, view = [], pkg.Buffer.view
+    monkeypatch.setattr(pkg.Buffer, "view", lambda self, *a: made.append(a) or view(self, *a))
+    pipe.forward_token(3, 0)
+    first = len(made)
+    pipe.forward_token(4, 1)
+    assert first <= 2 * 8 + cfg.num_hidden_layers and len(made) == first
