@@ -107,6 +107,29 @@ pub fn token_attention_tq_into(batch: &mut CommandBatch, q_raw: Option<&Buffer>,
     Ok(rotated != 0)
 }
 
+/// `lh_matmul_nt_qkv_attention_lanes_into` (include/local_hip.h) as `Kernels::matmul_nt_qkv_attention_lanes_into` has it for layers with
+/// caches of their own, and, without key and value projections and their outputs, for one that reads another layer's cache.
+#[allow(clippy::too_many_arguments)]
+pub fn matmul_nt_qkv_attention_lanes_into(batch: &mut CommandBatch, fmt: ffi::lh_quant, input: &Buffer, w_q: &Buffer,
+                                          w_k: Option<&Buffer>, w_v: Option<&Buffer>, k_dim: u32, q: &Buffer,
+                                          k: Option<&Buffer>, v: Option<&Buffer>, q_norm: Option<&Buffer>,
+                                          k_norm: Option<&Buffer>, levels: &Buffer, signs: &Buffer, rq: &Buffer,
+                                          k_codes: &Buffer, k_norms: &Buffer, v_codes: &Buffer, v_norms: &Buffer,
+                                          positions: &Buffer, out: &Buffer, out_f16: &Buffer, head_dim: u32, n_q_heads: u32,
+                                          n_kv_heads: u32, lanes: u32, eps: f32, theta: f32, partial_rotary_factor: f32,
+                                          window: u32, bits: u32, ring_capacity: u32, lane_capacity: u32) -> Result<()> {
+    // SAFETY: every pointer is null or comes from a live handle of this crate; the library validates sizes and shapes.
+    error::check(unsafe {
+        ffi::lh_matmul_nt_qkv_attention_lanes_into(batch.as_ptr(), fmt, input.as_ptr(), w_q.as_ptr(), opt(w_k), opt(w_v),
+                                                   k_dim, q.as_ptr(), opt(k), opt(v), opt(q_norm), opt(k_norm),
+                                                   levels.as_ptr(), signs.as_ptr(), rq.as_ptr(), k_codes.as_ptr(),
+                                                   k_norms.as_ptr(), v_codes.as_ptr(), v_norms.as_ptr(), positions.as_ptr(),
+                                                   out.as_ptr(), out_f16.as_ptr(), head_dim, n_q_heads, n_kv_heads, lanes,
+                                                   eps, theta, partial_rotary_factor, window, bits, ring_capacity,
+                                                   lane_capacity)
+    })
+}
+
 /// `lh_matvec_quant_norm_chain_gelu_into` (include/local_hip.h): gate and up projection (or, with `factor` instead of `up`, one
 /// projection) behind a chain of norms, and the GeGLU product of their results where the launch can form it (layer.rs:476-482,
 /// 495-500).  `Ok(true)`: `out` holds the product.  `Ok(false)`: `out` and `up_out` hold the projections' results.

@@ -171,6 +171,27 @@ def test_operations_without_a_generated_method_are_wrapped_by_hand():
         assert f"ffi::{name}(" in lib, name
 
 
+def test_steps_that_a_shared_cache_takes_without_keys_and_values():
+    """The two attention steps whose header lets a layer that reads another's cache leave keys and values out: lib.rs has them with the
+    header's parameters in its order, the ones that may be null as options."""
+    lib = open(os.path.join(ROOT, "local-hip", "src", "lib.rs")).read()
+    header = {f[0]: f for f in c_functions()}
+    for name, null in (("lh_token_attention_tq_into", {"q_raw", "k_raw", "v_raw", "k", "v", "q_norm", "k_norm"}),
+                       ("lh_matmul_nt_qkv_attention_lanes_into", {"w_k", "w_v", "k", "v", "q_norm", "k_norm"})):
+        sig, = re.findall(rf"pub fn {name[3:]}\(([^)]*)\)", lib)
+        params = [tuple(s.strip() for s in prm.split(":", 1)) for prm in sig.split(",")]
+        call, = re.findall(rf"ffi::{name}\(((?:[^()]|\([^()]*\))*)\)", lib)
+        args = [" ".join(a.split()) for a in call.split(",")]
+        cparams = header[name][2]
+        assert len(args) == len(cparams)
+        for (ctype, cname), (pname, ptype), arg in zip(cparams, params, args):
+            if "lh_buffer" in ctype:
+                assert (pname, ptype) == (cname, "Option<&Buffer>" if cname in null else "&Buffer"), (name, cname)
+                assert arg == (f"opt({cname})" if cname in null else f"{cname}.as_ptr()"), (name, cname)
+            elif ctype not in ("lh_batch*", "int*"):
+                assert (pname, arg) == (cname, cname), (name, cname)
+
+
 def test_safe_layer_argument_order_of_the_reference():
     """Three methods whose parameter lists were read off the reference (local-metal/src/kernels.rs:4819-4834, 5176-5193,
     5434-5452; kept here as data): the generated methods take exactly these parameters in exactly this order."""
