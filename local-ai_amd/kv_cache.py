@@ -113,41 +113,12 @@ class QuantizedKvCache:
                                                 self.levels, self.signs, vacc, attn_out, hd, seq_len, current_pos,
                                                 n_q_heads, self.n_kv_heads, window, self.bits, self.ring_capacity())
 
-    def prepare_token_into(self, batch, kernels: Kernels, q: Buffer, k, v, q_norm, k_norm, rq: Buffer, position: int,
-                           n_q_heads: int, eps: float, theta: float, partial_rotary_factor: float) -> None:
-        """One dispatch for a decoded token's head norms, RoPE, V norm, ``write_kv_gpu_into`` (quant_cache.rs:391-444)
-        and the query rotation that opens ``fused_attention_into`` (quant_cache.rs:560-570); ``k = v = None`` leaves
-        the cache alone (a KV-shared layer)."""
-        if k is not None and position + 1 > self.max_positions:
-            raise InvalidArgument(f"KV write [{position}..{position + 1}) exceeds capacity {self.max_positions}")
-        kernels.decode_qkv_prepare_into(batch, q, k, v, q_norm, k_norm, self.levels, self.signs, rq,
-                                        self.keys_q, self.key_norms, self.values_q, self.value_norms, self.head_dim,
-                                        n_q_heads, self.n_kv_heads, eps, position, theta, partial_rotary_factor, self.bits,
-                                        self.ring_capacity())
-
-    def attention_from_rotated_into(self, batch, kernels: Kernels, rq: Buffer, vacc: Buffer, attn_out: Buffer,
-                                    seq_len: int, current_pos: int, n_q_heads: int, window: int) -> None:
-        """quant_cache.rs:571-598: the attend and rotate-back steps of ``fused_attention_into`` for a query that
-        ``prepare_token_into`` has already rotated."""
-        hd = self.head_dim
-        kernels.flash_attention_tq_rotated_into(batch, rq, self.keys_q, self.key_norms, self.values_q, self.value_norms,
-                                                self.levels, self.signs, vacc, attn_out, hd, seq_len, current_pos,
-                                                n_q_heads, self.n_kv_heads, window, self.bits, self.ring_capacity())
-
-    def attention_from_rotated_lazy_into(self, batch, kernels: Kernels, rq: Buffer, vacc: Buffer, attn_out: Buffer,
-                                         seq_len: int, current_pos: int, n_q_heads: int, window: int) -> bool:
-        """quant_cache.rs:571-598 for a caller whose output projection can rotate its input itself: True when
-        ``attn_out`` holds the rotated f16 heads (the rotation rode in the merge launch), False when the f32 heads in
-        ``vacc`` are still in code space (quant_cache.rs:590-598 is left to the caller)."""
-        return kernels.flash_attention_tq_rotated_lazy_into(batch, rq, self.keys_q, self.key_norms, self.values_q,
-                                                            self.value_norms, self.levels, self.signs, vacc, attn_out,
-                                                            self.head_dim, seq_len, current_pos, n_q_heads,
-                                                            self.n_kv_heads, window, self.bits, self.ring_capacity())
-
     def attend_token_into(self, batch, kernels: Kernels, raw, q: Buffer, k, v, q_norm, k_norm, rq: Buffer, vacc: Buffer, attn_out: Buffer, position: int,
                           n_q_heads: int, window: int, eps: float, theta: float, partial_rotary_factor: float, lazy: bool) -> bool:
-        """``prepare_token_into`` on the rows ``raw`` (q, k, v), then ``attention_from_rotated_into`` or, ``lazy``, its lazy form, as one
-        step; True: ``attn_out`` holds the rotated f16 heads."""
+        """A decoded token's head norms, RoPE, V norm, ``write_kv_gpu_into`` (quant_cache.rs:391-444) of the rows ``raw`` (q, k, v) and
+        ``fused_attention_into`` (quant_cache.rs:548-598) as one step; ``k = v = None`` leaves the cache alone (a KV-shared layer).  True: ``attn_out``
+        holds the rotated f16 heads.  ``lazy``, for a caller whose output projection can rotate its input itself: False where that would be a launch of
+        its own; the f32 heads in ``vacc`` are then still in code space (quant_cache.rs:590-598 is left to the caller)."""
         if k is not None and position + 1 > self.max_positions:
             raise InvalidArgument(f"KV write [{position}..{position + 1}) exceeds capacity {self.max_positions}")
         return kernels.token_attention_tq_into(batch, raw, q, k, v, q_norm, k_norm, self.levels, self.signs, rq, self.keys_q, self.key_norms, self.values_q,
@@ -156,7 +127,8 @@ class QuantizedKvCache:
 
     def prepare_rows_into(self, batch, kernels: Kernels, q: Buffer, k, v, q_norm, k_norm, rq: Buffer, start_pos: int,
                           n_rows: int, n_q_heads: int, eps: float, theta: float, partial_rotary_factor: float) -> None:
-        """``prepare_token_into`` for the ``n_rows`` consecutive tokens of a prefill chunk."""
+        """One dispatch for head norms, RoPE, V norm, ``write_kv_gpu_into`` and the query rotation that opens ``fused_attention_into``
+        (quant_cache.rs:560-570) of the ``n_rows`` consecutive tokens of a prefill chunk; ``k = v = None`` leaves the cache alone."""
         if k is not None and start_pos + n_rows > self.max_positions:
             raise InvalidArgument(f"KV write [{start_pos}..{start_pos + n_rows}) exceeds capacity {self.max_positions}")
         kernels.decode_qkv_prepare_rows_into(batch, q, k, v, q_norm, k_norm, self.levels, self.signs, rq, self.keys_q,
@@ -267,24 +239,6 @@ class QuantizedUnifiedKvPool:
                                              n_q_heads, self.n_kv_heads, lanes, eps, 0, theta, partial_rotary_factor,
                                              self.bits, self.lane_ring_capacity, self.lane_stride())
 
-    def project_and_prepare_lanes_into(self, batch, kernels: Kernels, weight_type: int, x: Buffer, w_q: Buffer, w_k: Buffer,
-                                       w_v: Buffer, k_dim: int, q: Buffer, k: Buffer, v: Buffer, q_norm, k_norm, rq: Buffer,
-                                       positions: Buffer, active_lanes: int, n_q_heads: int, eps: float, theta: float,
-                                       partial_rotary_factor: float) -> None:
-        """The Q / K / V projections of every lane and ``prepare_lanes_into`` on their outputs as one encoded step."""
-        lanes = min(active_lanes, self.n_lanes)
-        kernels.matmul_nt_qkv_prepare_rows_into(batch, weight_type, x, w_q, w_k, w_v, k_dim, q, k, v, q_norm, k_norm,
-                                                self.levels, self.signs, rq, self.keys_q, self.key_norms, self.values_q,
-                                                self.value_norms, positions, self.head_dim, n_q_heads, self.n_kv_heads,
-                                                lanes, eps, 0, theta, partial_rotary_factor, self.bits,
-                                                self.lane_ring_capacity, self.lane_stride())
-
-    def project_queries_lanes_into(self, batch, kernels: Kernels, w_q, x: Buffer, q: Buffer, q_norm, rq: Buffer, positions: Buffer,
-                                   active_lanes: int, n_q_heads: int, eps: float, theta: float, partial_rotary_factor: float) -> None:
-        """The Q projection of every lane and ``prepare_lanes_into`` of the queries alone (a KV-shared layer) as one encoded step."""
-        kernels.matmul_nt_q_prepare_rows_into(batch, w_q.ty, x, w_q.buf, w_q.cols, q, q_norm, self.signs, rq, positions, self.head_dim, n_q_heads,
-                                              min(active_lanes, self.n_lanes), eps, 0, theta, partial_rotary_factor, self.lane_stride())
-
     def attention_from_rotated_into(self, batch, kernels: Kernels, rq: Buffer, vacc: Buffer, attn_out: Buffer,
                                     positions: Buffer, n_q_heads: int, window: int, active_lanes: int) -> None:
         """quant_unified_pool.rs:225-256: the attend and rotate-back steps of ``attention_into``."""
@@ -298,7 +252,7 @@ class QuantizedUnifiedKvPool:
     def project_and_attend_lanes_into(self, batch, kernels: Kernels, w_q, w_k, w_v, x: Buffer, q: Buffer, k, v, q_norm, k_norm, rq: Buffer, vacc: Buffer,
                                       attn_out: Buffer, positions: Buffer, active_lanes: int, n_q_heads: int, window: int, eps: float, theta: float,
                                       partial_rotary_factor: float) -> None:
-        """``project_and_prepare_lanes_into`` (without key and value projections: ``project_queries_lanes_into``) and
+        """The Q / K / V projections of every lane (a KV-shared layer: Q alone), ``prepare_lanes_into`` on their outputs and
         ``attention_from_rotated_into`` as one encoded step."""
         kernels.matmul_nt_qkv_attention_lanes_into(batch, w_q.ty, x, w_q.buf, w_k and w_k.buf, w_v and w_v.buf, w_q.cols, q, k, v, q_norm, k_norm, self.levels,
                                                    self.signs, rq, self.keys_q, self.key_norms, self.values_q, self.value_norms, positions, vacc, attn_out,
