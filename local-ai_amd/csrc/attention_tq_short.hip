@@ -40,6 +40,7 @@ struct ShortShared {
     uint8_t rqop[12][64][16];            // score operands per (plane, field) and lane
     float maxabs[kHeads], sum[kHeads];
     float fin_r[kMaxWaves][kHeads], fin_l[kMaxWaves][kHeads];
+    float none[kDim];                    // zeros
 };
 // S: workgroups of a query, 256 / S output dims each.
 template <int S>
@@ -87,6 +88,9 @@ __device__ __forceinline__ void short_body(const AttnPointers& a, const AttnPara
                                            float alpha, float beta, float gam, float delta, uint32_t qi, uint32_t kvh, uint32_t group, uint32_t nwaves, uint32_t parts, const Rotation& rotation) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), pcol = lane & 15, g = lane >> 4;
     constexpr int E = 4 / S;              // chunks of 16 code bytes, 64 dims
+    if (wave == nwaves - 1)
+#pragma unroll
+        for (int e = 0; e < E; e++) sh.none[64 * e + lane] = 0.0f;
     const float cmax = fmaxf(fmaxf(fabsf(beta), fabsf(0.5f * gam)), NPL == 3 ? fabsf(delta) : 0.0f), inv_cmax = cmax > 0.0f ? 1.0f / cmax : 0.0f;
 
     // ---- score operands: row r of the product is head (r / 4) + 4 ((r / 2) % 2), limb r % 2; k slot (word m, byte e) of row group g is code byte
@@ -290,12 +294,14 @@ __device__ __forceinline__ void short_body(const AttnPointers& a, const AttnPara
     const float f = r == -INFINITY ? 0.0f : exp2f(r - top), l = lh_group_sum(lane < parts ? f * sh.fin_l[lane][wave] : 0.0f, 16);
     const ShortWave<S>* const all = &mine - wave;
     float o[E] = {};
-    for (uint32_t w0 = 0; w0 < parts; w0 += 4) {                // (one at a time each is a trip to LDS; past the last: its values, with weight 0)
+    for (uint32_t w0 = 0; w0 < parts; w0 += 4) {                // (one at a time each is a trip to LDS; past the last: zeros)
         float x[4][E];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; u++)
+        for (uint32_t u = 0; u < 4; u++) {
+            const float* const sums = w0 + u < parts ? all[w0 + u].park[wave] : sh.none;
 #pragma unroll
-            for (int e = 0; e < E; e++) x[u][e] = all[std::min(w0 + u, parts - 1)].park[wave][64 * e + lane];
+            for (int e = 0; e < E; e++) x[u][e] = sums[64 * e + lane];
+        }
 #pragma unroll
         for (uint32_t u = 0; u < 4; u++) {
             const float fw = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(f), (int)(w0 + u)));

@@ -870,3 +870,25 @@ def test_lanes_in_one_step_refuses_before_anything_runs(pkg, gpu, oracle, lanes,
     assert batch.dispatch_count() > 0
     batch.commit_and_wait()
     assert not (q.as_array(np.float16) == 7).all()
+
+
+@pytest.mark.parametrize("position,window", [(700, 640), (575, 570), (511, 512), (130, 0)])
+def test_an_infinite_value_stays_an_infinity(pkg, gpu, oracle, position, window):
+    """One position's value norm beyond f16 in the last group of a short span, levels that do not cancel: infinite heads, and no 0 x infinity of a
+    part that is not there."""
+    ctx, K = gpu
+    hd, n_q = 256, 8
+    g = pkg.synth.rng(83, position)
+    levels = oracle.tq_levels(hd, 2)
+    levels = (levels + np.float32(1.5 * np.abs(levels).max())).astype(np.float32)             # all of one sign
+    slots = position + 1
+    norms = (14 * (0.8 + 0.4 * g.random(slots))).astype(np.float16)
+    values = norms.copy()
+    values[-2] = np.inf
+    rq, out = pkg.Buffer.from_slice(ctx, (g.standard_normal(n_q * hd) * 0.01).astype(np.float32)), pkg.Buffer.empty(ctx, n_q * hd * 4)
+    codes = [pkg.Buffer.from_slice(ctx, g.integers(0, 256, slots * hd // 4, dtype=np.uint8)) for _ in range(2)]
+    batch = pkg.CommandBatch(ctx)
+    K.flash_attention_tq_into(batch, rq, codes[0], pkg.Buffer.from_slice(ctx, norms), codes[1], pkg.Buffer.from_slice(ctx, values), pkg.Buffer.from_slice(ctx, levels), out, hd,
+                              slots, position, n_q, 1, window, 2, 0)
+    batch.commit_and_wait()
+    assert np.isposinf(out.as_array(np.float32)).all()
