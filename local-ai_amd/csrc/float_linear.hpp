@@ -36,11 +36,16 @@ struct VectorStage {
     const float* add;          // norm: may be null; residual: what is normed and added
     float* store;              // norm, residual: receives the sum (workgroup 0), may be null
     const float* norm_weight;  // gated: may be null
-    const void* gate;          // gated
-    uint32_t gate_f32, gate_act, gate_first, group;   // gated: the gate multiplies before the norm; elements per normed part
+    union {
+        const void* gate;            // gated
+        const float* outer_weight;   // residual and norm: of the norm
+    };
+    uint32_t gate_f32, gate_act, gate_first;          // gated: the gate multiplies before the norm
+    union {
+        uint32_t group;              // gated: elements per normed part
+        float outer_eps;             // residual and norm
+    };
     float eps;
-    const float* outer_weight; // residual and norm: of the norm
-    float outer_eps;
 };
 
 __device__ __forceinline__ void lh_ld8(const float* p, float (&v)[8]) {
@@ -184,7 +189,7 @@ struct LhSharedVector {
 };
 
 static inline bool lh_stage_aligned(const VectorStage& st) {
-    return (((uintptr_t)st.x | (uintptr_t)st.add | (uintptr_t)st.store | (uintptr_t)st.norm_weight | (uintptr_t)st.gate | (uintptr_t)st.outer_weight) & 15) == 0;
+    return (((uintptr_t)st.x | (uintptr_t)st.add | (uintptr_t)st.store | (uintptr_t)st.norm_weight | (uintptr_t)st.gate) & 15) == 0;
 }
 
 // Weights are read once per launch: streaming loads.
