@@ -723,7 +723,7 @@ int launch_recurrent(lh_context* ctx, const RecurrentArgs& a, const char* op) {
         // What is requested ahead past the last row is traffic for nothing, so that few rows have fewer ahead (selective 128 x 128, 128 heads, f32: 8 rows
         // 27.4 us with sixteen ahead, 20.5 with twelve; 16 rows 45.6, with eight 32.1; 64 rows 99.6, 85.6; bf16 20.0, 16.8; 30.3, 28.3; 73.1, 75.7).
         if (a.dq <= 128) { if (few) LH_REC(2, 4); else if (a.rows < 12) LH_REC(2, 12); else if (a.rows < 24) LH_REC(2, 8); else LH_REC(2, 16); }
-        else if (a.dq <= 256) { if (few) LH_REC(4, 4); else LH_REC(4, 8); }
+        else if (a.dq <= 256) { if (few) LH_REC(4, 4); else if (a.rows < 12 && sizeof(T) == 2) LH_REC(4, 12); else LH_REC(4, 8); }
         else LH_REC(8, 4);
 #undef LH_REC
         return lh_check_launch(op);
