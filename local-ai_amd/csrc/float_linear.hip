@@ -719,37 +719,46 @@ __global__ __launch_bounds__(512) void linear_phased_kernel(const LhLinear a) {
 // its middle terms and its leading terms, one after the other.  No term is zero, or an infinite weight would give NaN where it gives an
 // infinity times the value itself: a value of fewer bits passes its last one on to the terms below (values from 2^-110 up; smaller ones
 // lose bits below bf16's range).
-// (The products of a pass over 333 rows at width 1024: 184 us on average on the FMA units, 30 and 4.5 for the terms.  A lane makes one trip to
-// memory: with four, one behind the other, the terms of 333 rows of 1024 took 6.0 us, of 4096 6.8 and now 5.5.)
+// (The products of a pass over 333 rows at width 1024: 184 us on average on the FMA units, 30 and 4.5 for the terms.)
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, uint16_t* __restrict__ out, uint32_t rows, uint32_t K, uint32_t lda, uint32_t stride) {
-    const uint32_t k = (blockIdx.x * 64 + (threadIdx.x & 63)) * 4, row = blockIdx.y * 4 + threadIdx.x / 64;
-    if (row >= rows || k >= stride) return;
-    const float4 v = k < K ? *reinterpret_cast<const float4*>(x + (size_t)row * lda + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float f[4] = {v.x, v.y, v.z, v.w};
-    uint32_t t[3][4];
+    const uint32_t row = blockIdx.y * 4 + threadIdx.x / 64;
+    if (row >= rows) return;
+    for (uint32_t k = (blockIdx.x * 64 + (threadIdx.x & 63)) * 4; k < stride; k += gridDim.x * 256) {
+        const float4 v = k < K ? *reinterpret_cast<const float4*>(x + (size_t)row * lda + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float f[4] = {v.x, v.y, v.z, v.w};
+        uint32_t t[3][4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t u = __builtin_bit_cast(uint32_t, f[j]);
-        if ((u & 0x7F800000u) == 0x7F800000u) {           // infinite, or no number (which stays none when it is cut off)
-            t[0][j] = t[1][j] = t[2][j] = (u >> 16) | ((u & 0x007FFFFFu) ? 0x40u : 0u);
-            continue;
+        for (int j = 0; j < 4; j++) {
+            const uint32_t u = __builtin_bit_cast(uint32_t, f[j]);
+            if ((u & 0x7F800000u) == 0x7F800000u) {           // infinite, or no number (which stays none when it is cut off)
+                t[0][j] = t[1][j] = t[2][j] = (u >> 16) | ((u & 0x007FFFFFu) ? 0x40u : 0u);
+                continue;
+            }
+            const float hi = __builtin_bit_cast(float, u & 0xFFFF0000u), r = f[j] - hi;
+            // (the last bit of a bf16 value: seven places below its exponent, none where that is below the normal ones)
+            auto bit_of = [](float v, uint32_t places) {
+                const uint32_t e = __builtin_bit_cast(uint32_t, v) & 0x7F800000u, s = __builtin_bit_cast(uint32_t, v) & 0x80000000u;
+                return e > (places << 23) ? __builtin_bit_cast(float, (e - (places << 23)) | s) : 0.0f;
+            };
+            float top = hi, mid = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xFFFF0000u), low = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r - mid) & 0xFFFF0000u);
+            if (r == 0.0f) { mid = low = bit_of(hi, 8); top = hi - (mid + low); }
+            else if (r == mid) { low = bit_of(mid, 7); mid -= low; }
+            t[0][j] = __builtin_bit_cast(uint32_t, low) >> 16;
+            t[1][j] = __builtin_bit_cast(uint32_t, mid) >> 16;
+            t[2][j] = __builtin_bit_cast(uint32_t, top) >> 16;
         }
-        const float hi = __builtin_bit_cast(float, u & 0xFFFF0000u), r = f[j] - hi;
-        // (the last bit of a bf16 value: seven places below its exponent, none where that is below the normal ones)
-        auto bit_of = [](float v, uint32_t places) {
-            const uint32_t e = __builtin_bit_cast(uint32_t, v) & 0x7F800000u, s = __builtin_bit_cast(uint32_t, v) & 0x80000000u;
-            return e > (places << 23) ? __builtin_bit_cast(float, (e - (places << 23)) | s) : 0.0f;
-        };
-        float top = hi, mid = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xFFFF0000u), low = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r - mid) & 0xFFFF0000u);
-        if (r == 0.0f) { mid = low = bit_of(hi, 8); top = hi - (mid + low); }
-        else if (r == mid) { low = bit_of(mid, 7); mid -= low; }
-        t[0][j] = __builtin_bit_cast(uint32_t, low) >> 16;
-        t[1][j] = __builtin_bit_cast(uint32_t, mid) >> 16;
-        t[2][j] = __builtin_bit_cast(uint32_t, top) >> 16;
-    }
-    uint16_t* o = out + (size_t)row * 3 * stride + k;
+        uint16_t* o = out + (size_t)row * 3 * stride + k;
 #pragma unroll
-    for (int z = 0; z < 3; z++) *reinterpret_cast<uint2*>(o + (size_t)z * stride) = make_uint2(t[z][0] | t[z][1] << 16, t[z][2] | t[z][3] << 16);
+        for (int z = 0; z < 3; z++) *reinterpret_cast<uint2*>(o + (size_t)z * stride) = make_uint2(t[z][0] | t[z][1] << 16, t[z][2] | t[z][3] << 16);
+    }
+}
+
+// Workgroups for 256 columns each where that makes up to six a CU, for 1024 beyond.  Few are bound by a lane's trips to memory, one behind the other; many by how
+// they begin and end.  (With a product of 64 columns: 333 x 1024 12.7 us with four trips, 11.0 with one, 333 x 4096 27.8 and 27.2; 1000 x 2048 19.8 and 21.2, 2048 x 2048 21.9 and
+// 25.7, 4096 x 1024 18.5 and 21.5.)
+uint32_t split_grid(uint32_t rows, uint32_t stride, uint64_t cus) {
+    const uint32_t groups = (stride + 255) / 256;
+    return (uint64_t)groups * ((rows + 3) / 4) <= 6 * cus ? groups : (stride + 1023) / 1024;
 }
 
 // ---- f32 FMA -----------------------------------------------------------------------------------------------------------
@@ -1312,7 +1321,7 @@ int lh_launch_linear(lh_context* ctx, const LhLinear& given, const char* op) {
     if (a.a_f32 && a.K % 8 == 0 && a.lda % 4 == 0 && (((uintptr_t)a.A | (uintptr_t)a.W) & 15) == 0 && (uint64_t)a_rows * stride * 6 <= ctx->workspace_bytes &&
         a_rows <= 4 * 65535u) {
         if (a_rows == 0) return LH_OK;
-        hipLaunchKernelGGL(split_rows_kernel, dim3((stride + 255) / 256, (a_rows + 3) / 4), dim3(256), 0, ctx->stream, static_cast<const float*>(a.A),
+        hipLaunchKernelGGL(split_rows_kernel, dim3(split_grid(a_rows, stride, (uint64_t)ctx->cu_count), (a_rows + 3) / 4), dim3(256), 0, ctx->stream, static_cast<const float*>(a.A),
                            static_cast<uint16_t*>(ctx->workspace), a_rows, a.K, a.lda, stride);
         const int r = lh_check_launch(op);
         if (r != LH_OK) return r;

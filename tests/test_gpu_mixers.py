@@ -178,7 +178,7 @@ def test_activations_of_bf16_results(ai, gpu, act, m):
         assert np.array_equal(np.isnan(special), np.isnan(same)) and np.allclose(special, same, 2.0 ** -7, 1e-36, equal_nan=True), (special, same)
 
 
-@pytest.mark.parametrize("m,k,n", [(40, 72, 50), (333, 1024, 256), (2048, 64, 2048), (3, 4096, 16)])
+@pytest.mark.parametrize("m,k,n", [(40, 72, 50), (333, 1024, 256), (2048, 64, 2048), (3, 4096, 16), (1536, 1024, 32), (1537, 1024, 32), (1001, 2120, 40)])
 def test_f32_rows_as_terms(ai, gpu, m, k, n):
     """32-bit activations on the matrix cores: all 24 bits of every value, whatever its size, and what is infinite or no number comes
     out as f32 products and sums have it."""
