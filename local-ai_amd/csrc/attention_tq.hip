@@ -412,8 +412,8 @@ struct Preparation {
     uint32_t splits, part_cols;
 };
 
-bool apart(const lh_buffer* raw, const lh_buffer* out, size_t bytes) {
-    return raw && out && ((uintptr_t)raw->ptr + bytes <= (uintptr_t)out->ptr || (uintptr_t)out->ptr + bytes <= (uintptr_t)raw->ptr);
+bool apart(const lh_buffer* raw, size_t raw_bytes, const lh_buffer* out, size_t out_bytes) {
+    return raw && out && ((uintptr_t)raw->ptr + raw_bytes <= (uintptr_t)out->ptr || (uintptr_t)out->ptr + out_bytes <= (uintptr_t)raw->ptr);
 }
 
 // The preparation as attention_tq_token_kernel takes it; false: it has to run by itself.
@@ -431,7 +431,7 @@ bool token_preparation(const lh_context* ctx, const AttnParams& p, const AttnPoi
     if (!prep.partial) {
         const std::pair<const lh_buffer*, size_t> in[3] = {{a.q_raw, q_bytes}, {a.k_raw, kv_bytes}, {a.v_raw, kv_bytes}}, out[3] = {{a.q, q_bytes}, {a.k, kv_bytes}, {a.v, kv_bytes}};
         for (int i = 0; i < (kv ? 3 : 1); i++)
-            for (int o = 0; o < (kv ? 3 : 1); o++) if (!apart(in[i].first, out[o].first, std::max(in[i].second, out[o].second))) return false;
+            for (int o = 0; o < (kv ? 3 : 1); o++) if (!apart(in[i].first, in[i].second, out[o].first, out[o].second)) return false;
     }
     return max_span != 0 && mfma_supported(p, ptrs) && token_supported(ctx, p, t, max_span);
 }

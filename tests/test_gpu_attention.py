@@ -775,6 +775,38 @@ def test_token_in_one_step_equals_preparation_and_attention(pkg, gpu, oracle, n_
             assert np.abs(b["o16"].as_array(np.float16).astype(np.float32) - a["o16"].as_array(np.float16).astype(np.float32)).max() <= 1e-3 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("order", ["q k v Q K V", "Q K V q k v", "K q Q v k V", "v Q q K k V"])
+@pytest.mark.parametrize("own", [True, False])
+def test_token_in_one_step_of_rows_side_by_side(pkg, gpu, oracle, order, own):
+    """Raw rows (capitals) and prepared ones that touch in one allocation without sharing a byte: one launch, and what it leaves of rows far apart."""
+    ctx, K = gpu
+    hd, n_q, n_kv, position, window = 256, 16, 2, 600, 512
+    g = pkg.synth.rng(97, position)
+    lv, sg = pkg.Buffer.from_slice(ctx, oracle.tq_levels(hd, 2)), pkg.Buffer.from_slice(ctx, oracle.rotation_signs(hd))
+    rows = {n: (0.25 * g.standard_normal(c * hd, dtype=np.float32)).astype(np.float16) for n, c in (("q", n_q), ("k", n_kv), ("v", n_kv))}
+    codes, norms = ([g.integers(0, 256, (position + 1) * n_kv * hd // 4, dtype=np.uint8) for _ in range(2)], [(14 * (0.8 + 0.4 * g.random((position + 1) * n_kv))).astype(np.float16) for _ in range(2)])
+    sides = []
+    for together in (False, True):
+        whole, at, b = pkg.Buffer.from_slice(ctx, np.zeros(2 * (n_q + 2 * n_kv) * hd, np.float16)), 0, {}
+        for n in order.split():
+            size = rows[n.lower()].nbytes
+            b[n] = whole.view(at, size) if together else pkg.Buffer.empty(ctx, 4 * size)
+            at += size
+        for n in "QKV":
+            batch = pkg.CommandBatch(ctx)
+            batch.write(b[n], rows[n.lower()])
+            batch.commit_and_wait()
+        kc, vc, kn, vn = (pkg.Buffer.from_slice(ctx, x) for x in codes + norms)
+        rq, out, o16 = (pkg.Buffer.empty(ctx, n_q * hd * s) for s in (4, 4, 2))
+        batch = pkg.CommandBatch(ctx)
+        K.token_attention_tq_into(batch, [b["Q"], b["K"], b["V"]], b["q"], b["k"] if own else None, b["v"] if own else None, None, None, lv, sg, rq, kc, kn, vc, vn, out, o16, hd,
+                                  n_q, n_kv, 1e-6, position, 1e4, 1.0, window, 2, 0, True)
+        assert batch.dispatch_count() == 1
+        batch.commit_and_wait()
+        sides.append([b[n].as_array(np.float16)[:rows[n.lower()].size].copy() for n in ("qkvQKV" if own else "qQKV")] + [x.as_array(np.uint8).copy() for x in (kc, vc, kn, vn, out)])
+    assert all(np.array_equal(x, y) for x, y in zip(*sides))
+
+
 @pytest.mark.parametrize("fmt,lanes,n_q,n_kv,window,ring,cap", [
     ("q4_0", 64, 8, 1, 512, 1024, 1024), ("q4_0", 3, 8, 1, 512, 1024, 1024), ("q4_0", 12, 4, 1, 100, 128, 600), ("tq2_0", 33, 8, 2, 512, 512, 512), ("tq2_0", 1, 8, 1, 64, 0, 300),
     ("q4_0", 20, 4, 1, 0, 0, 560), ("q4_0", 20, 4, 1, 0, 0, 700), ("q4_0", 9, 4, 1, 0, 64, 64), ("q4_0", 128, 8, 1, 16, 64, 64), ("q4_0", 130, 8, 1, 16, 64, 64)])
