@@ -178,7 +178,7 @@ def test_activations_of_bf16_results(ai, gpu, act, m):
         assert np.array_equal(np.isnan(special), np.isnan(same)) and np.allclose(special, same, 2.0 ** -7, 1e-36, equal_nan=True), (special, same)
 
 
-@pytest.mark.parametrize("m,k,n", [(40, 72, 50), (333, 1024, 256), (2048, 64, 2048), (3, 4096, 16), (1536, 1024, 32), (1537, 1024, 32), (1001, 2120, 40)])
+@pytest.mark.parametrize("m,k,n", [(40, 72, 50), (333, 1024, 256), (2048, 64, 2048), (3, 4096, 16)])
 def test_f32_rows_as_terms(ai, gpu, m, k, n):
     """32-bit activations on the matrix cores: all 24 bits of every value, whatever its size, and what is infinite or no number comes
     out as f32 products and sums have it."""
@@ -204,6 +204,12 @@ def test_f32_rows_as_terms(ai, gpu, m, k, n):
     fine = np.isfinite(want)
     # a rounding for each 32 exact products of each of the three terms, and the product's own 32
     assert (np.abs(got[fine] - want[fine]) <= ((3 * k / 32 + 32) * 2.0 ** -24 * size)[fine]).all()
+
+
+@pytest.mark.parametrize("m,k,n", [(1536, 1024, 32), (1537, 1024, 32), (1001, 2120, 40)])
+def test_f32_rows_as_terms_around_the_line(ai, gpu, m, k, n):
+    """Around the workgroups beyond which a lane makes four trips, and with rows that end within one."""
+    test_f32_rows_as_terms(ai, gpu, m, k, n)
 
 
 @pytest.mark.parametrize("bits", [1, 2, 7, 8, 9, 15, 16, 17, 24])
@@ -617,9 +623,35 @@ def test_recurrence_over_rows(ai, gpu, dtype, dim, rows):
     assert not got[:, :, dim:].any()
 
 
+@pytest.mark.parametrize("heads,vdim,dim", [(16, 128, 128), (41, 50, 128), (41, 50, 100), (33, 64, 65), (17, 128, 160)])
+@pytest.mark.parametrize("rows", [1, 7, 8, 33])
+def test_recurrence_of_many_columns(ai, gpu, heads, vdim, dim, rows):
+    """Around the columns beyond which many rows share a wave's lanes, with fixed decays and with a head's steps computed from the token."""
+    ctx, K = gpu
+    g = np.random.default_rng(heads + dim + rows)
+    dq = K.linear_attention_padded_dim(dim)
+    q, k, v = (M.rounded(g.standard_normal(s) / np.sqrt(dim)) for s in ((rows, heads, dim), (rows, heads, dim), (rows, heads, vdim)))
+    decay, S = np.linspace(0.4, 1.0, heads).astype(np.float32), g.standard_normal((heads, dim, vdim)).astype(np.float32)
+    qp, kp = np.full((rows, heads, dq), 3.0), np.full((rows, heads, dq), 3.0)
+    qp[..., :dim], kp[..., :dim] = q, k
+    state = np.zeros((heads, vdim, dq), np.float32)
+    state[:, :, :dim] = S.transpose(0, 2, 1)
+    for dt in (ai.BF16, ai.F32):
+        st, out = ai.Buffer.from_slice(ctx, state), empty(ai, ctx, rows * heads * vdim, ai.F32)
+        batch = ai.CommandBatch(ctx)
+        K.linear_attention_recurrent_into(batch, upload(ai, ctx, qp, dt), upload(ai, ctx, kp, dt), upload(ai, ctx, v, dt), dt, st, ai.Buffer.from_slice(ctx, decay), out,
+                                          rows, heads, dim, vdim, 0.5)
+        batch.commit_and_wait()
+        want, end = O.lightning_recurrence(q, k, v, decay.astype(np.float64), S.astype(np.float64))
+        close(download(ai, out, rows * heads * vdim, ai.F32).reshape(rows, heads, vdim), 0.5 * want, F32_TOL, "output")
+        got = st.as_array(np.float32, heads * vdim * dq).reshape(heads, vdim, dq)
+        close(got[:, :, :dim], end.transpose(0, 2, 1), F32_TOL, "state")
+        assert not got[:, :, dim:].any()
+
+
 @pytest.mark.parametrize("heads,vdim,dim", [(16, 128, 128), (41, 50, 128), (41, 50, 100), (33, 64, 65), (17, 128, 160), (40, 128, 160), (81, 64, 256), (44, 117, 129), (3, 50, 300)])
 @pytest.mark.parametrize("rows", [1, 7, 8, 11, 12, 23, 24, 33])
-def test_recurrence_of_many_columns(ai, gpu, heads, vdim, dim, rows):
+def test_recurrence_of_few_and_of_many_columns(ai, gpu, heads, vdim, dim, rows):
     """Around the columns beyond which many rows share a wave's lanes, and the rows at which it has more of them ahead, with fixed decays and with a
     head's steps computed from the token."""
     ctx, K = gpu
@@ -886,7 +918,7 @@ def test_mixture_of_experts(ai, gpu, dtype, rows, experts, top, width, ff):
 
 
 @pytest.mark.parametrize("experts,top,width,ff", [(16, 2, 2048, 1024), (8, 2, 1024, 512), (17, 3, 2048, 1024), (5, 5, 512, 40), (32, 4, 1536, 1536), (33, 1, 4096, 900), (1, 1, 64, 8),
-                                                  (6, 2, 100, 24), (16, 2, 1368, 688), (33, 2, 1536, 256), (64, 4, 2048, 512), (32, 4, 1032, 512), (17, 2, 1024, 512)])
+                                                  (6, 2, 100, 24), (16, 2, 1368, 688)])
 def test_router_in_the_launch_of_the_experts(ai, gpu, experts, top, width, ff):
     """The bits of the router's product and of the experts' own launch behind it, with and without room for the router."""
     ctx, K = gpu
@@ -904,6 +936,12 @@ def test_router_in_the_launch_of_the_experts(ai, gpu, experts, top, width, ff):
         batch.commit_and_wait()
         got.append((lb.as_array(np.uint32), hid.as_array(np.uint32)))
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]) and got[0][1].any()
+
+
+@pytest.mark.parametrize("experts,top,width,ff", [(33, 2, 1536, 256), (64, 4, 2048, 512), (32, 4, 1032, 512), (17, 2, 1024, 512)])
+def test_router_beside_the_launch_of_the_experts(ai, gpu, experts, top, width, ff):
+    """Around the experts and columns at which the router has a launch of its own and the experts' has four or eight waves."""
+    test_router_in_the_launch_of_the_experts(ai, gpu, experts, top, width, ff)
 
 
 def test_equal_scores_go_to_the_lower_expert(ai, gpu):
