@@ -86,3 +86,16 @@ def test_a_first_token_makes_the_views_of_its_rows_once_for_each_size(pkg, gpu, 
     first = len(made)
     pipe.forward_token(4, 1)
     assert first <= 2 * 8 + cfg.num_hidden_layers and len(made) == first
+
+
+@pytest.mark.parametrize("head_dims", [(128, 256), (256, 512)])
+def test_a_tokens_projections_stand_apart_only_where_one_launch_may_prepare_and_attend(pkg, gpu, monkeypatch, head_dims):
+    """Heads of other than 256 dims are prepared where the projections leave them, as without the fused step."""
+    ctx, K = gpu
+    cfg = _config(pkg, 64, head_dims)
+    pipe = pkg.pipeline.DecodePipeline.from_host(ctx, K, cfg, pkg.synth.decode_model_tensors(cfg, pkg.synth.rng(5, 1), [512, 512, 512, 1024, 1024, 1024]), 256)
+    seen, step = {}, pkg.kv_cache.QuantizedKvCache.attend_token_into
+    monkeypatch.setattr(pkg.kv_cache.QuantizedKvCache, "attend_token_into",
+                        lambda self, batch, kernels, raw, q, *a: seen.setdefault(self.head_dim, set()).add(raw[0] is q) or step(self, batch, kernels, raw, q, *a))
+    pipe.forward_token(3, 0)
+    assert seen == {hd: {hd != 256} for hd in head_dims}
